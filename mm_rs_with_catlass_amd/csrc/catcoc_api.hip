@@ -26,6 +26,19 @@ int launch_gemm_f16(const GemmArgs &args, int variant, bool edge, void *stream);
 int launch_gemm_bf16(const GemmArgs &args, int variant, bool edge, void *stream);
 int launch_gemm_dma_f16(const GemmArgs &args, void *stream);
 int launch_gemm_dma_bf16(const GemmArgs &args, void *stream);
+int launch_gemm_flex_i8(const GemmArgs &args, int rowBlocks, void *stream);
+int launch_gemm_flex_f16(const GemmArgs &args, int rowBlocks, void *stream);
+int launch_gemm_flex_bf16(const GemmArgs &args, int rowBlocks, void *stream);
+
+static int launch_flex(uint32_t dtype, const GemmArgs &args, int rowBlocks, void *stream)
+{
+    switch (dtype) {
+        case DT_I8: return launch_gemm_flex_i8(args, rowBlocks, stream);
+        case DT_F16: return launch_gemm_flex_f16(args, rowBlocks, stream);
+        case DT_BF16: return launch_gemm_flex_bf16(args, rowBlocks, stream);
+        default: return (int)hipErrorInvalidValue;
+    }
+}
 
 static int launch_gemm(uint32_t dtype, const GemmArgs &args, int variant, bool edge, void *stream)
 {
@@ -78,11 +91,70 @@ struct Plan {
     uint32_t dtype;
     uint32_t blockNum;
     bool dma;     // full tiles, row-major operands: the direct-to-LDS kernel applies
+    int flexBlocks;          // 0 = no; else the launch can run in flexible mode (gemm_flex.h) on tiles of 64 * flexBlocks rows
     uint32_t kSlices;        // k slices per tile this launch would run with a workspace (1 = none)
     uint64_t kSliceBytes;    // workspace for that: partial tiles + counters
 };
 
 uint32_t elem_size(uint32_t dt) { return dt == DT_I8 ? 1u : 2u; }
+
+// Flexible mode (gemm_flex.h) for a launch whose schedule, kept rows and flags are filled in: fills args.fx and returns the
+// tile's rows / 64, or 0 when the launch cannot run there (A as [k,m], rows of k or columns not in 4-byte pieces, tiles of
+// another width).  `sums` = checksums were asked for: a row tile then holds whole tasks.
+int plan_flex(GemmArgs &a, uint32_t es, bool sums)
+{
+    const SchedParams &s = a.sched;
+    const uint64_t kBytes = (uint64_t)a.K * es;
+    if (a.transA || s.n0 != 256 || (s.m0 != 64 && s.m0 != 128) || kBytes % 4 != 0 || a.N % 4 != 0 || kBytes > 0x7fffffffull) return 0;
+    FlexParams &f = a.fx;
+    const uint64_t rows = s.op == OP_ALLGATHER ? (uint64_t)a.M * s.P : a.M;
+    if (rows >= (1u << 30)) return 0;
+    f.rows = (uint32_t)rows;
+    f.colTiles = ceil_div(a.N, 256u);
+    f.dRank = make_fast_div(s.mRank);
+    // the step of k that goes through registers with bounds checks: what whole steps leave, and the last step of all when
+    // rows of B end inside a 16-byte piece (the copies then read past the end of every row but the last)
+    f.tail = (uint32_t)(kBytes % 64);
+    if (f.tail == 0 && !a.transB && ((uint64_t)a.N * es) % 16 != 0) f.tail = 64;
+    // 128-row tiles, except where they would leave CUs without a tile
+    int blocks = ceil_div(f.rows, 128u) * f.colTiles >= 256u ? 2 : 1;
+    f.perRank = 0;
+    f.rowStep = 64u * blocks;
+    if (sums && (a.flags & GF_ROW_MASK)) {       // checksums per 128 x 128 block
+        if (f.rows > 64u) blocks = 2;
+        f.rowStep = 64u * blocks;
+    } else if (sums && s.op == OP_REDUCE_SCATTER && s.P > 1) {
+        if (s.loopsM > 1) {                      // a task is one tile row of one rank
+            f.perRank = 1;
+            blocks = (int)(s.m0 / 64u);
+        } else {                                 // a task is a rank's rows (at most m0)
+            if (s.mRank > 64u) blocks = 2;
+            f.rowStep = 64u * blocks / s.mRank * s.mRank;
+        }
+    }
+    f.rowTiles = f.perRank ? s.P * s.loopsM : ceil_div(f.rows, f.rowStep);
+    f.keptTile0 = 0;
+    f.keptTiles = 0;
+    if (s.op == OP_REDUCE_SCATTER && s.P > 1) {
+        f.keptTile0 = f.perRank ? a.keptRank * s.loopsM : a.keptBegin / f.rowStep;
+        f.keptTiles = f.perRank ? s.loopsM : (a.keptBegin + a.keptRows - 1u) / f.rowStep + 1u - f.keptTile0;
+    }
+    return blocks;
+}
+
+// What flexible mode asks of the pointers: operands on the 4-byte grid, everything the epilogue touches in its 8- and 16-byte
+// accesses on theirs.
+bool flex_ptrs_ok(const GemmArgs &a)
+{
+    auto on = [](const void *p, uintptr_t g) { return (uintptr_t)p % g == 0; };
+    if (!on(a.b, 4) || !on(a.d, 8) || !on(a.scaleN, 16) || !on(a.bias, 16) || !on(a.cAccum, 16) || !on(a.accDump, 16) || !on(a.outbound, 16)) return false;
+    for (uint32_t r = 0; r < a.sched.P || r == 0; ++r)
+        if (!on(a.a[r], 4)) return false;
+    if (a.nPeers && (a.peerLd % 4 != 0 || (uint64_t)a.peerLd * 4u * 160u > 0x7fffffffull)) return false;
+    for (uint32_t p = 0; p < a.nPeers; ++p)
+        if (!on(a.peers[p], 16)) return false;
+    return true;
+}
 
 // Everything a launcher checks before it launches; fills `plan` except the buffer pointers.
 int make_plan(int commType, int dataType, const CocTilingParams *t, const CatcocSymmetricDesc *d, uint32_t transA,
@@ -271,6 +343,7 @@ int make_plan(int commType, int dataType, const CocTilingParams *t, const Catcoc
             }
         }
     }
+    plan.flexBlocks = plan_flex(a, es, (a.flags & GF_OUTBOUND_STORE) == 0 && a.checksum != nullptr);
     // a workspace also lets the checksum halves of tiles that run as two workgroups meet (its counter block)
     if (a.skCount == nullptr && d->workspace != nullptr && (uintptr_t)d->workspace % 256 == 0 && d->workspaceBytes >= kCounterBlockBytes)
         a.skCount = (uint32_t *)d->workspace;
@@ -306,7 +379,9 @@ void launch_float(int commType, int dataType, void *stream, uint8_t *a, uint8_t 
     if (!dma) p.args.splitK = 0;   // the other kernels run every tile whole
     if (!dma && p.variant == 4) { fail(E_TILING, "m0 = 256 needs full tiles and 16-byte aligned row-major operands"); return; }
     if (!dma && p.args.transA) p.variant = 0;
+    const bool flex = !dma && p.flexBlocks != 0 && flex_ptrs_ok(p.args);
     const int e = dma ? (p.dtype == DT_F16 ? launch_gemm_dma_f16(p.args, stream) : launch_gemm_dma_bf16(p.args, stream))
+                  : flex ? launch_flex(p.dtype, p.args, p.flexBlocks, stream)
                       : launch_gemm(p.dtype, p.args, p.variant, p.edge, stream);
     if (e) { fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)e)); return; }
     ok();
@@ -317,7 +392,8 @@ struct SplitkPlan {
     GemmArgs args;
     uint32_t f, tiles, rowBlocks;
     uint64_t workspaceBytes;   // partial tiles + counters (0 when f == 1)
-    bool general;              // shape outside the fast routes: gemm_general_kernel on the 128x128 grid
+    bool general;              // shape outside the fast routes: flexible mode, or gemm_general_kernel on the 128x128 grid
+    int flexBlocks;            // (general) as Plan::flexBlocks
     bool wholeK;               // at most 32 rows against B as [n,k]: gemm_decode_nk_kernel, no k slices, no workspace
     bool large;                // many rows: the 128x256 direct-to-LDS kernel in row-mask mode runs instead of the split-K kernel
 };
@@ -392,8 +468,10 @@ int make_splitk_plan(const CocTilingParams *t, const CatcocSymmetricDesc *d, uin
     if (sp.general) {
         if (d->splitK > 1) return fail(E_TILING, "k %% 64 != 0 or n %% 128 != 0: this shape runs whole tiles on the general kernel; splitK %u is not available", d->splitK);
         const uint32_t stages = d->workspaceStages ? d->workspaceStages : kDefaultStages;
-        a.sched = make_sched(OP_ALLREDUCE, t->m, t->n, 1, 128, 128, cores, 1, stages, off, dir);
+        a.sched = make_sched(OP_ALLREDUCE, t->m, t->n, 1, 128, 256, cores, 1, stages, off, dir);
         a.flags |= GF_ROW_MASK;
+        sp.flexBlocks = plan_flex(a, 1, a.checksum != nullptr);
+        if (sp.flexBlocks == 0) a.sched = make_sched(OP_ALLREDUCE, t->m, t->n, 1, 128, 128, cores, 1, stages, off, dir);
         sp.f = 1;
         a.splitK = 0;
         sp.rowBlocks = 4;
@@ -457,7 +535,12 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
         a.scaleM = (const float *)scale_x1; a.scaleN = (const float *)scale_x2;
         a.bias = (const int32_t *)bias; a.cAccum = (int32_t *)c_accum;
         a.outDtype = outDataType;
-        const int eg = launch_gemm(DT_I8, a, 0, true, stream);
+        const bool flex = sp.flexBlocks != 0 && flex_ptrs_ok(a);
+        if (!flex && a.sched.n0 != 128) {
+            const SchedParams &g = a.sched;
+            a.sched = make_sched(OP_ALLREDUCE, a.M, a.N, 1, 128, 128, g.blockPerComm, 1, g.stages, g.off, g.dir);
+        }
+        const int eg = flex ? launch_flex(DT_I8, a, sp.flexBlocks, stream) : launch_gemm(DT_I8, a, 0, true, stream);
         if (eg) { fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)eg)); return; }
         ok();
         return;
@@ -534,7 +617,8 @@ void launch_quant(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_x1, uin
     if (!dma && p.variant == 4) { fail(E_TILING, "m0 = 256 needs full tiles, 16-byte aligned row-major operands and fp32 peers"); return; }
     if (!dma) p.args.splitK = 0;   // the other kernels run every tile whole
     if (!dma && p.args.transA) p.variant = 0;
-    const int e = dma ? launch_gemm_dma_i8(p.args, stream) : launch_gemm(p.dtype, p.args, p.variant, p.edge, stream);
+    const bool flex = !dma && p.flexBlocks != 0 && flex_ptrs_ok(p.args);
+    const int e = dma ? launch_gemm_dma_i8(p.args, stream) : flex ? launch_flex(p.dtype, p.args, p.flexBlocks, stream) : launch_gemm(p.dtype, p.args, p.variant, p.edge, stream);
     if (e) { fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)e)); return; }
     ok();
 }

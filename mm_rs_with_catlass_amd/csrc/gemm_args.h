@@ -27,6 +27,17 @@ enum : uint32_t {
                                   // values they reproduce bit for bit); sums and workspace stores leave the overlap out
 };
 
+// Launches in flexible mode (gemm_flex.h): row tiles over the rows of all ranks, wherever the ranks' boundaries lie.
+struct FlexParams {
+    uint32_t rows;                 // rows of the problem: M, or all shards' rows of an all-gather
+    uint32_t rowStep;              // rows of a row tile: the kernel's tile, or fewer when tasks must not be cut (checksums)
+    uint32_t perRank;              // one schedule tile row per row tile instead
+    uint32_t rowTiles, colTiles;
+    uint32_t keptTile0, keptTiles; // reduce-scatter: row tiles that hold kept rows (they start first)
+    uint32_t tail;                 // bytes of k (1 .. 64) of the last k step, which goes through registers with bounds checks; 0 = none
+    FastDiv dRank;                 // rows of one rank
+};
+
 struct GemmArgs {
     const void *a[kMaxRanks];      // A operand per rank (all-gather: the P shards; otherwise a[0])
     const void *b;
@@ -54,6 +65,7 @@ struct GemmArgs {
     int32_t *skPart;
     uint32_t *skCount;
     SchedParams sched;
+    FlexParams fx;
 };
 
 // Workgroups (before k slicing) a launch starts.

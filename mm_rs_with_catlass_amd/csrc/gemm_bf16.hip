@@ -22,4 +22,9 @@ int launch_gemm_dma_bf16(const GemmArgs &args, void *stream)
     }
     return launch_dma_128<DT_BF16>(args, (hipStream_t)stream);
 }
+
+int launch_gemm_flex_bf16(const GemmArgs &args, int rowBlocks, void *stream)
+{
+    return launch_flex<DT_BF16>(args, rowBlocks, (hipStream_t)stream);
+}
 }  // namespace catcoc

@@ -9,6 +9,7 @@
 
 #include <type_traits>
 
+#include "gemm_flex.h"
 #include "gemm_fused_kernel.h"
 
 namespace catcoc {
@@ -89,13 +90,20 @@ template <int WM, int NS = 3, bool AQ = false, bool TB = false> struct DmaPool
     static constexpr int BYTES = (WM == 4) ? (TB ? 5 * 256 * 128 : 4 * 256 * 64 + 4 * 64 * 256) : AQ ? ((NS / 2 + 1) * 128 * 128 + NS * 64 * 256) : NS * (128 * 64 + 64 * 256);
 };
 
+// Flexible mode: the ring, or the epilogue's staging areas and tables where those are larger.
+template <int MB, int NS> struct FlexPool
+{
+    static constexpr int RING = NS * (64 * MB * 64 + 64 * 256);
+    static constexpr int BYTES = RING > FLEX_POOL ? RING : FLEX_POOL;
+};
+
 // One tile (or one k slice of a tile) of the launch: position `pos` of the launch order, in the caller's LDS pool.
 // MB = 32-row blocks per wave (2; 1 = a 64-row tile of the four-wave geometry, or the eight-wave geometry W8); subRow =
 // first row of a 64-row tile inside its 128-row tile of the schedule.
 // AQ = A is copied per pair of k steps, 128 bytes per row (whole cache lines: half as many requests to L2 as two 64-byte
 // halves), as the 256-row geometry does; for the six-stage ring, whose launches have one workgroup per CU and feel every
 // request (with three stages and two workgroups per CU the same change measured slower).
-template <uint32_t DT, int WM, bool TB, bool RM, bool RG, bool TA, int MB, int NS = 3, bool PP = false, bool AQ = false, bool W8 = false>
+template <uint32_t DT, int WM, bool TB, bool RM, bool RG, bool TA, int MB, int NS = 3, bool PP = false, bool AQ = false, bool W8 = false, bool FX = false>
 __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *smem, uint32_t pos, uint32_t slice, uint32_t kSlices,
                                          uint32_t subRow)
 {
@@ -106,6 +114,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     static_assert(NS == 3 || (WM == 2 && NS >= 3 && NS <= 8), "deeper rings exist for the 128-row kernel");
     static_assert(MB == 2 || (MB == 1 && WM == 2 && (!RM || W8) && !RG && !TA), "64-row tiles exist for the four-wave geometry with A as [m,k]");
     static_assert(!W8 || (WM == 2 && MB == 1 && !RG && !TA), "eight waves on the 128-row tile: 32 rows per wave");
+    static_assert(!FX || (WM == 2 && !RM && !RG && !TA && !AQ && !W8 && !PP), "flexible mode exists for the plain ring of the four-wave geometry");
     static_assert(!AQ || (WM == 2 && NS == 6 && (MB == 2 || W8) && !TA), "pairs of A steps exist for the six-stage 128-row kernel with A as [m,k]");
     using Acc = typename AccOf<DT>::type;
     constexpr int ES = (DT == DT_I8) ? 1 : 2;   // bytes per operand element; a k step is 64 BYTES of K
@@ -113,13 +122,13 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     constexpr int NW = 2 * WR;          // waves
     constexpr int NT = 64 * NW;         // threads
     constexpr int BM = 32 * MB * WR;
-    constexpr bool HALF = MB == 1 && !W8;   // a 64-row half of a 128-row tile of the schedule
+    constexpr bool HALF = MB == 1 && !W8 && !FX;   // a 64-row half of a 128-row tile of the schedule
     constexpr int A_STAGE = BM * 64;
     constexpr int B_STAGE = 64 * 256;
     constexpr int A_DMA = BM / 16 / NW;  // 1 KiB copies per wave per stage
     constexpr int B_DMA = 16 / NW;
     constexpr int STEP_DMA = A_DMA + B_DMA;
-    constexpr int POOL = DmaPool<WM, NS, AQ, TB>::BYTES;
+    constexpr int POOL = FX ? FlexPool<MB, NS>::BYTES : DmaPool<WM, NS, AQ, TB>::BYTES;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -128,30 +137,41 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     const int c32 = lane & 31, h = lane >> 5;
 
     const SchedParams &sp = args.sched;
-    // the launch constants are all needed within the next few hundred instructions: naming them here lets the compiler
-    // fetch them as a few wide scalar loads instead of one load and one wait per use
-    asm volatile("" : : "s"(sp.xOk), "s"(sp.xRxLog), "s"(sp.xCxLog), "s"(sp.xRowsPer), "s"(sp.xColsPer), "s"(sp.xPerRank),
-                 "s"(sp.xCommLoops), "s"(sp.xLastPerRank), "s"(sp.coreLoops), "s"(sp.loopsM), "s"(sp.loopsN), "s"(sp.blockPerComm),
-                 "s"(sp.m0), "s"(sp.n0), "s"(sp.mRank), "s"(sp.off));
-    asm volatile("" : : "s"(sp.dColsPer.d), "s"(sp.dColsPer.m), "s"(sp.dLoopsM.d), "s"(sp.dLoopsM.m), "s"(sp.dBand.d), "s"(sp.dBand.m),
-                 "s"(sp.dPerRank.d), "s"(sp.dPerRank.m), "s"(sp.dStages.d), "s"(sp.dStages.m), "s"(sp.dBpc.d), "s"(sp.dBpc.m),
-                 "s"(args.keptRank), "s"(args.flags), "s"(args.K), "s"(args.N));
-    const bool linear = (args.flags & GF_LINEAR_ORDER) != 0;
-    if (pos >= sp.coreLoops) return;
     uint32_t task;
     TileInfo ti;
-    if (!linear && sp.xOk) {
-        xcd_launch_tile(sp, args.keptRank, pos, task, ti);
+    FlexTile ft;
+    if constexpr (FX) {
+        flex_tile(args, pos, ft);
+        task = ft.index;
+        ti.row = ft.row0;
+        ti.col = ft.col0;
+        ti.rowsValid = ft.rowsValid;
+        ti.colsValid = ft.colsValid;
+        ti.targetRank = ti.rowInRank = ti.wsRow = 0;
     } else {
-        task = launch_task(sp, pos, linear, args.keptRank);
-        TileInfo tg;   // (a separate object: filled in place, the tile of both routes ends up in memory instead of registers)
-        task_tile(sp, task, tg);
-        ti = tg;
-    }
-    if constexpr (HALF) {
-        ti.row += subRow;
-        ti.rowInRank += subRow;
-        ti.wsRow += subRow;
+        // the launch constants are all needed within the next few hundred instructions: naming them here lets the compiler
+        // fetch them as a few wide scalar loads instead of one load and one wait per use
+        asm volatile("" : : "s"(sp.xOk), "s"(sp.xRxLog), "s"(sp.xCxLog), "s"(sp.xRowsPer), "s"(sp.xColsPer), "s"(sp.xPerRank),
+                     "s"(sp.xCommLoops), "s"(sp.xLastPerRank), "s"(sp.coreLoops), "s"(sp.loopsM), "s"(sp.loopsN), "s"(sp.blockPerComm),
+                     "s"(sp.m0), "s"(sp.n0), "s"(sp.mRank), "s"(sp.off));
+        asm volatile("" : : "s"(sp.dColsPer.d), "s"(sp.dColsPer.m), "s"(sp.dLoopsM.d), "s"(sp.dLoopsM.m), "s"(sp.dBand.d), "s"(sp.dBand.m),
+                     "s"(sp.dPerRank.d), "s"(sp.dPerRank.m), "s"(sp.dStages.d), "s"(sp.dStages.m), "s"(sp.dBpc.d), "s"(sp.dBpc.m),
+                     "s"(args.keptRank), "s"(args.flags), "s"(args.K), "s"(args.N));
+        const bool linear = (args.flags & GF_LINEAR_ORDER) != 0;
+        if (pos >= sp.coreLoops) return;
+        if (!linear && sp.xOk) {
+            xcd_launch_tile(sp, args.keptRank, pos, task, ti);
+        } else {
+            task = launch_task(sp, pos, linear, args.keptRank);
+            TileInfo tg;   // (a separate object: filled in place, the tile of both routes ends up in memory instead of registers)
+            task_tile(sp, task, tg);
+            ti = tg;
+        }
+        if constexpr (HALF) {
+            ti.row += subRow;
+            ti.rowInRank += subRow;
+            ti.wsRow += subRow;
+        }
     }
     uint32_t shiftM = 0, shiftN = 0;   // RG: rows / columns at the start of the tile that belong to the neighbouring tile
     if constexpr (RG) {
@@ -163,7 +183,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     }
     // The kept tiles are the longest chain of a reduce-scatter launch (main loop, then the peers' partials):
     // their waves get priority over the other workgroup on the CU so that the chain starts its streaming early.
-    if (sp.op == OP_REDUCE_SCATTER && sp.P > 1 && ti.row >= args.keptBegin && ti.row < args.keptBegin + args.keptRows)
+    if (sp.op == OP_REDUCE_SCATTER && sp.P > 1 && ti.row + (FX ? ti.rowsValid - 1u : 0u) >= args.keptBegin && ti.row < args.keptBegin + args.keptRows)
         __builtin_amdgcn_s_setprio(3);
 
     const int64_t ldaB = args.lda * ES, ldbB = args.ldb * ES;  // row pitches in bytes
@@ -172,11 +192,14 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
                               (TA ? (int64_t)(gather ? ti.rowInRank : ti.row) * ES : (int64_t)(gather ? ti.rowInRank : ti.row) * ldaB);
     const unsigned char *Bg = (const unsigned char *)args.b + (TB ? (size_t)ti.col * ldbB : (size_t)ti.col * ES);
     // k steps (64 bytes of K each) of this workgroup: all of them, or its slice
-    const uint32_t nkAll = args.K * ES / 64;
+    // (FX: whole steps here; what is left of k, args.fx.tail bytes per row, goes through registers, see below)
+    const uint32_t nkAll = FX ? (args.K * ES - args.fx.tail) / 64 : args.K * ES / 64;
     uint32_t nk = nkAll;
+    size_t kOff = 0;   // bytes of k before this workgroup's first step
     if (kSlices > 1) {   // (at most 16 slices of fewer than 2^24 steps: 32-bit products)
         const uint32_t kFirst = nkAll * slice / kSlices;
         nk = nkAll * (slice + 1u) / kSlices - kFirst;
+        kOff = (size_t)kFirst * 64;
         Ag += TA ? (size_t)kFirst * (64 / ES) * ldaB : (size_t)kFirst * 64;
         Bg += TB ? (size_t)kFirst * 64 : (size_t)kFirst * (64 / ES) * ldbB;
     }
@@ -193,7 +216,10 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     const unsigned char *gA[A_DMA];
 #pragma unroll
     for (int jj = 0; jj < A_DMA; ++jj) {
-        if constexpr (!TA) {
+        if constexpr (FX) {
+            const uint32_t row = ti.row + umin(16u * (w + NW * jj) + (lane >> 2), ti.rowsValid - 1u);
+            gA[jj] = flex_row_ptr(args, row, ldaB) + kOff + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
+        } else if constexpr (!TA) {
             gA[jj] = Ag + (size_t)(16 * (w + NW * jj) + (lane >> 2)) * ldaB + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
         } else if constexpr (ES == 1) {
             const int row = 8 * (w + NW * jj) + (lane >> 3);
@@ -218,7 +244,20 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     const unsigned char *gB[B_DMA];
 #pragma unroll
     for (int jj = 0; jj < B_DMA; ++jj) {
-        if constexpr (TB) {
+        if constexpr (FX) {
+            // columns past the last one repeat it; a row that ends inside a 16-byte piece is read a few bytes into the next row,
+            // whose values land in columns nobody looks at (the last row of B is never read here: it belongs to the checked step)
+            const uint32_t last = ti.colsValid - 1u;
+            if constexpr (TB) {
+                gB[jj] = Bg + (size_t)umin(16u * (w + NW * jj) + (lane >> 2), last) * ldbB + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
+            } else if constexpr (ES == 1) {
+                const int row = 4 * (w + NW * jj) + (lane >> 4);
+                gB[jj] = Bg + (size_t)row * ldbB + (umin((lane & 15) ^ ((row & 7) << 1), last / 16u) * 16);
+            } else {
+                const int row = 2 * (w + NW * jj) + (lane >> 5);
+                gB[jj] = Bg + (size_t)row * ldbB + (umin((lane & 31) ^ ((row & 3) << 2), last / 8u) * 16);
+            }
+        } else if constexpr (TB) {
             gB[jj] = Bg + (size_t)(16 * (w + NW * jj) + (lane >> 2)) * ldbB + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
         } else if constexpr (ES == 1) {
             const int row = 4 * (w + NW * jj) + (lane >> 4);
@@ -566,6 +605,46 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
                 issue_a(offA(st));
                 issue_b(offB(st));
             }
+        if constexpr (FX) {
+            if (args.fx.tail != 0 && slice + 1u == kSlices) {
+                // What the whole steps leave of k comes FIRST, while the copies of the first stages are on their way: through
+                // registers with bounds checks into the one stage the prologue did not fill.  Sums do not mind the order of k.
+                const int tail = (int)args.fx.tail;
+                unsigned char *ta = smem + (NS - 1) * A_STAGE, *tb = smem + NS * A_STAGE + (NS - 1) * B_STAGE;
+                const size_t kEnd = (size_t)nkAll * 64;   // bytes of k in whole steps
+#pragma unroll
+                for (int q = 0; q < A_STAGE / 16 / NT; ++q) {
+                    const uint32_t idx = tid + NT * q, row = idx >> 2, c = idx & 3u;
+                    const unsigned char *src = flex_row_ptr(args, ti.row + umin(row, ti.rowsValid - 1u), ldaB) + kEnd + c * 16u;
+                    *(v4i *)(ta + row * 64 + ((c ^ ((row >> 2) & 3u)) * 16)) = load16_guarded(src, tail - (int)c * 16);
+                }
+#pragma unroll 4
+                for (int q = 0; q < B_STAGE / 16 / NT; ++q) {
+                    const uint32_t idx = tid + NT * q;
+                    const unsigned char *b = (const unsigned char *)args.b;
+                    if constexpr (TB) {
+                        const uint32_t row = idx >> 2, c = idx & 3u;
+                        *(v4i *)(tb + row * 64 + ((c ^ ((row >> 2) & 3u)) * 16)) =
+                            load16_guarded(b + (size_t)(ti.col + umin(row, ti.colsValid - 1u)) * ldbB + kEnd + c * 16u, tail - (int)c * 16);
+                    } else {
+                        constexpr int CH = 256 * ES / 16;   // pieces of a row of k
+                        const uint32_t row = idx / CH, c = idx % CH;
+                        const int inRow = (int)(ti.colsValid * ES) - (int)c * 16;
+                        *(v4i *)(tb + row * (256 * ES) + ((c ^ (ES == 1 ? (row & 7u) << 1 : (row & 3u) << 2)) * 16)) =
+                            load16_guarded(b + (kEnd / ES + row) * ldbB + (size_t)ti.col * ES + c * 16u, (int)row * ES < tail ? inRow : 0);
+                    }
+                }
+                __syncthreads();
+                load_a(fa0, ta, 0);
+                load_b(fb0, tb, 0);
+                load_a(fa1, ta, 1);
+                load_b(fb1, tb, 1);
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (step 0 hands the stage to a copy right after its barrier)
+                mma(fa0, fb0);
+                mma(fa1, fb1);
+            }
+        }
+        if (!FX || nk > 0) {
         // step 0 (peeled: no MFMAs pending yet)
         wait_steps(umin(NS - 2, nk - 1));
         barrier_keep_vmem();
@@ -601,6 +680,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             step(false);
         }
         mma(fa1, fb1);
+        }
     } else if constexpr (TB) {
         // ---- 256x256, B as [n][k] ---------------------------------------------------------------------
         // Both operands are rows of k: both sit in pair buffers (256 rows x 128 bytes = two k steps, whole 128-byte lines per
@@ -934,6 +1014,10 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
         }
     }
 
+    if constexpr (FX) {
+        flex_epilogue<DT, MB>(args, acc, smem, ft);
+        return;
+    }
     // ---- epilogue -----------------------------------------------------------------
     // acc[mb][nb][r] is element (row, col) of the tile with
     //   row = wm*32*MB + mb*32 + (r>>2)*8 + h*4 + (r&3),  col = wn*128 + nb*32 + c32
@@ -1430,6 +1514,28 @@ __global__ void __launch_bounds__(128 * WM * (W8 ? 2 : 1), NS == 3 ? 2 : 1) gemm
         }
     }
     dma_tile<DT, WM, TB, RM, RG, TA, W8 ? 1 : 2, NS, PP, AQ, W8>(args, smem, pos, slice, kSlices, 0);
+}
+
+// Flexible mode: tiles of 64 * MB rows over the rows of all ranks (gemm_flex.h).
+template <uint32_t DT, bool TB, int MB, int NS>
+__global__ void __launch_bounds__(256, 2) gemm_flex_kernel(const GemmArgs args)
+{
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[FlexPool<MB, NS>::BYTES];
+    dma_tile<DT, 2, TB, false, false, false, MB, NS, false, false, false, true>(args, smem, blockIdx.x, 0, 1, 0);
+}
+
+template <uint32_t DT>
+inline int launch_flex(const GemmArgs &args, int rowBlocks, hipStream_t s)
+{
+    const dim3 grid(args.fx.rowTiles * args.fx.colTiles), block(256);
+    if (rowBlocks == 1) {
+        if (args.transB) hipLaunchKernelGGL((gemm_flex_kernel<DT, true, 1, 4>), grid, block, 0, s, args);
+        else hipLaunchKernelGGL((gemm_flex_kernel<DT, false, 1, 4>), grid, block, 0, s, args);
+    } else {
+        if (args.transB) hipLaunchKernelGGL((gemm_flex_kernel<DT, true, 2, 3>), grid, block, 0, s, args);
+        else hipLaunchKernelGGL((gemm_flex_kernel<DT, false, 2, 3>), grid, block, 0, s, args);
+    }
+    return (int)hipGetLastError();
 }
 
 // Reduce-scatter launches of a single round of workgroups (no more tiles than the 512 slots of the GPU) run some tiles as two

@@ -22,4 +22,9 @@ int launch_gemm_dma_f16(const GemmArgs &args, void *stream)
     }
     return launch_dma_128<DT_F16>(args, (hipStream_t)stream);
 }
+
+int launch_gemm_flex_f16(const GemmArgs &args, int rowBlocks, void *stream)
+{
+    return launch_flex<DT_F16>(args, rowBlocks, (hipStream_t)stream);
+}
 }  // namespace catcoc

@@ -1,0 +1,323 @@
+// Tiles that need not line up with the schedule's tiles, and the epilogue that goes with them.
+//
+// A launch of the direct-to-LDS kernels in flexible mode (FX) cuts the rows of the whole problem -- all ranks' rows behind
+// each other -- into row tiles of its own, whatever the ranks' boundaries, and lets the row decide in the epilogue where its
+// values go: to the kept rows (peers added), to its place in the tile-linear workspace, or into its task's checksum.  With
+// eight ranks of 125 rows that is 8 tiles of 128 rows and not 8 tiles plus their edges, with eight ranks of 8 rows one tile
+// and not eight, and the shards of an all-gather share tiles in the same way.  Rows past the end repeat the last row on
+// the way in and are dropped on the way out; so are columns.
+//
+// The epilogue goes through LDS once (32 rows of a wave at a time), after which a lane holds four consecutive columns of a
+// row: every access to peers, output, workspace and dumps is 8 or 16 bytes per lane over whole row segments, and what a
+// row is to do is one table entry per row.
+//
+// Bound by the same things as the aligned kernels it shares its main loop with: the tile copies and the matrix pipes for long
+// k, the peers' stream for short k.  Measured against what ran these launches before (a kernel that staged its tiles through
+// registers, or one thread per output element), launches alternating: fp16 all-gather 8 x [1024,6148] x [6148,5120]
+// 243 ms -> 0.522 ms = 988 TFLOP/s (12296-byte rows, 8 bytes of k left over), W8A8 reduce-scatter 1000x1376x4096 with 125
+// rows per rank and stored tiles 276 -> 32 us, bf16 all-reduce 16x1024x8192 28.6 -> 18.2 us.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <type_traits>
+
+#include "gemm_fused_kernel.h"
+
+namespace catcoc {
+
+// ---- launch position -> tile ------------------------------------------------------------------------------------------
+struct FlexTile {
+    uint32_t row0, rowsValid;   // global rows (of all ranks) [row0, row0 + rowsValid)
+    uint32_t col0, colsValid;
+    uint32_t index;             // rowTile * colTiles + colTile
+};
+
+CATCOC_HD uint32_t flex_row_start(const GemmArgs &a, uint32_t rt, uint32_t &valid)
+{
+    const FlexParams &f = a.fx;
+    if (f.perRank) {   // one schedule tile row per row tile: checksums of tasks that are not whole ranks
+        const uint32_t rank = rt / a.sched.loopsM, mi = rt - rank * a.sched.loopsM;
+        valid = umin(a.sched.m0, a.sched.mRank - mi * a.sched.m0);
+        return rank * a.sched.mRank + mi * a.sched.m0;
+    }
+    const uint32_t row0 = rt * f.rowStep;
+    valid = umin(f.rowStep, f.rows - row0);
+    return row0;
+}
+
+// Consecutive workgroups go round-robin to the eight XCDs, each with an L2 of its own: XCD x takes the x-th contiguous
+// eighth of the tile sequence, and the sequence walks bands of eight tile rows, so that the tiles in flight on one XCD form
+// a compact block of the grid.  Row tiles with kept rows of a reduce-scatter launch come first (their epilogue streams the
+// peers' partials: the longest chain of the launch), dealt to the XCDs in the same way.
+CATCOC_HD uint32_t xcd_eighth(uint32_t pos, uint32_t count)
+{
+    const uint32_t x = pos & 7u, q = count >> 3, r = count & 7u;
+    return x * q + umin(x, r) + (pos >> 3);
+}
+
+CATCOC_HD void flex_tile(const GemmArgs &a, uint32_t pos, FlexTile &t)
+{
+    const FlexParams &f = a.fx;
+    const uint32_t first = f.keptTiles * f.colTiles;
+    const bool kept = pos < first;
+    uint32_t seq, rows;
+    if (kept) { rows = f.keptTiles; seq = xcd_eighth(pos, first); }
+    else { rows = f.rowTiles - f.keptTiles; seq = xcd_eighth(pos - first, rows * f.colTiles); }
+    const uint32_t BAND = 8u;
+    const uint32_t band = seq / (BAND * f.colTiles), in = seq - band * (BAND * f.colTiles);
+    const uint32_t w = umin(BAND, rows - band * BAND);
+    const uint32_t ct = in / w;
+    uint32_t rt = band * BAND + (in - ct * w);
+    if (kept) rt += f.keptTile0;
+    else if (rt >= f.keptTile0) rt += f.keptTiles;
+    t.row0 = flex_row_start(a, rt, t.rowsValid);
+    t.col0 = ct * 256u;
+    t.colsValid = umin(256u, a.N - t.col0);
+    t.index = rt * f.colTiles + ct;
+}
+
+// ---- a row's place ------------------------------------------------------------------------------------------------------
+// Row `ri` of rank `r` in column tile `ni`: its task, and its row of the tile-linear workspace (tile_sched.h: task_tile).
+__device__ __forceinline__ void flex_task_of(const SchedParams &s, uint32_t r, uint32_t ri, uint32_t ni, uint32_t &task, uint32_t &wsRow)
+{
+    const uint32_t mi = ri / s.m0;
+    const uint32_t inRank = swizzle_block_index(s.off, s.dir, s.loopsM, s.loopsN, mi, ni);
+    const uint32_t perRank = s.blockPerComm / s.P;
+    const uint32_t round = inRank / perRank, idx = inRank - round * perRank;
+    const uint32_t commLoops = ceil_div(s.coreLoops, s.blockPerComm);
+    const uint32_t actual = (round == commLoops - 1u) ? s.coreLoops - round * s.blockPerComm : s.blockPerComm;
+    const uint32_t b = r * (actual / s.P) + idx;
+    task = round * s.blockPerComm + b;
+    wsRow = ((round % s.stages) * s.blockPerComm + b) * s.m0 + (ri - mi * s.m0);
+}
+
+// Address of row v of the left operand (all-gather: row v of the shards behind each other).
+__device__ __forceinline__ const unsigned char *flex_row_ptr(const GemmArgs &a, uint32_t v, int64_t ldaB)
+{
+    if (a.sched.op == OP_ALLGATHER) {
+        uint32_t in;
+        const uint32_t r = fast_div(v, a.fx.dRank, in);
+        return (const unsigned char *)a.a[r] + (size_t)in * ldaB;
+    }
+    return (const unsigned char *)a.a[0] + (size_t)v * ldaB;
+}
+
+// 16 bytes of which the first `valid` exist (a multiple of four, at most 16 are read; the rest read as zero); 4-byte aligned.
+typedef int v4i_u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ v4i load16_guarded(const unsigned char *p, int valid)
+{
+    v4i v = {0, 0, 0, 0};
+    if (valid >= 16) {
+        v = *(const v4i_u *)p;
+    } else {
+        if (valid > 0) v.x = *(const int *)p;
+        if (valid > 4) v.y = *(const int *)(p + 4);
+        if (valid > 8) v.z = *(const int *)(p + 8);
+    }
+    return v;
+}
+
+// ---- epilogue -------------------------------------------------------------------------------------------------------------
+enum : uint32_t { FX_SKIP = 0u, FX_KEPT = 1u << 30, FX_OUT = 2u << 30, FX_SUM = 3u << 30, FX_KIND = 3u << 30, FX_INDEX = (1u << 30) - 1u };
+
+constexpr int FLEX_STAGING = 4 * 16384;                 // one 16 KiB area per wave
+constexpr int FLEX_POOL = FLEX_STAGING + 128 * 8 + 16 * 12;   // + the row table + the sums of up to 16 tasks
+
+// acc[mb][nb][r] of wave (wm, wn) is element (row, col) of the tile with
+//   row = wm*32*MB + mb*32 + (r>>2)*8 + h*4 + (r&3),  col = wn*128 + nb*32 + c32
+template <uint32_t DT, int MB>
+__device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename AccOf<DT>::type (&acc)[MB][4], unsigned char *smem, const FlexTile &t)
+{
+    constexpr bool I8 = DT == DT_I8;
+    using Sum = typename std::conditional<I8, long long, double>::type;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const uint32_t w = __builtin_amdgcn_readfirstlane((uint32_t)tid >> 6);
+    const uint32_t wm = w >> 1, wn = w & 1u;
+    const int c32 = lane & 31, h = lane >> 5;
+    const bool redI32 = I8 && (args.flags & GF_REDUCE_INT32) != 0;
+    const bool store = (args.flags & GF_OUTBOUND_STORE) != 0;
+
+    uint32_t *dst = (uint32_t *)(smem + FLEX_STAGING);      // [128] what row i of the tile does
+    float *rowScale = (float *)(dst + 128);                  // [128] W8A8 per-token scale
+    Sum *sums = (Sum *)(rowScale + 128);                     // [16] task sums (explicit kept rows: one per 128 columns)
+    uint32_t *sumTask = (uint32_t *)(sums + 16);             // [16]
+    __syncthreads();   // every wave has left the main loop's LDS reads behind
+    if (tid < 64 * MB) {
+        const uint32_t v = t.row0 + tid;
+        uint32_t e = FX_SKIP;
+        if ((uint32_t)tid < t.rowsValid) {
+            if (v - args.keptBegin < args.keptRows) {   // (unsigned: rows above keptBegin wrap)
+                e = FX_KEPT | (v - args.keptBegin);
+            } else if (args.flags & GF_ROW_MASK) {
+                e = args.checksum ? FX_SUM : FX_SKIP;
+            } else if (store || args.checksum) {
+                uint32_t ri, task, ws;
+                const uint32_t r = fast_div(v, args.fx.dRank, ri);
+                flex_task_of(args.sched, r, ri, t.col0 / args.sched.n0, task, ws);
+                if (store) {
+                    e = FX_OUT | ws;
+                } else {   // tiles with checksums hold whole tasks: task g of the tile starts at its row g * mRank
+                    const uint32_t g = args.fx.perRank ? 0u : tid / args.sched.mRank;
+                    e = FX_SUM | g;
+                    sumTask[g] = task;
+                }
+            }
+        }
+        dst[tid] = e;
+        if constexpr (I8) rowScale[tid] = args.scaleM[umin(v, args.fx.rows - 1u)];
+    }
+    if (tid < 16) sums[tid] = 0;
+    __syncthreads();
+
+    unsigned char *st = smem + w * 16384;
+    const uint32_t lrow = lane >> 5, chunk = lane & 31;
+    const uint32_t lcol = wn * 128u + chunk * 4u;            // the lane's four columns inside the tile
+    const bool colOk = lcol < t.colsValid;
+    const uint32_t gcol = t.col0 + lcol;
+    v4f sN = {1.f, 1.f, 1.f, 1.f};
+    v4i bv = {0, 0, 0, 0};
+    if constexpr (I8) {
+        if (colOk) {
+            sN = *(const v4f *)(args.scaleN + gcol);
+            if (args.bias) bv = *(const v4i *)(args.bias + gcol);
+        }
+    }
+    // peers: a base at the tile's first kept row, one 32-bit offset per row from there; a lane with nothing to read gets an
+    // offset behind the end of the descriptor (no memory is touched, zeros arrive)
+    const uint32_t kept0 = t.row0 > args.keptBegin ? t.row0 - args.keptBegin : 0u;
+    const uint32_t peerPitch = (uint32_t)args.peerLd * 4u;
+    Sum run = 0;              // of the rows of task `runOf` this lane has met since the last flush
+    uint32_t runOf = 0;
+
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const uint32_t wrow = (r >> 2) * 8 + h * 4 + (r & 3);
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) {
+                const auto e = acc[mb][nb][r];
+                *(int *)(st + wrow * 512 + (((nb * 32 + c32) * 4) ^ (h << 7))) = __builtin_bit_cast(int, e);
+            }
+        }
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {   // 16 rows: a lane has eight of them, two apart
+            v4i cur[8];
+            uint32_t d[8];
+            bool anyKept = false;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const uint32_t wrow = half * 16 + j * 2 + lrow;
+                cur[j] = *(const v4i *)(st + wrow * 512 + ((chunk * 16) ^ (((wrow >> 2) & 1) << 7)));
+                d[j] = dst[wm * 32 * MB + mb * 32 + wrow];
+                if constexpr (I8) cur[j] += bv;
+                if (!colOk) d[j] = FX_SKIP;
+                anyKept |= (d[j] & FX_KIND) == FX_KEPT;
+            }
+            anyKept = __ballot(anyKept) != 0;   // (wave-uniform)
+            if (args.accDump) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const uint32_t i = wm * 32 * MB + mb * 32 + half * 16 + j * 2 + lrow;
+                    if (colOk && i < t.rowsValid) *(v4i *)((int32_t *)args.accDump + (size_t)(t.row0 + i) * args.N + gcol) = cur[j];
+                }
+            }
+            uint32_t off[8];   // of the lane's rows in a peer's kept block
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                off[j] = (d[j] & FX_KIND) == FX_KEPT ? ((d[j] & FX_INDEX) - kept0) * peerPitch + gcol * 4u : 0xfffffff0u;
+            constexpr int NBUF = 3;
+            v4i buf[NBUF][8];
+            auto fetch = [&](v4i (&b)[8], uint32_t p) {
+                const float *base = (const float *)args.peers[umin(p, (uint32_t)kMaxRanks - 1u)] + (args.peerRowOffset + (int64_t)kept0) * args.peerLd;
+                const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, p < args.nPeers ? 0x7ffffff0 : 0, 0x00020000);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) b[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, off[j], 0, 2 /* nt */);
+            };
+            auto add_peers = [&](auto add) {   // peers in slot order, two of them in flight behind the one being added
+                if (!anyKept || args.nPeers == 0) return;
+#pragma unroll
+                for (int q = 0; q < NBUF - 1; ++q) fetch(buf[q], q);
+                for (uint32_t p = 0; p < args.nPeers; p += NBUF) {
+#pragma unroll
+                    for (int q = 0; q < NBUF; ++q) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        fetch(buf[(q + NBUF - 1) % NBUF], p + q + NBUF - 1);
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (p + q < args.nPeers) {
+#pragma unroll
+                            for (int j = 0; j < 8; ++j) add(cur[j], buf[q][j], j);
+                        }
+                    }
+                }
+            };
+            // (a row that is not kept adds the zeros its loads returned: nothing for int32; floats are added to kept rows only)
+            if constexpr (I8) {
+                if (redI32) add_peers([](v4i &c, const v4i &b, int) { c += b; });
+                if (args.cAccum) {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        if ((d[j] & FX_KIND) == FX_KEPT) *(v4i *)(args.cAccum + (size_t)(d[j] & FX_INDEX) * args.N + gcol) = cur[j];
+                }
+            }
+            if (!store && args.checksum) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if ((d[j] & FX_KIND) == FX_SUM) {
+                        const uint32_t g = (args.flags & GF_ROW_MASK) ? wn : (d[j] & FX_INDEX);
+                        if (g != runOf) {
+                            if (run != 0) __hip_atomic_fetch_add(sums + runOf, run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                            run = 0;
+                            runOf = g;
+                        }
+                        if constexpr (I8) run += ((long long)cur[j].x + cur[j].y) + ((long long)cur[j].z + cur[j].w);
+                        else run += ((double)i2f(cur[j].x) + (double)i2f(cur[j].y)) + ((double)i2f(cur[j].z) + (double)i2f(cur[j].w));
+                    }
+            }
+            if constexpr (I8) {   // dequantise: per-channel scale first, then per-token, each product rounded on its own
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (!(redI32 && (d[j] & FX_KIND) == FX_OUT)) {   // (tiles of other ranks leave as raw int32 there)
+                        const float sM = rowScale[wm * 32 * MB + mb * 32 + half * 16 + j * 2 + lrow];
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) cur[j][c] = f2i(__fmul_rn(__fmul_rn((float)cur[j][c], sN[c]), sM));
+                    }
+            }
+            if (!redI32)
+                add_peers([&](v4i &c, const v4i &b, int j) {
+                    if ((d[j] & FX_KIND) == FX_KEPT) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) c[e] = f2i(__fadd_rn(i2f(c[e]), i2f(b[e])));
+                    }
+                });
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const uint32_t kind = d[j] & FX_KIND, idx = d[j] & FX_INDEX;
+                if (kind == FX_KEPT) {
+                    uint32_t q[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) q[e] = f32_to_out16(i2f(cur[j][e]), args.outDtype) & 0xffffu;
+                    *(v2i *)((unsigned short *)args.d + (size_t)idx * args.ldd + gcol) = v2i{(int)(q[0] | (q[1] << 16)), (int)(q[2] | (q[3] << 16))};
+                } else if (kind == FX_OUT) {
+                    __builtin_nontemporal_store(cur[j], (v4i *)((float *)args.outbound + (size_t)idx * args.sched.n0 + lcol));
+                }
+            }
+        }
+    }
+    if (!store && args.checksum) {
+        if (run != 0) __hip_atomic_fetch_add(sums + runOf, run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __syncthreads();
+        if (args.flags & GF_ROW_MASK) {
+            const uint32_t cols128 = ceil_div(args.N, 128u);
+            if (tid < 2 && t.col0 / 128u + tid < cols128) ((Sum *)args.checksum)[(size_t)(t.row0 / 128u) * cols128 + t.col0 / 128u + tid] = sums[tid];
+        } else {
+            // task g of the tile (the only one when row tiles are tile rows of the schedule): its first row says whether it is
+            // one of the others', and only then sumTask[g] was written
+            const uint32_t g = tid, first = g * args.sched.mRank;
+            if (g < (args.fx.perRank ? 1u : 16u) && first < t.rowsValid && (dst[first] & FX_KIND) == FX_SUM) ((Sum *)args.checksum)[sumTask[g]] = sums[g];
+        }
+    }
+}
+
+}  // namespace catcoc

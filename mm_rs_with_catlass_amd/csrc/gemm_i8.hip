@@ -57,4 +57,9 @@ int launch_gemm_dma_i8(const GemmArgs &args, void *stream)
     }
     return launch_dma_128<DT_I8>(args, (hipStream_t)stream);
 }
+
+int launch_gemm_flex_i8(const GemmArgs &args, int rowBlocks, void *stream)
+{
+    return launch_flex<DT_I8>(args, rowBlocks, (hipStream_t)stream);
+}
 }  // namespace catcoc

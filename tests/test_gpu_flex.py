@@ -1,0 +1,108 @@
+"""GPU parity of launches in flexible mode (csrc/gemm_flex.h): row tiles over the rows of all ranks wherever the ranks'
+boundaries lie, k and n that fill no step and no tile.  Bars as in test_gpu_parity: int32 accumulators, checksums and W8A8
+outputs bit for bit, workspace tiles bit for bit, float outputs within the reference's gate."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from mm_rs_with_catlass_amd import lib as L
+from mm_rs_with_catlass_amd import ops
+from test_gpu_parity import TORCH_DT, _check_float, _need_gpu, _rand16, dev, dev16, host16, quant_case
+
+pytestmark = pytest.mark.gpu
+
+
+# (rows per rank, N, K, P, rank, weights as [n,k], int32 peers, m0, commInterval)
+@pytest.mark.parametrize("outbound", [False, True])
+@pytest.mark.parametrize("case", [(125, 512, 1376, 8, 5, True, False, 0, 1),     # one rank per tile; half a step of k left
+                                  (1, 260, 68, 16, 15, False, False, 0, 1),      # 16 tasks in one tile, rows of B end inside a 16-byte piece
+                                  (8, 256, 64, 8, 0, False, True, 0, 1),         # whole steps of k, raw int32 tiles
+                                  (9, 36, 4, 4, 1, True, False, 0, 1),           # no whole step of k at all
+                                  (63, 1028, 192, 4, 2, False, False, 0, 1),     # whole k, but B's last step is checked (N % 16)
+                                  (65, 772, 260, 8, 7, True, True, 0, 1),        # tiles straddle ranks
+                                  (200, 300, 320, 2, 1, False, False, 64, 2),    # caller's 64-row tiles, several per rank, two rounds
+                                  (300, 516, 100, 4, 3, True, False, 0, 1)])     # more than one tile per rank
+def test_quant_rs_any_rows_any_k(case, outbound):
+    rows, N, K, P, rank, tb, ri, m0, ci = case
+    M = rows * P
+    t = ops.default_tiling(M, K, N, P, m0=m0, n0=0, k0=0, commInterval=ci)
+    bn = 16 if ci > 1 else 0
+    r = quant_case(np.random.default_rng(rows), M, N, K, P, rank, bias=True, trans_b=tb, reduce_int32=ri, tiling=t, outbound=outbound,
+                   launches=2, block_num=bn)
+    assert r["exact"] == r["total"]
+    d = L.make_desc(rank, P, [16] * (P - 1), block_num=bn)
+    tr, row, col, ws = (C.c_uint32() for _ in range(4))
+    step = m0 or (64 if rows <= 64 else 128)
+    deq = r["acc"] if ri else oracle.dequant(r["acc"], r["s2"], r["s1"])
+    for task in range(r["ntasks"]):
+        L.load().catcoc_task_tile(L.QUANT_MATMUL_REDUCE_SCATTER, C.byref(t), C.byref(d), task, C.byref(tr), C.byref(row), C.byref(col), C.byref(ws))
+        if tr.value == rank:
+            continue
+        r1, c1 = min(row.value + step, (tr.value + 1) * rows), min(col.value + 256, N)
+        if outbound:
+            got = r["outbound"].cpu().numpy().reshape(-1, 256)[ws.value:ws.value + r1 - row.value, :c1 - col.value]
+            want = deq[row.value:r1, col.value:c1]
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), task
+        else:
+            assert int(r["checksum"][task]) == int(r["acc"][row.value:r1, col.value:c1].astype(np.int64).sum()), task
+
+
+# (op, rows (of a shard for all-gather), N, K, P, weights as [n,k])
+@pytest.mark.parametrize("dtype", [oracle.FP16, oracle.BF16])
+@pytest.mark.parametrize("case", [("allreduce", 1, 256, 128, 8, True), ("allreduce", 33, 516, 1000, 4, False), ("allreduce", 129, 260, 66, 2, False),
+                                  ("allgather", 3, 264, 516, 8, True), ("allgather", 65, 768, 1026, 4, False), ("allgather", 200, 1284, 6148, 2, False)])
+def test_float_any_rows_any_k(dtype, case):
+    _need_gpu()
+    op, m, N, K, P, tb = case
+    rng = np.random.default_rng(m + K)
+    B = _rand16(rng, (K, N), dtype, 0.02)
+    Bd = dev16(np.ascontiguousarray(B.T) if tb else B, dtype)
+    rank = P - 1
+    if op == "allgather":
+        shards = [_rand16(rng, (m, K), dtype) for _ in range(P)]
+        ds = [dev16(s, dtype) for s in shards]
+        dump = torch.zeros((m * P, N), dtype=torch.float32, device="cuda:0")
+        out = ops.allgather_matmul(ds[rank], ds[:rank], Bd, rank, P, trans_b=tb, acc_dump=dump)
+        torch.cuda.synchronize()
+        part = oracle.gemm_half_f32(np.concatenate(shards, 0), B, dtype)
+        full, want = part, oracle.allgather_matmul(shards, B, dtype)
+    else:
+        A = _rand16(rng, (m, K), dtype)
+        peers = [rng.standard_normal((m, N)).astype(np.float32) for _ in range(P - 1)]
+        part, want = oracle.matmul_reduce(A, B, dtype, 0, m, peers, want_partial=True)
+        full = part + sum(peers)
+        dump = torch.zeros((m, N), dtype=torch.float32, device="cuda:0")
+        out = ops.matmul_allreduce(dev16(A, dtype), Bd, [dev(p) for p in peers], rank, P, trans_b=tb, acc_dump=dump)
+        torch.cuda.synchronize()
+    _check_float(host16(out), want, full, dtype, K)
+    assert out.dtype == TORCH_DT[dtype]
+    # fp32 sums of K products in another order: each within K * 2^-24 of the sum of their magnitudes, here at most
+    # 4.5 * 4.5 * 0.02 * K per element (operands are normal, scales 1 and 0.02)
+    assert np.abs(dump.cpu().numpy() - part).max() <= K * 2.0 ** -24 * 0.41 * K + 1e-6
+
+
+@pytest.mark.parametrize("dtype", [oracle.FP16, oracle.BF16])
+def test_float_reduce_scatter_checksums_of_small_ranks(dtype):
+    """Several tasks in one tile: each one's sum, and the kept block with its peers."""
+    _need_gpu()
+    P, rows, N, K, rank = 8, 11, 300, 200, 3
+    rng = np.random.default_rng(31)
+    A, B = _rand16(rng, (P * rows, K), dtype), _rand16(rng, (K, N), dtype, 0.02)
+    peers = [rng.standard_normal((rows, N)).astype(np.float32) for _ in range(P - 1)]
+    part, want = oracle.matmul_reduce(A, B, dtype, rank * rows, rows, peers, want_partial=True)
+    cs = torch.zeros(2 * P, dtype=torch.float64, device="cuda:0")
+    out = ops.matmul_reduce_scatter(dev16(A, dtype), dev16(B, dtype), [dev(p) for p in peers], rank, P, checksum=cs)
+    torch.cuda.synchronize()
+    _check_float(host16(out), want, part[rank * rows:(rank + 1) * rows] + sum(peers), dtype, K)
+    t = ops.default_tiling(P * rows, K, N, P, m0=0, n0=0, k0=0)
+    d = L.make_desc(rank, P, [16] * (P - 1))
+    tr, row, col = C.c_uint32(), C.c_uint32(), C.c_uint32()
+    for task in range(2 * P):
+        L.load().catcoc_task_tile(L.MATMUL_REDUCE_SCATTER, C.byref(t), C.byref(d), task, C.byref(tr), C.byref(row), C.byref(col), None)
+        blk = part[row.value:row.value + rows, col.value:min(col.value + 256, N)].astype(np.float64)
+        # (fp32 accumulation in another order: K * 2^-24 of the magnitudes per element, as above)
+        bound = blk.size * K * 2.0 ** -24 * 0.41 * K + 1e-6
+        assert abs(float(cs[task]) - (0.0 if tr.value == rank else blk.sum())) <= bound, task
