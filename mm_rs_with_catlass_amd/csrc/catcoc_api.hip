@@ -91,6 +91,7 @@ struct Plan {
     uint32_t dtype;
     uint32_t blockNum;
     bool dma;     // full tiles, row-major operands: the direct-to-LDS kernel applies
+    bool preferFlex;         // run there although the aligned kernels would take it
     int flexBlocks;          // 0 = no; else the launch can run in flexible mode (gemm_flex.h) on tiles of 64 * flexBlocks rows
     uint32_t kSlices;        // k slices per tile this launch would run with a workspace (1 = none)
     uint64_t kSliceBytes;    // workspace for that: partial tiles + counters
@@ -100,8 +101,9 @@ uint32_t elem_size(uint32_t dt) { return dt == DT_I8 ? 1u : 2u; }
 
 // Flexible mode (gemm_flex.h) for a launch whose schedule, kept rows and flags are filled in: fills args.fx and returns the
 // tile's rows / 64, or 0 when the launch cannot run there (A as [k,m], rows of k or columns not in 4-byte pieces, tiles of
-// another width).  `sums` = checksums were asked for: a row tile then holds whole tasks.
-int plan_flex(GemmArgs &a, uint32_t es, bool sums)
+// another width).  `sums` = checksums were asked for and the tiles run whole: a row tile then holds whole tasks.  wantM0 =
+// the caller's tile rows (0: the library's choice), slices = k slices per tile.
+int plan_flex(GemmArgs &a, uint32_t es, bool sums, uint32_t wantM0, uint32_t slices)
 {
     const SchedParams &s = a.sched;
     const uint64_t kBytes = (uint64_t)a.K * es;
@@ -111,25 +113,28 @@ int plan_flex(GemmArgs &a, uint32_t es, bool sums)
     if (rows >= (1u << 30)) return 0;
     f.rows = (uint32_t)rows;
     f.colTiles = ceil_div(a.N, 256u);
+    f.slices = slices;
     f.dRank = make_fast_div(s.mRank);
     // the step of k that goes through registers with bounds checks: what whole steps leave, and the last step of all when
     // rows of B end inside a 16-byte piece (the copies then read past the end of every row but the last)
     f.tail = (uint32_t)(kBytes % 64);
     if (f.tail == 0 && !a.transB && ((uint64_t)a.N * es) % 16 != 0) f.tail = 64;
-    // 128-row tiles, except where they would leave CUs without a tile
-    int blocks = ceil_div(f.rows, 128u) * f.colTiles >= 256u ? 2 : 1;
+    // 64-row tiles as long as they are at most one per CU (measured figures: make_plan)
+    int blocks = wantM0 ? (int)(wantM0 / 64u) : slices > 1 || ceil_div(f.rows, 64u) * f.colTiles <= 256u ? 1 : 2;
     f.perRank = 0;
     f.rowStep = 64u * blocks;
-    if (sums && (a.flags & GF_ROW_MASK)) {       // checksums per 128 x 128 block
-        if (f.rows > 64u) blocks = 2;
-        f.rowStep = 64u * blocks;
-    } else if (sums && s.op == OP_REDUCE_SCATTER && s.P > 1) {
-        if (s.loopsM > 1) {                      // a task is one tile row of one rank
-            f.perRank = 1;
-            blocks = (int)(s.m0 / 64u);
-        } else {                                 // a task is a rank's rows (at most m0)
-            if (s.mRank > 64u) blocks = 2;
-            f.rowStep = 64u * blocks / s.mRank * s.mRank;
+    if (sums && slices <= 1) {
+        if (a.flags & GF_ROW_MASK) {                 // checksums per 128 x 128 block
+            if (f.rows > 64u) blocks = 2;
+            f.rowStep = 64u * blocks;
+        } else if (s.op == OP_REDUCE_SCATTER && s.P > 1) {
+            if (s.loopsM > 1) {                      // a task is one tile row of one rank
+                f.perRank = 1;
+                blocks = (int)(s.m0 / 64u);
+            } else {                                 // a task is a rank's rows (at most m0)
+                if (s.mRank > 64u) blocks = 2;
+                f.rowStep = 64u * blocks / s.mRank * s.mRank;
+            }
         }
     }
     f.rowTiles = f.perRank ? s.P * s.loopsM : ceil_div(f.rows, f.rowStep);
@@ -142,6 +147,40 @@ int plan_flex(GemmArgs &a, uint32_t es, bool sums)
     return blocks;
 }
 
+// k slices per tile a launch in flexible mode takes by itself.  A workgroup's k step takes 0.3 us as long as the CUs are not
+// full; a slice costs the second launch about 0.1 us of latency and rows x n words written and read back at 4 TB/s.  The sum
+// steps * 0.3 / f + f * (0.1 + 2e-6 * rows * n) is least at the root below.  Measured optimum / this rule, bf16 all-reduce:
+// 16x8192x1024 24 / 24, 100x8192x1024 16 / 16, 28x15360x768 32 / 31, 16x4096x4096 8-16 / 13, 64x2048x4096 6 / 6,
+// 100x1024x8192 2 / 2, 200x1024x2048 3 / 3, 400x6144x1024 8 / 8, 824x7296x1280 3 / 3 (one workgroup per CU at most).
+uint32_t flex_slices(uint32_t rows, uint32_t n, uint32_t tiles, uint32_t steps)
+{
+    const double f = sqrt(0.3 * steps / (0.1 + 2e-6 * (double)rows * (double)n));
+    const uint32_t r = umin(umin((uint32_t)(f + 0.5), tiles ? 256u / tiles : 1u), umin(steps / 4u, 64u));
+    return r < 2u ? 1u : r;
+}
+
+// The whole of it: tiles and k slices of a launch that may run in flexible mode.  *slices / *bytes report the slices it would
+// run with a large enough workspace and what that takes; with a smaller one (or none) it runs with what fits.  wantSlices =
+// the caller's own number (0: the library's).
+int plan_flex_slices(GemmArgs &a, uint32_t es, uint32_t wantM0, uint32_t wantSlices, void *workspace, uint64_t workspaceBytes, uint32_t *slices, uint64_t *bytes)
+{
+    const bool sums = (a.flags & GF_OUTBOUND_STORE) == 0 && a.checksum != nullptr;
+    const int whole = plan_flex(a, es, sums, wantM0, 1);
+    *slices = 1;
+    *bytes = 0;
+    if (whole == 0) return 0;
+    const uint32_t steps = (uint32_t)(((uint64_t)a.K * es - a.fx.tail) / 64u);
+    const uint32_t f = umin(umin(wantSlices ? wantSlices : flex_slices(a.fx.rows, a.N, ceil_div(a.fx.rows, 64u) * a.fx.colTiles, steps), 64u), steps);
+    if (f <= 1) return whole;
+    const uint64_t slice = (uint64_t)a.fx.rows * a.N * 4u;
+    *slices = f;
+    *bytes = kCounterBlockBytes + f * slice;
+    if (workspace == nullptr || (uintptr_t)workspace % 256 != 0 || workspaceBytes < kCounterBlockBytes + 2u * slice) return whole;
+    const uint64_t fit = (workspaceBytes - kCounterBlockBytes) / slice;
+    a.skPart = (int32_t *)((unsigned char *)workspace + kCounterBlockBytes);
+    return plan_flex(a, es, sums, wantM0, fit < f ? (uint32_t)fit : f);
+}
+
 // What flexible mode asks of the pointers: operands on the 4-byte grid, everything the epilogue touches in its 8- and 16-byte
 // accesses on theirs.
 bool flex_ptrs_ok(const GemmArgs &a)
@@ -150,7 +189,8 @@ bool flex_ptrs_ok(const GemmArgs &a)
     if (!on(a.b, 4) || !on(a.d, 8) || !on(a.scaleN, 16) || !on(a.bias, 16) || !on(a.cAccum, 16) || !on(a.accDump, 16) || !on(a.outbound, 16)) return false;
     for (uint32_t r = 0; r < a.sched.P || r == 0; ++r)
         if (!on(a.a[r], 4)) return false;
-    if (a.nPeers && (a.peerLd % 4 != 0 || (uint64_t)a.peerLd * 4u * 160u > 0x7fffffffull)) return false;
+    // (the epilogue addresses the peers' and the output's rows of a tile with 31-bit offsets from the tile's first one)
+    if ((a.nPeers && (a.peerLd % 4 != 0 || (uint64_t)a.peerLd * 4u * 160u > 0x7fffffffull)) || (uint64_t)a.ldd * 2u * 160u > 0x7fffffffull) return false;
     for (uint32_t p = 0; p < a.nPeers; ++p)
         if (!on(a.peers[p], 16)) return false;
     return true;
@@ -343,7 +383,29 @@ int make_plan(int commType, int dataType, const CocTilingParams *t, const Catcoc
             }
         }
     }
-    plan.flexBlocks = plan_flex(a, es, (a.flags & GF_OUTBOUND_STORE) == 0 && a.checksum != nullptr);
+    // Flexible mode takes what the aligned 128- and 256-row kernels do not, and of their launches those whose 64-row tiles leave
+    // CUs idle, or fill them once with a short k: twice the workgroups, half the peers per workgroup, k slices that spread the epilogue as well.
+    // 128-row tiles (k slices by the library where it takes them) against this, bf16, B as [k,n] / [n,k], launches
+    // alternating: 1024x1024x1024 21.1 / 21.8 -> 17.7 / 18.3 us, 1024x4096x1024 37.5 / 40.8 -> 24.6 / 27.3, 1024x1024x4096
+    // 27.4 / 28.6 -> 19.8 / 22.4; with seven peers 512x1024x1024 36.7 / 37.4 -> 15.9 / 16.6.  With more tiles, or one per CU and
+    // a long k, the larger tile's fewer bytes per product win (2048x4096x4096: 78.5 / 78.8 against 83.6 / 108;
+    // 512x8192x8192 in two k slices 93.0 / 102.5 against 111 / 130).  (Checksums stay: a 128-row task would need two workgroups.)
+    plan.flexBlocks = 0;
+    plan.preferFlex = false;
+    const uint64_t rowsAll = op == OP_ALLGATHER ? (uint64_t)t->m * P : t->m;
+    const uint64_t tiles64 = (rowsAll + 63) / 64 * ceil_div(t->n, 256u);
+    const bool fewTiles = tiles64 <= 128u || (tiles64 <= 256u && (uint64_t)t->k * es <= 4096u);
+    const uint32_t tuning = CATCOC_FLAG_LINEAR_ORDER | CATCOC_FLAG_KEPT_WHOLE | CATCOC_FLAG_KEPT_SPLIT;
+    if (!plan.dma) {
+        plan.flexBlocks = plan_flex_slices(a, es, t->m0, d->splitK, d->workspace, d->workspaceBytes, &plan.kSlices, &plan.kSliceBytes);
+    } else if (m0 == 128 && t->m0 == 0 && d->splitK == 0 && (d->flags & tuning) == 0 && fewTiles && !transA &&
+               !(op == OP_REDUCE_SCATTER && P > 1 && a.checksum != nullptr)) {
+        // (what a workspace takes is still said for the aligned kernel; this one uses the slices that fit into that)
+        uint32_t slices;
+        uint64_t bytes;
+        plan.flexBlocks = plan_flex_slices(a, es, 0, 0, d->workspace, d->workspaceBytes, &slices, &bytes);
+        if (plan.flexBlocks != 0) plan.preferFlex = true;
+    }
     // a workspace also lets the checksum halves of tiles that run as two workgroups meet (its counter block)
     if (a.skCount == nullptr && d->workspace != nullptr && (uintptr_t)d->workspace % 256 == 0 && d->workspaceBytes >= kCounterBlockBytes)
         a.skCount = (uint32_t *)d->workspace;
@@ -375,7 +437,8 @@ void launch_float(int commType, int dataType, void *stream, uint8_t *a, uint8_t 
     p.args.b = b;
     p.args.d = c;
     if (!check_ptr_align(p, a, b)) p.variant = 0;
-    const bool dma = p.dma && p.variant != 0 && (uintptr_t)b % 16 == 0 && (p.args.ldb * 2) % 16 == 0 && (uintptr_t)c % 16 == 0;
+    const bool preferFlex = p.preferFlex && flex_ptrs_ok(p.args);
+    const bool dma = !preferFlex && p.dma && p.variant != 0 && (uintptr_t)b % 16 == 0 && (p.args.ldb * 2) % 16 == 0 && (uintptr_t)c % 16 == 0;
     if (!dma) p.args.splitK = 0;   // the other kernels run every tile whole
     if (!dma && p.variant == 4) { fail(E_TILING, "m0 = 256 needs full tiles and 16-byte aligned row-major operands"); return; }
     if (!dma && p.args.transA) p.variant = 0;
@@ -392,7 +455,7 @@ struct SplitkPlan {
     GemmArgs args;
     uint32_t f, tiles, rowBlocks;
     uint64_t workspaceBytes;   // partial tiles + counters (0 when f == 1)
-    bool general;              // shape outside the fast routes: flexible mode, or gemm_general_kernel on the 128x128 grid
+    bool general = false;      // shape outside the fast routes: flexible mode, or gemm_general_kernel on the 128x128 grid
     int flexBlocks;            // (general) as Plan::flexBlocks
     bool wholeK;               // at most 32 rows against B as [n,k]: gemm_decode_nk_kernel, no k slices, no workspace
     bool large;                // many rows: the 128x256 direct-to-LDS kernel in row-mask mode runs instead of the split-K kernel
@@ -470,12 +533,16 @@ int make_splitk_plan(const CocTilingParams *t, const CatcocSymmetricDesc *d, uin
         const uint32_t stages = d->workspaceStages ? d->workspaceStages : kDefaultStages;
         a.sched = make_sched(OP_ALLREDUCE, t->m, t->n, 1, 128, 256, cores, 1, stages, off, dir);
         a.flags |= GF_ROW_MASK;
-        sp.flexBlocks = plan_flex(a, 1, a.checksum != nullptr);
-        if (sp.flexBlocks == 0) a.sched = make_sched(OP_ALLREDUCE, t->m, t->n, 1, 128, 128, cores, 1, stages, off, dir);
-        sp.f = 1;
-        a.splitK = 0;
         sp.rowBlocks = 4;
+        // (the plan says whole tiles and no workspace, as for any launch that can do without; a workspace that is there anyway
+        // is made use of)
+        uint64_t wouldTake;
+        uint32_t wouldSlice;
+        sp.flexBlocks = plan_flex_slices(a, 1, 0, 0, d->workspace, d->workspaceBytes, &wouldSlice, &wouldTake);
+        sp.f = 1;
         sp.workspaceBytes = 0;
+        if (sp.flexBlocks == 0) a.sched = make_sched(OP_ALLREDUCE, t->m, t->n, 1, 128, 128, cores, 1, stages, off, dir);
+        a.splitK = 0;
         return 0;
     }
     if (sp.large) {
@@ -612,7 +679,8 @@ void launch_quant(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_x1, uin
     if (!check_ptr_align(p, x1, x2) || (uintptr_t)scale_x2 % 16 != 0 || (bias && (uintptr_t)bias % 16 != 0) ||
         (c_accum && (uintptr_t)c_accum % 16 != 0) || (uintptr_t)d_out % 8 != 0)
         p.variant = 0;
-    bool dma = p.dma && p.variant != 0 && (uintptr_t)x2 % 16 == 0 && p.args.ldb % 16 == 0 && (uintptr_t)d_out % 16 == 0;
+    const bool preferFlex = p.preferFlex && flex_ptrs_ok(p.args);
+    bool dma = !preferFlex && p.dma && p.variant != 0 && (uintptr_t)x2 % 16 == 0 && p.args.ldb % 16 == 0 && (uintptr_t)d_out % 16 == 0;
     for (uint32_t s = 0; s < p.args.nPeers && dma; ++s) dma = (uintptr_t)p.args.peers[s] % 16 == 0;
     if (!dma && p.variant == 4) { fail(E_TILING, "m0 = 256 needs full tiles, 16-byte aligned row-major operands and fp32 peers"); return; }
     if (!dma) p.args.splitK = 0;   // the other kernels run every tile whole
@@ -865,6 +933,7 @@ void catcoc_launch_quant_matmul_reduce_scatter_static_scratch(void *stream, uint
     d.workspaceBytes = 0;
     // how much scratch would this launch use?  Plan it first, with the sizes only.
     uint64_t need = 0;
+    bool optional = false;   // (launches in flexible mode take the k slices that fit)
     {
         CatcocSymmetricDesc q = d;
         for (int i = 0; i < CATCOC_MAX_RANKS; ++i) if (!q.peers[i]) q.peers[i] = (const void *)16;
@@ -877,8 +946,10 @@ void catcoc_launch_quant_matmul_reduce_scatter_static_scratch(void *stream, uint
             q.flags &= ~CATCOC_OUTBOUND_MASK;
             if (make_plan(QUANT_MATMUL_REDUCE_SCATTER, INT8, tiling, &q, transA, transB, p)) return;
             need = p.kSliceBytes;
+            optional = p.flexBlocks != 0;
         }
     }
+    if (optional) need = need < (uint64_t)CATCOC_STATIC_SCRATCH_BYTES ? need : (uint64_t)CATCOC_STATIC_SCRATCH_BYTES;
     if (need > (uint64_t)CATCOC_STATIC_SCRATCH_BYTES) {
         fail(E_WORKSPACE, "this launch needs %llu bytes of scratch; the built-in scratch holds %llu "
                           "(use catcoc_launch_quant_matmul_reduce_scatter with a workspace of your own)",

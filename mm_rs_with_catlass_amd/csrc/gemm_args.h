@@ -35,6 +35,7 @@ struct FlexParams {
     uint32_t rowTiles, colTiles;
     uint32_t keptTile0, keptTiles; // reduce-scatter: row tiles that hold kept rows (they start first)
     uint32_t tail;                 // bytes of k (1 .. 64) of the last k step, which goes through registers with bounds checks; 0 = none
+    uint32_t slices;               // k slices per tile (0, 1 = whole tiles)
     FastDiv dRank;                 // rows of one rank
 };
 

@@ -103,8 +103,8 @@ template <int MB, int NS> struct FlexPool
 // AQ = A is copied per pair of k steps, 128 bytes per row (whole cache lines: half as many requests to L2 as two 64-byte
 // halves), as the 256-row geometry does; for the six-stage ring, whose launches have one workgroup per CU and feel every
 // request (with three stages and two workgroups per CU the same change measured slower).
-template <uint32_t DT, int WM, bool TB, bool RM, bool RG, bool TA, int MB, int NS = 3, bool PP = false, bool AQ = false, bool W8 = false, bool FX = false>
-__device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *smem, uint32_t pos, uint32_t slice, uint32_t kSlices,
+template <uint32_t DT, int WM, bool TB, bool RM, bool RG, bool TA, int MB, int NS = 3, bool PP = false, bool AQ = false, bool W8 = false, int FX = 0>
+__device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *smem, uint32_t pos, uint32_t slice /* FX: from pos */, uint32_t kSlices,
                                          uint32_t subRow)
 {
     static_assert(!RM || (DT == DT_I8 && WM == 2), "row-mask mode exists for the W8A8 128-row kernel");
@@ -141,7 +141,14 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     TileInfo ti;
     FlexTile ft;
     if constexpr (FX) {
-        flex_tile(args, pos, ft);
+        flex_tile(args, pos, ft, slice);
+        // (uniform, but worked out with vector divisions: back into scalar registers, where the buffer descriptors want them)
+        ft.row0 = __builtin_amdgcn_readfirstlane(ft.row0);
+        ft.rowsValid = __builtin_amdgcn_readfirstlane(ft.rowsValid);
+        ft.col0 = __builtin_amdgcn_readfirstlane(ft.col0);
+        ft.colsValid = __builtin_amdgcn_readfirstlane(ft.colsValid);
+        ft.index = __builtin_amdgcn_readfirstlane(ft.index);
+        slice = __builtin_amdgcn_readfirstlane(slice);
         task = ft.index;
         ti.row = ft.row0;
         ti.col = ft.col0;
@@ -612,26 +619,44 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
                 const int tail = (int)args.fx.tail;
                 unsigned char *ta = smem + (NS - 1) * A_STAGE, *tb = smem + NS * A_STAGE + (NS - 1) * B_STAGE;
                 const size_t kEnd = (size_t)nkAll * 64;   // bytes of k in whole steps
+                constexpr int PA = A_STAGE / 16 / NT, PB = B_STAGE / 16 / NT;   // pieces of 16 bytes per thread
+                v4i pa[PA], pb[PB];
 #pragma unroll
-                for (int q = 0; q < A_STAGE / 16 / NT; ++q) {
-                    const uint32_t idx = tid + NT * q, row = idx >> 2, c = idx & 3u;
-                    const unsigned char *src = flex_row_ptr(args, ti.row + umin(row, ti.rowsValid - 1u), ldaB) + kEnd + c * 16u;
-                    *(v4i *)(ta + row * 64 + ((c ^ ((row >> 2) & 3u)) * 16)) = load16_guarded(src, tail - (int)c * 16);
+                for (int q = 0; q < PA; ++q) {
+                    const uint32_t idx = tid + NT * q, row = idx >> 2;
+                    const int c = (idx & 3u) * 16;
+                    pa[q] = load16_guarded(flex_row_ptr(args, ti.row + umin(row, ti.rowsValid - 1u), ldaB) + kEnd + c, tail - c, tail - 4 - c);
                 }
-#pragma unroll 4
-                for (int q = 0; q < B_STAGE / 16 / NT; ++q) {
+#pragma unroll
+                for (int q = 0; q < PB; ++q) {
                     const uint32_t idx = tid + NT * q;
                     const unsigned char *b = (const unsigned char *)args.b;
                     if constexpr (TB) {
-                        const uint32_t row = idx >> 2, c = idx & 3u;
-                        *(v4i *)(tb + row * 64 + ((c ^ ((row >> 2) & 3u)) * 16)) =
-                            load16_guarded(b + (size_t)(ti.col + umin(row, ti.colsValid - 1u)) * ldbB + kEnd + c * 16u, tail - (int)c * 16);
+                        const uint32_t row = idx >> 2;
+                        const int c = (idx & 3u) * 16;
+                        pb[q] = load16_guarded(b + (size_t)(ti.col + umin(row, ti.colsValid - 1u)) * ldbB + kEnd + c, tail - c, tail - 4 - c);
                     } else {
                         constexpr int CH = 256 * ES / 16;   // pieces of a row of k
+                        const int row = idx / CH, c = (idx % CH) * 16, rows = tail / ES, width = ti.colsValid * ES;
+                        pb[q] = load16_guarded(b + (kEnd / ES + (row < rows ? row : rows - 1)) * ldbB + (size_t)ti.col * ES + c,
+                                               row < rows ? width - c : 0, width - 4 - c);
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < PA; ++q) {
+                    const uint32_t idx = tid + NT * q, row = idx >> 2, c = idx & 3u;
+                    *(v4i *)(ta + row * 64 + ((c ^ ((row >> 2) & 3u)) * 16)) = pa[q];
+                }
+#pragma unroll
+                for (int q = 0; q < PB; ++q) {
+                    const uint32_t idx = tid + NT * q;
+                    if constexpr (TB) {
+                        const uint32_t row = idx >> 2, c = idx & 3u;
+                        *(v4i *)(tb + row * 64 + ((c ^ ((row >> 2) & 3u)) * 16)) = pb[q];
+                    } else {
+                        constexpr int CH = 256 * ES / 16;
                         const uint32_t row = idx / CH, c = idx % CH;
-                        const int inRow = (int)(ti.colsValid * ES) - (int)c * 16;
-                        *(v4i *)(tb + row * (256 * ES) + ((c ^ (ES == 1 ? (row & 7u) << 1 : (row & 3u) << 2)) * 16)) =
-                            load16_guarded(b + (kEnd / ES + row) * ldbB + (size_t)ti.col * ES + c * 16u, (int)row * ES < tail ? inRow : 0);
+                        *(v4i *)(tb + row * (256 * ES) + ((c ^ (ES == 1 ? (row & 7u) << 1 : (row & 3u) << 2)) * 16)) = pb[q];
                     }
                 }
                 __syncthreads();
@@ -874,6 +899,12 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
 
 #undef CATCOC_FENCE
 
+    if constexpr (FX) {
+        if constexpr (FX == 2) flex_store_partial<MB>(args, acc, smem, ft, slice);
+        else flex_epilogue<DT, MB>(args, acc, smem, ft);
+        return;
+    }
+
     // ---- k slices meet --------------------------------------------------------------
     // Every slice writes its partial tile through to memory (device-scope stores, 16 bytes per lane, the tile in
     // register order: index (((mb*4 + nb)*4 + g)*256 + thread)*4 + j holds register r = 4g + j), a per-tile counter
@@ -1014,10 +1045,6 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
         }
     }
 
-    if constexpr (FX) {
-        flex_epilogue<DT, MB>(args, acc, smem, ft);
-        return;
-    }
     // ---- epilogue -----------------------------------------------------------------
     // acc[mb][nb][r] is element (row, col) of the tile with
     //   row = wm*32*MB + mb*32 + (r>>2)*8 + h*4 + (r&3),  col = wn*128 + nb*32 + c32
@@ -1516,24 +1543,39 @@ __global__ void __launch_bounds__(128 * WM * (W8 ? 2 : 1), NS == 3 ? 2 : 1) gemm
     dma_tile<DT, WM, TB, RM, RG, TA, W8 ? 1 : 2, NS, PP, AQ, W8>(args, smem, pos, slice, kSlices, 0);
 }
 
-// Flexible mode: tiles of 64 * MB rows over the rows of all ranks (gemm_flex.h).
-template <uint32_t DT, bool TB, int MB, int NS>
+// Flexible mode: tiles of 64 * MB rows over the rows of all ranks (gemm_flex.h).  SL: k slices (a kernel of their own: either
+// ending beside the other's costs the main loop its registers, 226 of them spilled).
+template <uint32_t DT, bool TB, int MB, int NS, bool SL>
 __global__ void __launch_bounds__(256, 2) gemm_flex_kernel(const GemmArgs args)
 {
     __shared__ __attribute__((aligned(1024))) unsigned char smem[FlexPool<MB, NS>::BYTES];
-    dma_tile<DT, 2, TB, false, false, false, MB, NS, false, false, false, true>(args, smem, blockIdx.x, 0, 1, 0);
+    dma_tile<DT, 2, TB, false, false, false, MB, NS, false, false, false, SL ? 2 : 1>(args, smem, blockIdx.x, 0, SL ? args.fx.slices : 1u, 0);
+}
+
+template <uint32_t DT, bool SL>
+inline void launch_flex_tiles(const GemmArgs &args, int rowBlocks, hipStream_t s)
+{
+    const FlexParams &f = args.fx;
+    const dim3 grid(f.rowTiles * f.colTiles * (SL ? f.slices : 1u)), block(256);
+    if (rowBlocks == 1) {
+        if (args.transB) hipLaunchKernelGGL((gemm_flex_kernel<DT, true, 1, 4, SL>), grid, block, 0, s, args);
+        else hipLaunchKernelGGL((gemm_flex_kernel<DT, false, 1, 4, SL>), grid, block, 0, s, args);
+    } else {
+        if (args.transB) hipLaunchKernelGGL((gemm_flex_kernel<DT, true, 2, 3, SL>), grid, block, 0, s, args);
+        else hipLaunchKernelGGL((gemm_flex_kernel<DT, false, 2, 3, SL>), grid, block, 0, s, args);
+    }
 }
 
 template <uint32_t DT>
 inline int launch_flex(const GemmArgs &args, int rowBlocks, hipStream_t s)
 {
-    const dim3 grid(args.fx.rowTiles * args.fx.colTiles), block(256);
-    if (rowBlocks == 1) {
-        if (args.transB) hipLaunchKernelGGL((gemm_flex_kernel<DT, true, 1, 4>), grid, block, 0, s, args);
-        else hipLaunchKernelGGL((gemm_flex_kernel<DT, false, 1, 4>), grid, block, 0, s, args);
+    const FlexParams &f = args.fx;
+    if (f.slices > 1) {
+        launch_flex_tiles<DT, true>(args, rowBlocks, s);
+        const uint32_t rowsPer = 4u * ceil_div(f.rows, 4u * 65535u);   // (a row per wave; the grid's second dimension ends at 65535)
+        hipLaunchKernelGGL((flex_finish_kernel<DT>), dim3(f.colTiles, ceil_div(f.rows, rowsPer)), dim3(256), 0, s, args, rowsPer);
     } else {
-        if (args.transB) hipLaunchKernelGGL((gemm_flex_kernel<DT, true, 2, 3>), grid, block, 0, s, args);
-        else hipLaunchKernelGGL((gemm_flex_kernel<DT, false, 2, 3>), grid, block, 0, s, args);
+        launch_flex_tiles<DT, false>(args, rowBlocks, s);
     }
     return (int)hipGetLastError();
 }

@@ -56,13 +56,20 @@ CATCOC_HD uint32_t xcd_eighth(uint32_t pos, uint32_t count)
     return x * q + umin(x, r) + (pos >> 3);
 }
 
-CATCOC_HD void flex_tile(const GemmArgs &a, uint32_t pos, FlexTile &t)
+CATCOC_HD void flex_tile(const GemmArgs &a, uint32_t pos, FlexTile &t, uint32_t &slice)
 {
     const FlexParams &f = a.fx;
-    const uint32_t first = f.keptTiles * f.colTiles;
+    const uint32_t first = f.slices > 1 ? 0u : f.keptTiles * f.colTiles;
     const bool kept = pos < first;
     uint32_t seq, rows;
-    if (kept) { rows = f.keptTiles; seq = xcd_eighth(pos, first); }
+    slice = 0;
+    if (f.slices > 1) {   // an XCD takes neighbouring tiles of the same k slice: they share its rows of A; no tile is longer than another
+        const uint32_t tiles = f.rowTiles * f.colTiles;
+        seq = xcd_eighth(pos, tiles * f.slices);
+        slice = seq / tiles;
+        seq -= slice * tiles;
+        rows = f.rowTiles;
+    } else if (kept) { rows = f.keptTiles; seq = xcd_eighth(pos, first); }
     else { rows = f.rowTiles - f.keptTiles; seq = xcd_eighth(pos - first, rows * f.colTiles); }
     const uint32_t BAND = 8u;
     const uint32_t band = seq / (BAND * f.colTiles), in = seq - band * (BAND * f.colTiles);
@@ -70,7 +77,7 @@ CATCOC_HD void flex_tile(const GemmArgs &a, uint32_t pos, FlexTile &t)
     const uint32_t ct = in / w;
     uint32_t rt = band * BAND + (in - ct * w);
     if (kept) rt += f.keptTile0;
-    else if (rt >= f.keptTile0) rt += f.keptTiles;
+    else if (f.slices <= 1 && rt >= f.keptTile0) rt += f.keptTiles;
     t.row0 = flex_row_start(a, rt, t.rowsValid);
     t.col0 = ct * 256u;
     t.colsValid = umin(256u, a.N - t.col0);
@@ -103,17 +110,17 @@ __device__ __forceinline__ const unsigned char *flex_row_ptr(const GemmArgs &a, 
     return (const unsigned char *)a.a[0] + (size_t)v * ldaB;
 }
 
-// 16 bytes of which the first `valid` exist (a multiple of four, at most 16 are read; the rest read as zero); 4-byte aligned.
-typedef int v4i_u __attribute__((ext_vector_type(4), aligned(4)));
-__device__ __forceinline__ v4i load16_guarded(const unsigned char *p, int valid)
+// 16 bytes from p of which the first `valid` exist (a multiple of four; zero or less: none), the rest as zeros.  A word that
+// does not exist is read at `last` instead, the offset from p of a word of the same row that does (it may be negative): no
+// branches, so the loads of all pieces of a thread are in flight together.  4-byte aligned.
+__device__ __forceinline__ v4i load16_guarded(const unsigned char *p, int valid, int last)
 {
-    v4i v = {0, 0, 0, 0};
-    if (valid >= 16) {
-        v = *(const v4i_u *)p;
-    } else {
-        if (valid > 0) v.x = *(const int *)p;
-        if (valid > 4) v.y = *(const int *)(p + 4);
-        if (valid > 8) v.z = *(const int *)(p + 8);
+    v4i v;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const int at = 4 * d < last ? 4 * d : last;   // (last = offset from p of the last word that exists; may be negative)
+        const int x = *(const int *)(p + at);
+        v[d] = 4 * d < valid ? x : 0;
     }
     return v;
 }
@@ -183,10 +190,40 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
             if (args.bias) bv = *(const v4i *)(args.bias + gcol);
         }
     }
-    // peers: a base at the tile's first kept row, one 32-bit offset per row from there; a lane with nothing to read gets an
-    // offset behind the end of the descriptor (no memory is touched, zeros arrive)
-    const uint32_t kept0 = t.row0 > args.keptBegin ? t.row0 - args.keptBegin : 0u;
-    const uint32_t peerPitch = (uint32_t)args.peerLd * 4u;
+    // Peers: a base at the tile's first kept row, one 32-bit offset per row from there; a lane with nothing to read gets an
+    // offset behind the end of the descriptor (no memory is touched, zeros arrive).  They are fetched for 16 rows of one peer
+    // at a time (8 KiB per wave) into a ring of NBUF register buffers that runs on from one 16-row block to the next: while a
+    // block adds its last peers the next block's first ones are on their way.  The ring turns a whole number of times per
+    // block, with empty descriptors in the turns past the last peer.  (A branch per row instead of
+    // selects and out-of-range offsets, and a ring that starts anew for every block: 22.9 instead of 19.8 us at 1024x1024x4096
+    // with one peer, bf16, 31.9 instead of 25.3 on 128-row tiles.)
+    constexpr int NBUF = 3;
+    const uint32_t keptEnd = args.keptBegin + args.keptRows;
+    const uint32_t kLo = args.keptBegin > t.row0 ? umin(args.keptBegin - t.row0, t.rowsValid) : 0u;   // the tile's kept rows: [kLo, kLo + kN)
+    const uint32_t kN = keptEnd > t.row0 + kLo ? umin(keptEnd - t.row0, t.rowsValid) - kLo : 0u;
+    const int64_t kept0 = (int64_t)t.row0 + kLo - args.keptBegin;   // (of no use, and possibly negative, when the tile has none)
+    const bool tileKept = args.nPeers != 0 && kN != 0;
+    const uint32_t peerPitch = (uint32_t)args.peerLd * 4u, lastKept = colOk ? kN : 0u;
+    const uint32_t turns = (args.nPeers + NBUF - 1u) / NBUF * NBUF;
+    v4i buf[NBUF][8];
+    auto fetch = [&](v4i (&b)[8], int blk, uint32_t at) {   // turn `at` of block blk (rows wm*32*MB + 16*blk ..); past its end: of the next
+        const bool next = at >= turns;
+        const uint32_t p = next ? at - turns : at;
+        const float *base = (const float *)args.peers[umin(p, (uint32_t)kMaxRanks - 1u)] + (args.peerRowOffset + kept0) * args.peerLd;
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, p < args.nPeers ? 0x7ffffff0 : 0, 0x00020000);
+        const uint32_t row = wm * 32 * MB + (blk + (next ? 1 : 0)) * 16 + lrow - kLo;   // (wraps in front of the kept rows)
+        const uint32_t end = next && blk + 1 >= 2 * MB ? 0u : lastKept, at0 = row * peerPitch + gcol * 4u;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            b[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, row + 2 * j < end ? at0 + 2 * j * peerPitch : 0xfffffff0u, 0, 2 /* nt */);
+    };
+    if (tileKept) {
+#pragma unroll
+        for (int q = 0; q < NBUF - 1; ++q) fetch(buf[q], 0, q);
+    }
+    // the output the same way: a base at the tile's first kept row, stores of rows that are not kept behind the end
+    const uint32_t outPitch = (uint32_t)args.ldd * 2u;
+    const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc((void *)((unsigned short *)args.d + kept0 * args.ldd), 0, 0x7ffffff0, 0x00020000);
     Sum run = 0;              // of the rows of task `runOf` this lane has met since the last flush
     uint32_t runOf = 0;
 
@@ -203,9 +240,9 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
         }
 #pragma unroll
         for (int half = 0; half < 2; ++half) {   // 16 rows: a lane has eight of them, two apart
+            __builtin_amdgcn_sched_barrier(0);   // (one block's registers at a time)
             v4i cur[8];
             uint32_t d[8];
-            bool anyKept = false;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const uint32_t wrow = half * 16 + j * 2 + lrow;
@@ -213,9 +250,7 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
                 d[j] = dst[wm * 32 * MB + mb * 32 + wrow];
                 if constexpr (I8) cur[j] += bv;
                 if (!colOk) d[j] = FX_SKIP;
-                anyKept |= (d[j] & FX_KIND) == FX_KEPT;
             }
-            anyKept = __ballot(anyKept) != 0;   // (wave-uniform)
             if (args.accDump) {
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
@@ -223,27 +258,13 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
                     if (colOk && i < t.rowsValid) *(v4i *)((int32_t *)args.accDump + (size_t)(t.row0 + i) * args.N + gcol) = cur[j];
                 }
             }
-            uint32_t off[8];   // of the lane's rows in a peer's kept block
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                off[j] = (d[j] & FX_KIND) == FX_KEPT ? ((d[j] & FX_INDEX) - kept0) * peerPitch + gcol * 4u : 0xfffffff0u;
-            constexpr int NBUF = 3;
-            v4i buf[NBUF][8];
-            auto fetch = [&](v4i (&b)[8], uint32_t p) {
-                const float *base = (const float *)args.peers[umin(p, (uint32_t)kMaxRanks - 1u)] + (args.peerRowOffset + (int64_t)kept0) * args.peerLd;
-                const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, p < args.nPeers ? 0x7ffffff0 : 0, 0x00020000);
-#pragma unroll
-                for (int j = 0; j < 8; ++j) b[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, off[j], 0, 2 /* nt */);
-            };
-            auto add_peers = [&](auto add) {   // peers in slot order, two of them in flight behind the one being added
-                if (!anyKept || args.nPeers == 0) return;
-#pragma unroll
-                for (int q = 0; q < NBUF - 1; ++q) fetch(buf[q], q);
-                for (uint32_t p = 0; p < args.nPeers; p += NBUF) {
+            auto add_peers = [&](auto add) {   // in slot order
+                if (!tileKept) return;
+                for (uint32_t p = 0; p < turns; p += NBUF) {
 #pragma unroll
                     for (int q = 0; q < NBUF; ++q) {
                         __builtin_amdgcn_sched_barrier(0);
-                        fetch(buf[(q + NBUF - 1) % NBUF], p + q + NBUF - 1);
+                        fetch(buf[(q + NBUF - 1) % NBUF], 2 * mb + half, p + q + NBUF - 1);
                         __builtin_amdgcn_sched_barrier(0);
                         if (p + q < args.nPeers) {
 #pragma unroll
@@ -252,13 +273,18 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
                     }
                 }
             };
-            // (a row that is not kept adds the zeros its loads returned: nothing for int32; floats are added to kept rows only)
+            const uint32_t blockRow = wm * 32 * MB + mb * 32 + half * 16 + lrow - kLo;   // of row j = 0, counted from the tile's first kept row
+            // (32-bit on purpose: the rows in front of the first kept one wrap, and a later row of the same lane is right again)
+            auto keptRow = [&](int j) -> uint32_t { return blockRow + 2u * (uint32_t)j; };
+            auto isKept = [&](int j) { return keptRow(j) < lastKept; };
+            // (a row that is not kept adds the zeros its loads returned: nothing for int32; floats are added to kept rows only,
+            // by selects: a branch per row costs more than the additions)
             if constexpr (I8) {
                 if (redI32) add_peers([](v4i &c, const v4i &b, int) { c += b; });
                 if (args.cAccum) {
 #pragma unroll
                     for (int j = 0; j < 8; ++j)
-                        if ((d[j] & FX_KIND) == FX_KEPT) *(v4i *)(args.cAccum + (size_t)(d[j] & FX_INDEX) * args.N + gcol) = cur[j];
+                        if (isKept(j)) *(v4i *)(args.cAccum + (kept0 + (int64_t)keptRow(j)) * args.N + gcol) = cur[j];
                 }
             }
             if (!store && args.checksum) {
@@ -277,31 +303,47 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
             }
             if constexpr (I8) {   // dequantise: per-channel scale first, then per-token, each product rounded on its own
 #pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (!(redI32 && (d[j] & FX_KIND) == FX_OUT)) {   // (tiles of other ranks leave as raw int32 there)
-                        const float sM = rowScale[wm * 32 * MB + mb * 32 + half * 16 + j * 2 + lrow];
+                for (int j = 0; j < 8; ++j) {
+                    const bool raw = redI32 && !isKept(j);   // (tiles of other ranks leave as raw int32 there)
+                    const float sM = rowScale[wm * 32 * MB + mb * 32 + half * 16 + j * 2 + lrow];
 #pragma unroll
-                        for (int c = 0; c < 4; ++c) cur[j][c] = f2i(__fmul_rn(__fmul_rn((float)cur[j][c], sN[c]), sM));
+                    for (int c = 0; c < 4; ++c) {
+                        const int v = f2i(__fmul_rn(__fmul_rn((float)cur[j][c], sN[c]), sM));
+                        cur[j][c] = raw ? cur[j][c] : v;
                     }
+                }
             }
             if (!redI32)
                 add_peers([&](v4i &c, const v4i &b, int j) {
-                    if ((d[j] & FX_KIND) == FX_KEPT) {
+                    const bool k = isKept(j);
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) c[e] = f2i(__fadd_rn(i2f(c[e]), i2f(b[e])));
+                    for (int e = 0; e < 4; ++e) {
+                        const int v = f2i(__fadd_rn(i2f(c[e]), i2f(b[e])));
+                        c[e] = k ? v : c[e];
                     }
                 });
+            if (store) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const uint32_t kind = d[j] & FX_KIND, idx = d[j] & FX_INDEX;
-                if (kind == FX_KEPT) {
-                    uint32_t q[4];
+                for (int j = 0; j < 8; ++j)
+                    if ((d[j] & FX_KIND) == FX_OUT)
+                        __builtin_nontemporal_store(cur[j], (v4i *)((float *)args.outbound + (size_t)(d[j] & FX_INDEX) * args.sched.n0 + lcol));
+            }
+            if (kN != 0) {   // (wave-uniform)
+                v2i pk[8];
+                auto pack = [&](auto cvt) {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) q[e] = f32_to_out16(i2f(cur[j][e]), args.outDtype) & 0xffffu;
-                    *(v2i *)((unsigned short *)args.d + (size_t)idx * args.ldd + gcol) = v2i{(int)(q[0] | (q[1] << 16)), (int)(q[2] | (q[3] << 16))};
-                } else if (kind == FX_OUT) {
-                    __builtin_nontemporal_store(cur[j], (v4i *)((float *)args.outbound + (size_t)idx * args.sched.n0 + lcol));
-                }
+                    for (int j = 0; j < 8; ++j) {
+                        uint32_t q[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) q[e] = cvt(i2f(cur[j][e])) & 0xffffu;
+                        pk[j] = v2i{(int)(q[0] | (q[1] << 16)), (int)(q[2] | (q[3] << 16))};
+                    }
+                };
+                if (args.outDtype == DT_BF16) pack([](float f) { return f32_to_bf16_bits(f); });
+                else pack([](float f) { return f32_to_f16_bits(f); });
+                const uint32_t at0 = blockRow * outPitch + gcol * 2u;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) __builtin_amdgcn_raw_buffer_store_b64(pk[j], rd, isKept(j) ? at0 + 2 * j * outPitch : 0xfffffff0u, 0, 0);
             }
         }
     }
@@ -317,6 +359,185 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
             const uint32_t g = tid, first = g * args.sched.mRank;
             if (g < (args.fx.perRank ? 1u : 16u) && first < t.rowsValid && (dst[first] & FX_KIND) == FX_SUM) ((Sum *)args.checksum)[sumTask[g]] = sums[g];
         }
+    }
+}
+
+// ---- k slices --------------------------------------------------------------------------------------------------------------
+// Few tiles and a long k: every tile's k range is cut into slices, one workgroup each, which store their 32-bit partial sums
+// to the workspace as rows of the problem ([slice][row][n]); a second launch adds the slices in slice order and does what
+// the epilogue above does.  A second launch costs about what the in-kernel hand-over of the aligned kernels costs (write
+// through, count, fetch: a chain of memory round trips on the workgroup that arrives last), and it spreads the rest -- f
+// partials and the peers' kept rows, which at few columns outweigh the operands -- over every CU instead of one per tile.
+template <int MB, typename Acc>
+__device__ __forceinline__ void flex_store_partial(const GemmArgs &args, Acc (&acc)[MB][4], unsigned char *smem, const FlexTile &t, uint32_t slice)
+{
+    const int tid = threadIdx.x, lane = tid & 63;
+    const uint32_t w = __builtin_amdgcn_readfirstlane((uint32_t)tid >> 6);
+    const uint32_t wm = w >> 1, wn = w & 1u;
+    const int c32 = lane & 31, h = lane >> 5;
+    // checksums: the second launch adds to them row by row
+    if (slice == 0 && args.checksum != nullptr && !(args.flags & GF_OUTBOUND_STORE) && (uint32_t)tid < t.rowsValid) {
+        const uint32_t v = t.row0 + tid;
+        long long *sum = (long long *)args.checksum;   // (zero in either type)
+        if (args.flags & GF_ROW_MASK) {
+            const uint32_t cols128 = ceil_div(args.N, 128u), c = t.col0 / 128u;
+            sum[(size_t)(v / 128u) * cols128 + c] = 0;
+            if (c + 1u < cols128) sum[(size_t)(v / 128u) * cols128 + c + 1u] = 0;
+        } else if (v - args.keptBegin >= args.keptRows) {
+            uint32_t ri, task, ws;
+            const uint32_t r = fast_div(v, args.fx.dRank, ri);
+            flex_task_of(args.sched, r, ri, t.col0 / args.sched.n0, task, ws);
+            sum[task] = 0;
+        }
+    }
+    __syncthreads();   // every wave has left the main loop's LDS reads behind
+    unsigned char *st = smem + w * 16384;
+    const uint32_t lrow = lane >> 5, chunk = lane & 31, lcol = wn * 128u + chunk * 4u;
+    int32_t *part = args.skPart + ((size_t)slice * args.fx.rows + t.row0) * args.N + t.col0 + lcol;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+        if (wm * 32 * MB + mb * 32 >= t.rowsValid) continue;   // (wave-uniform)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const uint32_t wrow = (r >> 2) * 8 + h * 4 + (r & 3);
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) {
+                const auto e = acc[mb][nb][r];
+                *(int *)(st + wrow * 512 + (((nb * 32 + c32) * 4) ^ (h << 7))) = __builtin_bit_cast(int, e);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const uint32_t wrow = j * 2 + lrow, i = wm * 32 * MB + mb * 32 + wrow;
+            const v4i v = *(const v4i *)(st + wrow * 512 + ((chunk * 16) ^ (((wrow >> 2) & 1) << 7)));
+            if (i < t.rowsValid && lcol < t.colsValid) *(v4i *)(part + (size_t)i * args.N) = v;
+        }
+    }
+}
+
+__device__ __forceinline__ void add_sum(unsigned long long *to, unsigned long long v) { atomicAdd(to, v); }
+__device__ __forceinline__ void add_sum(double *to, double v) { unsafeAtomicAdd(to, v); }
+
+// Workgroup (ct, y): columns [256 ct, +256) of rows [rowsPer * y, +rowsPer).  A wave takes one row at a time (everything about
+// the row is wave-uniform), a lane four columns of it: partials and peers are 1 KiB per wave instruction, all of them
+// requested before the first is used.
+template <uint32_t DT>
+__global__ void __launch_bounds__(256) flex_finish_kernel(const GemmArgs args, const uint32_t rowsPer)
+{
+    constexpr bool I8 = DT == DT_I8;
+    using Sum = typename std::conditional<I8, unsigned long long, double>::type;
+    const int lane = threadIdx.x & 63;
+    const uint32_t w = __builtin_amdgcn_readfirstlane((uint32_t)threadIdx.x >> 6);
+    const bool redI32 = I8 && (args.flags & GF_REDUCE_INT32) != 0;
+    const bool store = (args.flags & GF_OUTBOUND_STORE) != 0, rowMask = (args.flags & GF_ROW_MASK) != 0;
+    const bool sums = !store && args.checksum != nullptr;
+    const uint32_t row0 = blockIdx.y * rowsPer, rowEnd = umin(row0 + rowsPer, args.fx.rows);
+    const uint32_t lcol = lane * 4u, gcol = blockIdx.x * 256u + lcol;
+    const bool colOk = gcol < args.N;
+    const uint32_t slices = args.fx.slices;
+    v4f sN = {1.f, 1.f, 1.f, 1.f};
+    v4i bv = {0, 0, 0, 0};
+    if constexpr (I8) {
+        if (colOk) {
+            sN = *(const v4f *)(args.scaleN + gcol);
+            if (args.bias) bv = *(const v4i *)(args.bias + gcol);
+        }
+    }
+    for (uint32_t v = row0 + w; v < rowEnd; v += 4u) {
+        const bool kept = v - args.keptBegin < args.keptRows;
+        // the peers first: they do not wait for the sums
+        const uint32_t nP = kept ? args.nPeers : 0u;
+        const size_t peerAt = kept ? (size_t)(args.peerRowOffset + (v - args.keptBegin)) * args.peerLd + gcol : 0;
+        v4i pv[8], cur = {0, 0, 0, 0};
+        if (colOk) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                if ((uint32_t)q < nP) pv[q] = __builtin_nontemporal_load((const v4i *)((const int *)args.peers[q] + peerAt));
+            const int32_t *part = args.skPart + (size_t)v * args.N + gcol;
+            const size_t pitch = (size_t)args.fx.rows * args.N;
+            for (uint32_t s0 = 0; s0 < slices; s0 += 8u) {
+                v4i t[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    if (s0 + q < slices) t[q] = *(const v4i *)(part + (s0 + q) * pitch);
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    if (s0 + q < slices) {
+                        if constexpr (I8) {
+                            cur += t[q];
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) cur[e] = f2i(__fadd_rn(i2f(cur[e]), i2f(t[q][e])));
+                        }
+                    }
+            }
+            if constexpr (I8) cur += bv;
+            if (args.accDump) *(v4i *)((int32_t *)args.accDump + (size_t)v * args.N + gcol) = cur;
+        }
+        if (!kept) {
+            uint32_t ws = 0, task = 0;
+            if (!rowMask) {
+                uint32_t ri;
+                const uint32_t r = fast_div(v, args.fx.dRank, ri);
+                flex_task_of(args.sched, r, ri, blockIdx.x * 256u / args.sched.n0, task, ws);
+            }
+            if (sums) {
+                Sum s = 0;
+                if (colOk) {
+                    if constexpr (I8) s = (Sum)(((long long)cur.x + cur.y) + ((long long)cur.z + cur.w));
+                    else s = ((double)i2f(cur.x) + (double)i2f(cur.y)) + ((double)i2f(cur.z) + (double)i2f(cur.w));
+                }
+#pragma unroll
+                for (int o = 16; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+                Sum *to = (Sum *)args.checksum;
+                if (rowMask) {   // one sum per 128 columns
+                    if ((lane & 31) == 0 && colOk) add_sum(to + (size_t)(v / 128u) * ceil_div(args.N, 128u) + gcol / 128u, s);
+                } else {
+                    s += __shfl_xor(s, 32, 64);
+                    if (lane == 0) add_sum(to + task, s);
+                }
+            }
+            if (store && colOk) {
+                if constexpr (I8) {
+                    if (!redI32) {
+                        const float sM = args.scaleM[v];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) cur[e] = f2i(__fmul_rn(__fmul_rn((float)cur[e], sN[e]), sM));
+                    }
+                }
+                __builtin_nontemporal_store(cur, (v4i *)((float *)args.outbound + (size_t)ws * args.sched.n0 + lcol));
+            }
+            continue;
+        }
+        if (!colOk) continue;
+        auto addPeers = [&](auto add) {
+            for (uint32_t p0 = 0; p0 < nP; p0 += 8u) {
+                if (p0) {
+#pragma unroll
+                    for (int q = 0; q < 8; ++q)
+                        if (p0 + q < nP) pv[q] = __builtin_nontemporal_load((const v4i *)((const int *)args.peers[p0 + q] + peerAt));
+                }
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    if (p0 + q < nP) add(pv[q]);
+            }
+        };
+        if constexpr (I8) {
+            if (redI32) addPeers([&](const v4i &b) { cur += b; });
+            if (args.cAccum) *(v4i *)(args.cAccum + (size_t)(v - args.keptBegin) * args.N + gcol) = cur;
+            const float sM = args.scaleM[v];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) cur[e] = f2i(__fmul_rn(__fmul_rn((float)cur[e], sN[e]), sM));
+        }
+        if (!redI32)
+            addPeers([&](const v4i &b) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) cur[e] = f2i(__fadd_rn(i2f(cur[e]), i2f(b[e])));
+            });
+        uint32_t q[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[e] = f32_to_out16(i2f(cur[e]), args.outDtype) & 0xffffu;
+        *(v2i *)((unsigned short *)args.d + (size_t)(v - args.keptBegin) * args.ldd + gcol) = v2i{(int)(q[0] | (q[1] << 16)), (int)(q[2] | (q[3] << 16))};
     }
 }
 

@@ -15,6 +15,17 @@ from test_gpu_parity import TORCH_DT, _check_float, _need_gpu, _rand16, dev, dev
 pytestmark = pytest.mark.gpu
 
 
+def peers_of(rng, M, N, K, P, rank, ri):
+    """The peers quant_case draws from the same generator (after operands, scales and bias)."""
+    rng.integers(-127, 128, (M, K), dtype=np.int8)
+    rng.integers(-127, 128, (K, N), dtype=np.int8)
+    rng.uniform(0.005, 0.02, M), rng.uniform(0.001, 0.01, N), rng.integers(-1000, 1000, N, dtype=np.int32)
+    rows = M // P
+    if ri:
+        return [rng.integers(-2 ** 24, 2 ** 24, (rows, N), dtype=np.int32) for _ in range(P - 1)]
+    return [rng.standard_normal((rows, N)).astype(np.float32) for _ in range(P - 1)]
+
+
 # (rows per rank, N, K, P, rank, weights as [n,k], int32 peers, m0, commInterval)
 @pytest.mark.parametrize("outbound", [False, True])
 @pytest.mark.parametrize("case", [(125, 512, 1376, 8, 5, True, False, 0, 1),     # one rank per tile; half a step of k left
@@ -33,6 +44,23 @@ def test_quant_rs_any_rows_any_k(case, outbound):
     r = quant_case(np.random.default_rng(rows), M, N, K, P, rank, bias=True, trans_b=tb, reduce_int32=ri, tiling=t, outbound=outbound,
                    launches=2, block_num=bn)
     assert r["exact"] == r["total"]
+    # the same in k slices (a second launch adds them up); the counter block of the workspace stays zero
+    if K >= 128:
+        g = lambda a: None if a is None else dev(a)
+        ws = torch.zeros(65536 + 3 * M * N * 4, dtype=torch.uint8, device="cuda:0")
+        ws[65536:] = 0x55
+        peers = peers_of(np.random.default_rng(rows), M, N, K, P, rank, ri)
+        kw = {"outbound": torch.zeros_like(r["outbound"])} if outbound else {"checksum": torch.full_like(r["checksum"], 77)}
+        out = ops.quant_matmul_reduce_scatter(dev(r["x1"]), dev(np.ascontiguousarray(r["x2"].T) if tb else r["x2"]), dev(r["s1"]), dev(r["s2"]),
+                                              g(r["bias"]), [dev(p) for p in peers], rank, P, tiling=t, trans_b=tb, reduce_int32=ri,
+                                              block_num=bn, workspace=ws, split_k=3, **kw)
+        torch.cuda.synchronize()
+        assert np.array_equal(host16(out), r["out_want"]) and not ws[:65536].any() and bool((ws[65536:] != 0x55).any())
+        if outbound:
+            assert torch.equal(kw["outbound"].view(torch.int32), r["outbound"].view(torch.int32))
+        else:
+            others = r["checksum"] != 0
+            assert torch.equal(kw["checksum"][others], r["checksum"][others])
     d = L.make_desc(rank, P, [16] * (P - 1), block_num=bn)
     tr, row, col, ws = (C.c_uint32() for _ in range(4))
     step = m0 or (64 if rows <= 64 else 128)
@@ -79,6 +107,18 @@ def test_float_any_rows_any_k(dtype, case):
         torch.cuda.synchronize()
     _check_float(host16(out), want, full, dtype, K)
     assert out.dtype == TORCH_DT[dtype]
+    if K >= 512:   # in k slices: added in slice order, so twice the same bits
+        ws = torch.zeros(65536 + 5 * out.numel() * 4, dtype=torch.uint8, device="cuda:0")
+        again = []
+        for _ in range(2):
+            if op == "allgather":
+                o = ops.allgather_matmul(ds[rank], ds[:rank], Bd, rank, P, trans_b=tb, workspace=ws, split_k=5)
+            else:
+                o = ops.matmul_allreduce(dev16(A, dtype), Bd, [dev(p) for p in peers], rank, P, trans_b=tb, workspace=ws, split_k=5)
+            torch.cuda.synchronize()
+            again.append(host16(o))
+        assert np.array_equal(again[0], again[1])
+        _check_float(again[0], want, full, dtype, K)
     # fp32 sums of K products in another order: each within K * 2^-24 of the sum of their magnitudes, here at most
     # 4.5 * 4.5 * 0.02 * K per element (operands are normal, scales 1 and 0.02)
     assert np.abs(dump.cpu().numpy() - part).max() <= K * 2.0 ** -24 * 0.41 * K + 1e-6
