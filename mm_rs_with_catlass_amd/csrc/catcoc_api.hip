@@ -169,16 +169,23 @@ int plan_flex_slices(GemmArgs &a, uint32_t es, uint32_t wantM0, uint32_t wantSli
     *slices = 1;
     *bytes = 0;
     if (whole == 0) return 0;
-    const uint32_t steps = (uint32_t)(((uint64_t)a.K * es - a.fx.tail) / 64u);
-    const uint32_t f = umin(umin(wantSlices ? wantSlices : flex_slices(a.fx.rows, a.N, ceil_div(a.fx.rows, 64u) * a.fx.colTiles, steps), 64u), steps);
+    const uint32_t steps = (uint32_t)(((uint64_t)a.K * es - a.fx.tail) / 64u), tiles = ceil_div(a.fx.rows, 64u) * a.fx.colTiles;
+    // explicit kept rows: the other rows need no partial sums of their own (the dump, if there is one, does)
+    const bool keptOnly = (a.flags & GF_ROW_MASK) != 0 && a.accDump == nullptr;
+    const uint32_t stored = keptOnly ? a.keptRows : a.fx.rows;
+    const uint32_t f = umin(umin(wantSlices ? wantSlices : flex_slices(stored, a.N, tiles, steps), 64u), steps);
     if (f <= 1) return whole;
-    const uint64_t slice = (uint64_t)a.fx.rows * a.N * 4u;
+    const uint64_t sumBytes = keptOnly && sums ? (uint64_t)ceil_div(a.fx.rows, 128u) * ceil_div(a.N, 128u) * 16u : 0u;   // per slice
+    const uint64_t slice = ((uint64_t)stored * a.N * 4u + sumBytes + 15u) / 16u * 16u;
     *slices = f;
     *bytes = kCounterBlockBytes + f * slice;
     if (workspace == nullptr || (uintptr_t)workspace % 256 != 0 || workspaceBytes < kCounterBlockBytes + 2u * slice) return whole;
     const uint64_t fit = (workspaceBytes - kCounterBlockBytes) / slice;
-    a.skPart = (int32_t *)((unsigned char *)workspace + kCounterBlockBytes);
-    return plan_flex(a, es, sums, wantM0, fit < f ? (uint32_t)fit : f);
+    const uint32_t run = fit < f ? (uint32_t)fit : f;
+    a.fx.keptOnly = keptOnly ? 1u : 0u;
+    a.fx.sliceSums = (long long *)((unsigned char *)workspace + kCounterBlockBytes);
+    a.skPart = (int32_t *)((unsigned char *)workspace + kCounterBlockBytes + run * sumBytes);
+    return plan_flex(a, es, sums, wantM0, run);
 }
 
 // What flexible mode asks of the pointers: operands on the 4-byte grid, everything the epilogue touches in its 8- and 16-byte
@@ -457,6 +464,7 @@ struct SplitkPlan {
     uint64_t workspaceBytes;   // partial tiles + counters (0 when f == 1)
     bool general = false;      // shape outside the fast routes: flexible mode, or gemm_general_kernel on the 128x128 grid
     int flexBlocks;            // (general) as Plan::flexBlocks
+    bool preferFlex;           // sliced row tiles (flexible mode) run although the streaming kernels would take the launch
     bool wholeK;               // at most 32 rows against B as [n,k]: gemm_decode_nk_kernel, no k slices, no workspace
     bool large;                // many rows: the 128x256 direct-to-LDS kernel in row-mask mode runs instead of the split-K kernel
 };
@@ -484,6 +492,7 @@ int make_splitk_plan(const CocTilingParams *t, const CatcocSymmetricDesc *d, uin
     // one-thread-per-element kernel on the same 128x128 grid: a correctness path, whole tiles, no workspace
     sp.general = t->k % 64 != 0 || t->n % 128 != 0;
     sp.wholeK = false;
+    sp.preferFlex = false;
     const bool canLarge = !sp.general && t->m % 128 == 0 && t->n % 256 == 0 && d->keptRowBegin % 32 == 0 && d->keptRows % 32 == 0;
     const bool wantLarge = t->n0 == 256 && (t->m0 == 0 || t->m0 == 128);
     if (wantLarge && !canLarge)
@@ -544,6 +553,22 @@ int make_splitk_plan(const CocTilingParams *t, const CatcocSymmetricDesc *d, uin
         if (sp.flexBlocks == 0) a.sched = make_sched(OP_ALLREDUCE, t->m, t->n, 1, 128, 128, cores, 1, stages, off, dir);
         a.splitK = 0;
         return 0;
+    }
+    // Flexible mode (gemm_flex.h) where its 64-row tiles in k slices beat the streaming kernels: those hand a tile's slices and
+    // all its peers to one workgroup, the flexible launch spreads both over every CU, and of rows that are not kept it stores no
+    // partial sums.  Streaming kernels -> this, W8A8, seven peers, all rows kept unless said, launches alternating, us:
+    // 203x1792x4096 37.9 -> 18.5, 128x8192x1024 46.3 -> 15.0, 512x1024x1024 29.0 -> 14.1, 64x8192x8192 30.1 -> 24.5 (8 rows kept
+    // 22.7 -> 19.9), 203x8192x8192 56.6 -> 40.1, 16x8192x2048 with 2 rows kept 16.1 -> 13.1.  The other way round:
+    //  - weights of more than 64 MiB stream better through the deep rings of those kernels (64x16384x8192 42.0 / 43.5, as [n,k]
+    //    44.8 / 53.8; 388x15744x5376 94 / 111);
+    //  - at most 32 rows with a k that leaves nothing to slice, or little to win: a second launch costs 1 us (17x576x896 10.0 / 11.2,
+    //    8x1024x8192 10.4 / 10.1, 2x8192x8192 with one row kept, [n,k], 18.2 / 19.3);
+    //  - many rows in full tiles, few of them kept: the 128x256 tile's fewer bytes per product (512x8192x8192 with 64 rows kept
+    //    50 / 65, 512x4096x8192 with 256 rows kept 35 / 40, 256x8192x8192 and one peer 43.4 / 45.5).
+    if (t->m0 == 0 && t->n0 == 0 && d->splitK == 0 && d->blockNum == 0) {
+        const uint64_t weights = (uint64_t)t->k * t->n, work64 = (uint64_t)ceil_div(t->m, 64u) * ceil_div(t->n, 256u) * t->k;
+        sp.preferFlex = t->m <= 32 ? t->k >= 4096 && weights <= (32ull << 20)
+                                   : weights <= (64ull << 20) && (!sp.large || work64 <= 128u * 4096u || (d->keptRows == t->m && P > 2));
     }
     if (sp.large) {
         // one grid of 128x256 tiles over all of A's rows (no rank structure), k slices as for any few-tile launch
@@ -641,15 +666,36 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
     a.bias = (const int32_t *)bias;
     a.cAccum = (int32_t *)c_accum;
     a.outDtype = outDataType;
+    // The plan above says what the launch is refused for and what it asks of the workspace, whichever kernel runs.
+    const auto flex = [&]() {
+        if (!sp.preferFlex) return false;
+        GemmArgs g = a;
+        const uint32_t stages = d->workspaceStages ? d->workspaceStages : kDefaultStages;
+        g.sched = make_sched(OP_ALLREDUCE, a.M, a.N, 1, 128, 256, kDefaultBlockNum, 1, stages, a.sched.off, a.sched.dir);
+        g.flags |= GF_ROW_MASK;
+        g.splitK = 0;
+        g.skCount = nullptr;
+        uint32_t wouldSlice;
+        uint64_t wouldTake;
+        const int blocks = plan_flex_slices(g, 1, 0, 0, d->workspace, d->workspaceBytes, &wouldSlice, &wouldTake);
+        // (without the slices it would take, only where the streaming kernels run whole tiles as well)
+        if (blocks == 0 || (wouldSlice > 1 && g.fx.slices < 2 && (sp.large || sp.f > 1)) || !flex_ptrs_ok(g)) return false;
+        const int e = launch_flex(DT_I8, g, blocks, stream);
+        if (e) fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)e));
+        else ok();
+        return true;
+    };
     if (sp.large) {
         bool aligned = (uintptr_t)scale_x2 % 16 == 0 && (uintptr_t)d_out % 16 == 0 && (!bias || (uintptr_t)bias % 16 == 0) && a.peerLd % 4 == 0;
         for (uint32_t s = 0; s < a.nPeers && aligned; ++s) aligned = (uintptr_t)a.peers[s] % 16 == 0;
         if (!aligned) { fail(E_SHAPE, "128x256 tiles with explicit kept rows need 16-byte aligned scales, bias, peers and output"); return; }
+        if (flex()) return;
         const int el = launch_gemm_dma_i8(a, stream);
         if (el) { fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)el)); return; }
         ok();
         return;
     }
+    if (!sp.wholeK && flex()) return;
     const int e = sp.wholeK ? launch_gemm_decode_nk_i8(a, stream) : launch_gemm_splitk_i8(a, (int)sp.rowBlocks, sp.tiles * sp.f, stream);
     if (e) { fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)e)); return; }
     ok();

@@ -36,6 +36,8 @@ struct FlexParams {
     uint32_t keptTile0, keptTiles; // reduce-scatter: row tiles that hold kept rows (they start first)
     uint32_t tail;                 // bytes of k (1 .. 64) of the last k step, which goes through registers with bounds checks; 0 = none
     uint32_t slices;               // k slices per tile (0, 1 = whole tiles)
+    uint32_t keptOnly;             // k slices, explicit kept rows: partial sums of the kept rows only, the other rows as one sum per
+    long long *sliceSums;          // 64 x 128 block and slice: [128 x 128 block][slice][upper / lower 64 rows]
     FastDiv dRank;                 // rows of one rank
 };
 

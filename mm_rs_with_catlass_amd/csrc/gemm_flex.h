@@ -362,12 +362,35 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
     }
 }
 
+// Sum over the 64 lanes of a wave, in lane 63: cross-lane adds in the vector unit (a shuffle is a trip through the LDS unit).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ long long dpp_add64(long long v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), CTRL, ROWS, 0xf, false);
+    return v + (long long)(((unsigned long long)(uint32_t)hi << 32) | (uint32_t)lo);
+}
+__device__ __forceinline__ long long wave_sum64(long long v)
+{
+    v = dpp_add64<0x111, 0xf>(v);   // row_shr:1, 2, 4, 8: lane 15 of every row of 16 holds the row's sum
+    v = dpp_add64<0x112, 0xf>(v);
+    v = dpp_add64<0x114, 0xf>(v);
+    v = dpp_add64<0x118, 0xf>(v);
+    v = dpp_add64<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+    v = dpp_add64<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
 // ---- k slices --------------------------------------------------------------------------------------------------------------
 // Few tiles and a long k: every tile's k range is cut into slices, one workgroup each, which store their 32-bit partial sums
 // to the workspace as rows of the problem ([slice][row][n]); a second launch adds the slices in slice order and does what
 // the epilogue above does.  A second launch costs about what the in-kernel hand-over of the aligned kernels costs (write
 // through, count, fetch: a chain of memory round trips on the workgroup that arrives last), and it spreads the rest -- f
 // partials and the peers' kept rows, which at few columns outweigh the operands -- over every CU instead of one per tile.
+// Explicit kept rows (keptOnly): only they have partial sums in the workspace; what the others add to their checksums is summed
+// in registers and leaves as one number per 64 x 128 block and slice.  (With partial sums of all rows and an atomic add per row
+// of 128 sums in the second launch 203x1792x4096 with 26 kept rows took 22.0 us instead of 13.7, 128x1024x8192 with 16 27.1
+// instead of 12.6.)
 template <int MB, typename Acc>
 __device__ __forceinline__ void flex_store_partial(const GemmArgs &args, Acc (&acc)[MB][4], unsigned char *smem, const FlexTile &t, uint32_t slice)
 {
@@ -375,8 +398,46 @@ __device__ __forceinline__ void flex_store_partial(const GemmArgs &args, Acc (&a
     const uint32_t w = __builtin_amdgcn_readfirstlane((uint32_t)tid >> 6);
     const uint32_t wm = w >> 1, wn = w & 1u;
     const int c32 = lane & 31, h = lane >> 5;
+    uint32_t kLo = 0, kHi = t.rowsValid;   // the tile's rows whose partial sums are stored
+    if constexpr (std::is_same<Acc, v16i>::value) {
+        if (args.fx.keptOnly) {
+            const uint32_t end = t.row0 + t.rowsValid;
+            kLo = args.keptBegin > t.row0 ? umin(args.keptBegin - t.row0, t.rowsValid) : 0u;
+            kHi = umin(args.keptBegin + args.keptRows, end) - umin(t.row0, umin(args.keptBegin + args.keptRows, end));
+            if (args.checksum) {   // the other rows leave as one sum per 64 x 128 block
+                const uint32_t col = wn * 128u + c32, cols128 = ceil_div(args.N, 128u), c = t.col0 / 128u + wn;
+                long long sum = 0;
+                uint32_t others = 0;   // rows of this lane that are not kept
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const uint32_t row = wm * 32 * MB + mb * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
+                        const bool other = row < t.rowsValid && !(row >= kLo && row < kHi);
+                        others += other ? 1u : 0u;
+#pragma unroll
+                        for (int nb = 0; nb < 4; ++nb) sum += other && col + nb * 32 < t.colsValid ? (long long)acc[mb][nb][r] : 0ll;
+                    }
+                if (slice == 0 && args.bias) {
+#pragma unroll
+                    for (int nb = 0; nb < 4; ++nb)
+                        if (col + nb * 32 < t.colsValid) sum += (long long)args.bias[t.col0 + col + nb * 32] * others;
+                }
+                sum = wave_sum64(sum);
+                long long *sums = (long long *)(smem + FLEX_STAGING);
+                __syncthreads();   // (every wave has left the main loop's LDS reads behind)
+                if (lane == 63) sums[w] = sum;
+                __syncthreads();
+                if (wm == 0 && lane == 0 && c < cols128) {
+                    long long *to = args.fx.sliceSums + ((size_t)(t.row0 / 128u) * cols128 + c) * 2u * args.fx.slices + 2u * slice;
+                    to[(t.row0 / 64u) & 1u] = sums[wn] + sums[2 + wn];
+                }
+            }
+            if (kLo >= kHi) return;
+        }
+    }
     // checksums: the second launch adds to them row by row
-    if (slice == 0 && args.checksum != nullptr && !(args.flags & GF_OUTBOUND_STORE) && (uint32_t)tid < t.rowsValid) {
+    if (!args.fx.keptOnly && slice == 0 && args.checksum != nullptr && !(args.flags & GF_OUTBOUND_STORE) && (uint32_t)tid < t.rowsValid) {
         const uint32_t v = t.row0 + tid;
         long long *sum = (long long *)args.checksum;   // (zero in either type)
         if (args.flags & GF_ROW_MASK) {
@@ -393,10 +454,12 @@ __device__ __forceinline__ void flex_store_partial(const GemmArgs &args, Acc (&a
     __syncthreads();   // every wave has left the main loop's LDS reads behind
     unsigned char *st = smem + w * 16384;
     const uint32_t lrow = lane >> 5, chunk = lane & 31, lcol = wn * 128u + chunk * 4u;
-    int32_t *part = args.skPart + ((size_t)slice * args.fx.rows + t.row0) * args.N + t.col0 + lcol;
+    // (signed: the tile's first row may lie in front of the kept ones, which alone are stored)
+    const int64_t row0 = args.fx.keptOnly ? (int64_t)slice * args.keptRows + t.row0 - args.keptBegin : (int64_t)slice * args.fx.rows + t.row0;
+    int32_t *part = args.skPart + row0 * args.N + t.col0 + lcol;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
-        if (wm * 32 * MB + mb * 32 >= t.rowsValid) continue;   // (wave-uniform)
+        if (wm * 32 * MB + mb * 32 >= kHi || wm * 32 * MB + mb * 32 + 32 <= kLo) continue;   // (wave-uniform)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const uint32_t wrow = (r >> 2) * 8 + h * 4 + (r & 3);
@@ -410,7 +473,7 @@ __device__ __forceinline__ void flex_store_partial(const GemmArgs &args, Acc (&a
         for (int j = 0; j < 16; ++j) {
             const uint32_t wrow = j * 2 + lrow, i = wm * 32 * MB + mb * 32 + wrow;
             const v4i v = *(const v4i *)(st + wrow * 512 + ((chunk * 16) ^ (((wrow >> 2) & 1) << 7)));
-            if (i < t.rowsValid && lcol < t.colsValid) *(v4i *)(part + (size_t)i * args.N) = v;
+            if (i >= kLo && i < kHi && lcol < t.colsValid) *(v4i *)(part + (size_t)i * args.N) = v;
         }
     }
 }
@@ -431,7 +494,9 @@ __global__ void __launch_bounds__(256) flex_finish_kernel(const GemmArgs args, c
     const bool redI32 = I8 && (args.flags & GF_REDUCE_INT32) != 0;
     const bool store = (args.flags & GF_OUTBOUND_STORE) != 0, rowMask = (args.flags & GF_ROW_MASK) != 0;
     const bool sums = !store && args.checksum != nullptr;
-    const uint32_t row0 = blockIdx.y * rowsPer, rowEnd = umin(row0 + rowsPer, args.fx.rows);
+    const bool keptOnly = I8 && args.fx.keptOnly != 0;
+    const uint32_t first = keptOnly ? args.keptBegin : 0u, stored = keptOnly ? args.keptRows : args.fx.rows;   // the rows the partial sums hold
+    const uint32_t row0 = first + blockIdx.y * rowsPer, rowEnd = umin(row0 + rowsPer, first + stored);
     const uint32_t lcol = lane * 4u, gcol = blockIdx.x * 256u + lcol;
     const bool colOk = gcol < args.N;
     const uint32_t slices = args.fx.slices;
@@ -441,6 +506,22 @@ __global__ void __launch_bounds__(256) flex_finish_kernel(const GemmArgs args, c
         if (colOk) {
             sN = *(const v4f *)(args.scaleN + gcol);
             if (args.bias) bv = *(const v4i *)(args.bias + gcol);
+        }
+    }
+    if constexpr (I8) {
+        if (keptOnly && args.checksum) {   // a wave per 128 x 128 block of this column tile
+            const uint32_t cols128 = ceil_div(args.N, 128u), blocks = ceil_div(args.fx.rows, 128u) * 2u;
+            for (uint32_t e = blockIdx.y * 4u + (w ^ 3u); e < blocks; e += gridDim.y * 4u) {   // (few rows: they are the first waves')
+                const uint32_t rb = e >> 1, c = blockIdx.x * 2u + (e & 1u);
+                if (c >= cols128) continue;
+                const long long *from = args.fx.sliceSums + ((size_t)rb * cols128 + c) * 2u * slices;
+                const bool both = rb * 128u + 64u < args.fx.rows;   // (the last block may have no lower half)
+                long long s = 0;
+                for (uint32_t i = lane; i < 2u * slices; i += 64u)
+                    if (both || (i & 1u) == 0) s += from[i];
+                s = wave_sum64(s);
+                if (lane == 63) ((long long *)args.checksum)[(size_t)rb * cols128 + c] = s;
+            }
         }
     }
     for (uint32_t v = row0 + w; v < rowEnd; v += 4u) {
@@ -453,8 +534,8 @@ __global__ void __launch_bounds__(256) flex_finish_kernel(const GemmArgs args, c
 #pragma unroll
             for (int q = 0; q < 8; ++q)
                 if ((uint32_t)q < nP) pv[q] = __builtin_nontemporal_load((const v4i *)((const int *)args.peers[q] + peerAt));
-            const int32_t *part = args.skPart + (size_t)v * args.N + gcol;
-            const size_t pitch = (size_t)args.fx.rows * args.N;
+            const int32_t *part = args.skPart + (size_t)(v - first) * args.N + gcol;
+            const size_t pitch = (size_t)stored * args.N;
             for (uint32_t s0 = 0; s0 < slices; s0 += 8u) {
                 v4i t[8];
 #pragma unroll

@@ -146,3 +146,36 @@ def test_float_reduce_scatter_checksums_of_small_ranks(dtype):
         # (fp32 accumulation in another order: K * 2^-24 of the magnitudes per element, as above)
         bound = blk.size * K * 2.0 ** -24 * 0.41 * K + 1e-6
         assert abs(float(cs[task]) - (0.0 if tr.value == rank else blk.sum())) <= bound, task
+
+
+# (m, N, K, P, kept rows [begin, +count), weights as [n,k], int32 peers): kept rows that start, end or lie inside a 64-row tile,
+# a last row tile and a last 128-column block of their own, at most 32 rows with a long k, every row kept
+@pytest.mark.parametrize("case", [(65, 384, 512, 4, 63, 2, False, False), (130, 1152, 1024, 8, 60, 11, True, True), (200, 256, 448, 2, 64, 64, False, False),
+                                  (511, 640, 1792, 8, 510, 1, True, False), (5, 128, 4096, 8, 1, 2, False, True), (32, 512, 8192, 1, 0, 4, False, False),
+                                  (33, 128, 192, 2, 0, 33, True, False), (256, 512, 2048, 8, 0, 256, False, True), (384, 1024, 512, 4, 32, 96, True, False)])
+def test_quant_kept_rows_in_slices(case):
+    """Explicit kept rows in k slices: partial sums of the kept rows only, the other rows as sums per slice."""
+    _need_gpu()
+    M, N, K, P, kb, kr, tb, ri = case
+    rng = np.random.default_rng(M + N)
+    x1, x2 = rng.integers(-127, 128, (M, K), dtype=np.int8), rng.integers(-127, 128, (K, N), dtype=np.int8)
+    s1, s2 = rng.uniform(0.005, 0.02, M).astype(np.float32), rng.uniform(0.001, 0.01, N).astype(np.float32)
+    b = rng.integers(-1000, 1000, N, dtype=np.int32)
+    peers = [rng.integers(-2 ** 24, 2 ** 24, (kr, N), dtype=np.int32) if ri else rng.standard_normal((kr, N)).astype(np.float32) for _ in range(P - 1)]
+    acc, want = oracle.quant_matmul_reduce_scatter(x1, x2, s1, s2, b, kb, kr, peers, oracle.BF16, reduce_int32=ri)
+    need, _, tiles = ops.splitk_plan(M, K, N, P, kb, kr)
+    sums = np.array([[acc[r:r + 128, c:c + 128].astype(np.int64).sum() - acc[max(r, kb):max(min(r + 128, kb + kr), max(r, kb)), c:c + 128].astype(np.int64).sum()
+                      for c in range(0, N, 128)] for r in range(0, M, 128)]).ravel()
+    x2d = dev(np.ascontiguousarray(x2.T) if tb else x2)
+    for extra in (0, 1 << 20):   # as many slices as the query's workspace holds, and more
+        ws = torch.zeros(max(need, 65536) + extra, dtype=torch.uint8, device="cuda:0")
+        ws[65536:] = 0x55
+        cs = torch.full((tiles,), -7, dtype=torch.int64, device="cuda:0") if kr < M else None
+        ca = torch.full((kr, N), -7, dtype=torch.int32, device="cuda:0")
+        out = ops.quant_matmul_splitk(dev(x1), x2d, dev(s1), dev(s2), dev(b), [dev(p) for p in peers], P, kb, kr, workspace=ws, checksum=cs,
+                                      c_accum=ca, trans_b=tb, reduce_int32=ri)
+        torch.cuda.synchronize()
+        assert np.array_equal(host16(out), want) and not ws[:65536].any()
+        assert np.array_equal(ca.cpu().numpy(), acc[kb:kb + kr] + (sum(peers) if ri else 0))
+        if cs is not None:
+            assert np.array_equal(cs.cpu().numpy(), sums)
