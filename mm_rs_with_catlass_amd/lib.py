@@ -1,6 +1,7 @@
 """ctypes binding of libcatcoc_hip.so (declarations: include/catcoc_hip.h)."""
 import ctypes as C
 import os
+import struct
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG, "libcatcoc_hip.so")
@@ -51,6 +52,10 @@ class CatcocSymmetricDesc(C.Structure):
         ("pipelinedPlan", C.c_void_p),
     ]
 
+
+_DESC = struct.Struct("=11I4x%dQqq7Q" % MAX_RANKS)   # CatcocSymmetricDesc's fields in order
+assert _DESC.size == C.sizeof(CatcocSymmetricDesc)
+_NO_PEERS = (0,) * MAX_RANKS
 
 KernelFuncPtr = C.CFUNCTYPE(None, C.c_void_p, C.c_uint64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
                             C.c_void_p, C.POINTER(CocTilingParams), C.c_uint32, C.c_uint32)
@@ -214,21 +219,12 @@ def check():
 def make_desc(rank, rank_size, peers=(), peer_ld=0, peer_row_offset=0, flags=0, block_num=0, stages=0,
               swizzle=None, outbound=None, outbound_bytes=0, checksum=None, acc_dump=None):
     """Build a CatcocSymmetricDesc from raw device addresses (ints)."""
-    d = CatcocSymmetricDesc()
-    d.magic = DESC_MAGIC
-    d.rankIdx = rank
-    d.rankSize = rank_size
-    d.blockNum = block_num
-    d.workspaceStages = stages
-    if swizzle is not None:
-        d.swizzleOffset, d.swizzleDirection = swizzle
-    d.flags = flags
-    for i, p in enumerate(peers):
-        d.peers[i] = p
-    d.peerLd = peer_ld
-    d.peerRowOffset = peer_row_offset
-    d.outbound = outbound
-    d.outboundBytes = outbound_bytes
-    d.checksum = checksum
-    d.accDump = acc_dump
-    return d
+    off, direction = swizzle if swizzle is not None else (0, 0)
+    peers = [p or 0 for p in peers]
+    if len(peers) > MAX_RANKS:
+        raise IndexError("at most %d peers" % MAX_RANKS)
+    # (packed in one go: setting thirty fields one by one takes 4 us)
+    u32 = 0xffffffff
+    return CatcocSymmetricDesc.from_buffer_copy(_DESC.pack(
+        DESC_MAGIC, rank & u32, rank_size & u32, block_num & u32, stages & u32, off & u32, direction & u32, flags & u32, 0, 0, 0,
+        *peers, *_NO_PEERS[len(peers):], peer_ld, peer_row_offset, outbound or 0, outbound_bytes, checksum or 0, acc_dump or 0, 0, 0, 0))
