@@ -303,9 +303,10 @@ CATCOC_API uint64_t catcoc_get_workspace_size(int commType, int dataType, const 
 /* Launches with few 128x256 tiles (fewer than half the CUs' worth) can cut every tile's k range into k slices, one
  * workgroup each, that meet through `workspace` (partial tiles in 32-bit words + one counter per tile, zeroed once
  * by the caller, re-armed by every launch): returns the bytes needed and the slice count (1 and 0 bytes when the
- * launch would not be sliced: other tile shapes, ragged problems, enough tiles already; the operands' layouts do
- * not matter).  The count
- * is 2, 4 or 8 for W8A8 (integer partials add exactly) and 2 for fp16/bf16; desc->splitK, when non-zero, is taken as the
+ * launch would not be sliced: enough tiles already, or a k too short; the operands' layouts do not matter).  The count
+ * is 2, 4 or 8 for W8A8 (integer partials add exactly) and 2 for fp16/bf16, or any up to 64 for launches that fill no 128x256
+ * tiles; with few tiles and a long k the bytes are those of more slices than that, which such a launch takes where its tiles run
+ * in flexible mode (a smaller workspace, down to the reported count's 128x256 partial tiles, serves too).  desc->splitK, when non-zero, is taken as the
  * caller's own count (up to 8; three or more fp32 partials are added in slice order whichever slice arrives last, so
  * the result is reproducible for any count).  A launch
  * slices only when `workspace` is given.  Counterpart in the reference: SplitkMatmul's k split

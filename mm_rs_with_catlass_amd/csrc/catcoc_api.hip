@@ -151,11 +151,18 @@ int plan_flex(GemmArgs &a, uint32_t es, bool sums, uint32_t wantM0, uint32_t sli
 // full; a slice costs the second launch about 0.1 us of latency and rows x n words written and read back at 4 TB/s.  The sum
 // steps * 0.3 / f + f * (0.1 + 2e-6 * rows * n) is least at the root below.  Measured optimum / this rule, bf16 all-reduce:
 // 16x8192x1024 24 / 24, 100x8192x1024 16 / 16, 28x15360x768 32 / 31, 16x4096x4096 8-16 / 13, 64x2048x4096 6 / 6,
-// 100x1024x8192 2 / 2, 200x1024x2048 3 / 3, 400x6144x1024 8 / 8, 824x7296x1280 3 / 3 (one workgroup per CU at most).
-uint32_t flex_slices(uint32_t rows, uint32_t n, uint32_t tiles, uint32_t steps)
+// 100x1024x8192 2 / 2, 200x1024x2048 3 / 3, 400x6144x1024 8 / 8, 824x7296x1280 3 / 3.
+// At most one workgroup per CU, except where that leaves a fifth of the CUs idle (or, for 16-bit operands, allows two slices
+// only) and k is long: then two per CU, if the root asks for as many.  One -> two, bf16 all-reduce, one peer, B as [n,k] / [k,n],
+// us: 88 tiles, 512 steps 149 / 139 -> 87 / 76; 98 tiles, 484 steps 167 / 124 -> 102 / 87; 128 tiles, 256 steps 76 / 68 -> 63 / 56;
+// 160 tiles, 512 steps 379 / 221 -> 258 / 153.  Not where the CUs are busy: W8A8, 120 tiles, 255 steps 82 / 55 -> 92 / 62;
+// bf16, 64 tiles, 512 steps 78 / 66 -> 79 / 71, 240 tiles, 384 steps 219 / 127 -> 286 / 163.
+uint32_t flex_slices(uint32_t es, uint32_t rows, uint32_t n, uint32_t tiles, uint32_t steps)
 {
     const double f = sqrt(0.3 * steps / (0.1 + 2e-6 * (double)rows * (double)n));
-    const uint32_t r = umin(umin((uint32_t)(f + 0.5), tiles ? 256u / tiles : 1u), umin(steps / 4u, 64u));
+    const uint32_t least = umin((uint32_t)(f + 0.5), umin(steps / 4u, 64u)), once = tiles ? 256u / tiles : 1u, twice = tiles ? 512u / tiles : 1u;
+    const bool pays = steps >= 256u && least >= twice && once <= 2u && (tiles * once <= 200u || (es == 2u && once == 2u));
+    const uint32_t r = pays ? twice : umin(least, once);
     return r < 2u ? 1u : r;
 }
 
@@ -173,7 +180,7 @@ int plan_flex_slices(GemmArgs &a, uint32_t es, uint32_t wantM0, uint32_t wantSli
     // explicit kept rows: the other rows need no partial sums of their own (the dump, if there is one, does)
     const bool keptOnly = (a.flags & GF_ROW_MASK) != 0 && a.accDump == nullptr;
     const uint32_t stored = keptOnly ? a.keptRows : a.fx.rows;
-    const uint32_t f = umin(umin(wantSlices ? wantSlices : flex_slices(stored, a.N, tiles, steps), 64u), steps);
+    const uint32_t f = umin(umin(wantSlices ? wantSlices : flex_slices(es, stored, a.N, tiles, steps), 64u), steps);
     if (f <= 1) return whole;
     const uint64_t sumBytes = keptOnly && sums ? (uint64_t)ceil_div(a.fx.rows, 128u) * ceil_div(a.N, 128u) * 16u : 0u;   // per slice
     const uint64_t slice = ((uint64_t)stored * a.N * 4u + sumBytes + 15u) / 16u * 16u;
@@ -407,11 +414,19 @@ int make_plan(int commType, int dataType, const CocTilingParams *t, const Catcoc
         plan.flexBlocks = plan_flex_slices(a, es, t->m0, d->splitK, d->workspace, d->workspaceBytes, &plan.kSlices, &plan.kSliceBytes);
     } else if (m0 == 128 && t->m0 == 0 && d->splitK == 0 && (d->flags & tuning) == 0 && fewTiles && !transA &&
                !(op == OP_REDUCE_SCATTER && P > 1 && a.checksum != nullptr)) {
-        // (what a workspace takes is still said for the aligned kernel; this one uses the slices that fit into that)
+        // What a workspace takes is said for the aligned kernel, and this one uses the slices that fit into that, unless it would
+        // take four or more: all-reduce of 257x14336x512, bf16, seven peers, in 64 KiB of workspace (no slices) / in what its slices
+        // take: 156 / 21 us; 306x13824x2048 147 / 41; reduce-scatter 832x15232x800 of four ranks with stored tiles 157 / 52.
         uint32_t slices;
         uint64_t bytes;
         plan.flexBlocks = plan_flex_slices(a, es, 0, 0, d->workspace, d->workspaceBytes, &slices, &bytes);
-        if (plan.flexBlocks != 0) plan.preferFlex = true;
+        if (plan.flexBlocks != 0) {
+            plan.preferFlex = true;
+            if (slices >= 4 && bytes > plan.kSliceBytes) {
+                if (plan.kSlices == 1) plan.kSlices = slices;   // (the aligned kernel's count is what launches with A as [k,m] run)
+                plan.kSliceBytes = bytes;
+            }
+        }
     }
     // a workspace also lets the checksum halves of tiles that run as two workgroups meet (its counter block)
     if (a.skCount == nullptr && d->workspace != nullptr && (uintptr_t)d->workspace % 256 == 0 && d->workspaceBytes >= kCounterBlockBytes)

@@ -179,3 +179,60 @@ def test_quant_kept_rows_in_slices(case):
         assert np.array_equal(ca.cpu().numpy(), acc[kb:kb + kr] + (sum(peers) if ri else 0))
         if cs is not None:
             assert np.array_equal(cs.cpu().numpy(), sums)
+
+
+@pytest.mark.parametrize("case", [(257, 512, 4096, 8), (256, 256, 8192, 2), (131, 300, 2048, 4), (448, 3584, 8224, 2)])
+def test_float_allreduce_few_tiles_long_k(case):
+    """All-reduce launches whose workspace query asks for the flexible tiles' own slices: with that workspace, with less (the
+    slices that fit) and with none; aligned and ragged rows, two workgroups per CU (98 tiles)."""
+    _need_gpu()
+    M, N, K, P = case
+    rng = np.random.default_rng(M)
+    A, B = _rand16(rng, (M, K), oracle.BF16), _rand16(rng, (K, N), oracle.BF16, 0.02)
+    peers = [rng.standard_normal((M, N)).astype(np.float32) for _ in range(P - 1)]
+    part, want = oracle.matmul_reduce(A, B, oracle.BF16, 0, M, peers, want_partial=True)
+    need, f = ops.kslice_plan(L.MATMUL_ALLREDUCE, torch.bfloat16, M, K, N, 0, P)
+    assert need >= 65536 + 4 * M * N * 4 and (f == 2) == (M % 128 == 0)   # (an aligned launch's count is the aligned kernel's)
+    for size in (need, 65536 + 2 * M * N * 4 + 4096, 0):
+        ws = torch.zeros(size, dtype=torch.uint8, device="cuda:0") if size else None
+        if ws is not None:
+            ws[65536:] = 0x55
+        try:
+            out = ops.matmul_allreduce(dev16(A, oracle.BF16), dev16(B, oracle.BF16), [dev(p) for p in peers], P - 1, P, workspace=ws)
+        except L.CatcocError as e:   # (the aligned kernel's own two slices are the least an aligned launch takes with a workspace)
+            assert 0 < size < need and "workspace too small" in str(e) and M % 128 == 0
+            continue
+        torch.cuda.synchronize()
+        _check_float(host16(out), want, part + sum(peers), oracle.BF16, K)
+        assert ws is None or not ws[:65536].any()
+
+
+def test_float_reduce_scatter_ragged_few_tiles_long_k():
+    """Reduce-scatter with stored tiles on ragged rows: k slices in the workspace the query asks for, and whole tiles without it."""
+    _need_gpu()
+    P, rows, N, K, rank = 4, 150, 296, 4096, 2
+    M = P * rows
+    rng = np.random.default_rng(77)
+    A, B = _rand16(rng, (M, K), oracle.FP16), _rand16(rng, (K, N), oracle.FP16, 0.02)
+    peers = [rng.standard_normal((rows, N)).astype(np.float32) for _ in range(P - 1)]
+    part, want = oracle.matmul_reduce(A, B, oracle.FP16, rank * rows, rows, peers, want_partial=True)
+    t = ops.default_tiling(M, K, N, P, m0=0, n0=0, k0=0)
+    need, f = ops.kslice_plan(L.MATMUL_REDUCE_SCATTER, torch.float16, M, K, N, rank, P, tiling=t)
+    assert f >= 4 and need == 65536 + f * M * N * 4
+    d = L.make_desc(rank, P, [16] * (P - 1))
+    tr, row, col, wsr = (C.c_uint32() for _ in range(4))
+    tasks = L.load().catcoc_get_task_count(L.MATMUL_REDUCE_SCATTER, C.byref(t), C.byref(d))
+    size = L.load().catcoc_get_workspace_size(L.MATMUL_REDUCE_SCATTER, L.FP16, C.byref(t), C.byref(d))
+    for ws in (torch.zeros(need, dtype=torch.uint8, device="cuda:0"), None):
+        ob = torch.full((size // 4,), 3.0, dtype=torch.float32, device="cuda:0")
+        out = ops.matmul_reduce_scatter(dev16(A, oracle.FP16), dev16(np.ascontiguousarray(B.T), oracle.FP16), [dev(p) for p in peers], rank, P, tiling=t,
+                                        trans_b=True, outbound=ob, workspace=ws)
+        torch.cuda.synchronize()
+        _check_float(host16(out), want, part[rank * rows:(rank + 1) * rows] + sum(peers), oracle.FP16, K)
+        for task in range(tasks):
+            L.load().catcoc_task_tile(L.MATMUL_REDUCE_SCATTER, C.byref(t), C.byref(d), task, C.byref(tr), C.byref(row), C.byref(col), C.byref(wsr))
+            if tr.value == rank:
+                continue
+            r1, c1 = min(row.value + 128, (tr.value + 1) * rows), min(col.value + 256, N)
+            got = ob.cpu().numpy().reshape(-1, 256)[wsr.value:wsr.value + r1 - row.value, :c1 - col.value]
+            assert np.abs(got - part[row.value:r1, col.value:c1]).max() <= K * 2.0 ** -24 * 0.41 * K + 1e-6, task   # (as in the tests above)
