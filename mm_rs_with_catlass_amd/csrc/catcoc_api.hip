@@ -854,8 +854,20 @@ void launch_pipelined(bool quant, int dataType, void *computeStream, void *commS
     g.flags &= ~(uint32_t)GF_RAGGED;   // (ragged problems run the bounds-checked kernel here)
     if (!dma && p.variant == 4) { fail(E_TILING, "m0 = 256 needs full tiles and 16-byte aligned row-major operands"); return; }
     if (!dma && g.transA) p.variant = 0;
+    // A call of one round is one launch over all tasks: it runs in flexible mode what the aligned kernels do not take (ragged rows
+    // or columns, which otherwise meet a bounds-checked kernel with hundreds of spilled registers) and few tiles of a short k, as
+    // the fused operators do.  W8A8, GEMM launch and comm launch, us: 2048x1792x1440 53.6 -> 27.6, 1536x3904x640 88.0 -> 29.3;
+    // aligned 1024x1792x2048 27.4 -> 25.6, 512x8192x4096 58.3 -> 45.2 (512x576x4096 18.0 / 18.4: not below 1 KiB of k).
+    int flexBlocks = 0;
+    if (sp.coreLoops <= sp.blockPerComm) {
+        const uint32_t es1 = quant ? 1u : 2u;
+        const uint64_t tiles64 = (uint64_t)ceil_div(tiling->m, 64u) * ceil_div(tiling->n, 256u);
+        if (!dma || (m0 == 128 && !transA && (uint64_t)tiling->k * es1 >= 1024u && (tiles64 <= 128u || (tiles64 <= 256u && (uint64_t)tiling->k * es1 <= 4096u))))
+            flexBlocks = plan_flex(g, es1, false, 0, 1);
+        if (flexBlocks != 0 && !flex_ptrs_ok(g)) flexBlocks = 0;
+    }
     const bool commWritesOutput = quant && deterministic != 0 && P > 1 && (uintptr_t)scale_x2 % 16 == 0 && (uintptr_t)d_out % 8 == 0;
-    if (dma && commWritesOutput) g.flags |= GF_KEPT_INT32_ONLY;   // (the comm rounds write every kept row's output)
+    if ((dma || flexBlocks) && commWritesOutput) g.flags |= GF_KEPT_INT32_ONLY;   // (the comm rounds write every kept row's output)
 
     CommArgs c;
     memset(&c, 0, sizeof(c));
@@ -915,7 +927,8 @@ void launch_pipelined(bool quant, int dataType, void *computeStream, void *commS
         g.taskBase = first;
         g.taskCount = actual;
         if (he == hipSuccess)
-            e = dma ? (p.dtype == DT_I8 ? launch_gemm_dma_i8(g, computeStream)
+            e = flexBlocks ? launch_flex(p.dtype, g, flexBlocks, computeStream)
+                : dma ? (p.dtype == DT_I8 ? launch_gemm_dma_i8(g, computeStream)
                        : p.dtype == DT_F16 ? launch_gemm_dma_f16(g, computeStream) : launch_gemm_dma_bf16(g, computeStream))
                     : launch_gemm(p.dtype, g, p.variant, p.edge, computeStream);
         if (e == 0 && he == hipSuccess && !oneStream) he = hipEventRecord(ready[r], cs);   // "store finished"

@@ -328,7 +328,7 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
                     if ((d[j] & FX_KIND) == FX_OUT)
                         __builtin_nontemporal_store(cur[j], (v4i *)((float *)args.outbound + (size_t)(d[j] & FX_INDEX) * args.sched.n0 + lcol));
             }
-            if (kN != 0) {   // (wave-uniform)
+            if (kN != 0 && !(args.flags & GF_KEPT_INT32_ONLY)) {   // (wave-uniform)
                 v2i pk[8];
                 auto pack = [&](auto cvt) {
 #pragma unroll

@@ -236,3 +236,34 @@ def test_float_reduce_scatter_ragged_few_tiles_long_k():
             r1, c1 = min(row.value + 128, (tr.value + 1) * rows), min(col.value + 256, N)
             got = ob.cpu().numpy().reshape(-1, 256)[wsr.value:wsr.value + r1 - row.value, :c1 - col.value]
             assert np.abs(got - part[row.value:r1, col.value:c1]).max() <= K * 2.0 ** -24 * 0.41 * K + 1e-6, task   # (as in the tests above)
+
+
+# (rows per rank, N, K, P, rank, weights as [n,k]): one-round pipelined calls on ragged columns, ragged rows, and few aligned tiles
+@pytest.mark.parametrize("case", [(128, 640, 448, 8, 3, False), (256, 1440, 192, 4, 0, True), (72, 288, 100, 2, 1, False), (128, 512, 1792, 8, 7, True)])
+@pytest.mark.parametrize("deterministic", [True, False])
+def test_pipelined_quant_one_round(case, deterministic):
+    _need_gpu()
+    rows, N, K, P, rank, tb = case
+    M = rows * P
+    rng = np.random.default_rng(rows + N)
+    x1, x2 = rng.integers(-127, 128, (M, K), dtype=np.int8), rng.integers(-127, 128, (K, N), dtype=np.int8)
+    s1, s2 = rng.uniform(0.005, 0.02, M).astype(np.float32), rng.uniform(0.001, 0.01, N).astype(np.float32)
+    b = rng.integers(-1000, 1000, N, dtype=np.int32)
+    peers = [rng.integers(-2 ** 20, 2 ** 20, (rows, N), dtype=np.int32) for _ in range(P - 1)]
+    acc, want = oracle.quant_matmul_reduce_scatter(x1, x2, s1, s2, b, rank * rows, rows, peers, oracle.BF16, reduce_int32=True)
+    t = ops.default_tiling(M, K, N, P, m0=128, n0=256, k0=0)
+    d = L.make_desc(rank, P, [16] * (P - 1))
+    size = L.load().catcoc_get_workspace_size(L.QUANT_MATMUL_REDUCE_SCATTER, L.INT8, C.byref(t), C.byref(d))
+    assert ops.pipelined_round_count(L.QUANT_MATMUL_REDUCE_SCATTER, t, rank, P) == 1
+    ob = torch.full((size // 4,), -9, dtype=torch.int32, device="cuda:0")
+    out, sums = ops.pipelined_quant_matmul_reduce_scatter(dev(x1), dev(np.ascontiguousarray(x2.T) if tb else x2), dev(s1), dev(s2), dev(b), [dev(p) for p in peers],
+                                                          rank, P, ob, tiling=t, trans_b=tb, deterministic=deterministic)
+    torch.cuda.synchronize()
+    assert np.array_equal(sums.cpu().numpy(), acc[rank * rows:(rank + 1) * rows] + sum(peers)) and np.array_equal(host16(out), want)
+    tr, row, col, wsr = (C.c_uint32() for _ in range(4))
+    for task in range(L.load().catcoc_get_task_count(L.QUANT_MATMUL_REDUCE_SCATTER, C.byref(t), C.byref(d))):
+        L.load().catcoc_task_tile(L.QUANT_MATMUL_REDUCE_SCATTER, C.byref(t), C.byref(d), task, C.byref(tr), C.byref(row), C.byref(col), C.byref(wsr))
+        if tr.value != rank:
+            r1, c1 = min(row.value + 128, (tr.value + 1) * rows), min(col.value + 256, N)
+            got = ob.cpu().numpy().reshape(-1, 256)[wsr.value:wsr.value + r1 - row.value, :c1 - col.value]
+            assert np.array_equal(got, acc[row.value:r1, col.value:c1]), task
