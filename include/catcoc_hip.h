@@ -306,7 +306,8 @@ CATCOC_API uint64_t catcoc_get_workspace_size(int commType, int dataType, const 
  * launch would not be sliced: enough tiles already, or a k too short; the operands' layouts do not matter).  The count
  * is 2, 4 or 8 for W8A8 (integer partials add exactly) and 2 for fp16/bf16, or any up to 64 for launches that fill no 128x256
  * tiles; with few tiles and a long k the bytes are those of more slices than that, which such a launch takes where its tiles run
- * in flexible mode (a smaller workspace, down to the reported count's 128x256 partial tiles, serves too).  desc->splitK, when non-zero, is taken as the
+ * in flexible mode (a smaller workspace, down to the reported count's 128x256 partial tiles, serves too).  A count of one with some bytes: a reduce-scatter launch whose kept rows meet their peers in a
+ * second launch when it is given them.  desc->splitK, when non-zero, is taken as the
  * caller's own count (up to 8; three or more fp32 partials are added in slice order whichever slice arrives last, so
  * the result is reproducible for any count).  A launch
  * slices only when `workspace` is given.  Counterpart in the reference: SplitkMatmul's k split

@@ -114,6 +114,7 @@ int plan_flex(GemmArgs &a, uint32_t es, bool sums, uint32_t wantM0, uint32_t sli
     f.rows = (uint32_t)rows;
     f.colTiles = ceil_div(a.N, 256u);
     f.slices = slices;
+    f.late = 0;
     f.dRank = make_fast_div(s.mRank);
     // the step of k that goes through registers with bounds checks: what whole steps leave, and the last step of all when
     // rows of B end inside a 16-byte piece (the copies then read past the end of every row but the last)
@@ -166,6 +167,19 @@ uint32_t flex_slices(uint32_t es, uint32_t rows, uint32_t n, uint32_t tiles, uin
     return r < 2u ? 1u : r;
 }
 
+// Reduce-scatter launches of one round of tiles: the few workgroups with kept rows stream all the peers (64 KiB per peer and 64
+// rows, at about 35 GB/s per CU) while the other CUs are done.  With the workspace the query asks for, the kept rows leave as
+// 32-bit sums and a second launch adds the peers over every CU.  One launch / two, us, launches alternating: W8A8 P = 8
+// 1000x1376x4096 27.3 / 25.5 (checksums 32.6 / 25.9), 504x1376x4096 21.7 / 19.3, 4000x1376x2048 42.3 / 34.4, 1016x736x1024
+// 17.8 / 16.2; P = 4 240x1056x2048 15.6 / 13.7; bf16 P = 8 800x1040x4096 25.4 / 22.3, 2000x1040x4096 41.9 / 32.9.  Below 128 KiB of
+// peers per tile the second launch (1-2 us) has nothing to win (W8A8 P = 2, 300x1056x4096, 15.1: not taken).
+bool flex_late(const GemmArgs &a)
+{
+    const SchedParams &s = a.sched;
+    return s.op == OP_REDUCE_SCATTER && s.P > 1 && !(a.flags & (GF_ROW_MASK | GF_KEPT_INT32_ONLY)) && a.fx.rowTiles * a.fx.colTiles <= 256u &&
+           a.nPeers * umin(a.keptRows, 64u) >= 128u;
+}
+
 // The whole of it: tiles and k slices of a launch that may run in flexible mode.  *slices / *bytes report the slices it would
 // run with a large enough workspace and what that takes; with a smaller one (or none) it runs with what fits.  wantSlices =
 // the caller's own number (0: the library's).
@@ -181,7 +195,16 @@ int plan_flex_slices(GemmArgs &a, uint32_t es, uint32_t wantM0, uint32_t wantSli
     const bool keptOnly = (a.flags & GF_ROW_MASK) != 0 && a.accDump == nullptr;
     const uint32_t stored = keptOnly ? a.keptRows : a.fx.rows;
     const uint32_t f = umin(umin(wantSlices ? wantSlices : flex_slices(es, stored, a.N, tiles, steps), 64u), steps);
-    if (f <= 1) return whole;
+    if (f <= 1) {
+        if (wantSlices <= 1 && flex_late(a)) {
+            *bytes = kCounterBlockBytes + (uint64_t)a.keptRows * a.N * 4u;
+            if (workspace != nullptr && (uintptr_t)workspace % 256 == 0 && workspaceBytes >= *bytes) {
+                a.fx.late = 1;
+                a.skPart = (int32_t *)((unsigned char *)workspace + kCounterBlockBytes);
+            }
+        }
+        return whole;
+    }
     const uint64_t sumBytes = keptOnly && sums ? (uint64_t)ceil_div(a.fx.rows, 128u) * ceil_div(a.N, 128u) * 16u : 0u;   // per slice
     const uint64_t slice = ((uint64_t)stored * a.N * 4u + sumBytes + 15u) / 16u * 16u;
     *slices = f;

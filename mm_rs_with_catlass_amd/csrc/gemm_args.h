@@ -38,6 +38,7 @@ struct FlexParams {
     uint32_t slices;               // k slices per tile (0, 1 = whole tiles)
     uint32_t keptOnly;             // k slices, explicit kept rows: partial sums of the kept rows only, the other rows as one sum per
     long long *sliceSums;          // 64 x 128 block and slice: [128 x 128 block][slice][upper / lower 64 rows]
+    uint32_t late;                 // whole tiles whose kept rows leave as 32-bit sums; a second launch adds their peers
     FastDiv dRank;                 // rows of one rank
 };
 

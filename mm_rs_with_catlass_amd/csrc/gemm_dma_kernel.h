@@ -1572,11 +1572,13 @@ inline int launch_flex(const GemmArgs &args, int rowBlocks, hipStream_t s)
     const FlexParams &f = args.fx;
     if (f.slices > 1) {
         launch_flex_tiles<DT, true>(args, rowBlocks, s);
-        const uint32_t rows = f.keptOnly ? args.keptRows : f.rows;
-        const uint32_t rowsPer = 4u * ceil_div(rows, 4u * 65535u);   // (a row per wave; the grid's second dimension ends at 65535)
-        hipLaunchKernelGGL((flex_finish_kernel<DT>), dim3(f.colTiles, ceil_div(rows, rowsPer)), dim3(256), 0, s, args, rowsPer);
     } else {
         launch_flex_tiles<DT, false>(args, rowBlocks, s);
+    }
+    if (f.slices > 1 || f.late) {
+        const uint32_t rows = f.keptOnly || f.late ? args.keptRows : f.rows;
+        const uint32_t rowsPer = 4u * ceil_div(rows, 4u * 65535u);   // (a row per wave; the grid's second dimension ends at 65535)
+        hipLaunchKernelGGL((flex_finish_kernel<DT>), dim3(f.colTiles, ceil_div(rows, rowsPer)), dim3(256), 0, s, args, rowsPer);
     }
     return (int)hipGetLastError();
 }

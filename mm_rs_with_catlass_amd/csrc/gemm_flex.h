@@ -202,7 +202,8 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
     const uint32_t kLo = args.keptBegin > t.row0 ? umin(args.keptBegin - t.row0, t.rowsValid) : 0u;   // the tile's kept rows: [kLo, kLo + kN)
     const uint32_t kN = keptEnd > t.row0 + kLo ? umin(keptEnd - t.row0, t.rowsValid) - kLo : 0u;
     const int64_t kept0 = (int64_t)t.row0 + kLo - args.keptBegin;   // (of no use, and possibly negative, when the tile has none)
-    const bool tileKept = args.nPeers != 0 && kN != 0;
+    const bool late = args.fx.late != 0;   // the kept rows' peers are the second launch's
+    const bool tileKept = args.nPeers != 0 && kN != 0 && !late;
     const uint32_t peerPitch = (uint32_t)args.peerLd * 4u, lastKept = colOk ? kN : 0u;
     const uint32_t turns = (args.nPeers + NBUF - 1u) / NBUF * NBUF;
     v4i buf[NBUF][8];
@@ -277,11 +278,16 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
             // (32-bit on purpose: the rows in front of the first kept one wrap, and a later row of the same lane is right again)
             auto keptRow = [&](int j) -> uint32_t { return blockRow + 2u * (uint32_t)j; };
             auto isKept = [&](int j) { return keptRow(j) < lastKept; };
+            if (late && kN != 0) {   // (wave-uniform)
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (isKept(j)) *(v4i *)(args.skPart + (kept0 + (int64_t)keptRow(j)) * args.N + gcol) = cur[j];
+            }
             // (a row that is not kept adds the zeros its loads returned: nothing for int32; floats are added to kept rows only,
             // by selects: a branch per row costs more than the additions)
             if constexpr (I8) {
                 if (redI32) add_peers([](v4i &c, const v4i &b, int) { c += b; });
-                if (args.cAccum) {
+                if (args.cAccum && !late) {
 #pragma unroll
                     for (int j = 0; j < 8; ++j)
                         if (isKept(j)) *(v4i *)(args.cAccum + (kept0 + (int64_t)keptRow(j)) * args.N + gcol) = cur[j];
@@ -328,7 +334,7 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
                     if ((d[j] & FX_KIND) == FX_OUT)
                         __builtin_nontemporal_store(cur[j], (v4i *)((float *)args.outbound + (size_t)(d[j] & FX_INDEX) * args.sched.n0 + lcol));
             }
-            if (kN != 0 && !(args.flags & GF_KEPT_INT32_ONLY)) {   // (wave-uniform)
+            if (kN != 0 && !late && !(args.flags & GF_KEPT_INT32_ONLY)) {   // (wave-uniform)
                 v2i pk[8];
                 auto pack = [&](auto cvt) {
 #pragma unroll
@@ -391,6 +397,7 @@ __device__ __forceinline__ long long wave_sum64(long long v)
 // in registers and leaves as one number per 64 x 128 block and slice.  (With partial sums of all rows and an atomic add per row
 // of 128 sums in the second launch 203x1792x4096 with 26 kept rows took 22.0 us instead of 13.7, 128x1024x8192 with 16 27.1
 // instead of 12.6.)
+// The same second launch also serves whole tiles whose kept rows leave as sums (late): it then adds nothing but their peers.
 template <int MB, typename Acc>
 __device__ __forceinline__ void flex_store_partial(const GemmArgs &args, Acc (&acc)[MB][4], unsigned char *smem, const FlexTile &t, uint32_t slice)
 {
@@ -494,8 +501,8 @@ __global__ void __launch_bounds__(256) flex_finish_kernel(const GemmArgs args, c
     const bool redI32 = I8 && (args.flags & GF_REDUCE_INT32) != 0;
     const bool store = (args.flags & GF_OUTBOUND_STORE) != 0, rowMask = (args.flags & GF_ROW_MASK) != 0;
     const bool sums = !store && args.checksum != nullptr;
-    const bool keptOnly = I8 && args.fx.keptOnly != 0;
-    const uint32_t first = keptOnly ? args.keptBegin : 0u, stored = keptOnly ? args.keptRows : args.fx.rows;   // the rows the partial sums hold
+    const bool keptOnly = I8 && args.fx.keptOnly != 0, late = args.fx.late != 0;
+    const uint32_t first = keptOnly || late ? args.keptBegin : 0u, stored = keptOnly || late ? args.keptRows : args.fx.rows;   // the rows the partial sums hold
     const uint32_t row0 = first + blockIdx.y * rowsPer, rowEnd = umin(row0 + rowsPer, first + stored);
     const uint32_t lcol = lane * 4u, gcol = blockIdx.x * 256u + lcol;
     const bool colOk = gcol < args.N;
@@ -552,8 +559,8 @@ __global__ void __launch_bounds__(256) flex_finish_kernel(const GemmArgs args, c
                         }
                     }
             }
-            if constexpr (I8) cur += bv;
-            if (args.accDump) *(v4i *)((int32_t *)args.accDump + (size_t)v * args.N + gcol) = cur;
+            if (I8 && !late) cur += bv;   // (late: the first launch has added the bias and written the dump)
+            if (args.accDump && !late) *(v4i *)((int32_t *)args.accDump + (size_t)v * args.N + gcol) = cur;
         }
         if (!kept) {
             uint32_t ws = 0, task = 0;

@@ -267,3 +267,52 @@ def test_pipelined_quant_one_round(case, deterministic):
             r1, c1 = min(row.value + 128, (tr.value + 1) * rows), min(col.value + 256, N)
             got = ob.cpu().numpy().reshape(-1, 256)[wsr.value:wsr.value + r1 - row.value, :c1 - col.value]
             assert np.array_equal(got, acc[row.value:r1, col.value:c1]), task
+
+
+# (rows per rank, N, K, P, rank, weights as [n,k], int32 peers): kept rows inside one 64-row tile, across two, at the end; two rows per wave column
+@pytest.mark.parametrize("case", [(125, 516, 1376, 8, 5, True, False), (64, 260, 352, 4, 3, False, True), (16, 512, 416, 16, 0, True, False), (65, 1028, 100, 16, 8, False, False)])
+@pytest.mark.parametrize("outbound", [False, True])
+def test_reduce_scatter_peers_in_a_second_launch(case, outbound):
+    """Ragged reduce-scatter launches of one round of tiles, with the workspace their query asks for: the kept rows' peers are added
+    by a second launch.  The same sums in the same order as without a workspace: every output bit for bit, W8A8 also the oracle's."""
+    _need_gpu()
+    rows, N, K, P, rank, tb, ri = case
+    M = rows * P
+    rng = np.random.default_rng(rows + K)
+    x1, x2 = rng.integers(-127, 128, (M, K), dtype=np.int8), rng.integers(-127, 128, (K, N), dtype=np.int8)
+    s1, s2 = rng.uniform(0.005, 0.02, M).astype(np.float32), rng.uniform(0.001, 0.01, N).astype(np.float32)
+    b = rng.integers(-1000, 1000, N, dtype=np.int32)
+    peers = [rng.integers(-2 ** 24, 2 ** 24, (rows, N), dtype=np.int32) if ri else rng.standard_normal((rows, N)).astype(np.float32) for _ in range(P - 1)]
+    acc, want = oracle.quant_matmul_reduce_scatter(x1, x2, s1, s2, b, rank * rows, rows, peers, oracle.BF16, reduce_int32=ri)
+    t = ops.default_tiling(M, K, N, P, m0=0, n0=0, k0=0)
+    d = L.make_desc(rank, P, [16] * (P - 1))
+    tasks = L.load().catcoc_get_task_count(L.QUANT_MATMUL_REDUCE_SCATTER, C.byref(t), C.byref(d))
+    size = L.load().catcoc_get_workspace_size(L.QUANT_MATMUL_REDUCE_SCATTER, L.INT8, C.byref(t), C.byref(d)) // 4
+    flip = lambda w: np.ascontiguousarray(w.T) if tb else w
+    dp = [dev(p) for p in peers]
+    A, B = _rand16(rng, (M, K), oracle.FP16), _rand16(rng, (K, N), oracle.FP16, 0.02)
+    for quant in (True, False) if not ri else (True,):
+        need, f = ops.kslice_plan(L.QUANT_MATMUL_REDUCE_SCATTER if quant else L.MATMUL_REDUCE_SCATTER, torch.int8 if quant else torch.float16, M, K, N, rank, P, tiling=t)
+        assert (need, f) == (65536 + rows * N * 4, 1) or f > 1
+        got = []
+        for ws in (torch.zeros(65536 + rows * N * 4, dtype=torch.uint8, device="cuda:0"), None):
+            kw = {"outbound": torch.full((size,), 3, dtype=torch.int32 if ri else torch.float32, device="cuda:0")} if outbound else \
+                 {"checksum": torch.full((tasks,), 77, dtype=torch.int64 if quant else torch.float64, device="cuda:0")}
+            kw.update(tiling=t, trans_b=tb, workspace=ws, split_k=1)
+            dump = torch.zeros((M, N), dtype=torch.int32 if quant else torch.float32, device="cuda:0")
+            if quant:
+                ca = torch.full((rows, N), -7, dtype=torch.int32, device="cuda:0")
+                out = ops.quant_matmul_reduce_scatter(dev(x1), dev(flip(x2)), dev(s1), dev(s2), dev(b), dp, rank, P, reduce_int32=ri, c_accum=ca, acc_dump=dump, **kw)
+                torch.cuda.synchronize()
+                assert np.array_equal(host16(out), want) and np.array_equal(dump.cpu().numpy(), acc)
+                assert np.array_equal(ca.cpu().numpy(), acc[rank * rows:(rank + 1) * rows] + (sum(peers) if ri else 0))
+            else:
+                out = ops.matmul_reduce_scatter(dev16(A, oracle.FP16), dev16(flip(B), oracle.FP16), dp, rank, P, acc_dump=dump, **kw)
+                torch.cuda.synchronize()
+            assert ws is None or (not ws[:65536].any() and bool(ws[65536:].any()))
+            got.append([out, dump, kw.get("outbound", kw.get("checksum"))])
+        for with_ws, without in zip(*got):
+            if with_ws.dtype == torch.float64:   # (64-bit sums of a tile meet in any order: 2^-52 of 2^15 magnitudes of at most 0.41 * K)
+                assert float((with_ws - without).abs().max()) <= 2.0 ** -37 * 0.41 * K
+            else:
+                assert torch.equal(with_ws, without)
