@@ -171,13 +171,13 @@ uint32_t flex_slices(uint32_t es, uint32_t rows, uint32_t n, uint32_t tiles, uin
 // rows, at about 35 GB/s per CU) while the other CUs are done.  With the workspace the query asks for, the kept rows leave as
 // 32-bit sums and a second launch adds the peers over every CU.  One launch / two, us, launches alternating: W8A8 P = 8
 // 1000x1376x4096 27.3 / 25.5 (checksums 32.6 / 25.9), 504x1376x4096 21.7 / 19.3, 4000x1376x2048 42.3 / 34.4, 1016x736x1024
-// 17.8 / 16.2; P = 4 240x1056x2048 15.6 / 13.7; bf16 P = 8 800x1040x4096 25.4 / 22.3, 2000x1040x4096 41.9 / 32.9.  Below 128 KiB of
-// peers per tile the second launch (1-2 us) has nothing to win (W8A8 P = 2, 300x1056x4096, 15.1: not taken).
+// 17.8 / 16.2; bf16 P = 8 800x1040x4096 25.4 / 22.3, 2000x1040x4096 41.9 / 32.9.  Below 256 KiB of peers per tile the second launch
+// (2-3 us) has nothing to win (bf16 P = 4 200x1040x8192, 150 KiB: 18.0 / 20.4 us; not taken).
 bool flex_late(const GemmArgs &a)
 {
     const SchedParams &s = a.sched;
     return s.op == OP_REDUCE_SCATTER && s.P > 1 && !(a.flags & (GF_ROW_MASK | GF_KEPT_INT32_ONLY)) && a.fx.rowTiles * a.fx.colTiles <= 256u &&
-           a.nPeers * umin(a.keptRows, 64u) >= 128u;
+           a.nPeers * umin(a.keptRows, 64u) >= 256u;
 }
 
 // The whole of it: tiles and k slices of a launch that may run in flexible mode.  *slices / *bytes report the slices it would
@@ -194,7 +194,11 @@ int plan_flex_slices(GemmArgs &a, uint32_t es, uint32_t wantM0, uint32_t wantSli
     // explicit kept rows: the other rows need no partial sums of their own (the dump, if there is one, does)
     const bool keptOnly = (a.flags & GF_ROW_MASK) != 0 && a.accDump == nullptr;
     const uint32_t stored = keptOnly ? a.keptRows : a.fx.rows;
-    const uint32_t f = umin(umin(wantSlices ? wantSlices : flex_slices(es, stored, a.N, tiles, steps), 64u), steps);
+    uint32_t own = flex_slices(es, stored, a.N, tiles, steps);
+    // (a reduce-scatter's other rows are done after the first launch: two slices' traffic is more than they save.  Whole / two
+    // slices, bf16, four ranks, 200x1040x8192 18.1 / 33.2 with checksums, 18.8 / 23.6 us with stored tiles)
+    if (own == 2 && !keptOnly && a.sched.op == OP_REDUCE_SCATTER && a.sched.P > 1) own = 1;
+    const uint32_t f = umin(umin(wantSlices ? wantSlices : own, 64u), steps);
     if (f <= 1) {
         if (wantSlices <= 1 && flex_late(a)) {
             *bytes = kCounterBlockBytes + (uint64_t)a.keptRows * a.N * 4u;

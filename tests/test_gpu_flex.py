@@ -270,7 +270,7 @@ def test_pipelined_quant_one_round(case, deterministic):
 
 
 # (rows per rank, N, K, P, rank, weights as [n,k], int32 peers): kept rows inside one 64-row tile, across two, at the end; two rows per wave column
-@pytest.mark.parametrize("case", [(125, 516, 1376, 8, 5, True, False), (64, 260, 352, 4, 3, False, True), (16, 512, 416, 16, 0, True, False), (65, 1028, 100, 16, 8, False, False)])
+@pytest.mark.parametrize("case", [(125, 516, 1376, 8, 5, True, False), (64, 260, 352, 8, 3, False, True), (18, 512, 416, 16, 0, True, False), (65, 1028, 100, 16, 8, False, False)])
 @pytest.mark.parametrize("outbound", [False, True])
 def test_reduce_scatter_peers_in_a_second_launch(case, outbound):
     """Ragged reduce-scatter launches of one round of tiles, with the workspace their query asks for: the kept rows' peers are added
