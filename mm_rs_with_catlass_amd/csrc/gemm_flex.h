@@ -15,7 +15,7 @@
 // k, the peers' stream for short k.  Measured against what ran these launches before (a kernel that staged its tiles through
 // registers, or one thread per output element), launches alternating: fp16 all-gather 8 x [1024,6148] x [6148,5120]
 // 243 ms -> 0.522 ms = 988 TFLOP/s (12296-byte rows, 8 bytes of k left over), W8A8 reduce-scatter 1000x1376x4096 with 125
-// rows per rank and stored tiles 276 -> 32 us, bf16 all-reduce 16x1024x8192 28.6 -> 18.2 us.
+// rows per rank and stored tiles 277 -> 26 us, bf16 all-reduce 16x1024x8192 28.7 -> 13.0 us.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
