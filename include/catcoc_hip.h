@@ -149,8 +149,9 @@ typedef struct CatcocSymmetricDesc {
      * CATCOC_WORKSPACE_COUNTER_BYTES hold one arrival counter per tile, at the same place for every shape and slice
      * count; the partial tiles follow.  The caller ZEROES the counter block (or simply the whole buffer) once before
      * the first use; every launch leaves the counters at zero again, so launches of any shapes may share one
-     * workspace that is large enough for each of them.  Launches that share a workspace must not overlap (same
-     * stream, or ordered by events). */
+     * workspace that is large enough for each of them.  A launch touches no byte past what its query reports, however
+     * large the workspace is, and where that is 0 nothing behind the counter block.  Launches that share a workspace
+     * must not overlap (same stream, or ordered by events). */
     void *workspace;
     uint64_t workspaceBytes;
     /* Round-pipelined operators only: the events they order their two streams with, made once by

@@ -180,46 +180,65 @@ bool flex_late(const GemmArgs &a)
            a.nPeers * umin(a.keptRows, 64u) >= 256u;
 }
 
-// The whole of it: tiles and k slices of a launch that may run in flexible mode.  *slices / *bytes report the slices it would
-// run with a large enough workspace and what that takes; with a smaller one (or none) it runs with what fits.  wantSlices =
-// the caller's own number (0: the library's).
-int plan_flex_slices(GemmArgs &a, uint32_t es, uint32_t wantM0, uint32_t wantSlices, void *workspace, uint64_t workspaceBytes, uint32_t *slices, uint64_t *bytes)
+// Tiles and k slices of a launch that may run in flexible mode, in two halves: what it would take, and what it takes of the
+// workspace it is given.  A launch is given no more of its workspace than its query asks for (the rest may be another
+// launch's), so the first half must not depend on the operands' layouts, which the query does not know.
+struct FlexSlices {
+    int whole;             // rows / 64 of its tiles without k slices; 0: it cannot run in flexible mode
+    uint32_t slices;       // k slices with a large enough workspace
+    uint64_t bytes;        // what they take (one slice and some bytes: the peers' second launch)
+    uint64_t slice, sums;  // of that per slice: all, and the sums of rows that are not kept
+    bool keptOnly;
+};
+
+// Fills args.fx for whole tiles.  wantSlices = the caller's own number (0: the library's).
+FlexSlices flex_choose(GemmArgs &a, uint32_t es, uint32_t wantM0, uint32_t wantSlices)
 {
     const bool sums = (a.flags & GF_OUTBOUND_STORE) == 0 && a.checksum != nullptr;
-    const int whole = plan_flex(a, es, sums, wantM0, 1);
-    *slices = 1;
-    *bytes = 0;
-    if (whole == 0) return 0;
-    const uint32_t steps = (uint32_t)(((uint64_t)a.K * es - a.fx.tail) / 64u), tiles = ceil_div(a.fx.rows, 64u) * a.fx.colTiles;
+    FlexSlices c = {plan_flex(a, es, sums, wantM0, 1), 1, 0, 0, 0, false};
+    if (c.whole == 0) return c;
+    // (whole k steps as with B as [k,n]: with B as [n,k] there is one more where rows of B would end inside a 16-byte piece)
+    const uint64_t kBytes = (uint64_t)a.K * es;
+    const uint32_t steps = (uint32_t)(kBytes / 64u) - (kBytes % 64u == 0 && ((uint64_t)a.N * es) % 16u != 0 ? 1u : 0u);
+    const uint32_t tiles = ceil_div(a.fx.rows, 64u) * a.fx.colTiles;
     // explicit kept rows: the other rows need no partial sums of their own (the dump, if there is one, does)
-    const bool keptOnly = (a.flags & GF_ROW_MASK) != 0 && a.accDump == nullptr;
-    const uint32_t stored = keptOnly ? a.keptRows : a.fx.rows;
+    c.keptOnly = (a.flags & GF_ROW_MASK) != 0 && a.accDump == nullptr;
+    const uint32_t stored = c.keptOnly ? a.keptRows : a.fx.rows;
     uint32_t own = flex_slices(es, stored, a.N, tiles, steps);
     // (a reduce-scatter's other rows are done after the first launch: two slices' traffic is more than they save.  Whole / two
     // slices, bf16, four ranks, 200x1040x8192 18.1 / 33.2 with checksums, 18.8 / 23.6 us with stored tiles)
-    if (own == 2 && !keptOnly && a.sched.op == OP_REDUCE_SCATTER && a.sched.P > 1) own = 1;
+    if (own == 2 && !c.keptOnly && a.sched.op == OP_REDUCE_SCATTER && a.sched.P > 1) own = 1;
     const uint32_t f = umin(umin(wantSlices ? wantSlices : own, 64u), steps);
     if (f <= 1) {
-        if (wantSlices <= 1 && flex_late(a)) {
-            *bytes = kCounterBlockBytes + (uint64_t)a.keptRows * a.N * 4u;
-            if (workspace != nullptr && (uintptr_t)workspace % 256 == 0 && workspaceBytes >= *bytes) {
-                a.fx.late = 1;
-                a.skPart = (int32_t *)((unsigned char *)workspace + kCounterBlockBytes);
-            }
-        }
-        return whole;
+        if (wantSlices <= 1 && flex_late(a)) c.bytes = kCounterBlockBytes + (uint64_t)a.keptRows * a.N * 4u;
+        return c;
     }
-    const uint64_t sumBytes = keptOnly && sums ? (uint64_t)ceil_div(a.fx.rows, 128u) * ceil_div(a.N, 128u) * 16u : 0u;   // per slice
-    const uint64_t slice = ((uint64_t)stored * a.N * 4u + sumBytes + 15u) / 16u * 16u;
-    *slices = f;
-    *bytes = kCounterBlockBytes + f * slice;
-    if (workspace == nullptr || (uintptr_t)workspace % 256 != 0 || workspaceBytes < kCounterBlockBytes + 2u * slice) return whole;
-    const uint64_t fit = (workspaceBytes - kCounterBlockBytes) / slice;
-    const uint32_t run = fit < f ? (uint32_t)fit : f;
-    a.fx.keptOnly = keptOnly ? 1u : 0u;
-    a.fx.sliceSums = (long long *)((unsigned char *)workspace + kCounterBlockBytes);
-    a.skPart = (int32_t *)((unsigned char *)workspace + kCounterBlockBytes + run * sumBytes);
-    return plan_flex(a, es, sums, wantM0, run);
+    c.slices = f;
+    c.sums = c.keptOnly && sums ? (uint64_t)ceil_div(a.fx.rows, 128u) * ceil_div(a.N, 128u) * 16u : 0u;
+    c.slice = ((uint64_t)stored * a.N * 4u + c.sums + 15u) / 16u * 16u;
+    c.bytes = kCounterBlockBytes + f * c.slice;
+    return c;
+}
+
+// The slices that fit (none: whole tiles), in args.fx; returns the tile's rows / 64.
+int flex_use(GemmArgs &a, uint32_t es, uint32_t wantM0, const FlexSlices &c, void *workspace, uint64_t workspaceBytes)
+{
+    if (c.bytes == 0 || workspace == nullptr || (uintptr_t)workspace % 256 != 0) return c.whole;
+    unsigned char *part = (unsigned char *)workspace + kCounterBlockBytes;
+    if (c.slices <= 1) {
+        if (workspaceBytes >= c.bytes) {
+            a.fx.late = 1;
+            a.skPart = (int32_t *)part;
+        }
+        return c.whole;
+    }
+    if (workspaceBytes < kCounterBlockBytes + 2u * c.slice) return c.whole;
+    const uint64_t fit = (workspaceBytes - kCounterBlockBytes) / c.slice;
+    const uint32_t run = fit < c.slices ? (uint32_t)fit : c.slices;
+    a.fx.keptOnly = c.keptOnly ? 1u : 0u;
+    a.fx.sliceSums = (long long *)part;
+    a.skPart = (int32_t *)(part + run * c.sums);
+    return plan_flex(a, es, (a.flags & GF_OUTBOUND_STORE) == 0 && a.checksum != nullptr, wantM0, run);
 }
 
 // What flexible mode asks of the pointers: operands on the 4-byte grid, everything the epilogue touches in its 8- and 16-byte
@@ -438,22 +457,23 @@ int make_plan(int commType, int dataType, const CocTilingParams *t, const Catcoc
     const bool fewTiles = tiles64 <= 128u || (tiles64 <= 256u && (uint64_t)t->k * es <= 4096u);
     const uint32_t tuning = CATCOC_FLAG_LINEAR_ORDER | CATCOC_FLAG_KEPT_WHOLE | CATCOC_FLAG_KEPT_SPLIT;
     if (!plan.dma) {
-        plan.flexBlocks = plan_flex_slices(a, es, t->m0, d->splitK, d->workspace, d->workspaceBytes, &plan.kSlices, &plan.kSliceBytes);
+        const FlexSlices c = flex_choose(a, es, t->m0, d->splitK);
+        plan.kSlices = c.slices;
+        plan.kSliceBytes = c.bytes;
+        plan.flexBlocks = flex_use(a, es, t->m0, c, d->workspace, d->workspaceBytes);
     } else if (m0 == 128 && t->m0 == 0 && d->splitK == 0 && (d->flags & tuning) == 0 && fewTiles && !transA &&
                !(op == OP_REDUCE_SCATTER && P > 1 && a.checksum != nullptr)) {
         // What a workspace takes is said for the aligned kernel, and this one uses the slices that fit into that, unless it would
         // take four or more: all-reduce of 257x14336x512, bf16, seven peers, in 64 KiB of workspace (no slices) / in what its slices
         // take: 156 / 21 us; 306x13824x2048 147 / 41; reduce-scatter 832x15232x800 of four ranks with stored tiles 157 / 52.
-        uint32_t slices;
-        uint64_t bytes;
-        plan.flexBlocks = plan_flex_slices(a, es, 0, 0, d->workspace, d->workspaceBytes, &slices, &bytes);
-        if (plan.flexBlocks != 0) {
-            plan.preferFlex = true;
-            if (slices >= 4 && bytes > plan.kSliceBytes) {
-                if (plan.kSlices == 1) plan.kSlices = slices;   // (the aligned kernel's count is what launches with A as [k,m] run)
-                plan.kSliceBytes = bytes;
-            }
+        // (Rows of B that end inside a 16-byte piece have an aligned kernel as [n,k] only: the query speaks of flexible tiles.)
+        const FlexSlices c = flex_choose(a, es, 0, 0);
+        plan.preferFlex = c.whole != 0;
+        if (plan.preferFlex && ((c.slices >= 4 && c.bytes > plan.kSliceBytes) || ((uint64_t)t->n * es) % 16 != 0)) {
+            if (plan.kSlices == 1) plan.kSlices = c.slices;   // (the aligned kernel's count is what launches with A as [k,m] run)
+            plan.kSliceBytes = c.bytes;
         }
+        plan.flexBlocks = flex_use(a, es, 0, c, d->workspace, d->workspaceBytes < plan.kSliceBytes ? d->workspaceBytes : plan.kSliceBytes);
     }
     // a workspace also lets the checksum halves of tiles that run as two workgroups meet (its counter block)
     if (a.skCount == nullptr && d->workspace != nullptr && (uintptr_t)d->workspace % 256 == 0 && d->workspaceBytes >= kCounterBlockBytes)
@@ -585,11 +605,8 @@ int make_splitk_plan(const CocTilingParams *t, const CatcocSymmetricDesc *d, uin
         a.sched = make_sched(OP_ALLREDUCE, t->m, t->n, 1, 128, 256, cores, 1, stages, off, dir);
         a.flags |= GF_ROW_MASK;
         sp.rowBlocks = 4;
-        // (the plan says whole tiles and no workspace, as for any launch that can do without; a workspace that is there anyway
-        // is made use of)
-        uint64_t wouldTake;
-        uint32_t wouldSlice;
-        sp.flexBlocks = plan_flex_slices(a, 1, 0, 0, d->workspace, d->workspaceBytes, &wouldSlice, &wouldTake);
+        // (whole tiles: the query promises that such a launch touches no workspace)
+        sp.flexBlocks = plan_flex(a, 1, a.checksum != nullptr, 0, 1);
         sp.f = 1;
         sp.workspaceBytes = 0;
         if (sp.flexBlocks == 0) a.sched = make_sched(OP_ALLREDUCE, t->m, t->n, 1, 128, 128, cores, 1, stages, off, dir);
@@ -717,11 +734,10 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
         g.flags |= GF_ROW_MASK;
         g.splitK = 0;
         g.skCount = nullptr;
-        uint32_t wouldSlice;
-        uint64_t wouldTake;
-        const int blocks = plan_flex_slices(g, 1, 0, 0, d->workspace, d->workspaceBytes, &wouldSlice, &wouldTake);
+        const FlexSlices c = flex_choose(g, 1, 0, 0);
+        const int blocks = flex_use(g, 1, 0, c, d->workspace, d->workspaceBytes < sp.workspaceBytes ? d->workspaceBytes : sp.workspaceBytes);
         // (without the slices it would take, only where the streaming kernels run whole tiles as well)
-        if (blocks == 0 || (wouldSlice > 1 && g.fx.slices < 2 && (sp.large || sp.f > 1)) || !flex_ptrs_ok(g)) return false;
+        if (blocks == 0 || (c.slices > 1 && g.fx.slices < 2 && (sp.large || sp.f > 1)) || !flex_ptrs_ok(g)) return false;
         const int e = launch_flex(DT_I8, g, blocks, stream);
         if (e) fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)e));
         else ok();
@@ -1044,6 +1060,7 @@ void catcoc_launch_quant_matmul_reduce_scatter_static_scratch(void *stream, uint
             need = sp.workspaceBytes;
         } else {
             Plan p;
+            if ((q.flags & CATCOC_OUTBOUND_MASK) == CATCOC_OUTBOUND_STORE) q.checksum = nullptr;   // (the launch will not look at it)
             q.flags &= ~CATCOC_OUTBOUND_MASK;
             if (make_plan(QUANT_MATMUL_REDUCE_SCATTER, INT8, tiling, &q, transA, transB, p)) return;
             need = p.kSliceBytes;
@@ -1152,6 +1169,7 @@ uint64_t catcoc_get_kslice_workspace_size(int commType, int dataType, const CocT
     CatcocSymmetricDesc d;
     if (desc == nullptr || tiling == nullptr) { fail(E_NULL, "tiling and desc must be non-NULL"); return 0; }
     d = *desc;
+    if ((d.flags & CATCOC_OUTBOUND_MASK) == CATCOC_OUTBOUND_STORE) d.checksum = nullptr;   // (the launch will not look at it)
     d.flags &= ~CATCOC_OUTBOUND_MASK;
     d.workspace = nullptr;
     const uint32_t forced = d.splitK;

@@ -316,3 +316,55 @@ def test_reduce_scatter_peers_in_a_second_launch(case, outbound):
                 assert float((with_ws - without).abs().max()) <= 2.0 ** -37 * 0.41 * K
             else:
                 assert torch.equal(with_ws, without)
+
+
+# (kind, rows, N, K, P, kept rows or 0): launches whose flexible tiles would take k slices, or a second launch for the peers, that
+# their query does not ask for: explicit kept rows off the 64/128 grid and in full tiles with a short k; aligned all-reduce with a k
+# too short for the aligned kernel's slices; aligned reduce-scatter with stored tiles and a short k
+@pytest.mark.parametrize("case", [("decode", 40, 260, 2052, 4, 40), ("decode", 130, 1100, 516, 2, 12), ("decode", 512, 1024, 768, 8, 512),
+                                  ("allreduce", 512, 1024, 480, 2, 0), ("quant_rs", 1024, 4096, 256, 8, 0), ("float_rs", 1024, 4096, 128, 8, 0)])
+@pytest.mark.parametrize("tb", [False, True])
+def test_workspace_past_the_queried_bytes_is_not_touched(case, tb):
+    """A launch uses no byte of a workspace past what its query says, also when that is none: the rest may be in use elsewhere."""
+    _need_gpu()
+    kind, M, N, K, P, kr = case
+    g = torch.Generator(device="cuda:0").manual_seed(M + K)
+    quant = kind in ("decode", "quant_rs")
+    rows = kr or (M // P if kind.endswith("rs") else M)
+    peers = [torch.randn((rows, N), device="cuda:0", generator=g) for _ in range(P - 1)]
+    kw, rank = {}, P - 1
+    if quant:
+        a = torch.randint(-127, 128, (M, K), dtype=torch.int8, device="cuda:0", generator=g)
+        b = torch.randint(-127, 128, (N, K) if tb else (K, N), dtype=torch.int8, device="cuda:0", generator=g)
+        s1, s2 = (torch.empty(x, device="cuda:0").uniform_(0.001, 0.02, generator=g) for x in (M, N))
+    else:
+        a = torch.randn((M, K), device="cuda:0", generator=g).half()
+        b = torch.randn((N, K) if tb else (K, N), device="cuda:0", generator=g).half()
+    if kind == "decode":
+        need = ops.splitk_plan(M, K, N, P, 0, kr)[0]
+        run = lambda ws: ops.quant_matmul_splitk(a, b, s1, s2, None, peers, P, 0, kr, trans_b=tb, workspace=ws)
+    else:
+        comm, dt = {"allreduce": (L.MATMUL_ALLREDUCE, torch.float16), "quant_rs": (L.QUANT_MATMUL_REDUCE_SCATTER, torch.int8),
+                    "float_rs": (L.MATMUL_REDUCE_SCATTER, torch.float16)}[kind]
+        t = ops.default_tiling(M, K, N, P, m0=0, n0=0, k0=0)
+        need = ops.kslice_plan(comm, dt, M, K, N, rank, P, tiling=t)[0]
+        if kind != "allreduce":
+            d = L.make_desc(rank, P, [16] * (P - 1))
+            size = L.load().catcoc_get_workspace_size(comm, L.INT8 if quant else L.FP16, C.byref(t), C.byref(d)) // 4
+            kw = {"outbound": torch.zeros(size, device="cuda:0")}
+        if kind == "quant_rs":
+            run = lambda ws: ops.quant_matmul_reduce_scatter(a, b, s1, s2, None, peers, rank, P, tiling=t, trans_b=tb, workspace=ws, **kw)
+        elif kind == "float_rs":
+            run = lambda ws: ops.matmul_reduce_scatter(a, b, peers, rank, P, tiling=t, trans_b=tb, workspace=ws, **kw)
+        else:
+            run = lambda ws: ops.matmul_allreduce(a, b, peers, rank, P, tiling=t, trans_b=tb, workspace=ws)
+    end = max(need, 65536)
+    got = []
+    for extra in (0, 16 << 20):
+        ws = torch.zeros(end + extra, dtype=torch.uint8, device="cuda:0")
+        ws[65536:] = 0x55
+        out = run(ws)
+        torch.cuda.synchronize()
+        assert bool((ws[end:] == 0x55).all()) and not ws[:65536].any()
+        got.append(out.clone())
+    assert torch.equal(got[0].view(torch.int16), got[1].view(torch.int16))
