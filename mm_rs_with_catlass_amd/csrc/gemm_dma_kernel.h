@@ -1580,6 +1580,8 @@ inline int launch_flex(const GemmArgs &args, int rowBlocks, hipStream_t s)
         const uint32_t rowsPer = 4u * ceil_div(rows, 4u * 65535u);   // (a row per wave; the grid's second dimension ends at 65535)
         hipLaunchKernelGGL((flex_finish_kernel<DT>), dim3(f.colTiles, ceil_div(rows, rowsPer)), dim3(256), 0, s, args, rowsPer);
     }
+    if (DT != DT_I8 && f.slices > 1 && args.sched.op == OP_REDUCE_SCATTER && args.sched.P > 1 && args.checksum != nullptr && !(args.flags & GF_OUTBOUND_STORE))
+        hipLaunchKernelGGL((flex_sums_kernel<DT>), dim3(f.colTiles * args.sched.P * args.sched.loopsM), dim3(64), 0, s, args);
     return (int)hipGetLastError();
 }
 

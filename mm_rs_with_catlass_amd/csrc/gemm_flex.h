@@ -129,7 +129,33 @@ __device__ __forceinline__ v4i load16_guarded(const unsigned char *p, int valid,
 enum : uint32_t { FX_SKIP = 0u, FX_KEPT = 1u << 30, FX_OUT = 2u << 30, FX_SUM = 3u << 30, FX_KIND = 3u << 30, FX_INDEX = (1u << 30) - 1u };
 
 constexpr int FLEX_STAGING = 4 * 16384;                 // one 16 KiB area per wave
-constexpr int FLEX_POOL = FLEX_STAGING + 128 * 8 + 16 * 12;   // + the row table + the sums of up to 16 tasks
+constexpr int FLEX_POOL = FLEX_STAGING + 128 * 8 + 16 * 8 * 8 + 16 * 4;   // + the row table + the sums of up to 16 tasks, per half wave
+
+// Sums over lanes, always in the same order: cross-lane adds in the vector unit (a shuffle is a trip through the LDS unit).
+template <int CTRL, int ROWS, typename T>
+__device__ __forceinline__ T dpp_add64(T v)
+{
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+    return v + __builtin_bit_cast(T, ((unsigned long long)(uint32_t)hi << 32) | (uint32_t)lo);
+}
+// over each half of a wave, in its last lane
+template <typename T>
+__device__ __forceinline__ T half_sum64(T v)
+{
+    v = dpp_add64<0x111, 0xf>(v);   // row_shr:1, 2, 4, 8: lane 15 of every row of 16 holds the row's sum
+    v = dpp_add64<0x112, 0xf>(v);
+    v = dpp_add64<0x114, 0xf>(v);
+    v = dpp_add64<0x118, 0xf>(v);
+    return dpp_add64<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+}
+// over the 64 lanes, in lane 63
+template <typename T>
+__device__ __forceinline__ T wave_sum64(T v)
+{
+    return dpp_add64<0x143, 0xc>(half_sum64(v));   // row_bcast:31 into rows 2 and 3
+}
 
 // acc[mb][nb][r] of wave (wm, wn) is element (row, col) of the tile with
 //   row = wm*32*MB + mb*32 + (r>>2)*8 + h*4 + (r&3),  col = wn*128 + nb*32 + c32
@@ -147,8 +173,10 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
 
     uint32_t *dst = (uint32_t *)(smem + FLEX_STAGING);      // [128] what row i of the tile does
     float *rowScale = (float *)(dst + 128);                  // [128] W8A8 per-token scale
-    Sum *sums = (Sum *)(rowScale + 128);                     // [16] task sums (explicit kept rows: one per 128 columns)
-    uint32_t *sumTask = (uint32_t *)(sums + 16);             // [16]
+    // Sums of the tile's tasks (explicit kept rows: of its 128-column halves), [16][half wave]: a place per writer and a fixed
+    // order of adding them up, so that sums of floats are the same bits in every launch.
+    Sum *sums = (Sum *)(rowScale + 128);
+    uint32_t *sumTask = (uint32_t *)(sums + 16 * 8);         // [16]
     __syncthreads();   // every wave has left the main loop's LDS reads behind
     if (tid < 64 * MB) {
         const uint32_t v = t.row0 + tid;
@@ -174,7 +202,7 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
         dst[tid] = e;
         if constexpr (I8) rowScale[tid] = args.scaleM[umin(v, args.fx.rows - 1u)];
     }
-    if (tid < 16) sums[tid] = 0;
+    if (tid < 16 * 8) sums[tid] = 0;
     __syncthreads();
 
     unsigned char *st = smem + w * 16384;
@@ -225,8 +253,13 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
     // the output the same way: a base at the tile's first kept row, stores of rows that are not kept behind the end
     const uint32_t outPitch = (uint32_t)args.ldd * 2u;
     const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc((void *)((unsigned short *)args.d + kept0 * args.ldd), 0, 0x7ffffff0, 0x00020000);
-    Sum run = 0;              // of the rows of task `runOf` this lane has met since the last flush
-    uint32_t runOf = 0;
+    Sum run = 0;              // of the rows of task `runOf`, the one this half wave is in (the rows of a task are neighbours)
+    uint32_t runOf = (args.flags & GF_ROW_MASK) ? wn : 0u;
+    auto flush = [&]() {
+        const Sum s = half_sum64(run);
+        if (chunk == 31u) sums[runOf * 8u + w * 2u + lrow] = s;
+        run = 0;
+    };
 
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
@@ -250,7 +283,6 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
                 cur[j] = *(const v4i *)(st + wrow * 512 + ((chunk * 16) ^ (((wrow >> 2) & 1) << 7)));
                 d[j] = dst[wm * 32 * MB + mb * 32 + wrow];
                 if constexpr (I8) cur[j] += bv;
-                if (!colOk) d[j] = FX_SKIP;
             }
             if (args.accDump) {
 #pragma unroll
@@ -296,15 +328,16 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
             if (!store && args.checksum) {
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
-                    if ((d[j] & FX_KIND) == FX_SUM) {
+                    if ((d[j] & FX_KIND) == FX_SUM) {   // (the same for the 32 lanes of a row)
                         const uint32_t g = (args.flags & GF_ROW_MASK) ? wn : (d[j] & FX_INDEX);
                         if (g != runOf) {
-                            if (run != 0) __hip_atomic_fetch_add(sums + runOf, run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                            run = 0;
+                            flush();
                             runOf = g;
                         }
-                        if constexpr (I8) run += ((long long)cur[j].x + cur[j].y) + ((long long)cur[j].z + cur[j].w);
-                        else run += ((double)i2f(cur[j].x) + (double)i2f(cur[j].y)) + ((double)i2f(cur[j].z) + (double)i2f(cur[j].w));
+                        Sum v;
+                        if constexpr (I8) v = ((long long)cur[j].x + cur[j].y) + ((long long)cur[j].z + cur[j].w);
+                        else v = ((double)i2f(cur[j].x) + (double)i2f(cur[j].y)) + ((double)i2f(cur[j].z) + (double)i2f(cur[j].w));
+                        run += colOk ? v : (Sum)0;
                     }
             }
             if constexpr (I8) {   // dequantise: per-channel scale first, then per-token, each product rounded on its own
@@ -331,7 +364,7 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
             if (store) {
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
-                    if ((d[j] & FX_KIND) == FX_OUT)
+                    if (colOk && (d[j] & FX_KIND) == FX_OUT)
                         __builtin_nontemporal_store(cur[j], (v4i *)((float *)args.outbound + (size_t)(d[j] & FX_INDEX) * args.sched.n0 + lcol));
             }
             if (kN != 0 && !late && !(args.flags & GF_KEPT_INT32_ONLY)) {   // (wave-uniform)
@@ -354,37 +387,23 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
         }
     }
     if (!store && args.checksum) {
-        if (run != 0) __hip_atomic_fetch_add(sums + runOf, run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        flush();
         __syncthreads();
+        auto total = [&](uint32_t g) {
+            Sum s = 0;
+            for (uint32_t i = 0; i < 8u; ++i) s += sums[g * 8u + i];
+            return s;
+        };
         if (args.flags & GF_ROW_MASK) {
             const uint32_t cols128 = ceil_div(args.N, 128u);
-            if (tid < 2 && t.col0 / 128u + tid < cols128) ((Sum *)args.checksum)[(size_t)(t.row0 / 128u) * cols128 + t.col0 / 128u + tid] = sums[tid];
+            if (tid < 2 && t.col0 / 128u + tid < cols128) ((Sum *)args.checksum)[(size_t)(t.row0 / 128u) * cols128 + t.col0 / 128u + tid] = total(tid);
         } else {
             // task g of the tile (the only one when row tiles are tile rows of the schedule): its first row says whether it is
             // one of the others', and only then sumTask[g] was written
             const uint32_t g = tid, first = g * args.sched.mRank;
-            if (g < (args.fx.perRank ? 1u : 16u) && first < t.rowsValid && (dst[first] & FX_KIND) == FX_SUM) ((Sum *)args.checksum)[sumTask[g]] = sums[g];
+            if (g < (args.fx.perRank ? 1u : 16u) && first < t.rowsValid && (dst[first] & FX_KIND) == FX_SUM) ((Sum *)args.checksum)[sumTask[g]] = total(g);
         }
     }
-}
-
-// Sum over the 64 lanes of a wave, in lane 63: cross-lane adds in the vector unit (a shuffle is a trip through the LDS unit).
-template <int CTRL, int ROWS>
-__device__ __forceinline__ long long dpp_add64(long long v)
-{
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), CTRL, ROWS, 0xf, false);
-    return v + (long long)(((unsigned long long)(uint32_t)hi << 32) | (uint32_t)lo);
-}
-__device__ __forceinline__ long long wave_sum64(long long v)
-{
-    v = dpp_add64<0x111, 0xf>(v);   // row_shr:1, 2, 4, 8: lane 15 of every row of 16 holds the row's sum
-    v = dpp_add64<0x112, 0xf>(v);
-    v = dpp_add64<0x114, 0xf>(v);
-    v = dpp_add64<0x118, 0xf>(v);
-    v = dpp_add64<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
-    v = dpp_add64<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
-    return v;
 }
 
 // ---- k slices --------------------------------------------------------------------------------------------------------------
@@ -443,10 +462,10 @@ __device__ __forceinline__ void flex_store_partial(const GemmArgs &args, Acc (&a
             if (kLo >= kHi) return;
         }
     }
-    // checksums: the second launch adds to them row by row
-    if (!args.fx.keptOnly && slice == 0 && args.checksum != nullptr && !(args.flags & GF_OUTBOUND_STORE) && (uint32_t)tid < t.rowsValid) {
+    // checksums of whole numbers: the second launch adds to them (sums of floats are added up by a third, in row order)
+    if (std::is_same<Acc, v16i>::value && !args.fx.keptOnly && slice == 0 && args.checksum != nullptr && !(args.flags & GF_OUTBOUND_STORE) && (uint32_t)tid < t.rowsValid) {
         const uint32_t v = t.row0 + tid;
-        long long *sum = (long long *)args.checksum;   // (zero in either type)
+        long long *sum = (long long *)args.checksum;
         if (args.flags & GF_ROW_MASK) {
             const uint32_t cols128 = ceil_div(args.N, 128u), c = t.col0 / 128u;
             sum[(size_t)(v / 128u) * cols128 + c] = 0;
@@ -484,9 +503,6 @@ __device__ __forceinline__ void flex_store_partial(const GemmArgs &args, Acc (&a
         }
     }
 }
-
-__device__ __forceinline__ void add_sum(unsigned long long *to, unsigned long long v) { atomicAdd(to, v); }
-__device__ __forceinline__ void add_sum(double *to, double v) { unsafeAtomicAdd(to, v); }
 
 // Workgroup (ct, y): columns [256 ct, +256) of rows [rowsPer * y, +rowsPer).  A wave takes one row at a time (everything about
 // the row is wave-uniform), a lane four columns of it: partials and peers are 1 KiB per wave instruction, all of them
@@ -531,8 +547,10 @@ __global__ void __launch_bounds__(256) flex_finish_kernel(const GemmArgs args, c
             }
         }
     }
-    // A task's rows add to one address, one atomic after the other (0.15 us each): the waves of a workgroup meet in LDS first.
-    // bf16 reduce-scatter 504x4112x1024, eight ranks, an atomic per row / per workgroup: 32.3 / 24.5 us.
+    // Checksums of whole numbers: a task's rows add to one address, one atomic after the other (0.15 us each), so the waves of a
+    // workgroup meet in LDS first (504x4112x1024, eight ranks, an atomic per row / per workgroup: 32.3 / 24.5 us).  Floats
+    // are not added in order of arrival: a row's sum takes the place of the row's partial sums, which nobody reads again, for
+    // flex_sums_kernel.
     __shared__ Sum waveSum[4];
     __shared__ uint32_t waveTask[4];
     Sum run = 0;
@@ -583,17 +601,22 @@ __global__ void __launch_bounds__(256) flex_finish_kernel(const GemmArgs args, c
                 }
 #pragma unroll
                 for (int o = 16; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-                Sum *to = (Sum *)args.checksum;
-                if (rowMask) {   // one sum per 128 columns
-                    if ((lane & 31) == 0 && colOk) add_sum(to + (size_t)(v / 128u) * ceil_div(args.N, 128u) + gcol / 128u, s);
+                if constexpr (I8) {
+                    Sum *to = (Sum *)args.checksum;
+                    if (rowMask) {   // one sum per 128 columns
+                        if ((lane & 31) == 0 && colOk) atomicAdd(to + (size_t)(v / 128u) * ceil_div(args.N, 128u) + gcol / 128u, s);
+                    } else {
+                        s += __shfl_xor(s, 32, 64);
+                        if (task != runOf) {
+                            if (lane == 0 && runOf != 0xffffffffu) atomicAdd(to + runOf, run);
+                            run = 0;
+                            runOf = task;
+                        }
+                        run += s;
+                    }
                 } else {
                     s += __shfl_xor(s, 32, 64);
-                    if (task != runOf) {
-                        if (lane == 0 && runOf != 0xffffffffu) add_sum(to + runOf, run);
-                        run = 0;
-                        runOf = task;
-                    }
-                    run += s;
+                    if (lane == 0) *(double *)(args.skPart + (size_t)(v - first) * args.N + gcol) = s;   // (8 bytes of at least 16)
                 }
             }
             if (store && colOk) {
@@ -638,7 +661,7 @@ __global__ void __launch_bounds__(256) flex_finish_kernel(const GemmArgs args, c
         for (int e = 0; e < 4; ++e) q[e] = f32_to_out16(i2f(cur[e]), args.outDtype) & 0xffffu;
         *(v2i *)((unsigned short *)args.d + (size_t)(v - args.keptBegin) * args.ldd + gcol) = v2i{(int)(q[0] | (q[1] << 16)), (int)(q[2] | (q[3] << 16))};
     }
-    if (sums && !rowMask) {
+    if (I8 && sums && !rowMask) {
         if (lane == 0) {
             waveSum[w] = run;
             waveTask[w] = runOf;
@@ -653,9 +676,32 @@ __global__ void __launch_bounds__(256) flex_finish_kernel(const GemmArgs args, c
                     if (i < threadIdx.x) firstOf = false;
                     all += waveSum[i];
                 }
-            if (firstOf) add_sum((Sum *)args.checksum + mine, all);
+            if constexpr (I8) {
+                if (firstOf) atomicAdd((Sum *)args.checksum + mine, all);
+            }
         }
     }
+}
+
+// Checksums of float launches in k slices: workgroup b * colTiles + ct, one wave, is the task of column tile ct in tile row b of
+// all ranks' tile rows, and adds the sums of its rows (at most 128) that flex_finish_kernel left in slice 0, always in the same
+// order.
+// A launch more than adding in order of arrival in flex_finish_kernel, whose last bits differ from launch to launch; bf16, eight
+// ranks, us: 504x4112x1024 21.2 / 23.5, 88x1024x4096 13.8 / 15.0, 64x4096x8192 23.1 / 26.2.
+template <uint32_t DT>
+__global__ void __launch_bounds__(64) flex_sums_kernel(const GemmArgs args)
+{
+    const SchedParams &sp = args.sched;
+    const uint32_t b = blockIdx.x / args.fx.colTiles, ct = blockIdx.x - b * args.fx.colTiles, rank = b / sp.loopsM, mi = b - rank * sp.loopsM;
+    const uint32_t row0 = rank * sp.mRank + mi * sp.m0, rows = umin(sp.m0, sp.mRank - mi * sp.m0);
+    if (row0 - args.keptBegin < args.keptRows) return;
+    const int32_t *from = args.skPart + (size_t)row0 * args.N + ct * 256u;
+    double s = 0;
+    for (uint32_t r = threadIdx.x; r < rows; r += 64u) s += *(const double *)(from + (size_t)r * args.N);
+    uint32_t task, ws;
+    flex_task_of(sp, rank, mi * sp.m0, ct, task, ws);
+    s = wave_sum64(s);
+    if (threadIdx.x == 63) ((double *)args.checksum)[task] = s;
 }
 
 }  // namespace catcoc

@@ -368,3 +368,47 @@ def test_workspace_past_the_queried_bytes_is_not_touched(case, tb):
         assert bool((ws[end:] == 0x55).all()) and not ws[:65536].any()
         got.append(out.clone())
     assert torch.equal(got[0].view(torch.int16), got[1].view(torch.int16))
+
+
+# (rows per rank, N, K, P, m0, ranks' tasks): several tasks in one tile (also with kept rows in its middle), tasks that cross from one
+# wave's rows to the next, one task per tile, several tile rows per rank, k slices (a second launch) with all of these
+@pytest.mark.parametrize("dtype", [oracle.FP16, oracle.BF16])
+@pytest.mark.parametrize("case", [(11, 300, 200, 8, 0, 0), (1, 260, 132, 16, 0, 0), (63, 1028, 196, 4, 0, 0), (125, 516, 100, 8, 0, 0), (300, 516, 100, 4, 0, 0),
+                                  (200, 300, 320, 2, 64, 0), (63, 512, 4112, 8, 0, 0), (11, 300, 200, 8, 0, 3), (150, 296, 4104, 4, 0, 0), (200, 300, 320, 2, 64, 2),
+                                  (1, 260, 132, 16, 0, 2)])
+def test_float_checksums_are_reproducible(case, dtype):
+    """Checksums of float tiles: the sums of the dumped partials (64-bit sums in any order: 2^-52 of the magnitudes per addition),
+    and the same bits in every launch.  Rows and columns differ in size by up to 2^20, so that these sums are not exact."""
+    _need_gpu()
+    rows, N, K, P, m0, slices = case
+    M, rank = rows * P, P // 2
+    g = torch.Generator(device="cuda:0").manual_seed(rows)
+    size = lambda *shape: torch.exp2(-torch.randint(0, 11, shape, device="cuda:0", generator=g).float())
+    A = (torch.randn((M, K), device="cuda:0", generator=g) * size(M, 1)).to(TORCH_DT[dtype])
+    B = (torch.randn((K, N), device="cuda:0", generator=g) * size(1, N)).to(TORCH_DT[dtype])
+    peers = [torch.randn((rows, N), device="cuda:0", generator=g) for _ in range(P - 1)]
+    t = ops.default_tiling(M, K, N, P, m0=m0, n0=0, k0=0)
+    d = L.make_desc(rank, P, [16] * (P - 1))
+    tasks = L.load().catcoc_get_task_count(L.MATMUL_REDUCE_SCATTER, C.byref(t), C.byref(d))
+    need, f = ops.kslice_plan(L.MATMUL_REDUCE_SCATTER, TORCH_DT[dtype], M, K, N, rank, P, tiling=t, split_k=slices)
+    assert f == slices or (slices == 0 and (f > 1) == (K > 4000))
+    ws = torch.zeros(max(need, 65536), dtype=torch.uint8, device="cuda:0")
+    dump = torch.zeros((M, N), dtype=torch.float32, device="cuda:0")
+    seen = []
+    for _ in range(12):
+        cs = torch.full((tasks,), 77.0, dtype=torch.float64, device="cuda:0")
+        ops.matmul_reduce_scatter(A, B, peers, rank, P, tiling=t, checksum=cs, acc_dump=dump, workspace=ws, split_k=slices)
+        torch.cuda.synchronize()
+        seen.append(cs.cpu().numpy().view(np.int64))
+    part = dump.cpu().numpy().astype(np.float64)
+    step = m0 or (64 if rows <= 64 else 128)
+    tr, row, col = C.c_uint32(), C.c_uint32(), C.c_uint32()
+    for task in range(tasks):
+        L.load().catcoc_task_tile(L.MATMUL_REDUCE_SCATTER, C.byref(t), C.byref(d), task, C.byref(tr), C.byref(row), C.byref(col), None)
+        blk = part[row.value:min(row.value + step, (tr.value + 1) * rows), col.value:min(col.value + 256, N)]
+        got = seen[0].view(np.float64)[task]
+        if tr.value == rank:
+            assert got == 77.0, task
+        else:
+            assert abs(got - blk.sum()) <= 2 * blk.size * 2.0 ** -52 * np.abs(blk).sum(), task
+    assert all(np.array_equal(s, seen[0]) for s in seen[1:])
