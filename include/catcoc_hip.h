@@ -304,14 +304,17 @@ CATCOC_API uint64_t catcoc_get_workspace_size(int commType, int dataType, const 
 /* Launches with few 128x256 tiles (fewer than half the CUs' worth) can cut every tile's k range into k slices, one
  * workgroup each, that meet through `workspace` (partial tiles in 32-bit words + one counter per tile, zeroed once
  * by the caller, re-armed by every launch): returns the bytes needed and the slice count (1 and 0 bytes when the
- * launch would not be sliced: enough tiles already, or a k too short; the operands' layouts do not matter).  The count
- * is 2, 4 or 8 for W8A8 (integer partials add exactly) and 2 for fp16/bf16, or any up to 64 for launches that fill no 128x256
- * tiles; with few tiles and a long k the bytes are those of more slices than that, which such a launch takes where its tiles run
- * in flexible mode (a smaller workspace, down to the reported count's 128x256 partial tiles, serves too).  A count of one with some bytes: a reduce-scatter launch whose kept rows meet their peers in a
- * second launch when it is given them.  desc->splitK, when non-zero, is taken as the
- * caller's own count (up to 8; three or more fp32 partials are added in slice order whichever slice arrives last, so
- * the result is reproducible for any count).  A launch
- * slices only when `workspace` is given.  Counterpart in the reference: SplitkMatmul's k split
+ * launch would not be sliced: enough tiles already, or a k too short; the operands' layouts do not matter).
+ *  - Launches of full 128x256 tiles: the count is 2, 4 or 8 for W8A8 (integer partials add exactly) and 2 for fp16/bf16.  With
+ *    few tiles and a long k the bytes are those of more slices than that, which the launch takes where its tiles run in
+ *    flexible mode (64-row tiles that need not line up with ranks; a smaller workspace, down to the reported count's
+ *    128x256 partial tiles, serves too).  desc->splitK, when non-zero, is taken as the caller's own count, up to 8.
+ *  - Ragged launches of few tiles run flexible tiles in any count up to 64; desc->splitK, when 2 or more, is the caller's own
+ *    count (no more than there are k steps).  A smaller workspace runs the slices that fit into it, none runs whole tiles.
+ *  - A count of one with some bytes: a reduce-scatter launch whose kept rows meet their peers in a second launch when it is
+ *    given them.
+ * Float partials are added in slice order, so results are reproducible for any count.  A launch slices only when
+ * `workspace` is given.  Counterpart in the reference: SplitkMatmul's k split
  * (3rdparty/catlass/include/catlass/gemm/kernel/splitk_matmul.hpp:68-148), which its communication kernels do not
  * use. */
 CATCOC_API uint64_t catcoc_get_kslice_workspace_size(int commType, int dataType, const CocTilingParams *tiling,

@@ -461,15 +461,16 @@ int make_plan(int commType, int dataType, const CocTilingParams *t, const Catcoc
         plan.kSlices = c.slices;
         plan.kSliceBytes = c.bytes;
         plan.flexBlocks = flex_use(a, es, t->m0, c, d->workspace, d->workspaceBytes);
-    } else if (m0 == 128 && t->m0 == 0 && d->splitK == 0 && (d->flags & tuning) == 0 && fewTiles && !transA &&
+    } else if (m0 == 128 && t->m0 == 0 && (d->splitK == 0 || (plan.edge && d->splitK > 1)) && (d->flags & tuning) == 0 && fewTiles && !transA &&
                !(op == OP_REDUCE_SCATTER && P > 1 && a.checksum != nullptr)) {
         // What a workspace takes is said for the aligned kernel, and this one uses the slices that fit into that, unless it would
         // take four or more: all-reduce of 257x14336x512, bf16, seven peers, in 64 KiB of workspace (no slices) / in what its slices
         // take: 156 / 21 us; 306x13824x2048 147 / 41; reduce-scatter 832x15232x800 of four ranks with stored tiles 157 / 52.
         // (Rows of B that end inside a 16-byte piece have an aligned kernel as [n,k] only: the query speaks of flexible tiles.)
-        const FlexSlices c = flex_choose(a, es, 0, 0);
+        // Ragged rows or columns have k slices here only, so a caller's own count of them is for this kernel.
+        const FlexSlices c = flex_choose(a, es, 0, d->splitK);
         plan.preferFlex = c.whole != 0;
-        if (plan.preferFlex && ((c.slices >= 4 && c.bytes > plan.kSliceBytes) || ((uint64_t)t->n * es) % 16 != 0)) {
+        if (plan.preferFlex && ((c.slices >= 4 && c.bytes > plan.kSliceBytes) || ((uint64_t)t->n * es) % 16 != 0 || d->splitK > 1)) {
             if (plan.kSlices == 1) plan.kSlices = c.slices;   // (the aligned kernel's count is what launches with A as [k,m] run)
             plan.kSliceBytes = c.bytes;
         }

@@ -592,3 +592,15 @@ def test_kept_split_choice_by_tile_count_and_k_length():
     assert split(RS, L.FP16, 8 * 296, 512, 1344, 8) == 0              # ragged problems keep whole tiles
     assert split(L.MATMUL_ALLREDUCE, L.FP16, 1024, 512, 1024, 2) == 0 # no kept-rank block to split
     assert split(Q, L.INT8, 4096, 1792, 4096, 1) == 0                 # no peers to stream
+
+
+def test_ragged_slice_count_is_accepted_as_the_callers_own(so):
+    # the count and the bytes the query reports for a ragged launch are what it reports when the count is passed back as desc.splitK
+    from mm_rs_with_catlass_amd import ops
+    import torch
+    for comm, dt, m, k, n, p in ((L.MATMUL_ALLREDUCE, torch.bfloat16, 257, 14336, 512, 8), (L.MATMUL_ALLREDUCE, torch.float16, 300, 2048, 1032, 2),
+                                 (L.QUANT_MATMUL_REDUCE_SCATTER, torch.int8, 600, 8192, 272, 4), (L.MATMUL_REDUCE_SCATTER, torch.bfloat16, 600, 4096, 296, 4)):
+        need, f = ops.kslice_plan(comm, dt, m, k, n, 0, p)
+        assert f > 1 and ops.kslice_plan(comm, dt, m, k, n, 0, p, split_k=f) == (need, f)
+        assert ops.kslice_plan(comm, dt, m, k, n, 0, p, split_k=2) == (65536 + 2 * m * n * 4, 2)
+        assert ops.kslice_plan(comm, dt, m, k, n, 0, p, split_k=1)[1] == 1

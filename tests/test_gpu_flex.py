@@ -412,3 +412,22 @@ def test_float_checksums_are_reproducible(case, dtype):
         else:
             assert abs(got - blk.sum()) <= 2 * blk.size * 2.0 ** -52 * np.abs(blk).sum(), task
     assert all(np.array_equal(s, seen[0]) for s in seen[1:])
+
+
+# (rows, N, K, P): ragged rows, ragged columns, whole k steps: the aligned kernels take these launches whole, their slices are flexible
+@pytest.mark.parametrize("case", [(257, 512, 4096, 8), (300, 1032, 2048, 2)])
+def test_ragged_launch_takes_the_slice_count_its_query_reports(case):
+    _need_gpu()
+    M, N, K, P = case
+    g = torch.Generator(device="cuda:0").manual_seed(M)
+    A, B = torch.randn((M, K), device="cuda:0", generator=g).bfloat16(), torch.randn((K, N), device="cuda:0", generator=g).bfloat16()
+    peers = [torch.randn((M, N), device="cuda:0", generator=g) for _ in range(P - 1)]
+    need, f = ops.kslice_plan(L.MATMUL_ALLREDUCE, torch.bfloat16, M, K, N, 0, P)
+    outs = []
+    for sk in (0, f):
+        ws = torch.zeros(need, dtype=torch.uint8, device="cuda:0")
+        out = ops.matmul_allreduce(A, B, peers, 0, P, workspace=ws, split_k=sk)
+        torch.cuda.synchronize()
+        assert f > 1 and bool(ws[65536:].any())
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])
