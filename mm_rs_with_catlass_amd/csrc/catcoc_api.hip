@@ -1319,7 +1319,7 @@ uint32_t catcoc_kept_split_tiles(int commType, int dataType, const CocTilingPara
     for (int i = 0; i < CATCOC_MAX_RANKS; ++i) if (!d.peers[i]) d.peers[i] = (const void *)16;
     if (make_plan(commType, dataType, tiling, &d, transA, transB, p)) return 0;
     ok();
-    if (!p.dma || p.args.sched.m0 != 128) return 0;
+    if (!p.dma || p.preferFlex || p.args.sched.m0 != 128) return 0;   // (flexible tiles are never split)
     return 8u * split_kept_tiles(p.args, p.args.K * elem_size(p.dtype) / 64u);
 }
 
@@ -1333,7 +1333,7 @@ uint32_t catcoc_tail_split_tiles(int commType, int dataType, const CocTilingPara
     for (int i = 0; i < CATCOC_MAX_RANKS; ++i) if (!d.peers[i]) d.peers[i] = (const void *)16;
     if (make_plan(commType, dataType, tiling, &d, transA, transB, p)) return 0;
     ok();
-    if (!p.dma || p.args.sched.m0 != 128) return 0;
+    if (!p.dma || p.preferFlex || p.args.sched.m0 != 128) return 0;   // (flexible tiles are never split)
     return 8u * split_tail_tiles(p.args, split_kept_tiles(p.args, p.args.K * elem_size(p.dtype) / 64u));
 }
 

@@ -604,3 +604,14 @@ def test_ragged_slice_count_is_accepted_as_the_callers_own(so):
         assert f > 1 and ops.kslice_plan(comm, dt, m, k, n, 0, p, split_k=f) == (need, f)
         assert ops.kslice_plan(comm, dt, m, k, n, 0, p, split_k=2) == (65536 + 2 * m * n * 4, 2)
         assert ops.kslice_plan(comm, dt, m, k, n, 0, p, split_k=1)[1] == 1
+
+
+def test_kept_split_queries_of_launches_on_flexible_tiles(so):
+    # few tiles and a short k run flexible tiles, which are never split, unless the launch takes checksums or is told its order
+    from mm_rs_with_catlass_amd import ops
+    for comm, dt, m, k, n in ((L.QUANT_MATMUL_REDUCE_SCATTER, L.INT8, 1024, 1792, 4096), (L.MATMUL_REDUCE_SCATTER, L.FP16, 1024, 1024, 4096)):
+        t = ops.default_tiling(m, k, n, 8, m0=0, n0=0, k0=0)
+        for checksum, flags, want in ((0, 0, 0), (4096, 0, n // 256), (0, L.FLAG_KEPT_SPLIT, n // 256), (0, L.FLAG_KEPT_WHOLE, 0)):
+            d = L.make_desc(0, 8, [16] * 7, flags=flags, checksum=checksum)
+            assert so.catcoc_kept_split_tiles(comm, dt, C.byref(t), C.byref(d), 0, 1) == want
+            assert so.catcoc_tail_split_tiles(comm, dt, C.byref(t), C.byref(d), 0, 1) == 0
