@@ -220,11 +220,19 @@ def make_desc(rank, rank_size, peers=(), peer_ld=0, peer_row_offset=0, flags=0, 
               swizzle=None, outbound=None, outbound_bytes=0, checksum=None, acc_dump=None):
     """Build a CatcocSymmetricDesc from raw device addresses (ints)."""
     off, direction = swizzle if swizzle is not None else (0, 0)
-    peers = [p or 0 for p in peers]
-    if len(peers) > MAX_RANKS:
+    addresses = [p or 0 for p in peers]
+    if len(addresses) > MAX_RANKS:
         raise IndexError("at most %d peers" % MAX_RANKS)
-    # (packed in one go: setting thirty fields one by one takes 4 us)
     u32 = 0xffffffff
-    return CatcocSymmetricDesc.from_buffer_copy(_DESC.pack(
-        DESC_MAGIC, rank & u32, rank_size & u32, block_num & u32, stages & u32, off & u32, direction & u32, flags & u32, 0, 0, 0,
-        *peers, *_NO_PEERS[len(peers):], peer_ld, peer_row_offset, outbound or 0, outbound_bytes, checksum or 0, acc_dump or 0, 0, 0, 0))
+    try:   # (packed in one go: setting thirty fields one by one takes 4 us)
+        return CatcocSymmetricDesc.from_buffer_copy(_DESC.pack(
+            DESC_MAGIC, rank & u32, rank_size & u32, block_num & u32, stages & u32, off & u32, direction & u32, flags & u32, 0, 0, 0,
+            *addresses, *_NO_PEERS[len(addresses):], peer_ld, peer_row_offset, outbound or 0, outbound_bytes, checksum or 0, acc_dump or 0,
+            0, 0, 0))
+    except (struct.error, TypeError):   # ctypes objects and negative numbers: what a field itself takes
+        d = CatcocSymmetricDesc(magic=DESC_MAGIC, rankIdx=rank, rankSize=rank_size, blockNum=block_num, workspaceStages=stages, swizzleOffset=off,
+                                swizzleDirection=direction, flags=flags, peerLd=peer_ld, peerRowOffset=peer_row_offset, outbound=outbound,
+                                outboundBytes=outbound_bytes, checksum=checksum, accDump=acc_dump)
+        for i, p in enumerate(addresses):
+            d.peers[i] = p
+        return d

@@ -615,3 +615,17 @@ def test_kept_split_queries_of_launches_on_flexible_tiles(so):
             d = L.make_desc(0, 8, [16] * 7, flags=flags, checksum=checksum)
             assert so.catcoc_kept_split_tiles(comm, dt, C.byref(t), C.byref(d), 0, 1) == want
             assert so.catcoc_tail_split_tiles(comm, dt, C.byref(t), C.byref(d), 0, 1) == 0
+
+
+def test_descriptor_takes_what_its_fields_take(so):
+    # plain addresses are packed in one go; ctypes objects and numbers outside a field's range as ctypes takes them
+    want = bytes(L.make_desc(3, 4, [16, 32, 48], peer_ld=8, outbound=64, outbound_bytes=128, checksum=256, acc_dump=512, flags=5))
+    got = L.make_desc(C.c_uint32(3), 4, [C.c_void_p(16), C.c_uint64(32).value, C.c_void_p(48)], peer_ld=8, outbound=C.c_void_p(64),
+                      outbound_bytes=C.c_uint64(128), checksum=C.c_void_p(256), acc_dump=C.c_void_p(512), flags=C.c_uint32(5))
+    assert bytes(got) == want
+    d = L.make_desc(0, 2, [-16], outbound=-4096, outbound_bytes=-1, peer_row_offset=1 << 63)
+    assert (d.peers[0], d.outbound, d.outboundBytes, d.peerRowOffset) == (2 ** 64 - 16, 2 ** 64 - 4096, 2 ** 64 - 1, -2 ** 63)
+    with pytest.raises(TypeError):
+        L.make_desc(0, 2, ["16"])
+    with pytest.raises(IndexError):
+        L.make_desc(0, 2, [16] * 17)
