@@ -26,6 +26,22 @@ def peers_of(rng, M, N, K, P, rank, ri):
     return [rng.standard_normal((rows, N)).astype(np.float32) for _ in range(P - 1)]
 
 
+def sum_bound(A, B, dtype):
+    """How far two fp32 sums of the same K products may be apart, per element: each is within 4 sqrt(K) 2^-24 |a||b| of the exact
+    sum (roundings of K additions that are independent, four standard deviations; sum |a_i b_i| <= |a||b|).  At K = 6148 that
+    is a tenth of what four products more or less make."""
+    a, b = oracle.half_to_f32(A, dtype), oracle.half_to_f32(B, dtype)
+    return 8 * np.sqrt(A.shape[1]) * 2.0 ** -24 * np.outer(np.linalg.norm(a, axis=1), np.linalg.norm(b, axis=0)) + 1e-9
+
+
+def tasks_of(comm, t, d):
+    """(task, target rank, first row, first column, workspace row) of every task of a launch."""
+    tr, row, col, ws = (C.c_uint32() for _ in range(4))
+    for task in range(L.load().catcoc_get_task_count(comm, C.byref(t), C.byref(d))):
+        L.load().catcoc_task_tile(comm, C.byref(t), C.byref(d), task, C.byref(tr), C.byref(row), C.byref(col), C.byref(ws))
+        yield task, tr.value, row.value, col.value, ws.value
+
+
 # (rows per rank, N, K, P, rank, weights as [n,k], int32 peers, m0, commInterval)
 @pytest.mark.parametrize("outbound", [False, True])
 @pytest.mark.parametrize("case", [(125, 512, 1376, 8, 5, True, False, 0, 1),     # one rank per tile; half a step of k left
@@ -119,9 +135,7 @@ def test_float_any_rows_any_k(dtype, case):
             again.append(host16(o))
         assert np.array_equal(again[0], again[1])
         _check_float(again[0], want, full, dtype, K)
-    # fp32 sums of K products in another order: each within K * 2^-24 of the sum of their magnitudes, here at most
-    # 4.5 * 4.5 * 0.02 * K per element (operands are normal, scales 1 and 0.02)
-    assert np.abs(dump.cpu().numpy() - part).max() <= K * 2.0 ** -24 * 0.41 * K + 1e-6
+    assert (np.abs(dump.cpu().numpy() - part) <= sum_bound(np.concatenate(shards, 0) if op == "allgather" else A, B, dtype)).all()
 
 
 @pytest.mark.parametrize("dtype", [oracle.FP16, oracle.BF16])
@@ -139,13 +153,13 @@ def test_float_reduce_scatter_checksums_of_small_ranks(dtype):
     _check_float(host16(out), want, part[rank * rows:(rank + 1) * rows] + sum(peers), dtype, K)
     t = ops.default_tiling(P * rows, K, N, P, m0=0, n0=0, k0=0)
     d = L.make_desc(rank, P, [16] * (P - 1))
+    bounds = sum_bound(A, B, dtype)
     tr, row, col = C.c_uint32(), C.c_uint32(), C.c_uint32()
     for task in range(2 * P):
         L.load().catcoc_task_tile(L.MATMUL_REDUCE_SCATTER, C.byref(t), C.byref(d), task, C.byref(tr), C.byref(row), C.byref(col), None)
-        blk = part[row.value:row.value + rows, col.value:min(col.value + 256, N)].astype(np.float64)
-        # (fp32 accumulation in another order: K * 2^-24 of the magnitudes per element, as above)
-        bound = blk.size * K * 2.0 ** -24 * 0.41 * K + 1e-6
-        assert abs(float(cs[task]) - (0.0 if tr.value == rank else blk.sum())) <= bound, task
+        at = np.s_[row.value:row.value + rows, col.value:min(col.value + 256, N)]
+        blk = part[at].astype(np.float64)
+        assert abs(float(cs[task]) - (0.0 if tr.value == rank else blk.sum())) <= bounds[at].sum(), task
 
 
 # (m, N, K, P, kept rows [begin, +count), weights as [n,k], int32 peers): kept rows that start, end or lie inside a 64-row tile,
@@ -167,7 +181,7 @@ def test_quant_kept_rows_in_slices(case):
     sums = np.array([[acc[r:r + 128, c:c + 128].astype(np.int64).sum() - acc[max(r, kb):max(min(r + 128, kb + kr), max(r, kb)), c:c + 128].astype(np.int64).sum()
                       for c in range(0, N, 128)] for r in range(0, M, 128)]).ravel()
     x2d = dev(np.ascontiguousarray(x2.T) if tb else x2)
-    for extra in (0, 1 << 20):   # as many slices as the query's workspace holds, and more
+    for extra in (0, 1 << 20):   # the query's workspace, and a larger one, whose rest stays as it was
         ws = torch.zeros(max(need, 65536) + extra, dtype=torch.uint8, device="cuda:0")
         ws[65536:] = 0x55
         cs = torch.full((tiles,), -7, dtype=torch.int64, device="cuda:0") if kr < M else None
@@ -176,6 +190,8 @@ def test_quant_kept_rows_in_slices(case):
                                       c_accum=ca, trans_b=tb, reduce_int32=ri)
         torch.cuda.synchronize()
         assert np.array_equal(host16(out), want) and not ws[:65536].any()
+        assert need == 0 or K < 512 or bool((ws[65536:need] != 0x55).any())   # (slices did run; eight k steps make two of them)
+        assert bool((ws[max(need, 65536):] == 0x55).all())
         assert np.array_equal(ca.cpu().numpy(), acc[kb:kb + kr] + (sum(peers) if ri else 0))
         if cs is not None:
             assert np.array_equal(cs.cpu().numpy(), sums)
@@ -223,6 +239,7 @@ def test_float_reduce_scatter_ragged_few_tiles_long_k():
     tr, row, col, wsr = (C.c_uint32() for _ in range(4))
     tasks = L.load().catcoc_get_task_count(L.MATMUL_REDUCE_SCATTER, C.byref(t), C.byref(d))
     size = L.load().catcoc_get_workspace_size(L.MATMUL_REDUCE_SCATTER, L.FP16, C.byref(t), C.byref(d))
+    bounds = sum_bound(A, B, oracle.FP16)
     for ws in (torch.zeros(need, dtype=torch.uint8, device="cuda:0"), None):
         ob = torch.full((size // 4,), 3.0, dtype=torch.float32, device="cuda:0")
         out = ops.matmul_reduce_scatter(dev16(A, oracle.FP16), dev16(np.ascontiguousarray(B.T), oracle.FP16), [dev(p) for p in peers], rank, P, tiling=t,
@@ -235,7 +252,7 @@ def test_float_reduce_scatter_ragged_few_tiles_long_k():
                 continue
             r1, c1 = min(row.value + 128, (tr.value + 1) * rows), min(col.value + 256, N)
             got = ob.cpu().numpy().reshape(-1, 256)[wsr.value:wsr.value + r1 - row.value, :c1 - col.value]
-            assert np.abs(got - part[row.value:r1, col.value:c1]).max() <= K * 2.0 ** -24 * 0.41 * K + 1e-6, task   # (as in the tests above)
+            assert (np.abs(got - part[row.value:r1, col.value:c1]) <= bounds[row.value:r1, col.value:c1]).all(), task
 
 
 # (rows per rank, N, K, P, rank, weights as [n,k]): one-round pipelined calls on ragged columns, ragged rows, and few aligned tiles
@@ -291,6 +308,7 @@ def test_reduce_scatter_peers_in_a_second_launch(case, outbound):
     flip = lambda w: np.ascontiguousarray(w.T) if tb else w
     dp = [dev(p) for p in peers]
     A, B = _rand16(rng, (M, K), oracle.FP16), _rand16(rng, (K, N), oracle.FP16, 0.02)
+    bounds = sum_bound(A, B, oracle.FP16)
     for quant in (True, False) if not ri else (True,):
         need, f = ops.kslice_plan(L.QUANT_MATMUL_REDUCE_SCATTER if quant else L.MATMUL_REDUCE_SCATTER, torch.int8 if quant else torch.float16, M, K, N, rank, P, tiling=t)
         assert (need, f) == (65536 + rows * N * 4, 1) or f > 1
@@ -309,13 +327,20 @@ def test_reduce_scatter_peers_in_a_second_launch(case, outbound):
             else:
                 out = ops.matmul_reduce_scatter(dev16(A, oracle.FP16), dev16(flip(B), oracle.FP16), dp, rank, P, acc_dump=dump, **kw)
                 torch.cuda.synchronize()
+                part, fwant = oracle.matmul_reduce(A, B, oracle.FP16, rank * rows, rows, peers, want_partial=True)
+                _check_float(host16(out), fwant, part[rank * rows:(rank + 1) * rows] + sum(peers), oracle.FP16, K)
+                assert (np.abs(dump.cpu().numpy() - part) <= bounds).all()
+                for task, target, r0, c0, w0 in tasks_of(L.MATMUL_REDUCE_SCATTER, t, d):
+                    at = np.s_[r0:min(r0 + (64 if rows <= 64 else 128), (target + 1) * rows), c0:min(c0 + 256, N)]
+                    own = dump.cpu().numpy()[at]
+                    if target != rank and outbound:
+                        assert np.array_equal(kw["outbound"].cpu().numpy().reshape(-1, 256)[w0:w0 + own.shape[0], :own.shape[1]], own), task
+                    elif target != rank:
+                        assert abs(float(kw["checksum"][task]) - own.sum(dtype=np.float64)) <= own.size * 2.0 ** -51 * np.abs(own).sum(), task
             assert ws is None or (not ws[:65536].any() and bool(ws[65536:].any()))
             got.append([out, dump, kw.get("outbound", kw.get("checksum"))])
         for with_ws, without in zip(*got):
-            if with_ws.dtype == torch.float64:   # (64-bit sums of a tile meet in any order: 2^-52 of 2^15 magnitudes of at most 0.41 * K)
-                assert float((with_ws - without).abs().max()) <= 2.0 ** -37 * 0.41 * K
-            else:
-                assert torch.equal(with_ws, without)
+            assert torch.equal(with_ws, without)
 
 
 # (kind, rows, N, K, P, kept rows or 0): launches whose flexible tiles would take k slices, or a second launch for the peers, that
@@ -431,3 +456,208 @@ def test_ragged_launch_takes_the_slice_count_its_query_reports(case):
         assert f > 1 and bool(ws[65536:].any())
         outs.append(out)
     assert torch.equal(outs[0], outs[1])
+
+
+# (rows per rank, N, K, P, rank, weights as [n,k], int32 peers, slices: 1 = peers in a second launch, swizzle)
+@pytest.mark.parametrize("outbound", [False, True])
+@pytest.mark.parametrize("case", [(125, 516, 1376, 8, 5, True, False, 1, (3, 0)), (125, 516, 1376, 8, 5, False, False, 3, (2, 1)), (40, 260, 516, 4, 1, False, True, 3, (1, 0)),
+                                  (200, 1028, 260, 8, 2, True, True, 1, (2, 0)), (200, 772, 260, 8, 7, False, True, 4, (3, 1))])
+def test_two_launches_with_a_window_of_the_peers_and_other_swizzles(case, outbound):
+    """k slices and the peers' second launch: peers that are wider than n and start at a row of their own, other swizzles of the
+    schedule, dumps and int32 sums."""
+    _need_gpu()
+    rows, N, K, P, rank, tb, ri, slices, swizzle = case
+    M, off, step = rows * P, 5, 64 if rows <= 64 else 128
+    rng = np.random.default_rng(rows + K + slices)
+    x1, x2 = rng.integers(-127, 128, (M, K), dtype=np.int8), rng.integers(-127, 128, (K, N), dtype=np.int8)
+    s1, s2 = rng.uniform(0.005, 0.02, M).astype(np.float32), rng.uniform(0.001, 0.01, N).astype(np.float32)
+    b = rng.integers(-1000, 1000, N, dtype=np.int32)
+    wide = [rng.integers(-2 ** 24, 2 ** 24, (rows + off + 2, N + 12), dtype=np.int32) if ri else rng.standard_normal((rows + off + 2, N + 12)).astype(np.float32)
+            for _ in range(P - 1)]
+    peers = [np.ascontiguousarray(p[off:off + rows, :N]) for p in wide]
+    t = ops.default_tiling(M, K, N, P, m0=0, n0=0, k0=0)
+    flip = lambda w: np.ascontiguousarray(w.T) if tb else w
+    for quant in (True,) if ri else (True, False):
+        comm = L.QUANT_MATMUL_REDUCE_SCATTER if quant else L.MATMUL_REDUCE_SCATTER
+        d = L.make_desc(rank, P, [16] * (P - 1), swizzle=swizzle)
+        tasks = list(tasks_of(comm, t, d))
+        size = L.load().catcoc_get_workspace_size(comm, L.INT8 if quant else L.BF16, C.byref(t), C.byref(d)) // 4
+        kw = {"outbound": torch.full((size,), 3, dtype=torch.int32 if ri else torch.float32, device="cuda:0")} if outbound else \
+             {"checksum": torch.full((len(tasks),), 77, dtype=torch.int64 if quant else torch.float64, device="cuda:0")}
+        ws = torch.zeros(65536 + (rows if slices == 1 else M * slices) * N * 4, dtype=torch.uint8, device="cuda:0")
+        dump = torch.zeros((M, N), dtype=torch.int32 if quant else torch.float32, device="cuda:0")
+        kw.update(tiling=t, trans_b=tb, workspace=ws, split_k=slices, swizzle=swizzle, peer_row_offset=off, acc_dump=dump)
+        own = np.s_[rank * rows:(rank + 1) * rows]
+        if quant:
+            acc, want = oracle.quant_matmul_reduce_scatter(x1, x2, s1, s2, b, rank * rows, rows, peers, oracle.BF16, reduce_int32=ri)
+            ca = torch.full((rows, N), -7, dtype=torch.int32, device="cuda:0")
+            out = ops.quant_matmul_reduce_scatter(dev(x1), dev(flip(x2)), dev(s1), dev(s2), dev(b), [dev(p) for p in wide], rank, P, reduce_int32=ri, c_accum=ca, **kw)
+            torch.cuda.synchronize()
+            assert np.array_equal(host16(out), want) and np.array_equal(dump.cpu().numpy(), acc)
+            assert np.array_equal(ca.cpu().numpy(), acc[own] + (sum(peers) if ri else 0))
+            tiles = acc if ri or not outbound else oracle.dequant(acc, s2, s1)
+        else:
+            A, B = _rand16(rng, (M, K), oracle.BF16), _rand16(rng, (K, N), oracle.BF16, 0.02)
+            part, want = oracle.matmul_reduce(A, B, oracle.BF16, rank * rows, rows, peers, want_partial=True)
+            out = ops.matmul_reduce_scatter(dev16(A, oracle.BF16), dev16(flip(B), oracle.BF16), [dev(p) for p in wide], rank, P, **kw)
+            torch.cuda.synchronize()
+            _check_float(host16(out), want, part[own] + sum(peers), oracle.BF16, K)
+            tiles = dump.cpu().numpy()
+            assert (np.abs(tiles - part) <= sum_bound(A, B, oracle.BF16)).all()
+        assert not ws[:65536].any() and bool(ws[65536:].any())
+        for task, target, r0, c0, w0 in tasks:
+            blk = tiles[r0:min(r0 + step, (target + 1) * rows), c0:min(c0 + 256, N)]
+            if target == rank:
+                assert outbound or int(kw["checksum"][task]) == 77
+            elif outbound:
+                got = kw["outbound"].cpu().numpy().reshape(-1, 256)[w0:w0 + blk.shape[0], :blk.shape[1]]
+                assert np.array_equal(got.view(np.uint32), blk.view(np.uint32)), task
+            elif quant:
+                assert int(kw["checksum"][task]) == int(blk.astype(np.int64).sum()), task
+            else:
+                assert abs(float(kw["checksum"][task]) - blk.sum(dtype=np.float64)) <= blk.size * 2.0 ** -51 * np.abs(blk).sum(), task
+
+
+# (M, N, K, P, kept rows [begin, +count), int32 peers): k and n off the 64/128 grid, no dump, sums of the rows that are not kept
+@pytest.mark.parametrize("tb", [False, True])
+@pytest.mark.parametrize("case", [(130, 260, 1100, 2, 60, 11, False), (203, 416, 4100, 8, 0, 26, True), (203, 420, 416, 4, 190, 13, False), (40, 100, 132, 1, 3, 30, False)])
+def test_quant_kept_rows_off_the_grid_without_a_dump(case, tb):
+    _need_gpu()
+    M, N, K, P, kb, kr, ri = case
+    rng = np.random.default_rng(M + K)
+    x1, x2 = rng.integers(-127, 128, (M, K), dtype=np.int8), rng.integers(-127, 128, (K, N), dtype=np.int8)
+    s1, s2 = rng.uniform(0.005, 0.02, M).astype(np.float32), rng.uniform(0.001, 0.01, N).astype(np.float32)
+    b = rng.integers(-1000, 1000, N, dtype=np.int32)
+    peers = [rng.integers(-2 ** 24, 2 ** 24, (kr, N), dtype=np.int32) if ri else rng.standard_normal((kr, N)).astype(np.float32) for _ in range(P - 1)]
+    acc, want = oracle.quant_matmul_reduce_scatter(x1, x2, s1, s2, b, kb, kr, peers, oracle.BF16, reduce_int32=ri)
+    cs = torch.full((-(-M // 128) * -(-N // 128),), -7, dtype=torch.int64, device="cuda:0")
+    ca = torch.full((kr, N), -7, dtype=torch.int32, device="cuda:0")
+    out = ops.quant_matmul_splitk(dev(x1), dev(np.ascontiguousarray(x2.T) if tb else x2), dev(s1), dev(s2), dev(b), [dev(p) for p in peers], P, kb, kr,
+                                  checksum=cs, c_accum=ca, trans_b=tb, reduce_int32=ri)
+    torch.cuda.synchronize()
+    assert np.array_equal(host16(out), want) and np.array_equal(ca.cpu().numpy(), acc[kb:kb + kr] + (sum(peers) if ri else 0))
+    others = acc.astype(np.int64)
+    others[kb:kb + kr] = 0
+    assert np.array_equal(cs.cpu().numpy(), [others[r:r + 128, c:c + 128].sum() for r in range(0, M, 128) for c in range(0, N, 128)])
+
+
+# (rows per rank, N, K, P, rank, weights as [n,k])
+@pytest.mark.parametrize("case", [(128, 640, 448, 8, 3, False), (256, 1440, 192, 4, 0, True), (72, 288, 100, 2, 1, False), (128, 512, 1024, 8, 7, True)])
+@pytest.mark.parametrize("dtype", [oracle.FP16, oracle.BF16])
+def test_pipelined_float_one_round(case, dtype):
+    """One-round calls of the 16-bit pipelined operator on ragged columns, ragged rows and few aligned tiles: the reduced block as
+    the oracle replays it from the dumped partials, the other ranks' tiles as they were dumped."""
+    _need_gpu()
+    rows, N, K, P, rank, tb = case
+    M = rows * P
+    rng = np.random.default_rng(rows + N)
+    A, B = _rand16(rng, (M, K), dtype), _rand16(rng, (K, N), dtype, 0.05)
+    peers = [_rand16(rng, (rows, N), dtype) for _ in range(P - 1)]
+    t = ops.default_tiling(M, K, N, P, m0=128, n0=256, k0=0, commInterval=1)
+    d = L.make_desc(rank, P, [16] * (P - 1))
+    assert ops.pipelined_round_count(L.MATMUL_REDUCE_SCATTER, t, rank, P) == 1
+    ob = torch.full((L.load().catcoc_get_workspace_size(L.MATMUL_REDUCE_SCATTER, dtype, C.byref(t), C.byref(d)) // 4,), -9.0, device="cuda:0")
+    dump = torch.zeros((M, N), dtype=torch.float32, device="cuda:0")
+    out = ops.pipelined_matmul_reduce_scatter(dev16(A, dtype), dev16(np.ascontiguousarray(B.T) if tb else B, dtype), [dev16(p, dtype) for p in peers], rank, P, ob,
+                                              tiling=t, trans_b=tb, acc_dump=dump)
+    torch.cuda.synchronize()
+    part = dump.cpu().numpy()
+    assert (np.abs(part - oracle.gemm_half_f32(A, B, dtype)) <= sum_bound(A, B, dtype)).all()
+    assert np.array_equal(host16(out), oracle.pipelined_reduce_half(part[rank * rows:(rank + 1) * rows], peers, dtype, M, P, rank, 128, 256, 256, 1, 64, 256, 1))
+    for task, target, r0, c0, w0 in tasks_of(L.MATMUL_REDUCE_SCATTER, t, d):
+        if target != rank:
+            blk = part[r0:min(r0 + 128, (target + 1) * rows), c0:min(c0 + 256, N)]
+            assert np.array_equal(ob.cpu().numpy().reshape(-1, 256)[w0:w0 + blk.shape[0], :blk.shape[1]], blk), task
+
+
+def test_launches_of_several_kernels_replay_from_a_hip_graph():
+    """Flexible launches of two and three kernels (k slices, the peers' second launch, the sums of float tasks): every replay, with
+    eager work in between, equals the eager result."""
+    _need_gpu()
+    g = torch.Generator(device="cuda:0").manual_seed(3)
+    rand = lambda *shape: torch.randn(shape, device="cuda:0", generator=g)
+    byte = lambda *shape: torch.randint(-127, 128, shape, dtype=torch.int8, device="cuda:0", generator=g)
+    scale = lambda n: torch.empty(n, device="cuda:0").uniform_(0.001, 0.02, generator=g)
+    state = []
+
+    def call(fn, outputs, need):
+        ws = torch.zeros(max(need, 65536), dtype=torch.uint8, device="cuda:0")
+        state.append((lambda: fn(ws), outputs, ws))
+    # float reduce-scatter with checksums in slices, the same with stored tiles
+    P, rows, N, K = 8, 63, 516, 4112
+    A, B, peers = rand(P * rows, K).bfloat16(), rand(K, N).bfloat16(), [rand(rows, N) for _ in range(P - 1)]
+    t = ops.default_tiling(P * rows, K, N, P, m0=0, n0=0, k0=0)
+    need, f = ops.kslice_plan(L.MATMUL_REDUCE_SCATTER, torch.bfloat16, P * rows, K, N, 1, P, tiling=t)
+    assert f > 2
+    cs, out = torch.zeros(P * 3, dtype=torch.float64, device="cuda:0"), torch.zeros((rows, N), dtype=torch.bfloat16, device="cuda:0")
+    call(lambda ws: ops.matmul_reduce_scatter(A, B, peers, 1, P, tiling=t, checksum=cs, out=out, workspace=ws), [out, cs], need)
+    # W8A8 reduce-scatter, the peers in a second launch
+    x1, x2, s1, s2 = byte(1000, 352), byte(352, 516), scale(1000), scale(516)
+    qpeers = [rand(125, 516) for _ in range(7)]
+    need, f = ops.kslice_plan(L.QUANT_MATMUL_REDUCE_SCATTER, torch.int8, 1000, 352, 516, 5, 8)
+    qout, qcs = torch.zeros((125, 516), dtype=torch.bfloat16, device="cuda:0"), torch.zeros(24, dtype=torch.int64, device="cuda:0")
+    assert f == 1 and need > 65536 or f > 1
+    call(lambda ws: ops.quant_matmul_reduce_scatter(x1, x2, s1, s2, None, qpeers, 5, 8, checksum=qcs, out=qout, workspace=ws), [qout, qcs], need)
+    # all-reduce in slices, W8A8 decode in slices with sums of the other rows
+    need, f = ops.kslice_plan(L.MATMUL_ALLREDUCE, torch.float16, 33, 4096, 512, 0, 2)
+    a, b, ap, ao = rand(33, 4096).half(), rand(4096, 512).half(), [rand(33, 512)], torch.zeros((33, 512), dtype=torch.float16, device="cuda:0")
+    assert f > 1
+    call(lambda ws: ops.matmul_allreduce(a, b, ap, 0, 2, out=ao, workspace=ws), [ao], need)
+    d1, d2, e1, e2 = byte(130, 1024), byte(1024, 640), scale(130), scale(640)
+    dp, do, dcs = [rand(12, 640)], torch.zeros((12, 640), dtype=torch.bfloat16, device="cuda:0"), torch.zeros(10, dtype=torch.int64, device="cuda:0")
+    need = ops.splitk_plan(130, 1024, 640, 2, 60, 12)[0]
+    call(lambda ws: ops.quant_matmul_splitk(d1, d2, e1, e2, None, dp, 2, 60, 12, checksum=dcs, out=do, workspace=ws), [do, dcs], need)
+
+    for fn, _, _ in state:
+        fn()
+    torch.cuda.synchronize()
+    want = [[o.clone() for o in outputs] for _, outputs, _ in state]
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        for fn, _, _ in state:
+            fn()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            for fn, _, _ in state:
+                fn()
+    for replay in range(3):
+        for fn, outputs, ws in state:
+            for o in outputs:
+                o.fill_(replay + 1)
+            ws[65536:] = 0x3c   # (what an earlier launch left there does not matter)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for (fn, outputs, ws), w in zip(state, want):
+            for o, x in zip(outputs, w):
+                same = (o == x) | (o == replay + 1) if o.dim() == 1 else o == x   # (sums of the kept rank's tasks are not written)
+                assert bool(same.all()) and not ws[:65536].any()
+        for fn, _, _ in state:   # eager work between the replays
+            fn()
+        torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("slices", [0, 3])
+@pytest.mark.parametrize("tb", [False, True])
+def test_values_that_are_not_finite_stay_in_their_rows_and_columns(slices, tb):
+    """Rows and columns past the edge of a tile repeat the last one and rows of B are read past their end: an infinity or NaN there
+    reaches no other row or column, nor do those of the k remainder or of peers."""
+    _need_gpu()
+    M, N, K, P = 65, 260, 1028, 3
+    rng = np.random.default_rng(9)
+    A, B = _rand16(rng, (M, K), oracle.FP16, 1.0), _rand16(rng, (K, N), oracle.FP16, 0.02)
+    inf, nan = 0x7c00, 0x7e00
+    A[64, 3], A[0, K - 1], B[5, 259], B[K - 1, 7] = inf, nan, inf, nan
+    peers = [rng.standard_normal((M, N)).astype(np.float32) for _ in range(P - 1)]
+    peers[0][63, 100], peers[1][10, 258] = np.inf, np.nan
+    ws = torch.zeros(65536 + 3 * M * N * 4, dtype=torch.uint8, device="cuda:0") if slices else None
+    out = ops.matmul_allreduce(dev16(A, oracle.FP16), dev16(np.ascontiguousarray(B.T) if tb else B, oracle.FP16), [dev(p) for p in peers], 0, P, trans_b=tb,
+                               workspace=ws, split_k=slices)
+    torch.cuda.synchronize()
+    with np.errstate(invalid="ignore"):
+        want = oracle.half_to_f32(A, oracle.FP16).astype(np.float64) @ oracle.half_to_f32(B, oracle.FP16).astype(np.float64) + peers[0] + peers[1]
+    got = oracle.half_to_f32(host16(out), oracle.FP16)
+    finite = np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isfinite(got), finite) and np.array_equal(np.sign(got[np.isinf(want)]), np.sign(want[np.isinf(want)]))
+    assert (np.abs(got[finite] - want[finite]) <= 2.0 ** -10 * np.abs(want[finite]) + 4e-3).all()   # (one rounding to fp16, fp32 sums as in sum_bound)
+    assert (~finite).sum() == 2 * N + 2 * (M - 2) + 2
