@@ -555,23 +555,32 @@ __global__ void __launch_bounds__(256) flex_finish_kernel(const GemmArgs args, c
     __shared__ uint32_t waveTask[4];
     Sum run = 0;
     uint32_t runOf = 0xffffffffu;
+    // A row's addresses are wave-uniform but for the lane's columns: descriptors in scalar registers and one offset register for
+    // every load.  (With 64-bit addresses in vector registers the compiler at times puts them where an earlier load is still to
+    // arrive, and waits for it: the peers' loads then go one by one, bf16 all-reduce 16x8192x1024 of eight ranks 13.0 / 13.8 us.)
+    const uint32_t laneAt = lane * 16u;
+    auto load = [&](const int32_t *p, auto aux) {
+        return __builtin_amdgcn_raw_buffer_load_b128(__builtin_amdgcn_make_buffer_rsrc((void *)p, 0, 1024, 0x00020000), laneAt, 0, decltype(aux)::value);
+    };
+    constexpr std::integral_constant<int, 0> KEEP{};
+    constexpr std::integral_constant<int, 2> NT{};
     for (uint32_t v = row0 + w; v < rowEnd; v += 4u) {
         const bool kept = v - args.keptBegin < args.keptRows;
         // the peers first: they do not wait for the sums
         const uint32_t nP = kept ? args.nPeers : 0u;
-        const size_t peerAt = kept ? (size_t)(args.peerRowOffset + (v - args.keptBegin)) * args.peerLd + gcol : 0;
+        const size_t peerAt = kept ? (size_t)(args.peerRowOffset + (v - args.keptBegin)) * args.peerLd + blockIdx.x * 256u : 0;
         v4i pv[8], cur = {0, 0, 0, 0};
         if (colOk) {
 #pragma unroll
             for (int q = 0; q < 8; ++q)
-                if ((uint32_t)q < nP) pv[q] = __builtin_nontemporal_load((const v4i *)((const int *)args.peers[q] + peerAt));
-            const int32_t *part = args.skPart + (size_t)(v - first) * args.N + gcol;
+                if ((uint32_t)q < nP) pv[q] = load((const int *)args.peers[q] + peerAt, NT);
+            const int32_t *part = args.skPart + (size_t)(v - first) * args.N + blockIdx.x * 256u;
             const size_t pitch = (size_t)stored * args.N;
             for (uint32_t s0 = 0; s0 < slices; s0 += 8u) {
                 v4i t[8];
 #pragma unroll
                 for (int q = 0; q < 8; ++q)
-                    if (s0 + q < slices) t[q] = *(const v4i *)(part + (s0 + q) * pitch);
+                    if (s0 + q < slices) t[q] = load(part + (s0 + q) * pitch, KEEP);
 #pragma unroll
                 for (int q = 0; q < 8; ++q)
                     if (s0 + q < slices) {
@@ -637,7 +646,7 @@ __global__ void __launch_bounds__(256) flex_finish_kernel(const GemmArgs args, c
                 if (p0) {
 #pragma unroll
                     for (int q = 0; q < 8; ++q)
-                        if (p0 + q < nP) pv[q] = __builtin_nontemporal_load((const v4i *)((const int *)args.peers[p0 + q] + peerAt));
+                        if (p0 + q < nP) pv[q] = load((const int *)args.peers[p0 + q] + peerAt, NT);
                 }
 #pragma unroll
                 for (int q = 0; q < 8; ++q)
@@ -687,7 +696,7 @@ __global__ void __launch_bounds__(256) flex_finish_kernel(const GemmArgs args, c
 // all ranks' tile rows, and adds the sums of its rows (at most 128) that flex_finish_kernel left in slice 0, always in the same
 // order.
 // A launch more than adding in order of arrival in flex_finish_kernel, whose last bits differ from launch to launch; bf16, eight
-// ranks, us: 504x4112x1024 21.2 / 23.5, 88x1024x4096 13.8 / 15.0, 64x4096x8192 23.1 / 26.2.
+// ranks, us: 504x4112x1024 21.1 / 22.1, 88x1024x4096 13.6 / 14.8, 64x4096x8192 22.5 / 24.2.
 template <uint32_t DT>
 __global__ void __launch_bounds__(64) flex_sums_kernel(const GemmArgs args)
 {
