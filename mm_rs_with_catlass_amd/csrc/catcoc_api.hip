@@ -475,6 +475,16 @@ int make_plan(int commType, int dataType, const CocTilingParams *t, const Catcoc
             plan.kSliceBytes = c.bytes;
         }
         plan.flexBlocks = flex_use(a, es, 0, c, d->workspace, d->workspaceBytes < plan.kSliceBytes ? d->workspaceBytes : plan.kSliceBytes);
+        // A reduce-scatter that gets neither slices nor a second launch for its peers, and whose kept tiles the aligned kernel runs as
+        // two workgroups each: there the halves shorten the same chain without the flexible tiles' set-up.  Aligned / flexible tiles,
+        // stored tiles, no workspace, us: k of 1 KiB or less, W8A8 512x512x4096 of four ranks 9.6 / 11.3, fp16 1024x512x4096 of two
+        // 11.7 / 13.5 (2 KiB: 512x2048x4096 17.3 / 17.3, 16 bits 512x1024x4096 16.0 / 15.2); more than 128 tiles, W8A8 2048x2048x2048 of
+        // eight ranks 25.9 / 27.8, as [n,k] 26.1 / 29.5, of four 19.5 / 22.8, 20.1 / 24.3, k = 4096 29.9 / 32.0, 35.2 / 36.2, of eight
+        // 35.9 / 37.2, 41.6 / 41.5; with one peer and B as [k,n] the larger k is the flexible tiles' (768x4096x4096 28.9 / 26.7).
+        const uint64_t kBytes = (uint64_t)t->k * es;
+        if (plan.preferFlex && op == OP_REDUCE_SCATTER && a.fx.slices <= 1 && a.fx.late == 0 &&
+            (kBytes <= 1024 || (tiles64 > 128u && (kBytes <= 2048 || nPeers > 1 || transB))) && split_kept_tiles(a, (uint32_t)(kBytes / 64)) != 0)
+            plan.preferFlex = false;
     }
     // a workspace also lets the checksum halves of tiles that run as two workgroups meet (its counter block)
     if (a.skCount == nullptr && d->workspace != nullptr && (uintptr_t)d->workspace % 256 == 0 && d->workspaceBytes >= kCounterBlockBytes)

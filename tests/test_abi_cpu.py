@@ -607,14 +607,21 @@ def test_ragged_slice_count_is_accepted_as_the_callers_own(so):
 
 
 def test_kept_split_queries_of_launches_on_flexible_tiles(so):
-    # few tiles and a short k run flexible tiles, which are never split, unless the launch takes checksums or is told its order
+    # few tiles run flexible tiles, which are never split, unless the launch takes checksums or is told its order
     from mm_rs_with_catlass_amd import ops
-    for comm, dt, m, k, n in ((L.QUANT_MATMUL_REDUCE_SCATTER, L.INT8, 1024, 1792, 4096), (L.MATMUL_REDUCE_SCATTER, L.FP16, 1024, 1024, 4096)):
-        t = ops.default_tiling(m, k, n, 8, m0=0, n0=0, k0=0)
-        for checksum, flags, want in ((0, 0, 0), (4096, 0, n // 256), (0, L.FLAG_KEPT_SPLIT, n // 256), (0, L.FLAG_KEPT_WHOLE, 0)):
-            d = L.make_desc(0, 8, [16] * 7, flags=flags, checksum=checksum)
-            assert so.catcoc_kept_split_tiles(comm, dt, C.byref(t), C.byref(d), 0, 1) == want
-            assert so.catcoc_tail_split_tiles(comm, dt, C.byref(t), C.byref(d), 0, 1) == 0
+
+    def split(comm, dt, m, k, n, p, checksum=0, flags=0, tb=1):
+        t = ops.default_tiling(m, k, n, p, m0=0, n0=0, k0=0)
+        d = L.make_desc(0, p, [16] * (p - 1), flags=flags, checksum=checksum)
+        assert so.catcoc_tail_split_tiles(comm, dt, C.byref(t), C.byref(d), 0, tb) == 0
+        return so.catcoc_kept_split_tiles(comm, dt, C.byref(t), C.byref(d), 0, tb)
+    Q, RS = L.QUANT_MATMUL_REDUCE_SCATTER, L.MATMUL_REDUCE_SCATTER
+    for comm, dt, k in ((Q, L.INT8, 2048), (RS, L.FP16, 1024)):
+        assert split(comm, dt, 512, k, 4096, 4) == 0 and split(comm, dt, 512, k, 4096, 4, flags=L.FLAG_KEPT_WHOLE) == 0
+        assert split(comm, dt, 512, k, 4096, 4, checksum=4096) == 16 and split(comm, dt, 512, k, 4096, 4, flags=L.FLAG_KEPT_SPLIT) == 16
+        # split kept tiles beat flexible ones with a short k, and from 128 64-row tiles on (one peer, B as [k,n]: up to 2 KiB of k)
+        assert split(comm, dt, 512, k // 2, 4096, 4) == 16 and split(comm, dt, 1024, k, 4096, 8) == 16 and split(comm, dt, 1024, 2 * k, 4096, 8) == 16
+        assert split(comm, dt, 768, 2 * k, 4096, 2) == 48 and split(comm, dt, 768, 2 * k, 4096, 2, tb=0) == 0 and split(comm, dt, 768, k, 4096, 2, tb=0) == 48
 
 
 def test_descriptor_takes_what_its_fields_take(so):
