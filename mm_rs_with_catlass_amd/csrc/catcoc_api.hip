@@ -632,12 +632,14 @@ int make_splitk_plan(const CocTilingParams *t, const CatcocSymmetricDesc *d, uin
     //  - weights of more than 64 MiB stream better through the deep rings of those kernels (64x16384x8192 42.0 / 43.5, as [n,k]
     //    44.8 / 53.8; 388x15744x5376 94 / 111);
     //  - at most 32 rows with a k that leaves nothing to slice, or little to win: a second launch costs 1 us (17x576x896 10.0 / 11.2,
-    //    8x1024x8192 10.4 / 10.1, 2x8192x8192 with one row kept, [n,k], 18.2 / 19.3);
+    //    8x1024x8192 10.4 / 10.1, 2x8192x8192 with one row kept, [n,k], 18.2 / 19.3), or with so many columns that partial sums of
+    //    more than a few kept rows outweigh the rest (24x4096x8192 13.9 / 15.8, 12x4608x7168 of eight ranks, [n,k], 1.11 times;
+    //    with 5120 or 6144 columns 0.9-1.0 as [k,n], 1.02-1.11 as [n,k]);
     //  - many rows in full tiles, few of them kept: the 128x256 tile's fewer bytes per product (512x8192x8192 with 64 rows kept
     //    50 / 65, 512x4096x8192 with 256 rows kept 35 / 40, 256x8192x8192 and one peer 43.4 / 45.5).
     if (t->m0 == 0 && t->n0 == 0 && d->splitK == 0 && d->blockNum == 0) {
         const uint64_t weights = (uint64_t)t->k * t->n, work64 = (uint64_t)ceil_div(t->m, 64u) * ceil_div(t->n, 256u) * t->k;
-        sp.preferFlex = t->m <= 32 ? t->k >= 4096 && weights <= (32ull << 20)
+        sp.preferFlex = t->m <= 32 ? t->k >= 4096 && weights <= (32ull << 20) && t->n <= (transB && d->keptRows > t->m / 4 ? 4096u : 6144u)
                                    : weights <= (64ull << 20) && (!sp.large || work64 <= 128u * 4096u || (d->keptRows == t->m && P > 2));
     }
     if (sp.large) {
@@ -681,6 +683,31 @@ int make_splitk_plan(const CocTilingParams *t, const CatcocSymmetricDesc *d, uin
         return fail(E_TILING, "split-K: %u tiles exceed the %u the workspace counts", sp.tiles, kMaxCountedTiles);
     sp.workspaceBytes = f > 1 ? kCounterBlockBytes + (uint64_t)f * sp.tiles * 128u * 128u * 4u : 0;
     return 0;
+}
+
+// Launches with explicit kept rows that preferFlex leaves to the streaming kernels all the same, by what only a planned launch
+// says.  Streaming / flexible, W8A8, us, B as [k,n] unless said:
+//  - whole tiles with checksums are 128 rows high, and one workgroup has all of a kept tile's peers: 128x256x2048 with 16 rows
+//    kept of eight ranks 10.9 / 22.7, of one 9.8 / 12.8, 512x512x8192 with 128 kept 25.7 / 27.4, 203x4096x16384 with 25 kept
+//    33.7 / 45.3 (the other way up to 1 KiB of k where the streaming kernels would slice or run more than one round:
+//    64x448x4096 of two ranks 12.3 / 11.3, 300x1024x16384 of eight 25.0 / 21.3);
+//  - whole tiles without, k too short for slices: few kept rows (64x192x4096 with 8 kept of eight ranks 8.5 / 13.6, 256x192x4096
+//    with 32 kept 11.6 / 15.4), all of fewer than 48 rows with several peers (33x256x2048 11.5 / 12.8); with half the rows kept,
+//    64 at least, the flexible tiles win (128x192x4096 with 64 kept 14.6 / 12.0);
+//  - full 128x256 tiles, one peer at most: more 64-row tiles than CUs (384x1024x16384 with 96 kept of one rank 13.3 / 15.6), and a
+//    long k without peers where two slices leave CUs idle or B is [n,k] (384x4096x4096 23.8 / 25.9, 512x4096x4096 [n,k]
+//    26.8 / 29.8).
+bool decode_flex_pays(const GemmArgs &g, bool large)
+{
+    const uint32_t tiles64 = ceil_div(g.M, 64u) * g.fx.colTiles;
+    if (large && g.nPeers <= 1 && tiles64 > 256u) return false;
+    if (large && g.nPeers == 0 && g.keptRows == g.M && g.K >= 4096 && tiles64 > 64u && (tiles64 <= 96u || g.transB)) return false;
+    if (g.fx.slices >= 2) return true;
+    if (g.checksum != nullptr) return !large && g.K > 256 && g.K <= 1024 && (g.nPeers <= 1 || g.K >= 512);
+    if (g.K >= 512) return true;
+    if (g.keptRows == g.M) return g.M >= 48 || g.nPeers <= 1;
+    if (g.keptRows >= 64 && g.keptRows >= g.M - g.keptRows) return true;
+    return !large && (g.K > 256 ? g.nPeers <= 1 || g.M >= 128 : g.nPeers == 0);
 }
 
 void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_x1, uint8_t *scale_x2, uint8_t *bias,
@@ -748,7 +775,7 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
         const FlexSlices c = flex_choose(g, 1, 0, 0);
         const int blocks = flex_use(g, 1, 0, c, d->workspace, d->workspaceBytes < sp.workspaceBytes ? d->workspaceBytes : sp.workspaceBytes);
         // (without the slices it would take, only where the streaming kernels run whole tiles as well)
-        if (blocks == 0 || (c.slices > 1 && g.fx.slices < 2 && (sp.large || sp.f > 1)) || !flex_ptrs_ok(g)) return false;
+        if (blocks == 0 || (c.slices > 1 && g.fx.slices < 2 && (sp.large || sp.f > 1)) || !decode_flex_pays(g, sp.large) || !flex_ptrs_ok(g)) return false;
         const int e = launch_flex(DT_I8, g, blocks, stream);
         if (e) fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)e));
         else ok();
