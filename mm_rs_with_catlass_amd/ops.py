@@ -432,8 +432,7 @@ def pipelined_quant_matmul_reduce_scatter(x1, x2, scale_x1, scale_x2, bias, peer
         _want(outbound, "outbound", (torch.int32, torch.float32))
     if c_accum is None:
         c_accum = torch.empty((rows, n), dtype=torch.int32, device=x1.device)
-    if c_accum is not None:
-        _want(c_accum, "c_accum", torch.int32, 2, None, (rows, n))
+    _want(c_accum, "c_accum", torch.int32, 2, None, (rows, n))
     if out is None:
         out = torch.empty((rows, n), dtype=out_dtype, device=x1.device)
     _want(out, "out", (torch.float16, torch.bfloat16), 2, None, (rows, n))
