@@ -141,10 +141,11 @@ typedef struct CatcocSymmetricDesc {
     int64_t peerRowOffset;
     void *outbound;           /* OUTBOUND_STORE target, rows (stage*blockPerComm + blockIdxInComm)*m0, n0 columns */
     uint64_t outboundBytes;   /* capacity of `outbound` */
-    int64_t *checksum;        /* OUTBOUND_CHECKSUM target: one int64 per task (W8A8) / one double per task (float) */
+    int64_t *checksum;        /* OUTBOUND_CHECKSUM target: one int64 per task (W8A8) / one double per task (float), added up in
+                                 a fixed order: the same bits in every launch of the same problem with the same k slices */
     void *accDump;            /* optional full [m,n] int32 (W8A8) or fp32 (float) local partial, for bit-exact checks */
-    /* Scratch in HBM for launches whose k range is cut into slices: the skinny-M split-K path
-     * (catcoc_get_splitk_workspace_size() bytes) and few-tile launches of the large-tile kernel
+    /* Scratch in HBM for launches whose k range is cut into slices or whose peers join in a second launch: the skinny-M
+     * split-K path (catcoc_get_splitk_workspace_size() bytes) and every other launch of few tiles, aligned or ragged
      * (catcoc_get_kslice_workspace_size() bytes, optional there).  256-byte aligned.  Layout: the first
      * CATCOC_WORKSPACE_COUNTER_BYTES hold one arrival counter per tile, at the same place for every shape and slice
      * count; the partial tiles follow.  The caller ZEROES the counter block (or simply the whole buffer) once before
@@ -210,11 +211,12 @@ CATCOC_API void catcoc_launch_quant_matmul_reduce_scatter(void *stream, uint64_t
 
 /* The same operator for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Arguments and results are exactly those
- * of catcoc_launch_quant_matmul_reduce_scatter, except that desc->workspace / workspaceBytes are ignored: launches that
- * cut their k range into slices (the skinny-M split-K path; few-tile launches of the large-tile kernel) meet through a
- * scratch array built into the library, CATCOC_STATIC_SCRATCH_BYTES per GPU, which each GPU the library runs on holds
- * until the process ends.  The call allocates nothing.  A launch that needs more scratch than that is rejected
- * (catcoc_last_error() says how much it needs).  All calls on one GPU share that GPU's array: calls that overlap on
+ * of catcoc_launch_quant_matmul_reduce_scatter, except that desc->workspace / workspaceBytes are ignored: every launch whose
+ * query asks for a workspace uses a scratch array built into the library instead, CATCOC_STATIC_SCRATCH_BYTES per GPU, which each
+ * GPU the library runs on holds until the process ends.  These are the launches that cut their k range into slices (the skinny-M
+ * split-K path; few tiles, aligned or ragged) and reduce-scatter launches whose kept rows meet their peers in a second launch.
+ * The call allocates nothing.  A launch that needs more scratch than that is rejected (catcoc_last_error() says how much it
+ * needs); one whose slices are optional runs those that fit.  All calls on one GPU share that GPU's array: calls that overlap on
  * one GPU (different streams, no ordering between them) race; calls on one stream, or ordered by events, are fine.
  * Nothing is cleared at run time: the array is zero when the library's code is loaded on a GPU, and every launch leaves
  * its counter block at zero again for the next, also when it is replayed from a HIP graph. */
@@ -325,8 +327,9 @@ CATCOC_API uint64_t catcoc_get_kslice_workspace_size(int commType, int dataType,
  * tile and receives the sum of the accumulators of the tile's rows that are not kept).  The path takes int8 A [m,k]
  * and B [k,n] (or, with transB, [n,k]: a weight matrix stored output-major), peers [keptRows, n] as fp32 added after
  * the dequantisation or, with CATCOC_FLAG_REDUCE_INT32, int32 added before it.  k in whole 64-byte steps and n in whole
- * 128-column tiles run the streaming kernels; any other k or n runs whole tiles on a one-thread-per-element kernel
- * (correct, slow, no k split).  At most 32 rows against B as [n,k] (k in whole 128-byte chunks, desc->splitK 0 or 1, no
+ * 128-column tiles run the streaming kernels, or flexible tiles (64 x 256, k slices in the same workspace) where those are
+ * faster; any other k and n that are multiples of four run flexible tiles over the whole k, without a workspace, and the rest a
+ * one-thread-per-element kernel (correct, slow).  At most 32 rows against B as [n,k] (k in whole 128-byte chunks, desc->splitK 0 or 1, no
  * `checksum`) need no k split at all: one workgroup per 32 columns walks the whole k range, and such a launch neither needs
  * nor touches the workspace, whatever this query (which does not know the layout) reports.  CATCOC_OUTBOUND_STORE does not apply (explicit kept rows have no rank structure to lay
  * tiles out by).  It stands in for SplitkMatmul (3rdparty/catlass/include/catlass/gemm/kernel/splitk_matmul.hpp:68-330)

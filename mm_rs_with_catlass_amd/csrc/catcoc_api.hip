@@ -100,8 +100,8 @@ struct Plan {
 uint32_t elem_size(uint32_t dt) { return dt == DT_I8 ? 1u : 2u; }
 
 // Flexible mode (gemm_flex.h) for a launch whose schedule, kept rows and flags are filled in: fills args.fx and returns the
-// tile's rows / 64, or 0 when the launch cannot run there (A as [k,m], rows of k or columns not in 4-byte pieces, tiles of
-// another width).  `sums` = checksums were asked for and the tiles run whole: a row tile then holds whole tasks.  wantM0 =
+// tile's rows / 64, or 0 when the launch cannot run there (A as [k,m], rows of k not in 4-byte pieces, n no multiple of
+// four, tiles of another width).  `sums` = checksums were asked for and the tiles run whole: a row tile then holds whole tasks.  wantM0 =
 // the caller's tile rows (0: the library's choice), slices = k slices per tile.
 int plan_flex(GemmArgs &a, uint32_t es, bool sums, uint32_t wantM0, uint32_t slices)
 {
@@ -561,8 +561,9 @@ int make_splitk_plan(const CocTilingParams *t, const CatcocSymmetricDesc *d, uin
     const uint32_t P = d->rankSize;
     if (P == 0 || P > CATCOC_MAX_RANKS) return fail(E_RANK, "rankSize %u out of range 1..%d", P, CATCOC_MAX_RANKS);
     if (transA) return fail(E_SHAPE, "the explicit-kept-rows (split-K) path takes A as [m,k] (B as [k,n] or, with transB, as [n,k])");
-    // shapes the two fast routes cannot take (k not in whole 64-byte steps, n not in whole 128-column tiles) run the
-    // one-thread-per-element kernel on the same 128x128 grid: a correctness path, whole tiles, no workspace
+    // shapes the two fast routes cannot take (k not in whole 64-byte steps, n not in whole 128-column tiles) run flexible tiles
+    // where k and n are multiples of four, else the one-thread-per-element kernel on the 128x128 grid, a correctness path: whole
+    // tiles and no workspace either way
     sp.general = t->k % 64 != 0 || t->n % 128 != 0;
     sp.wholeK = false;
     sp.preferFlex = false;
@@ -611,7 +612,7 @@ int make_splitk_plan(const CocTilingParams *t, const CatcocSymmetricDesc *d, uin
     const uint32_t kTiles = ceil_div(t->k, 256u);
     sp.tiles = ceil_div(t->m, 128u) * ceil_div(t->n, 128u);
     if (sp.general) {
-        if (d->splitK > 1) return fail(E_TILING, "k %% 64 != 0 or n %% 128 != 0: this shape runs whole tiles on the general kernel; splitK %u is not available", d->splitK);
+        if (d->splitK > 1) return fail(E_TILING, "k %% 64 != 0 or n %% 128 != 0: this shape runs whole tiles on the general kernels; splitK %u is not available", d->splitK);
         const uint32_t stages = d->workspaceStages ? d->workspaceStages : kDefaultStages;
         a.sched = make_sched(OP_ALLREDUCE, t->m, t->n, 1, 128, 256, cores, 1, stages, off, dir);
         a.flags |= GF_ROW_MASK;

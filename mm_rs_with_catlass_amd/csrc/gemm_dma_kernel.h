@@ -203,7 +203,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     const uint32_t nkAll = FX ? (args.K * ES - args.fx.tail) / 64 : args.K * ES / 64;
     uint32_t nk = nkAll;
     size_t kOff = 0;   // bytes of k before this workgroup's first step
-    if (kSlices > 1) {   // (at most 16 slices of fewer than 2^24 steps: 32-bit products)
+    if (kSlices > 1) {   // (32-bit products: at most 64 slices of a k of up to 2^31 bytes, 2^25 steps, in flexible mode; 8 and 2^26 else)
         const uint32_t kFirst = nkAll * slice / kSlices;
         nk = nkAll * (slice + 1u) / kSlices - kFirst;
         kOff = (size_t)kFirst * 64;

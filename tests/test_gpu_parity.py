@@ -634,8 +634,8 @@ def test_quant_decode_rows_against_stored_weights(case):
 @pytest.mark.parametrize("case", [(40, 200, 100, 4, 5, 20, False, False), (130, 264, 192, 2, 100, 30, True, False), (17, 128, 72, 8, 0, 17, False, True),
                                   (260, 136, 1000, 4, 120, 140, True, True)])
 def test_quant_explicit_kept_rows_on_odd_shapes(case):
-    # k that is not whole 64-byte steps or n that is not whole 128-column tiles: the explicit-kept-rows launch runs the
-    # one-thread-per-element kernel on the same 128x128 grid (kept rows need not line up with tiles); everything it writes
+    # k that is not whole 64-byte steps or n that is not whole 128-column tiles: the explicit-kept-rows launch runs flexible
+    # tiles, or one thread per element where k or n is no multiple of four (kept rows need not line up with tiles); everything it writes
     # against the oracle: accumulators, kept int32 block, output, checksums of the rows that are not kept
     _need_gpu()
     M, N, K, P, kb, kr, tb, ri = case
