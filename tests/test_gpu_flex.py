@@ -661,3 +661,46 @@ def test_values_that_are_not_finite_stay_in_their_rows_and_columns(slices, tb):
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isfinite(got), finite) and np.array_equal(np.sign(got[np.isinf(want)]), np.sign(want[np.isinf(want)]))
     assert (np.abs(got[finite] - want[finite]) <= 2.0 ** -10 * np.abs(want[finite]) + 4e-3).all()   # (one rounding to fp16, fp32 sums as in sum_bound)
     assert (~finite).sum() == 2 * N + 2 * (M - 2) + 2
+
+
+# (M, N, K, P, kept rows, checksums): explicit kept rows on both sides of every line between the streaming kernels and flexible tiles
+@pytest.mark.parametrize("case", [(32, 4096, 4096, 2, 32, False), (32, 6272, 4096, 2, 8, True), (33, 256, 256, 2, 33, False), (33, 256, 256, 3, 33, False),
+                                  (48, 128, 448, 8, 48, False), (64, 384, 256, 1, 8, False), (64, 384, 256, 1, 8, True), (64, 384, 320, 2, 8, True),
+                                  (64, 384, 320, 3, 8, True), (128, 256, 320, 8, 16, False), (128, 256, 256, 8, 64, False), (128, 256, 448, 8, 63, False),
+                                  (256, 256, 448, 8, 128, False), (256, 256, 448, 8, 96, False), (256, 256, 448, 2, 128, True), (384, 1536, 4096, 1, 384, False),
+                                  (512, 8448, 128, 2, 256, False)])
+@pytest.mark.parametrize("tb", [False, True])
+def test_decode_on_both_sides_of_the_choice_of_kernels(case, tb):
+    _need_gpu()
+    M, N, K, P, kr, sums = case
+    rng = np.random.default_rng(M + K)
+    x1, x2 = rng.integers(-127, 128, (M, K), dtype=np.int8), rng.integers(-127, 128, (K, N), dtype=np.int8)
+    s1, s2 = rng.uniform(0.005, 0.02, M).astype(np.float32), rng.uniform(0.001, 0.01, N).astype(np.float32)
+    peers = [rng.standard_normal((kr, N)).astype(np.float32) for _ in range(P - 1)]
+    acc, want = oracle.quant_matmul_reduce_scatter(x1, x2, s1, s2, None, 0, kr, peers, oracle.BF16)
+    need, _, tiles = ops.splitk_plan(M, K, N, P, 0, kr)
+    ws = torch.zeros(max(need, 65536), dtype=torch.uint8, device="cuda:0")
+    cs = torch.full((tiles,), -7, dtype=torch.int64, device="cuda:0") if sums else None
+    ca = torch.full((kr, N), -7, dtype=torch.int32, device="cuda:0")
+    out = ops.quant_matmul_splitk(dev(x1), dev(np.ascontiguousarray(x2.T) if tb else x2), dev(s1), dev(s2), None, [dev(p) for p in peers], P, 0, kr, workspace=ws,
+                                  checksum=cs, c_accum=ca, trans_b=tb)
+    torch.cuda.synchronize()
+    assert np.array_equal(host16(out), want) and np.array_equal(ca.cpu().numpy(), acc[:kr]) and not ws[:65536].any()
+    if sums:
+        acc[:kr] = 0
+        assert np.array_equal(cs.cpu().numpy(), [acc[r:r + 128, c:c + 128].astype(np.int64).sum() for r in range(0, M, 128) for c in range(0, N, 128)])
+
+
+# (M, N, K, P): stored tiles without a workspace, kept tiles that the aligned kernel splits, k and tile counts around the lines
+@pytest.mark.parametrize("case", [(512, 4096, 1024, 4), (512, 4096, 1088, 4), (768, 4096, 2048, 2), (768, 4096, 2112, 2), (1024, 2048, 1024, 8)])
+@pytest.mark.parametrize("tb", [False, True])
+def test_stored_tiles_on_both_sides_of_the_choice_of_kernels(case, tb):
+    M, N, K, P = case
+    t = ops.default_tiling(M, K, N, P, m0=0, n0=0, k0=0)
+    r = quant_case(np.random.default_rng(K), M, N, K, P, P - 1, trans_b=tb, tiling=t, outbound=True)
+    assert r["exact"] == r["total"]
+    d = L.make_desc(P - 1, P, [16] * (P - 1))
+    deq, ob = oracle.dequant(r["acc"], r["s2"], r["s1"]), r["outbound"].cpu().numpy().reshape(-1, 256)
+    for task, target, r0, c0, w0 in tasks_of(L.QUANT_MATMUL_REDUCE_SCATTER, t, d):
+        if target != P - 1:
+            assert np.array_equal(ob[w0:w0 + 128].view(np.uint32), deq[r0:r0 + 128, c0:c0 + 256].view(np.uint32)), task
