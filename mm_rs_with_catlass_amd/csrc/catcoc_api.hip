@@ -948,7 +948,21 @@ void launch_pipelined(bool quant, int dataType, void *computeStream, void *commS
             flexBlocks = plan_flex(g, es1, false, 0, 1);
         if (flexBlocks != 0 && !flex_ptrs_ok(g)) flexBlocks = 0;
     }
-    const bool commWritesOutput = quant && deterministic != 0 && P > 1 && (uintptr_t)scale_x2 % 16 == 0 && (uintptr_t)d_out % 8 == 0;
+    // A W8A8 call of one round on aligned tiles has no round to overlap its comm launch with, and int32 sums come out the same in
+    // any order: the fused operator's epilogue adds the peers, under the other tiles' main loops, and one launch writes tiles, sums
+    // and output.  That hides the peers (nPeers x 128 KiB through the CU of a kept tile) where workgroups are still waiting for a slot,
+    // where half the CUs are free and kept tiles run as halves, and where the peers are few; in between the second launch's
+    // stream over every CU is shorter than the chain it replaces.  Two launches -> one, us, launches alternating: 512 tiles of eight ranks
+    // 4096x1792x4096 55.2 -> 48.3, as [n,k] 58.8 -> 50.2, 384 tiles 3072x1024x8192 61.3 -> 55.5, 128 tiles 1024x8192x4096 73.4 -> 61.7, two
+    // ranks 4096x4096x2048 58.3 -> 50.9, four 2048x512x4096 24.6 -> 21.0; not 288 tiles of eight 2048x2048x4608 47.6 -> 56.3, 256 of
+    // four 2048x4096x4096 52.8 -> 59.8.
+    const bool oneRound = sp.coreLoops <= sp.blockPerComm;
+    const bool fused = quant && dma && flexBlocks == 0 && P > 1 && oneRound &&
+                       (sp.coreLoops >= 384u || sp.coreLoops <= 128u || P == 2 || (P <= 4 && tiling->k <= 2048u));
+    if (fused) g.nPeers = P - 1;
+    // (a single round may run in the order of the fused operators: 4096x8192x8192 of two ranks, as [n,k], two launches 405 -> 337)
+    if (oneRound && (given->flags & CATCOC_FLAG_LINEAR_ORDER) == 0) g.flags &= ~(uint32_t)GF_LINEAR_ORDER;
+    const bool commWritesOutput = quant && !fused && deterministic != 0 && P > 1 && (uintptr_t)scale_x2 % 16 == 0 && (uintptr_t)d_out % 8 == 0;
     if ((dma || flexBlocks) && commWritesOutput) g.flags |= GF_KEPT_INT32_ONLY;   // (the comm rounds write every kept row's output)
 
     CommArgs c;
@@ -1007,7 +1021,7 @@ void launch_pipelined(bool quant, int dataType, void *computeStream, void *commS
         const uint32_t first = r * bpc, actual = umin(bpc, sp.coreLoops - first);
         if (r >= stages && !oneStream) he = hipStreamWaitEvent(cs, done[r - stages], 0);   // "compute finished" of the stage's last user
         g.taskBase = first;
-        g.taskCount = actual;
+        g.taskCount = oneRound ? 0 : actual;
         if (he == hipSuccess)
             e = flexBlocks ? launch_flex(p.dtype, g, flexBlocks, computeStream)
                 : dma ? (p.dtype == DT_I8 ? launch_gemm_dma_i8(g, computeStream)
@@ -1017,10 +1031,10 @@ void launch_pipelined(bool quant, int dataType, void *computeStream, void *commS
         if (e == 0 && he == hipSuccess && !oneStream) he = hipStreamWaitEvent(ms, ready[r], 0);
         c.roundFirstIdx = r * perRank;
         c.dataLoops = (actual / P) * (m0 / cb);
-        if (e == 0 && he == hipSuccess && P > 1 && c.dataLoops > 0) e = launch_comm_reduce(c, cores, deterministic != 0, ms);
+        if (e == 0 && he == hipSuccess && P > 1 && c.dataLoops > 0 && !fused) e = launch_comm_reduce(c, cores, deterministic != 0, ms);
         if (e == 0 && he == hipSuccess && !oneStream) he = hipEventRecord(done[r], ms);
     }
-    if (e == 0 && he == hipSuccess && quant && !fuseDequant)   // the pass after all rounds: dequantise the reduced int32 block
+    if (e == 0 && he == hipSuccess && quant && !fuseDequant && !fused)   // the pass after all rounds: dequantise the reduced int32 block
         e = launch_dequant_rows((const int32_t *)c_accum, tiling->n, (const float *)scale_x2, (const float *)scale_x1 + (size_t)d.rankIdx * sp.mRank,
                                 d_out, tiling->n, sp.mRank, tiling->n, outDt, ms);
     if (e == 0 && he == hipSuccess && !oneStream) he = hipEventRecord(fin, ms);

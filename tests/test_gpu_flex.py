@@ -286,6 +286,37 @@ def test_pipelined_quant_one_round(case, deterministic):
             assert np.array_equal(got, acc[row.value:r1, col.value:c1]), task
 
 
+# one-round pipelined calls on aligned tiles whose peers the GEMM launch adds (two ranks; four with a short k), and one that keeps its comm launch
+@pytest.mark.parametrize("case", [(128, 512, 576, 2, 1, True), (256, 256, 960, 2, 0, False), (128, 512, 64, 4, 2, False), (128, 512, 960, 8, 6, True), (256, 3072, 512, 8, 4, True)])
+@pytest.mark.parametrize("deterministic", [True, False])
+def test_pipelined_quant_one_round_on_aligned_tiles(case, deterministic):
+    test_pipelined_quant_one_round(case, deterministic)
+
+
+@pytest.mark.parametrize("tb", [False, True])
+def test_pipelined_quant_one_round_equals_two(tb):
+    """384 tiles: one round (the GEMM launch adds the peers) against two rounds with comm launches."""
+    _need_gpu()
+    M, N, K, P, rank = 1024, 12288, 64, 8, 5
+    rows = M // P
+    g = torch.Generator(device="cuda:0").manual_seed(11)
+    x1, x2 = (torch.randint(-127, 128, s, dtype=torch.int8, device="cuda:0", generator=g) for s in ((M, K), (N, K) if tb else (K, N)))
+    s1, s2 = (torch.empty(c, device="cuda:0").uniform_(0.001, 0.02, generator=g) for c in (M, N))
+    peers = [torch.randint(-2 ** 20, 2 ** 20, (rows, N), dtype=torch.int32, device="cuda:0", generator=g) for _ in range(P - 1)]
+    got = []
+    for interval in (2, 1):
+        t = ops.default_tiling(M, K, N, P, m0=128, n0=256, k0=0, commInterval=interval)
+        assert ops.pipelined_round_count(L.QUANT_MATMUL_REDUCE_SCATTER, t, rank, P) == 3 - interval
+        d = L.make_desc(rank, P, [16] * (P - 1))
+        size = L.load().catcoc_get_workspace_size(L.QUANT_MATMUL_REDUCE_SCATTER, L.INT8, C.byref(t), C.byref(d))
+        ob = torch.zeros(size // 4, dtype=torch.int32, device="cuda:0")
+        got.append(ops.pipelined_quant_matmul_reduce_scatter(x1, x2, s1, s2, None, peers, rank, P, ob, tiling=t, trans_b=tb))
+    torch.cuda.synchronize()
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    want = x1[rank * rows:(rank + 1) * rows].float() @ (x2.T if tb else x2).float()   # (exact: |sums| < 2^24)
+    assert torch.equal(got[0][1], want.to(torch.int32) + sum(peers))
+
+
 # (rows per rank, N, K, P, rank, weights as [n,k], int32 peers): kept rows inside one 64-row tile, across two, at the end; two rows per wave column
 @pytest.mark.parametrize("case", [(125, 516, 1376, 8, 5, True, False), (64, 260, 352, 8, 3, False, True), (18, 512, 416, 16, 0, True, False), (65, 1028, 100, 16, 8, False, False)])
 @pytest.mark.parametrize("outbound", [False, True])
