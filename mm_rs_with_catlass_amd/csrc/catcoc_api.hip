@@ -29,6 +29,7 @@ int launch_gemm_dma_bf16(const GemmArgs &args, void *stream);
 int launch_gemm_flex_i8(const GemmArgs &args, int rowBlocks, void *stream);
 int launch_gemm_flex_f16(const GemmArgs &args, int rowBlocks, void *stream);
 int launch_gemm_flex_bf16(const GemmArgs &args, int rowBlocks, void *stream);
+int launch_gemm_few(uint32_t dtype, const GemmArgs &args, int tileRows, int tileCols, void *stream);
 
 static int launch_flex(uint32_t dtype, const GemmArgs &args, int rowBlocks, void *stream)
 {
@@ -76,6 +77,12 @@ void ok()
 
 enum { E_NULL = 1, E_DESC = 2, E_SHAPE = 3, E_RANK = 4, E_TILING = 5, E_DTYPE = 6, E_WORKSPACE = 7, E_LAUNCH = 8 };
 
+void launched(int e)
+{
+    if (e) fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)e));
+    else ok();
+}
+
 constexpr uint32_t kDefaultBlockNum = 256;  // one scheduling slot per CU of an MI355X
 constexpr uint32_t kDefaultStages = 2;      // WORKSPACE_STAGES, examples/dynamic_tiling/include/info.h:18
 // Every workspace starts with one block of per-tile arrival counters at a fixed place and of a fixed size, whatever the
@@ -92,6 +99,7 @@ struct Plan {
     uint32_t blockNum;
     bool dma;     // full tiles, row-major operands: the direct-to-LDS kernel applies
     bool preferFlex;         // run there although the aligned kernels would take it
+    bool mayFew;             // the caller left tiles, slices and order to the library: few small tiles are a choice (few_choose)
     int flexBlocks;          // 0 = no; else the launch can run in flexible mode (gemm_flex.h) on tiles of 64 * flexBlocks rows
     uint32_t kSlices;        // k slices per tile this launch would run with a workspace (1 = none)
     uint64_t kSliceBytes;    // workspace for that: partial tiles + counters
@@ -254,6 +262,70 @@ bool flex_ptrs_ok(const GemmArgs &a)
     for (uint32_t p = 0; p < a.nPeers; ++p)
         if (!on(a.peers[p], 16)) return false;
     return true;
+}
+
+// One launch of few small tiles (gemm_few.h) for calls whose 64x256 tiles leave CUs idle.  What a launch of them takes, us, from the
+// workgroups per CU, the KiB a workgroup pulls in through its CU, the operands' and the peers' and outputs' MB (rows of B as [k,n] of
+// less than a cache line cost them again), and what the other kernels take, from 16-bit GFLOP, the same MB and KiB of k: both fitted to
+// 280 calls of every operator, 1 to 8064 rows, k 512 to 16384, n 512 to 8192, both sides timed (GPU time of calls behind each other).
+// The tile with the least is within 1.01 of the best one's time on average, and the launch is taken where it is less than 0.95 of the
+// other's: those 280 calls then take 0.77 of their time, 16x1024x8192 bf16 of eight ranks 12.9 -> 7.4, 512x1024x1024 fp16 of two 14.2 ->
+// 8.4, 203x1792x4096 W8A8 of eight 19.7 -> 13.8, 576x4128x4480 bf16 106 -> 75, the worst 1.2 times as long (few of them: bf16 5x6656x6656).
+struct FewTile {
+    int rows, cols;   // 0: the launch is not one for them
+    double us;
+};
+
+FewTile few_tile(const GemmArgs &a, uint32_t es, uint64_t rows)
+{
+    const double kB = (double)a.K * es, mb = 1e-6 * kB * ((double)a.N + rows);
+    const double moved = 4e-6 * a.N * ((double)a.nPeers * a.keptRows + ((a.flags & GF_OUTBOUND_STORE) ? rows : rows / 2));
+    FewTile best = {0, 0, 0.0};
+    static const int tiles[3][2] = {{32, 32}, {32, 64}, {64, 64}};
+    for (auto &t : tiles) {
+        const uint64_t wgs = (uint64_t)ceil_div((uint32_t)rows, t[0]) * ceil_div(a.N, t[1]);
+        const double perCu = wgs > 256 ? wgs / 256.0 : 1.0, rounds = (double)((wgs + 255u) / 256u);
+        const bool narrow = !a.transB && t[1] * es < 128u;
+        const double us = 2.3 + 2.5 * perCu + 0.0122 * rounds * kB * (t[0] + t[1]) / 1024.0 + (narrow ? 0.207 : 0.037) * mb + 0.31 * moved;
+        if (best.rows == 0 || us < best.us) best = {t[0], t[1], us};
+    }
+    return best;
+}
+
+// Whether a launch (operands, schedule, kept rows, flags and pointers filled in) runs there; fills args.fx.  `only`: nothing else
+// takes the shape at any speed.
+FewTile few_choose(GemmArgs &a, uint32_t es, bool only)
+{
+    const FewTile no = {0, 0, 0.0};
+    const SchedParams &s = a.sched;
+    const uint64_t kBytes = (uint64_t)a.K * es, ldaB = (uint64_t)a.lda * es, ldbB = (uint64_t)a.ldb * es;
+    const uint64_t rows = s.op == OP_ALLGATHER ? (uint64_t)a.M * s.P : a.M;
+    // (4-byte pieces of k; whole 16-byte pieces of a row of B as [k,n]; 32-bit offsets inside a tile)
+    if (a.transA || kBytes % 4 != 0 || kBytes < 16 || (!a.transB && ldbB % 16 != 0) || a.N % 4 != 0 || ldaB * 160u > 0x7fffffffull || ldbB * 160u > 0x7fffffffull ||
+        rows >= (1u << 30) || s.n0 != 256 || (s.m0 != 64 && s.m0 != 128))
+        return no;
+    // checksums of tasks that several of these tiles make up are the other kernels', and so are decode launches that also want the kept
+    // rows' int32 block (k slices leave it on the way)
+    if ((a.flags & GF_OUTBOUND_STORE) == 0 && a.checksum != nullptr && ((a.flags & GF_ROW_MASK) || a.keptRows < rows)) return no;
+    if ((a.flags & GF_ROW_MASK) && a.cAccum != nullptr && !only) return no;
+    const FewTile t = few_tile(a, es, rows);
+    if (!only) {
+        const double kB = (double)kBytes, mb = 1e-6 * kB * ((double)a.N + rows);
+        const double moved = 4e-6 * a.N * ((double)a.nPeers * a.keptRows + ((a.flags & GF_OUTBOUND_STORE) ? rows : rows / 2));
+        const double other = 9.8 + 1.58 * (1e-9 * es * rows * a.K * a.N) + 0.147 * mb + 0.136 * moved + 0.117 * kB / 1024.0;
+        // How much less: large weights stream better through the others' deeper rings where a tile's rows of them are no whole lines or
+        // not aligned, and with B as [k,n] or
+        // shards of an all-gather, 256 rows or more, these launches take 1.14 of the estimate.
+        const double share = mb > 40.0 && (!a.transB || kBytes % 16 != 0) ? 0.75 : rows >= 256 && (!a.transB || s.op == OP_ALLGATHER) ? 0.76 : 0.95;
+        if (t.us > share * other || (uint64_t)ceil_div((uint32_t)rows, t.rows) * ceil_div(a.N, t.cols) > 768u) return no;
+    }
+    if (!flex_ptrs_ok(a)) return no;
+    a.fx.rows = (uint32_t)rows;
+    a.fx.rowTiles = ceil_div(a.fx.rows, t.rows);
+    a.fx.colTiles = ceil_div(a.N, t.cols);
+    a.fx.dRank = make_fast_div(s.mRank);
+    a.splitK = 0;
+    return t;
 }
 
 // Everything a launcher checks before it launches; fills `plan` except the buffer pointers.
@@ -452,6 +524,7 @@ int make_plan(int commType, int dataType, const CocTilingParams *t, const Catcoc
     // 512x8192x8192 in two k slices 93.0 / 102.5 against 111 / 130).  (Checksums stay: a 128-row task would need two workgroups.)
     plan.flexBlocks = 0;
     plan.preferFlex = false;
+    plan.mayFew = t->m0 == 0 && d->splitK == 0 && (d->flags & (CATCOC_FLAG_LINEAR_ORDER | CATCOC_FLAG_KEPT_WHOLE | CATCOC_FLAG_KEPT_SPLIT)) == 0;
     const uint64_t rowsAll = op == OP_ALLGATHER ? (uint64_t)t->m * P : t->m;
     const uint64_t tiles64 = (rowsAll + 63) / 64 * ceil_div(t->n, 256u);
     const bool fewTiles = tiles64 <= 128u || (tiles64 <= 256u && (uint64_t)t->k * es <= 4096u);
@@ -517,6 +590,11 @@ void launch_float(int commType, int dataType, void *stream, uint8_t *a, uint8_t 
     p.args.b = b;
     p.args.d = c;
     if (!check_ptr_align(p, a, b)) p.variant = 0;
+    if (p.mayFew) {
+        GemmArgs g = p.args;
+        const FewTile t = few_choose(g, elem_size(p.dtype), false);
+        if (t.rows) { launched(launch_gemm_few(p.dtype, g, t.rows, t.cols, stream)); return; }
+    }
     const bool preferFlex = p.preferFlex && flex_ptrs_ok(p.args);
     const bool dma = !preferFlex && p.dma && p.variant != 0 && (uintptr_t)b % 16 == 0 && (p.args.ldb * 2) % 16 == 0 && (uintptr_t)c % 16 == 0;
     if (!dma) p.args.splitK = 0;   // the other kernels run every tile whole
@@ -538,6 +616,7 @@ struct SplitkPlan {
     bool general = false;      // shape outside the fast routes: flexible mode, or gemm_general_kernel on the 128x128 grid
     int flexBlocks;            // (general) as Plan::flexBlocks
     bool preferFlex;           // sliced row tiles (flexible mode) run although the streaming kernels would take the launch
+    bool mayFew;               // as Plan::mayFew
     bool wholeK;               // at most 32 rows against B as [n,k]: gemm_decode_nk_kernel, no k slices, no workspace
     bool large;                // many rows: the 128x256 direct-to-LDS kernel in row-mask mode runs instead of the split-K kernel
 };
@@ -567,6 +646,7 @@ int make_splitk_plan(const CocTilingParams *t, const CatcocSymmetricDesc *d, uin
     sp.general = t->k % 64 != 0 || t->n % 128 != 0;
     sp.wholeK = false;
     sp.preferFlex = false;
+    sp.mayFew = t->m0 == 0 && t->n0 == 0 && d->splitK == 0 && d->blockNum == 0;
     const bool canLarge = !sp.general && t->m % 128 == 0 && t->n % 256 == 0 && d->keptRowBegin % 32 == 0 && d->keptRows % 32 == 0;
     const bool wantLarge = t->n0 == 256 && (t->m0 == 0 || t->m0 == 128);
     if (wantLarge && !canLarge)
@@ -725,6 +805,11 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
         a.scaleM = (const float *)scale_x1; a.scaleN = (const float *)scale_x2;
         a.bias = (const int32_t *)bias; a.cAccum = (int32_t *)c_accum;
         a.outDtype = outDataType;
+        if (sp.mayFew) {   // (the rest of these shapes runs whole 64x256 tiles or one thread per element, many times slower)
+            GemmArgs g = a;
+            const FewTile t = few_choose(g, 1, true);
+            if (t.rows) { launched(launch_gemm_few(DT_I8, g, t.rows, t.cols, stream)); return; }
+        }
         const bool flex = sp.flexBlocks != 0 && flex_ptrs_ok(a);
         if (!flex && a.sched.n0 != 128) {
             const SchedParams &g = a.sched;
@@ -766,13 +851,19 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
     a.outDtype = outDataType;
     // The plan above says what the launch is refused for and what it asks of the workspace, whichever kernel runs.
     const auto flex = [&]() {
-        if (!sp.preferFlex) return false;
+        const bool few = sp.mayFew, deepK = sp.wholeK && a.M <= 8 && a.K > 8192 && a.N <= 4096;
+        if (!few && !sp.preferFlex) return false;
         GemmArgs g = a;
         const uint32_t stages = d->workspaceStages ? d->workspaceStages : kDefaultStages;
         g.sched = make_sched(OP_ALLREDUCE, a.M, a.N, 1, 128, 256, kDefaultBlockNum, 1, stages, a.sched.off, a.sched.dir);
         g.flags |= GF_ROW_MASK;
         g.splitK = 0;
         g.skCount = nullptr;
+        if (few && !deepK) {
+            const FewTile t = few_choose(g, 1, sp.wholeK && a.cAccum == nullptr);
+            if (t.rows) { launched(launch_gemm_few(DT_I8, g, t.rows, t.cols, stream)); return true; }
+        }
+        if (!sp.preferFlex || sp.wholeK) return false;
         const FlexSlices c = flex_choose(g, 1, 0, 0);
         const int blocks = flex_use(g, 1, 0, c, d->workspace, d->workspaceBytes < sp.workspaceBytes ? d->workspaceBytes : sp.workspaceBytes);
         // (without the slices it would take, only where the streaming kernels run whole tiles as well)
@@ -792,7 +883,7 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
         ok();
         return;
     }
-    if (!sp.wholeK && flex()) return;
+    if (flex()) return;
     const int e = sp.wholeK ? launch_gemm_decode_nk_i8(a, stream) : launch_gemm_splitk_i8(a, (int)sp.rowBlocks, sp.tiles * sp.f, stream);
     if (e) { fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)e)); return; }
     ok();
@@ -822,6 +913,11 @@ void launch_quant(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_x1, uin
     if (!check_ptr_align(p, x1, x2) || (uintptr_t)scale_x2 % 16 != 0 || (bias && (uintptr_t)bias % 16 != 0) ||
         (c_accum && (uintptr_t)c_accum % 16 != 0) || (uintptr_t)d_out % 8 != 0)
         p.variant = 0;
+    if (p.mayFew) {
+        GemmArgs g = p.args;
+        const FewTile t = few_choose(g, elem_size(p.dtype), false);
+        if (t.rows) { launched(launch_gemm_few(p.dtype, g, t.rows, t.cols, stream)); return; }
+    }
     const bool preferFlex = p.preferFlex && flex_ptrs_ok(p.args);
     bool dma = !preferFlex && p.dma && p.variant != 0 && (uintptr_t)x2 % 16 == 0 && p.args.ldb % 16 == 0 && (uintptr_t)d_out % 16 == 0;
     for (uint32_t s = 0; s < p.args.nPeers && dma; ++s) dma = (uintptr_t)p.args.peers[s] % 16 == 0;

@@ -1,0 +1,142 @@
+"""GPU parity of the one-launch kernels for few small tiles (csrc/gemm_few.h) at the edges of their tiles and of k: W8A8 outputs,
+workspace tiles and dumps bit for bit, float sums within the bound of two orders of the same additions."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from mm_rs_with_catlass_amd import lib as L
+from mm_rs_with_catlass_amd import ops
+from test_gpu_flex import sum_bound, tasks_of
+from test_gpu_parity import _need_gpu, _rand16, dev, dev16, host16
+
+pytestmark = pytest.mark.gpu
+
+
+# (rows, N, K, P, weights as [n,k]): one row; a tile less, full, one more; columns that end inside a tile and a 16-byte piece of the
+# output; k of one piece, less than a chunk, 4, 8 and 12 bytes into a piece (the first of a chunk, a later one), fewer chunks than waves
+@pytest.mark.parametrize("dtype", [oracle.FP16, oracle.BF16])
+@pytest.mark.parametrize("case", [(1, 4, 8, 2, True), (1, 36, 514, 8, True), (31, 32, 64, 3, False), (32, 264, 66, 16, False), (33, 100, 324, 8, True),
+                                  (64, 4096, 128, 2, True), (65, 1032, 1030, 4, False), (129, 72, 2052, 11, False), (200, 3996, 192, 1, True)])
+def test_float_allreduce(case, dtype):
+    _need_gpu()
+    M, N, K, P, tb = case
+    rng = np.random.default_rng(M + K)
+    A, B = _rand16(rng, (M, K), dtype), _rand16(rng, (K, N), dtype, 0.05)
+    peers = [rng.standard_normal((M + 3, N + 4)).astype(np.float32) for _ in range(P - 1)]
+    dump = torch.full((M, N), 7.0, dtype=torch.float32, device="cuda:0")
+    out = ops.matmul_allreduce(dev16(A, dtype), dev16(np.ascontiguousarray(B.T) if tb else B, dtype), [dev(p) for p in peers], 0, P, trans_b=tb,
+                               peer_row_offset=3, acc_dump=dump)
+    torch.cuda.synchronize()
+    got, want = dump.cpu().numpy(), oracle.half_to_f32(A, dtype).astype(np.float64) @ oracle.half_to_f32(B, dtype).astype(np.float64)
+    assert (np.abs(got - want) <= sum_bound(A, B, dtype)).all()
+    for p in peers:   # from the kernel's own sums on every step has one right answer
+        got = got + p[3:, :N]
+    assert np.array_equal(host16(out), oracle.f32_to_half(got, dtype))
+
+
+@pytest.mark.parametrize("case", [(1, 260, 130, 8, True), (7, 64, 256, 5, False), (33, 136, 1028, 2, True), (40, 520, 98, 3, False)])
+def test_float_allgather_tiles_across_shards(case):
+    _need_gpu()
+    m, N, K, P, tb = case
+    rng = np.random.default_rng(m + K)
+    B = _rand16(rng, (K, N), oracle.BF16, 0.05)
+    shards = [_rand16(rng, (m, K), oracle.BF16) for _ in range(P)]
+    rank = P // 2
+    ds = [dev16(s, oracle.BF16) for s in shards]
+    dump = torch.full((m * P, N), 7.0, dtype=torch.float32, device="cuda:0")
+    out = ops.allgather_matmul(ds[rank], ds[:rank] + ds[rank + 1:], dev16(np.ascontiguousarray(B.T) if tb else B, oracle.BF16), rank, P, trans_b=tb, acc_dump=dump)
+    torch.cuda.synchronize()
+    A = np.concatenate(shards)
+    want = oracle.half_to_f32(A, oracle.BF16).astype(np.float64) @ oracle.half_to_f32(B, oracle.BF16).astype(np.float64)
+    assert (np.abs(dump.cpu().numpy() - want) <= sum_bound(A, B, oracle.BF16)).all()
+    assert np.array_equal(host16(out), oracle.f32_to_half(dump.cpu().numpy(), oracle.BF16))
+
+
+# (rows, N, K, P, first kept row, kept rows, weights as [n,k], int32 peers)
+@pytest.mark.parametrize("case", [(1, 128, 128, 8, 0, 1, True, False), (17, 384, 1344, 16, 3, 9, True, True), (32, 36, 20, 2, 31, 1, True, False),
+                                  (33, 260, 1236, 4, 30, 3, False, True), (70, 48, 130 * 2, 8, 0, 70, False, False), (203, 1792, 1776, 8, 64, 100, False, False)])
+def test_quant_kept_rows(case):
+    _need_gpu()
+    M, N, K, P, kb, kr, tb, ri = case
+    rng = np.random.default_rng(M + N)
+    x1, x2 = rng.integers(-127, 128, (M, K), dtype=np.int8), rng.integers(-127, 128, (K, N), dtype=np.int8)
+    s1, s2 = rng.uniform(0.005, 0.02, M).astype(np.float32), rng.uniform(0.001, 0.01, N).astype(np.float32)
+    b = rng.integers(-1000, 1000, N, dtype=np.int32)
+    peers = [rng.integers(-2 ** 24, 2 ** 24, (kr, N), dtype=np.int32) if ri else rng.standard_normal((kr, N)).astype(np.float32) for _ in range(P - 1)]
+    acc, want = oracle.quant_matmul_reduce_scatter(x1, x2, s1, s2, b, kb, kr, peers, oracle.BF16, reduce_int32=ri)
+    dump = torch.full((M, N), -7, dtype=torch.int32, device="cuda:0")
+    need = ops.splitk_plan(M, K, N, P, kb, kr)[0]
+    ws = torch.zeros(max(need, 65536), dtype=torch.uint8, device="cuda:0")
+    out = ops.quant_matmul_splitk(dev(x1), dev(np.ascontiguousarray(x2.T) if tb else x2), dev(s1), dev(s2), dev(b), [dev(p) for p in peers], P, kb, kr,
+                                  workspace=ws, acc_dump=dump, trans_b=tb, reduce_int32=ri)
+    torch.cuda.synchronize()
+    assert np.array_equal(host16(out), want) and np.array_equal(dump.cpu().numpy(), acc) and not ws[:65536].any()
+
+
+# (rows per rank, N, K, P, rank, weights as [n,k], int32 peers): kept rows inside a tile and across two, other ranks' rows beside them
+@pytest.mark.parametrize("case", [(5, 260, 132, 8, 3, True, False), (20, 512, 416, 4, 0, False, True), (33, 300, 1000, 16, 15, True, False), (61, 128, 272, 2, 1, False, False)])
+def test_reduce_scatter_stored_tiles(case):
+    _need_gpu()
+    rows, N, K, P, rank, tb, ri = case
+    M = rows * P
+    rng = np.random.default_rng(M + N)
+    flip = lambda w: np.ascontiguousarray(w.T) if tb else w
+    x1, x2 = rng.integers(-127, 128, (M, K), dtype=np.int8), rng.integers(-127, 128, (K, N), dtype=np.int8)
+    s1, s2 = rng.uniform(0.005, 0.02, M).astype(np.float32), rng.uniform(0.001, 0.01, N).astype(np.float32)
+    b = rng.integers(-1000, 1000, N, dtype=np.int32)
+    peers = [rng.integers(-2 ** 24, 2 ** 24, (rows, N), dtype=np.int32) if ri else rng.standard_normal((rows, N)).astype(np.float32) for _ in range(P - 1)]
+    acc, want = oracle.quant_matmul_reduce_scatter(x1, x2, s1, s2, b, rank * rows, rows, peers, oracle.BF16, reduce_int32=ri)
+    A, B = _rand16(rng, (M, K), oracle.FP16), _rand16(rng, (K, N), oracle.FP16, 0.05)
+    t = ops.default_tiling(M, K, N, P, m0=0, n0=0, k0=0)
+    d = L.make_desc(rank, P, [16] * (P - 1))
+    for quant in (True,) if ri else (True, False):
+        comm = L.QUANT_MATMUL_REDUCE_SCATTER if quant else L.MATMUL_REDUCE_SCATTER
+        size = L.load().catcoc_get_workspace_size(comm, L.INT8 if quant else L.FP16, C.byref(t), C.byref(d)) // 4
+        ob = torch.full((size,), 3, dtype=torch.int32 if ri else torch.float32, device="cuda:0")
+        if quant:
+            sums = torch.full((rows, N), -7, dtype=torch.int32, device="cuda:0")
+            out = ops.quant_matmul_reduce_scatter(dev(x1), dev(flip(x2)), dev(s1), dev(s2), dev(b), [dev(p) for p in peers], rank, P, tiling=t, trans_b=tb,
+                                                  reduce_int32=ri, outbound=ob, c_accum=sums)
+            full = acc if ri else oracle.dequant(acc, s2, s1)
+            kept = acc[rank * rows:(rank + 1) * rows] + (sum(peers) if ri else 0)
+            assert np.array_equal(host16(out), want) and np.array_equal(sums.cpu().numpy(), kept)
+        else:
+            dump = torch.zeros((M, N), dtype=torch.float32, device="cuda:0")
+            out = ops.matmul_reduce_scatter(dev16(A, oracle.FP16), dev16(flip(B), oracle.FP16), [dev(p) for p in peers], rank, P, tiling=t, trans_b=tb,
+                                            outbound=ob, acc_dump=dump)
+            full = dump.cpu().numpy()
+            exact = oracle.half_to_f32(A, oracle.FP16).astype(np.float64) @ oracle.half_to_f32(B, oracle.FP16).astype(np.float64)
+            assert (np.abs(full - exact) <= sum_bound(A, B, oracle.FP16)).all()
+            got = full[rank * rows:(rank + 1) * rows]
+            for p in peers:
+                got = got + p
+            assert np.array_equal(host16(out), oracle.f32_to_half(got, oracle.FP16))
+        step = 64 if rows <= 64 else 128
+        tiles = ob.cpu().numpy().reshape(-1, 256)
+        for task, r, row, col, ws in tasks_of(comm, t, d):
+            if r != rank:
+                r1, c1 = min(row + step, (r + 1) * rows), min(col + 256, N)
+                assert np.array_equal(tiles[ws:ws + r1 - row, :c1 - col].view(np.uint32), full[row:r1, col:c1].view(np.uint32)), task
+
+
+@pytest.mark.parametrize("case", [(35, 72, 520 + 66, 4, True), (35, 72, 520 + 66, 4, False), (3, 40, 1024, 2, True)])
+def test_values_that_are_not_finite_stay_in_their_row_and_column(case):
+    """Infinities in the last element of k: the pieces past the end of k hold them too and must not reach a sum."""
+    _need_gpu()
+    M, N, K, P, tb = case
+    rng = np.random.default_rng(K)
+    A, B = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
+    A[M // 2, K - 1], B[K - 1, N // 3], B[K - 17, 1] = -np.inf, np.inf, np.nan
+    ab, bb = oracle.f32_to_half(A, oracle.BF16), oracle.f32_to_half(B, oracle.BF16)
+    peers = [rng.standard_normal((M, N)).astype(np.float32) for _ in range(P - 1)]
+    out = ops.matmul_allreduce(dev16(ab, oracle.BF16), dev16(np.ascontiguousarray(bb.T) if tb else bb, oracle.BF16), [dev(p) for p in peers], 0, P, trans_b=tb)
+    torch.cuda.synchronize()
+    got = oracle.half_to_f32(host16(out), oracle.BF16)
+    with np.errstate(all="ignore"):
+        want = oracle.half_to_f32(ab, oracle.BF16).astype(np.float64) @ oracle.half_to_f32(bb, oracle.BF16).astype(np.float64) + sum(peers)
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isfinite(got), fin) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    assert (np.abs(got[fin] - want[fin]) <= 2.0 ** -8 * np.abs(want[fin]) + 1e-2).all()   # (half a last place of 8 bits, and the sums' own bound)
