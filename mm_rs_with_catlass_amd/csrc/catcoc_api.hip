@@ -29,6 +29,7 @@ int launch_gemm_dma_bf16(const GemmArgs &args, void *stream);
 int launch_gemm_flex_i8(const GemmArgs &args, int rowBlocks, void *stream);
 int launch_gemm_flex_f16(const GemmArgs &args, int rowBlocks, void *stream);
 int launch_gemm_flex_bf16(const GemmArgs &args, int rowBlocks, void *stream);
+int launch_gemm_mid(uint32_t dtype, const GemmArgs &args, int tileRows, void *stream);
 int launch_gemm_few(uint32_t dtype, const GemmArgs &args, int tileRows, int tileCols, void *stream);
 
 static int launch_flex(uint32_t dtype, const GemmArgs &args, int rowBlocks, void *stream)
@@ -99,7 +100,7 @@ struct Plan {
     uint32_t blockNum;
     bool dma;     // full tiles, row-major operands: the direct-to-LDS kernel applies
     bool preferFlex;         // run there although the aligned kernels would take it
-    bool mayFew;             // the caller left tiles, slices and order to the library: few small tiles are a choice (few_choose)
+    bool maySmall;           // the caller left tiles, slices and order to the library: small tiles are a choice (small_tile)
     int flexBlocks;          // 0 = no; else the launch can run in flexible mode (gemm_flex.h) on tiles of 64 * flexBlocks rows
     uint32_t kSlices;        // k slices per tile this launch would run with a workspace (1 = none)
     uint64_t kSliceBytes;    // workspace for that: partial tiles + counters
@@ -264,39 +265,73 @@ bool flex_ptrs_ok(const GemmArgs &a)
     return true;
 }
 
-// One launch of few small tiles (gemm_few.h) for calls whose 64x256 tiles leave CUs idle.  What a launch of them takes, us, from the
-// workgroups per CU, the KiB a workgroup pulls in through its CU, the operands' and the peers' and outputs' MB (rows of B as [k,n] of
-// less than a cache line cost them again), and what the other kernels take, from 16-bit GFLOP, the same MB and KiB of k: both fitted to
-// 280 calls of every operator, 1 to 8064 rows, k 512 to 16384, n 512 to 8192, both sides timed (GPU time of calls behind each other).
-// The tile with the least is within 1.01 of the best one's time on average, and the launch is taken where it is less than 0.95 of the
-// other's: those 280 calls then take 0.77 of their time, 16x1024x8192 bf16 of eight ranks 12.9 -> 7.4, 512x1024x1024 fp16 of two 14.2 ->
-// 8.4, 203x1792x4096 W8A8 of eight 19.7 -> 13.8, 576x4128x4480 bf16 106 -> 75, the worst 1.2 times as long (few of them: bf16 5x6656x6656).
-struct FewTile {
+// ---- one launch of small tiles (gemm_few.h, gemm_mid.h) or the larger tiles' kernels ------------------------------------------------
+// Both sides of the choice are estimates in us, fitted to 390 calls of every operator (1 to 8064 rows, k 512 to 16384, n 512 to 8192,
+// 2 to 8 ranks, GPU time of calls behind each other; half of the estimates are within 0.10 of the small tiles' times and 0.05 of the
+// others', nine in ten within 0.22 and 0.15): what a launch costs by itself, per workgroup of a CU, per KiB a workgroup pulls in
+// through its CU, per MB of operands, per MB of peers and outputs.  Rows of k off the 16-byte grid and B as [k,n] cost more per KiB,
+// rows of a B tile that are no whole cache line more per MB.  The choice takes the tile with the least, and small tiles where that is
+// at most the share below of the others' estimate: up to there no call measured lost more than 0.06 (aligned tiles: none lost; at
+// 0.9 up to 0.15).  These 390 calls then take 0.78 of their time, the best choice for each would be 0.775.  Some of them, other
+// kernels -> 32x32 .. 64x64, 64x128 or 128x128 tiles: bf16 16x1024x8192 of eight ranks 12.9 -> 7.4, W8A8 203x1792x4096 19.7 -> 13.8, fp16
+// 3167x9856x640 182 -> 77, bf16 649x9984x4096 185 -> 83, all-gather 278x4736x4864 of two 87 -> 46, W8A8 760x7264x3072 68 -> 45; the other
+// way round fp16 1116x4000x4160 78 / 92, 8144x5120x1696 188 / 203.
+constexpr double kAlignedShare = 0.77, kOtherShare = 0.90;
+struct SmallTile {
     int rows, cols;   // 0: the launch is not one for them
-    double us;
+};
+struct SmallTileCost {
+    int rows, cols;
+    double launch, workgroup, kib, mb, partLine, moved, off16, kn;
+};
+constexpr SmallTileCost kSmallTiles[5] = {{32, 32, 1.84, 2.42, 0.0118, 0.051, 0.044, 0.234, 0.0049, 0.0053}, {32, 64, 2.00, 2.86, 0.0101, 0.079, 0.220, 0.248, 0.0039, 0.0014},
+                                          {64, 64, 1.59, 3.86, 0.0120, 0.038, 0.174, 0.238, 0.0033, 0.0010}, {64, 128, 1.85, 5.03, 0.0097, 0.162, 0.0, 0.223, 0.0039, 0.0010},
+                                          {128, 128, 2.30, 6.83, 0.0086, 0.219, 0.0, 0.221, 0.0043, 0.0012}};
+
+struct CallSize {
+    double rows, kib, mb, moved;   // rows of the problem, KiB of a row of k, MB of operands, MB of peers and outputs
 };
 
-FewTile few_tile(const GemmArgs &a, uint32_t es, uint64_t rows)
+CallSize call_size(const GemmArgs &a, uint32_t es)
 {
-    const double kB = (double)a.K * es, mb = 1e-6 * kB * ((double)a.N + rows);
-    const double moved = 4e-6 * a.N * ((double)a.nPeers * a.keptRows + ((a.flags & GF_OUTBOUND_STORE) ? rows : rows / 2));
-    FewTile best = {0, 0, 0.0};
-    static const int tiles[3][2] = {{32, 32}, {32, 64}, {64, 64}};
-    for (auto &t : tiles) {
-        const uint64_t wgs = (uint64_t)ceil_div((uint32_t)rows, t[0]) * ceil_div(a.N, t[1]);
-        const double perCu = wgs > 256 ? wgs / 256.0 : 1.0, rounds = (double)((wgs + 255u) / 256u);
-        const bool narrow = !a.transB && t[1] * es < 128u;
-        const double us = 2.3 + 2.5 * perCu + 0.0122 * rounds * kB * (t[0] + t[1]) / 1024.0 + (narrow ? 0.207 : 0.037) * mb + 0.31 * moved;
-        if (best.rows == 0 || us < best.us) best = {t[0], t[1], us};
-    }
-    return best;
+    const double rows = a.sched.op == OP_ALLGATHER ? (double)a.M * a.sched.P : (double)a.M, kB = (double)a.K * es;
+    return {rows, kB / 1024.0, 1e-6 * kB * (a.N + rows), 1e-6 * a.N * (4.0 * a.nPeers * a.keptRows + (a.sched.op == OP_REDUCE_SCATTER ? 4.0 : 2.0) * rows)};
 }
 
-// Whether a launch (operands, schedule, kept rows, flags and pointers filled in) runs there; fills args.fx.  `only`: nothing else
-// takes the shape at any speed.
-FewTile few_choose(GemmArgs &a, uint32_t es, bool only)
+// 128-row tiles of the aligned kernels (256-row ones: rounds of one workgroup per CU at the rate of long loops).
+double aligned_us(const GemmArgs &a, uint32_t es)
 {
-    const FewTile no = {0, 0, 0.0};
+    const CallSize c = call_size(a, es);
+    const double f = a.splitK > 1 ? a.splitK : 1.0, rounds = ceil(a.sched.coreLoops * f / 256.0), steps = c.kib * 16.0 / f;
+    if (a.sched.m0 == 256) return 10.0 + 0.78 * rounds * steps;
+    return 4.9 + rounds * (steps * (0.343 + (a.transB ? 0.048 : 0.0)) - 1.48) + (f > 1.0 ? 10.0 : 0.0) + (a.sched.op == OP_REDUCE_SCATTER ? 1.91 * a.nPeers : 0.0) +
+           0.14 * c.moved + 0.478 * c.mb;
+}
+
+// Flexible tiles as plan_flex left them in args.fx (blocks = rows / 64): whole, with a second launch for the peers, in k slices.
+double flex_us(const GemmArgs &a, uint32_t es, int blocks)
+{
+    const CallSize c = call_size(a, es);
+    const double f = a.fx.slices > 1 ? a.fx.slices : 1.0, rounds = ceil((double)a.fx.rowTiles * a.fx.colTiles * f / 256.0), steps = rounds * c.kib * 16.0 / f;
+    if (f > 1.0)
+        return 8.0 + steps * (a.transB ? 0.465 : 0.398) + 4e-6 * 0.1265 * f * (a.fx.keptOnly ? (double)a.keptRows : c.rows) * a.N + 0.227 * c.moved + 0.09 * c.mb;
+    if (a.fx.late) return 8.1 + steps * (a.transB ? 0.59 : 0.44) + 0.45 * c.moved;
+    return 3.75 + steps * (0.237 + (a.transB ? 0.118 : 0.0) + (blocks == 2 ? 0.224 : 0.0)) + 2.2 * rounds +
+           (a.sched.op == OP_REDUCE_SCATTER ? 1.1 * a.nPeers : 0.0) + 0.16 * c.moved + 0.132 * c.mb;
+}
+
+// The streaming kernels for explicit kept rows, roughly.
+double streaming_us(const GemmArgs &a)
+{
+    const CallSize c = call_size(a, 1);
+    return 9.8 + 1.58e-9 * c.rows * a.K * a.N + 0.147 * c.mb + 0.136 * c.moved + 0.117 * c.kib;
+}
+
+// The small tile a launch (operands, schedule, kept rows, flags and pointers filled in) runs, where the others would take `other` us;
+// fills args.fx for it.
+SmallTile small_tile(GemmArgs &a, uint32_t es, double other)
+{
+    const SmallTile no = {0, 0};
     const SchedParams &s = a.sched;
     const uint64_t kBytes = (uint64_t)a.K * es, ldaB = (uint64_t)a.lda * es, ldbB = (uint64_t)a.ldb * es;
     const uint64_t rows = s.op == OP_ALLGATHER ? (uint64_t)a.M * s.P : a.M;
@@ -304,28 +339,38 @@ FewTile few_choose(GemmArgs &a, uint32_t es, bool only)
     if (a.transA || kBytes % 4 != 0 || kBytes < 16 || (!a.transB && ldbB % 16 != 0) || a.N % 4 != 0 || ldaB * 160u > 0x7fffffffull || ldbB * 160u > 0x7fffffffull ||
         rows >= (1u << 30) || s.n0 != 256 || (s.m0 != 64 && s.m0 != 128))
         return no;
-    // checksums of tasks that several of these tiles make up are the other kernels', and so are decode launches that also want the kept
-    // rows' int32 block (k slices leave it on the way)
-    if ((a.flags & GF_OUTBOUND_STORE) == 0 && a.checksum != nullptr && ((a.flags & GF_ROW_MASK) || a.keptRows < rows)) return no;
-    if ((a.flags & GF_ROW_MASK) && a.cAccum != nullptr && !only) return no;
-    const FewTile t = few_tile(a, es, rows);
-    if (!only) {
-        const double kB = (double)kBytes, mb = 1e-6 * kB * ((double)a.N + rows);
-        const double moved = 4e-6 * a.N * ((double)a.nPeers * a.keptRows + ((a.flags & GF_OUTBOUND_STORE) ? rows : rows / 2));
-        const double other = 9.8 + 1.58 * (1e-9 * es * rows * a.K * a.N) + 0.147 * mb + 0.136 * moved + 0.117 * kB / 1024.0;
-        // How much less: large weights stream better through the others' deeper rings where a tile's rows of them are no whole lines or
-        // not aligned, and with B as [k,n] or
-        // shards of an all-gather, 256 rows or more, these launches take 1.14 of the estimate.
-        const double share = mb > 40.0 && (!a.transB || kBytes % 16 != 0) ? 0.75 : rows >= 256 && (!a.transB || s.op == OP_ALLGATHER) ? 0.76 : 0.95;
-        if (t.us > share * other || (uint64_t)ceil_div((uint32_t)rows, t.rows) * ceil_div(a.N, t.cols) > 768u) return no;
+    // Checksums: of tasks of a reduce-scatter the other kernels', of the 128x128 blocks of explicit kept rows those of a tile that
+    // has all rows of one.  Decode launches that also want the kept rows' int32 block stay where their k slices leave it on the way.
+    const bool rowMask = (a.flags & GF_ROW_MASK) != 0, sums = (a.flags & GF_OUTBOUND_STORE) == 0 && a.checksum != nullptr && (rowMask || a.keptRows < rows);
+    if ((sums && !rowMask) || (rowMask && a.cAccum != nullptr)) return no;
+    const CallSize c = call_size(a, es);
+    const SmallTileCost *best = nullptr;
+    double least = 0.0;
+    uint64_t tiles = 0;
+    for (const SmallTileCost &t : kSmallTiles) {
+        if (sums && (t.cols != 128 || (t.rows < 128 && rows > (uint64_t)t.rows))) continue;
+        const uint64_t n = (rows + t.rows - 1) / t.rows * ceil_div(a.N, t.cols);
+        const double perCu = n > 256 ? n / 256.0 : 1.0, kib = (double)((n + 255) / 256) * c.kib * (t.rows + t.cols);
+        const double us = t.launch + t.workgroup * perCu + kib * (t.kib + (kBytes % 16 ? t.off16 : 0.0) + (a.transB ? 0.0 : t.kn)) + c.mb * t.mb +
+                          (!a.transB && t.cols * es < 128u ? c.mb * t.partLine : 0.0) + c.moved * t.moved;
+        if (best == nullptr || us < least) {
+            best = &t;
+            least = us;
+            tiles = n;
+        }
     }
-    if (!flex_ptrs_ok(a)) return no;
+    if (best == nullptr || least > other || tiles > (1u << 24) || !flex_ptrs_ok(a)) return no;
     a.fx.rows = (uint32_t)rows;
-    a.fx.rowTiles = ceil_div(a.fx.rows, t.rows);
-    a.fx.colTiles = ceil_div(a.N, t.cols);
+    a.fx.rowTiles = (uint32_t)((rows + best->rows - 1) / best->rows);
+    a.fx.colTiles = ceil_div(a.N, best->cols);
     a.fx.dRank = make_fast_div(s.mRank);
     a.splitK = 0;
-    return t;
+    return {best->rows, best->cols};
+}
+
+void launch_small(uint32_t dtype, const GemmArgs &a, const SmallTile &t, void *stream)
+{
+    launched(t.cols == 128 ? launch_gemm_mid(dtype, a, t.rows, stream) : launch_gemm_few(dtype, a, t.rows, t.cols, stream));
 }
 
 // Everything a launcher checks before it launches; fills `plan` except the buffer pointers.
@@ -524,7 +569,7 @@ int make_plan(int commType, int dataType, const CocTilingParams *t, const Catcoc
     // 512x8192x8192 in two k slices 93.0 / 102.5 against 111 / 130).  (Checksums stay: a 128-row task would need two workgroups.)
     plan.flexBlocks = 0;
     plan.preferFlex = false;
-    plan.mayFew = t->m0 == 0 && d->splitK == 0 && (d->flags & (CATCOC_FLAG_LINEAR_ORDER | CATCOC_FLAG_KEPT_WHOLE | CATCOC_FLAG_KEPT_SPLIT)) == 0;
+    plan.maySmall = t->m0 == 0 && d->splitK == 0 && (d->flags & (CATCOC_FLAG_LINEAR_ORDER | CATCOC_FLAG_KEPT_WHOLE | CATCOC_FLAG_KEPT_SPLIT)) == 0;
     const uint64_t rowsAll = op == OP_ALLGATHER ? (uint64_t)t->m * P : t->m;
     const uint64_t tiles64 = (rowsAll + 63) / 64 * ceil_div(t->n, 256u);
     const bool fewTiles = tiles64 <= 128u || (tiles64 <= 256u && (uint64_t)t->k * es <= 4096u);
@@ -558,6 +603,8 @@ int make_plan(int commType, int dataType, const CocTilingParams *t, const Catcoc
         if (plan.preferFlex && op == OP_REDUCE_SCATTER && a.fx.slices <= 1 && a.fx.late == 0 &&
             (kBytes <= 1024 || (tiles64 > 128u && (kBytes <= 2048 || nPeers > 1 || transB))) && split_kept_tiles(a, (uint32_t)(kBytes / 64)) != 0)
             plan.preferFlex = false;
+        // (four slices or more of ragged rows or columns with B as [k,n]: a caller's count of them and the library's own give the same bits)
+        if (plan.preferFlex && plan.edge && !transB && a.fx.slices >= 4) plan.maySmall = false;
     }
     // a workspace also lets the checksum halves of tiles that run as two workgroups meet (its counter block)
     if (a.skCount == nullptr && d->workspace != nullptr && (uintptr_t)d->workspace % 256 == 0 && d->workspaceBytes >= kCounterBlockBytes)
@@ -578,6 +625,16 @@ int check_ptr_align(const Plan &p, const void *a, const void *b)
     return okA && okB;
 }
 
+bool launched_small(const Plan &p, bool dma, bool flex, void *stream)
+{
+    if (!p.maySmall) return false;
+    GemmArgs g = p.args;
+    const uint32_t es = elem_size(p.dtype);
+    const SmallTile t = small_tile(g, es, dma ? kAlignedShare * aligned_us(p.args, es) : flex ? kOtherShare * flex_us(p.args, es, p.flexBlocks) : 1e30);
+    if (t.rows) launch_small(p.dtype, g, t, stream);
+    return t.rows != 0;
+}
+
 void launch_float(int commType, int dataType, void *stream, uint8_t *a, uint8_t *b, uint8_t *c, uint8_t *symmetricPtr,
                   CocTilingParams *tiling, uint32_t transA, uint32_t transB)
 {
@@ -590,17 +647,13 @@ void launch_float(int commType, int dataType, void *stream, uint8_t *a, uint8_t 
     p.args.b = b;
     p.args.d = c;
     if (!check_ptr_align(p, a, b)) p.variant = 0;
-    if (p.mayFew) {
-        GemmArgs g = p.args;
-        const FewTile t = few_choose(g, elem_size(p.dtype), false);
-        if (t.rows) { launched(launch_gemm_few(p.dtype, g, t.rows, t.cols, stream)); return; }
-    }
     const bool preferFlex = p.preferFlex && flex_ptrs_ok(p.args);
     const bool dma = !preferFlex && p.dma && p.variant != 0 && (uintptr_t)b % 16 == 0 && (p.args.ldb * 2) % 16 == 0 && (uintptr_t)c % 16 == 0;
     if (!dma) p.args.splitK = 0;   // the other kernels run every tile whole
     if (!dma && p.variant == 4) { fail(E_TILING, "m0 = 256 needs full tiles and 16-byte aligned row-major operands"); return; }
     if (!dma && p.args.transA) p.variant = 0;
     const bool flex = !dma && p.flexBlocks != 0 && flex_ptrs_ok(p.args);
+    if (launched_small(p, dma, flex, stream)) return;
     const int e = dma ? (p.dtype == DT_F16 ? launch_gemm_dma_f16(p.args, stream) : launch_gemm_dma_bf16(p.args, stream))
                   : flex ? launch_flex(p.dtype, p.args, p.flexBlocks, stream)
                       : launch_gemm(p.dtype, p.args, p.variant, p.edge, stream);
@@ -616,7 +669,7 @@ struct SplitkPlan {
     bool general = false;      // shape outside the fast routes: flexible mode, or gemm_general_kernel on the 128x128 grid
     int flexBlocks;            // (general) as Plan::flexBlocks
     bool preferFlex;           // sliced row tiles (flexible mode) run although the streaming kernels would take the launch
-    bool mayFew;               // as Plan::mayFew
+    bool maySmall;             // as Plan::maySmall
     bool wholeK;               // at most 32 rows against B as [n,k]: gemm_decode_nk_kernel, no k slices, no workspace
     bool large;                // many rows: the 128x256 direct-to-LDS kernel in row-mask mode runs instead of the split-K kernel
 };
@@ -646,7 +699,7 @@ int make_splitk_plan(const CocTilingParams *t, const CatcocSymmetricDesc *d, uin
     sp.general = t->k % 64 != 0 || t->n % 128 != 0;
     sp.wholeK = false;
     sp.preferFlex = false;
-    sp.mayFew = t->m0 == 0 && t->n0 == 0 && d->splitK == 0 && d->blockNum == 0;
+    sp.maySmall = t->m0 == 0 && t->n0 == 0 && d->splitK == 0 && d->blockNum == 0;
     const bool canLarge = !sp.general && t->m % 128 == 0 && t->n % 256 == 0 && d->keptRowBegin % 32 == 0 && d->keptRows % 32 == 0;
     const bool wantLarge = t->n0 == 256 && (t->m0 == 0 || t->m0 == 128);
     if (wantLarge && !canLarge)
@@ -805,10 +858,10 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
         a.scaleM = (const float *)scale_x1; a.scaleN = (const float *)scale_x2;
         a.bias = (const int32_t *)bias; a.cAccum = (int32_t *)c_accum;
         a.outDtype = outDataType;
-        if (sp.mayFew) {   // (the rest of these shapes runs whole 64x256 tiles or one thread per element, many times slower)
+        if (sp.maySmall) {   // (the rest of these shapes runs whole 64x256 tiles or one thread per element, many times slower)
             GemmArgs g = a;
-            const FewTile t = few_choose(g, 1, true);
-            if (t.rows) { launched(launch_gemm_few(DT_I8, g, t.rows, t.cols, stream)); return; }
+            const SmallTile t = small_tile(g, 1, 1e30);
+            if (t.rows) { launch_small(DT_I8, g, t, stream); return; }
         }
         const bool flex = sp.flexBlocks != 0 && flex_ptrs_ok(a);
         if (!flex && a.sched.n0 != 128) {
@@ -851,23 +904,32 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
     a.outDtype = outDataType;
     // The plan above says what the launch is refused for and what it asks of the workspace, whichever kernel runs.
     const auto flex = [&]() {
-        const bool few = sp.mayFew, deepK = sp.wholeK && a.M <= 8 && a.K > 8192 && a.N <= 4096;
-        if (!few && !sp.preferFlex) return false;
+        // (at most eight rows of a long k and few columns as [n,k]: the whole-k kernel's rings of eight rows hold more of B than a 32x32
+        // tile's.  8x16384x2048 13.3 / 13.9, 1x12288x1024 10.8 / 11.5; the others 1x8192x8192 16.0 / 15.1, 16x4096x8192 10.6 / 9.4)
+        const bool deepK = sp.wholeK && a.M <= 8 && a.K > 8192 && a.N <= 4096;
+        if (deepK || (!sp.maySmall && !sp.preferFlex)) return false;
         GemmArgs g = a;
         const uint32_t stages = d->workspaceStages ? d->workspaceStages : kDefaultStages;
         g.sched = make_sched(OP_ALLREDUCE, a.M, a.N, 1, 128, 256, kDefaultBlockNum, 1, stages, a.sched.off, a.sched.dir);
         g.flags |= GF_ROW_MASK;
         g.splitK = 0;
         g.skCount = nullptr;
-        if (few && !deepK) {
-            const FewTile t = few_choose(g, 1, sp.wholeK && a.cAccum == nullptr);
-            if (t.rows) { launched(launch_gemm_few(DT_I8, g, t.rows, t.cols, stream)); return true; }
+        GemmArgs small = g;
+        int blocks = 0;
+        if (sp.preferFlex && !sp.wholeK) {
+            const FlexSlices c = flex_choose(g, 1, 0, 0);
+            blocks = flex_use(g, 1, 0, c, d->workspace, d->workspaceBytes < sp.workspaceBytes ? d->workspaceBytes : sp.workspaceBytes);
+            // (without the slices it would take, only where the streaming kernels run whole tiles as well)
+            if ((c.slices > 1 && g.fx.slices < 2 && (sp.large || sp.f > 1)) || !decode_flex_pays(g, sp.large) || !flex_ptrs_ok(g)) blocks = 0;
         }
-        if (!sp.preferFlex || sp.wholeK) return false;
-        const FlexSlices c = flex_choose(g, 1, 0, 0);
-        const int blocks = flex_use(g, 1, 0, c, d->workspace, d->workspaceBytes < sp.workspaceBytes ? d->workspaceBytes : sp.workspaceBytes);
-        // (without the slices it would take, only where the streaming kernels run whole tiles as well)
-        if (blocks == 0 || (c.slices > 1 && g.fx.slices < 2 && (sp.large || sp.f > 1)) || !decode_flex_pays(g, sp.large) || !flex_ptrs_ok(g)) return false;
+        if (sp.maySmall) {
+            const SmallTile t = small_tile(small, 1, sp.wholeK ? 1e30 : kOtherShare * (blocks ? flex_us(g, 1, blocks) : streaming_us(g)));
+            if (t.rows) {
+                launch_small(DT_I8, small, t, stream);
+                return true;
+            }
+        }
+        if (blocks == 0) return false;
         const int e = launch_flex(DT_I8, g, blocks, stream);
         if (e) fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)e));
         else ok();
@@ -913,11 +975,6 @@ void launch_quant(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_x1, uin
     if (!check_ptr_align(p, x1, x2) || (uintptr_t)scale_x2 % 16 != 0 || (bias && (uintptr_t)bias % 16 != 0) ||
         (c_accum && (uintptr_t)c_accum % 16 != 0) || (uintptr_t)d_out % 8 != 0)
         p.variant = 0;
-    if (p.mayFew) {
-        GemmArgs g = p.args;
-        const FewTile t = few_choose(g, elem_size(p.dtype), false);
-        if (t.rows) { launched(launch_gemm_few(p.dtype, g, t.rows, t.cols, stream)); return; }
-    }
     const bool preferFlex = p.preferFlex && flex_ptrs_ok(p.args);
     bool dma = !preferFlex && p.dma && p.variant != 0 && (uintptr_t)x2 % 16 == 0 && p.args.ldb % 16 == 0 && (uintptr_t)d_out % 16 == 0;
     for (uint32_t s = 0; s < p.args.nPeers && dma; ++s) dma = (uintptr_t)p.args.peers[s] % 16 == 0;
@@ -925,6 +982,7 @@ void launch_quant(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_x1, uin
     if (!dma) p.args.splitK = 0;   // the other kernels run every tile whole
     if (!dma && p.args.transA) p.variant = 0;
     const bool flex = !dma && p.flexBlocks != 0 && flex_ptrs_ok(p.args);
+    if (launched_small(p, dma, flex, stream)) return;
     const int e = dma ? launch_gemm_dma_i8(p.args, stream) : flex ? launch_flex(p.dtype, p.args, p.flexBlocks, stream) : launch_gemm(p.dtype, p.args, p.variant, p.edge, stream);
     if (e) { fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)e)); return; }
     ok();

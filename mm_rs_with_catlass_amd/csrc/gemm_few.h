@@ -13,7 +13,7 @@
 // small rather than sliced: 64x256 tiles in k slices used 64 to 128 CUs, and the second launch that added the slices and the peers cost
 // 3.5 to 6 us.  GPU time per call, k slices and second launch -> this: bf16 16x1024x8192, eight ranks, 12.9 -> 7.4 us, fp16
 // 512x1024x1024, two ranks, 14.2 -> 8.4, W8A8 203x1792x4096, eight ranks, all rows kept, 19.7 -> 13.8 (33 MB, 23 of them the
-// peers'), off the 64-byte and 128-column grid 2x13472x2432 57 -> 23, 46x15872x3360 144 -> 21.  Which launches: few_choose().
+// peers'), off the 64-byte and 128-column grid 2x13472x2432 57 -> 23, 46x15872x3360 144 -> 21.  Which launches: small_tile().
 // k is divided among the waves because that takes neither barriers nor a shared ring; what it costs is LDS reads (a 64x64 tile reads
 // two fragments per two MFMAs, all the LDS can give), so long loops over many tiles belong to the larger tiles.
 #pragma once

@@ -1,4 +1,4 @@
-"""GPU parity of the one-launch kernels for few small tiles (csrc/gemm_few.h) at the edges of their tiles and of k: W8A8 outputs,
+"""GPU parity of the one-launch kernels for small tiles (csrc/gemm_few.h, csrc/gemm_mid.h) at the edges of their tiles and of k: W8A8 outputs,
 workspace tiles and dumps bit for bit, float sums within the bound of two orders of the same additions."""
 import ctypes as C
 
@@ -140,3 +140,66 @@ def test_values_that_are_not_finite_stay_in_their_row_and_column(case):
     fin = np.isfinite(want)
     assert np.array_equal(np.isfinite(got), fin) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
     assert (np.abs(got[fin] - want[fin]) <= 2.0 ** -8 * np.abs(want[fin]) + 1e-2).all()   # (half a last place of 8 bits, and the sums' own bound)
+
+
+# (rows, N, K, P, first kept row, kept rows, weights as [n,k]): checksums, which tiles of 64x128 (up to 64 rows) and 128x128 leave; rows
+# and columns one past a tile, k of one chunk and less, of a few bytes more than whole chunks, more chunks than stages
+@pytest.mark.parametrize("case", [(40, 128, 100, 2, 3, 10, True), (64, 132, 132, 8, 0, 8, True), (65, 260, 1236, 4, 60, 5, False), (128, 112, 776, 3, 128 - 40, 40, False),
+                                  (129, 516, 648, 8, 128, 1, True), (300, 240, 2440, 6, 100, 150, False), (18, 48, 36, 1, 2, 4, True)])
+def test_quant_kept_rows_with_checksums(case):
+    _need_gpu()
+    M, N, K, P, kb, kr, tb = case
+    rng = np.random.default_rng(M + N)
+    x1, x2 = rng.integers(-127, 128, (M, K), dtype=np.int8), rng.integers(-127, 128, (K, N), dtype=np.int8)
+    s1, s2 = rng.uniform(0.005, 0.02, M).astype(np.float32), rng.uniform(0.001, 0.01, N).astype(np.float32)
+    b = rng.integers(-1000, 1000, N, dtype=np.int32)
+    peers = [rng.standard_normal((kr, N)).astype(np.float32) for _ in range(P - 1)]
+    acc, want = oracle.quant_matmul_reduce_scatter(x1, x2, s1, s2, b, kb, kr, peers, oracle.BF16)
+    others = acc.astype(np.int64)
+    others[kb:kb + kr] = 0
+    sums = np.array([others[r:r + 128, c:c + 128].sum() for r in range(0, M, 128) for c in range(0, N, 128)])
+    cs = torch.full((sums.size,), -7, dtype=torch.int64, device="cuda:0")
+    dump = torch.full((M, N), -7, dtype=torch.int32, device="cuda:0")
+    out = ops.quant_matmul_splitk(dev(x1), dev(np.ascontiguousarray(x2.T) if tb else x2), dev(s1), dev(s2), dev(b), [dev(p) for p in peers], P, kb, kr,
+                                  workspace=torch.zeros(1 << 20, dtype=torch.uint8, device="cuda:0"), checksum=cs, acc_dump=dump, trans_b=tb)
+    torch.cuda.synchronize()
+    assert np.array_equal(host16(out), want) and np.array_equal(dump.cpu().numpy(), acc) and np.array_equal(cs.cpu().numpy(), sums)
+
+
+# (operator, rows (of a shard), N, K, P, rank, weights as [n,k]): 64x128 and 128x128 tiles of the float operators
+@pytest.mark.parametrize("case", [("allreduce", 1000, 1544, 1234, 4, 0, False), ("allreduce", 650, 3332, 2310, 3, 0, True), ("allgather", 278, 4864, 4744, 2, 1, False), ("allreduce", 610, 4608, 5000, 8, 0, False),
+                                  ("reduce_scatter", 1392, 1540, 2820, 8, 5, True), ("reduce_scatter", 600, 4104, 1032, 2, 1, False)])
+def test_float_larger_tiles(case):
+    _need_gpu()
+    op, m, N, K, P, rank, tb = case
+    g = torch.Generator(device="cuda:0").manual_seed(m)
+    rand = lambda *shape: torch.randn(shape, device="cuda:0", generator=g)
+    M = m * P if op == "allgather" else m
+    A, B = rand(M, K).bfloat16(), (rand(K, N) * 0.05).bfloat16()
+    Bd = B.T.contiguous() if tb else B
+    rows = {"allreduce": m, "allgather": 0, "reduce_scatter": m // P}[op]
+    peers = [rand(rows, N) for _ in range(P - 1)] if rows else []
+    dump = torch.full((M, N), 7.0, device="cuda:0")
+    if op == "allgather":
+        shards = [s.contiguous() for s in A.split(m)]
+        out = ops.allgather_matmul(shards[rank], shards[:rank] + shards[rank + 1:], Bd, rank, P, trans_b=tb, acc_dump=dump)
+        got = dump
+    elif op == "allreduce":
+        out = ops.matmul_allreduce(A, Bd, peers, 0, P, trans_b=tb, acc_dump=dump)
+        got = dump
+    else:
+        t = ops.default_tiling(M, K, N, P, m0=0, n0=0, k0=0)
+        d = L.make_desc(rank, P, [16] * (P - 1))
+        ob = torch.full((L.load().catcoc_get_workspace_size(L.MATMUL_REDUCE_SCATTER, L.BF16, C.byref(t), C.byref(d)) // 4,), 3.0, device="cuda:0")
+        out = ops.matmul_reduce_scatter(A, Bd, peers, rank, P, tiling=t, trans_b=tb, outbound=ob, acc_dump=dump)
+        tiles, full = ob.cpu().numpy().reshape(-1, 256), dump.cpu().numpy()
+        for task, r, row, col, ws in tasks_of(L.MATMUL_REDUCE_SCATTER, t, d):
+            if r != rank:
+                r1, c1 = min(row + 128, (r + 1) * rows), min(col + 256, N)
+                assert np.array_equal(tiles[ws:ws + r1 - row, :c1 - col], full[row:r1, col:c1]), task
+        got = dump[rank * rows:(rank + 1) * rows]
+    bound = 8 * K ** 0.5 * 2.0 ** -24 * torch.outer(A.double().norm(dim=1), B.double().norm(dim=0)) + 1e-9   # (as sum_bound)
+    assert ((dump.double() - A.double() @ B.double()).abs() <= bound).all()
+    for p in peers:
+        got = got + p
+    assert torch.equal(out, got.bfloat16())
