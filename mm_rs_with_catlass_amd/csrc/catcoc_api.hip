@@ -30,6 +30,7 @@ int launch_gemm_flex_i8(const GemmArgs &args, int rowBlocks, void *stream);
 int launch_gemm_flex_f16(const GemmArgs &args, int rowBlocks, void *stream);
 int launch_gemm_flex_bf16(const GemmArgs &args, int rowBlocks, void *stream);
 int launch_gemm_mid(uint32_t dtype, const GemmArgs &args, int tileRows, void *stream);
+int launch_gemm_mixed(uint32_t dtype, const GemmArgs &args, void *stream);
 int launch_gemm_few(uint32_t dtype, const GemmArgs &args, int tileRows, int tileCols, void *stream);
 
 static int launch_flex(uint32_t dtype, const GemmArgs &args, int rowBlocks, void *stream)
@@ -265,28 +266,30 @@ bool flex_ptrs_ok(const GemmArgs &a)
     return true;
 }
 
-// ---- one launch of small tiles (gemm_few.h, gemm_mid.h) or the larger tiles' kernels ------------------------------------------------
-// Both sides of the choice are estimates in us, fitted to 390 calls of every operator (1 to 8064 rows, k 512 to 16384, n 512 to 8192,
-// 2 to 8 ranks, GPU time of calls behind each other; half of the estimates are within 0.10 of the small tiles' times and 0.05 of the
-// others', nine in ten within 0.22 and 0.15): what a launch costs by itself, per workgroup of a CU, per KiB a workgroup pulls in
-// through its CU, per MB of operands, per MB of peers and outputs.  Rows of k off the 16-byte grid and B as [k,n] cost more per KiB,
-// rows of a B tile that are no whole cache line more per MB.  The choice takes the tile with the least, and small tiles where that is
-// at most the share below of the others' estimate: up to there no call measured lost more than 0.06 (aligned tiles: none lost; at
-// 0.9 up to 0.15).  These 390 calls then take 0.78 of their time, the best choice for each would be 0.775.  Some of them, other
-// kernels -> 32x32 .. 64x64, 64x128 or 128x128 tiles: bf16 16x1024x8192 of eight ranks 12.9 -> 7.4, W8A8 203x1792x4096 19.7 -> 13.8, fp16
-// 3167x9856x640 182 -> 77, bf16 649x9984x4096 185 -> 83, all-gather 278x4736x4864 of two 87 -> 46, W8A8 760x7264x3072 68 -> 45; the other
-// way round fp16 1116x4000x4160 78 / 92, 8144x5120x1696 188 / 203.
-constexpr double kAlignedShare = 0.77, kOtherShare = 0.90;
+// ---- one launch of small or mixed tiles (gemm_few.h, gemm_mid.h, gemm_mixed.h) or the other kernels ------------------------------------
+// Both sides of the choice are estimates in us, fitted to 460 calls of every operator (1 to 8192 rows, k 512 to 16384, n 512 to 8192,
+// 2 to 8 ranks, up to 6e11 operations, GPU time of calls behind each other): what a launch costs by itself, per workgroup of a CU, per
+// KiB a workgroup pulls in through its CU (more from the second round of workgroups on: the first leaves the caches cold), per MB of
+// operands, per MB of peers and outputs; rows of k off the 16-byte grid and B as [k,n] cost more per KiB, rows of a B tile that are no whole
+// cache line more per MB.  Half of the estimates are within 0.10 of the tiles' times and 0.06 of the others', nine in ten within 0.22
+// and 0.16.  The choice takes the tiles with the least, where that is at most the share below of the others' estimate: beyond it calls
+// start to lose (aligned tiles at 0.9: up to 0.15, flexible ones at 1.0: up to 0.3), up to it three of 413 lost more than 0.04.  Calls
+// that had aligned tiles take 0.82 of their time, those that had flexible ones 0.78; the best choice for each would be 0.79 and 0.76.
+// Some of them, other kernels -> 32x32 .. 64x64, 64x128 or 128x128 tiles: bf16 16x1024x8192 of eight ranks 12.9 -> 7.4, W8A8
+// 203x1792x4096 19.7 -> 13.8, fp16 3167x9856x640 182 -> 77, bf16 649x9984x4096 185 -> 83, all-gather 278x4736x4864 of two 87 -> 46, W8A8
+// 760x7264x3072 68 -> 45; the other way round fp16 1116x4000x4160 78 / 92, 8144x5120x1696 188 / 203.  -> mixed: see gemm_mixed.h.
+constexpr double kAlignedShare = 0.85, kOtherShare = 0.87;
 struct SmallTile {
-    int rows, cols;   // 0: the launch is not one for them
+    int rows, cols;   // 0: the launch is not one for them; 256x256: the large ones of a mixed launch
 };
 struct SmallTileCost {
     int rows, cols;
-    double launch, workgroup, kib, mb, partLine, moved, off16, kn;
+    double launch, workgroup, kib, mb, partLine, moved, off16, kn, later;
 };
-constexpr SmallTileCost kSmallTiles[5] = {{32, 32, 1.84, 2.42, 0.0118, 0.051, 0.044, 0.234, 0.0049, 0.0053}, {32, 64, 2.00, 2.86, 0.0101, 0.079, 0.220, 0.248, 0.0039, 0.0014},
-                                          {64, 64, 1.59, 3.86, 0.0120, 0.038, 0.174, 0.238, 0.0033, 0.0010}, {64, 128, 1.85, 5.03, 0.0097, 0.162, 0.0, 0.223, 0.0039, 0.0010},
-                                          {128, 128, 2.30, 6.83, 0.0086, 0.219, 0.0, 0.221, 0.0043, 0.0012}};
+constexpr SmallTileCost kSmallTiles[5] = {
+    {32, 32, 1.84, 2.42, 0.0118, 0.051, 0.044, 0.234, 0.0049, 0.0053, 0.0},  {32, 64, 2.00, 2.86, 0.0101, 0.079, 0.220, 0.248, 0.0039, 0.0014, 0.0},
+    {64, 64, 1.59, 3.86, 0.0120, 0.038, 0.174, 0.238, 0.0033, 0.0010, 0.0},  {64, 128, 3.47, 3.94, 0.0086, 0.187, 0.0, 0.174, 0.0040, 0.0008, 0.0039},
+    {128, 128, 4.98, 4.59, 0.0085, 0.235, 0.0, 0.185, 0.0045, 0.0010, 0.0051}};
 
 struct CallSize {
     double rows, kib, mb, moved;   // rows of the problem, KiB of a row of k, MB of operands, MB of peers and outputs
@@ -302,22 +305,70 @@ CallSize call_size(const GemmArgs &a, uint32_t es)
 double aligned_us(const GemmArgs &a, uint32_t es)
 {
     const CallSize c = call_size(a, es);
-    const double f = a.splitK > 1 ? a.splitK : 1.0, rounds = ceil(a.sched.coreLoops * f / 256.0), steps = c.kib * 16.0 / f;
+    const double f = a.splitK > 1 ? a.splitK : 1.0, wgs = a.sched.coreLoops * f, rounds = ceil(wgs / 256.0), steps = c.kib * 16.0 / f;
     if (a.sched.m0 == 256) return 10.0 + 0.78 * rounds * steps;
-    return 4.9 + rounds * (steps * (0.343 + (a.transB ? 0.048 : 0.0)) - 1.48) + (f > 1.0 ? 10.0 : 0.0) + (a.sched.op == OP_REDUCE_SCATTER ? 1.91 * a.nPeers : 0.0) +
-           0.14 * c.moved + 0.478 * c.mb;
+    return 6.6 + rounds * (steps * (0.325 + (a.transB ? 0.060 : 0.0) - (es == 1 ? 0.019 : 0.0)) - 2.0) + (wgs > 512.0 ? 0.104 * (wgs / 256.0 - 2.0) * steps : 0.0) +
+           (f > 1.0 ? 10.0 : 0.0) + (a.sched.op == OP_REDUCE_SCATTER ? 1.88 * a.nPeers : 0.0) + 0.134 * c.moved + 0.505 * c.mb;
 }
 
 // Flexible tiles as plan_flex left them in args.fx (blocks = rows / 64): whole, with a second launch for the peers, in k slices.
 double flex_us(const GemmArgs &a, uint32_t es, int blocks)
 {
     const CallSize c = call_size(a, es);
-    const double f = a.fx.slices > 1 ? a.fx.slices : 1.0, rounds = ceil((double)a.fx.rowTiles * a.fx.colTiles * f / 256.0), steps = rounds * c.kib * 16.0 / f;
+    const double f = a.fx.slices > 1 ? a.fx.slices : 1.0, wgs = (double)a.fx.rowTiles * a.fx.colTiles * f, rounds = ceil(wgs / 256.0), steps = c.kib * 16.0 / f;
     if (f > 1.0)
-        return 8.0 + steps * (a.transB ? 0.465 : 0.398) + 4e-6 * 0.1265 * f * (a.fx.keptOnly ? (double)a.keptRows : c.rows) * a.N + 0.227 * c.moved + 0.09 * c.mb;
-    if (a.fx.late) return 8.1 + steps * (a.transB ? 0.59 : 0.44) + 0.45 * c.moved;
-    return 3.75 + steps * (0.237 + (a.transB ? 0.118 : 0.0) + (blocks == 2 ? 0.224 : 0.0)) + 2.2 * rounds +
-           (a.sched.op == OP_REDUCE_SCATTER ? 1.1 * a.nPeers : 0.0) + 0.16 * c.moved + 0.132 * c.mb;
+        return 8.0 + rounds * steps * (a.transB ? 0.471 : 0.402) + 4e-6 * 0.1175 * f * (a.fx.keptOnly ? (double)a.keptRows : c.rows) * a.N + 0.225 * c.moved + 0.088 * c.mb;
+    if (a.fx.late) return 8.1 + rounds * steps * (a.transB ? 0.59 : 0.44) + 0.45 * c.moved;
+    return 2.5 + rounds * (steps * (0.239 + (a.transB ? 0.126 : 0.0) + (blocks == 2 ? 0.230 : 0.0)) + 3.2) - (wgs > 256.0 ? 0.0855 * wgs / 256.0 * steps : 0.0) +
+           (a.sched.op == OP_REDUCE_SCATTER ? 1.11 * a.nPeers : 0.0) + 0.156 * c.moved + 0.150 * c.mb;
+}
+
+// Rows of a mixed launch that run on 256x256 tiles: all but a reduce-scatter's kept ones and what fills the CUs that whole rounds of
+// large tiles leave idle.  A CU takes one workgroup at a time, the large ones first; `us` is when the last is done.
+struct MixedRows {
+    uint32_t large;
+    double us;
+};
+
+MixedRows mixed_rows(const GemmArgs &a, uint32_t es, uint32_t rows)
+{
+    const double chunks = call_size(a, es).kib * 8.0;
+    const uint32_t kept = a.sched.op == OP_REDUCE_SCATTER && a.sched.P > 1 ? a.keptRows : 0u;
+    const double large = 9.0 + 1.70 * chunks + (kept ? 0.0 : 4.4 * a.nPeers), small = 8.0 + 0.55 * chunks + 1.1 * a.nPeers;
+    const uint32_t largeCols = ceil_div(a.N, 256u), smallCols = ceil_div(a.N, 128u);
+    MixedRows best = {0, 0.0};
+    for (uint32_t t = 1; t <= ceil_div(rows - kept, 256u); ++t) {
+        const uint32_t r = umin(256u * t, rows - kept);
+        const double nLarge = (double)t * largeCols, nSmall = (double)ceil_div(rows - r, 128u) * smallCols;
+        const double full = floor(nLarge / 256.0), part = nLarge - 256.0 * full;
+        double us = full * large;
+        if (part == 0.0) {
+            us += ceil(nSmall / 256.0) * small;
+        } else {
+            const double idle = (256.0 - part) * floor(large / small), beside = ceil(nSmall / (256.0 - part)) * small;
+            if (nSmall <= idle) us += beside > large ? beside : large;
+            else us += large + ceil((nSmall - idle) / 256.0) * small;
+        }
+        if (best.large == 0 || us < best.us) best = {r, us};
+    }
+    return best;
+}
+
+void plan_mixed(GemmArgs &a, uint32_t es, uint32_t rows, uint32_t large)
+{
+    FlexParams &f = a.fx;
+    f.rows = large;
+    f.rowStep = 256;
+    f.perRank = 0;
+    f.rowTiles = ceil_div(large, 256u);
+    f.colTiles = ceil_div(a.N, 256u);
+    f.keptTile0 = f.keptTiles = 0;
+    f.tail = (uint32_t)((uint64_t)a.K * es % 128u);
+    f.slices = 1;
+    f.keptOnly = f.late = 0;
+    f.holeRows = rows - large;
+    f.hole0 = a.sched.op == OP_REDUCE_SCATTER && a.sched.P > 1 ? umin(a.keptBegin, large) : large;
+    f.largeTiles = f.rowTiles * f.colTiles;
 }
 
 // The streaming kernels for explicit kept rows, roughly.
@@ -351,7 +402,7 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other)
         if (sums && (t.cols != 128 || (t.rows < 128 && rows > (uint64_t)t.rows))) continue;
         const uint64_t n = (rows + t.rows - 1) / t.rows * ceil_div(a.N, t.cols);
         const double perCu = n > 256 ? n / 256.0 : 1.0, kib = (double)((n + 255) / 256) * c.kib * (t.rows + t.cols);
-        const double us = t.launch + t.workgroup * perCu + kib * (t.kib + (kBytes % 16 ? t.off16 : 0.0) + (a.transB ? 0.0 : t.kn)) + c.mb * t.mb +
+        const double us = t.launch + t.workgroup * perCu + kib * (t.kib + (kBytes % 16 ? t.off16 : 0.0) + (a.transB ? 0.0 : t.kn) + (n > 256 ? t.later : 0.0)) + c.mb * t.mb +
                           (!a.transB && t.cols * es < 128u ? c.mb * t.partLine : 0.0) + c.moved * t.moved;
         if (best == nullptr || us < least) {
             best = &t;
@@ -359,18 +410,31 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other)
             tiles = n;
         }
     }
-    if (best == nullptr || least > other || tiles > (1u << 24) || !flex_ptrs_ok(a)) return no;
+    if (best == nullptr) return no;
+    // (from half a round of large tiles' work on; k in at least a few pairs of steps; two ranks keep so many rows that small tiles are
+    // most of the launch: W8A8 3906x5600x3200 113 / 131, fp16 4790x6016x6272 369 / 394)
+    MixedRows mixed = {0, 0.0};
+    if (!sums && rows >= 512 && !(s.op == OP_REDUCE_SCATTER && s.P == 2) && kBytes >= 1024 && rows * a.N >= 128ull * 256ull * 256ull) {
+        mixed = mixed_rows(a, es, (uint32_t)rows);
+        mixed.us = mixed.us * (kBytes % 16 ? 0.81 : 0.68) + 0.113 * c.moved + 0.35 * c.mb;
+        if (mixed.us > least) mixed.large = 0;
+    }
+    if ((mixed.large ? mixed.us : least) > other || tiles > (1u << 24) || !flex_ptrs_ok(a)) return no;
+    a.fx.dRank = make_fast_div(s.mRank);
+    a.splitK = 0;
+    if (mixed.large) {
+        plan_mixed(a, es, (uint32_t)rows, mixed.large);
+        return {256, 256};
+    }
     a.fx.rows = (uint32_t)rows;
     a.fx.rowTiles = (uint32_t)((rows + best->rows - 1) / best->rows);
     a.fx.colTiles = ceil_div(a.N, best->cols);
-    a.fx.dRank = make_fast_div(s.mRank);
-    a.splitK = 0;
     return {best->rows, best->cols};
 }
 
 void launch_small(uint32_t dtype, const GemmArgs &a, const SmallTile &t, void *stream)
 {
-    launched(t.cols == 128 ? launch_gemm_mid(dtype, a, t.rows, stream) : launch_gemm_few(dtype, a, t.rows, t.cols, stream));
+    launched(t.cols == 256 ? launch_gemm_mixed(dtype, a, stream) : t.cols == 128 ? launch_gemm_mid(dtype, a, t.rows, stream) : launch_gemm_few(dtype, a, t.rows, t.cols, stream));
 }
 
 // Everything a launcher checks before it launches; fills `plan` except the buffer pointers.
@@ -904,9 +968,10 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
     a.outDtype = outDataType;
     // The plan above says what the launch is refused for and what it asks of the workspace, whichever kernel runs.
     const auto flex = [&]() {
-        // (at most eight rows of a long k and few columns as [n,k]: the whole-k kernel's rings of eight rows hold more of B than a 32x32
-        // tile's.  8x16384x2048 13.3 / 13.9, 1x12288x1024 10.8 / 11.5; the others 1x8192x8192 16.0 / 15.1, 16x4096x8192 10.6 / 9.4)
-        const bool deepK = sp.wholeK && a.M <= 8 && a.K > 8192 && a.N <= 4096;
+        // (few rows of a long k and few columns as [n,k]: the whole-k kernel's rings for up to eight rows hold more of B than a 32x32
+        // tile's.  8x16384x2048 13.3 / 13.9, 1x12288x1024 10.8 / 11.5, 1x8192x512 8.6 / 9.0; not 8x8192x2048 10.2 / 9.6, 8x12288x3072
+        // 13.6 / 11.9, 1x8192x8192 16.0 / 15.1, 16x4096x8192 10.6 / 9.4)
+        const bool deepK = sp.wholeK && (a.M <= 4 ? a.K >= 8192 && a.N <= (a.K > 8192 ? 4096u : 2048u) : a.M <= 8 && a.K > 12288 && a.N <= 2048);
         if (deepK || (!sp.maySmall && !sp.preferFlex)) return false;
         GemmArgs g = a;
         const uint32_t stages = d->workspaceStages ? d->workspaceStages : kDefaultStages;

@@ -40,6 +40,8 @@ struct FlexParams {
     long long *sliceSums;          // 64 x 128 block and slice: [128 x 128 block][slice][upper / lower 64 rows]
     uint32_t late;                 // whole tiles whose kept rows leave as 32-bit sums; a second launch adds their peers
     FastDiv dRank;                 // rows of one rank
+    uint32_t hole0, holeRows;      // mixed launches (gemm_mixed.h): rows [hole0, +holeRows) run on the small tiles, `rows` counts the others
+    uint32_t largeTiles;           // workgroups that run a 256x256 tile
 };
 
 struct GemmArgs {

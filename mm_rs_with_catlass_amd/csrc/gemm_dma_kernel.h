@@ -114,7 +114,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     static_assert(NS == 3 || (WM == 2 && NS >= 3 && NS <= 8), "deeper rings exist for the 128-row kernel");
     static_assert(MB == 2 || (MB == 1 && WM == 2 && (!RM || W8) && !RG && !TA), "64-row tiles exist for the four-wave geometry with A as [m,k]");
     static_assert(!W8 || (WM == 2 && MB == 1 && !RG && !TA), "eight waves on the 128-row tile: 32 rows per wave");
-    static_assert(!FX || (WM == 2 && !RM && !RG && !TA && !AQ && !W8 && !PP), "flexible mode exists for the plain ring of the four-wave geometry");
+    static_assert(!FX || (!RM && !RG && !TA && !AQ && !W8 && !PP && (WM == 2 || FX == 1)), "flexible mode exists for the plain rings, k slices for the four-wave geometry");
     static_assert(!AQ || (WM == 2 && NS == 6 && (MB == 2 || W8) && !TA), "pairs of A steps exist for the six-stage 128-row kernel with A as [m,k]");
     using Acc = typename AccOf<DT>::type;
     constexpr int ES = (DT == DT_I8) ? 1 : 2;   // bytes per operand element; a k step is 64 BYTES of K
@@ -128,7 +128,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     constexpr int A_DMA = BM / 16 / NW;  // 1 KiB copies per wave per stage
     constexpr int B_DMA = 16 / NW;
     constexpr int STEP_DMA = A_DMA + B_DMA;
-    constexpr int POOL = FX ? FlexPool<MB, NS>::BYTES : DmaPool<WM, NS, AQ, TB>::BYTES;
+    constexpr int POOL = FX && WM == 2 ? FlexPool<MB, NS>::BYTES : FX ? 160 * 1024 : DmaPool<WM, NS, AQ, TB>::BYTES;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -225,7 +225,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     for (int jj = 0; jj < A_DMA; ++jj) {
         if constexpr (FX) {
             const uint32_t row = ti.row + umin(16u * (w + NW * jj) + (lane >> 2), ti.rowsValid - 1u);
-            gA[jj] = flex_row_ptr(args, row, ldaB) + kOff + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
+            gA[jj] = flex_row_ptr(args, flex_row(args, row), ldaB) + kOff + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
         } else if constexpr (!TA) {
             gA[jj] = Ag + (size_t)(16 * (w + NW * jj) + (lane >> 2)) * ldaB + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
         } else if constexpr (ES == 1) {
@@ -441,6 +441,38 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     };
 #undef CATCOC_MMA
     auto nothing = [] {};
+    // Flexible mode on 256 rows: what whole pairs of steps leave of k (up to 128 bytes per row) comes first, through registers with
+    // bounds checks into the LDS of A's first pair and of B's first pair or two stages.
+    auto tail_pair = [&](unsigned char *sa, unsigned char *sb, auto read_a, auto read_b) {
+        const int tail = (int)args.fx.tail;
+        const size_t kEnd = (size_t)nkAll * 64;   // bytes of k in whole pairs
+        const unsigned char *b = (const unsigned char *)args.b;
+#pragma unroll 1
+        for (int q = 0; q < 256 * 8 / NT; ++q) {
+            const uint32_t idx = tid + NT * q, row = idx >> 3, p = idx & 7u, slot = (p ^ ((row >> 1) & 7u)) * 16u;
+            const int c = p * 16;
+            *(v4i *)(sa + row * 128 + slot) =
+                load16_guarded(flex_row_ptr(args, flex_row(args, ti.row + umin(row, ti.rowsValid - 1u)), ldaB) + kEnd + c, tail - c, tail - 4 - c);
+            if constexpr (TB) {
+                *(v4i *)(sb + row * 128 + slot) = load16_guarded(b + (size_t)(ti.col + umin(row, ti.colsValid - 1u)) * ldbB + kEnd + c, tail - c, tail - 4 - c);
+            } else {
+                constexpr int CH = 256 * ES / 16;   // pieces of a row of k; the stages of both steps lie behind each other
+                const int r = idx / CH, cb = (idx % CH) * 16, rows = tail / ES, width = ti.colsValid * ES;
+                *(v4i *)(sb + r * (256 * ES) + (((idx % CH) ^ (ES == 1 ? (r & 7u) << 1 : (r & 3u) << 2)) * 16)) =
+                    load16_guarded(b + (kEnd / ES + (r < rows ? r : rows - 1)) * ldbB + (size_t)ti.col * ES + cb, r < rows ? width - cb : 0, width - 4 - cb);
+            }
+        }
+        __syncthreads();
+        for (uint32_t t = 0; t < (tail > 64 ? 2u : 1u); ++t) {
+            read_a(fa0, t, 0);
+            read_b(fb0, t, 0);
+            read_a(fa1, t, 1);
+            read_b(fb1, t, 1);
+            mma(fa0, fb0);
+            mma(fa1, fb1);
+        }
+        __syncthreads();   // (the prologue's copies land here)
+    };
 
     if constexpr (WM == 2 && AQ) {
         // ---- NS B stages, NS / 2 + 1 A pair buffers.  B runs NS - 1 steps ahead as in the plain ring; pair q (steps 2q,
@@ -625,7 +657,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
                 for (int q = 0; q < PA; ++q) {
                     const uint32_t idx = tid + NT * q, row = idx >> 2;
                     const int c = (idx & 3u) * 16;
-                    pa[q] = load16_guarded(flex_row_ptr(args, ti.row + umin(row, ti.rowsValid - 1u), ldaB) + kEnd + c, tail - c, tail - 4 - c);
+                    pa[q] = load16_guarded(flex_row_ptr(args, flex_row(args, ti.row + umin(row, ti.rowsValid - 1u)), ldaB) + kEnd + c, tail - c, tail - 4 - c);
                 }
 #pragma unroll
                 for (int q = 0; q < PB; ++q) {
@@ -723,8 +755,14 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
 #pragma unroll
         for (int jj = 0; jj < APC; ++jj) {
             const int row = 8 * (w + NW * jj) + (lane >> 3);
-            gP[jj] = Ag + (size_t)row * ldaB + (((lane & 7) ^ ((row >> 1) & 7)) * 16);
-            gQ[jj] = Bg + (size_t)row * ldbB + (((lane & 7) ^ ((row >> 1) & 7)) * 16);
+            const uint32_t piece = ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+            if constexpr (FX) {
+                gP[jj] = flex_row_ptr(args, flex_row(args, ti.row + umin((uint32_t)row, ti.rowsValid - 1u)), ldaB) + piece;
+                gQ[jj] = Bg + (size_t)umin((uint32_t)row, ti.colsValid - 1u) * ldbB + piece;
+            } else {
+                gP[jj] = Ag + (size_t)row * ldaB + piece;
+                gQ[jj] = Bg + (size_t)row * ldbB + piece;
+            }
         }
         auto issue_ap = [&](uint32_t q) {   // pairs are issued in increasing q
 #pragma unroll
@@ -753,6 +791,10 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
         auto issue_even_b = [&](uint32_t kt, bool guard) {
             if ((kt & 1) == 0 && (!guard || kt + 4 < nk)) issue_bp((kt + 4) >> 1);
         };
+        if constexpr (FX) {
+            if (args.fx.tail != 0) tail_pair(stAP(0), stBP(0), [&](v4i (&af)[MB], uint32_t t, int kk) { load_ap(af, t, kk); },
+                                             [&](v4i (&bf)[4], uint32_t t, int kk) { bpar = t; load_b(bf, stBP(0), kk); });
+        }
         // prologue in steady-state order: A pair 0, B pairs 0 and 1
         issue_ap(0);
         issue_bp(0);
@@ -824,7 +866,9 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
 #pragma unroll
         for (int jj = 0; jj < APC; ++jj) {
             const int row = 8 * (w + NW * jj) + (lane >> 3);
-            gP[jj] = Ag + (size_t)row * ldaB + (((lane & 7) ^ ((row >> 1) & 7)) * 16);
+            const uint32_t piece = ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+            if constexpr (FX) gP[jj] = flex_row_ptr(args, flex_row(args, ti.row + umin((uint32_t)row, ti.rowsValid - 1u)), ldaB) + piece;
+            else gP[jj] = Ag + (size_t)row * ldaB + piece;
         }
         auto issue_ap = [&](uint32_t q) {   // pairs are issued in increasing q
 #pragma unroll
@@ -848,6 +892,10 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
         auto issue_step_a = [&](uint32_t kt, bool guard) {
             if ((kt & 1) == 0 && (!guard || kt + 2 < nk)) issue_ap((kt + 2) >> 1);
         };
+        if constexpr (FX) {
+            if (args.fx.tail != 0) tail_pair(stAP(0), stB(0), [&](v4i (&af)[MB], uint32_t t, int kk) { load_ap(af, t, kk); },
+                                             [&](v4i (&bf)[4], uint32_t t, int kk) { load_b(bf, stB(t), kk); });
+        }
         // prologue in steady-state order: B0, B1, pair 0, B2
         issue_b(offB4(0));
         if (nk > 1) issue_b(offB4(1));
@@ -901,7 +949,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
 
     if constexpr (FX) {
         if constexpr (FX == 2) flex_store_partial<MB>(args, acc, smem, ft, slice);
-        else flex_epilogue<DT, MB>(args, acc, smem, ft);
+        else flex_epilogue<DT, MB, NW>(args, acc, smem, ft);
         return;
     }
 

@@ -99,6 +99,9 @@ __device__ __forceinline__ void flex_task_of(const SchedParams &s, uint32_t r, u
     wsRow = ((round % s.stages) * s.blockPerComm + b) * s.m0 + (ri - mi * s.m0);
 }
 
+// Row of the problem that row v of the flexible tiles is: behind the hole that a mixed launch leaves to its small tiles.
+CATCOC_HD uint32_t flex_row(const GemmArgs &a, uint32_t v) { return a.fx.holeRows != 0 && v >= a.fx.hole0 ? v + a.fx.holeRows : v; }
+
 // Address of row v of the left operand (all-gather: row v of the shards behind each other).
 __device__ __forceinline__ const unsigned char *flex_row_ptr(const GemmArgs &a, uint32_t v, int64_t ldaB)
 {
@@ -130,6 +133,7 @@ enum : uint32_t { FX_SKIP = 0u, FX_KEPT = 1u << 30, FX_OUT = 2u << 30, FX_SUM = 
 
 constexpr int FLEX_STAGING = 4 * 16384;                 // one 16 KiB area per wave
 constexpr int FLEX_POOL = FLEX_STAGING + 128 * 8 + 16 * 8 * 8 + 16 * 4;   // + the row table + the sums of up to 16 tasks, per half wave
+constexpr int FLEX_POOL8 = 2 * FLEX_STAGING + 256 * 8 + 16 * 16 * 8 + 16 * 4;   // of eight waves and 256 rows
 
 // Sums over lanes, always in the same order: cross-lane adds in the vector unit (a shuffle is a trip through the LDS unit).
 template <int CTRL, int ROWS, typename T>
@@ -159,10 +163,12 @@ __device__ __forceinline__ T wave_sum64(T v)
 
 // acc[mb][nb][r] of wave (wm, wn) is element (row, col) of the tile with
 //   row = wm*32*MB + mb*32 + (r>>2)*8 + h*4 + (r&3),  col = wn*128 + nb*32 + c32
-template <uint32_t DT, int MB>
+// NW waves, two of them side by side: tiles of 16 * MB * NW rows.
+template <uint32_t DT, int MB, int NW = 4>
 __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename AccOf<DT>::type (&acc)[MB][4], unsigned char *smem, const FlexTile &t)
 {
     constexpr bool I8 = DT == DT_I8;
+    constexpr uint32_t ROWS = 16u * MB * NW, TABLE = NW == 4 ? 128u : ROWS;
     using Sum = typename std::conditional<I8, long long, double>::type;
     const int tid = threadIdx.x, lane = tid & 63;
     const uint32_t w = __builtin_amdgcn_readfirstlane((uint32_t)tid >> 6);
@@ -171,15 +177,15 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
     const bool redI32 = I8 && (args.flags & GF_REDUCE_INT32) != 0;
     const bool store = (args.flags & GF_OUTBOUND_STORE) != 0;
 
-    uint32_t *dst = (uint32_t *)(smem + FLEX_STAGING);      // [128] what row i of the tile does
-    float *rowScale = (float *)(dst + 128);                  // [128] W8A8 per-token scale
+    uint32_t *dst = (uint32_t *)(smem + NW * 16384);         // [TABLE] what row i of the tile does
+    float *rowScale = (float *)(dst + TABLE);                // [TABLE] W8A8 per-token scale
     // Sums of the tile's tasks (explicit kept rows: of its 128-column halves), [16][half wave]: a place per writer and a fixed
     // order of adding them up, so that sums of floats are the same bits in every launch.
-    Sum *sums = (Sum *)(rowScale + 128);
-    uint32_t *sumTask = (uint32_t *)(sums + 16 * 8);         // [16]
+    Sum *sums = (Sum *)(rowScale + TABLE);
+    uint32_t *sumTask = (uint32_t *)(sums + 16 * 2 * NW);    // [16]
     __syncthreads();   // every wave has left the main loop's LDS reads behind
-    if (tid < 64 * MB) {
-        const uint32_t v = t.row0 + tid;
+    if ((uint32_t)tid < ROWS) {
+        const uint32_t v = flex_row(args, t.row0 + tid);
         uint32_t e = FX_SKIP;
         if ((uint32_t)tid < t.rowsValid) {
             if (v - args.keptBegin < args.keptRows) {   // (unsigned: rows above keptBegin wrap)
@@ -200,9 +206,9 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
             }
         }
         dst[tid] = e;
-        if constexpr (I8) rowScale[tid] = args.scaleM[umin(v, args.fx.rows - 1u)];
+        if constexpr (I8) rowScale[tid] = args.scaleM[flex_row(args, umin(t.row0 + tid, args.fx.rows - 1u))];
     }
-    if (tid < 16 * 8) sums[tid] = 0;
+    if (tid < 16 * 2 * NW) sums[tid] = 0;
     __syncthreads();
 
     unsigned char *st = smem + w * 16384;
@@ -228,7 +234,8 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
     constexpr int NBUF = 3;
     const uint32_t keptEnd = args.keptBegin + args.keptRows;
     const uint32_t kLo = args.keptBegin > t.row0 ? umin(args.keptBegin - t.row0, t.rowsValid) : 0u;   // the tile's kept rows: [kLo, kLo + kN)
-    const uint32_t kN = keptEnd > t.row0 + kLo ? umin(keptEnd - t.row0, t.rowsValid) - kLo : 0u;
+    const bool none = args.fx.holeRows != 0 && args.sched.op == OP_REDUCE_SCATTER;   // (a mixed launch: they lie in the hole)
+    const uint32_t kN = !none && keptEnd > t.row0 + kLo ? umin(keptEnd - t.row0, t.rowsValid) - kLo : 0u;
     const int64_t kept0 = (int64_t)t.row0 + kLo - args.keptBegin;   // (of no use, and possibly negative, when the tile has none)
     const bool late = args.fx.late != 0;   // the kept rows' peers are the second launch's
     const bool tileKept = args.nPeers != 0 && kN != 0 && !late;
@@ -257,7 +264,7 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
     uint32_t runOf = (args.flags & GF_ROW_MASK) ? wn : 0u;
     auto flush = [&]() {
         const Sum s = half_sum64(run);
-        if (chunk == 31u) sums[runOf * 8u + w * 2u + lrow] = s;
+        if (chunk == 31u) sums[runOf * (2u * NW) + w * 2u + lrow] = s;
         run = 0;
     };
 
@@ -288,7 +295,7 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     const uint32_t i = wm * 32 * MB + mb * 32 + half * 16 + j * 2 + lrow;
-                    if (colOk && i < t.rowsValid) *(v4i *)((int32_t *)args.accDump + (size_t)(t.row0 + i) * args.N + gcol) = cur[j];
+                    if (colOk && i < t.rowsValid) *(v4i *)((int32_t *)args.accDump + (size_t)flex_row(args, t.row0 + i) * args.N + gcol) = cur[j];
                 }
             }
             auto add_peers = [&](auto add) {   // in slot order
@@ -391,7 +398,7 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
         __syncthreads();
         auto total = [&](uint32_t g) {
             Sum s = 0;
-            for (uint32_t i = 0; i < 8u; ++i) s += sums[g * 8u + i];
+            for (uint32_t i = 0; i < 2u * NW; ++i) s += sums[g * (2u * NW) + i];
             return s;
         };
         if (args.flags & GF_ROW_MASK) {

@@ -34,8 +34,10 @@ template <int MB> struct MidGeom
     static constexpr int UN = BM * BN / 4 / NT;     // groups of four columns per thread: 8 or 4
 };
 
+// Tile number pos of the rowTiles x colTiles over rows [rowBase, rowEnd) and all columns.  GA: A's rows are looked up one by one (all-gather:
+// they lie in the ranks' shards, one behind the other).
 template <uint32_t DT, bool TB, int MB, bool GA>
-__global__ void __launch_bounds__(512, 1) gemm_mid_kernel(const GemmArgs args)
+__device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *smem, uint32_t pos, uint32_t rowTiles, uint32_t colTiles, uint32_t rowBase, uint32_t rowEnd)
 {
     using G = MidGeom<MB>;
     using Acc = typename AccOf<DT>::type;
@@ -43,24 +45,22 @@ __global__ void __launch_bounds__(512, 1) gemm_mid_kernel(const GemmArgs args)
     constexpr int ES = I8 ? 1 : 2;
     constexpr int ACP = G::ACP, BCP = G::BCP, BM = G::BM, BN = G::BN, UN = G::UN, NS = G::NS, NT = G::NT;
     constexpr int PF = 3;                            // peers whose values are in flight or in registers at a time
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[G::POOL];
-
-    const uint32_t N = args.N, K = args.K, rows = args.fx.rows, rowTiles = args.fx.rowTiles, colTiles = args.fx.colTiles, flags = args.flags, keptBegin = args.keptBegin, keptRows = args.keptRows;
+    const uint32_t N = args.N, K = args.K, flags = args.flags, keptBegin = args.keptBegin, keptRows = args.keptRows;
     const int64_t peerLd = args.peerLd, peerRowOffset = args.peerRowOffset;
     const void *const a0 = args.a[0], *const b0 = args.b;
     asm volatile("" : : "s"(a0), "s"(b0), "s"(args.d), "s"(args.lda), "s"(args.ldb), "s"(args.ldd), "s"(peerLd), "s"(peerRowOffset),
-                 "s"(N), "s"(K), "s"(args.nPeers), "s"(keptBegin), "s"(keptRows), "s"(flags), "s"(args.outDtype), "s"(rows), "s"(rowTiles), "s"(colTiles));
+                 "s"(N), "s"(K), "s"(args.nPeers), "s"(keptBegin), "s"(keptRows), "s"(flags), "s"(args.outDtype), "s"(rowEnd), "s"(rowTiles), "s"(colTiles));
     const int tid = threadIdx.x, lane = tid & 63;
     const uint32_t w = __builtin_amdgcn_readfirstlane((uint32_t)tid >> 6);
     const uint32_t wg = w >> 2, wm = (w >> 1) & 1u, wn = w & 1u;   // half of the chunk, position
     const int c32 = lane & 31, h = lane >> 5;
     const SchedParams &sp = args.sched;
     // XCD x takes the x-th eighth of the tiles, in bands of eight tile rows: what is in flight on it is a compact block of the grid
-    const uint32_t seq = xcd_eighth(blockIdx.x, rowTiles * colTiles);
+    const uint32_t seq = xcd_eighth(pos, rowTiles * colTiles);
     const uint32_t band = seq / (8u * colTiles), in = seq - band * (8u * colTiles), bw = umin(8u, rowTiles - band * 8u);
     const uint32_t ct = in / bw, rt = band * 8u + (in - ct * bw);
-    const uint32_t row0 = rt * BM, col0 = ct * BN;
-    const uint32_t rowsValid = umin((uint32_t)BM, rows - row0), colsValid = umin((uint32_t)BN, N - col0);
+    const uint32_t row0 = rowBase + rt * BM, col0 = ct * BN;
+    const uint32_t rowsValid = umin((uint32_t)BM, rowEnd - row0), colsValid = umin((uint32_t)BN, N - col0);
     const uint32_t ldaB = (uint32_t)args.lda * ES, ldbB = (uint32_t)args.ldb * ES;
 
     // ---- the stream
@@ -179,34 +179,14 @@ __global__ void __launch_bounds__(512, 1) gemm_mid_kernel(const GemmArgs args)
             }
         }
     };
-    // ---- the peers of this thread's groups of four columns
-    const bool redI32 = I8 && (flags & GF_REDUCE_INT32) != 0;
-    const uint32_t keptEnd = keptBegin + keptRows;
-    const uint32_t kLo = keptBegin > row0 ? umin(keptBegin - row0, rowsValid) : 0u;   // the tile's kept rows: [kLo, kLo + kN)
-    const uint32_t kN = keptEnd > row0 + kLo ? umin(keptEnd - row0, rowsValid) - kLo : 0u;
-    const int64_t kept0 = (int64_t)row0 + kLo - keptBegin;   // (of no use, and possibly negative, when the tile has none)
-    constexpr uint32_t LPR = BN / 4;                 // lanes per row
-    const uint32_t urow = (uint32_t)tid / LPR, chunk = (uint32_t)tid % LPR;   // group j: row urow + j * (NT / LPR)
-    const uint32_t lcol = chunk * 4u, gcol = col0 + lcol;
-    const bool colOk = lcol < colsValid;
-    const uint32_t nPeers = kN ? args.nPeers : 0u;
-    v4i pv[PF][UN];
-    auto fetch = [&](v4i (&b)[UN], const void *from, bool there) {   // (an empty descriptor: zeros, no memory touched)
-        const float *base = (const float *)from + (peerRowOffset + kept0) * peerLd;
-        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, there ? 0x7ffffff0 : 0, 0x00020000);
-#pragma unroll
-        for (int j = 0; j < UN; ++j) {
-            const uint32_t r = urow + j * (NT / LPR) - kLo;   // (wraps in front of the kept rows)
-            b[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, r < kN && colOk ? r * ((uint32_t)peerLd * 4u) + gcol * 4u : 0xfffffff0u, 0, 2 /* nt */);
-        }
-    };
     v4f sN = {1.f, 1.f, 1.f, 1.f};
     v4i bv = {0, 0, 0, 0};
     float sM = 0.f;
     if constexpr (I8) {
-        if (colOk) {
-            sN = *(const v4f *)(args.scaleN + gcol);
-            if (args.bias) bv = *(const v4i *)(args.bias + gcol);
+        const uint32_t lc = ((uint32_t)tid % (BN / 4)) * 4u;
+        if (lc < colsValid) {
+            sN = *(const v4f *)(args.scaleN + col0 + lc);
+            if (args.bias) bv = *(const v4i *)(args.bias + col0 + lc);
         }
         if (tid < BM) sM = args.scaleM[row0 + umin((uint32_t)tid, rowsValid - 1u)];
     }
@@ -223,14 +203,14 @@ __global__ void __launch_bounds__(512, 1) gemm_mid_kernel(const GemmArgs args)
     // Fragment reads and copies behind the MFMAs, where they issue while the matrix pipe is busy: reads in one go in front of them hold
     // the MFMAs up until the LDS unit has taken all of them, one read behind each of eight MFMAs leaves the last one's latency to the
     // barrier (4096x4096x1024 bf16 48.2 us, 45, this order 43.7).
-    auto step = [&](auto S, auto COPY, uint32_t i) {
+    auto step = [&](auto S, auto COPY, uint32_t i) {   // COPY: in the middle of the range, every chunk in flight
         constexpr int s = decltype(S)::value;
         constexpr bool copy = decltype(COPY)::value;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if constexpr (copy) {
             CATCOC_WAIT_VMCNT((NS - 2) * G::CP);
         } else {
-            if (i + 1u < nChunks) wait_copies_but<G::CP, NS - 2>(nChunks - (i + 2u));
+            if (i + 1u < nChunks) wait_copies_but<G::CP, NS - 2>(umin(nChunks, i + NS) - (i + 2u));
             if (i + 1u == nChunks && lastBytes != 128u) mask_last(s);
         }
         barrier_keep_vmem();
@@ -250,8 +230,7 @@ __global__ void __launch_bounds__(512, 1) gemm_mid_kernel(const GemmArgs args)
                     read1(1 - s, 2 * q + 1);
                 }
             }
-            if constexpr (copy)
-                if (q == (MB == 2 ? 5 : 3)) issue(i + NS, old);
+            if (q == (MB == 2 ? 5 : 3) && (copy || i + NS < nChunks)) issue(i + NS, old);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -264,12 +243,34 @@ __global__ void __launch_bounds__(512, 1) gemm_mid_kernel(const GemmArgs args)
             step(S1, std::true_type{}, i + 1u);
         }
         for (; i < nChunks; i += 2u) {
-            if (i + NS < nChunks) step(S0, std::true_type{}, i);
-            else step(S0, std::false_type{}, i);
+            step(S0, std::false_type{}, i);
             if (i + 1u < nChunks) step(S1, std::false_type{}, i + 1u);
         }
     }
 
+    // ---- what a thread finishes: groups of four columns (worked out here: ahead of the loop it would cost registers the loop needs)
+    int t2 = tid;
+    asm volatile("" : "+v"(t2));
+    const bool redI32 = I8 && (flags & GF_REDUCE_INT32) != 0;
+    const uint32_t keptEnd = keptBegin + keptRows;
+    const uint32_t kLo = keptBegin > row0 ? umin(keptBegin - row0, rowsValid) : 0u;   // the tile's kept rows: [kLo, kLo + kN)
+    const uint32_t kN = keptEnd > row0 + kLo ? umin(keptEnd - row0, rowsValid) - kLo : 0u;
+    const int64_t kept0 = (int64_t)row0 + kLo - keptBegin;   // (of no use, and possibly negative, when the tile has none)
+    constexpr uint32_t LPR = BN / 4;                 // lanes per row
+    const uint32_t urow = (uint32_t)t2 / LPR, chunk = (uint32_t)t2 % LPR;   // group j: row urow + j * (NT / LPR)
+    const uint32_t lcol = chunk * 4u, gcol = col0 + lcol;
+    const bool colOk = lcol < colsValid;
+    const uint32_t nPeers = kN ? args.nPeers : 0u;
+    v4i pv[PF][UN];
+    auto fetch = [&](v4i (&b)[UN], const void *from, bool there) {   // (an empty descriptor: zeros, no memory touched)
+        const float *base = (const float *)from + (peerRowOffset + kept0) * peerLd;
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, there ? 0x7ffffff0 : 0, 0x00020000);
+#pragma unroll
+        for (int j = 0; j < UN; ++j) {
+            const uint32_t r = urow + j * (NT / LPR) - kLo;   // (wraps in front of the kept rows)
+            b[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, r < kN && colOk ? r * ((uint32_t)peerLd * 4u) + gcol * 4u : 0xfffffff0u, 0, 2 /* nt */);
+        }
+    };
     // ---- the two partial tiles meet; the first peers are on their way meanwhile
 #pragma unroll
     for (int p = 0; p < PF; ++p)
@@ -284,9 +285,9 @@ __global__ void __launch_bounds__(512, 1) gemm_mid_kernel(const GemmArgs args)
         for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const uint32_t row = (wm * MB + mb) * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
+                const uint32_t row = (wm * MB + mb) * 32 + (r >> 2) * 8 + (uint32_t)((t2 >> 5) & 1) * 4 + (r & 3);
                 const auto e = acc[mb][nb][r];
-                *(int *)(smem + ((wg * BM + row) * BN + (((wn * 2 + nb) * 32 + c32) ^ ((uint32_t)h * SWZ << 5))) * 4) = __builtin_bit_cast(int, e);
+                *(int *)(smem + ((wg * BM + row) * BN + (((wn * 2 + nb) * 32 + (t2 & 31)) ^ ((uint32_t)((t2 >> 5) & 1) * SWZ << 5))) * 4) = __builtin_bit_cast(int, e);
             }
     const bool store = (flags & GF_OUTBOUND_STORE) != 0;
     if (tid < BM) {
@@ -402,6 +403,13 @@ __global__ void __launch_bounds__(512, 1) gemm_mid_kernel(const GemmArgs args)
             __builtin_nontemporal_store(cur[j], (v4i *)((float *)args.outbound + (size_t)(d[j] & FX_INDEX) * sp.n0 + (col0 % sp.n0) + lcol));
         }
     }
+}
+
+template <uint32_t DT, bool TB, int MB, bool GA>
+__global__ void __launch_bounds__(512, 1) gemm_mid_kernel(const GemmArgs args)
+{
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[MidGeom<MB>::POOL];
+    mid_tile<DT, TB, MB, GA>(args, smem, blockIdx.x, args.fx.rowTiles, args.fx.colTiles, 0u, args.fx.rows);
 }
 
 template <uint32_t DT, bool TB, bool GA>

@@ -1,0 +1,43 @@
+// 256x256 tiles for as many rounds of workgroups as are full, small ones for the rest: large problems whose tiles do not come out even.
+//
+// The large tile is the one with the fewest bytes per product (gemm_dma_kernel.h, 256 rows on eight waves) in flexible mode: rows past
+// a rank's end, columns and bytes of k past the last one are nobody's business.  With one workgroup per CU a launch lasts as many rounds
+// as its fullest CU, and a last round of a few tiles costs as much as a full one; and a reduce-scatter's kept rows, in a few large
+// tiles, would wait for the peers' stream through as many CUs.  So some rows run on 128x128 tiles (gemm_mid.h) in the same launch: the
+// kept ones and as many more as fill the CUs that the large tiles leave idle.  The large tiles start first.
+//
+// Bound by the matrix pipes at their power limit: a large tile takes 9 + 1.7 us per 128 bytes of k, a small one 8 + 0.55 (about 1.0
+// PFLOP/s in 16 bits where all CUs have work; a library product of 8192 cubed 1.15).  GPU time per call, 128-row tiles -> this: fp16
+// reduce-scatter 8144x5120x1696 of eight ranks, as [n,k] (7126 rows on 196 large tiles, the kept 1018 on 112 small ones beside them), 197
+// -> 170 us, W8A8 2680x3200x6912 120 -> 84, 1384x6080x7936 134 -> 88, 3824x5632x6400 216 -> 155, bf16 reduce-scatter 4236x4952x3904 of four
+// 280 -> 200, all-gather 8 x [845,3328] x [3328,3936] 217 -> 186.  Which launches: small_tile().
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "gemm_mid.h"
+
+namespace catcoc {
+
+template <uint32_t DT, bool TB>
+__global__ void __launch_bounds__(512, 1) gemm_mixed_kernel(const GemmArgs args)
+{
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[160 * 1024];
+    const FlexParams &f = args.fx;
+    if (blockIdx.x < f.largeTiles) {
+        dma_tile<DT, 4, TB, false, false, false, 2, 3, false, false, false, 1>(args, smem, blockIdx.x, 0, 1u, 0);
+    } else {
+        mid_tile<DT, TB, 2, DT != DT_I8>(args, smem, blockIdx.x - f.largeTiles, ceil_div(f.holeRows, 128u), ceil_div(args.N, 128u), f.hole0, f.hole0 + f.holeRows);
+    }
+}
+
+template <uint32_t DT>
+inline int launch_mixed(const GemmArgs &args, void *stream)
+{
+    const dim3 grid(args.fx.largeTiles + ceil_div(args.fx.holeRows, 128u) * ceil_div(args.N, 128u)), block(512);
+    if (args.transB) hipLaunchKernelGGL((gemm_mixed_kernel<DT, true>), grid, block, 0, (hipStream_t)stream, args);
+    else hipLaunchKernelGGL((gemm_mixed_kernel<DT, false>), grid, block, 0, (hipStream_t)stream, args);
+    return (int)hipGetLastError();
+}
+
+}  // namespace catcoc

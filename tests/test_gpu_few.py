@@ -1,4 +1,4 @@
-"""GPU parity of the one-launch kernels for small tiles (csrc/gemm_few.h, csrc/gemm_mid.h) at the edges of their tiles and of k: W8A8 outputs,
+"""GPU parity of the one-launch kernels for small tiles (csrc/gemm_few.h, csrc/gemm_mid.h) and for mixed ones (csrc/gemm_mixed.h) at the edges of their tiles and of k: W8A8 outputs,
 workspace tiles and dumps bit for bit, float sums within the bound of two orders of the same additions."""
 import ctypes as C
 
@@ -166,8 +166,15 @@ def test_quant_kept_rows_with_checksums(case):
     assert np.array_equal(host16(out), want) and np.array_equal(dump.cpu().numpy(), acc) and np.array_equal(cs.cpu().numpy(), sums)
 
 
+def one_round(comm, M, K, N, P, rank):
+    """Tiling and descriptor of a call whose tiles all have a place of their own in the symmetric workspace."""
+    t, d = ops.default_tiling(M, K, N, P, m0=0, n0=0, k0=0), L.make_desc(rank, P, [16] * (P - 1))
+    t.commInterval = max(1, -(-L.load().catcoc_get_task_count(comm, C.byref(t), C.byref(d)) // 256))
+    return t, d
+
+
 # (operator, rows (of a shard), N, K, P, rank, weights as [n,k]): 64x128 and 128x128 tiles of the float operators
-@pytest.mark.parametrize("case", [("allreduce", 1000, 1544, 1234, 4, 0, False), ("allreduce", 650, 3332, 2310, 3, 0, True), ("allgather", 278, 4864, 4744, 2, 1, False), ("allreduce", 610, 4608, 5000, 8, 0, False),
+@pytest.mark.parametrize("case", [("allreduce", 1000, 1544, 1234, 4, 0, False), ("allreduce", 650, 3332, 2310, 3, 0, True), ("allgather", 278, 4864, 4736, 2, 1, False), ("allreduce", 610, 4608, 5000, 8, 0, False),
                                   ("reduce_scatter", 1392, 1540, 2820, 8, 5, True), ("reduce_scatter", 600, 4104, 1032, 2, 1, False)])
 def test_float_larger_tiles(case):
     _need_gpu()
@@ -188,8 +195,7 @@ def test_float_larger_tiles(case):
         out = ops.matmul_allreduce(A, Bd, peers, 0, P, trans_b=tb, acc_dump=dump)
         got = dump
     else:
-        t = ops.default_tiling(M, K, N, P, m0=0, n0=0, k0=0)
-        d = L.make_desc(rank, P, [16] * (P - 1))
+        t, d = one_round(L.MATMUL_REDUCE_SCATTER, M, K, N, P, rank)
         ob = torch.full((L.load().catcoc_get_workspace_size(L.MATMUL_REDUCE_SCATTER, L.BF16, C.byref(t), C.byref(d)) // 4,), 3.0, device="cuda:0")
         out = ops.matmul_reduce_scatter(A, Bd, peers, rank, P, tiling=t, trans_b=tb, outbound=ob, acc_dump=dump)
         tiles, full = ob.cpu().numpy().reshape(-1, 256), dump.cpu().numpy()
@@ -203,3 +209,45 @@ def test_float_larger_tiles(case):
     for p in peers:
         got = got + p
     assert torch.equal(out, got.bfloat16())
+
+
+# (rows per rank, N, K, P, rank, weights as [n,k], int32 peers): launches of 256x256 and 128x128 tiles; the kept rows (on small tiles) at the
+# start, in the middle and at the end, k of whole pairs of steps and 4 to 124 bytes more, columns past a tile
+@pytest.mark.parametrize("case", [(335, 6912, 3204, 8, 5, False, False), (543, 3844, 3836, 8, 0, True, True), (664, 3460, 5888, 8, 7, True, False)])
+def test_quant_mixed_tiles(case):
+    _need_gpu()
+    rows, N, K, P, rank, tb, ri = case
+    M = rows * P
+    g = torch.Generator(device="cuda:0").manual_seed(rows)
+    x1, x2 = (torch.randint(-127, 128, shape, dtype=torch.int8, device="cuda:0", generator=g) for shape in ((M, K), (K, N)))
+    s1, s2 = (torch.empty(c, device="cuda:0").uniform_(0.001, 0.02, generator=g) for c in (M, N))
+    b = torch.randint(-1000, 1000, (N,), dtype=torch.int32, device="cuda:0", generator=g)
+    peers = [torch.randint(-2 ** 20, 2 ** 20, (rows, N), dtype=torch.int32, device="cuda:0", generator=g) if ri else torch.randn((rows, N), device="cuda:0", generator=g)
+             for _ in range(P - 1)]
+    t, d = one_round(L.QUANT_MATMUL_REDUCE_SCATTER, M, K, N, P, rank)
+    size = L.load().catcoc_get_workspace_size(L.QUANT_MATMUL_REDUCE_SCATTER, L.INT8, C.byref(t), C.byref(d)) // 4
+    ob = torch.full((size,), 3, dtype=torch.int32 if ri else torch.float32, device="cuda:0")
+    dump, sums = torch.full((M, N), -7, dtype=torch.int32, device="cuda:0"), torch.full((rows, N), -7, dtype=torch.int32, device="cuda:0")
+    out = ops.quant_matmul_reduce_scatter(x1, x2.T.contiguous() if tb else x2, s1, s2, b, peers, rank, P, tiling=t, trans_b=tb, reduce_int32=ri, outbound=ob,
+                                          acc_dump=dump, c_accum=sums)
+    acc = (x1.double() @ x2.double()).to(torch.int32) + b   # (exact)
+    kept = acc[rank * rows:(rank + 1) * rows]
+    if ri:
+        kept = kept + sum(peers)
+    assert torch.equal(dump, acc) and torch.equal(sums, kept)
+    deq = lambda a, sm: (a.float() * s2) * sm[:, None]
+    want = deq(kept, s1[rank * rows:(rank + 1) * rows])
+    for p in ([] if ri else peers):
+        want = want + p
+    assert torch.equal(out, want.bfloat16())
+    full, tiles = (acc if ri else deq(acc, s1)), ob.reshape(-1, 256)
+    for task, r, row, col, ws in tasks_of(L.QUANT_MATMUL_REDUCE_SCATTER, t, d):
+        if r != rank:
+            r1, c1 = min(row + 128, (r + 1) * rows), min(col + 256, N)
+            assert torch.equal(tiles[ws:ws + r1 - row, :c1 - col], full[row:r1, col:c1]), task
+
+
+@pytest.mark.parametrize("case", [("allgather", 845, 3940, 3330, 8, 3, True), ("allgather", 822, 2308, 6560, 8, 0, True), ("allreduce", 3438, 5892, 3712, 4, 0, True),
+                                  ("reduce_scatter", 6184, 3072, 10752, 8, 2, False)])
+def test_float_mixed_tiles(case):
+    test_float_larger_tiles(case)
