@@ -371,6 +371,17 @@ void plan_mixed(GemmArgs &a, uint32_t es, uint32_t rows, uint32_t large)
     f.largeTiles = f.rowTiles * f.colTiles;
 }
 
+// Deals a reduce-scatter's kept rows out to the row tiles over `rows` rows (all of them, or those a mixed launch leaves).
+void deal_rows(GemmArgs &a, uint32_t es, uint32_t rows, uint32_t tileRows)
+{
+    const uint32_t tiles = ceil_div(rows, tileRows);
+    if (a.sched.op != OP_REDUCE_SCATTER || a.sched.P == 1 || (a.flags & GF_ROW_MASK) || tiles < 2 || (uint64_t)a.M * a.lda * es > 0x7fffffffull) return;
+    a.fx.dealRows = rows / tiles;
+    a.fx.dealRest = rows % tiles;
+    a.fx.dealKept = a.keptRows / tiles;
+    a.fx.dealKeptRest = a.keptRows % tiles;
+}
+
 // The streaming kernels for explicit kept rows, roughly.
 double streaming_us(const GemmArgs &a)
 {
@@ -419,16 +430,21 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other)
         mixed.us = mixed.us * (kBytes % 16 ? 0.81 : 0.68) + 0.113 * c.moved + 0.35 * c.mb;
         if (mixed.us > least) mixed.large = 0;
     }
+    // (with the kept rows dealt out the shares' margin is not needed: 199 reduce-scatters then take 1.009 of the best choice's time for each, 1.018
+    // with it; two of them lost 0.12 and 0.20, one of the two with the margin as well)
+    if (s.op == OP_REDUCE_SCATTER && !rowMask && (mixed.large || best->cols == 128)) other *= 1.15;
     if ((mixed.large ? mixed.us : least) > other || tiles > (1u << 24) || !flex_ptrs_ok(a)) return no;
     a.fx.dRank = make_fast_div(s.mRank);
     a.splitK = 0;
     if (mixed.large) {
         plan_mixed(a, es, (uint32_t)rows, mixed.large);
+        if (a.fx.holeRows) deal_rows(a, es, a.fx.holeRows, 128);
         return {256, 256};
     }
     a.fx.rows = (uint32_t)rows;
     a.fx.rowTiles = (uint32_t)((rows + best->rows - 1) / best->rows);
     a.fx.colTiles = ceil_div(a.N, best->cols);
+    if (best->cols == 128) deal_rows(a, es, (uint32_t)rows, best->rows);
     return {best->rows, best->cols};
 }
 

@@ -9,9 +9,14 @@
 // Bound by the matrix pipes at their power limit where the operands come out of the caches (0.47 us per chunk of a 128x128 tile, bf16 at
 // 1.09 GHz of MFMA issue, as the larger tiles' loops; without MFMAs the copies and reads alone take 0.32, without copies 0.35), by
 // HBM else (0.6), and by a fixed 5.5 us (launch apart) of first copies, partial tiles and output.  GPU time per call, other kernels -> this:
-// all-gather 8 x [512,4096] x [4096,1024] bf16 42.2 -> 39.6 us, W8A8 1000x1376x4096 of eight ranks, stored tiles, 26.2 -> 23.8, fp16
-// 683x7680x4864 153 -> 77, all-gather 278x4736x4864 of two 87 -> 46, W8A8 499x9120x2048 with 63 rows kept 99 -> 51.  Which launches:
-// small_tile().
+// all-gather 8 x [512,4096] x [4096,1024] bf16 42.2 -> 39.6 us, fp16 683x7680x4864 153 -> 77, all-gather 278x4736x4864 of two 87 -> 46, W8A8
+// 499x9120x2048 with 63 rows kept 99 -> 51.  Which launches: small_tile().
+//
+// A reduce-scatter's kept rows are dealt out to all row tiles.  One CU draws no more than about 40 bytes a nanosecond out of HBM, so
+// tiles of kept rows only (448 KiB of peers each with eight ranks) take 12 us longer than their neighbours; in shares of 16 rows a tile
+// the peers are all in flight at once and take under 2.  Tiles of consecutive rows -> dealt: W8A8 1000x1376x4096 of eight ranks, stored
+// tiles, 26.9 -> 19.6 us (other kernels 28.1), 2000x1376x4096 48.3 -> 36.2 (37.2), fp16 2784x960x2816 46.4 -> 33.1 (48.0), of two ranks and
+// W8A8 1000x1376x4096 24.6 -> 19.3.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -59,8 +64,19 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
     const uint32_t seq = xcd_eighth(pos, rowTiles * colTiles);
     const uint32_t band = seq / (8u * colTiles), in = seq - band * (8u * colTiles), bw = umin(8u, rowTiles - band * 8u);
     const uint32_t ct = in / bw, rt = band * 8u + (in - ct * bw);
-    const uint32_t row0 = rowBase + rt * BM, col0 = ct * BN;
-    const uint32_t rowsValid = umin((uint32_t)BM, rowEnd - row0), colsValid = umin((uint32_t)BN, N - col0);
+    const uint32_t col0 = ct * BN, colsValid = umin((uint32_t)BN, N - col0);
+    // Row i of the tile is row rowOf(i) of the problem.  Dealt rows: the tile's share of the kept ones (the first nk; kf kept rows belong to
+    // tiles in front), then its share of the others.
+    const FlexParams &f = args.fx;
+    const bool dealt = f.dealRows != 0;
+    const uint32_t row0 = dealt ? 0u : rowBase + rt * BM;   // what addresses of A's rows are relative to
+    const uint32_t first = dealt ? deal_begin(rt, f.dealRows, f.dealRest) : rt * BM, kf = dealt ? deal_begin(rt, f.dealKept, f.dealKeptRest) : 0u;
+    const uint32_t nk = dealt ? deal_begin(rt + 1u, f.dealKept, f.dealKeptRest) - kf : 0u;
+    const uint32_t rowsValid = dealt ? deal_begin(rt + 1u, f.dealRows, f.dealRest) - first : umin((uint32_t)BM, rowEnd - row0);
+    auto rowOf = [&](uint32_t i) -> uint32_t {
+        const uint32_t o = rowBase + first - kf + i - nk;
+        return !dealt ? row0 + i : i < nk ? keptBegin + kf + i : o >= keptBegin ? o + keptRows : o;
+    };
     const uint32_t ldaB = (uint32_t)args.lda * ES, ldbB = (uint32_t)args.ldb * ES;
 
     // ---- the stream
@@ -90,8 +106,8 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
 #pragma unroll
     for (int j = 0; j < ACP; ++j) {
         const uint32_t row = umin(arow(j), rowsValid - 1u);
-        if constexpr (GA) gA[j] = flex_row_ptr(args, row0 + row, ldaB) + apiece(j) * 16u;
-        else offA[j] = row * ldaB + apiece(j) * 16u;
+        if constexpr (GA) gA[j] = flex_row_ptr(args, rowOf(row), ldaB) + apiece(j) * 16u;
+        else offA[j] = (rowOf(row) - row0) * ldaB + apiece(j) * 16u;
     }
 #pragma unroll
     for (int j = 0; j < BCP; ++j) {
@@ -188,7 +204,7 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
             sN = *(const v4f *)(args.scaleN + col0 + lc);
             if (args.bias) bv = *(const v4i *)(args.bias + col0 + lc);
         }
-        if (tid < BM) sM = args.scaleM[row0 + umin((uint32_t)tid, rowsValid - 1u)];
+        if (tid < BM) sM = args.scaleM[rowOf(umin((uint32_t)tid, rowsValid - 1u))];
     }
 
     // Chunk i: its fragments are on their way since chunk i - 1; once they are here and this wave's copies of chunk i + 1 have
@@ -253,28 +269,39 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
     asm volatile("" : "+v"(t2));
     const bool redI32 = I8 && (flags & GF_REDUCE_INT32) != 0;
     const uint32_t keptEnd = keptBegin + keptRows;
-    const uint32_t kLo = keptBegin > row0 ? umin(keptBegin - row0, rowsValid) : 0u;   // the tile's kept rows: [kLo, kLo + kN)
-    const uint32_t kN = keptEnd > row0 + kLo ? umin(keptEnd - row0, rowsValid) - kLo : 0u;
-    const int64_t kept0 = (int64_t)row0 + kLo - keptBegin;   // (of no use, and possibly negative, when the tile has none)
+    const uint32_t kLo = !dealt && keptBegin > row0 ? umin(keptBegin - row0, rowsValid) : 0u;   // the tile's kept rows: [kLo, kLo + kN)
+    const uint32_t kN = dealt ? nk : keptEnd > row0 + kLo ? umin(keptEnd - row0, rowsValid) - kLo : 0u;
+    const int64_t keptRow0 = dealt ? (int64_t)kf : (int64_t)row0 - keptBegin;   // row i of the tile, if kept, is kept row keptRow0 + i
+    const int64_t kept0 = keptRow0 + kLo;   // (of no use, and possibly negative, when the tile has none)
     constexpr uint32_t LPR = BN / 4;                 // lanes per row
     const uint32_t urow = (uint32_t)t2 / LPR, chunk = (uint32_t)t2 % LPR;   // group j: row urow + j * (NT / LPR)
     const uint32_t lcol = chunk * 4u, gcol = col0 + lcol;
     const bool colOk = lcol < colsValid;
     const uint32_t nPeers = kN ? args.nPeers : 0u;
-    v4i pv[PF][UN];
-    auto fetch = [&](v4i (&b)[UN], const void *from, bool there) {   // (an empty descriptor: zeros, no memory touched)
+    // Dealt kept rows lie in a thread's first group or two: the registers of PF peers' eight groups then hold all peers at once.
+    v4i pv[PF * UN];
+    auto by_groups = [&](auto go) {
+        if (dealt && nk <= NT / LPR) go(std::integral_constant<int, 1>{});
+        else if (dealt && nk <= 2 * (NT / LPR)) go(std::integral_constant<int, 2>{});
+        else go(std::integral_constant<int, UN>{});
+    };
+    auto peers_at_once = [](int groups) constexpr -> int { return groups == UN ? PF : groups == 1 ? 8 : 4; };
+    auto fetch = [&](auto GR, int at, const void *from) {
+        constexpr int groups = decltype(GR)::value;
         const float *base = (const float *)from + (peerRowOffset + kept0) * peerLd;
-        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, there ? 0x7ffffff0 : 0, 0x00020000);
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, 0x7ffffff0, 0x00020000);
 #pragma unroll
-        for (int j = 0; j < UN; ++j) {
+        for (int j = 0; j < groups; ++j) {
             const uint32_t r = urow + j * (NT / LPR) - kLo;   // (wraps in front of the kept rows)
-            b[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, r < kN && colOk ? r * ((uint32_t)peerLd * 4u) + gcol * 4u : 0xfffffff0u, 0, 2 /* nt */);
+            pv[at * groups + j] = __builtin_amdgcn_raw_buffer_load_b128(rs, r < kN && colOk ? r * ((uint32_t)peerLd * 4u) + gcol * 4u : 0xfffffff0u, 0, 2 /* nt */);
         }
     };
     // ---- the two partial tiles meet; the first peers are on their way meanwhile
+    by_groups([&](auto GR) {
 #pragma unroll
-    for (int p = 0; p < PF; ++p)
-        if ((uint32_t)p < nPeers) fetch(pv[p], args.peers[p], true);
+        for (int p = 0; p < peers_at_once(decltype(GR)::value); ++p)
+            if ((uint32_t)p < nPeers) fetch(GR, p, args.peers[p]);
+    });
     __syncthreads();   // every wave has left the ring
     uint32_t *dst = (uint32_t *)(smem + G::MEET);   // [BM] what row i of the tile does
     float *rowScale = (float *)(dst + BM);         // [BM] W8A8 per-token scale
@@ -291,7 +318,7 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
             }
     const bool store = (flags & GF_OUTBOUND_STORE) != 0;
     if (tid < BM) {
-        const uint32_t v = row0 + tid;
+        const uint32_t v = rowOf(tid);
         uint32_t e = FX_SKIP;
         if ((uint32_t)tid < rowsValid) {
             if (v - keptBegin < keptRows) {
@@ -350,27 +377,30 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
 #pragma unroll
         for (int j = 0; j < UN; ++j) {
             const uint32_t row = urow + j * (NT / LPR);
-            if (row < rowsValid) *(v4i *)((int32_t *)args.accDump + (size_t)(row0 + row) * N + gcol) = cur[j];
+            if (row < rowsValid) *(v4i *)((int32_t *)args.accDump + (size_t)rowOf(row) * N + gcol) = cur[j];
         }
     }
     auto isKept = [&](int j) { return d[j] == FX_KEPT; };
     auto add_peers = [&](auto add) {   // in slot order; a row that is not kept adds the zeros its loads returned
-        for (uint32_t p = 0; p < nPeers; p += PF) {
+        by_groups([&](auto GR) {
+            constexpr int groups = decltype(GR)::value, atOnce = peers_at_once(groups);
+            for (uint32_t p = 0; p < nPeers; p += atOnce) {
 #pragma unroll
-            for (int q = 0; q < PF; ++q)
-                if (p + q < nPeers) {
+                for (int q = 0; q < atOnce; ++q)
+                    if (p + q < nPeers) {
 #pragma unroll
-                    for (int j = 0; j < UN; ++j) add(cur[j], pv[q][j], j);
-                    if (p + q + PF < nPeers) fetch(pv[q], args.peers[p + q + PF], true);
-                }
-        }
+                        for (int j = 0; j < groups; ++j) add(cur[j], pv[q * groups + j], j);
+                        if (p + q + atOnce < nPeers) fetch(GR, q, args.peers[p + q + atOnce]);
+                    }
+            }
+        });
     };
     if constexpr (I8) {
         if (redI32) add_peers([](v4i &c, const v4i &b, int) { c += b; });
         if (args.cAccum) {
 #pragma unroll
             for (int j = 0; j < UN; ++j)
-                if (isKept(j)) *(v4i *)(args.cAccum + (size_t)(row0 + urow + j * (NT / LPR) - keptBegin) * N + gcol) = cur[j];
+                if (isKept(j)) *(v4i *)(args.cAccum + (size_t)(keptRow0 + urow + j * (NT / LPR)) * N + gcol) = cur[j];
         }
 #pragma unroll
         for (int j = 0; j < UN; ++j) {   // per-channel scale first, then per-token, each product rounded on its own
@@ -398,7 +428,7 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
             uint32_t q[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) q[e] = f32_to_out16(i2f(cur[j][e]), args.outDtype) & 0xffffu;
-            *(v2i *)((unsigned short *)args.d + (size_t)(row0 + row - keptBegin) * args.ldd + gcol) = v2i{(int)(q[0] | (q[1] << 16)), (int)(q[2] | (q[3] << 16))};
+            *(v2i *)((unsigned short *)args.d + (size_t)(keptRow0 + row) * args.ldd + gcol) = v2i{(int)(q[0] | (q[1] << 16)), (int)(q[2] | (q[3] << 16))};
         } else if ((d[j] & FX_KIND) == FX_OUT) {
             __builtin_nontemporal_store(cur[j], (v4i *)((float *)args.outbound + (size_t)(d[j] & FX_INDEX) * sp.n0 + (col0 % sp.n0) + lcol));
         }

@@ -251,3 +251,16 @@ def test_quant_mixed_tiles(case):
                                   ("reduce_scatter", 6184, 3072, 10752, 8, 2, False)])
 def test_float_mixed_tiles(case):
     test_float_larger_tiles(case)
+
+
+# Kept rows dealt out to the 128- and 64-row tiles: 16 or fewer to a tile (one group of a thread's rows; of 16 ranks more peers than fit at
+# once), up to 32, up to 64 and as many as two ranks leave, tiles of unequal shares, first, last and a middle rank, columns past a tile
+@pytest.mark.parametrize("case", [(125, 4096, 1376, 8, 5, True, False), (65, 4096, 1040, 16, 15, False, True), (59, 4100, 1028, 16, 0, True, False), (123, 5116, 1660, 4, 1, True, False),
+                                  (500, 4096, 1376, 2, 1, True, True), (103, 1792, 1732, 8, 3, False, False), (299, 544, 1280, 8, 7, True, False)])
+def test_quant_dealt_rows(case):
+    test_quant_mixed_tiles(case)
+
+
+@pytest.mark.parametrize("case", [("reduce_scatter", 936, 6148, 1666, 8, 3, True), ("reduce_scatter", 1684, 2304, 520, 4, 0, False), ("reduce_scatter", 2400, 548, 1280, 16, 15, True)])
+def test_float_dealt_rows(case):
+    test_float_larger_tiles(case)
