@@ -1,7 +1,8 @@
-"""Builds libcatcoc_hip.so (the C-ABI library with the gfx950 kernels) in-tree with hipcc."""
+"""Builds libcatcoc_hip.so (the C-ABI library with the gfx950 kernels) in-tree with hipcc, and _host.so (the operators' calls from Python)."""
 import glob
 import os
 import subprocess
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 PKG = os.path.dirname(os.path.abspath(__file__))
@@ -9,6 +10,7 @@ ROOT = os.path.dirname(PKG)
 LIB = os.path.join(PKG, "libcatcoc_hip.so")
 HOST_EXAMPLE = os.path.join(PKG, "catcoc_quant_rs_host")   # C++ host driving the library through its C ABI alone
 FACADE_EXAMPLE = os.path.join(PKG, "catcoc_facade_host")  # C++ host written against the template facade (catcoc_hip/dgemm.hpp)
+HOST_CALL = os.path.join(PKG, "_host.so")
 OBJ_DIR = os.path.join(PKG, "csrc", "build")
 
 HIPCC_FLAGS = [
@@ -41,8 +43,24 @@ def build(verbose=False, extra=(), jobs=8):
             print(r.stderr)
         return obj
 
+    def host_call():   # plain C++ against torch's headers
+        import torch
+        t = os.path.dirname(torch.__file__)
+        cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+               "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I", os.path.join(ROOT, "include"),
+               "-I", os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), "-I", os.path.join(t, "include"),
+               "-I", os.path.join(t, "include", "torch", "csrc", "api", "include"), "-I", sysconfig.get_paths()["include"],
+               os.path.join(PKG, "csrc", "host_call.cpp"), "-o", HOST_CALL, "-L", os.path.join(t, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError("%s failed for host_call.cpp:\n%s" % (cmd[0], r.stderr))
+
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(host_call)
         objs = list(ex.map(compile_one, sources()))
+        host.result()
     # Link WITHOUT naming a HIP runtime: the library binds to the libamdhip64 its host process has
     # already loaded (a C/C++ host links it itself; a torch process carries its own copy, and a second
     # runtime in one process cannot open the device).

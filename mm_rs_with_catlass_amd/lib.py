@@ -205,6 +205,19 @@ def load():
     return L
 
 
+def load_host():
+    """The compiled call of an operator (csrc/host_call.cpp).  No fallback either: it is built with the library."""
+    L = load()
+    try:
+        from . import _host
+    except ImportError as e:
+        raise CatcocError("_host.so cannot be loaded (%s). Build it with `python -m mm_rs_with_catlass_amd._build` or __graft_entry__.build()." % e) from e
+    _host.attach(*(C.cast(getattr(L, n), C.c_void_p).value for n in (
+        "catcoc_get_kernel", "catcoc_launch_quant_matmul_reduce_scatter", "catcoc_get_task_count", "catcoc_default_tiling", "catcoc_last_status", "catcoc_last_error")),
+        CatcocError, CocTilingParams)
+    return _host
+
+
 def last_error():
     return load().catcoc_last_error().decode()
 

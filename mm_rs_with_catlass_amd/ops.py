@@ -46,6 +46,13 @@ def _stream():
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())   # of torch.cuda.current_stream(), without the object around it
 
 
+def _call(*args):
+    """The operator call in csrc/host_call.cpp, which takes this name's place: the output, or None where the call is one for the code below it."""
+    global _call
+    _call = _l.load_host().call
+    return _call(*args)
+
+
 def _ptr(t):
     return None if t is None else t.data_ptr()
 
@@ -125,6 +132,13 @@ def _kept_flag(kept_split):
     return 0 if kept_split is None else (_l.FLAG_KEPT_SPLIT if kept_split else _l.FLAG_KEPT_WHOLE)
 
 
+def _flags(outbound, linear_order, kept_split):
+    f = _l.OUTBOUND_STORE if outbound is not None else 0
+    if linear_order:
+        f |= _l.FLAG_LINEAR_ORDER
+    return f if kept_split is None else f | _kept_flag(kept_split)
+
+
 def _attach_workspace(d, workspace, split_k):
     """Optional scratch for k-sliced launches (kslice_plan() says how large) and the caller's own slice count."""
     d.splitK = split_k
@@ -174,8 +188,7 @@ def prepare_quant_matmul_reduce_scatter(x1, x2, scale_x1, scale_x2, bias=None, p
     t = tiling if tiling is not None else default_tiling(m, k, n, rank_size, m0=0, n0=0, k0=0)
     if (t.m, t.k, t.n) != (m, k, n):
         _fail("tiling says m,k,n = %d,%d,%d; the operands say %d,%d,%d", t.m, t.k, t.n, m, k, n)
-    flags = (_l.OUTBOUND_STORE if outbound is not None else 0) | (_l.FLAG_REDUCE_INT32 if reduce_int32 else 0) | \
-        (_l.FLAG_LINEAR_ORDER if linear_order else 0) | _kept_flag(kept_split)
+    flags = _flags(outbound, linear_order, kept_split) | (_l.FLAG_REDUCE_INT32 if reduce_int32 else 0)
     d = _desc(rank, rank_size, ptrs, peer_ld, peer_row_offset, flags, block_num, stages, swizzle, outbound, checksum, acc_dump)
     _attach_workspace(d, workspace, split_k)
     if checksum is not None:
@@ -209,6 +222,11 @@ def quant_matmul_reduce_scatter(x1, x2, scale_x1, scale_x2, bias=None, peers=(),
     tensor of kslice_plan() bytes with which a launch of few tiles cuts its k range into slices.
     Returns d_out [m/rank_size, n].
     """
+    done = _call(_l.QUANT_MATMUL_REDUCE_SCATTER, x1, x2, scale_x1, scale_x2, bias, peers, rank, rank_size, tiling, trans_a, trans_b, peer_row_offset,
+                 _flags(outbound, linear_order, kept_split) | (_l.FLAG_REDUCE_INT32 if reduce_int32 else 0), outbound, checksum, acc_dump, c_accum, workspace, out,
+                 out_dtype, block_num, stages, swizzle, split_k, 0, 0, 0)
+    if done is not None:
+        return done
     launch, out = prepare_quant_matmul_reduce_scatter(
         x1, x2, scale_x1, scale_x2, bias, peers, rank, rank_size, out_dtype, tiling, trans_b, peer_row_offset,
         reduce_int32, outbound, checksum, acc_dump, c_accum, block_num, stages, swizzle, linear_order, out, workspace, split_k,
@@ -284,9 +302,16 @@ def prepare_quant_matmul_splitk(x1, x2, scale_x1, scale_x2, bias=None, peers=(),
     return launch, out
 
 
-def quant_matmul_splitk(*args, **kw):
+def quant_matmul_splitk(x1, x2, scale_x1, scale_x2, bias=None, peers=(), rank_size=1, kept_row_begin=0, kept_rows=None, out_dtype=torch.bfloat16, split_k=0,
+                        workspace=None, checksum=None, acc_dump=None, c_accum=None, peer_row_offset=0, block_num=0, swizzle=None, out=None, n0=0, trans_b=False,
+                        reduce_int32=False):
     """One launch of prepare_quant_matmul_splitk(); returns d_out [kept_rows, n]."""
-    launch, out = prepare_quant_matmul_splitk(*args, **kw)
+    done = _call(4, x1, x2, scale_x1, scale_x2, bias, peers, 0, rank_size, None, False, trans_b, peer_row_offset, _l.FLAG_REDUCE_INT32 if reduce_int32 else 0, None,
+                 checksum, acc_dump, c_accum, workspace, out, out_dtype, block_num, 0, swizzle, split_k, kept_row_begin, kept_rows, n0)
+    if done is not None:
+        return done
+    launch, out = prepare_quant_matmul_splitk(x1, x2, scale_x1, scale_x2, bias, peers, rank_size, kept_row_begin, kept_rows, out_dtype, split_k, workspace, checksum,
+                                              acc_dump, c_accum, peer_row_offset, block_num, swizzle, out, n0, trans_b, reduce_int32)
     launch()
     _l.check()
     return out
@@ -332,7 +357,7 @@ def _float_op(comm_type, a, b, c_shape, peers, rank, rank_size, tiling, trans_a,
     t = tiling if tiling is not None else default_tiling(m_for_tiling, k, n, rank_size, m0=0, n0=0, k0=0)
     if (t.m, t.k, t.n) != (m_for_tiling, k, n):
         _fail("tiling says m,k,n = %d,%d,%d; the operands say %d,%d,%d", t.m, t.k, t.n, m_for_tiling, k, n)
-    flags = (_l.OUTBOUND_STORE if outbound is not None else 0) | (_l.FLAG_LINEAR_ORDER if linear_order else 0) | _kept_flag(kept_split)
+    flags = _flags(outbound, linear_order, kept_split)
     d = _desc(rank, rank_size, ptrs, peer_ld, peer_row_offset, flags, block_num, stages, swizzle, outbound, checksum, acc_dump)
     _attach_workspace(d, workspace, split_k)
     if checksum is not None:
@@ -351,6 +376,10 @@ def matmul_reduce_scatter(a, b, peers=(), rank=0, rank_size=1, tiling=None, tran
                           peer_row_offset=0, outbound=None, checksum=None, acc_dump=None, block_num=0, stages=0,
                           swizzle=None, linear_order=False, out=None, workspace=None, split_k=0, kept_split=None):
     """fp16/bf16 matmul -> reduce-scatter share: a [m,k], b [k,n], peers fp32; returns [m/rank_size, n]."""
+    done = _call(_l.MATMUL_REDUCE_SCATTER, a, b, None, None, None, peers, rank, rank_size, tiling, trans_a, trans_b, peer_row_offset, _flags(outbound, linear_order, kept_split), outbound, checksum, acc_dump, None, workspace, out,
+                 None, block_num, stages, swizzle, split_k, 0, 0, 0)
+    if done is not None:
+        return done
     m = a.shape[1] if trans_a else a.shape[0]
     return _float_op(_l.MATMUL_REDUCE_SCATTER, a, b, lambda n: (m // max(rank_size, 1), n), peers, rank, rank_size,
                      tiling, trans_a, trans_b, peer_row_offset, outbound, checksum, acc_dump, block_num, stages,
@@ -361,6 +390,10 @@ def matmul_allreduce(a, b, peers=(), rank=0, rank_size=1, tiling=None, trans_a=F
                      peer_row_offset=0, acc_dump=None, block_num=0, stages=0, swizzle=None, linear_order=False,
                      out=None, workspace=None, split_k=0):
     """fp16/bf16 matmul -> all-reduce share: every row is kept; peers are full [m,n] fp32 partials."""
+    done = _call(_l.MATMUL_ALLREDUCE, a, b, None, None, None, peers, rank, rank_size, tiling, trans_a, trans_b, peer_row_offset, _l.FLAG_LINEAR_ORDER if linear_order else 0, None, None, acc_dump, None, workspace, out,
+                 None, block_num, stages, swizzle, split_k, 0, 0, 0)
+    if done is not None:
+        return done
     m = a.shape[1] if trans_a else a.shape[0]
     return _float_op(_l.MATMUL_ALLREDUCE, a, b, lambda n: (m, n), peers, rank, rank_size, tiling, trans_a, trans_b,
                      peer_row_offset, None, None, acc_dump, block_num, stages, swizzle, linear_order, out, m, workspace, split_k)
@@ -370,6 +403,10 @@ def allgather_matmul(a_local, peer_shards, b, rank=0, rank_size=1, tiling=None, 
                      block_num=0, stages=0, swizzle=None, linear_order=False, out=None, workspace=None, split_k=0):
     """all-gather -> matmul: a_local [m,k] is this rank's shard, peer_shards the other ranks' shards in
     ascending rank order (separate buffers, read in place); returns [m*rank_size, n]."""
+    done = _call(_l.ALLGATHER_MATMUL, a_local, b, None, None, None, peer_shards, rank, rank_size, tiling, False, trans_b, 0, _l.FLAG_LINEAR_ORDER if linear_order else 0, None, None, acc_dump, None, workspace, out,
+                 None, block_num, stages, swizzle, split_k, 0, 0, 0)
+    if done is not None:
+        return done
     m = a_local.shape[0]
     return _float_op(_l.ALLGATHER_MATMUL, a_local, b, lambda n: (m * rank_size, n), peer_shards, rank, rank_size,
                      tiling, False, trans_b, 0, None, None, acc_dump, block_num, stages, swizzle, linear_order, out, m,
