@@ -448,9 +448,9 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other)
     return {best->rows, best->cols};
 }
 
-void launch_small(uint32_t dtype, const GemmArgs &a, const SmallTile &t, void *stream)
+int launch_small(uint32_t dtype, const GemmArgs &a, const SmallTile &t, void *stream)
 {
-    launched(t.cols == 256 ? launch_gemm_mixed(dtype, a, stream) : t.cols == 128 ? launch_gemm_mid(dtype, a, t.rows, stream) : launch_gemm_few(dtype, a, t.rows, t.cols, stream));
+    return t.cols == 256 ? launch_gemm_mixed(dtype, a, stream) : t.cols == 128 ? launch_gemm_mid(dtype, a, t.rows, stream) : launch_gemm_few(dtype, a, t.rows, t.cols, stream);
 }
 
 // Everything a launcher checks before it launches; fills `plan` except the buffer pointers.
@@ -711,7 +711,7 @@ bool launched_small(const Plan &p, bool dma, bool flex, void *stream)
     GemmArgs g = p.args;
     const uint32_t es = elem_size(p.dtype);
     const SmallTile t = small_tile(g, es, dma ? kAlignedShare * aligned_us(p.args, es) : flex ? kOtherShare * flex_us(p.args, es, p.flexBlocks) : 1e30);
-    if (t.rows) launch_small(p.dtype, g, t, stream);
+    if (t.rows) launched(launch_small(p.dtype, g, t, stream));
     return t.rows != 0;
 }
 
@@ -941,7 +941,7 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
         if (sp.maySmall) {   // (the rest of these shapes runs whole 64x256 tiles or one thread per element, many times slower)
             GemmArgs g = a;
             const SmallTile t = small_tile(g, 1, 1e30);
-            if (t.rows) { launch_small(DT_I8, g, t, stream); return; }
+            if (t.rows) { launched(launch_small(DT_I8, g, t, stream)); return; }
         }
         const bool flex = sp.flexBlocks != 0 && flex_ptrs_ok(a);
         if (!flex && a.sched.n0 != 128) {
@@ -1006,7 +1006,7 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
         if (sp.maySmall) {
             const SmallTile t = small_tile(small, 1, sp.wholeK ? 1e30 : kOtherShare * (blocks ? flex_us(g, 1, blocks) : streaming_us(g)));
             if (t.rows) {
-                launch_small(DT_I8, small, t, stream);
+                launched(launch_small(DT_I8, small, t, stream));
                 return true;
             }
         }
@@ -1192,9 +1192,22 @@ void launch_pipelined(bool quant, int dataType, void *computeStream, void *commS
     // ranks 4096x4096x2048 58.3 -> 50.9, four 2048x512x4096 24.6 -> 21.0; not 288 tiles of eight 2048x2048x4608 47.6 -> 56.3, 256 of
     // four 2048x4096x4096 52.8 -> 59.8.
     const bool oneRound = sp.coreLoops <= sp.blockPerComm;
-    const bool fused = quant && dma && flexBlocks == 0 && P > 1 && oneRound &&
-                       (sp.coreLoops >= 384u || sp.coreLoops <= 128u || P == 2 || (P <= 4 && tiling->k <= 2048u));
+    bool fused = quant && dma && flexBlocks == 0 && P > 1 && oneRound &&
+                 (sp.coreLoops >= 384u || sp.coreLoops <= 128u || P == 2 || (P <= 4 && tiling->k <= 2048u));
     if (fused) g.nPeers = P - 1;
+    // Small or mixed tiles do the same in one launch, for problems of any alignment.  The fused operator's choice, with the comm launch on the
+    // other side where it is not fused, and where the two come out close the other side (estimates within 0.2 of each other: 0.04 to 0.09
+    // lost in seven of 71 calls without that).  GEMM and comm launch -> one, us, one row-block round of eight ranks: 1024x3904x768 40.4 ->
+    // 16.3, 2048x10672x1024 68.8 -> 38.7, 3072x2304x6176 91.5 -> 70.9, 4096x8960x7072 325 -> 280, of four 512x3604x640 45.0 -> 11.8, of two
+    // 1792x6784x1024 49.7 -> 24.7; the other way round 4096x1792x4096 48.9 / 59.7, 3072x576x1792 24.1 / 26.6.
+    SmallTile small = {0, 0};
+    GemmArgs gs = g;
+    if (quant && P > 1 && oneRound && (given->flags & (CATCOC_FLAG_LINEAR_ORDER | CATCOC_FLAG_KEPT_WHOLE | CATCOC_FLAG_KEPT_SPLIT)) == 0) {
+        const double comm = fused ? 0.0 : 4.5 + 0.8 * (P - 1) + 0.1e-6 * 4.0 * (P - 1) * g.keptRows * g.N;
+        gs.nPeers = P - 1;
+        small = small_tile(gs, 1, flexBlocks ? 0.8 * kOtherShare * (flex_us(g, 1, flexBlocks) + comm) : dma ? 0.8 * kAlignedShare * (aligned_us(g, 1) + comm) : 1e30);
+    }
+    if (small.rows) fused = true;
     // (a single round may run in the order of the fused operators: 4096x8192x8192 of two ranks, as [n,k], two launches 405 -> 337)
     if (oneRound && (given->flags & CATCOC_FLAG_LINEAR_ORDER) == 0) g.flags &= ~(uint32_t)GF_LINEAR_ORDER;
     const bool commWritesOutput = quant && !fused && deterministic != 0 && P > 1 && (uintptr_t)scale_x2 % 16 == 0 && (uintptr_t)d_out % 8 == 0;
@@ -1258,7 +1271,8 @@ void launch_pipelined(bool quant, int dataType, void *computeStream, void *commS
         g.taskBase = first;
         g.taskCount = oneRound ? 0 : actual;
         if (he == hipSuccess)
-            e = flexBlocks ? launch_flex(p.dtype, g, flexBlocks, computeStream)
+            e = small.rows ? launch_small(p.dtype, gs, small, computeStream)
+                : flexBlocks ? launch_flex(p.dtype, g, flexBlocks, computeStream)
                 : dma ? (p.dtype == DT_I8 ? launch_gemm_dma_i8(g, computeStream)
                        : p.dtype == DT_F16 ? launch_gemm_dma_f16(g, computeStream) : launch_gemm_dma_bf16(g, computeStream))
                     : launch_gemm(p.dtype, g, p.variant, p.edge, computeStream);

@@ -293,6 +293,12 @@ def test_pipelined_quant_one_round_on_aligned_tiles(case, deterministic):
     test_pipelined_quant_one_round(case, deterministic)
 
 
+# one-round pipelined calls that one launch of small tiles takes: 128 and 64 rows by 128 columns, 32 and 64 rows by 64, ranks of ragged rows
+@pytest.mark.parametrize("case", [(512, 2048, 1664, 4, 1, True), (128, 1408, 1504, 8, 6, True), (61, 1540, 1236, 8, 2, True), (96, 1040, 1280, 8, 0, False), (384, 1024, 1028, 2, 1, True)])
+def test_pipelined_quant_one_round_on_small_tiles(case):
+    test_pipelined_quant_one_round(case, True)
+
+
 @pytest.mark.parametrize("tb", [False, True])
 def test_pipelined_quant_one_round_equals_two(tb):
     """384 tiles: one round (the GEMM launch adds the peers) against two rounds with comm launches."""
