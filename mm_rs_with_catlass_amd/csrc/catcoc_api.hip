@@ -317,7 +317,7 @@ double flex_us(const GemmArgs &a, uint32_t es, int blocks)
     const CallSize c = call_size(a, es);
     const double f = a.fx.slices > 1 ? a.fx.slices : 1.0, wgs = (double)a.fx.rowTiles * a.fx.colTiles * f, rounds = ceil(wgs / 256.0), steps = c.kib * 16.0 / f;
     if (f > 1.0)
-        return 8.0 + rounds * steps * (a.transB ? 0.471 : 0.402) + 4e-6 * 0.1175 * f * (a.fx.keptOnly ? (double)a.keptRows : c.rows) * a.N + 0.225 * c.moved + 0.088 * c.mb;
+        return 9.1 + rounds * steps * (a.transB ? 0.434 : 0.345) + 4e-6 * 0.095 * f * (a.fx.keptOnly ? (double)a.keptRows : c.rows) * a.N + 0.263 * c.moved + 0.112 * c.mb;
     if (a.fx.late) return 8.1 + rounds * steps * (a.transB ? 0.59 : 0.44) + 0.45 * c.moved;
     return 2.5 + rounds * (steps * (0.239 + (a.transB ? 0.126 : 0.0) + (blocks == 2 ? 0.230 : 0.0)) + 3.2) - (wgs > 256.0 ? 0.0855 * wgs / 256.0 * steps : 0.0) +
            (a.sched.op == OP_REDUCE_SCATTER ? 1.11 * a.nPeers : 0.0) + 0.156 * c.moved + 0.150 * c.mb;
@@ -401,8 +401,8 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other)
     if (a.transA || kBytes % 4 != 0 || kBytes < 16 || (!a.transB && ldbB % 16 != 0) || a.N % 4 != 0 || ldaB * 160u > 0x7fffffffull || ldbB * 160u > 0x7fffffffull ||
         rows >= (1u << 30) || s.n0 != 256 || (s.m0 != 64 && s.m0 != 128))
         return no;
-    // Checksums: of tasks of a reduce-scatter the other kernels', of the 128x128 blocks of explicit kept rows those of a tile that
-    // has all rows of one.  Decode launches that also want the kept rows' int32 block stay where their k slices leave it on the way.
+    // Checksums: of tasks of a reduce-scatter the other kernels'; of the 128x128 blocks of explicit kept rows, tiles that have all of one,
+    // or those that meet in the workspace's counter block (block_add).  Decode launches that also want the kept rows' int32 block stay where their k slices leave it on the way.
     const bool rowMask = (a.flags & GF_ROW_MASK) != 0, sums = (a.flags & GF_OUTBOUND_STORE) == 0 && a.checksum != nullptr && (rowMask || a.keptRows < rows);
     if ((sums && !rowMask) || (rowMask && a.cAccum != nullptr)) return no;
     const CallSize c = call_size(a, es);
@@ -410,9 +410,10 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other)
     double least = 0.0;
     uint64_t tiles = 0;
     for (const SmallTileCost &t : kSmallTiles) {
-        if (sums && (t.cols != 128 || (t.rows < 128 && rows > (uint64_t)t.rows))) continue;
+        if (sums && (t.cols != 128 || (t.rows < 128 && rows > (uint64_t)t.rows)) && (a.skCount == nullptr || (rows + 127) / 128 * ceil_div(a.N, 128u) > kCounterBlockBytes / 8u))
+            continue;
         const uint64_t n = (rows + t.rows - 1) / t.rows * ceil_div(a.N, t.cols);
-        const double perCu = n > 256 ? n / 256.0 : 1.0, kib = (double)((n + 255) / 256) * c.kib * (t.rows + t.cols);
+        const double rounds = (double)((n + 255) / 256), perCu = t.cols < 128 || n <= 256 ? rounds : n / 256.0, kib = rounds * c.kib * (t.rows + t.cols);
         const double us = t.launch + t.workgroup * perCu + kib * (t.kib + (kBytes % 16 ? t.off16 : 0.0) + (a.transB ? 0.0 : t.kn) + (n > 256 ? t.later : 0.0)) + c.mb * t.mb +
                           (!a.transB && t.cols * es < 128u ? c.mb * t.partLine : 0.0) + c.moved * t.moved;
         if (best == nullptr || us < least) {
@@ -924,6 +925,12 @@ bool decode_flex_pays(const GemmArgs &g, bool large)
     return !large && (g.K > 256 ? g.nPeers <= 1 || g.M >= 128 : g.nPeers == 0);
 }
 
+// The workspace's counter block, if the caller gave one.
+uint32_t *counter_block(const CatcocSymmetricDesc &d)
+{
+    return d.workspace != nullptr && (uintptr_t)d.workspace % 256 == 0 && d.workspaceBytes >= kCounterBlockBytes ? (uint32_t *)d.workspace : nullptr;
+}
+
 void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_x1, uint8_t *scale_x2, uint8_t *bias,
                          uint8_t *c_accum, uint8_t *d_out, const CatcocSymmetricDesc *d, CocTilingParams *tiling,
                          uint32_t transA, uint32_t transB, uint32_t outDataType)
@@ -940,6 +947,7 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
         a.outDtype = outDataType;
         if (sp.maySmall) {   // (the rest of these shapes runs whole 64x256 tiles or one thread per element, many times slower)
             GemmArgs g = a;
+            g.skCount = counter_block(*d);
             const SmallTile t = small_tile(g, 1, 1e30);
             if (t.rows) { launched(launch_small(DT_I8, g, t, stream)); return; }
         }
@@ -996,6 +1004,7 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
         g.splitK = 0;
         g.skCount = nullptr;
         GemmArgs small = g;
+        small.skCount = counter_block(*d);
         int blocks = 0;
         if (sp.preferFlex && !sp.wholeK) {
             const FlexSlices c = flex_choose(g, 1, 0, 0);
@@ -1196,8 +1205,8 @@ void launch_pipelined(bool quant, int dataType, void *computeStream, void *commS
                  (sp.coreLoops >= 384u || sp.coreLoops <= 128u || P == 2 || (P <= 4 && tiling->k <= 2048u));
     if (fused) g.nPeers = P - 1;
     // Small or mixed tiles do the same in one launch, for problems of any alignment.  The fused operator's choice, with the comm launch on the
-    // other side where it is not fused, and where the two come out close the other side (estimates within 0.2 of each other: 0.04 to 0.09
-    // lost in seven of 71 calls without that).  GEMM and comm launch -> one, us, one row-block round of eight ranks: 1024x3904x768 40.4 ->
+    // other side where it is not fused, and 0.9 of that (102 calls: none loses; at 1.0 eight lose 0.02 to 0.14, at 0.8 eight more miss 0.06 to
+    // 0.6).  GEMM and comm launch -> one, us, one row-block round of eight ranks: 1024x3904x768 40.4 ->
     // 16.3, 2048x10672x1024 68.8 -> 38.7, 3072x2304x6176 91.5 -> 70.9, 4096x8960x7072 325 -> 280, of four 512x3604x640 45.0 -> 11.8, of two
     // 1792x6784x1024 49.7 -> 24.7; the other way round 4096x1792x4096 48.9 / 59.7, 3072x576x1792 24.1 / 26.6.
     SmallTile small = {0, 0};
@@ -1205,7 +1214,7 @@ void launch_pipelined(bool quant, int dataType, void *computeStream, void *commS
     if (quant && P > 1 && oneRound && (given->flags & (CATCOC_FLAG_LINEAR_ORDER | CATCOC_FLAG_KEPT_WHOLE | CATCOC_FLAG_KEPT_SPLIT)) == 0) {
         const double comm = fused ? 0.0 : 4.5 + 0.8 * (P - 1) + 0.1e-6 * 4.0 * (P - 1) * g.keptRows * g.N;
         gs.nPeers = P - 1;
-        small = small_tile(gs, 1, flexBlocks ? 0.8 * kOtherShare * (flex_us(g, 1, flexBlocks) + comm) : dma ? 0.8 * kAlignedShare * (aligned_us(g, 1) + comm) : 1e30);
+        small = small_tile(gs, 1, flexBlocks ? 0.9 * kOtherShare * (flex_us(g, 1, flexBlocks) + comm) : dma ? 0.9 * kAlignedShare * (aligned_us(g, 1) + comm) : 1e30);
     }
     if (small.rows) fused = true;
     // (a single round may run in the order of the fused operators: 4096x8192x8192 of two ranks, as [n,k], two launches 405 -> 337)

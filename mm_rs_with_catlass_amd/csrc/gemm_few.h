@@ -13,7 +13,9 @@
 // small rather than sliced: 64x256 tiles in k slices used 64 to 128 CUs, and the second launch that added the slices and the peers cost
 // 3.5 to 6 us.  GPU time per call, k slices and second launch -> this: bf16 16x1024x8192, eight ranks, 12.9 -> 7.4 us, fp16
 // 512x1024x1024, two ranks, 14.2 -> 8.4, W8A8 203x1792x4096, eight ranks, all rows kept, 19.7 -> 13.8 (33 MB, 23 of them the
-// peers'), off the 64-byte and 128-column grid 2x13472x2432 57 -> 23, 46x15872x3360 144 -> 21.  Which launches: small_tile().
+// peers'), off the 64-byte and 128-column grid 2x13472x2432 57 -> 23, 46x15872x3360 144 -> 21; explicit kept rows with the others'
+// sums (BlockSum) 2x1408x640 9.6 -> 5.9, 128x2416x1280 24 -> 8.7, 283x14256x1024 77 -> 29, 462x2336x1536 24 -> 12.6.  Which launches:
+// small_tile().
 // k is divided among the waves because that takes neither barriers nor a shared ring; what it costs is LDS reads (a 64x64 tile reads
 // two fragments per two MFMAs, all the LDS can give), so long loops over many tiles belong to the larger tiles.
 #pragma once
@@ -32,6 +34,35 @@ __device__ __forceinline__ void dma16_base(const unsigned char *base, uint32_t o
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(ldsAddr) : "memory", "m0");
 }
 
+// Explicit kept rows: the other rows' sum of a 128x128 block, to which the tiles in it add theirs.  One 64-bit word per block in the
+// workspace's counter block: a tile adds its sum and 2^56 in one atomic, so the count of tiles that are through is in the top byte (a sum
+// has less than 2^46), and the tile that finds all others in it has the whole sum, stores it, and leaves the word at zero for the next
+// launch.  Nothing else goes from workgroup to workgroup, so nothing has to be waited for or fenced.  block_add() is one thread's call;
+// what it returns is for block_finish() at the end of the kernel, so that the atomic's trip is not waited for.
+struct BlockSum {
+    unsigned long long before, mine;
+    uint32_t tiles, block;   // tiles of the block; its number
+};
+
+template <int BM, int BN>
+__device__ __forceinline__ BlockSum block_add(const GemmArgs &args, uint32_t row0, uint32_t col0, uint32_t rows, long long sum)
+{
+    const uint32_t br = row0 / 128u, bc = col0 / 128u;
+    BlockSum s;
+    s.tiles = ceil_div(umin(128u, rows - br * 128u), (uint32_t)BM) * ceil_div(umin(128u, args.N - bc * 128u), (uint32_t)BN);
+    s.block = br * ceil_div(args.N, 128u) + bc;
+    s.mine = (unsigned long long)sum + (1ull << 56);
+    s.before = s.tiles == 1u ? 0ull : __hip_atomic_fetch_add((unsigned long long *)args.skCount + s.block, s.mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return s;
+}
+
+__device__ __forceinline__ void block_finish(const GemmArgs &args, const BlockSum &s)
+{
+    if ((uint32_t)((s.before + (1ull << 55)) >> 56) != s.tiles - 1u) return;
+    ((long long *)args.checksum)[s.block] = (long long)(s.before + s.mine - ((unsigned long long)s.tiles << 56));
+    if (s.tiles != 1u) __hip_atomic_store((unsigned long long *)args.skCount + s.block, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // MB, NB: 32-row and 32-column blocks of the tile.
 template <int MB, int NB> struct FewGeom
 {
@@ -41,7 +72,7 @@ template <int MB, int NB> struct FewGeom
     static constexpr int CP = ACP + BN / 8;         // copies per chunk
     static constexpr int WAVE_POOL = NS * STAGE;
     static constexpr int MEET = 4 * BM * BN * 4;
-    static constexpr int POOL = 4 * WAVE_POOL > MEET + BM * 4 ? 4 * WAVE_POOL : MEET + BM * 4;   // the rings, or the partial tiles and the row table
+    static constexpr int POOL = 4 * WAVE_POOL > MEET + BM * 4 + 32 ? 4 * WAVE_POOL : MEET + BM * 4 + 32;   // the rings, or the partial tiles, the row table and the waves' sums
     static constexpr int UN = BM * BN / 4 / 256;    // groups of four columns per thread
 };
 
@@ -338,6 +369,21 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
         if constexpr (I8) cur[j] += bv;
         d[j] = dst[row];
     }
+    BlockSum blockSum;
+    const bool sums = I8 && (flags & GF_ROW_MASK) && args.checksum;
+    if constexpr (I8) {
+        if (sums) {
+            long long sum = 0;
+#pragma unroll
+            for (int j = 0; j < UN; ++j)
+                if (colOk && d[j] != FX_KEPT && urow + j * (256 / LPR) < rowsValid) sum += ((long long)cur[j].x + cur[j].y) + ((long long)cur[j].z + cur[j].w);
+            sum = wave_sum64(sum);
+            long long *red = (long long *)(dst + BM);
+            if (lane == 63) red[w] = sum;
+            __syncthreads();
+            if (tid == 0) blockSum = block_add<BM, BN>(args, row0, col0, rows, (red[0] + red[1]) + (red[2] + red[3]));
+        }
+    }
     if (!colOk) return;
     if (args.accDump) {
 #pragma unroll
@@ -398,6 +444,9 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
         } else if ((d[j] & FX_KIND) == FX_OUT) {
             __builtin_nontemporal_store(cur[j], (v4i *)((float *)args.outbound + (size_t)(d[j] & FX_INDEX) * sp.n0 + (col0 % sp.n0) + lcol));
         }
+    }
+    if constexpr (I8) {
+        if (sums && tid == 0) block_finish(args, blockSum);
     }
 }
 

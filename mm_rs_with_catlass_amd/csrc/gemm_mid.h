@@ -354,8 +354,10 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
         if constexpr (I8) cur[j] += bv;
         d[j] = dst[row];
     }
+    BlockSum blockSum;
+    const bool sums = I8 && (flags & GF_ROW_MASK) && args.checksum;
     if constexpr (I8) {
-        if ((flags & GF_ROW_MASK) && args.checksum) {   // explicit kept rows: the others' sum per 128 x 128 block, which is the tile (of 64 rows: all rows there are)
+        if (sums) {   // explicit kept rows: the others' sum per 128x128 block
             long long sum = 0;
 #pragma unroll
             for (int j = 0; j < UN; ++j)
@@ -368,7 +370,7 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
                 long long all = 0;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) all += red[i];
-                ((long long *)args.checksum)[(size_t)(row0 / 128u) * ceil_div(N, 128u) + col0 / 128u] = all;
+                blockSum = block_add<BM, BN>(args, row0, col0, rowEnd, all);
             }
         }
     }
@@ -432,6 +434,9 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
         } else if ((d[j] & FX_KIND) == FX_OUT) {
             __builtin_nontemporal_store(cur[j], (v4i *)((float *)args.outbound + (size_t)(d[j] & FX_INDEX) * sp.n0 + (col0 % sp.n0) + lcol));
         }
+    }
+    if constexpr (I8) {
+        if (sums && tid == 0) block_finish(args, blockSum);
     }
 }
 

@@ -264,3 +264,37 @@ def test_quant_dealt_rows(case):
 @pytest.mark.parametrize("case", [("reduce_scatter", 936, 6148, 1666, 8, 3, True), ("reduce_scatter", 1684, 2304, 520, 4, 0, False), ("reduce_scatter", 2400, 548, 1280, 16, 15, True)])
 def test_float_dealt_rows(case):
     test_float_larger_tiles(case)
+
+
+# (rows, N, K, P, first kept row, kept rows, weights as [n,k]): sums of 128x128 blocks that several tiles add up: 32x32, 32x64, 64x64 and 64x128
+# tiles, blocks of one tile and of few at the edges, blocks whose rows are all kept, negative and positive sums
+@pytest.mark.parametrize("case", [(1, 132, 96, 2, 0, 1, True), (33, 300, 1416, 8, 5, 7, False), (128, 1280, 2416, 8, 0, 128, True), (130, 516, 416, 4, 1, 128, True), (300, 1408, 512, 8, 200, 40, True),
+                                  (80, 2784, 1060, 4, 60, 20, True), (462, 1536, 2336, 4, 0, 116, True), (409, 2688, 6232, 4, 300, 103, True)])
+def test_quant_kept_rows_block_sums(case):
+    _need_gpu()
+    M, N, K, P, kb, kr, tb = case
+    g = torch.Generator(device="cuda:0").manual_seed(M + N)
+    x1, x2 = (torch.randint(-127, 128, shape, dtype=torch.int8, device="cuda:0", generator=g) for shape in ((M, K), (K, N)))
+    x1[: M // 2] = x1[: M // 2].abs()   # (sums of either sign and size)
+    x2[:, N // 2:] = x2[:, N // 2:].abs()
+    s1, s2 = (torch.empty(c, device="cuda:0").uniform_(0.001, 0.02, generator=g) for c in (M, N))
+    peers = [torch.randn((kr, N), device="cuda:0", generator=g) for _ in range(P - 1)]
+    ws = torch.zeros(max(ops.splitk_plan(M, K, N, P, kb, kr)[0], 65536), dtype=torch.uint8, device="cuda:0")
+    acc = (x1.double() @ x2.double()).to(torch.int64)
+    others = acc.clone()
+    others[kb:kb + kr] = 0
+    want = torch.stack([others[r:r + 128, c:c + 128].sum() for r in range(0, M, 128) for c in range(0, N, 128)])
+    out = None
+    for w in (ws, ws, None):   # (the counter block is left at zero; without one the other kernels run)
+        if w is None and (K % 64 == 0 and N % 128 == 0):
+            continue
+        cs = torch.full((want.numel(),), -7, dtype=torch.int64, device="cuda:0")
+        got = ops.quant_matmul_splitk(x1, x2.T.contiguous() if tb else x2, s1, s2, None, peers, P, kb, kr, workspace=w, checksum=cs, trans_b=tb)
+        torch.cuda.synchronize()
+        assert torch.equal(cs, want) and not ws[:65536].any()
+        assert out is None or torch.equal(got, out)
+        out = got
+    y = (acc[kb:kb + kr].float() * s2) * s1[kb:kb + kr, None]
+    for p in peers:
+        y = y + p
+    assert torch.equal(out, y.bfloat16())
