@@ -101,6 +101,8 @@ struct Plan {
     uint32_t blockNum;
     bool dma;     // full tiles, row-major operands: the direct-to-LDS kernel applies
     bool preferFlex;         // run there although the aligned kernels would take it
+    uint32_t *counters;      // the workspace's counter block (NULL: none), and the bytes behind it that the launch may use
+    uint64_t room;
     bool maySmall;           // the caller left tiles, slices and order to the library: small tiles are a choice (small_tile)
     int flexBlocks;          // 0 = no; else the launch can run in flexible mode (gemm_flex.h) on tiles of 64 * flexBlocks rows
     uint32_t kSlices;        // k slices per tile this launch would run with a workspace (1 = none)
@@ -389,9 +391,12 @@ double streaming_us(const GemmArgs &a)
     return 9.8 + 1.58e-9 * c.rows * a.K * a.N + 0.147 * c.mb + 0.136 * c.moved + 0.117 * c.kib;
 }
 
+// Sliced small tiles: of a row tile that somebody keeps or stores, every slice leaves its partial tile in the workspace.
+uint64_t few_partials(const SmallTileCost &t, uint32_t keptTiles, uint32_t n, uint32_t slices) { return (uint64_t)keptTiles * ceil_div(n, (uint32_t)t.cols) * slices * t.rows * t.cols * 4u; }
+
 // The small tile a launch (operands, schedule, kept rows, flags and pointers filled in) runs, where the others would take `other` us;
-// fills args.fx for it.
-SmallTile small_tile(GemmArgs &a, uint32_t es, double other)
+// fills args.fx for it.  room: the bytes behind the workspace's counter block (a.skCount, if there is one) that the launch may use.
+SmallTile small_tile(GemmArgs &a, uint32_t es, double other, uint64_t room = 0)
 {
     const SmallTile no = {0, 0};
     const SchedParams &s = a.sched;
@@ -409,17 +414,30 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other)
     const SmallTileCost *best = nullptr;
     double least = 0.0;
     uint64_t tiles = 0;
+    uint32_t slices = 1;
+    // (rows nobody keeps leave their sums only)
+    const bool keptOnly = rowMask && a.accDump == nullptr;
+    auto kept_tile0 = [&](uint32_t step) { return keptOnly ? a.keptBegin / step : 0u; };
+    auto kept_tiles = [&](uint32_t step) { return keptOnly ? (a.keptBegin + a.keptRows - 1u) / step + 1u - kept_tile0(step) : (uint32_t)ceil_div((uint32_t)rows, step); };
     for (const SmallTileCost &t : kSmallTiles) {
-        if (sums && (t.cols != 128 || (t.rows < 128 && rows > (uint64_t)t.rows)) && (a.skCount == nullptr || (rows + 127) / 128 * ceil_div(a.N, 128u) > kCounterBlockBytes / 8u))
+        if (sums && (t.cols != 128 || (t.rows < 128 && rows > (uint64_t)t.rows)) && (a.skCount == nullptr || (rows + 127) / 128 * ceil_div(a.N, 128u) > kCounterBlockBytes / 16u))
             continue;
         const uint64_t n = (rows + t.rows - 1) / t.rows * ceil_div(a.N, t.cols);
-        const double rounds = (double)((n + 255) / 256), perCu = t.cols < 128 || n <= 256 ? rounds : n / 256.0, kib = rounds * c.kib * (t.rows + t.cols);
-        const double us = t.launch + t.workgroup * perCu + kib * (t.kib + (kBytes % 16 ? t.off16 : 0.0) + (a.transB ? 0.0 : t.kn) + (n > 256 ? t.later : 0.0)) + c.mb * t.mb +
-                          (!a.transB && t.cols * es < 128u ? c.mb * t.partLine : 0.0) + c.moved * t.moved;
-        if (best == nullptr || us < least) {
-            best = &t;
-            least = us;
-            tiles = n;
+        const double rounds = (double)((n + 255) / 256), perCu = t.cols < 128 || n <= 256 ? rounds : n / 256.0;
+        const double perKib = (t.rows + t.cols) * rounds * (t.kib + (kBytes % 16 ? t.off16 : 0.0) + (a.transB ? 0.0 : t.kn) + (n > 256 ? t.later : 0.0));
+        const double rest = t.launch + t.workgroup * perCu + c.mb * t.mb + (!a.transB && t.cols * es < 128u ? c.mb * t.partLine : 0.0) + c.moved * t.moved;
+        for (const uint32_t f : {1u, 2u, 3u, 4u, 6u, 8u}) {
+            // (at most a workgroup per CU, two chunks of k per wave; k of whole numbers short enough that a slice's sums and the whole are the same)
+            if (f > 1 && (t.cols >= 128 || n * f > 256 || kBytes < f * 1024u || (es == 1 && a.K > 131072u) || a.skCount == nullptr ||
+                          few_partials(t, kept_tiles(t.rows), a.N, f) > room))
+                break;
+            const double us = rest + perKib * c.kib / f + (f > 1 ? 2.2 + 1.5e-4 * f * t.rows * t.cols : 0.0);
+            if (best == nullptr || us < least) {
+                best = &t;
+                least = us;
+                tiles = n;
+                slices = f;
+            }
         }
     }
     if (best == nullptr) return no;
@@ -445,6 +463,10 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other)
     a.fx.rows = (uint32_t)rows;
     a.fx.rowTiles = (uint32_t)((rows + best->rows - 1) / best->rows);
     a.fx.colTiles = ceil_div(a.N, best->cols);
+    a.fx.slices = slices;
+    a.fx.keptTile0 = kept_tile0(best->rows);
+    a.fx.keptTiles = kept_tiles(best->rows);
+    if (slices > 1) a.skPart = (int32_t *)((unsigned char *)a.skCount + kCounterBlockBytes);
     if (best->cols == 128) deal_rows(a, es, (uint32_t)rows, best->rows);
     return {best->rows, best->cols};
 }
@@ -452,6 +474,19 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other)
 int launch_small(uint32_t dtype, const GemmArgs &a, const SmallTile &t, void *stream)
 {
     return t.cols == 256 ? launch_gemm_mixed(dtype, a, stream) : t.cols == 128 ? launch_gemm_mid(dtype, a, t.rows, stream) : launch_gemm_few(dtype, a, t.rows, t.cols, stream);
+}
+
+// The workspace's counter block, if the caller gave one.
+uint32_t *counter_block(const CatcocSymmetricDesc &d)
+{
+    return d.workspace != nullptr && (uintptr_t)d.workspace % 256 == 0 && d.workspaceBytes >= kCounterBlockBytes ? (uint32_t *)d.workspace : nullptr;
+}
+
+// The bytes behind it that a launch may use whose query says `query`.
+uint64_t counter_room(const CatcocSymmetricDesc &d, uint64_t query)
+{
+    const uint64_t bytes = d.workspaceBytes < query ? d.workspaceBytes : query;
+    return counter_block(d) != nullptr && bytes > kCounterBlockBytes ? bytes - kCounterBlockBytes : 0u;
 }
 
 // Everything a launcher checks before it launches; fills `plan` except the buffer pointers.
@@ -687,6 +722,8 @@ int make_plan(int commType, int dataType, const CocTilingParams *t, const Catcoc
         // (four slices or more of ragged rows or columns with B as [k,n]: a caller's count of them and the library's own give the same bits)
         if (plan.preferFlex && plan.edge && !transB && a.fx.slices >= 4) plan.maySmall = false;
     }
+    plan.counters = counter_block(*d);
+    plan.room = counter_room(*d, plan.kSliceBytes);
     // a workspace also lets the checksum halves of tiles that run as two workgroups meet (its counter block)
     if (a.skCount == nullptr && d->workspace != nullptr && (uintptr_t)d->workspace % 256 == 0 && d->workspaceBytes >= kCounterBlockBytes)
         a.skCount = (uint32_t *)d->workspace;
@@ -710,8 +747,9 @@ bool launched_small(const Plan &p, bool dma, bool flex, void *stream)
 {
     if (!p.maySmall) return false;
     GemmArgs g = p.args;
+    g.skCount = p.counters;
     const uint32_t es = elem_size(p.dtype);
-    const SmallTile t = small_tile(g, es, dma ? kAlignedShare * aligned_us(p.args, es) : flex ? kOtherShare * flex_us(p.args, es, p.flexBlocks) : 1e30);
+    const SmallTile t = small_tile(g, es, dma ? kAlignedShare * aligned_us(p.args, es) : flex ? kOtherShare * flex_us(p.args, es, p.flexBlocks) : 1e30, p.room);
     if (t.rows) launched(launch_small(p.dtype, g, t, stream));
     return t.rows != 0;
 }
@@ -925,12 +963,6 @@ bool decode_flex_pays(const GemmArgs &g, bool large)
     return !large && (g.K > 256 ? g.nPeers <= 1 || g.M >= 128 : g.nPeers == 0);
 }
 
-// The workspace's counter block, if the caller gave one.
-uint32_t *counter_block(const CatcocSymmetricDesc &d)
-{
-    return d.workspace != nullptr && (uintptr_t)d.workspace % 256 == 0 && d.workspaceBytes >= kCounterBlockBytes ? (uint32_t *)d.workspace : nullptr;
-}
-
 void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_x1, uint8_t *scale_x2, uint8_t *bias,
                          uint8_t *c_accum, uint8_t *d_out, const CatcocSymmetricDesc *d, CocTilingParams *tiling,
                          uint32_t transA, uint32_t transB, uint32_t outDataType)
@@ -1013,7 +1045,7 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
             if ((c.slices > 1 && g.fx.slices < 2 && (sp.large || sp.f > 1)) || !decode_flex_pays(g, sp.large) || !flex_ptrs_ok(g)) blocks = 0;
         }
         if (sp.maySmall) {
-            const SmallTile t = small_tile(small, 1, sp.wholeK ? 1e30 : kOtherShare * (blocks ? flex_us(g, 1, blocks) : streaming_us(g)));
+            const SmallTile t = small_tile(small, 1, sp.wholeK ? 1e30 : kOtherShare * (blocks ? flex_us(g, 1, blocks) : streaming_us(g)), counter_room(*d, sp.workspaceBytes));
             if (t.rows) {
                 launched(launch_small(DT_I8, small, t, stream));
                 return true;

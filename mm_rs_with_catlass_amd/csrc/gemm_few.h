@@ -1,4 +1,4 @@
-// Few small tiles, each over the whole k range, in ONE launch: the calls whose 64x256 tiles would leave most CUs idle (a decode batch
+// Few small tiles, each over the whole k range or in k slices, in ONE launch: the calls whose 64x256 tiles would leave most CUs idle (a decode batch
 // of a float model, a short prompt, a mixed batch of W8A8 rows).
 //
 // A tile is 32 or 64 rows by 32 or 64 columns, a workgroup of four waves per tile, and the waves divide k between them instead of
@@ -16,6 +16,12 @@
 // peers'), off the 64-byte and 128-column grid 2x13472x2432 57 -> 23, 46x15872x3360 144 -> 21; explicit kept rows with the others'
 // sums (BlockSum) 2x1408x640 9.6 -> 5.9, 128x2416x1280 24 -> 8.7, 283x14256x1024 77 -> 29, 462x2336x1536 24 -> 12.6.  Which launches:
 // small_tile().
+// Where even small tiles are fewer than half the CUs and k is long, a tile has up to eight workgroups, one k slice each (SL).  They meet in the
+// workspace: every slice leaves its partial tile there (4 to 16 KiB, past the caches that other XCDs do not see) and counts itself, and the last
+// to arrive adds all of them in slice order, then the peers, and writes the output.  That costs 2.2 us and the partials' trip through one CU,
+// against 5 for a second launch over 64x256 tiles' slices.  64x256 tiles and second launch -> this: bf16 7x11264x1024 of eight ranks 15.5 ->
+// 10.8 us, fp16 1x13256x1024 all-gather 18.2 -> 11.9, 44x6000x640 reduce-scatter of two 17.0 -> 10.0, W8A8 59x8960x512 14.5 -> 9.6,
+// 9x4864x512 with 3 rows kept, as [k,n], 11.5 -> 9.2, bf16 31x10784x2048 20.1 -> 16.6.
 // k is divided among the waves because that takes neither barriers nor a shared ring; what it costs is LDS reads (a 64x64 tile reads
 // two fragments per two MFMAs, all the LDS can give), so long loops over many tiles belong to the larger tiles.
 #pragma once
@@ -35,24 +41,25 @@ __device__ __forceinline__ void dma16_base(const unsigned char *base, uint32_t o
 }
 
 // Explicit kept rows: the other rows' sum of a 128x128 block, to which the tiles in it add theirs.  One 64-bit word per block in the
-// workspace's counter block: a tile adds its sum and 2^56 in one atomic, so the count of tiles that are through is in the top byte (a sum
-// has less than 2^46), and the tile that finds all others in it has the whole sum, stores it, and leaves the word at zero for the next
+// workspace's counter block, behind the sliced tiles' counters: a tile (a k slice of one) adds its sum and 2^56 in one atomic, so the count of
+// those that are through is in the top byte (a sum has less than 2^50), and the tile that finds all others in it has the whole sum, stores it, and leaves the word at zero for the next
 // launch.  Nothing else goes from workgroup to workgroup, so nothing has to be waited for or fenced.  block_add() is one thread's call;
 // what it returns is for block_finish() at the end of the kernel, so that the atomic's trip is not waited for.
 struct BlockSum {
     unsigned long long before, mine;
-    uint32_t tiles, block;   // tiles of the block; its number
+    uint32_t tiles, block;   // tiles of the block, times slices; its number
 };
+constexpr uint32_t FEW_TILE_COUNTERS = 8192;   // of 4 bytes; then as many bytes again for the blocks' words
 
 template <int BM, int BN>
-__device__ __forceinline__ BlockSum block_add(const GemmArgs &args, uint32_t row0, uint32_t col0, uint32_t rows, long long sum)
+__device__ __forceinline__ BlockSum block_add(const GemmArgs &args, uint32_t row0, uint32_t col0, uint32_t rows, uint32_t slices, long long sum)
 {
     const uint32_t br = row0 / 128u, bc = col0 / 128u;
     BlockSum s;
-    s.tiles = ceil_div(umin(128u, rows - br * 128u), (uint32_t)BM) * ceil_div(umin(128u, args.N - bc * 128u), (uint32_t)BN);
+    s.tiles = slices * ceil_div(umin(128u, rows - br * 128u), (uint32_t)BM) * ceil_div(umin(128u, args.N - bc * 128u), (uint32_t)BN);
     s.block = br * ceil_div(args.N, 128u) + bc;
     s.mine = (unsigned long long)sum + (1ull << 56);
-    s.before = s.tiles == 1u ? 0ull : __hip_atomic_fetch_add((unsigned long long *)args.skCount + s.block, s.mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s.before = s.tiles == 1u ? 0ull : __hip_atomic_fetch_add((unsigned long long *)(args.skCount + FEW_TILE_COUNTERS) + s.block, s.mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return s;
 }
 
@@ -60,7 +67,7 @@ __device__ __forceinline__ void block_finish(const GemmArgs &args, const BlockSu
 {
     if ((uint32_t)((s.before + (1ull << 55)) >> 56) != s.tiles - 1u) return;
     ((long long *)args.checksum)[s.block] = (long long)(s.before + s.mine - ((unsigned long long)s.tiles << 56));
-    if (s.tiles != 1u) __hip_atomic_store((unsigned long long *)args.skCount + s.block, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (s.tiles != 1u) __hip_atomic_store((unsigned long long *)(args.skCount + FEW_TILE_COUNTERS) + s.block, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // MB, NB: 32-row and 32-column blocks of the tile.
@@ -72,12 +79,12 @@ template <int MB, int NB> struct FewGeom
     static constexpr int CP = ACP + BN / 8;         // copies per chunk
     static constexpr int WAVE_POOL = NS * STAGE;
     static constexpr int MEET = 4 * BM * BN * 4;
-    static constexpr int POOL = 4 * WAVE_POOL > MEET + BM * 4 + 32 ? 4 * WAVE_POOL : MEET + BM * 4 + 32;   // the rings, or the partial tiles, the row table and the waves' sums
+    static constexpr int POOL = 4 * WAVE_POOL > MEET + BM * 4 + 48 ? 4 * WAVE_POOL : MEET + BM * 4 + 48;   // the rings, or the partial tiles, the row table, the waves' sums and a flag
     static constexpr int UN = BM * BN / 4 / 256;    // groups of four columns per thread
 };
 
-// GA: all-gather; the rows of A lie in the ranks' shards, one behind the other.
-template <uint32_t DT, bool TB, int MB, int NB, bool GA>
+// GA: all-gather; the rows of A lie in the ranks' shards, one behind the other.  SL: k slices, args.fx.slices workgroups per tile.
+template <uint32_t DT, bool TB, int MB, int NB, bool GA, bool SL>
 __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
 {
     using G = FewGeom<MB, NB>;
@@ -106,8 +113,10 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
     const int c32 = lane & 31, h = lane >> 5;
     const SchedParams &sp = args.sched;
     // XCD x takes the x-th eighth of the tiles, row tiles of a column strip behind each other: they share its columns of B
-    const uint32_t seq = xcd_eighth(blockIdx.x, rowTiles * colTiles);
-    const uint32_t ct = seq / rowTiles, rt = seq - ct * rowTiles;
+    // (and the slices of a tile are neighbours)
+    const uint32_t slices = SL ? args.fx.slices : 1u, seq = xcd_eighth(blockIdx.x, rowTiles * colTiles * slices);
+    const uint32_t tile = SL ? seq / slices : seq, slice = seq - tile * slices;
+    const uint32_t ct = tile / rowTiles, rt = tile - ct * rowTiles;
     const uint32_t row0 = rt * BM, col0 = ct * BN;
     const uint32_t rowsValid = umin((uint32_t)BM, rows - row0), colsValid = umin((uint32_t)BN, N - col0);
     const uint32_t ldaB = (uint32_t)args.lda * ES, ldbB = (uint32_t)args.ldb * ES;
@@ -128,9 +137,10 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
     const uint32_t kBytes = K * ES;
     const uint32_t nChunks = (kBytes + 127u) / 128u;
     const uint32_t lastBytes = kBytes - (nChunks - 1u) * 128u, lastWhole = lastBytes / 16u;   // bytes of k in the last chunk, whole pieces of it
-    const uint32_t mine = nChunks > w ? (nChunks - w + 3u) / 4u : 0u;     // chunks w, w + 4, ...
+    const uint32_t chunk0 = SL ? slice * nChunks / slices : 0u, chunks = (SL ? (slice + 1u) * nChunks / slices : nChunks) - chunk0;   // the slice's
+    const uint32_t cw = chunk0 + w, mine = chunks > w ? (chunks - w + 3u) / 4u : 0u;     // chunks cw, cw + 4, ...
     // every column strip starts its walk over k somewhere else (and wraps): the rows are often a power of two apart
-    uint32_t at = mine ? (ct * 40u + (blockIdx.x & 7u) * 5u) % mine : 0u;                           // the wave's next chunk is w + 4 * at
+    uint32_t at = mine ? (ct * 40u + (blockIdx.x & 7u) * 5u) % mine : 0u;                           // the wave's next chunk is cw + 4 * at
     const unsigned char *Ab = (const unsigned char *)a0 + (size_t)row0 * ldaB;
     const unsigned char *Bb = (const unsigned char *)b0 + (TB ? (size_t)col0 * ldbB : (size_t)col0 * ES);
     const size_t bChunk = TB ? (size_t)128 : (size_t)(128 / ES) * ldbB;
@@ -152,7 +162,7 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
     unsigned char *ring = smem + w * G::WAVE_POOL;
     const uint32_t ring0 = (uint32_t)(uintptr_t)(CATCOC_LDS unsigned char *)ring;
     auto issue = [&](uint32_t st) {   // this wave's next chunk into stage st
-        const uint32_t c = w + 4u * at, lds = ring0 + st * G::STAGE;
+        const uint32_t c = cw + 4u * at, lds = ring0 + st * G::STAGE;
         const unsigned char *a = Ab + (size_t)c * 128, *b = Bb + c * bChunk;
         if (c + 1u != nChunks || lastBytes == 128u) {
 #pragma unroll
@@ -218,7 +228,7 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
                 }
             }
         }
-        const uint32_t c = w + 4u * atRead;
+        const uint32_t c = cw + 4u * atRead;
         atRead = atRead + 1u == mine ? 0u : atRead + 1u;
         if (c + 1u == nChunks && lastBytes != 128u) {
 #pragma unroll
@@ -259,7 +269,7 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
     v4f sN = {1.f, 1.f, 1.f, 1.f};
     v4i bv = {0, 0, 0, 0};
     float sM[UN];
-    auto fetch_all = [&]() {
+    auto fetch_peers = [&]() {
         if (nPeers) {
 #pragma unroll
             for (int p = 0; p < PF; ++p) {
@@ -267,10 +277,13 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
                 else if ((uint32_t)p < nPeers) fetch(pv[p], peer[p], true);
             }
         }
+    };
+    auto fetch_all = [&]() {
+        if constexpr (!SL) fetch_peers();   // (else the last slice's)
         if constexpr (I8) {
             if (colOk) {
                 sN = *(const v4f *)(args.scaleN + gcol);
-                if (args.bias) bv = *(const v4i *)(args.bias + gcol);
+                if (args.bias && slice == 0u) bv = *(const v4i *)(args.bias + gcol);
             }
 #pragma unroll
             for (int j = 0; j < UN; ++j) sM[j] = args.scaleM[row0 + umin(urow + j * (256 / LPR), rowsValid - 1u)];
@@ -381,7 +394,58 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
             long long *red = (long long *)(dst + BM);
             if (lane == 63) red[w] = sum;
             __syncthreads();
-            if (tid == 0) blockSum = block_add<BM, BN>(args, row0, col0, rows, (red[0] + red[1]) + (red[2] + red[3]));
+            if (tid == 0) blockSum = block_add<BM, BN>(args, row0, col0, rows, slices, (red[0] + red[1]) + (red[2] + red[3]));
+        }
+    }
+    // ---- k slices: the last to arrive has the sum of all, in slice order
+    if constexpr (SL) {
+        const uint32_t keptTile = rt - args.fx.keptTile0;
+        bool last = false;
+        if (keptTile < args.fx.keptTiles) {   // (others: rows nobody keeps, whose sums are on their way)
+            constexpr int DEVICE_SCOPE = 16, WORDS = BM * BN;   // sc1
+            int32_t *const part = args.skPart + (size_t)(ct * args.fx.keptTiles + keptTile) * slices * WORDS;
+            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)part, 0, (int)(slices * WORDS * 4u), 0x00020000);
+#pragma unroll
+            for (int j = 0; j < UN; ++j) __builtin_amdgcn_raw_buffer_store_b128(cur[j], rs, (slice * WORDS + (j * 256 + tid) * 4) * 4, 0, DEVICE_SCOPE);
+            CATCOC_WAIT_VMCNT(0);   // once the stores are acknowledged the slice may be counted
+            __syncthreads();
+            volatile uint32_t *flag = (volatile uint32_t *)(dst + BM + 8);
+            uint32_t *const count = args.skCount + ct * args.fx.keptTiles + keptTile;
+            if (tid == 0) *flag = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            last = *flag == slices - 1u;
+            if (last) {
+                if (tid == 0) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                constexpr int AT_ONCE = UN == 4 ? 2 : 4;
+                for (uint32_t o = 0; o < slices; o += AT_ONCE) {   // (past the last one: zeros for whole numbers; floats add none)
+                    v4i t[AT_ONCE][UN];
+#pragma unroll
+                    for (int q = 0; q < AT_ONCE; ++q)
+#pragma unroll
+                        for (int j = 0; j < UN; ++j) t[q][j] = __builtin_amdgcn_raw_buffer_load_b128(rs, ((o + q) * WORDS + (j * 256 + tid) * 4) * 4, 0, DEVICE_SCOPE);
+                    if (o == 0) fetch_peers();
+#pragma unroll
+                    for (int q = 0; q < AT_ONCE; ++q)
+#pragma unroll
+                        for (int j = 0; j < UN; ++j) {
+                            if constexpr (I8) {
+                                cur[j] = o + q == 0 ? t[q][j] : cur[j] + t[q][j];
+                            } else {
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) {
+                                    const int v = f2i(__fadd_rn(i2f(cur[j][e]), i2f(t[q][j][e])));
+                                    cur[j][e] = o + q == 0 ? t[q][j][e] : o + q < slices ? v : cur[j][e];
+                                }
+                            }
+                        }
+                }
+            }
+        }
+        if (!last) {
+            if constexpr (I8) {
+                if (sums && tid == 0) block_finish(args, blockSum);
+            }
+            return;
         }
     }
     if (!colOk) return;
@@ -450,15 +514,21 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
     }
 }
 
+template <uint32_t DT, bool TB, bool GA, bool SL>
+inline int launch_few_sl(const GemmArgs &args, int tileRows, int tileCols, hipStream_t s)
+{
+    const dim3 grid(args.fx.rowTiles * args.fx.colTiles * args.fx.slices), block(256);
+    if (tileRows == 32 && tileCols == 32) hipLaunchKernelGGL((gemm_few_kernel<DT, TB, 1, 1, GA, SL>), grid, block, 0, s, args);
+    else if (tileRows == 32 && tileCols == 64) hipLaunchKernelGGL((gemm_few_kernel<DT, TB, 1, 2, GA, SL>), grid, block, 0, s, args);
+    else if (tileRows == 64 && tileCols == 64) hipLaunchKernelGGL((gemm_few_kernel<DT, TB, 2, 2, GA, SL>), grid, block, 0, s, args);
+    else return (int)hipErrorInvalidValue;
+    return (int)hipGetLastError();
+}
+
 template <uint32_t DT, bool TB, bool GA>
 inline int launch_few_tb(const GemmArgs &args, int tileRows, int tileCols, hipStream_t s)
 {
-    const dim3 grid(args.fx.rowTiles * args.fx.colTiles), block(256);
-    if (tileRows == 32 && tileCols == 32) hipLaunchKernelGGL((gemm_few_kernel<DT, TB, 1, 1, GA>), grid, block, 0, s, args);
-    else if (tileRows == 32 && tileCols == 64) hipLaunchKernelGGL((gemm_few_kernel<DT, TB, 1, 2, GA>), grid, block, 0, s, args);
-    else if (tileRows == 64 && tileCols == 64) hipLaunchKernelGGL((gemm_few_kernel<DT, TB, 2, 2, GA>), grid, block, 0, s, args);
-    else return (int)hipErrorInvalidValue;
-    return (int)hipGetLastError();
+    return args.fx.slices > 1 ? launch_few_sl<DT, TB, GA, true>(args, tileRows, tileCols, s) : launch_few_sl<DT, TB, GA, false>(args, tileRows, tileCols, s);
 }
 
 template <uint32_t DT>

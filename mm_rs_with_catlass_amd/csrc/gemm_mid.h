@@ -370,7 +370,7 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
                 long long all = 0;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) all += red[i];
-                blockSum = block_add<BM, BN>(args, row0, col0, rowEnd, all);
+                blockSum = block_add<BM, BN>(args, row0, col0, rowEnd, 1u, all);
             }
         }
     }

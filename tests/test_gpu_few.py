@@ -298,3 +298,94 @@ def test_quant_kept_rows_block_sums(case):
     for p in peers:
         y = y + p
     assert torch.equal(out, y.bfloat16())
+
+
+def sliced_workspace(need):
+    """A workspace of more than the query asks for: counters at zero, marks behind what a launch may touch."""
+    ws = torch.zeros(need + 4096, dtype=torch.uint8, device="cuda:0")
+    ws[need:] = 0x5a
+    return ws
+
+
+def check_workspace(ws, need):
+    assert not ws[:65536].any() and (ws[need:] == 0x5a).all() and ws[65536:need].any()   # (the last: slices ran)
+
+
+# (operator, rows (of a shard), N, K, P, rank, weights as [n,k]): small tiles in k slices; k of odd chunks, rows and columns past a tile, more peers than
+# registers hold at once, slices of unequal length
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", [("allreduce", 33, 896, 6656, 4, 0, False), ("allreduce", 7, 1024, 11262, 8, 0, True), ("allreduce", 20, 516, 8190, 16, 0, True), ("allgather", 2, 1536, 8448, 4, 3, True),
+                                  ("allgather", 13, 1024, 14500, 8, 0, True), ("reduce_scatter", 44, 640, 6000, 2, 1, True), ("reduce_scatter", 112, 512, 6144, 4, 2, False)])
+def test_float_k_slices(case, dtype):
+    _need_gpu()
+    op, m, N, K, P, rank, tb = case
+    g = torch.Generator(device="cuda:0").manual_seed(m)
+    rand = lambda *shape: torch.randn(shape, device="cuda:0", generator=g)
+    M = m * P if op == "allgather" else m
+    A, B = rand(M, K).to(dtype), (rand(K, N) * 0.05).to(dtype)
+    Bd = B.T.contiguous() if tb else B
+    rows = {"allreduce": m, "allgather": 0, "reduce_scatter": m // P}[op]
+    peers = [rand(rows, N) for _ in range(P - 1)] if rows else []
+    comm = {"allreduce": L.MATMUL_ALLREDUCE, "allgather": L.ALLGATHER_MATMUL, "reduce_scatter": L.MATMUL_REDUCE_SCATTER}[op]
+    need = ops.kslice_plan(comm, dtype, m, K, N, rank, P)[0]
+    ws, first = sliced_workspace(need), None
+    for _ in range(3):
+        dump = torch.full((M, N), 7.0, device="cuda:0")
+        if op == "allgather":
+            shards = [s.contiguous() for s in A.split(m)]
+            out = ops.allgather_matmul(shards[rank], shards[:rank] + shards[rank + 1:], Bd, rank, P, trans_b=tb, acc_dump=dump, workspace=ws)
+            got = dump
+        elif op == "allreduce":
+            out = ops.matmul_allreduce(A, Bd, peers, 0, P, trans_b=tb, acc_dump=dump, workspace=ws)
+            got = dump
+        else:
+            t, d = one_round(comm, M, K, N, P, rank)
+            ob = torch.full((L.load().catcoc_get_workspace_size(comm, L.FP16, C.byref(t), C.byref(d)) // 4,), 3.0, device="cuda:0")
+            out = ops.matmul_reduce_scatter(A, Bd, peers, rank, P, tiling=t, trans_b=tb, outbound=ob, acc_dump=dump, workspace=ws)
+            tiles, full = ob.cpu().numpy().reshape(-1, 256), dump.cpu().numpy()
+            for task, r, row, col, place in tasks_of(comm, t, d):
+                if r != rank:
+                    r1, c1 = min(row + 64, (r + 1) * rows), min(col + 256, N)
+                    assert np.array_equal(tiles[place:place + r1 - row, :c1 - col], full[row:r1, col:c1]), task
+            got = dump[rank * rows:(rank + 1) * rows]
+        torch.cuda.synchronize()
+        check_workspace(ws, need)
+        assert first is None or torch.equal(first, dump)   # (slice order, whichever arrives last)
+        first = dump
+    bound = 8 * K ** 0.5 * 2.0 ** -24 * torch.outer(A.double().norm(dim=1), B.double().norm(dim=0)) + 1e-9   # (as sum_bound)
+    assert ((dump.double() - A.double() @ B.double()).abs() <= bound).all()
+    for p in peers:
+        got = got + p
+    assert torch.equal(out, got.to(dtype))
+
+
+# (rows, N, K, P, first kept row, kept rows, weights as [n,k], int32 peers, dump): as above; of rows that are not kept only the sums, or all of them
+@pytest.mark.parametrize("case", [(51, 1920, 12800, 4, 30, 13, True, False, False), (51, 1920, 12800, 4, 30, 13, True, False, True), (67, 640, 4992, 8, 0, 67, False, True, False),
+                                  (134, 768, 4736, 8, 60, 17, False, False, False), (2, 512, 7680, 4, 1, 1, True, True, False), (24, 2560, 14848, 8, 21, 3, False, False, False)])
+def test_quant_k_slices(case):
+    _need_gpu()
+    M, N, K, P, kb, kr, tb, ri, with_dump = case
+    g = torch.Generator(device="cuda:0").manual_seed(M + N)
+    x1, x2 = (torch.randint(-127, 128, shape, dtype=torch.int8, device="cuda:0", generator=g) for shape in ((M, K), (K, N)))
+    s1, s2 = (torch.empty(c, device="cuda:0").uniform_(0.001, 0.02, generator=g) for c in (M, N))
+    b = torch.randint(-1000, 1000, (N,), dtype=torch.int32, device="cuda:0", generator=g)
+    peers = [torch.randint(-2 ** 20, 2 ** 20, (kr, N), dtype=torch.int32, device="cuda:0", generator=g) if ri else torch.randn((kr, N), device="cuda:0", generator=g)
+             for _ in range(P - 1)]
+    acc = (x1.double() @ x2.double()).to(torch.int64) + b
+    others = acc.clone()
+    others[kb:kb + kr] = 0
+    sums = torch.stack([others[r:r + 128, c:c + 128].sum() for r in range(0, M, 128) for c in range(0, N, 128)])
+    y = acc[kb:kb + kr].to(torch.int32) + (sum(peers) if ri else 0)
+    y = (y.float() * s2) * s1[kb:kb + kr, None]
+    for p in ([] if ri else peers):
+        y = y + p
+    need = ops.splitk_plan(M, K, N, P, kb, kr)[0]
+    ws = sliced_workspace(need)
+    for _ in range(3):
+        cs = torch.full((sums.numel(),), -7, dtype=torch.int64, device="cuda:0")
+        dump = torch.full((M, N), -7, dtype=torch.int32, device="cuda:0") if with_dump else None
+        out = ops.quant_matmul_splitk(x1, x2.T.contiguous() if tb else x2, s1, s2, b, peers, P, kb, kr, workspace=ws, checksum=cs, acc_dump=dump, trans_b=tb, reduce_int32=ri)
+        torch.cuda.synchronize()
+        check_workspace(ws, need)
+        assert torch.equal(cs, sums) and torch.equal(out, y.bfloat16())
+        assert dump is None or torch.equal(dump, acc.to(torch.int32))
