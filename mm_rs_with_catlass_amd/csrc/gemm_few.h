@@ -14,7 +14,7 @@
 // 3.5 to 6 us.  GPU time per call, k slices and second launch -> this: bf16 16x1024x8192, eight ranks, 12.9 -> 7.4 us, fp16
 // 512x1024x1024, two ranks, 14.2 -> 8.4, W8A8 203x1792x4096, eight ranks, all rows kept, 19.7 -> 13.8 (33 MB, 23 of them the
 // peers'), off the 64-byte and 128-column grid 2x13472x2432 57 -> 23, 46x15872x3360 144 -> 21; explicit kept rows with the others'
-// sums (BlockSum) 2x1408x640 9.6 -> 5.9, 128x2416x1280 24 -> 8.7, 283x14256x1024 77 -> 29, 462x2336x1536 24 -> 12.6.  Which launches:
+// sums (MetSum) 2x1408x640 9.6 -> 5.9, 128x2416x1280 24 -> 8.7, 283x14256x1024 77 -> 29, 462x2336x1536 24 -> 12.6.  Which launches:
 // small_tile().
 // Where even small tiles are fewer than half the CUs and k is long, a tile has up to eight workgroups, one k slice each (SL).  They meet in the
 // workspace: every slice leaves its partial tile there (4 to 16 KiB, past the caches that other XCDs do not see) and counts itself, and the last
@@ -40,34 +40,81 @@ __device__ __forceinline__ void dma16_base(const unsigned char *base, uint32_t o
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(ldsAddr) : "memory", "m0");
 }
 
-// Explicit kept rows: the other rows' sum of a 128x128 block, to which the tiles in it add theirs.  One 64-bit word per block in the
-// workspace's counter block, behind the sliced tiles' counters: a tile (a k slice of one) adds its sum and 2^56 in one atomic, so the count of
-// those that are through is in the top byte (a sum has less than 2^50), and the tile that finds all others in it has the whole sum, stores it, and leaves the word at zero for the next
-// launch.  Nothing else goes from workgroup to workgroup, so nothing has to be waited for or fenced.  block_add() is one thread's call;
-// what it returns is for block_finish() at the end of the kernel, so that the atomic's trip is not waited for.
-struct BlockSum {
+// Sums of whole numbers that several tiles add up: of the rows of a 128x128 block that are not kept (explicit kept rows), of a task of a
+// reduce-scatter.  One 64-bit word per sum in the workspace's counter block, behind the sliced tiles' counters: a tile (a k slice of one) adds
+// its part and 2^56 in one atomic, so the count of those that are through is in the top byte (a sum has less than 2^50), and the one that
+// finds all others in it has the whole sum, stores it, and leaves the word at zero for the next launch.  Nothing else goes from workgroup
+// to workgroup, so nothing has to be waited for or fenced.  Both are one thread's calls; what sum_add() returns is for sum_finish() as
+// late as there is something else to do, so that the atomic's trip is not waited for.
+struct MetSum {
     unsigned long long before, mine;
-    uint32_t tiles, block;   // tiles of the block, times slices; its number
+    uint32_t parts, word;   // tiles times slices that add to it; its number
 };
-constexpr uint32_t FEW_TILE_COUNTERS = 8192;   // of 4 bytes; then as many bytes again for the blocks' words
+constexpr uint32_t FEW_TILE_COUNTERS = 8192;   // of 4 bytes; then as many bytes again for the sums' words
 
-template <int BM, int BN>
-__device__ __forceinline__ BlockSum block_add(const GemmArgs &args, uint32_t row0, uint32_t col0, uint32_t rows, uint32_t slices, long long sum)
+__device__ __forceinline__ MetSum sum_add(const GemmArgs &args, uint32_t word, uint32_t parts, long long sum)
 {
-    const uint32_t br = row0 / 128u, bc = col0 / 128u;
-    BlockSum s;
-    s.tiles = slices * ceil_div(umin(128u, rows - br * 128u), (uint32_t)BM) * ceil_div(umin(128u, args.N - bc * 128u), (uint32_t)BN);
-    s.block = br * ceil_div(args.N, 128u) + bc;
+    MetSum s;
+    s.parts = parts;
+    s.word = word;
     s.mine = (unsigned long long)sum + (1ull << 56);
-    s.before = s.tiles == 1u ? 0ull : __hip_atomic_fetch_add((unsigned long long *)(args.skCount + FEW_TILE_COUNTERS) + s.block, s.mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s.before = parts == 1u ? 0ull : __hip_atomic_fetch_add((unsigned long long *)(args.skCount + FEW_TILE_COUNTERS) + word, s.mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return s;
 }
 
-__device__ __forceinline__ void block_finish(const GemmArgs &args, const BlockSum &s)
+__device__ __forceinline__ void sum_finish(const GemmArgs &args, const MetSum &s)
 {
-    if ((uint32_t)((s.before + (1ull << 55)) >> 56) != s.tiles - 1u) return;
-    ((long long *)args.checksum)[s.block] = (long long)(s.before + s.mine - ((unsigned long long)s.tiles << 56));
-    if (s.tiles != 1u) __hip_atomic_store((unsigned long long *)(args.skCount + FEW_TILE_COUNTERS) + s.block, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if ((uint32_t)((s.before + (1ull << 55)) >> 56) != s.parts - 1u) return;
+    ((long long *)args.checksum)[s.word] = (long long)(s.before + s.mine - ((unsigned long long)s.parts << 56));
+    if (s.parts != 1u) __hip_atomic_store((unsigned long long *)(args.skCount + FEW_TILE_COUNTERS) + s.word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The block a tile lies in.
+template <int BM, int BN>
+__device__ __forceinline__ MetSum block_add(const GemmArgs &args, uint32_t row0, uint32_t col0, uint32_t rows, uint32_t slices, long long sum)
+{
+    const uint32_t br = row0 / 128u, bc = col0 / 128u;
+    return sum_add(args, br * ceil_div(args.N, 128u) + bc,
+                   slices * ceil_div(umin(128u, rows - br * 128u), (uint32_t)BM) * ceil_div(umin(128u, args.N - bc * 128u), (uint32_t)BN), sum);
+}
+
+// The tasks that a tile has rows of (dst: FX_SUM and the task; the rows of a task are neighbours).  A row's sum goes to LDS, and the thread of a
+// task's first row adds up its rows and adds that to the task's word.  cur: groups of four columns, as both kernels finish them; rowOf(i): row i
+// of the tile; tiles(begin, end): row tiles that have some of the rows from begin up to end.
+template <int BN, int NT, int UN, typename RowOf, typename Tiles>
+__device__ __forceinline__ void task_sums(const GemmArgs &args, long long *rowSum, const uint32_t *dst, const v4i (&cur)[UN], uint32_t tid, bool colOk, uint32_t col0, uint32_t rowsValid,
+                                          uint32_t slices, RowOf rowOf, Tiles tiles)
+{
+    constexpr uint32_t LPR = BN / 4;
+#pragma unroll
+    for (int j = 0; j < UN; ++j) {
+        long long v = colOk ? ((long long)cur[j].x + cur[j].y) + ((long long)cur[j].z + cur[j].w) : 0;
+        v = dpp_add64<0x111, 0xf>(v);   // row_shr:1, 2, 4: eight lanes' sum in the last of them, 8: sixteen lanes', row_bcast:15: 32 lanes'
+        v = dpp_add64<0x112, 0xf>(v);
+        v = dpp_add64<0x114, 0xf>(v);
+        if constexpr (LPR >= 16) v = dpp_add64<0x118, 0xf>(v);
+        if constexpr (LPR >= 32) v = dpp_add64<0x142, 0xa>(v);
+        if (tid % LPR == LPR - 1u) rowSum[tid / LPR + j * (NT / LPR)] = v;
+    }
+    __syncthreads();
+    if (tid >= rowsValid) return;
+    const uint32_t e = dst[tid];
+    if ((e & FX_KIND) != FX_SUM || (tid != 0u && dst[tid - 1u] == e)) return;
+    const SchedParams &sp = args.sched;
+    uint32_t ri;
+    const uint32_t v = rowOf(tid), r = fast_div(v, args.fx.dRank, ri), mi = ri / sp.m0;
+    const uint32_t begin = r * sp.mRank + mi * sp.m0, end = begin + umin(sp.m0, sp.mRank - mi * sp.m0);   // the task's rows
+    const uint32_t upTo = umin(end - v + tid, rowsValid);
+    long long sum[4] = {0, 0, 0, 0};
+    uint32_t i = tid;
+    for (; i + 4u <= upTo; i += 4u) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sum[q] += rowSum[i + q];
+    }
+    for (; i < upTo; ++i) sum[0] += rowSum[i];
+    const uint32_t colBegin = col0 / sp.n0 * sp.n0;
+    sum_finish(args, sum_add(args, e & FX_INDEX, slices * tiles(begin, end) * ceil_div(umin(sp.n0, args.N - colBegin), (uint32_t)BN),
+                             (sum[0] + sum[1]) + (sum[2] + sum[3])));
 }
 
 // MB, NB: 32-row and 32-column blocks of the tile.
@@ -79,7 +126,7 @@ template <int MB, int NB> struct FewGeom
     static constexpr int CP = ACP + BN / 8;         // copies per chunk
     static constexpr int WAVE_POOL = NS * STAGE;
     static constexpr int MEET = 4 * BM * BN * 4;
-    static constexpr int POOL = 4 * WAVE_POOL > MEET + BM * 4 + 48 ? 4 * WAVE_POOL : MEET + BM * 4 + 48;   // the rings, or the partial tiles, the row table, the waves' sums and a flag
+    static constexpr int POOL = 4 * WAVE_POOL > MEET + BM * 12 + 48 ? 4 * WAVE_POOL : MEET + BM * 12 + 48;   // the rings, or the partial tiles, the row table, the waves' sums, a flag and the rows' sums
     static constexpr int UN = BM * BN / 4 / 256;    // groups of four columns per thread
 };
 
@@ -344,7 +391,7 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
                 const auto e = acc[mb][nb][r];
                 *(int *)(smem + ((w * BM + row) * BN + ((nb * 32 + c32) ^ ((uint32_t)h * SWZ << 5))) * 4) = __builtin_bit_cast(int, e);
             }
-    const bool store = (flags & GF_OUTBOUND_STORE) != 0;
+    const bool store = (flags & GF_OUTBOUND_STORE) != 0, taskSums = I8 && !store && (flags & GF_ROW_MASK) == 0 && args.checksum != nullptr;
     if (tid < BM) {
         const uint32_t v = row0 + tid;
         uint32_t e = FX_SKIP;
@@ -356,6 +403,11 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
                 const uint32_t r = fast_div(v, args.fx.dRank, ri);
                 flex_task_of(sp, r, ri, col0 / sp.n0, task, ws);
                 e = FX_OUT | ws;
+            } else if (I8 && taskSums) {
+                uint32_t ri, task, ws;
+                const uint32_t r = fast_div(v, args.fx.dRank, ri);
+                flex_task_of(sp, r, ri, col0 / sp.n0, task, ws);
+                e = FX_SUM | task;
             }
         }
         dst[tid] = e;
@@ -382,7 +434,7 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
         if constexpr (I8) cur[j] += bv;
         d[j] = dst[row];
     }
-    BlockSum blockSum;
+    MetSum blockSum;
     const bool sums = I8 && (flags & GF_ROW_MASK) && args.checksum;
     if constexpr (I8) {
         if (sums) {
@@ -396,6 +448,9 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
             __syncthreads();
             if (tid == 0) blockSum = block_add<BM, BN>(args, row0, col0, rows, slices, (red[0] + red[1]) + (red[2] + red[3]));
         }
+        if (taskSums)
+            task_sums<BN, 256, UN>(args, (long long *)(dst + BM + 12), dst, cur, tid, colOk, col0, rowsValid, slices, [&](uint32_t i) { return row0 + i; },
+                                   [](uint32_t begin, uint32_t end) { return (end - 1u) / BM - begin / BM + 1u; });
     }
     // ---- k slices: the last to arrive has the sum of all, in slice order
     if constexpr (SL) {
@@ -405,8 +460,11 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
             constexpr int DEVICE_SCOPE = 16, WORDS = BM * BN;   // sc1
             int32_t *const part = args.skPart + (size_t)(ct * args.fx.keptTiles + keptTile) * slices * WORDS;
             const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)part, 0, (int)(slices * WORDS * 4u), 0x00020000);
+            uint32_t at[UN];   // of the rows that count; the others' lie behind the end
 #pragma unroll
-            for (int j = 0; j < UN; ++j) __builtin_amdgcn_raw_buffer_store_b128(cur[j], rs, (slice * WORDS + (j * 256 + tid) * 4) * 4, 0, DEVICE_SCOPE);
+            for (int j = 0; j < UN; ++j) at[j] = !args.fx.keptOnly || d[j] == FX_KEPT ? (j * 256u + (uint32_t)tid) * 16u : 0x7ffffff0u;
+#pragma unroll
+            for (int j = 0; j < UN; ++j) __builtin_amdgcn_raw_buffer_store_b128(cur[j], rs, at[j], slice * (WORDS * 4), DEVICE_SCOPE);
             CATCOC_WAIT_VMCNT(0);   // once the stores are acknowledged the slice may be counted
             __syncthreads();
             volatile uint32_t *flag = (volatile uint32_t *)(dst + BM + 8);
@@ -422,7 +480,7 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
 #pragma unroll
                     for (int q = 0; q < AT_ONCE; ++q)
 #pragma unroll
-                        for (int j = 0; j < UN; ++j) t[q][j] = __builtin_amdgcn_raw_buffer_load_b128(rs, ((o + q) * WORDS + (j * 256 + tid) * 4) * 4, 0, DEVICE_SCOPE);
+                        for (int j = 0; j < UN; ++j) t[q][j] = __builtin_amdgcn_raw_buffer_load_b128(rs, at[j], (o + q) * (WORDS * 4u), DEVICE_SCOPE);
                     if (o == 0) fetch_peers();
 #pragma unroll
                     for (int q = 0; q < AT_ONCE; ++q)
@@ -443,7 +501,7 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
         }
         if (!last) {
             if constexpr (I8) {
-                if (sums && tid == 0) block_finish(args, blockSum);
+                if (sums && tid == 0) sum_finish(args, blockSum);
             }
             return;
         }
@@ -510,7 +568,7 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
         }
     }
     if constexpr (I8) {
-        if (sums && tid == 0) block_finish(args, blockSum);
+        if (sums && tid == 0) sum_finish(args, blockSum);
     }
 }
 

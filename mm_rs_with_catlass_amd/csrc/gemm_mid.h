@@ -35,7 +35,7 @@ template <int MB> struct MidGeom
     static constexpr int NS = 160 * 1024 / STAGE;   // 5 (128 rows) or 6 stages
     static constexpr int ACP = BM / 64, BCP = 2, CP = ACP + BCP;   // 1 KiB copies per chunk and wave
     static constexpr int MEET = 2 * BM * BN * 4;
-    static constexpr int POOL = NS * STAGE > MEET + BM * 8 + 64 ? NS * STAGE : MEET + BM * 8 + 64;   // the ring, or the partial tiles, the row table and the waves' sums
+    static constexpr int POOL = NS * STAGE > MEET + BM * 16 + 64 ? NS * STAGE : MEET + BM * 16 + 64;   // the ring, or the partial tiles, the row table, the waves' and the rows' sums
     static constexpr int UN = BM * BN / 4 / NT;     // groups of four columns per thread: 8 or 4
 };
 
@@ -316,7 +316,7 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
                 const auto e = acc[mb][nb][r];
                 *(int *)(smem + ((wg * BM + row) * BN + (((wn * 2 + nb) * 32 + (t2 & 31)) ^ ((uint32_t)((t2 >> 5) & 1) * SWZ << 5))) * 4) = __builtin_bit_cast(int, e);
             }
-    const bool store = (flags & GF_OUTBOUND_STORE) != 0;
+    const bool store = (flags & GF_OUTBOUND_STORE) != 0, taskSums = I8 && !store && (flags & GF_ROW_MASK) == 0 && args.checksum != nullptr;
     if (tid < BM) {
         const uint32_t v = rowOf(tid);
         uint32_t e = FX_SKIP;
@@ -328,6 +328,11 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
                 const uint32_t r = fast_div(v, args.fx.dRank, ri);
                 flex_task_of(sp, r, ri, col0 / sp.n0, task, ws);
                 e = FX_OUT | ws;
+            } else if (I8 && taskSums) {
+                uint32_t ri, task, ws;
+                const uint32_t r = fast_div(v, args.fx.dRank, ri);
+                flex_task_of(sp, r, ri, col0 / sp.n0, task, ws);
+                e = FX_SUM | task;
             }
         }
         dst[tid] = e;
@@ -354,7 +359,7 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
         if constexpr (I8) cur[j] += bv;
         d[j] = dst[row];
     }
-    BlockSum blockSum;
+    MetSum blockSum;
     const bool sums = I8 && (flags & GF_ROW_MASK) && args.checksum;
     if constexpr (I8) {
         if (sums) {   // explicit kept rows: the others' sum per 128x128 block
@@ -372,6 +377,20 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
                 for (int i = 0; i < 8; ++i) all += red[i];
                 blockSum = block_add<BM, BN>(args, row0, col0, rowEnd, 1u, all);
             }
+        }
+        if (taskSums) {
+            // (dealt rows: the tile of row x of those that are not kept, from a first guess)
+            auto first_other = [&](uint32_t t) { return deal_begin(t, f.dealRows, f.dealRest) - deal_begin(t, f.dealKept, f.dealKeptRest); };
+            auto tile_of = [&](uint32_t v) -> uint32_t {
+                if (!dealt) return v / BM;
+                const uint32_t x = v >= keptEnd ? v - keptRows : v;
+                uint32_t t = umin((uint32_t)((float)x * (float)rowTiles / (float)(rowEnd - keptRows)), rowTiles - 1u);
+                while (first_other(t) > x) --t;
+                while (first_other(t + 1u) <= x) ++t;
+                return t;
+            };
+            task_sums<BN, NT, UN>(args, (long long *)(rowScale + BM + 16), dst, cur, (uint32_t)t2, colOk, col0, rowsValid, 1u, rowOf,
+                                  [&](uint32_t begin, uint32_t end) { return tile_of(end - 1u) - tile_of(begin) + 1u; });
         }
     }
     if (!colOk) return;
@@ -436,7 +455,7 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
         }
     }
     if constexpr (I8) {
-        if (sums && tid == 0) block_finish(args, blockSum);
+        if (sums && tid == 0) sum_finish(args, blockSum);
     }
 }
 

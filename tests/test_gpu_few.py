@@ -389,3 +389,40 @@ def test_quant_k_slices(case):
         check_workspace(ws, need)
         assert torch.equal(cs, sums) and torch.equal(out, y.bfloat16())
         assert dump is None or torch.equal(dump, acc.to(torch.int32))
+
+
+# (rows per rank, N, K, P, rank, weights as [n,k], int32 peers): sums of tasks that several tiles add up: ranks of a few rows (many tasks to a tile), of a
+# tile and a bit, of several task rows; columns that end in a task's first and second half; a long k (slices), 128-column tiles
+@pytest.mark.parametrize("case", [(1, 256, 100, 8, 3, True, False), (2, 1000, 516, 16, 9, True, True), (5, 388, 1040, 8, 0, True, False), (33, 640, 416, 4, 3, False, True), (130, 900, 772, 2, 1, True, False),
+                                  (8, 768, 15776, 2, 0, False, False), (69, 1024, 1024, 8, 5, True, False), (166, 768, 512, 8, 2, True, False), (219, 640, 9984, 8, 7, True, True), (300, 1800, 644, 4, 1, True, False)])
+def test_quant_task_sums(case):
+    _need_gpu()
+    rows, N, K, P, rank, tb, ri = case
+    M = rows * P
+    g = torch.Generator(device="cuda:0").manual_seed(rows)
+    x1, x2 = (torch.randint(-127, 128, shape, dtype=torch.int8, device="cuda:0", generator=g) for shape in ((M, K), (K, N)))
+    x1[: M // 2] = x1[: M // 2].abs()
+    x2[:, N // 2:] = x2[:, N // 2:].abs()
+    s1, s2 = (torch.empty(c, device="cuda:0").uniform_(0.001, 0.02, generator=g) for c in (M, N))
+    b = torch.randint(-1000, 1000, (N,), dtype=torch.int32, device="cuda:0", generator=g)
+    peers = [torch.randint(-2 ** 20, 2 ** 20, (rows, N), dtype=torch.int32, device="cuda:0", generator=g) if ri else torch.randn((rows, N), device="cuda:0", generator=g)
+             for _ in range(P - 1)]
+    t, d = one_round(L.QUANT_MATMUL_REDUCE_SCATTER, M, K, N, P, rank)
+    tasks = list(tasks_of(L.QUANT_MATMUL_REDUCE_SCATTER, t, d))
+    acc = ((x1.double() @ x2.double()).to(torch.int64) + b).cpu()
+    step = 64 if rows <= 64 else 128
+    want = torch.full((len(tasks),), 77, dtype=torch.int64)
+    for task, r, row, col, ws in tasks:
+        if r != rank:
+            want[task] = acc[row:min(row + step, (r + 1) * rows), col:min(col + 256, N)].sum()
+    kept = acc[rank * rows:(rank + 1) * rows].to(torch.int32).to("cuda:0")
+    y = ((kept + sum(peers) if ri else kept).float() * s2) * s1[rank * rows:(rank + 1) * rows, None]
+    for p in ([] if ri else peers):
+        y = y + p
+    need = ops.kslice_plan(L.QUANT_MATMUL_REDUCE_SCATTER, L.INT8, M, K, N, rank, P, tiling=t)[0]
+    ws = torch.zeros(max(need, 65536), dtype=torch.uint8, device="cuda:0")
+    for w in (ws, ws, None):
+        cs = torch.full((len(tasks),), 77, dtype=torch.int64, device="cuda:0")
+        out = ops.quant_matmul_reduce_scatter(x1, x2.T.contiguous() if tb else x2, s1, s2, b, peers, rank, P, tiling=t, trans_b=tb, reduce_int32=ri, checksum=cs, workspace=w)
+        torch.cuda.synchronize()
+        assert torch.equal(cs.cpu(), want) and torch.equal(out, y.bfloat16()) and not ws[:65536].any()
