@@ -426,3 +426,44 @@ def test_quant_task_sums(case):
         out = ops.quant_matmul_reduce_scatter(x1, x2.T.contiguous() if tb else x2, s1, s2, b, peers, rank, P, tiling=t, trans_b=tb, reduce_int32=ri, checksum=cs, workspace=w)
         torch.cuda.synchronize()
         assert torch.equal(cs.cpu(), want) and torch.equal(out, y.bfloat16()) and not ws[:65536].any()
+
+
+def test_small_tiles_replay_from_a_hip_graph():
+    """A block-sum call, a sliced one and a task-sum one on one workspace in a captured graph: every replay, on new inputs and with eager calls in
+    between, gives what an eager call gives."""
+    _need_gpu()
+    g = torch.Generator(device="cuda:0").manual_seed(5)
+    i8 = lambda *s: torch.randint(-127, 128, s, dtype=torch.int8, device="cuda:0", generator=g)
+    ws = torch.zeros(32 << 20, dtype=torch.uint8, device="cuda:0")
+    s1, s2 = torch.full((400,), 0.01, device="cuda:0"), torch.full((1024,), 0.02, device="cuda:0")
+    x1, x2 = i8(51, 12800), i8(768, 12800)
+    y1, y2 = i8(400, 1024), i8(1024, 1024)
+    peers = [torch.randn((13, 768), device="cuda:0", generator=g) for _ in range(3)]
+    more = [torch.randn((50, 1024), device="cuda:0", generator=g) for _ in range(7)]
+    t, d = one_round(L.QUANT_MATMUL_REDUCE_SCATTER, 400, 1024, 1024, 8, 3)
+    tasks = len(list(tasks_of(L.QUANT_MATMUL_REDUCE_SCATTER, t, d)))
+
+    def calls(o):
+        ops.quant_matmul_splitk(x1, x2, s1[:51], s2[:768], None, peers, 4, 30, 13, workspace=ws, checksum=o[1], out=o[0], trans_b=True)
+        ops.quant_matmul_reduce_scatter(y1, y2, s1, s2, None, more, 3, 8, tiling=t, trans_b=True, checksum=o[3], out=o[2], workspace=ws)
+        ops.quant_matmul_splitk(y1[:100], y2, s1[:100], s2, None, [more[0][:9]], 2, 60, 9, workspace=ws, checksum=o[5], out=o[4], trans_b=True)
+
+    def outputs():
+        z = lambda *s, **k: torch.zeros(s, device="cuda:0", **k)
+        return [z(13, 768, dtype=torch.bfloat16), z(6, dtype=torch.int64), z(50, 1024, dtype=torch.bfloat16), z(tasks, dtype=torch.int64), z(9, 1024, dtype=torch.bfloat16), z(8, dtype=torch.int64)]
+
+    captured, eager = outputs(), outputs()
+    calls(captured)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        calls(captured)
+    for i in range(4):
+        x1.copy_(i8(51, 12800))
+        y2.copy_(i8(1024, 1024))
+        calls(eager)
+        for o in captured:
+            o.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(captured, eager)) and captured[1].any() and captured[3].any() and not ws[:65536].any(), i
