@@ -147,8 +147,8 @@ typedef struct CatcocSymmetricDesc {
     /* Scratch in HBM for launches whose k range is cut into slices or whose peers join in a second launch: the skinny-M
      * split-K path (catcoc_get_splitk_workspace_size() bytes) and every other launch of few tiles, aligned or ragged
      * (catcoc_get_kslice_workspace_size() bytes, optional there).  256-byte aligned.  Layout: the first
-     * CATCOC_WORKSPACE_COUNTER_BYTES hold one arrival counter per tile, at the same place for every shape and slice
-     * count; the partial tiles follow.  The caller ZEROES the counter block (or simply the whole buffer) once before
+     * CATCOC_WORKSPACE_COUNTER_BYTES hold arrival counters of tiles and sums that several tiles add up, at the same place for
+     * every shape and slice count; the partial tiles follow.  The caller ZEROES the counter block (or simply the whole buffer) once before
      * the first use; every launch leaves the counters at zero again, so launches of any shapes may share one
      * workspace that is large enough for each of them.  A launch touches no byte past what its query reports, however
      * large the workspace is, and where that is 0 nothing behind the counter block.  Launches that share a workspace

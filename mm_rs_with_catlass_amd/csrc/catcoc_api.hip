@@ -270,7 +270,8 @@ bool flex_ptrs_ok(const GemmArgs &a)
 
 // ---- one launch of small or mixed tiles (gemm_few.h, gemm_mid.h, gemm_mixed.h) or the other kernels ------------------------------------
 // Both sides of the choice are estimates in us, fitted to 460 calls of every operator (1 to 8192 rows, k 512 to 16384, n 512 to 8192,
-// 2 to 8 ranks, up to 6e11 operations, GPU time of calls behind each other): what a launch costs by itself, per workgroup of a CU, per
+// 2 to 8 ranks, up to 6e11 operations, GPU time of calls behind each other; what concerns slices, sums, dealt rows and whole rounds of
+// few tiles, to another 480): what a launch costs by itself, per round of workgroups (128 columns: per workgroup of a CU), per
 // KiB a workgroup pulls in through its CU (more from the second round of workgroups on: the first leaves the caches cold), per MB of
 // operands, per MB of peers and outputs; rows of k off the 16-byte grid and B as [k,n] cost more per KiB, rows of a B tile that are no whole
 // cache line more per MB.  Half of the estimates are within 0.10 of the tiles' times and 0.06 of the others', nine in ten within 0.22

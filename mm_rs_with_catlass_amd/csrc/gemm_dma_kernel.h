@@ -225,7 +225,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     for (int jj = 0; jj < A_DMA; ++jj) {
         if constexpr (FX) {
             const uint32_t row = ti.row + umin(16u * (w + NW * jj) + (lane >> 2), ti.rowsValid - 1u);
-            gA[jj] = flex_row_ptr(args, flex_row(args, row), ldaB) + kOff + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
+            gA[jj] = flex_row_ptr(args, flex_row<WM == 4>(args, row), ldaB) + kOff + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
         } else if constexpr (!TA) {
             gA[jj] = Ag + (size_t)(16 * (w + NW * jj) + (lane >> 2)) * ldaB + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
         } else if constexpr (ES == 1) {
@@ -452,7 +452,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             const uint32_t idx = tid + NT * q, row = idx >> 3, p = idx & 7u, slot = (p ^ ((row >> 1) & 7u)) * 16u;
             const int c = p * 16;
             *(v4i *)(sa + row * 128 + slot) =
-                load16_guarded(flex_row_ptr(args, flex_row(args, ti.row + umin(row, ti.rowsValid - 1u)), ldaB) + kEnd + c, tail - c, tail - 4 - c);
+                load16_guarded(flex_row_ptr(args, flex_row<WM == 4>(args, ti.row + umin(row, ti.rowsValid - 1u)), ldaB) + kEnd + c, tail - c, tail - 4 - c);
             if constexpr (TB) {
                 *(v4i *)(sb + row * 128 + slot) = load16_guarded(b + (size_t)(ti.col + umin(row, ti.colsValid - 1u)) * ldbB + kEnd + c, tail - c, tail - 4 - c);
             } else {
@@ -657,7 +657,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
                 for (int q = 0; q < PA; ++q) {
                     const uint32_t idx = tid + NT * q, row = idx >> 2;
                     const int c = (idx & 3u) * 16;
-                    pa[q] = load16_guarded(flex_row_ptr(args, flex_row(args, ti.row + umin(row, ti.rowsValid - 1u)), ldaB) + kEnd + c, tail - c, tail - 4 - c);
+                    pa[q] = load16_guarded(flex_row_ptr(args, flex_row<WM == 4>(args, ti.row + umin(row, ti.rowsValid - 1u)), ldaB) + kEnd + c, tail - c, tail - 4 - c);
                 }
 #pragma unroll
                 for (int q = 0; q < PB; ++q) {
@@ -757,7 +757,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             const int row = 8 * (w + NW * jj) + (lane >> 3);
             const uint32_t piece = ((lane & 7) ^ ((row >> 1) & 7)) * 16;
             if constexpr (FX) {
-                gP[jj] = flex_row_ptr(args, flex_row(args, ti.row + umin((uint32_t)row, ti.rowsValid - 1u)), ldaB) + piece;
+                gP[jj] = flex_row_ptr(args, flex_row<WM == 4>(args, ti.row + umin((uint32_t)row, ti.rowsValid - 1u)), ldaB) + piece;
                 gQ[jj] = Bg + (size_t)umin((uint32_t)row, ti.colsValid - 1u) * ldbB + piece;
             } else {
                 gP[jj] = Ag + (size_t)row * ldaB + piece;
@@ -867,7 +867,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
         for (int jj = 0; jj < APC; ++jj) {
             const int row = 8 * (w + NW * jj) + (lane >> 3);
             const uint32_t piece = ((lane & 7) ^ ((row >> 1) & 7)) * 16;
-            if constexpr (FX) gP[jj] = flex_row_ptr(args, flex_row(args, ti.row + umin((uint32_t)row, ti.rowsValid - 1u)), ldaB) + piece;
+            if constexpr (FX) gP[jj] = flex_row_ptr(args, flex_row<WM == 4>(args, ti.row + umin((uint32_t)row, ti.rowsValid - 1u)), ldaB) + piece;
             else gP[jj] = Ag + (size_t)row * ldaB + piece;
         }
         auto issue_ap = [&](uint32_t q) {   // pairs are issued in increasing q

@@ -14,8 +14,9 @@
 // Bound by the same things as the aligned kernels it shares its main loop with: the tile copies and the matrix pipes for long
 // k, the peers' stream for short k.  Measured against what ran these launches before (a kernel that staged its tiles through
 // registers, or one thread per output element), launches alternating: fp16 all-gather 8 x [1024,6148] x [6148,5120]
-// 243 ms -> 0.522 ms = 988 TFLOP/s (12296-byte rows, 8 bytes of k left over), W8A8 reduce-scatter 1000x1376x4096 with 125
-// rows per rank and stored tiles 277 -> 26 us, bf16 all-reduce 16x1024x8192 28.7 -> 13.0 us.
+// 243 ms -> 0.522 ms = 988 TFLOP/s (12296-byte rows, 8 bytes of k left over), W8A8 64x8192x8192 with 8 rows kept 22.7 -> 19.9 us.
+// Smaller launches are small tiles' (gemm_few.h, gemm_mid.h): W8A8 reduce-scatter 1000x1376x4096 of eight ranks, stored tiles, 277 us
+// before either, 26 here, 18 there, bf16 all-reduce 16x1024x8192 28.7, 13.0, 6.5.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -99,8 +100,10 @@ __device__ __forceinline__ void flex_task_of(const SchedParams &s, uint32_t r, u
     wsRow = ((round % s.stages) * s.blockPerComm + b) * s.m0 + (ri - mi * s.m0);
 }
 
-// Row of the problem that row v of the flexible tiles is: behind the hole that a mixed launch leaves to its small tiles.
-CATCOC_HD uint32_t flex_row(const GemmArgs &a, uint32_t v) { return a.fx.holeRows != 0 && v >= a.fx.hole0 ? v + a.fx.holeRows : v; }
+// Row of the problem that row v of the flexible tiles is: behind the hole that a mixed launch (eight waves, 256-row tiles) leaves to its small
+// tiles.  (The other launches have none, and the two arguments are a trip to host memory: 0.3 us of 26.)
+template <bool HOLE>
+CATCOC_HD uint32_t flex_row(const GemmArgs &a, uint32_t v) { return HOLE && a.fx.holeRows != 0 && v >= a.fx.hole0 ? v + a.fx.holeRows : v; }
 
 // Address of row v of the left operand (all-gather: row v of the shards behind each other).
 __device__ __forceinline__ const unsigned char *flex_row_ptr(const GemmArgs &a, uint32_t v, int64_t ldaB)
@@ -185,7 +188,7 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
     uint32_t *sumTask = (uint32_t *)(sums + 16 * 2 * NW);    // [16]
     __syncthreads();   // every wave has left the main loop's LDS reads behind
     if ((uint32_t)tid < ROWS) {
-        const uint32_t v = flex_row(args, t.row0 + tid);
+        const uint32_t v = flex_row<NW == 8>(args, t.row0 + tid);
         uint32_t e = FX_SKIP;
         if ((uint32_t)tid < t.rowsValid) {
             if (v - args.keptBegin < args.keptRows) {   // (unsigned: rows above keptBegin wrap)
@@ -206,7 +209,7 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
             }
         }
         dst[tid] = e;
-        if constexpr (I8) rowScale[tid] = args.scaleM[flex_row(args, umin(t.row0 + tid, args.fx.rows - 1u))];
+        if constexpr (I8) rowScale[tid] = args.scaleM[flex_row<NW == 8>(args, umin(t.row0 + tid, args.fx.rows - 1u))];
     }
     if (tid < 16 * 2 * NW) sums[tid] = 0;
     __syncthreads();
@@ -234,7 +237,7 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
     constexpr int NBUF = 3;
     const uint32_t keptEnd = args.keptBegin + args.keptRows;
     const uint32_t kLo = args.keptBegin > t.row0 ? umin(args.keptBegin - t.row0, t.rowsValid) : 0u;   // the tile's kept rows: [kLo, kLo + kN)
-    const bool none = args.fx.holeRows != 0 && args.sched.op == OP_REDUCE_SCATTER;   // (a mixed launch: they lie in the hole)
+    const bool none = NW == 8 && args.fx.holeRows != 0 && args.sched.op == OP_REDUCE_SCATTER;   // (a mixed launch: they lie in the hole)
     const uint32_t kN = !none && keptEnd > t.row0 + kLo ? umin(keptEnd - t.row0, t.rowsValid) - kLo : 0u;
     const int64_t kept0 = (int64_t)t.row0 + kLo - args.keptBegin;   // (of no use, and possibly negative, when the tile has none)
     const bool late = args.fx.late != 0;   // the kept rows' peers are the second launch's
@@ -295,7 +298,7 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     const uint32_t i = wm * 32 * MB + mb * 32 + half * 16 + j * 2 + lrow;
-                    if (colOk && i < t.rowsValid) *(v4i *)((int32_t *)args.accDump + (size_t)flex_row(args, t.row0 + i) * args.N + gcol) = cur[j];
+                    if (colOk && i < t.rowsValid) *(v4i *)((int32_t *)args.accDump + (size_t)flex_row<NW == 8>(args, t.row0 + i) * args.N + gcol) = cur[j];
                 }
             }
             auto add_peers = [&](auto add) {   // in slot order
