@@ -407,10 +407,11 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other, uint64_t room = 0)
     if (a.transA || kBytes % 4 != 0 || kBytes < 16 || (!a.transB && ldbB % 16 != 0) || a.N % 4 != 0 || ldaB * 160u > 0x7fffffffull || ldbB * 160u > 0x7fffffffull ||
         rows >= (1u << 30) || s.n0 != 256 || (s.m0 != 64 && s.m0 != 128))
         return no;
-    // Checksums: of tasks, whole numbers only (the order of the tiles' additions is open), and of the 128x128 blocks of explicit kept rows,
-    // for tiles that meet in the workspace's counter block (sum_add) or have all of a block.  Decode launches that also want the kept rows' int32 block stay where their k slices leave it on the way.
+    // Checksums: of tasks, and of the 128x128 blocks of explicit kept rows, for tiles that meet in the workspace's counter block (sum_add,
+    // sum_in_order) or have all of a block.  Decode launches that also want the kept rows' int32 block stay where their k slices leave it on
+    // the way.
     const bool rowMask = (a.flags & GF_ROW_MASK) != 0, sums = (a.flags & GF_OUTBOUND_STORE) == 0 && a.checksum != nullptr && (rowMask || a.keptRows < rows);
-    if ((sums && !rowMask && (es != 1 || a.skCount == nullptr || s.coreLoops > kCounterBlockBytes / 16u)) || (rowMask && a.cAccum != nullptr)) return no;
+    if ((sums && !rowMask && (a.skCount == nullptr || s.coreLoops > kCounterBlockBytes / 16u)) || (rowMask && a.cAccum != nullptr)) return no;
     const CallSize c = call_size(a, es);
     const SmallTileCost *best = nullptr;
     double least = 0.0;
@@ -420,14 +421,21 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other, uint64_t room = 0)
     const bool keptOnly = rowMask && a.accDump == nullptr;
     auto kept_tile0 = [&](uint32_t step) { return keptOnly ? a.keptBegin / step : 0u; };
     auto kept_tiles = [&](uint32_t step) { return keptOnly ? (a.keptBegin + a.keptRows - 1u) / step + 1u - kept_tile0(step) : (uint32_t)ceil_div((uint32_t)rows, step); };
+    // (floats: what a task's tiles add has places of its own there, as many as row tiles can have some of its rows, by column tiles)
+    auto sum_parts = [&](const SmallTileCost &t) -> uint32_t {
+        const uint32_t dealt = ceil_div((uint32_t)rows, t.rows), h = umin(s.m0, s.mRank);
+        const uint32_t least = t.cols != 128 || dealt < 2 ? t.rows : (uint32_t)rows / dealt - a.keptRows / dealt - 1u;   // rows of others that a tile has
+        return (int32_t)least < 1 ? 0u : ((h + least - 2u) / least + 1u) * (256u / t.cols);
+    };
     for (const SmallTileCost &t : kSmallTiles) {
+        if (sums && es != 1 && (sum_parts(t) == 0 || s.coreLoops * sum_parts(t) > kCounterBlockBytes / 16u)) continue;
         if (sums && rowMask && (t.cols != 128 || (t.rows < 128 && rows > (uint64_t)t.rows)) && (a.skCount == nullptr || (rows + 127) / 128 * ceil_div(a.N, 128u) > kCounterBlockBytes / 16u))
             continue;
         const uint64_t n = (rows + t.rows - 1) / t.rows * ceil_div(a.N, t.cols);
         const double rounds = (double)((n + 255) / 256), perCu = t.cols < 128 || n <= 256 ? rounds : n / 256.0;
         const double perKib = (t.rows + t.cols) * rounds * (t.kib + (kBytes % 16 ? t.off16 : 0.0) + (a.transB ? 0.0 : t.kn) + (n > 256 ? t.later : 0.0));
         const double rest = t.launch + t.workgroup * perCu + c.mb * t.mb + (!a.transB && t.cols * es < 128u ? c.mb * t.partLine : 0.0) + c.moved * t.moved +
-                            (sums && !rowMask ? (t.cols == 128 ? 2.0 : 0.7) * rounds : 0.0);   // (the tasks' sums)
+                            (sums && !rowMask ? (t.cols == 128 ? 2.0 : 0.7) * rounds + (es != 1 ? 0.5 + 0.05 * sum_parts(t) : 0.0) : 0.0);   // (the tasks' sums)
         for (const uint32_t f : {1u, 2u, 3u, 4u, 6u, 8u}) {
             // (at most a workgroup per CU, two chunks of k per wave; k of whole numbers short enough that a slice's sums and the whole are the same)
             if (f > 1 && (t.cols >= 128 || n * f > 256 || kBytes < f * 1024u || (es == 1 && a.K > 131072u) || a.skCount == nullptr ||
@@ -467,6 +475,7 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other, uint64_t room = 0)
     a.fx.colTiles = ceil_div(a.N, best->cols);
     a.fx.slices = slices;
     a.fx.keptOnly = keptOnly ? 1u : 0u;
+    a.fx.sumParts = sums && es != 1 ? sum_parts(*best) : 0u;
     a.fx.keptTile0 = kept_tile0(best->rows);
     a.fx.keptTiles = kept_tiles(best->rows);
     if (slices > 1) a.skPart = (int32_t *)((unsigned char *)a.skCount + kCounterBlockBytes);

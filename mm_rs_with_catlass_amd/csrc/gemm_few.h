@@ -51,6 +51,7 @@ struct MetSum {
     uint32_t parts, word;   // tiles times slices that add to it; its number
 };
 constexpr uint32_t FEW_TILE_COUNTERS = 8192;   // of 4 bytes; then as many bytes again for the sums' words
+constexpr uint32_t FEW_TASK_COUNTERS = 1024;   // the first of those that count the parts of a task's sum of floats
 
 __device__ __forceinline__ MetSum sum_add(const GemmArgs &args, uint32_t word, uint32_t parts, long long sum)
 {
@@ -78,17 +79,52 @@ __device__ __forceinline__ MetSum block_add(const GemmArgs &args, uint32_t row0,
                    slices * ceil_div(umin(128u, rows - br * 128u), (uint32_t)BM) * ceil_div(umin(128u, args.N - bc * 128u), (uint32_t)BN), sum);
 }
 
-// The tasks that a tile has rows of (dst: FX_SUM and the task; the rows of a task are neighbours).  A row's sum goes to LDS, and the thread of a
-// task's first row adds up its rows and adds that to the task's word.  cur: groups of four columns, as both kernels finish them; rowOf(i): row i
-// of the tile; tiles(begin, end): row tiles that have some of the rows from begin up to end.
-template <int BN, int NT, int UN, typename RowOf, typename Tiles>
-__device__ __forceinline__ void task_sums(const GemmArgs &args, long long *rowSum, const uint32_t *dst, const v4i (&cur)[UN], uint32_t tid, bool colOk, uint32_t col0, uint32_t rowsValid,
-                                          uint32_t slices, RowOf rowOf, Tiles tiles)
+// Float reduce-scatters with checksums, tiles that line up with the tasks (and up to three launches) -> these: fp16 2904x2364x640 of eight
+// ranks 44 -> 20 us, bf16 664x3840x512 of four 64 -> 20, 1084x3328x1536 50 -> 28; 70 drawn calls take 0.72 of their time.
+// Sums of floats need an order: every tile's part has a place of its own (place of parts), an exchange puts it there and is through when it
+// returns, and the tile that counts last adds the parts in order and leaves zeros behind.
+__device__ __forceinline__ void sum_in_order(const GemmArgs &args, uint32_t task, uint32_t parts, uint32_t place, double sum)
 {
+    if (parts > 1u) {
+        unsigned long long *const at = (unsigned long long *)(args.skCount + FEW_TILE_COUNTERS) + (size_t)task * args.fx.sumParts;
+        uint32_t *const count = args.skCount + FEW_TASK_COUNTERS + task;
+        (void)__hip_atomic_exchange(at + place, __builtin_bit_cast(unsigned long long, sum), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        CATCOC_WAIT_VMCNT(0);
+        if (__hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != parts - 1u) return;
+        __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        sum = 0.0;
+        for (uint32_t i = 0; i < parts; i += 8u) {   // (eight on their way at a time)
+            unsigned long long p[8];
+#pragma unroll
+            for (uint32_t q = 0; q < 8u; ++q) p[q] = i + q < parts ? __hip_atomic_load(at + i + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+#pragma unroll
+            for (uint32_t q = 0; q < 8u; ++q)
+                if (i + q < parts) {
+                    sum += __builtin_bit_cast(double, p[q]);
+                    __hip_atomic_store(at + i + q, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+        }
+    }
+    ((double *)args.checksum)[task] = sum;
+}
+
+// The tasks that a tile has rows of (dst: FX_SUM and the task; the rows of a task are neighbours).  A row's sum goes to LDS, and the thread of a
+// task's first row adds up its rows and adds that to the task's word.  cur: groups of four columns, as both kernels finish them; rt: the row
+// tile; rowOf(i): row i of it; tileOf(v): the row tile that has row v.
+template <uint32_t DT, int BN, int NT, int UN, typename RowOf, typename TileOf>
+__device__ __forceinline__ void task_sums(const GemmArgs &args, void *rowSums, const uint32_t *dst, const v4i (&cur)[UN], uint32_t tid, bool colOk, uint32_t rt, uint32_t col0,
+                                          uint32_t rowsValid, uint32_t slices, RowOf rowOf, TileOf tileOf)
+{
+    constexpr bool I8 = DT == DT_I8;
+    using Sum = typename std::conditional<I8, long long, double>::type;
+    Sum *const rowSum = (Sum *)rowSums;
     constexpr uint32_t LPR = BN / 4;
 #pragma unroll
     for (int j = 0; j < UN; ++j) {
-        long long v = colOk ? ((long long)cur[j].x + cur[j].y) + ((long long)cur[j].z + cur[j].w) : 0;
+        Sum v;
+        if constexpr (I8) v = ((long long)cur[j].x + cur[j].y) + ((long long)cur[j].z + cur[j].w);
+        else v = ((double)i2f(cur[j].x) + (double)i2f(cur[j].y)) + ((double)i2f(cur[j].z) + (double)i2f(cur[j].w));
+        v = colOk ? v : (Sum)0;
         v = dpp_add64<0x111, 0xf>(v);   // row_shr:1, 2, 4: eight lanes' sum in the last of them, 8: sixteen lanes', row_bcast:15: 32 lanes'
         v = dpp_add64<0x112, 0xf>(v);
         v = dpp_add64<0x114, 0xf>(v);
@@ -105,16 +141,18 @@ __device__ __forceinline__ void task_sums(const GemmArgs &args, long long *rowSu
     const uint32_t v = rowOf(tid), r = fast_div(v, args.fx.dRank, ri), mi = ri / sp.m0;
     const uint32_t begin = r * sp.mRank + mi * sp.m0, end = begin + umin(sp.m0, sp.mRank - mi * sp.m0);   // the task's rows
     const uint32_t upTo = umin(end - v + tid, rowsValid);
-    long long sum[4] = {0, 0, 0, 0};
+    Sum sum[4] = {0, 0, 0, 0};
     uint32_t i = tid;
     for (; i + 4u <= upTo; i += 4u) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) sum[q] += rowSum[i + q];
     }
     for (; i < upTo; ++i) sum[0] += rowSum[i];
-    const uint32_t colBegin = col0 / sp.n0 * sp.n0;
-    sum_finish(args, sum_add(args, e & FX_INDEX, slices * tiles(begin, end) * ceil_div(umin(sp.n0, args.N - colBegin), (uint32_t)BN),
-                             (sum[0] + sum[1]) + (sum[2] + sum[3])));
+    const uint32_t colBegin = col0 / sp.n0 * sp.n0, first = tileOf(begin), colTiles = ceil_div(umin(sp.n0, args.N - colBegin), (uint32_t)BN);
+    const uint32_t parts = (tileOf(end - 1u) - first + 1u) * colTiles;
+    const Sum mine = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+    if constexpr (I8) sum_finish(args, sum_add(args, e & FX_INDEX, slices * parts, mine));
+    else sum_in_order(args, e & FX_INDEX, parts, (rt - first) * colTiles + (col0 - colBegin) / BN, mine);
 }
 
 // MB, NB: 32-row and 32-column blocks of the tile.
@@ -391,7 +429,7 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
                 const auto e = acc[mb][nb][r];
                 *(int *)(smem + ((w * BM + row) * BN + ((nb * 32 + c32) ^ ((uint32_t)h * SWZ << 5))) * 4) = __builtin_bit_cast(int, e);
             }
-    const bool store = (flags & GF_OUTBOUND_STORE) != 0, taskSums = I8 && !store && (flags & GF_ROW_MASK) == 0 && args.checksum != nullptr;
+    const bool store = (flags & GF_OUTBOUND_STORE) != 0, taskSums = !store && (flags & GF_ROW_MASK) == 0 && args.checksum != nullptr && sp.op == OP_REDUCE_SCATTER;
     if (tid < BM) {
         const uint32_t v = row0 + tid;
         uint32_t e = FX_SKIP;
@@ -403,7 +441,7 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
                 const uint32_t r = fast_div(v, args.fx.dRank, ri);
                 flex_task_of(sp, r, ri, col0 / sp.n0, task, ws);
                 e = FX_OUT | ws;
-            } else if (I8 && taskSums) {
+            } else if (taskSums) {
                 uint32_t ri, task, ws;
                 const uint32_t r = fast_div(v, args.fx.dRank, ri);
                 flex_task_of(sp, r, ri, col0 / sp.n0, task, ws);
@@ -434,6 +472,10 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
         if constexpr (I8) cur[j] += bv;
         d[j] = dst[row];
     }
+    auto add_task_sums = [&]() {   // (whole numbers: every slice's part; floats: of the sums they end up as)
+        task_sums<DT, BN, 256, UN>(args, dst + BM + 12, dst, cur, tid, colOk, rt, col0, rowsValid, I8 ? slices : 1u, [&](uint32_t i) { return row0 + i; },
+                                   [](uint32_t v) { return v / BM; });
+    };
     MetSum blockSum;
     const bool sums = I8 && (flags & GF_ROW_MASK) && args.checksum;
     if constexpr (I8) {
@@ -448,9 +490,7 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
             __syncthreads();
             if (tid == 0) blockSum = block_add<BM, BN>(args, row0, col0, rows, slices, (red[0] + red[1]) + (red[2] + red[3]));
         }
-        if (taskSums)
-            task_sums<BN, 256, UN>(args, (long long *)(dst + BM + 12), dst, cur, tid, colOk, col0, rowsValid, slices, [&](uint32_t i) { return row0 + i; },
-                                   [](uint32_t begin, uint32_t end) { return (end - 1u) / BM - begin / BM + 1u; });
+        if (taskSums) add_task_sums();
     }
     // ---- k slices: the last to arrive has the sum of all, in slice order
     if constexpr (SL) {
@@ -505,6 +545,9 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
             }
             return;
         }
+    }
+    if constexpr (!I8) {
+        if (taskSums) add_task_sums();
     }
     if (!colOk) return;
     if (args.accDump) {

@@ -316,7 +316,7 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
                 const auto e = acc[mb][nb][r];
                 *(int *)(smem + ((wg * BM + row) * BN + (((wn * 2 + nb) * 32 + (t2 & 31)) ^ ((uint32_t)((t2 >> 5) & 1) * SWZ << 5))) * 4) = __builtin_bit_cast(int, e);
             }
-    const bool store = (flags & GF_OUTBOUND_STORE) != 0, taskSums = I8 && !store && (flags & GF_ROW_MASK) == 0 && args.checksum != nullptr;
+    const bool store = (flags & GF_OUTBOUND_STORE) != 0, taskSums = !store && (flags & GF_ROW_MASK) == 0 && args.checksum != nullptr && sp.op == OP_REDUCE_SCATTER;
     if (tid < BM) {
         const uint32_t v = rowOf(tid);
         uint32_t e = FX_SKIP;
@@ -328,7 +328,7 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
                 const uint32_t r = fast_div(v, args.fx.dRank, ri);
                 flex_task_of(sp, r, ri, col0 / sp.n0, task, ws);
                 e = FX_OUT | ws;
-            } else if (I8 && taskSums) {
+            } else if (taskSums) {
                 uint32_t ri, task, ws;
                 const uint32_t r = fast_div(v, args.fx.dRank, ri);
                 flex_task_of(sp, r, ri, col0 / sp.n0, task, ws);
@@ -378,20 +378,19 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
                 blockSum = block_add<BM, BN>(args, row0, col0, rowEnd, 1u, all);
             }
         }
-        if (taskSums) {
-            // (dealt rows: the tile of row x of those that are not kept, from a first guess)
-            auto first_other = [&](uint32_t t) { return deal_begin(t, f.dealRows, f.dealRest) - deal_begin(t, f.dealKept, f.dealKeptRest); };
-            auto tile_of = [&](uint32_t v) -> uint32_t {
-                if (!dealt) return v / BM;
-                const uint32_t x = v >= keptEnd ? v - keptRows : v;
-                uint32_t t = umin((uint32_t)((float)x * (float)rowTiles / (float)(rowEnd - keptRows)), rowTiles - 1u);
-                while (first_other(t) > x) --t;
-                while (first_other(t + 1u) <= x) ++t;
-                return t;
-            };
-            task_sums<BN, NT, UN>(args, (long long *)(rowScale + BM + 16), dst, cur, (uint32_t)t2, colOk, col0, rowsValid, 1u, rowOf,
-                                  [&](uint32_t begin, uint32_t end) { return tile_of(end - 1u) - tile_of(begin) + 1u; });
-        }
+    }
+    if (taskSums) {
+        // (dealt rows: the tile of row x of those that are not kept, from a first guess)
+        auto first_other = [&](uint32_t t) { return deal_begin(t, f.dealRows, f.dealRest) - deal_begin(t, f.dealKept, f.dealKeptRest); };
+        auto tile_of = [&](uint32_t v) -> uint32_t {
+            if (!dealt) return v / BM;
+            const uint32_t x = v >= keptEnd ? v - keptRows : v;
+            uint32_t t = umin((uint32_t)((float)x * (float)rowTiles / (float)(rowEnd - keptRows)), rowTiles - 1u);
+            while (first_other(t) > x) --t;
+            while (first_other(t + 1u) <= x) ++t;
+            return t;
+        };
+        task_sums<DT, BN, NT, UN>(args, rowScale + BM + 16, dst, cur, (uint32_t)t2, colOk, rt, col0, rowsValid, 1u, rowOf, tile_of);
     }
     if (!colOk) return;
     if (args.accDump) {

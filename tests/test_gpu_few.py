@@ -467,3 +467,40 @@ def test_small_tiles_replay_from_a_hip_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(captured, eager)) and captured[1].any() and captured[3].any() and not ws[:65536].any(), i
+
+
+# (rows per rank, N, K, P, rank, weights as [n,k]): as test_quant_task_sums; sums of floats are added in one order
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", [(1, 256, 100, 8, 3, True), (5, 388, 1040, 8, 0, True), (33, 640, 416, 4, 3, False), (130, 900, 772, 2, 1, True), (37, 1024, 12672, 4, 2, False),
+                                  (43, 1920, 1152, 2, 0, True), (363, 640, 2364, 8, 6, False), (301, 1800, 646, 4, 1, True)])
+def test_float_task_sums(case, dtype):
+    _need_gpu()
+    rows, N, K, P, rank, tb = case
+    M = rows * P
+    g = torch.Generator(device="cuda:0").manual_seed(rows)
+    A, B = torch.randn((M, K), device="cuda:0", generator=g).to(dtype), (torch.randn((K, N), device="cuda:0", generator=g) * 0.05).to(dtype)
+    Bd = B.T.contiguous() if tb else B
+    peers = [torch.randn((rows, N), device="cuda:0", generator=g) for _ in range(P - 1)]
+    comm = L.MATMUL_REDUCE_SCATTER
+    t, d = one_round(comm, M, K, N, P, rank)
+    tasks = list(tasks_of(comm, t, d))
+    step = 64 if rows <= 64 else 128
+    need = ops.kslice_plan(comm, dtype, M, K, N, rank, P, tiling=t)[0]
+    ws = torch.zeros(max(need, 65536), dtype=torch.uint8, device="cuda:0")
+    first = None
+    for _ in range(4):
+        cs, dump = torch.full((len(tasks),), 77.0, dtype=torch.float64, device="cuda:0"), torch.zeros((M, N), device="cuda:0")
+        out = ops.matmul_reduce_scatter(A, Bd, peers, rank, P, tiling=t, trans_b=tb, checksum=cs, acc_dump=dump, workspace=ws)
+        torch.cuda.synchronize()
+        assert not ws[:65536].any() and (first is None or torch.equal(first, cs))
+        first = cs
+    bound = 8 * K ** 0.5 * 2.0 ** -24 * torch.outer(A.double().norm(dim=1), B.double().norm(dim=0)) + 1e-9   # (as sum_bound)
+    assert ((dump.double() - A.double() @ B.double()).abs() <= bound).all()
+    full, got = dump.double().cpu(), cs.cpu()
+    for task, r, row, col, _ in tasks:
+        own = full[row:min(row + step, (r + 1) * rows), col:min(col + 256, N)]
+        assert got[task] == 77.0 if r == rank else abs(got[task] - own.sum()) <= own.numel() * 2.0 ** -51 * own.abs().sum(), task
+    y = dump[rank * rows:(rank + 1) * rows]
+    for p in peers:
+        y = y + p
+    assert torch.equal(out, y.to(dtype))
