@@ -462,6 +462,8 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other, uint64_t room = 0)
     // (with the kept rows dealt out the shares' margin is not needed: 199 reduce-scatters then take 1.009 of the best choice's time for each, 1.018
     // with it; two of them lost 0.12 and 0.20, one of the two with the margin as well)
     if (s.op == OP_REDUCE_SCATTER && !rowMask && !sums && (mixed.large || best->cols == 128)) other *= 1.15;
+    // (all-reduce and all-gather: 52 of 64 rows and more take 1.013 of the best choice's time for each, 1.025 without this; the same one loses)
+    if (s.op != OP_REDUCE_SCATTER && !rowMask) other *= 1.05;
     if ((mixed.large ? mixed.us : least) > other || tiles > (1u << 24) || !flex_ptrs_ok(a)) return no;
     a.fx.dRank = make_fast_div(s.mRank);
     a.splitK = 0;

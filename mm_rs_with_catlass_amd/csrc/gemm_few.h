@@ -80,7 +80,7 @@ __device__ __forceinline__ MetSum block_add(const GemmArgs &args, uint32_t row0,
 }
 
 // Float reduce-scatters with checksums, tiles that line up with the tasks (and up to three launches) -> these: fp16 2904x2364x640 of eight
-// ranks 44 -> 20 us, bf16 664x3840x512 of four 64 -> 20, 1084x3328x1536 50 -> 28; 70 drawn calls take 0.72 of their time.
+// ranks 44 -> 25 us, bf16 664x3840x512 of four 63 -> 18, fp16 1084x3328x1536 51 -> 27; 70 drawn calls take 0.72 of their time.
 // Sums of floats need an order: every tile's part has a place of its own (place of parts), an exchange puts it there and is through when it
 // returns, and the tile that counts last adds the parts in order and leaves zeros behind.
 __device__ __forceinline__ void sum_in_order(const GemmArgs &args, uint32_t task, uint32_t parts, uint32_t place, double sum)
