@@ -48,7 +48,7 @@ __device__ __forceinline__ void dma16_base(const unsigned char *base, uint32_t o
 // late as there is something else to do, so that the atomic's trip is not waited for.
 struct MetSum {
     unsigned long long before, mine;
-    uint32_t parts, word;   // tiles times slices that add to it; its number
+    uint32_t parts, word;   // tiles times slices that add to it (256 at most: 40 tiles, or a sliced launch's workgroups); its number
 };
 constexpr uint32_t FEW_TILE_COUNTERS = 8192;   // of 4 bytes; then as many bytes again for the sums' words
 constexpr uint32_t FEW_TASK_COUNTERS = 1024;   // the first of those that count the parts of a task's sum of floats
