@@ -432,7 +432,10 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other, uint64_t room = 0)
         if (sums && rowMask && (t.cols != 128 || (t.rows < 128 && rows > (uint64_t)t.rows)) && (a.skCount == nullptr || (rows + 127) / 128 * ceil_div(a.N, 128u) > kCounterBlockBytes / 16u))
             continue;
         const uint64_t n = (rows + t.rows - 1) / t.rows * ceil_div(a.N, t.cols);
-        const double rounds = (double)((n + 255) / 256), perCu = t.cols < 128 || n <= 256 ? rounds : n / 256.0;
+        if (t.cols < 128 && n > 512) continue;   // (beyond two rounds their operands leave the caches: all-gather 8 x [682,9000] x [9000,672] 234, larger tiles 181)
+        // (a second round of 128-wide tiles is a whole one where k is short: the workgroups are mostly start and end. W8A8
+        // reduce-scatters of [3320,640] x [640,640] over 4 ranks 15.8 on them, 12.6 on smaller ones; pipelined [3072,512] x [512,768] 15.7, 12.4)
+        const double rounds = (double)((n + 255) / 256), perCu = t.cols < 128 || n <= (kBytes <= 1024 ? 512u : 256u) ? rounds : n / 256.0;
         const double perKib = (t.rows + t.cols) * rounds * (t.kib + (kBytes % 16 ? t.off16 : 0.0) + (a.transB ? 0.0 : t.kn) + (n > 256 ? t.later : 0.0));
         const double rest = t.launch + t.workgroup * perCu + c.mb * t.mb + (!a.transB && t.cols * es < 128u ? c.mb * t.partLine : 0.0) + c.moved * t.moved +
                             (sums && !rowMask ? (t.cols == 128 ? 2.0 : 0.7) * rounds + (es != 1 ? 0.5 + 0.05 * sum_parts(t) : 0.0) : 0.0);   // (the tasks' sums)
