@@ -333,10 +333,13 @@ struct MixedRows {
     double us;
 };
 
+// A reduce-scatter's kept rows, with their peers, all run on the small tiles; with one rank every row is kept and there are no peers.
+bool kept_apart(const GemmArgs &a) { return a.sched.op == OP_REDUCE_SCATTER && a.sched.P > 1; }
+
 MixedRows mixed_rows(const GemmArgs &a, uint32_t es, uint32_t rows)
 {
     const double chunks = call_size(a, es).kib * 8.0;
-    const uint32_t kept = a.sched.op == OP_REDUCE_SCATTER && a.sched.P > 1 ? a.keptRows : 0u;
+    const uint32_t kept = kept_apart(a) ? a.keptRows : 0u;
     const double large = 9.0 + 1.70 * chunks + (kept ? 0.0 : 4.4 * a.nPeers), small = 8.0 + 0.55 * chunks + 1.1 * a.nPeers;
     const uint32_t largeCols = ceil_div(a.N, 256u), smallCols = ceil_div(a.N, 128u);
     MixedRows best = {0, 0.0};
@@ -370,7 +373,8 @@ void plan_mixed(GemmArgs &a, uint32_t es, uint32_t rows, uint32_t large)
     f.slices = 1;
     f.keptOnly = f.late = 0;
     f.holeRows = rows - large;
-    f.hole0 = a.sched.op == OP_REDUCE_SCATTER && a.sched.P > 1 ? umin(a.keptBegin, large) : large;
+    f.keptInHole = kept_apart(a) ? 1u : 0u;
+    f.hole0 = f.keptInHole ? umin(a.keptBegin, large) : large;
     f.largeTiles = f.rowTiles * f.colTiles;
 }
 

@@ -237,7 +237,7 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
     constexpr int NBUF = 3;
     const uint32_t keptEnd = args.keptBegin + args.keptRows;
     const uint32_t kLo = args.keptBegin > t.row0 ? umin(args.keptBegin - t.row0, t.rowsValid) : 0u;   // the tile's kept rows: [kLo, kLo + kN)
-    const bool none = NW == 8 && args.fx.holeRows != 0 && args.sched.op == OP_REDUCE_SCATTER;   // (a mixed launch: they lie in the hole)
+    const bool none = NW == 8 && args.fx.keptInHole != 0;   // (mixed launches)
     const uint32_t kN = !none && keptEnd > t.row0 + kLo ? umin(keptEnd - t.row0, t.rowsValid) - kLo : 0u;
     const int64_t kept0 = (int64_t)t.row0 + kLo - args.keptBegin;   // (of no use, and possibly negative, when the tile has none)
     const bool late = args.fx.late != 0;   // the kept rows' peers are the second launch's

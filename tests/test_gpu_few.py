@@ -166,6 +166,11 @@ def test_quant_kept_rows_with_checksums(case):
     assert np.array_equal(host16(out), want) and np.array_equal(dump.cpu().numpy(), acc) and np.array_equal(cs.cpu().numpy(), sums)
 
 
+def marked(rows, N, dtype):
+    """An output that says which of its elements a launch left alone."""
+    return torch.full((rows, N), 12345.0, dtype=dtype, device="cuda:0")
+
+
 def one_round(comm, M, K, N, P, rank):
     """Tiling and descriptor of a call whose tiles all have a place of their own in the symmetric workspace."""
     t, d = ops.default_tiling(M, K, N, P, m0=0, n0=0, k0=0), L.make_desc(rank, P, [16] * (P - 1))
@@ -197,7 +202,7 @@ def test_float_larger_tiles(case):
     else:
         t, d = one_round(L.MATMUL_REDUCE_SCATTER, M, K, N, P, rank)
         ob = torch.full((L.load().catcoc_get_workspace_size(L.MATMUL_REDUCE_SCATTER, L.BF16, C.byref(t), C.byref(d)) // 4,), 3.0, device="cuda:0")
-        out = ops.matmul_reduce_scatter(A, Bd, peers, rank, P, tiling=t, trans_b=tb, outbound=ob, acc_dump=dump)
+        out = ops.matmul_reduce_scatter(A, Bd, peers, rank, P, tiling=t, trans_b=tb, outbound=ob, acc_dump=dump, out=marked(rows, N, torch.bfloat16))
         tiles, full = ob.cpu().numpy().reshape(-1, 256), dump.cpu().numpy()
         for task, r, row, col, ws in tasks_of(L.MATMUL_REDUCE_SCATTER, t, d):
             if r != rank:
@@ -212,8 +217,10 @@ def test_float_larger_tiles(case):
 
 
 # (rows per rank, N, K, P, rank, weights as [n,k], int32 peers): launches of 256x256 and 128x128 tiles; the kept rows (on small tiles) at the
-# start, in the middle and at the end, k of whole pairs of steps and 4 to 124 bytes more, columns past a tile
-@pytest.mark.parametrize("case", [(335, 6912, 3204, 8, 5, False, False), (543, 3844, 3836, 8, 0, True, True), (664, 3460, 5888, 8, 7, True, False)])
+# start, in the middle and at the end, k of whole pairs of steps and 4 to 124 bytes more, columns past a tile; one rank, whose kept rows are
+# on tiles of both kinds
+@pytest.mark.parametrize("case", [(335, 6912, 3204, 8, 5, False, False), (543, 3844, 3836, 8, 0, True, True), (664, 3460, 5888, 8, 7, True, False), (4344, 3844, 3836, 1, 0, True, False),
+                                  (3700, 3840, 3072, 1, 0, False, False)])
 def test_quant_mixed_tiles(case):
     _need_gpu()
     rows, N, K, P, rank, tb, ri = case
@@ -229,7 +236,7 @@ def test_quant_mixed_tiles(case):
     ob = torch.full((size,), 3, dtype=torch.int32 if ri else torch.float32, device="cuda:0")
     dump, sums = torch.full((M, N), -7, dtype=torch.int32, device="cuda:0"), torch.full((rows, N), -7, dtype=torch.int32, device="cuda:0")
     out = ops.quant_matmul_reduce_scatter(x1, x2.T.contiguous() if tb else x2, s1, s2, b, peers, rank, P, tiling=t, trans_b=tb, reduce_int32=ri, outbound=ob,
-                                          acc_dump=dump, c_accum=sums)
+                                          acc_dump=dump, c_accum=sums, out=marked(rows, N, torch.bfloat16))
     acc = (x1.double() @ x2.double()).to(torch.int32) + b   # (exact)
     kept = acc[rank * rows:(rank + 1) * rows]
     if ri:
@@ -248,7 +255,7 @@ def test_quant_mixed_tiles(case):
 
 
 @pytest.mark.parametrize("case", [("allgather", 845, 3940, 3330, 8, 3, True), ("allgather", 822, 2308, 6560, 8, 0, True), ("allreduce", 3438, 5892, 3712, 4, 0, True),
-                                  ("reduce_scatter", 6184, 3072, 10752, 8, 2, False)])
+                                  ("reduce_scatter", 6184, 3072, 10752, 8, 2, False), ("reduce_scatter", 8144, 1696, 5120, 1, 0, True), ("reduce_scatter", 3000, 4096, 4096, 1, 0, False)])
 def test_float_mixed_tiles(case):
     test_float_larger_tiles(case)
 
