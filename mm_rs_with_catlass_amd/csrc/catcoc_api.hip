@@ -444,8 +444,9 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other, uint64_t room = 0)
         const double rest = t.launch + t.workgroup * perCu + c.mb * t.mb + (!a.transB && t.cols * es < 128u ? c.mb * t.partLine : 0.0) + c.moved * t.moved +
                             (sums && !rowMask ? (t.cols == 128 ? 2.0 : 0.7) * rounds + (es != 1 ? 0.5 + 0.05 * sum_parts(t) : 0.0) : 0.0);   // (the tasks' sums)
         for (const uint32_t f : {1u, 2u, 3u, 4u, 6u, 8u}) {
-            // (at most a workgroup per CU, two chunks of k per wave; k of whole numbers short enough that a slice's sums and the whole are the same)
-            if (f > 1 && (t.cols >= 128 || n * f > 256 || kBytes < f * 1024u || (es == 1 && a.K > 131072u) || a.skCount == nullptr ||
+            // (at most a workgroup per CU, two chunks of k per wave; k of whole numbers short enough that their whole sum is within 32 bits, as
+            // the slices' sums are that checksums are added up from: 131072 products of -128 and -128 are one past the end)
+            if (f > 1 && (t.cols >= 128 || n * f > 256 || kBytes < f * 1024u || (es == 1 && a.K >= 131072u) || a.skCount == nullptr ||
                           few_partials(t, kept_tiles(t.rows), a.N, f) > room))
                 break;
             const double us = rest + perKib * c.kib / f + (f > 1 ? 2.2 + 1.5e-4 * f * umin(t.rows, keptOnly ? a.keptRows : (uint32_t)rows) * t.cols : 0.0);

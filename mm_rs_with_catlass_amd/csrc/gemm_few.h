@@ -113,7 +113,7 @@ __device__ __forceinline__ void sum_in_order(const GemmArgs &args, uint32_t task
 // tile; rowOf(i): row i of it; tileOf(v): the row tile that has row v.
 template <uint32_t DT, int BN, int NT, int UN, typename RowOf, typename TileOf>
 __device__ __forceinline__ void task_sums(const GemmArgs &args, void *rowSums, const uint32_t *dst, const v4i (&cur)[UN], uint32_t tid, bool colOk, uint32_t rt, uint32_t col0,
-                                          uint32_t rowsValid, uint32_t slices, RowOf rowOf, TileOf tileOf)
+                                          uint32_t rowsValid, RowOf rowOf, TileOf tileOf)
 {
     constexpr bool I8 = DT == DT_I8;
     using Sum = typename std::conditional<I8, long long, double>::type;
@@ -151,7 +151,7 @@ __device__ __forceinline__ void task_sums(const GemmArgs &args, void *rowSums, c
     const uint32_t colBegin = col0 / sp.n0 * sp.n0, first = tileOf(begin), colTiles = ceil_div(umin(sp.n0, args.N - colBegin), (uint32_t)BN);
     const uint32_t parts = (tileOf(end - 1u) - first + 1u) * colTiles;
     const Sum mine = (sum[0] + sum[1]) + (sum[2] + sum[3]);
-    if constexpr (I8) sum_finish(args, sum_add(args, e & FX_INDEX, slices * parts, mine));
+    if constexpr (I8) sum_finish(args, sum_add(args, e & FX_INDEX, parts, mine));
     else sum_in_order(args, e & FX_INDEX, parts, (rt - first) * colTiles + (col0 - colBegin) / BN, mine);
 }
 
@@ -469,28 +469,34 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
                 for (int e = 0; e < 4; ++e) cur[j][e] = f2i(__fadd_rn(i2f(cur[j][e]), i2f(t[e])));
             }
         }
-        if constexpr (I8) cur[j] += bv;
+        if constexpr (I8 && !SL) cur[j] += bv;
         d[j] = dst[row];
     }
-    auto add_task_sums = [&]() {   // (whole numbers: every slice's part; floats: of the sums they end up as)
-        task_sums<DT, BN, 256, UN>(args, dst + BM + 12, dst, cur, tid, colOk, rt, col0, rowsValid, I8 ? slices : 1u, [&](uint32_t i) { return row0 + i; },
-                                   [](uint32_t v) { return v / BM; });
+    auto add_task_sums = [&]() {   // (of the sums the rows end up as: where k is sliced, the last slice's)
+        task_sums<DT, BN, 256, UN>(args, dst + BM + 12, dst, cur, tid, colOk, rt, col0, rowsValid, [&](uint32_t i) { return row0 + i; }, [](uint32_t v) { return v / BM; });
     };
     MetSum blockSum;
     const bool sums = I8 && (flags & GF_ROW_MASK) && args.checksum;
     if constexpr (I8) {
         if (sums) {
+            // (a slice's own sum and the bias may be past 32 bits where the whole sum and the bias are not: the bias counts in 64)
             long long sum = 0;
+            const long long bias = SL ? ((long long)bv.x + bv.y) + ((long long)bv.z + bv.w) : 0ll;
 #pragma unroll
             for (int j = 0; j < UN; ++j)
-                if (colOk && d[j] != FX_KEPT && urow + j * (256 / LPR) < rowsValid) sum += ((long long)cur[j].x + cur[j].y) + ((long long)cur[j].z + cur[j].w);
+                if (colOk && d[j] != FX_KEPT && urow + j * (256 / LPR) < rowsValid) sum += ((long long)cur[j].x + cur[j].y) + ((long long)cur[j].z + cur[j].w) + bias;
             sum = wave_sum64(sum);
             long long *red = (long long *)(dst + BM);
             if (lane == 63) red[w] = sum;
             __syncthreads();
             if (tid == 0) blockSum = block_add<BM, BN>(args, row0, col0, rows, slices, (red[0] + red[1]) + (red[2] + red[3]));
         }
-        if (taskSums) add_task_sums();
+        if constexpr (SL) {
+#pragma unroll
+            for (int j = 0; j < UN; ++j) cur[j] += bv;   // (slice 0's; as 32-bit words the slices add up to the right ones)
+        } else {
+            if (taskSums) add_task_sums();
+        }
     }
     // ---- k slices: the last to arrive has the sum of all, in slice order
     if constexpr (SL) {
@@ -546,7 +552,7 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
             return;
         }
     }
-    if constexpr (!I8) {
+    if constexpr (!I8 || SL) {
         if (taskSums) add_task_sums();
     }
     if (!colOk) return;

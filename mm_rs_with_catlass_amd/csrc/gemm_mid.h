@@ -390,7 +390,7 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
             while (first_other(t + 1u) <= x) ++t;
             return t;
         };
-        task_sums<DT, BN, NT, UN>(args, rowScale + BM + 16, dst, cur, (uint32_t)t2, colOk, rt, col0, rowsValid, 1u, rowOf, tile_of);
+        task_sums<DT, BN, NT, UN>(args, rowScale + BM + 16, dst, cur, (uint32_t)t2, colOk, rt, col0, rowsValid, rowOf, tile_of);
     }
     if (!colOk) return;
     if (args.accDump) {

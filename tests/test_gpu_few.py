@@ -511,3 +511,47 @@ def test_float_task_sums(case, dtype):
     for p in peers:
         y = y + p
     assert torch.equal(out, y.to(dtype))
+
+
+# (rows, N, K, P, first kept row or rank, kept rows or 0: a reduce-scatter's, weights as [n,k]): sums of W8A8 tiles in k slices under a bias at either end of
+# its range: the whole accumulators are the bias itself, a slice's own sum and the bias are past the end
+@pytest.mark.parametrize("case", [(64, 512, 8192, 8, 20, 8, True), (70, 384, 8192, 2, 69, 1, False), (16, 768, 15776, 2, 0, 0, False), (40, 512, 8192, 4, 3, 0, True)])
+def test_sums_of_k_slices_with_a_bias_at_the_end_of_its_range(case):
+    _need_gpu()
+    M, N, K, P, at, kr, tb = case
+    g = torch.Generator(device="cuda:0").manual_seed(M + N)
+    u, v = (torch.randint(90, 128, shape, dtype=torch.int8, device="cuda:0", generator=g) for shape in ((M, K // 2), (K // 2, N)))
+    up = torch.arange(N, device="cuda:0") % 3 != 0   # (more of one sign: what the two kinds of columns are off by does not cancel)
+    v = torch.where(up, v, -v)
+    x1, x2 = torch.cat([u, u], 1), torch.cat([v, -v], 0)
+    b = torch.randint(0, 1000, (N,), dtype=torch.int32, device="cuda:0", generator=g)
+    b = torch.where(up, 2 ** 31 - 1 - b, -2 ** 31 + b)
+    s1, s2 = (torch.empty(c, device="cuda:0").uniform_(0.001, 0.02, generator=g) for c in (M, N))
+    acc = b.to(torch.int64).expand(M, N)
+    rows, first = (kr, at) if kr else (M // P, at * (M // P))
+    peers = [torch.randn((rows, N), device="cuda:0", generator=g) for _ in range(P - 1)]
+    y = (b.float() * s2) * s1[first:first + rows, None]
+    for p in peers:
+        y = y + p
+    x2d = x2.T.contiguous() if tb else x2
+    if kr:
+        need = ops.splitk_plan(M, K, N, P, at, kr)[0]
+        others = acc.clone()
+        others[first:first + rows] = 0
+        want = torch.stack([others[r:r + 128, c:c + 128].sum() for r in range(0, M, 128) for c in range(0, N, 128)]).cpu()
+        run = lambda cs, ws: ops.quant_matmul_splitk(x1, x2d, s1, s2, b, peers, P, at, kr, workspace=ws, checksum=cs, trans_b=tb)
+    else:
+        t, d = one_round(L.QUANT_MATMUL_REDUCE_SCATTER, M, K, N, P, at)
+        need = ops.kslice_plan(L.QUANT_MATMUL_REDUCE_SCATTER, L.INT8, M, K, N, at, P, tiling=t)[0]
+        tasks = list(tasks_of(L.QUANT_MATMUL_REDUCE_SCATTER, t, d))
+        want = torch.full((len(tasks),), 77, dtype=torch.int64)
+        for task, r, row, col, _ in tasks:
+            if r != at:
+                want[task] = acc[row:min(row + 64, (r + 1) * rows), col:min(col + 256, N)].sum()
+        run = lambda cs, ws: ops.quant_matmul_reduce_scatter(x1, x2d, s1, s2, b, peers, at, P, tiling=t, trans_b=tb, checksum=cs, workspace=ws)
+    ws = sliced_workspace(need)
+    cs = torch.full((want.numel(),), 77, dtype=torch.int64, device="cuda:0")
+    out = run(cs, ws)
+    torch.cuda.synchronize()
+    check_workspace(ws, need)
+    assert torch.equal(out, y.bfloat16()) and torch.equal(cs.cpu(), want)
