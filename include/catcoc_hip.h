@@ -408,15 +408,17 @@ CATCOC_API uint32_t catcoc_task_tiles(int commType, const CocTilingParams *tilin
  * long ones).  A bijection on [0, task count);
  * 0xffffffff for wg out of range or rejected arguments.  (A reduce-scatter launch that splits its kept tiles, see
  * CATCOC_FLAG_KEPT_SPLIT, runs each as two 64-row workgroups placed first in the same order; this function still
- * describes the order by tile.  Launches in flexible mode -- ragged ones, and aligned ones of few tiles -- cut the problem into
- * tiles of their own, in an order of their own: for them this is the schedule's order and says nothing about workgroups, here and
- * in catcoc_launch_tile.)  No counterpart in the reference, where AI core i
+ * describes the order by tile.  Launches on flexible, small or mixed tiles -- ragged ones, aligned ones of few tiles or of a number
+ * that does not come out even -- cut the problem into tiles of their own, in an order of their own: for them this is the
+ * schedule's order and says nothing about workgroups, here and in catcoc_launch_tile.  desc.flags with
+ * CATCOC_FLAG_LINEAR_ORDER, or m0 in the tiling, keeps a launch of whole tiles off them.)  No counterpart in the reference, where AI core i
  * simply runs tasks i, i + BLOCK_NUM, ... (quant_matmul_reduce_scatter.hpp:166-170). */
 CATCOC_API uint32_t catcoc_launch_task(int commType, const CocTilingParams *tiling, const CatcocSymmetricDesc *desc,
                                        uint32_t wg);
 /* How many kept tiles a launch of this shape would run as two 64-row workgroups each (see CATCOC_FLAG_KEPT_SPLIT;
- * 0 = none, flexible tiles included: the launch then has one workgroup per task on the aligned kernels, else that many
- * workgroups more; pass the descriptor the launch will use, desc.checksum and all).  For tools that size or
+ * 0 = none, flexible, small and mixed tiles included: the launch then has one workgroup per task on the aligned kernels, else
+ * that many workgroups more; pass the descriptor the launch will use, desc.flags, checksum and workspace too: a launch
+ * that neither stores nor sums the other ranks' tiles runs aligned tiles where one that does runs smaller ones).  For tools that size or
  * reason about the grid.  No counterpart in the reference. */
 CATCOC_API uint32_t catcoc_kept_split_tiles(int commType, int dataType, const CocTilingParams *tiling,
                                             const CatcocSymmetricDesc *desc, uint32_t transA, uint32_t transB);

@@ -765,13 +765,23 @@ int check_ptr_align(const Plan &p, const void *a, const void *b)
     return okA && okB;
 }
 
-bool launched_small(const Plan &p, bool dma, bool flex, void *stream)
+// The small tile that a planned launch runs, if any (g: its arguments); dma, flex: what it would run else.
+SmallTile planned_small(const Plan &p, bool dma, bool flex, GemmArgs &g)
 {
-    if (!p.maySmall) return false;
-    GemmArgs g = p.args;
+    if (!p.maySmall) return {0, 0};
+    g = p.args;
+    // Whole tiles of other ranks that are neither stored nor summed: no operator's use, but what tools ask about and time (catcoc_kept_split_tiles,
+    // catcoc_launch_tile); these launches run the tiles and the order that the queries know.
+    if ((dma || p.preferFlex) && (g.flags & GF_OUTBOUND_STORE) == 0 && g.checksum == nullptr && g.sched.op == OP_REDUCE_SCATTER && splittable_kept_tiles(g) != 0) return {0, 0};
     g.skCount = p.counters;
     const uint32_t es = elem_size(p.dtype);
-    const SmallTile t = small_tile(g, es, dma ? kAlignedShare * aligned_us(p.args, es) : flex ? kOtherShare * flex_us(p.args, es, p.flexBlocks) : 1e30, p.room);
+    return small_tile(g, es, dma ? kAlignedShare * aligned_us(p.args, es) : flex ? kOtherShare * flex_us(p.args, es, p.flexBlocks) : 1e30, p.room);
+}
+
+bool launched_small(const Plan &p, bool dma, bool flex, void *stream)
+{
+    GemmArgs g;
+    const SmallTile t = planned_small(p, dma, flex, g);
     if (t.rows) launched(launch_small(p.dtype, g, t, stream));
     return t.rows != 0;
 }
@@ -1673,32 +1683,30 @@ uint32_t catcoc_launch_task(int commType, const CocTilingParams *tiling, const C
     return launch_task(s, wg, (p.args.flags & GF_LINEAR_ORDER) != 0, p.args.keptRank);
 }
 
+// The plan of a launch that may run kept tiles as halves: on the aligned 128-row kernel, on no flexible or small tiles.
+static bool plan_halves(int commType, int dataType, const CocTilingParams *tiling, const CatcocSymmetricDesc *desc, uint32_t transA, uint32_t transB, Plan &p)
+{
+    if (desc == nullptr || tiling == nullptr) { fail(E_NULL, "tiling and desc must be non-NULL"); return false; }
+    CatcocSymmetricDesc d = *desc;
+    for (int i = 0; i < CATCOC_MAX_RANKS; ++i) if (!d.peers[i]) d.peers[i] = (const void *)16;
+    if (make_plan(commType, dataType, tiling, &d, transA, transB, p)) return false;
+    ok();
+    GemmArgs g;
+    return p.dma && !p.preferFlex && p.args.sched.m0 == 128 && planned_small(p, true, false, g).rows == 0;
+}
+
 uint32_t catcoc_kept_split_tiles(int commType, int dataType, const CocTilingParams *tiling, const CatcocSymmetricDesc *desc,
                                  uint32_t transA, uint32_t transB)
 {
     Plan p;
-    CatcocSymmetricDesc d;
-    if (desc == nullptr || tiling == nullptr) { fail(E_NULL, "tiling and desc must be non-NULL"); return 0; }
-    d = *desc;
-    for (int i = 0; i < CATCOC_MAX_RANKS; ++i) if (!d.peers[i]) d.peers[i] = (const void *)16;
-    if (make_plan(commType, dataType, tiling, &d, transA, transB, p)) return 0;
-    ok();
-    if (!p.dma || p.preferFlex || p.args.sched.m0 != 128) return 0;   // (flexible tiles are never split)
-    return 8u * split_kept_tiles(p.args, p.args.K * elem_size(p.dtype) / 64u);
+    return plan_halves(commType, dataType, tiling, desc, transA, transB, p) ? 8u * split_kept_tiles(p.args, p.args.K * elem_size(p.dtype) / 64u) : 0u;
 }
 
 uint32_t catcoc_tail_split_tiles(int commType, int dataType, const CocTilingParams *tiling, const CatcocSymmetricDesc *desc,
                                  uint32_t transA, uint32_t transB)
 {
     Plan p;
-    CatcocSymmetricDesc d;
-    if (desc == nullptr || tiling == nullptr) { fail(E_NULL, "tiling and desc must be non-NULL"); return 0; }
-    d = *desc;
-    for (int i = 0; i < CATCOC_MAX_RANKS; ++i) if (!d.peers[i]) d.peers[i] = (const void *)16;
-    if (make_plan(commType, dataType, tiling, &d, transA, transB, p)) return 0;
-    ok();
-    if (!p.dma || p.preferFlex || p.args.sched.m0 != 128) return 0;   // (flexible tiles are never split)
-    return 8u * split_tail_tiles(p.args, split_kept_tiles(p.args, p.args.K * elem_size(p.dtype) / 64u));
+    return plan_halves(commType, dataType, tiling, desc, transA, transB, p) ? 8u * split_tail_tiles(p.args, split_kept_tiles(p.args, p.args.K * elem_size(p.dtype) / 64u)) : 0u;
 }
 
 uint32_t catcoc_workgroup_task(uint32_t wg, uint32_t tasks, uint32_t flags)

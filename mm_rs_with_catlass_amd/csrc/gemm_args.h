@@ -84,6 +84,16 @@ struct GemmArgs {
 // Workgroups (before k slicing) a launch starts.
 inline uint32_t launch_positions(const GemmArgs &a) { return a.taskCount ? a.taskCount : a.sched.coreLoops; }
 
+// Kept tiles per XCD that a launch could run as two workgroups each, whatever the choice.
+inline uint32_t splittable_kept_tiles(const GemmArgs &a)
+{
+    const SchedParams &s = a.sched;
+    if (s.m0 != 128 || a.splitK > 1 || a.taskBase != 0 || a.taskCount != 0 || (a.flags & (GF_LINEAR_ORDER | GF_ROW_MASK | GF_RAGGED)) ||
+        a.transA || a.nPeers == 0 || a.keptBegin != a.keptRank * s.mRank || a.keptRows != s.mRank)
+        return 0;
+    return xcd_uniform_kept(s, a.keptRank);
+}
+
 // Kept tiles per XCD when a launch qualifies for gemm_dma_split_kept_kernel, else 0: a whole reduce-scatter launch in the
 // XCD-block order, A as [m,k], the kept rows exactly the kept rank's block with peers to stream, and by default either
 // fewer tiles than CUs or at most one round of workgroups (512 tiles) with at most 80 k steps per tile.  Measured with
@@ -95,12 +105,9 @@ inline uint32_t launch_positions(const GemmArgs &a) { return a.taskCount ? a.tas
 inline uint32_t split_kept_tiles(const GemmArgs &a, uint32_t kSteps)
 {
     const SchedParams &s = a.sched;
-    if (s.m0 != 128 || a.splitK > 1 || a.taskBase != 0 || a.taskCount != 0 || (a.flags & (GF_LINEAR_ORDER | GF_ROW_MASK | GF_RAGGED)) ||
-        a.transA || a.nPeers == 0 || a.keptBegin != a.keptRank * s.mRank || a.keptRows != s.mRank)
-        return 0;
     if (a.flags & GF_KEPT_WHOLE) return 0;
     if (!(a.flags & GF_KEPT_SPLIT) && !(s.coreLoops < 256u || (s.coreLoops <= 512u && kSteps <= 80u))) return 0;
-    return xcd_uniform_kept(s, a.keptRank);
+    return splittable_kept_tiles(a);
 }
 
 // Tiles per XCD at the END of the launch order that a launch with split kept tiles also runs as two 64-row workgroups: the

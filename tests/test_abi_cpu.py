@@ -624,6 +624,26 @@ def test_kept_split_queries_of_launches_on_flexible_tiles(so):
         assert split(comm, dt, 768, 2 * k, 4096, 2) == 48 and split(comm, dt, 768, 2 * k, 4096, 2, tb=0) == 0 and split(comm, dt, 768, k, 4096, 2, tb=0) == 48
 
 
+def test_kept_split_queries_of_launches_on_small_and_mixed_tiles(so):
+    # launches whose other ranks' tiles are stored, or summed with a workspace, run small tiles or mixed ones, none of them split, where those are
+    # faster; with tiles the caller chose they do not
+    from mm_rs_with_catlass_amd import ops
+
+    def split(comm, dt, m, k, n, p, tb, store=True, **tiling):
+        t = ops.default_tiling(m, k, n, p, **dict(dict(m0=0, n0=0, k0=0), **tiling))
+        d = L.make_desc(3, p, [16] * (p - 1), flags=L.OUTBOUND_STORE if store else 0, outbound=4096 if store else None, outbound_bytes=1 << 40,
+                        checksum=None if store else 4096)
+        d.workspace, d.workspaceBytes = None if store else 4096, 0 if store else 65536
+        r = [q(comm, dt, C.byref(t), C.byref(d), 0, tb) for q in (so.catcoc_kept_split_tiles, so.catcoc_tail_split_tiles)]
+        L.check()
+        return r
+    Q, RS = L.QUANT_MATMUL_REDUCE_SCATTER, L.MATMUL_REDUCE_SCATTER
+    for comm, dt in ((Q, L.INT8), (RS, L.FP16), (RS, L.BF16)):
+        assert split(comm, dt, 2048, 1792, 2048, 8, 0) == [0, 0] and split(comm, dt, 2048, 1792, 2048, 8, 0, m0=128, n0=256) == [16, 0]
+    assert split(Q, L.INT8, 4096, 1792, 4096, 8, 1) == [0, 0]                     # (256x256 and 128x128 tiles)
+    assert split(Q, L.INT8, 4096, 1792, 4096, 8, 1, store=False) == [64, 64] == split(Q, L.INT8, 4096, 1792, 4096, 8, 0, m0=128, n0=256)
+
+
 def test_descriptor_takes_what_its_fields_take(so):
     # plain addresses are packed in one go; ctypes objects and numbers outside a field's range as ctypes takes them
     want = bytes(L.make_desc(3, 4, [16, 32, 48], peer_ld=8, outbound=64, outbound_bytes=128, checksum=256, acc_dump=512, flags=5))
