@@ -102,7 +102,9 @@ typedef void (*CatcocKernelFuncPtr)(void *stream, uint64_t fftsAddr, uint8_t *a,
 /* Reduce-scatter launches of one round of workgroups (at most 512 tiles of 128x256 with at most 80 k steps of 64 bytes,
  * or fewer than 256 tiles) run every kept tile as two 64-row workgroups, which halves the chain of peer partials a
  * workgroup adds; the library decides by those two numbers.  KEPT_WHOLE never splits, KEPT_SPLIT splits whenever the launch allows it (whole
- * tiles, A as [m,k], XCD-aware order): tuning knobs like the tiling's, results are bit-identical either way. */
+ * tiles, A as [m,k], XCD-aware order): tuning knobs like the tiling's, results are bit-identical either way and without a flag.  For
+ * that the flags leave a launch that runs small or mixed tiles, or k slices, where it is: nothing is split there.  m0 = 128 in the
+ * tiling asks for the aligned kernels, whose float sums are added in another order than small tiles'. */
 #define CATCOC_FLAG_KEPT_WHOLE 0x10u
 #define CATCOC_FLAG_KEPT_SPLIT 0x20u
 /* A launch with split kept tiles has more workgroups than the GPU has slots for; the tiles that wait for a slot (they get the

@@ -707,17 +707,16 @@ int make_plan(int commType, int dataType, const CocTilingParams *t, const Catcoc
     // 512x8192x8192 in two k slices 93.0 / 102.5 against 111 / 130).  (Checksums stay: a 128-row task would need two workgroups.)
     plan.flexBlocks = 0;
     plan.preferFlex = false;
-    plan.maySmall = t->m0 == 0 && d->splitK == 0 && (d->flags & (CATCOC_FLAG_LINEAR_ORDER | CATCOC_FLAG_KEPT_WHOLE | CATCOC_FLAG_KEPT_SPLIT)) == 0;
+    plan.maySmall = t->m0 == 0 && d->splitK == 0 && (d->flags & CATCOC_FLAG_LINEAR_ORDER) == 0;
     const uint64_t rowsAll = op == OP_ALLGATHER ? (uint64_t)t->m * P : t->m;
     const uint64_t tiles64 = (rowsAll + 63) / 64 * ceil_div(t->n, 256u);
     const bool fewTiles = tiles64 <= 128u || (tiles64 <= 256u && (uint64_t)t->k * es <= 4096u);
-    const uint32_t tuning = CATCOC_FLAG_LINEAR_ORDER | CATCOC_FLAG_KEPT_WHOLE | CATCOC_FLAG_KEPT_SPLIT;
     if (!plan.dma) {
         const FlexSlices c = flex_choose(a, es, t->m0, d->splitK);
         plan.kSlices = c.slices;
         plan.kSliceBytes = c.bytes;
         plan.flexBlocks = flex_use(a, es, t->m0, c, d->workspace, d->workspaceBytes);
-    } else if (m0 == 128 && t->m0 == 0 && (d->splitK == 0 || (plan.edge && d->splitK > 1)) && (d->flags & tuning) == 0 && fewTiles && !transA &&
+    } else if (m0 == 128 && t->m0 == 0 && (d->splitK == 0 || (plan.edge && d->splitK > 1)) && (d->flags & CATCOC_FLAG_LINEAR_ORDER) == 0 && fewTiles && !transA &&
                !(op == OP_REDUCE_SCATTER && P > 1 && a.checksum != nullptr)) {
         // What a workspace takes is said for the aligned kernel, and this one uses the slices that fit into that, unless it would
         // take four or more: all-reduce of 257x14336x512, bf16, seven peers, in 64 KiB of workspace (no slices) / in what its slices
@@ -737,10 +736,14 @@ int make_plan(int commType, int dataType, const CocTilingParams *t, const Catcoc
         // 11.7 / 13.5 (2 KiB: 512x2048x4096 17.3 / 17.3, 16 bits 512x1024x4096 16.0 / 15.2); more than 128 tiles, W8A8 2048x2048x2048 of
         // eight ranks 25.9 / 27.8, as [n,k] 26.1 / 29.5, of four 19.5 / 22.8, 20.1 / 24.3, k = 4096 29.9 / 32.0, 35.2 / 36.2, of eight
         // 35.9 / 37.2, 41.6 / 41.5; with one peer and B as [k,n] the larger k is the flexible tiles' (768x4096x4096 28.9 / 26.7).
+        // (The caller's choice between halves and whole tiles does not enter: keep_aligned.)
         const uint64_t kBytes = (uint64_t)t->k * es;
+        const uint32_t flags = a.flags;
+        a.flags &= ~(uint32_t)(GF_KEPT_WHOLE | GF_KEPT_SPLIT);
         if (plan.preferFlex && op == OP_REDUCE_SCATTER && a.fx.slices <= 1 && a.fx.late == 0 &&
             (kBytes <= 1024 || (tiles64 > 128u && (kBytes <= 2048 || nPeers > 1 || transB))) && split_kept_tiles(a, (uint32_t)(kBytes / 64)) != 0)
             plan.preferFlex = false;
+        a.flags = flags;
         // (four slices or more of ragged rows or columns with B as [k,n]: a caller's count of them and the library's own give the same bits)
         if (plan.preferFlex && plan.edge && !transB && a.fx.slices >= 4) plan.maySmall = false;
     }
@@ -778,6 +781,10 @@ SmallTile planned_small(const Plan &p, bool dma, bool flex, GemmArgs &g)
     return small_tile(g, es, dma ? kAlignedShare * aligned_us(p.args, es) : flex ? kOtherShare * flex_us(p.args, es, p.flexBlocks) : 1e30, p.room);
 }
 
+// CATCOC_FLAG_KEPT_WHOLE and CATCOC_FLAG_KEPT_SPLIT change no bit of a result: sums of floats in another order would.  So they do not enter the
+// choice of small tiles or of k slices, and only move a launch of whole flexible tiles, which add in the aligned kernel's order, there.
+bool keep_aligned(const GemmArgs &a) { return (a.flags & (GF_KEPT_WHOLE | GF_KEPT_SPLIT)) != 0 && a.fx.slices <= 1 && splittable_kept_tiles(a) != 0; }
+
 bool launched_small(const Plan &p, bool dma, bool flex, void *stream)
 {
     GemmArgs g;
@@ -799,12 +806,14 @@ void launch_float(int commType, int dataType, void *stream, uint8_t *a, uint8_t 
     p.args.d = c;
     if (!check_ptr_align(p, a, b)) p.variant = 0;
     const bool preferFlex = p.preferFlex && flex_ptrs_ok(p.args);
-    const bool dma = !preferFlex && p.dma && p.variant != 0 && (uintptr_t)b % 16 == 0 && (p.args.ldb * 2) % 16 == 0 && (uintptr_t)c % 16 == 0;
+    const bool aligned = p.dma && p.variant != 0 && (uintptr_t)b % 16 == 0 && (p.args.ldb * 2) % 16 == 0 && (uintptr_t)c % 16 == 0;
+    bool dma = !preferFlex && aligned;
     if (!dma) p.args.splitK = 0;   // the other kernels run every tile whole
     if (!dma && p.variant == 4) { fail(E_TILING, "m0 = 256 needs full tiles and 16-byte aligned row-major operands"); return; }
     if (!dma && p.args.transA) p.variant = 0;
     const bool flex = !dma && p.flexBlocks != 0 && flex_ptrs_ok(p.args);
     if (launched_small(p, dma, flex, stream)) return;
+    if (aligned && keep_aligned(p.args)) dma = true;
     const int e = dma ? (p.dtype == DT_F16 ? launch_gemm_dma_f16(p.args, stream) : launch_gemm_dma_bf16(p.args, stream))
                   : flex ? launch_flex(p.dtype, p.args, p.flexBlocks, stream)
                       : launch_gemm(p.dtype, p.args, p.variant, p.edge, stream);
@@ -1130,13 +1139,15 @@ void launch_quant(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_x1, uin
         (c_accum && (uintptr_t)c_accum % 16 != 0) || (uintptr_t)d_out % 8 != 0)
         p.variant = 0;
     const bool preferFlex = p.preferFlex && flex_ptrs_ok(p.args);
-    bool dma = !preferFlex && p.dma && p.variant != 0 && (uintptr_t)x2 % 16 == 0 && p.args.ldb % 16 == 0 && (uintptr_t)d_out % 16 == 0;
-    for (uint32_t s = 0; s < p.args.nPeers && dma; ++s) dma = (uintptr_t)p.args.peers[s] % 16 == 0;
+    bool aligned = p.dma && p.variant != 0 && (uintptr_t)x2 % 16 == 0 && p.args.ldb % 16 == 0 && (uintptr_t)d_out % 16 == 0;
+    for (uint32_t s = 0; s < p.args.nPeers && aligned; ++s) aligned = (uintptr_t)p.args.peers[s] % 16 == 0;
+    bool dma = !preferFlex && aligned;
     if (!dma && p.variant == 4) { fail(E_TILING, "m0 = 256 needs full tiles, 16-byte aligned row-major operands and fp32 peers"); return; }
     if (!dma) p.args.splitK = 0;   // the other kernels run every tile whole
     if (!dma && p.args.transA) p.variant = 0;
     const bool flex = !dma && p.flexBlocks != 0 && flex_ptrs_ok(p.args);
     if (launched_small(p, dma, flex, stream)) return;
+    if (aligned && keep_aligned(p.args)) dma = true;
     const int e = dma ? launch_gemm_dma_i8(p.args, stream) : flex ? launch_flex(p.dtype, p.args, p.flexBlocks, stream) : launch_gemm(p.dtype, p.args, p.variant, p.edge, stream);
     if (e) { fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)e)); return; }
     ok();
@@ -1692,7 +1703,9 @@ static bool plan_halves(int commType, int dataType, const CocTilingParams *tilin
     if (make_plan(commType, dataType, tiling, &d, transA, transB, p)) return false;
     ok();
     GemmArgs g;
-    return p.dma && !p.preferFlex && p.args.sched.m0 == 128 && planned_small(p, true, false, g).rows == 0;
+    if (!p.dma || p.args.sched.m0 != 128) return false;
+    if (p.preferFlex) p.args.splitK = 0;   // (as the launchers)
+    return planned_small(p, !p.preferFlex, p.preferFlex, g).rows == 0 && (!p.preferFlex || keep_aligned(p.args));
 }
 
 uint32_t catcoc_kept_split_tiles(int commType, int dataType, const CocTilingParams *tiling, const CatcocSymmetricDesc *desc,

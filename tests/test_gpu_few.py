@@ -555,3 +555,34 @@ def test_sums_of_k_slices_with_a_bias_at_the_end_of_its_range(case):
     torch.cuda.synchronize()
     check_workspace(ws, need)
     assert torch.equal(out, y.bfloat16()) and torch.equal(cs.cpu(), want)
+
+
+# (rows, N, K, P, rank, weights as [n,k], workspace): what a caller says about halves of kept tiles changes no bit, whichever tiles run: 128x128, 32x64 and mixed
+# tiles, small ones in k slices, whole flexible tiles or aligned ones instead, flexible ones in k slices
+@pytest.mark.parametrize("kind", [torch.float16, torch.bfloat16, torch.int8])
+@pytest.mark.parametrize("case", [(2048, 2048, 1792, 8, 3, False, False), (1024, 512, 512, 8, 7, True, False), (4096, 4096, 1792, 8, 2, True, False), (512, 512, 6144, 4, 2, False, True),
+                                  (512, 4096, 1024, 4, 1, True, False), (1024, 1024, 8192, 2, 0, True, True)])
+def test_halves_of_kept_tiles_change_no_bit(case, kind):
+    _need_gpu()
+    M, N, K, P, rank, tb, slices = case
+    g = torch.Generator(device="cuda:0").manual_seed(M + K)
+    quant = kind == torch.int8
+    if quant:
+        a, b = (torch.randint(-127, 128, s, dtype=torch.int8, device="cuda:0", generator=g) for s in ((M, K), (N, K) if tb else (K, N)))
+    else:
+        a, b = torch.randn((M, K), device="cuda:0", generator=g).to(kind), (torch.randn((N, K) if tb else (K, N), device="cuda:0", generator=g) * 0.05).to(kind)
+    s1, s2 = (torch.empty(c, device="cuda:0").uniform_(0.001, 0.02, generator=g) for c in (M, N))
+    peers = [torch.randn((M // P, N), device="cuda:0", generator=g) for _ in range(P - 1)]
+    comm = L.QUANT_MATMUL_REDUCE_SCATTER if quant else L.MATMUL_REDUCE_SCATTER
+    t, d = one_round(comm, M, K, N, P, rank)
+    size = L.load().catcoc_get_workspace_size(comm, L.INT8 if quant else L.FP16, C.byref(t), C.byref(d)) // 4
+    need = max(ops.kslice_plan(comm, kind, M, K, N, rank, P, tiling=t)[0], 65536)
+    results = []
+    for choice in (None, False, True, "kept-only"):
+        ob, dump = torch.full((size,), 3.0, device="cuda:0"), torch.zeros((M, N), dtype=torch.int32 if quant else torch.float32, device="cuda:0")
+        kw = dict(tiling=t, trans_b=tb, outbound=ob, acc_dump=dump, kept_split=choice, workspace=torch.zeros(need, dtype=torch.uint8, device="cuda:0") if slices else None)
+        out = ops.quant_matmul_reduce_scatter(a, b, s1, s2, None, peers, rank, P, **kw) if quant else ops.matmul_reduce_scatter(a, b, peers, rank, P, **kw)
+        torch.cuda.synchronize()
+        results.append((out, dump, ob))
+    for r in results[1:]:
+        assert all(torch.equal(x, y) for x, y in zip(r, results[0]))
