@@ -586,3 +586,19 @@ def test_halves_of_kept_tiles_change_no_bit(case, kind):
         results.append((out, dump, ob))
     for r in results[1:]:
         assert all(torch.equal(x, y) for x, y in zip(r, results[0]))
+
+
+# (rows, N, K, weights as [n,k], k slices): 32x32, 32x64, 64x64 tiles, whole and in k slices, 64x128 and 128x128 ones
+@pytest.mark.parametrize("case", [(100, 2048, 1024, True, False), (512, 1024, 1024, False, False), (1000, 512, 2052, True, False), (96, 512, 8192, True, True), (300, 1032, 6148, True, True),
+                                  (650, 3332, 2310, True, False)])
+def test_equal_rows_have_equal_sums_wherever_they_lie(case):
+    _need_gpu()
+    M, N, K, tb, slices = case
+    g = torch.Generator(device="cuda:0").manual_seed(M)
+    A = torch.randn((1, K), device="cuda:0", generator=g).bfloat16().expand(M, K).contiguous()
+    B = torch.randn((N, K) if tb else (K, N), device="cuda:0", generator=g).bfloat16()
+    need = ops.kslice_plan(L.MATMUL_ALLREDUCE, torch.bfloat16, M, K, N, 0, 2)[0]
+    dump = torch.zeros((M, N), device="cuda:0")
+    ops.matmul_allreduce(A, B, [torch.zeros((M, N), device="cuda:0")], 0, 2, trans_b=tb, acc_dump=dump, workspace=torch.zeros(need, dtype=torch.uint8, device="cuda:0") if slices else None)
+    torch.cuda.synchronize()
+    assert torch.equal(dump, dump[:1].expand(M, N))
