@@ -435,6 +435,24 @@ CATCOC_API uint32_t catcoc_tail_split_tiles(int commType, int dataType, const Co
  * tests compare that route with catcoc_launch_task + catcoc_task_tile).  Returns 0 past the end of the launch. */
 CATCOC_API int catcoc_launch_tile(int commType, const CocTilingParams *tiling, const CatcocSymmetricDesc *desc, uint32_t wg,
                                   uint32_t *task, uint32_t *targetRank, uint32_t *row, uint32_t *col, uint32_t *wsRow);
+/* What the GEMM launch of the calling thread's last accepted call ran (a call of several rounds: the last round), for tests that are
+ * about one kernel and for tools.  No counterpart in the reference. */
+enum {
+    CATCOC_KERNEL_NONE = 0,
+    CATCOC_KERNEL_GENERAL = 1,   /* bounds-checked kernels */
+    CATCOC_KERNEL_ALIGNED = 2,   /* 128x256 and 256x256 tiles of whole or ragged problems */
+    CATCOC_KERNEL_FLEXIBLE = 3,  /* 64x256 and 128x256 tiles over any rows */
+    CATCOC_KERNEL_SMALL = 4,     /* 32x32 to 128x128 tiles; 256x256: mixed with 128x128 ones */
+    CATCOC_KERNEL_STREAMING = 5  /* explicit kept rows: 128x128 tiles in k slices, 32 columns over the whole k */
+};
+typedef struct CatcocLaunchInfo {
+    uint32_t kernel;             /* CATCOC_KERNEL_* */
+    uint32_t tileRows, tileCols;
+    uint32_t kSlices;            /* 1 = none */
+    uint32_t dealt;              /* small tiles of 128 columns: a reduce-scatter's kept rows are dealt out to all row tiles */
+    uint32_t largeTiles;         /* mixed tiles: how many are 256x256 */
+} CatcocLaunchInfo;
+CATCOC_API void catcoc_last_launch(CatcocLaunchInfo *info);
 /* The task workgroup `wg` of a launch with `tasks` tasks runs (XCD-aware chunking unless
  * CATCOC_FLAG_LINEAR_ORDER); a bijection on [0,tasks). */
 CATCOC_API uint32_t catcoc_workgroup_task(uint32_t wg, uint32_t tasks, uint32_t flags);

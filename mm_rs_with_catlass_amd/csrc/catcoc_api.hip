@@ -33,8 +33,12 @@ int launch_gemm_mid(uint32_t dtype, const GemmArgs &args, int tileRows, void *st
 int launch_gemm_mixed(uint32_t dtype, const GemmArgs &args, void *stream);
 int launch_gemm_few(uint32_t dtype, const GemmArgs &args, int tileRows, int tileCols, void *stream);
 
+// What the calling thread launched last (catcoc_last_launch).
+static thread_local CatcocLaunchInfo g_launch;
+
 static int launch_flex(uint32_t dtype, const GemmArgs &args, int rowBlocks, void *stream)
 {
+    g_launch = {CATCOC_KERNEL_FLEXIBLE, 64u * rowBlocks, 256, args.fx.slices > 1 ? args.fx.slices : 1u, 0, 0};
     switch (dtype) {
         case DT_I8: return launch_gemm_flex_i8(args, rowBlocks, stream);
         case DT_F16: return launch_gemm_flex_f16(args, rowBlocks, stream);
@@ -45,10 +49,22 @@ static int launch_flex(uint32_t dtype, const GemmArgs &args, int rowBlocks, void
 
 static int launch_gemm(uint32_t dtype, const GemmArgs &args, int variant, bool edge, void *stream)
 {
+    g_launch = {CATCOC_KERNEL_GENERAL, args.sched.m0, args.sched.n0, 1, 0, 0};
     switch (dtype) {
         case DT_I8: return launch_gemm_i8(args, variant, edge, stream);
         case DT_F16: return launch_gemm_f16(args, variant, edge, stream);
         case DT_BF16: return launch_gemm_bf16(args, variant, edge, stream);
+        default: return (int)hipErrorInvalidValue;
+    }
+}
+
+static int launch_gemm_dma(uint32_t dtype, const GemmArgs &args, void *stream)
+{
+    g_launch = {CATCOC_KERNEL_ALIGNED, args.sched.m0, args.sched.n0, args.splitK > 1 ? args.splitK : 1u, 0, 0};
+    switch (dtype) {
+        case DT_I8: return launch_gemm_dma_i8(args, stream);
+        case DT_F16: return launch_gemm_dma_f16(args, stream);
+        case DT_BF16: return launch_gemm_dma_bf16(args, stream);
         default: return (int)hipErrorInvalidValue;
     }
 }
@@ -495,6 +511,7 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other, uint64_t room = 0)
 
 int launch_small(uint32_t dtype, const GemmArgs &a, const SmallTile &t, void *stream)
 {
+    g_launch = {CATCOC_KERNEL_SMALL, (uint32_t)t.rows, (uint32_t)t.cols, t.cols < 128 ? a.fx.slices : 1u, a.fx.dealRows != 0, t.cols == 256 ? a.fx.largeTiles : 0u};
     return t.cols == 256 ? launch_gemm_mixed(dtype, a, stream) : t.cols == 128 ? launch_gemm_mid(dtype, a, t.rows, stream) : launch_gemm_few(dtype, a, t.rows, t.cols, stream);
 }
 
@@ -814,7 +831,7 @@ void launch_float(int commType, int dataType, void *stream, uint8_t *a, uint8_t 
     const bool flex = !dma && p.flexBlocks != 0 && flex_ptrs_ok(p.args);
     if (launched_small(p, dma, flex, stream)) return;
     if (aligned && keep_aligned(p.args)) dma = true;
-    const int e = dma ? (p.dtype == DT_F16 ? launch_gemm_dma_f16(p.args, stream) : launch_gemm_dma_bf16(p.args, stream))
+    const int e = dma ? launch_gemm_dma(p.dtype, p.args, stream)
                   : flex ? launch_flex(p.dtype, p.args, p.flexBlocks, stream)
                       : launch_gemm(p.dtype, p.args, p.variant, p.edge, stream);
     if (e) { fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)e)); return; }
@@ -1103,12 +1120,13 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
         for (uint32_t s = 0; s < a.nPeers && aligned; ++s) aligned = (uintptr_t)a.peers[s] % 16 == 0;
         if (!aligned) { fail(E_SHAPE, "128x256 tiles with explicit kept rows need 16-byte aligned scales, bias, peers and output"); return; }
         if (flex()) return;
-        const int el = launch_gemm_dma_i8(a, stream);
+        const int el = launch_gemm_dma(DT_I8, a, stream);
         if (el) { fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)el)); return; }
         ok();
         return;
     }
     if (flex()) return;
+    g_launch = {CATCOC_KERNEL_STREAMING, sp.wholeK ? 32u : 128u, sp.wholeK ? 32u : 128u, sp.f, 0, 0};
     const int e = sp.wholeK ? launch_gemm_decode_nk_i8(a, stream) : launch_gemm_splitk_i8(a, (int)sp.rowBlocks, sp.tiles * sp.f, stream);
     if (e) { fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)e)); return; }
     ok();
@@ -1148,7 +1166,7 @@ void launch_quant(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_x1, uin
     const bool flex = !dma && p.flexBlocks != 0 && flex_ptrs_ok(p.args);
     if (launched_small(p, dma, flex, stream)) return;
     if (aligned && keep_aligned(p.args)) dma = true;
-    const int e = dma ? launch_gemm_dma_i8(p.args, stream) : flex ? launch_flex(p.dtype, p.args, p.flexBlocks, stream) : launch_gemm(p.dtype, p.args, p.variant, p.edge, stream);
+    const int e = dma ? launch_gemm_dma(p.dtype, p.args, stream) : flex ? launch_flex(p.dtype, p.args, p.flexBlocks, stream) : launch_gemm(p.dtype, p.args, p.variant, p.edge, stream);
     if (e) { fail(E_LAUNCH, "kernel launch failed: %s", hipGetErrorString((hipError_t)e)); return; }
     ok();
 }
@@ -1357,8 +1375,7 @@ void launch_pipelined(bool quant, int dataType, void *computeStream, void *commS
         if (he == hipSuccess)
             e = small.rows ? launch_small(p.dtype, gs, small, computeStream)
                 : flexBlocks ? launch_flex(p.dtype, g, flexBlocks, computeStream)
-                : dma ? (p.dtype == DT_I8 ? launch_gemm_dma_i8(g, computeStream)
-                       : p.dtype == DT_F16 ? launch_gemm_dma_f16(g, computeStream) : launch_gemm_dma_bf16(g, computeStream))
+                : dma ? launch_gemm_dma(p.dtype, g, computeStream)
                     : launch_gemm(p.dtype, g, p.variant, p.edge, computeStream);
         if (e == 0 && he == hipSuccess && !oneStream) he = hipEventRecord(ready[r], cs);   // "store finished"
         if (e == 0 && he == hipSuccess && !oneStream) he = hipStreamWaitEvent(ms, ready[r], 0);
@@ -1721,6 +1738,8 @@ uint32_t catcoc_tail_split_tiles(int commType, int dataType, const CocTilingPara
     Plan p;
     return plan_halves(commType, dataType, tiling, desc, transA, transB, p) ? 8u * split_tail_tiles(p.args, split_kept_tiles(p.args, p.args.K * elem_size(p.dtype) / 64u)) : 0u;
 }
+
+void catcoc_last_launch(CatcocLaunchInfo *info) { *info = g_launch; }
 
 uint32_t catcoc_workgroup_task(uint32_t wg, uint32_t tasks, uint32_t flags)
 {

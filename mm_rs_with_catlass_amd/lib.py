@@ -53,6 +53,13 @@ class CatcocSymmetricDesc(C.Structure):
     ]
 
 
+KERNEL_GENERAL, KERNEL_ALIGNED, KERNEL_FLEXIBLE, KERNEL_SMALL, KERNEL_STREAMING = 1, 2, 3, 4, 5
+
+
+class CatcocLaunchInfo(C.Structure):
+    _fields_ = [(n, C.c_uint32) for n in ("kernel", "tileRows", "tileCols", "kSlices", "dealt", "largeTiles")]
+
+
 _DESC = struct.Struct("=11I4x%dQqq7Q" % MAX_RANKS)   # CatcocSymmetricDesc's fields in order
 assert _DESC.size == C.sizeof(CatcocSymmetricDesc)
 _NO_PEERS = (0,) * MAX_RANKS
@@ -77,6 +84,7 @@ EXPORTS = [
     "catcoc_check_comm_interval_allreduce", "catcoc_check_comm_interval_allgather", "catcoc_get_splitk_factor",
     "catcoc_default_tiling", "catcoc_swizzle_block_coord", "catcoc_splitk_block_coord", "catcoc_splitk_actual_k", "catcoc_splitk_launch_task",
     "catcoc_allgather_block_coord", "catcoc_comm_block_idx", "catcoc_task_tile", "catcoc_workgroup_task", "catcoc_launch_task", "catcoc_launch_tile", "catcoc_kept_split_tiles", "catcoc_tail_split_tiles",
+    "catcoc_last_launch",
     "catcoc_device_info", "catcoc_version",
     "catcoc_pipelined_quant_matmul_reduce_scatter", "catcoc_pipelined_matmul_reduce_scatter", "catcoc_reduce_add",
     "catcoc_verify", "catcoc_comm_block_idx_ex", "catcoc_comm_core_loop", "catcoc_task_tiles",
@@ -151,6 +159,8 @@ def load():
     L.catcoc_kept_split_tiles.restype = u32
     L.catcoc_tail_split_tiles.argtypes = [C.c_int, C.c_int, C.POINTER(CocTilingParams), C.POINTER(CatcocSymmetricDesc), u32, u32]
     L.catcoc_tail_split_tiles.restype = u32
+    L.catcoc_last_launch.argtypes = [C.POINTER(CatcocLaunchInfo)]
+    L.catcoc_last_launch.restype = None
     L.catcoc_get_task_count.argtypes = [C.c_int, C.POINTER(CocTilingParams), C.POINTER(CatcocSymmetricDesc)]
     L.catcoc_get_task_count.restype = u32
     L.catcoc_get_tilings.argtypes = [C.POINTER(CocTilingParams), C.c_int, C.c_int, C.c_int, C.POINTER(CocTilingParams), C.c_int]
@@ -216,6 +226,13 @@ def load_host():
         "catcoc_get_kernel", "catcoc_launch_quant_matmul_reduce_scatter", "catcoc_get_task_count", "catcoc_default_tiling", "catcoc_last_status", "catcoc_last_error")),
         CatcocError, CocTilingParams)
     return _host
+
+
+def last_launch():
+    """What this thread's last accepted call ran."""
+    info = CatcocLaunchInfo()
+    load().catcoc_last_launch(C.byref(info))
+    return info
 
 
 def last_error():

@@ -15,20 +15,32 @@ from test_gpu_parity import _need_gpu, _rand16, dev, dev16, host16
 pytestmark = pytest.mark.gpu
 
 
+def ran():
+    """The tiles that the last launch ran, as the cases name them: those of another kernel than this file's with its name, k slices behind a stroke,
+    256x256 ones beside 128x128 ones."""
+    i = L.last_launch()
+    kernel = {L.KERNEL_SMALL: "", L.KERNEL_FLEXIBLE: "flexible ", L.KERNEL_ALIGNED: "aligned "}[i.kernel]
+    assert (i.largeTiles != 0) == (i.kernel == L.KERNEL_SMALL and i.tileRows == 256)
+    return "%s%dx%d%s%s" % (kernel, i.tileRows, i.tileCols, "/%d" % i.kSlices if i.kSlices > 1 else "", " dealt" if i.dealt else "")
+
+
 # (rows, N, K, P, weights as [n,k]): one row; a tile less, full, one more; columns that end inside a tile and a 16-byte piece of the
-# output; k of one piece, less than a chunk, 4, 8 and 12 bytes into a piece (the first of a chunk, a later one), fewer chunks than waves
+# output; k of one piece, less than a chunk, 4, 8 and 12 bytes into a piece (the first of a chunk, a later one), fewer chunks than waves; tiles of 32x64 and 64x64
 @pytest.mark.parametrize("dtype", [oracle.FP16, oracle.BF16])
-@pytest.mark.parametrize("case", [(1, 4, 8, 2, True), (1, 36, 514, 8, True), (31, 32, 64, 3, False), (32, 264, 66, 16, False), (33, 100, 324, 8, True),
-                                  (64, 4096, 128, 2, True), (65, 1032, 1030, 4, False), (129, 72, 2052, 11, False), (200, 3996, 192, 1, True)])
+@pytest.mark.parametrize("case", [(1, 4, 8, 2, True, "32x32"), (1, 36, 514, 8, True, "32x32"), (31, 32, 64, 3, False, "32x32"), (32, 264, 66, 16, False, "32x32"),
+                                  (33, 100, 324, 8, True, "32x32"), (64, 4096, 128, 2, True, "32x32"), (65, 1032, 1030, 4, False, "32x32"),
+                                  (129, 72, 2052, 11, False, "32x32"), (200, 3996, 192, 1, True, "64x64"), (407, 1256, 160, 2, False, "64x64"),
+                                  (290, 1064, 1034, 3, False, "32x64"), (203, 1376, 84, 3, True, "32x64"), (370, 1688, 124, 2, True, "64x64")])
 def test_float_allreduce(case, dtype):
     _need_gpu()
-    M, N, K, P, tb = case
+    M, N, K, P, tb, tiles = case
     rng = np.random.default_rng(M + K)
     A, B = _rand16(rng, (M, K), dtype), _rand16(rng, (K, N), dtype, 0.05)
     peers = [rng.standard_normal((M + 3, N + 4)).astype(np.float32) for _ in range(P - 1)]
     dump = torch.full((M, N), 7.0, dtype=torch.float32, device="cuda:0")
     out = ops.matmul_allreduce(dev16(A, dtype), dev16(np.ascontiguousarray(B.T) if tb else B, dtype), [dev(p) for p in peers], 0, P, trans_b=tb,
                                peer_row_offset=3, acc_dump=dump)
+    assert ran() == tiles
     torch.cuda.synchronize()
     got, want = dump.cpu().numpy(), oracle.half_to_f32(A, dtype).astype(np.float64) @ oracle.half_to_f32(B, dtype).astype(np.float64)
     assert (np.abs(got - want) <= sum_bound(A, B, dtype)).all()
@@ -37,10 +49,12 @@ def test_float_allreduce(case, dtype):
     assert np.array_equal(host16(out), oracle.f32_to_half(got, dtype))
 
 
-@pytest.mark.parametrize("case", [(1, 260, 130, 8, True), (7, 64, 256, 5, False), (33, 136, 1028, 2, True), (40, 520, 98, 3, False)])
+@pytest.mark.parametrize("case", [(1, 260, 130, 8, True, "32x32"), (7, 64, 256, 5, False, "32x32"), (33, 136, 1028, 2, True, "32x32"), (40, 520, 98, 3, False, "32x32"),
+                                  (257, 280, 102, 4, False, "32x64"), (112, 1328, 108, 2, True, "32x64"), (92, 1928, 146, 3, False, "64x64"),
+                                  (275, 488, 96, 4, True, "64x64"), (256, 1644, 400, 3, True, "64x128"), (271, 1944, 832, 2, False, "64x128")])
 def test_float_allgather_tiles_across_shards(case):
     _need_gpu()
-    m, N, K, P, tb = case
+    m, N, K, P, tb, tiles = case
     rng = np.random.default_rng(m + K)
     B = _rand16(rng, (K, N), oracle.BF16, 0.05)
     shards = [_rand16(rng, (m, K), oracle.BF16) for _ in range(P)]
@@ -48,6 +62,7 @@ def test_float_allgather_tiles_across_shards(case):
     ds = [dev16(s, oracle.BF16) for s in shards]
     dump = torch.full((m * P, N), 7.0, dtype=torch.float32, device="cuda:0")
     out = ops.allgather_matmul(ds[rank], ds[:rank] + ds[rank + 1:], dev16(np.ascontiguousarray(B.T) if tb else B, oracle.BF16), rank, P, trans_b=tb, acc_dump=dump)
+    assert ran() == tiles
     torch.cuda.synchronize()
     A = np.concatenate(shards)
     want = oracle.half_to_f32(A, oracle.BF16).astype(np.float64) @ oracle.half_to_f32(B, oracle.BF16).astype(np.float64)
@@ -56,11 +71,15 @@ def test_float_allgather_tiles_across_shards(case):
 
 
 # (rows, N, K, P, first kept row, kept rows, weights as [n,k], int32 peers)
-@pytest.mark.parametrize("case", [(1, 128, 128, 8, 0, 1, True, False), (17, 384, 1344, 16, 3, 9, True, True), (32, 36, 20, 2, 31, 1, True, False),
-                                  (33, 260, 1236, 4, 30, 3, False, True), (70, 48, 130 * 2, 8, 0, 70, False, False), (203, 1792, 1776, 8, 64, 100, False, False)])
+@pytest.mark.parametrize("case", [(1, 128, 128, 8, 0, 1, True, False, "32x32"), (17, 384, 1344, 16, 3, 9, True, True, "32x32"),
+                                  (32, 36, 20, 2, 31, 1, True, False, "32x32"), (33, 260, 1236, 4, 30, 3, False, True, "flexible 64x256"),
+                                  (70, 48, 260, 8, 0, 70, False, False, "32x32"), (203, 1792, 1776, 8, 64, 100, False, False, "32x64"),
+                                  (336, 1696, 140, 3, 0, 336, False, True, "64x64"), (286, 1964, 124, 5, 0, 286, True, False, "64x64"),
+                                  (645, 2608, 1344, 2, 0, 645, False, False, "64x128"), (514, 2224, 2092, 2, 0, 514, True, False, "64x128"),
+                                  (387, 1424, 80, 4, 0, 387, False, False, "64x64")])
 def test_quant_kept_rows(case):
     _need_gpu()
-    M, N, K, P, kb, kr, tb, ri = case
+    M, N, K, P, kb, kr, tb, ri, tiles = case
     rng = np.random.default_rng(M + N)
     x1, x2 = rng.integers(-127, 128, (M, K), dtype=np.int8), rng.integers(-127, 128, (K, N), dtype=np.int8)
     s1, s2 = rng.uniform(0.005, 0.02, M).astype(np.float32), rng.uniform(0.001, 0.01, N).astype(np.float32)
@@ -72,15 +91,17 @@ def test_quant_kept_rows(case):
     ws = torch.zeros(max(need, 65536), dtype=torch.uint8, device="cuda:0")
     out = ops.quant_matmul_splitk(dev(x1), dev(np.ascontiguousarray(x2.T) if tb else x2), dev(s1), dev(s2), dev(b), [dev(p) for p in peers], P, kb, kr,
                                   workspace=ws, acc_dump=dump, trans_b=tb, reduce_int32=ri)
+    assert ran() == tiles
     torch.cuda.synchronize()
     assert np.array_equal(host16(out), want) and np.array_equal(dump.cpu().numpy(), acc) and not ws[:65536].any()
 
 
 # (rows per rank, N, K, P, rank, weights as [n,k], int32 peers): kept rows inside a tile and across two, other ranks' rows beside them
-@pytest.mark.parametrize("case", [(5, 260, 132, 8, 3, True, False), (20, 512, 416, 4, 0, False, True), (33, 300, 1000, 16, 15, True, False), (61, 128, 272, 2, 1, False, False)])
+@pytest.mark.parametrize("case", [(5, 260, 132, 8, 3, True, False, "32x32", "32x32"), (20, 512, 416, 4, 0, False, True, "32x32", "32x32"),
+                                  (33, 300, 1000, 16, 15, True, False, "32x32", "32x32"), (61, 128, 272, 2, 1, False, False, "32x32", "32x32")])
 def test_reduce_scatter_stored_tiles(case):
     _need_gpu()
-    rows, N, K, P, rank, tb, ri = case
+    rows, N, K, P, rank, tb, ri, *kinds = case
     M = rows * P
     rng = np.random.default_rng(M + N)
     flip = lambda w: np.ascontiguousarray(w.T) if tb else w
@@ -114,6 +135,7 @@ def test_reduce_scatter_stored_tiles(case):
             for p in peers:
                 got = got + p
             assert np.array_equal(host16(out), oracle.f32_to_half(got, oracle.FP16))
+        assert ran() == kinds[0 if quant else 1]
         step = 64 if rows <= 64 else 128
         tiles = ob.cpu().numpy().reshape(-1, 256)
         for task, r, row, col, ws in tasks_of(comm, t, d):
@@ -122,17 +144,18 @@ def test_reduce_scatter_stored_tiles(case):
                 assert np.array_equal(tiles[ws:ws + r1 - row, :c1 - col].view(np.uint32), full[row:r1, col:c1].view(np.uint32)), task
 
 
-@pytest.mark.parametrize("case", [(35, 72, 520 + 66, 4, True), (35, 72, 520 + 66, 4, False), (3, 40, 1024, 2, True)])
+@pytest.mark.parametrize("case", [(35, 72, 586, 4, True, "32x32"), (35, 72, 586, 4, False, "32x32"), (3, 40, 1024, 2, True, "32x32")])
 def test_values_that_are_not_finite_stay_in_their_row_and_column(case):
     """Infinities in the last element of k: the pieces past the end of k hold them too and must not reach a sum."""
     _need_gpu()
-    M, N, K, P, tb = case
+    M, N, K, P, tb, tiles = case
     rng = np.random.default_rng(K)
     A, B = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
     A[M // 2, K - 1], B[K - 1, N // 3], B[K - 17, 1] = -np.inf, np.inf, np.nan
     ab, bb = oracle.f32_to_half(A, oracle.BF16), oracle.f32_to_half(B, oracle.BF16)
     peers = [rng.standard_normal((M, N)).astype(np.float32) for _ in range(P - 1)]
     out = ops.matmul_allreduce(dev16(ab, oracle.BF16), dev16(np.ascontiguousarray(bb.T) if tb else bb, oracle.BF16), [dev(p) for p in peers], 0, P, trans_b=tb)
+    assert ran() == tiles
     torch.cuda.synchronize()
     got = oracle.half_to_f32(host16(out), oracle.BF16)
     with np.errstate(all="ignore"):
@@ -142,13 +165,15 @@ def test_values_that_are_not_finite_stay_in_their_row_and_column(case):
     assert (np.abs(got[fin] - want[fin]) <= 2.0 ** -8 * np.abs(want[fin]) + 1e-2).all()   # (half a last place of 8 bits, and the sums' own bound)
 
 
-# (rows, N, K, P, first kept row, kept rows, weights as [n,k]): checksums, which tiles of 64x128 (up to 64 rows) and 128x128 leave; rows
+# (rows, N, K, P, first kept row, kept rows, weights as [n,k], tiles): checksums of tiles smaller than a block and as large, with a dump; rows
 # and columns one past a tile, k of one chunk and less, of a few bytes more than whole chunks, more chunks than stages
-@pytest.mark.parametrize("case", [(40, 128, 100, 2, 3, 10, True), (64, 132, 132, 8, 0, 8, True), (65, 260, 1236, 4, 60, 5, False), (128, 112, 776, 3, 128 - 40, 40, False),
-                                  (129, 516, 648, 8, 128, 1, True), (300, 240, 2440, 6, 100, 150, False), (18, 48, 36, 1, 2, 4, True)])
+@pytest.mark.parametrize("case", [(40, 128, 100, 2, 3, 10, True, "32x32"), (64, 132, 132, 8, 0, 8, True, "32x32"), (65, 260, 1236, 4, 60, 5, False, "flexible 128x256"),
+                                  (128, 112, 776, 3, 88, 40, False, "32x32"), (129, 516, 648, 8, 128, 1, True, "32x32"), (300, 240, 2440, 6, 100, 150, False, "32x32"),
+                                  (18, 48, 36, 1, 2, 4, True, "32x32"), (454, 2416, 96, 16, 101, 1, False, "64x128"), (560, 2132, 112, 8, 37, 330, True, "64x128"),
+                                  (700, 4608, 1296, 2, 130, 300, False, "128x128"), (650, 4612, 1292, 3, 600, 50, True, "128x128")])
 def test_quant_kept_rows_with_checksums(case):
     _need_gpu()
-    M, N, K, P, kb, kr, tb = case
+    M, N, K, P, kb, kr, tb, tiles = case
     rng = np.random.default_rng(M + N)
     x1, x2 = rng.integers(-127, 128, (M, K), dtype=np.int8), rng.integers(-127, 128, (K, N), dtype=np.int8)
     s1, s2 = rng.uniform(0.005, 0.02, M).astype(np.float32), rng.uniform(0.001, 0.01, N).astype(np.float32)
@@ -162,6 +187,7 @@ def test_quant_kept_rows_with_checksums(case):
     dump = torch.full((M, N), -7, dtype=torch.int32, device="cuda:0")
     out = ops.quant_matmul_splitk(dev(x1), dev(np.ascontiguousarray(x2.T) if tb else x2), dev(s1), dev(s2), dev(b), [dev(p) for p in peers], P, kb, kr,
                                   workspace=torch.zeros(1 << 20, dtype=torch.uint8, device="cuda:0"), checksum=cs, acc_dump=dump, trans_b=tb)
+    assert ran() == tiles
     torch.cuda.synchronize()
     assert np.array_equal(host16(out), want) and np.array_equal(dump.cpu().numpy(), acc) and np.array_equal(cs.cpu().numpy(), sums)
 
@@ -178,12 +204,16 @@ def one_round(comm, M, K, N, P, rank):
     return t, d
 
 
-# (operator, rows (of a shard), N, K, P, rank, weights as [n,k]): 64x128 and 128x128 tiles of the float operators
-@pytest.mark.parametrize("case", [("allreduce", 1000, 1544, 1234, 4, 0, False), ("allreduce", 650, 3332, 2310, 3, 0, True), ("allgather", 278, 4864, 4736, 2, 1, False), ("allreduce", 610, 4608, 5000, 8, 0, False),
-                                  ("reduce_scatter", 1392, 1540, 2820, 8, 5, True), ("reduce_scatter", 600, 4104, 1032, 2, 1, False)])
+# (operator, rows (of a shard), N, K, P, rank, weights as [n,k], tiles): 64x128 and 128x128 tiles of the float operators, and calls near them
+@pytest.mark.parametrize("case", [("allreduce", 1000, 1544, 1234, 4, 0, False, "flexible 64x256"), ("allreduce", 650, 3332, 2310, 3, 0, True, "128x128"),
+                                  ("allgather", 278, 4864, 4736, 2, 1, False, "128x128"), ("allreduce", 610, 4608, 5000, 8, 0, False, "flexible 64x256"),
+                                  ("reduce_scatter", 1392, 1540, 2820, 8, 5, True, "128x128 dealt"), ("reduce_scatter", 600, 4104, 1032, 2, 1, False, "flexible 64x256"),
+                                  ("allreduce", 644, 1492, 460, 3, 0, True, "64x128"), ("allreduce", 417, 2344, 808, 2, 0, False, "64x128"),
+                                  ("allgather", 530, 464, 432, 4, 2, True, "64x128"), ("allgather", 600, 688, 760, 3, 0, False, "64x128"),
+                                  ("allgather", 276, 776, 530, 16, 11, True, "128x128"), ("allgather", 431, 1104, 1090, 8, 4, False, "128x128")])
 def test_float_larger_tiles(case):
     _need_gpu()
-    op, m, N, K, P, rank, tb = case
+    op, m, N, K, P, rank, tb, kind = case
     g = torch.Generator(device="cuda:0").manual_seed(m)
     rand = lambda *shape: torch.randn(shape, device="cuda:0", generator=g)
     M = m * P if op == "allgather" else m
@@ -209,6 +239,7 @@ def test_float_larger_tiles(case):
                 r1, c1 = min(row + 128, (r + 1) * rows), min(col + 256, N)
                 assert np.array_equal(tiles[ws:ws + r1 - row, :c1 - col], full[row:r1, col:c1]), task
         got = dump[rank * rows:(rank + 1) * rows]
+    assert ran() == kind
     bound = 8 * K ** 0.5 * 2.0 ** -24 * torch.outer(A.double().norm(dim=1), B.double().norm(dim=0)) + 1e-9   # (as sum_bound)
     assert ((dump.double() - A.double() @ B.double()).abs() <= bound).all()
     for p in peers:
@@ -219,11 +250,12 @@ def test_float_larger_tiles(case):
 # (rows per rank, N, K, P, rank, weights as [n,k], int32 peers): launches of 256x256 and 128x128 tiles; the kept rows (on small tiles) at the
 # start, in the middle and at the end, k of whole pairs of steps and 4 to 124 bytes more, columns past a tile; one rank, whose kept rows are
 # on tiles of both kinds
-@pytest.mark.parametrize("case", [(335, 6912, 3204, 8, 5, False, False), (543, 3844, 3836, 8, 0, True, True), (664, 3460, 5888, 8, 7, True, False), (4344, 3844, 3836, 1, 0, True, False),
-                                  (3700, 3840, 3072, 1, 0, False, False)])
+@pytest.mark.parametrize("case", [(335, 6912, 3204, 8, 5, False, False, "256x256 dealt"), (543, 3844, 3836, 8, 0, True, True, "256x256 dealt"),
+                                  (664, 3460, 5888, 8, 7, True, False, "256x256 dealt"), (4344, 3844, 3836, 1, 0, True, False, "256x256"),
+                                  (3700, 3840, 3072, 1, 0, False, False, "256x256")])
 def test_quant_mixed_tiles(case):
     _need_gpu()
-    rows, N, K, P, rank, tb, ri = case
+    rows, N, K, P, rank, tb, ri, kind = case
     M = rows * P
     g = torch.Generator(device="cuda:0").manual_seed(rows)
     x1, x2 = (torch.randint(-127, 128, shape, dtype=torch.int8, device="cuda:0", generator=g) for shape in ((M, K), (K, N)))
@@ -237,6 +269,7 @@ def test_quant_mixed_tiles(case):
     dump, sums = torch.full((M, N), -7, dtype=torch.int32, device="cuda:0"), torch.full((rows, N), -7, dtype=torch.int32, device="cuda:0")
     out = ops.quant_matmul_reduce_scatter(x1, x2.T.contiguous() if tb else x2, s1, s2, b, peers, rank, P, tiling=t, trans_b=tb, reduce_int32=ri, outbound=ob,
                                           acc_dump=dump, c_accum=sums, out=marked(rows, N, torch.bfloat16))
+    assert ran() == kind
     acc = (x1.double() @ x2.double()).to(torch.int32) + b   # (exact)
     kept = acc[rank * rows:(rank + 1) * rows]
     if ri:
@@ -254,32 +287,41 @@ def test_quant_mixed_tiles(case):
             assert torch.equal(tiles[ws:ws + r1 - row, :c1 - col], full[row:r1, col:c1]), task
 
 
-@pytest.mark.parametrize("case", [("allgather", 845, 3940, 3330, 8, 3, True), ("allgather", 822, 2308, 6560, 8, 0, True), ("allreduce", 3438, 5892, 3712, 4, 0, True),
-                                  ("reduce_scatter", 6184, 3072, 10752, 8, 2, False), ("reduce_scatter", 8144, 1696, 5120, 1, 0, True), ("reduce_scatter", 3000, 4096, 4096, 1, 0, False)])
+@pytest.mark.parametrize("case", [("allgather", 845, 3940, 3330, 8, 3, True, "256x256"), ("allgather", 822, 2308, 6560, 8, 0, True, "256x256"),
+                                  ("allreduce", 3438, 5892, 3712, 4, 0, True, "256x256"), ("reduce_scatter", 6184, 3072, 10752, 8, 2, False, "256x256 dealt"),
+                                  ("reduce_scatter", 8144, 1696, 5120, 1, 0, True, "256x256"), ("reduce_scatter", 3000, 4096, 4096, 1, 0, False, "256x256")])
 def test_float_mixed_tiles(case):
     test_float_larger_tiles(case)
 
 
 # Kept rows dealt out to the 128- and 64-row tiles: 16 or fewer to a tile (one group of a thread's rows; of 16 ranks more peers than fit at
-# once), up to 32, up to 64 and as many as two ranks leave, tiles of unequal shares, first, last and a middle rank, columns past a tile
-@pytest.mark.parametrize("case", [(125, 4096, 1376, 8, 5, True, False), (65, 4096, 1040, 16, 15, False, True), (59, 4100, 1028, 16, 0, True, False), (123, 5116, 1660, 4, 1, True, False),
-                                  (500, 4096, 1376, 2, 1, True, True), (103, 1792, 1732, 8, 3, False, False), (299, 544, 1280, 8, 7, True, False)])
+# once), up to 32, up to 64 and as many as two ranks leave, tiles of unequal shares, first, last and a middle rank, columns past a tile; one rank, where none is dealt
+@pytest.mark.parametrize("case", [(125, 4096, 1376, 8, 5, True, False, "128x128 dealt"), (65, 4096, 1040, 16, 15, False, True, "128x128 dealt"),
+                                  (59, 4100, 1028, 16, 0, True, False, "64x128 dealt"), (123, 5116, 1660, 4, 1, True, False, "128x128 dealt"),
+                                  (500, 4096, 1376, 2, 1, True, True, "128x128 dealt"), (103, 1792, 1732, 8, 3, False, False, "64x128 dealt"),
+                                  (299, 544, 1280, 8, 7, True, False, "64x128 dealt"), (406, 2504, 496, 1, 0, True, False, "64x128"),
+                                  (615, 1616, 1656, 1, 0, False, False, "64x128")])
 def test_quant_dealt_rows(case):
     test_quant_mixed_tiles(case)
 
 
-@pytest.mark.parametrize("case", [("reduce_scatter", 936, 6148, 1666, 8, 3, True), ("reduce_scatter", 1684, 2304, 520, 4, 0, False), ("reduce_scatter", 2400, 548, 1280, 16, 15, True)])
+@pytest.mark.parametrize("case", [("reduce_scatter", 936, 6148, 1666, 8, 3, True, "flexible 128x256"),
+                                  ("reduce_scatter", 1684, 2304, 520, 4, 0, False, "flexible 64x256"), ("reduce_scatter", 2400, 548, 1280, 16, 15, True, "64x128 dealt"),
+                                  ("reduce_scatter", 480, 2344, 126, 8, 6, False, "64x128 dealt"), ("reduce_scatter", 510, 2344, 114, 2, 1, True, "64x128 dealt"),
+                                  ("reduce_scatter", 1392, 1544, 1820, 8, 0, False, "128x128 dealt"), ("reduce_scatter", 1392, 1540, 1820, 4, 3, True, "128x128 dealt")])
 def test_float_dealt_rows(case):
     test_float_larger_tiles(case)
 
 
 # (rows, N, K, P, first kept row, kept rows, weights as [n,k]): sums of 128x128 blocks that several tiles add up: 32x32, 32x64, 64x64 and 64x128
 # tiles, blocks of one tile and of few at the edges, blocks whose rows are all kept, negative and positive sums
-@pytest.mark.parametrize("case", [(1, 132, 96, 2, 0, 1, True), (33, 300, 1416, 8, 5, 7, False), (128, 1280, 2416, 8, 0, 128, True), (130, 516, 416, 4, 1, 128, True), (300, 1408, 512, 8, 200, 40, True),
-                                  (80, 2784, 1060, 4, 60, 20, True), (462, 1536, 2336, 4, 0, 116, True), (409, 2688, 6232, 4, 300, 103, True)])
+@pytest.mark.parametrize("case", [(1, 132, 96, 2, 0, 1, True, "32x32", "64x128"), (33, 300, 1416, 8, 5, 7, False, "flexible 64x256", "flexible 64x256"),
+                                  (128, 1280, 2416, 8, 0, 128, True, "32x32", "128x128"), (130, 516, 416, 4, 1, 128, True, "32x32", "128x128"),
+                                  (300, 1408, 512, 8, 200, 40, True, "32x64", None), (80, 2784, 1060, 4, 60, 20, True, "32x64", "128x128"),
+                                  (462, 1536, 2336, 4, 0, 116, True, "64x64", "128x128"), (409, 2688, 6232, 4, 300, 103, True, "64x128", "128x128")])
 def test_quant_kept_rows_block_sums(case):
     _need_gpu()
-    M, N, K, P, kb, kr, tb = case
+    M, N, K, P, kb, kr, tb, *tiles = case
     g = torch.Generator(device="cuda:0").manual_seed(M + N)
     x1, x2 = (torch.randint(-127, 128, shape, dtype=torch.int8, device="cuda:0", generator=g) for shape in ((M, K), (K, N)))
     x1[: M // 2] = x1[: M // 2].abs()   # (sums of either sign and size)
@@ -293,10 +335,11 @@ def test_quant_kept_rows_block_sums(case):
     want = torch.stack([others[r:r + 128, c:c + 128].sum() for r in range(0, M, 128) for c in range(0, N, 128)])
     out = None
     for w in (ws, ws, None):   # (the counter block is left at zero; without one the other kernels run)
-        if w is None and (K % 64 == 0 and N % 128 == 0):
+        if w is None and tiles[1] is None:   # (needs one)
             continue
         cs = torch.full((want.numel(),), -7, dtype=torch.int64, device="cuda:0")
         got = ops.quant_matmul_splitk(x1, x2.T.contiguous() if tb else x2, s1, s2, None, peers, P, kb, kr, workspace=w, checksum=cs, trans_b=tb)
+        assert ran() == tiles[0 if w is not None else 1]
         torch.cuda.synchronize()
         assert torch.equal(cs, want) and not ws[:65536].any()
         assert out is None or torch.equal(got, out)
@@ -321,11 +364,15 @@ def check_workspace(ws, need):
 # (operator, rows (of a shard), N, K, P, rank, weights as [n,k]): small tiles in k slices; k of odd chunks, rows and columns past a tile, more peers than
 # registers hold at once, slices of unequal length
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("case", [("allreduce", 33, 896, 6656, 4, 0, False), ("allreduce", 7, 1024, 11262, 8, 0, True), ("allreduce", 20, 516, 8190, 16, 0, True), ("allgather", 2, 1536, 8448, 4, 3, True),
-                                  ("allgather", 13, 1024, 14500, 8, 0, True), ("reduce_scatter", 44, 640, 6000, 2, 1, True), ("reduce_scatter", 112, 512, 6144, 4, 2, False)])
+@pytest.mark.parametrize("case", [("allreduce", 33, 896, 6656, 4, 0, False, "32x32/4"), ("allreduce", 7, 1024, 11262, 8, 0, True, "32x32/6"),
+                                  ("allreduce", 20, 516, 8190, 16, 0, True, "32x32/8"), ("allgather", 2, 1536, 8448, 4, 3, True, "32x32/4"),
+                                  ("allgather", 13, 1024, 14500, 8, 0, True, "32x64/4"), ("reduce_scatter", 44, 640, 6000, 2, 1, True, "32x32/6"),
+                                  ("reduce_scatter", 112, 512, 6144, 4, 2, False, "32x32/4"), ("allreduce", 33, 1576, 5874, 8, 0, False, "64x64/8"),
+                                  ("allreduce", 33, 1536, 6442, 3, 0, True, "64x64/8"), ("allreduce", 34, 2072, 3430, 8, 0, True, "32x64/3"),
+                                  ("allreduce", 334, 304, 5808, 2, 0, False, "32x64/4")])
 def test_float_k_slices(case, dtype):
     _need_gpu()
-    op, m, N, K, P, rank, tb = case
+    op, m, N, K, P, rank, tb, kind = case
     g = torch.Generator(device="cuda:0").manual_seed(m)
     rand = lambda *shape: torch.randn(shape, device="cuda:0", generator=g)
     M = m * P if op == "allgather" else m
@@ -355,6 +402,7 @@ def test_float_k_slices(case, dtype):
                     r1, c1 = min(row + 64, (r + 1) * rows), min(col + 256, N)
                     assert np.array_equal(tiles[place:place + r1 - row, :c1 - col], full[row:r1, col:c1]), task
             got = dump[rank * rows:(rank + 1) * rows]
+        assert ran() == kind
         torch.cuda.synchronize()
         check_workspace(ws, need)
         assert first is None or torch.equal(first, dump)   # (slice order, whichever arrives last)
@@ -367,11 +415,12 @@ def test_float_k_slices(case, dtype):
 
 
 # (rows, N, K, P, first kept row, kept rows, weights as [n,k], int32 peers, dump): as above; of rows that are not kept only the sums, or all of them
-@pytest.mark.parametrize("case", [(51, 1920, 12800, 4, 30, 13, True, False, False), (51, 1920, 12800, 4, 30, 13, True, False, True), (67, 640, 4992, 8, 0, 67, False, True, False),
-                                  (134, 768, 4736, 8, 60, 17, False, False, False), (2, 512, 7680, 4, 1, 1, True, True, False), (24, 2560, 14848, 8, 21, 3, False, False, False)])
+@pytest.mark.parametrize("case", [(51, 1920, 12800, 4, 30, 13, True, False, False, "64x64/8"), (51, 1920, 12800, 4, 30, 13, True, False, True, "32x32/2"),
+                                  (67, 640, 4992, 8, 0, 67, False, True, False, "32x32/4"), (134, 768, 4736, 8, 60, 17, False, False, False, "32x32/2"),
+                                  (2, 512, 7680, 4, 1, 1, True, True, False, "32x32/6"), (24, 2560, 14848, 8, 21, 3, False, False, False, "32x32/3")])
 def test_quant_k_slices(case):
     _need_gpu()
-    M, N, K, P, kb, kr, tb, ri, with_dump = case
+    M, N, K, P, kb, kr, tb, ri, with_dump, tiles = case
     g = torch.Generator(device="cuda:0").manual_seed(M + N)
     x1, x2 = (torch.randint(-127, 128, shape, dtype=torch.int8, device="cuda:0", generator=g) for shape in ((M, K), (K, N)))
     s1, s2 = (torch.empty(c, device="cuda:0").uniform_(0.001, 0.02, generator=g) for c in (M, N))
@@ -392,6 +441,7 @@ def test_quant_k_slices(case):
         cs = torch.full((sums.numel(),), -7, dtype=torch.int64, device="cuda:0")
         dump = torch.full((M, N), -7, dtype=torch.int32, device="cuda:0") if with_dump else None
         out = ops.quant_matmul_splitk(x1, x2.T.contiguous() if tb else x2, s1, s2, b, peers, P, kb, kr, workspace=ws, checksum=cs, acc_dump=dump, trans_b=tb, reduce_int32=ri)
+        assert ran() == tiles
         torch.cuda.synchronize()
         check_workspace(ws, need)
         assert torch.equal(cs, sums) and torch.equal(out, y.bfloat16())
@@ -400,11 +450,16 @@ def test_quant_k_slices(case):
 
 # (rows per rank, N, K, P, rank, weights as [n,k], int32 peers): sums of tasks that several tiles add up: ranks of a few rows (many tasks to a tile), of a
 # tile and a bit, of several task rows; columns that end in a task's first and second half; a long k (slices), 128-column tiles
-@pytest.mark.parametrize("case", [(1, 256, 100, 8, 3, True, False), (2, 1000, 516, 16, 9, True, True), (5, 388, 1040, 8, 0, True, False), (33, 640, 416, 4, 3, False, True), (130, 900, 772, 2, 1, True, False),
-                                  (8, 768, 15776, 2, 0, False, False), (69, 1024, 1024, 8, 5, True, False), (166, 768, 512, 8, 2, True, False), (219, 640, 9984, 8, 7, True, True), (300, 1800, 644, 4, 1, True, False)])
+@pytest.mark.parametrize("case", [(1, 256, 100, 8, 3, True, False, "32x32"), (2, 1000, 516, 16, 9, True, True, "32x32"), (5, 388, 1040, 8, 0, True, False, "32x32"),
+                                  (33, 640, 416, 4, 3, False, True, "32x32"), (130, 900, 772, 2, 1, True, False, "32x64"),
+                                  (8, 768, 15776, 2, 0, False, False, "32x32/8"), (69, 1024, 1024, 8, 5, True, False, "64x64"),
+                                  (166, 768, 512, 8, 2, True, False, "64x64"), (219, 640, 9984, 8, 7, True, True, "64x128 dealt"),
+                                  (300, 1800, 644, 4, 1, True, False, "flexible 128x256"), (88, 1984, 116, 8, 4, False, False, "64x128 dealt"),
+                                  (43, 2192, 164, 16, 13, False, True, "64x128 dealt"), (96, 1984, 1504, 2, 1, False, False, "32x64"),
+                                  (91, 1664, 1320, 4, 3, False, False, "64x64"), (184, 1440, 128, 8, 1, False, False, "128x128 dealt")])
 def test_quant_task_sums(case):
     _need_gpu()
-    rows, N, K, P, rank, tb, ri = case
+    rows, N, K, P, rank, tb, ri, tiles = case
     M = rows * P
     g = torch.Generator(device="cuda:0").manual_seed(rows)
     x1, x2 = (torch.randint(-127, 128, shape, dtype=torch.int8, device="cuda:0", generator=g) for shape in ((M, K), (K, N)))
@@ -428,9 +483,10 @@ def test_quant_task_sums(case):
         y = y + p
     need = ops.kslice_plan(L.QUANT_MATMUL_REDUCE_SCATTER, L.INT8, M, K, N, rank, P, tiling=t)[0]
     ws = torch.zeros(max(need, 65536), dtype=torch.uint8, device="cuda:0")
-    for w in (ws, ws, None):
+    for w in (ws, ws, None):   # (without counters sums are not small tiles')
         cs = torch.full((len(tasks),), 77, dtype=torch.int64, device="cuda:0")
         out = ops.quant_matmul_reduce_scatter(x1, x2.T.contiguous() if tb else x2, s1, s2, b, peers, rank, P, tiling=t, trans_b=tb, reduce_int32=ri, checksum=cs, workspace=w)
+        assert ran() == tiles if w is not None else L.last_launch().kernel != L.KERNEL_SMALL
         torch.cuda.synchronize()
         assert torch.equal(cs.cpu(), want) and torch.equal(out, y.bfloat16()) and not ws[:65536].any()
 
@@ -478,11 +534,13 @@ def test_small_tiles_replay_from_a_hip_graph():
 
 # (rows per rank, N, K, P, rank, weights as [n,k]): as test_quant_task_sums; sums of floats are added in one order
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("case", [(1, 256, 100, 8, 3, True), (5, 388, 1040, 8, 0, True), (33, 640, 416, 4, 3, False), (130, 900, 772, 2, 1, True), (37, 1024, 12672, 4, 2, False),
-                                  (43, 1920, 1152, 2, 0, True), (363, 640, 2364, 8, 6, False), (301, 1800, 646, 4, 1, True)])
+@pytest.mark.parametrize("case", [(1, 256, 100, 8, 3, True, "32x32"), (5, 388, 1040, 8, 0, True, "32x32"), (33, 640, 416, 4, 3, False, "32x32"),
+                                  (130, 900, 772, 2, 1, True, "32x64"), (37, 1024, 12672, 4, 2, False, "flexible 64x256/17"), (43, 1920, 1152, 2, 0, True, "32x32"),
+                                  (363, 640, 2364, 8, 6, False, "64x128 dealt"), (301, 1800, 646, 4, 1, True, "128x128 dealt"), (72, 1000, 94, 8, 2, False, "64x64"),
+                                  (85, 836, 4584, 4, 2, True, "64x64/3"), (24, 1312, 5824, 4, 0, False, "32x64/4"), (264, 1104, 128, 8, 1, False, "128x128 dealt")])
 def test_float_task_sums(case, dtype):
     _need_gpu()
-    rows, N, K, P, rank, tb = case
+    rows, N, K, P, rank, tb, tiles = case
     M = rows * P
     g = torch.Generator(device="cuda:0").manual_seed(rows)
     A, B = torch.randn((M, K), device="cuda:0", generator=g).to(dtype), (torch.randn((K, N), device="cuda:0", generator=g) * 0.05).to(dtype)
@@ -498,6 +556,7 @@ def test_float_task_sums(case, dtype):
     for _ in range(4):
         cs, dump = torch.full((len(tasks),), 77.0, dtype=torch.float64, device="cuda:0"), torch.zeros((M, N), device="cuda:0")
         out = ops.matmul_reduce_scatter(A, Bd, peers, rank, P, tiling=t, trans_b=tb, checksum=cs, acc_dump=dump, workspace=ws)
+        assert ran() == tiles
         torch.cuda.synchronize()
         assert not ws[:65536].any() and (first is None or torch.equal(first, cs))
         first = cs
@@ -515,10 +574,11 @@ def test_float_task_sums(case, dtype):
 
 # (rows, N, K, P, first kept row or rank, kept rows or 0: a reduce-scatter's, weights as [n,k]): sums of W8A8 tiles in k slices under a bias at either end of
 # its range: the whole accumulators are the bias itself, a slice's own sum and the bias are past the end
-@pytest.mark.parametrize("case", [(64, 512, 8192, 8, 20, 8, True), (70, 384, 8192, 2, 69, 1, False), (16, 768, 15776, 2, 0, 0, False), (40, 512, 8192, 4, 3, 0, True)])
+@pytest.mark.parametrize("case", [(64, 512, 8192, 8, 20, 8, True, "32x32/8"), (70, 384, 8192, 2, 69, 1, False, "32x32/6"), (16, 768, 15776, 2, 0, 0, False, "32x32/8"),
+                                  (40, 512, 8192, 4, 3, 0, True, "32x32/6")])
 def test_sums_of_k_slices_with_a_bias_at_the_end_of_its_range(case):
     _need_gpu()
-    M, N, K, P, at, kr, tb = case
+    M, N, K, P, at, kr, tb, tiles = case
     g = torch.Generator(device="cuda:0").manual_seed(M + N)
     u, v = (torch.randint(90, 128, shape, dtype=torch.int8, device="cuda:0", generator=g) for shape in ((M, K // 2), (K // 2, N)))
     up = torch.arange(N, device="cuda:0") % 3 != 0   # (more of one sign: what the two kinds of columns are off by does not cancel)
@@ -552,19 +612,26 @@ def test_sums_of_k_slices_with_a_bias_at_the_end_of_its_range(case):
     ws = sliced_workspace(need)
     cs = torch.full((want.numel(),), 77, dtype=torch.int64, device="cuda:0")
     out = run(cs, ws)
+    assert ran() == tiles
     torch.cuda.synchronize()
     check_workspace(ws, need)
     assert torch.equal(out, y.bfloat16()) and torch.equal(cs.cpu(), want)
 
 
-# (rows, N, K, P, rank, weights as [n,k], workspace): what a caller says about halves of kept tiles changes no bit, whichever tiles run: 128x128, 32x64 and mixed
-# tiles, small ones in k slices, whole flexible tiles or aligned ones instead, flexible ones in k slices
+# (rows, N, K, P, rank, weights as [n,k], workspace, tiles without and with a choice: floats, W8A8): what a caller says about halves of kept tiles changes no
+# bit, whichever tiles run: small and mixed ones, in k slices, whole flexible tiles or aligned ones instead, flexible ones in k slices
 @pytest.mark.parametrize("kind", [torch.float16, torch.bfloat16, torch.int8])
-@pytest.mark.parametrize("case", [(2048, 2048, 1792, 8, 3, False, False), (1024, 512, 512, 8, 7, True, False), (4096, 4096, 1792, 8, 2, True, False), (512, 512, 6144, 4, 2, False, True),
-                                  (512, 4096, 1024, 4, 1, True, False), (1024, 1024, 8192, 2, 0, True, True)])
+@pytest.mark.parametrize("case", [(2048, 2048, 1792, 8, 3, False, False, "128x128 dealt", "128x128 dealt", "128x128 dealt", "128x128 dealt"),
+                                  (1024, 512, 512, 8, 7, True, False, "32x64", "32x64", "32x64", "32x64"),
+                                  (4096, 4096, 1792, 8, 2, True, False, "256x256 dealt", "256x256 dealt", "256x256 dealt", "256x256 dealt"),
+                                  (512, 512, 6144, 4, 2, False, True, "32x64/2", "32x64/2", "32x32", "32x32"),
+                                  (512, 4096, 1024, 4, 1, True, False, "64x128 dealt", "64x128 dealt", "64x128 dealt", "64x128 dealt"),
+                                  (1024, 1024, 8192, 2, 0, True, True, "64x64", "64x64", "64x64", "64x64"),
+                                  (512, 8192, 512, 2, 1, True, True, "flexible 64x256", "aligned 128x256", "aligned 128x256", "aligned 128x256"),
+                                  (512, 1024, 8192, 2, 1, False, True, "flexible 64x256/8", "flexible 64x256/8", "flexible 64x256/6", "flexible 64x256/6")])
 def test_halves_of_kept_tiles_change_no_bit(case, kind):
     _need_gpu()
-    M, N, K, P, rank, tb, slices = case
+    M, N, K, P, rank, tb, slices, *tiles = case
     g = torch.Generator(device="cuda:0").manual_seed(M + K)
     quant = kind == torch.int8
     if quant:
@@ -582,6 +649,7 @@ def test_halves_of_kept_tiles_change_no_bit(case, kind):
         ob, dump = torch.full((size,), 3.0, device="cuda:0"), torch.zeros((M, N), dtype=torch.int32 if quant else torch.float32, device="cuda:0")
         kw = dict(tiling=t, trans_b=tb, outbound=ob, acc_dump=dump, kept_split=choice, workspace=torch.zeros(need, dtype=torch.uint8, device="cuda:0") if slices else None)
         out = ops.quant_matmul_reduce_scatter(a, b, s1, s2, None, peers, rank, P, **kw) if quant else ops.matmul_reduce_scatter(a, b, peers, rank, P, **kw)
+        assert ran() == tiles[2 * quant + (choice in (False, True))]
         torch.cuda.synchronize()
         results.append((out, dump, ob))
     for r in results[1:]:
@@ -589,16 +657,17 @@ def test_halves_of_kept_tiles_change_no_bit(case, kind):
 
 
 # (rows, N, K, weights as [n,k], k slices): 32x32, 32x64, 64x64 tiles, whole and in k slices, 64x128 and 128x128 ones
-@pytest.mark.parametrize("case", [(100, 2048, 1024, True, False), (512, 1024, 1024, False, False), (1000, 512, 2052, True, False), (96, 512, 8192, True, True), (300, 1032, 6148, True, True),
-                                  (650, 3332, 2310, True, False)])
+@pytest.mark.parametrize("case", [(100, 2048, 1024, True, False, "32x32"), (512, 1024, 1024, False, False, "32x64"), (1000, 512, 2052, True, False, "32x64"),
+                                  (96, 512, 8192, True, True, "32x32/4"), (300, 1032, 6148, True, True, "64x64/3"), (650, 3332, 2310, True, False, "128x128")])
 def test_equal_rows_have_equal_sums_wherever_they_lie(case):
     _need_gpu()
-    M, N, K, tb, slices = case
+    M, N, K, tb, slices, tiles = case
     g = torch.Generator(device="cuda:0").manual_seed(M)
     A = torch.randn((1, K), device="cuda:0", generator=g).bfloat16().expand(M, K).contiguous()
     B = torch.randn((N, K) if tb else (K, N), device="cuda:0", generator=g).bfloat16()
     need = ops.kslice_plan(L.MATMUL_ALLREDUCE, torch.bfloat16, M, K, N, 0, 2)[0]
     dump = torch.zeros((M, N), device="cuda:0")
     ops.matmul_allreduce(A, B, [torch.zeros((M, N), device="cuda:0")], 0, 2, trans_b=tb, acc_dump=dump, workspace=torch.zeros(need, dtype=torch.uint8, device="cuda:0") if slices else None)
+    assert ran() == tiles
     torch.cuda.synchronize()
     assert torch.equal(dump, dump[:1].expand(M, N))

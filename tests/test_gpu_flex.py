@@ -255,10 +255,10 @@ def test_float_reduce_scatter_ragged_few_tiles_long_k():
             assert (np.abs(got - part[row.value:r1, col.value:c1]) <= bounds[row.value:r1, col.value:c1]).all(), task
 
 
-# (rows per rank, N, K, P, rank, weights as [n,k]): one-round pipelined calls on ragged columns, ragged rows, and few aligned tiles
+# (rows per rank, N, K, P, rank, weights as [n,k]): one-round pipelined calls on ragged columns, ragged rows, and few aligned tiles: all on small tiles
 @pytest.mark.parametrize("case", [(128, 640, 448, 8, 3, False), (256, 1440, 192, 4, 0, True), (72, 288, 100, 2, 1, False), (128, 512, 1792, 8, 7, True)])
 @pytest.mark.parametrize("deterministic", [True, False])
-def test_pipelined_quant_one_round(case, deterministic):
+def test_pipelined_quant_one_round(case, deterministic, kernel=L.KERNEL_SMALL):
     _need_gpu()
     rows, N, K, P, rank, tb = case
     M = rows * P
@@ -268,29 +268,34 @@ def test_pipelined_quant_one_round(case, deterministic):
     b = rng.integers(-1000, 1000, N, dtype=np.int32)
     peers = [rng.integers(-2 ** 20, 2 ** 20, (rows, N), dtype=np.int32) for _ in range(P - 1)]
     acc, want = oracle.quant_matmul_reduce_scatter(x1, x2, s1, s2, b, rank * rows, rows, peers, oracle.BF16, reduce_int32=True)
-    t = ops.default_tiling(M, K, N, P, m0=128, n0=256, k0=0)
+    t = ops.default_tiling(M, K, N, P, m0=128, n0=256, k0=0, commInterval=max(1, -(-(P * -(-rows // 128) * -(-N // 256)) // 256)))
     d = L.make_desc(rank, P, [16] * (P - 1))
     size = L.load().catcoc_get_workspace_size(L.QUANT_MATMUL_REDUCE_SCATTER, L.INT8, C.byref(t), C.byref(d))
     assert ops.pipelined_round_count(L.QUANT_MATMUL_REDUCE_SCATTER, t, rank, P) == 1
     ob = torch.full((size // 4,), -9, dtype=torch.int32, device="cuda:0")
     out, sums = ops.pipelined_quant_matmul_reduce_scatter(dev(x1), dev(np.ascontiguousarray(x2.T) if tb else x2), dev(s1), dev(s2), dev(b), [dev(p) for p in peers],
                                                           rank, P, ob, tiling=t, trans_b=tb, deterministic=deterministic)
+    assert L.last_launch().kernel == kernel
     torch.cuda.synchronize()
     assert np.array_equal(sums.cpu().numpy(), acc[rank * rows:(rank + 1) * rows] + sum(peers)) and np.array_equal(host16(out), want)
     tr, row, col, wsr = (C.c_uint32() for _ in range(4))
+    tiles = ob.cpu().numpy().reshape(-1, 256)
     for task in range(L.load().catcoc_get_task_count(L.QUANT_MATMUL_REDUCE_SCATTER, C.byref(t), C.byref(d))):
         L.load().catcoc_task_tile(L.QUANT_MATMUL_REDUCE_SCATTER, C.byref(t), C.byref(d), task, C.byref(tr), C.byref(row), C.byref(col), C.byref(wsr))
         if tr.value != rank:
             r1, c1 = min(row.value + 128, (tr.value + 1) * rows), min(col.value + 256, N)
-            got = ob.cpu().numpy().reshape(-1, 256)[wsr.value:wsr.value + r1 - row.value, :c1 - col.value]
+            got = tiles[wsr.value:wsr.value + r1 - row.value, :c1 - col.value]
             assert np.array_equal(got, acc[row.value:r1, col.value:c1]), task
 
 
-# one-round pipelined calls on aligned tiles whose peers the GEMM launch adds (two ranks; four with a short k), and one that keeps its comm launch
-@pytest.mark.parametrize("case", [(128, 512, 576, 2, 1, True), (256, 256, 960, 2, 0, False), (128, 512, 64, 4, 2, False), (128, 512, 960, 8, 6, True), (256, 3072, 512, 8, 4, True)])
+# one-round pipelined calls of whole tiles: few of them, on small ones; on aligned ones, whose peers the GEMM launch adds (two ranks, four with a short k, few
+# tiles, more than there are CUs); and one that keeps its comm launch
+@pytest.mark.parametrize("case", [(128, 512, 576, 2, 1, True), (256, 256, 960, 2, 0, False), (128, 512, 64, 4, 2, False), (128, 512, 960, 8, 6, True), (256, 3072, 512, 8, 4, True),
+                                  (384, 1536, 576, 4, 1, False), (384, 3072, 576, 2, 0, True), (512, 3072, 576, 8, 7, False), (384, 4096, 448, 8, 3, True)])
 @pytest.mark.parametrize("deterministic", [True, False])
 def test_pipelined_quant_one_round_on_aligned_tiles(case, deterministic):
-    test_pipelined_quant_one_round(case, deterministic)
+    rows, N, K, P, _, _ = case
+    test_pipelined_quant_one_round(case, deterministic, L.KERNEL_ALIGNED if rows * P * N >= 48 * 128 * 256 else L.KERNEL_SMALL)
 
 
 # one-round pipelined calls that one launch of small tiles takes: 128 and 64 rows by 128 columns, 32 and 64 rows by 64, ranks of ragged rows
@@ -317,6 +322,7 @@ def test_pipelined_quant_one_round_equals_two(tb):
         size = L.load().catcoc_get_workspace_size(L.QUANT_MATMUL_REDUCE_SCATTER, L.INT8, C.byref(t), C.byref(d))
         ob = torch.zeros(size // 4, dtype=torch.int32, device="cuda:0")
         got.append(ops.pipelined_quant_matmul_reduce_scatter(x1, x2, s1, s2, None, peers, rank, P, ob, tiling=t, trans_b=tb))
+        assert L.last_launch().kernel == L.KERNEL_ALIGNED
     torch.cuda.synchronize()
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
     want = x1[rank * rows:(rank + 1) * rows].float() @ (x2.T if tb else x2).float()   # (exact: |sums| < 2^24)
@@ -741,3 +747,31 @@ def test_stored_tiles_on_both_sides_of_the_choice_of_kernels(case, tb):
     for task, target, r0, c0, w0 in tasks_of(L.QUANT_MATMUL_REDUCE_SCATTER, t, d):
         if target != P - 1:
             assert np.array_equal(ob[w0:w0 + 128].view(np.uint32), deq[r0:r0 + 128, c0:c0 + 256].view(np.uint32)), task
+
+
+@pytest.fixture
+def flexible(monkeypatch):
+    """Ragged calls of the operators in the schedule's order: on flexible tiles, where small ones would else take some.  Every launch is seen to run there."""
+    def ordered(op):
+        def call(*a, **kw):
+            out = op(*a, **dict(kw, linear_order=True))
+            assert L.last_launch().kernel == L.KERNEL_FLEXIBLE
+            return out
+        return call
+    for name in ("matmul_allreduce", "allgather_matmul", "quant_matmul_reduce_scatter"):
+        monkeypatch.setattr(ops, name, ordered(getattr(ops, name)))
+
+
+@pytest.mark.parametrize("dtype", [oracle.FP16, oracle.BF16])
+@pytest.mark.parametrize("case", [("allreduce", 1, 256, 128, 8, True), ("allgather", 3, 264, 516, 8, True), ("allgather", 65, 768, 1026, 4, False)])
+def test_float_any_rows_any_k_on_flexible_tiles(dtype, case, flexible):
+    test_float_any_rows_any_k(dtype, case)
+
+
+@pytest.mark.parametrize("case", [(125, 512, 1376, 8, 5, True, False, 0, 1), (8, 256, 64, 8, 0, False, True, 0, 1), (65, 772, 260, 8, 7, True, True, 0, 1), (300, 516, 100, 4, 3, True, False, 0, 1)])
+def test_quant_rs_any_rows_any_k_on_flexible_tiles(case, flexible):
+    test_quant_rs_any_rows_any_k(case, True)
+
+
+def test_values_that_are_not_finite_on_flexible_tiles(flexible):
+    test_values_that_are_not_finite_stay_in_their_rows_and_columns(0, True)
