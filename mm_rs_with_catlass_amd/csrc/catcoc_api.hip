@@ -1083,9 +1083,14 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
     // The plan above says what the launch is refused for and what it asks of the workspace, whichever kernel runs.
     const auto flex = [&]() {
         // (few rows of a long k and few columns as [n,k]: the whole-k kernel's rings for up to eight rows hold more of B than a 32x32
-        // tile's.  8x16384x2048 13.3 / 13.9, 1x12288x1024 10.8 / 11.5, 1x8192x512 8.6 / 9.0; not 8x8192x2048 10.2 / 9.6, 8x12288x3072
-        // 13.6 / 11.9, 1x8192x8192 16.0 / 15.1, 16x4096x8192 10.6 / 9.4)
-        const bool deepK = sp.wholeK && (a.M <= 4 ? a.K >= 8192 && a.N <= (a.K > 8192 ? 4096u : 2048u) : a.M <= 8 && a.K > 12288 && a.N <= 2048);
+        // tile's.  Whole k / small tiles, us: 8x16384x2048 13.3 / 13.9, 1x12288x1024 10.8 / 11.5, 1x8192x512 8.6 / 9.0; not 8x8192x2048 10.2 / 9.6,
+        // 8x12288x3072 13.6 / 11.9, 1x8192x8192 16.0 / 15.1, 16x4096x8192 10.6 / 9.4.  And weights that stay in the cache, where a long k is a chain
+        // of waits: eight ranks, 12x16384x512 with 2 rows kept 12.1 / 13.0, 16x24576x256 with 2 16.5 / 17.4, 9x32768x128 with all 18.7 / 21.3, 8x12288x512
+        // with one 10.3 / 10.8.  All else of 9 to 32 rows is small tiles': calls with k of 4096 to 32768 and n of 128 to 8192 take 0.74 to 1.05 of
+        // the whole-k kernel's time, 20x32768x256 with 3 rows kept 1.07.)
+        const bool few = 4u * a.keptRows <= a.M, cached = (uint64_t)a.K * a.N <= (10u << 20);
+        const bool deepK = sp.wholeK && (a.M <= 4 ? a.K >= 8192 && a.N <= (a.K > 8192 ? 4096u : 2048u) : a.M <= 8 ? a.K > (few && cached ? 11264u : 12288u) && a.N <= 2048 :
+                                         a.M <= 16 && cached && a.K >= (few ? 14336u : 24576u));
         if (deepK || (!sp.maySmall && !sp.preferFlex)) return false;
         GemmArgs g = a;
         const uint32_t stages = d->workspaceStages ? d->workspaceStages : kDefaultStages;

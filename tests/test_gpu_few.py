@@ -350,6 +350,25 @@ def test_quant_kept_rows_block_sums(case):
     assert torch.equal(out, y.bfloat16())
 
 
+# (rows, N, K, kept rows): up to 16 rows of a long k against few columns, on both sides of the line between the whole-k kernel and 32x32 tiles
+@pytest.mark.parametrize("case", [(12, 640, 16384, 3, L.KERNEL_STREAMING), (16, 256, 14336, 4, L.KERNEL_STREAMING), (16, 128, 24576, 16, L.KERNEL_STREAMING), (8, 512, 12288, 2, L.KERNEL_STREAMING),
+                                  (12, 672, 16384, 3, L.KERNEL_SMALL), (12, 512, 16384, 4, L.KERNEL_SMALL), (16, 256, 14208, 4, L.KERNEL_SMALL), (17, 512, 16384, 3, L.KERNEL_SMALL),
+                                  (16, 128, 24448, 16, L.KERNEL_SMALL), (8, 512, 12288, 3, L.KERNEL_SMALL)])
+def test_quant_few_rows_of_a_long_k(case):
+    _need_gpu()
+    M, N, K, kr, kernel = case
+    g = torch.Generator(device="cuda:0").manual_seed(M + N)
+    x1, x2 = (torch.randint(-127, 128, s, dtype=torch.int8, device="cuda:0", generator=g) for s in ((M, K), (N, K)))
+    s1, s2 = (torch.empty(c, device="cuda:0").uniform_(0.001, 0.02, generator=g) for c in (M, N))
+    peers = [torch.randn((kr, N), device="cuda:0", generator=g) for _ in range(7)]
+    out = ops.quant_matmul_splitk(x1, x2, s1, s2, None, peers, 8, M - kr, kr, trans_b=True)
+    assert L.last_launch().kernel == kernel
+    y = ((x1[M - kr:].double() @ x2.T.double()).float() * s2) * s1[M - kr:, None]
+    for p in peers:
+        y = y + p
+    assert torch.equal(out, y.bfloat16())
+
+
 def sliced_workspace(need):
     """A workspace of more than the query asks for: counters at zero, marks behind what a launch may touch."""
     ws = torch.zeros(need + 4096, dtype=torch.uint8, device="cuda:0")
