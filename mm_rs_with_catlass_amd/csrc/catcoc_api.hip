@@ -428,10 +428,9 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other, uint64_t room = 0)
         rows >= (1u << 30) || s.n0 != 256 || (s.m0 != 64 && s.m0 != 128))
         return no;
     // Checksums: of tasks, and of the 128x128 blocks of explicit kept rows, for tiles that meet in the workspace's counter block (sum_add,
-    // sum_in_order) or have all of a block.  Decode launches that also want the kept rows' int32 block stay where their k slices leave it on
-    // the way.
+    // sum_in_order) or have all of a block.
     const bool rowMask = (a.flags & GF_ROW_MASK) != 0, sums = (a.flags & GF_OUTBOUND_STORE) == 0 && a.checksum != nullptr && (rowMask || a.keptRows < rows);
-    if ((sums && !rowMask && (a.skCount == nullptr || s.coreLoops > kCounterBlockBytes / 16u)) || (rowMask && a.cAccum != nullptr)) return no;
+    if (sums && !rowMask && (a.skCount == nullptr || s.coreLoops > kCounterBlockBytes / 16u)) return no;
     const CallSize c = call_size(a, es);
     const SmallTileCost *best = nullptr;
     double least = 0.0;
@@ -1109,7 +1108,10 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
         }
         if (sp.maySmall) {
             const SmallTile t = small_tile(small, 1, sp.wholeK ? 1e30 : kOtherShare * (blocks ? flex_us(g, 1, blocks) : streaming_us(g)), counter_room(*d, sp.workspaceBytes));
-            if (t.rows) {
+            // (a call that takes the kept rows' int32 block as well and would run in k slices runs in k slices, as the query says; whole small
+            // tiles would be faster: 203x1792x4096 with all rows kept 18.5 / 10.8 us, 512x1024x1024 of two ranks 12.8 / 6.3)
+            const bool sliced = blocks ? g.fx.slices > 1 : sp.f > 1;
+            if (t.rows && !(a.cAccum != nullptr && sliced && small.fx.slices <= 1)) {
                 launched(launch_small(DT_I8, small, t, stream));
                 return true;
             }

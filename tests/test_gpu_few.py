@@ -19,7 +19,7 @@ def ran():
     """The tiles that the last launch ran, as the cases name them: those of another kernel than this file's with its name, k slices behind a stroke,
     256x256 ones beside 128x128 ones."""
     i = L.last_launch()
-    kernel = {L.KERNEL_SMALL: "", L.KERNEL_FLEXIBLE: "flexible ", L.KERNEL_ALIGNED: "aligned "}[i.kernel]
+    kernel = {L.KERNEL_SMALL: "", L.KERNEL_FLEXIBLE: "flexible ", L.KERNEL_ALIGNED: "aligned ", L.KERNEL_STREAMING: "streaming "}[i.kernel]
     assert (i.largeTiles != 0) == (i.kernel == L.KERNEL_SMALL and i.tileRows == 256)
     return "%s%dx%d%s%s" % (kernel, i.tileRows, i.tileCols, "/%d" % i.kSlices if i.kSlices > 1 else "", " dealt" if i.dealt else "")
 
@@ -367,6 +367,43 @@ def test_quant_few_rows_of_a_long_k(case):
     for p in peers:
         y = y + p
     assert torch.equal(out, y.bfloat16())
+
+
+# (rows, N, K, P, first kept row, kept rows, weights as [n,k], int32 peers, checksums, tiles): the kept rows' int32 block from every tile, whole and in k
+# slices; where the streaming kernels or flexible tiles would run k slices, whole small tiles are not taken
+@pytest.mark.parametrize("case", [(46, 3360, 15872, 8, 40, 6, False, False, True, "32x32"), (129, 516, 648, 8, 128, 1, True, True, True, "32x32"),
+                                  (8, 8192, 1024, 8, 0, 8, True, False, False, "32x32"), (300, 1284, 2416, 8, 260, 40, True, False, True, "32x64"),
+                                  (203, 1376, 84, 3, 50, 70, True, True, False, "32x64"), (286, 1964, 124, 5, 0, 286, True, False, False, "64x64"),
+                                  (336, 1696, 140, 3, 0, 336, False, True, False, "64x64"), (645, 2612, 1340, 2, 0, 300, True, True, True, "64x128"),
+                                  (447, 2816, 1056, 4, 100, 112, False, False, False, "64x128"), (700, 4608, 1296, 2, 130, 300, False, True, False, "128x128"),
+                                  (650, 4612, 1292, 3, 600, 50, True, False, True, "128x128"), (51, 1920, 12800, 4, 30, 13, True, False, True, "64x64/8"),
+                                  (64, 512, 8192, 8, 0, 8, True, True, False, "32x32/8"), (67, 640, 4992, 8, 0, 67, False, False, False, "32x32/4"),
+                                  (203, 4096, 1792, 8, 0, 203, True, False, False, "flexible 64x256/2"), (17, 384, 1344, 16, 3, 9, True, True, False, "streaming 128x128/4")])
+def test_quant_kept_rows_int32_block(case):
+    _need_gpu()
+    M, N, K, P, kb, kr, tb, ri, with_sums, tiles = case
+    g = torch.Generator(device="cuda:0").manual_seed(M + N)
+    x1, x2 = (torch.randint(-127, 128, shape, dtype=torch.int8, device="cuda:0", generator=g) for shape in ((M, K), (K, N)))
+    s1, s2 = (torch.empty(c, device="cuda:0").uniform_(0.001, 0.02, generator=g) for c in (M, N))
+    b = torch.randint(-1000, 1000, (N,), dtype=torch.int32, device="cuda:0", generator=g)
+    peers = [torch.randint(-2 ** 20, 2 ** 20, (kr, N), dtype=torch.int32, device="cuda:0", generator=g) if ri else torch.randn((kr, N), device="cuda:0", generator=g)
+             for _ in range(P - 1)]
+    acc = (x1.double() @ x2.double()).to(torch.int64) + b
+    others = acc.clone()
+    others[kb:kb + kr] = 0
+    sums = torch.stack([others[r:r + 128, c:c + 128].sum() for r in range(0, M, 128) for c in range(0, N, 128)])
+    block = acc[kb:kb + kr].to(torch.int32) + (sum(peers) if ri else 0)
+    y = (block.float() * s2) * s1[kb:kb + kr, None]
+    for p in ([] if ri else peers):
+        y = y + p
+    ws = torch.zeros(max(ops.splitk_plan(M, K, N, P, kb, kr)[0], 65536), dtype=torch.uint8, device="cuda:0")
+    cs = torch.full((sums.numel(),), -7, dtype=torch.int64, device="cuda:0") if with_sums else None
+    ca = torch.full((kr + 1, N), -7, dtype=torch.int32, device="cuda:0")
+    out = ops.quant_matmul_splitk(x1, x2.T.contiguous() if tb else x2, s1, s2, b, peers, P, kb, kr, workspace=ws, checksum=cs, c_accum=ca, trans_b=tb, reduce_int32=ri)
+    assert ran() == tiles
+    torch.cuda.synchronize()
+    assert torch.equal(ca[:kr], block) and (ca[kr] == -7).all() and torch.equal(out, y.bfloat16()) and not ws[:65536].any()
+    assert cs is None or torch.equal(cs, sums)
 
 
 def sliced_workspace(need):
