@@ -760,8 +760,11 @@ int make_plan(int commType, int dataType, const CocTilingParams *t, const Catcoc
             (kBytes <= 1024 || (tiles64 > 128u && (kBytes <= 2048 || nPeers > 1 || transB))) && split_kept_tiles(a, (uint32_t)(kBytes / 64)) != 0)
             plan.preferFlex = false;
         a.flags = flags;
-        // (four slices or more of ragged rows or columns with B as [k,n]: a caller's count of them and the library's own give the same bits)
-        if (plan.preferFlex && plan.edge && !transB && a.fx.slices >= 4) plan.maySmall = false;
+        // (Floats on ragged rows or columns, B as [k,n], four slices or more: these run the count that the query reports, so that a caller who names it
+        // has the bits of one who leaves it open.  All others may run small tiles, which add in another order.  What that holds back, flexible /
+        // small tiles, us, bf16 all-reduce of eight ranks: 257x4096x512 14.3 / 9.9, 300x2048x1032 15.8 / 10.0, 131x8192x1288 17.8 / 19.6.  Whole numbers
+        // are the same in any order: W8A8 290x2496x736 12.7 -> 7.7, two ranks 500x3776x640 15.1 -> 9.2, 30 calls take 0.58 to 0.97 of their time)
+        if (plan.preferFlex && plan.edge && !transB && es != 1 && a.fx.slices >= 4) plan.maySmall = false;
     }
     plan.counters = counter_block(*d);
     plan.room = counter_room(*d, plan.kSliceBytes);

@@ -406,6 +406,36 @@ def test_quant_kept_rows_int32_block(case):
     assert cs is None or torch.equal(cs, sums)
 
 
+# (rows per rank, N, K, P): ragged rows or columns against [k,n] weights, of floats four k slices or more (test_ragged_launch_takes_the_slice_count_its_query_reports)
+@pytest.mark.parametrize("case", [(145, 736, 2496, 2, "32x32"), (250, 640, 3776, 2, "32x64"), (284, 576, 3776, 4, "64x64"), (160, 544, 7232, 1, "32x32/3")])
+def test_quant_ragged_slices_or_small_tiles(case):
+    """Whole numbers: a caller's slice count and the library's small tiles leave the same bits."""
+    _need_gpu()
+    rows, N, K, P, tiles = case
+    M, rank = rows * P, P - 1
+    g = torch.Generator(device="cuda:0").manual_seed(M + N)
+    x1, x2 = (torch.randint(-127, 128, shape, dtype=torch.int8, device="cuda:0", generator=g) for shape in ((M, K), (K, N)))
+    s1, s2 = (torch.empty(c, device="cuda:0").uniform_(0.001, 0.02, generator=g) for c in (M, N))
+    peers = [torch.randn((rows, N), device="cuda:0", generator=g) for _ in range(P - 1)]
+    t = ops.default_tiling(M, K, N, P, m0=0, n0=0, k0=0)
+    d = L.make_desc(rank, P, [16] * (P - 1))
+    size = L.load().catcoc_get_workspace_size(L.QUANT_MATMUL_REDUCE_SCATTER, L.INT8, C.byref(t), C.byref(d)) // 4
+    need, f = ops.kslice_plan(L.QUANT_MATMUL_REDUCE_SCATTER, torch.int8, M, K, N, rank, P)
+    assert f >= 4
+    y = ((x1[rank * rows:].double() @ x2.double()).float() * s2) * s1[rank * rows:, None]
+    for p in peers:
+        y = y + p
+    got = []
+    for split_k, kind in ((0, tiles), (f, "flexible 64x256/%d" % f)):
+        ws, ob = torch.zeros(need, dtype=torch.uint8, device="cuda:0"), torch.full((size,), 3.0, device="cuda:0")
+        out = ops.quant_matmul_reduce_scatter(x1, x2, s1, s2, None, peers, rank, P, tiling=t, outbound=ob, workspace=ws, split_k=split_k)
+        assert ran() == kind
+        torch.cuda.synchronize()
+        assert torch.equal(out, y.bfloat16())
+        got.append(ob)
+    assert torch.equal(got[0], got[1])
+
+
 def sliced_workspace(need):
     """A workspace of more than the query asks for: counters at zero, marks behind what a launch may touch."""
     ws = torch.zeros(need + 4096, dtype=torch.uint8, device="cuda:0")
