@@ -320,12 +320,11 @@ CallSize call_size(const GemmArgs &a, uint32_t es)
     return {rows, kB / 1024.0, 1e-6 * kB * (a.N + rows), 1e-6 * a.N * (4.0 * a.nPeers * a.keptRows + (a.sched.op == OP_REDUCE_SCATTER ? 4.0 : 2.0) * rows)};
 }
 
-// 128-row tiles of the aligned kernels (256-row ones: rounds of one workgroup per CU at the rate of long loops).
+// 128-row tiles of the aligned kernels (launches of 256-row ones run nothing else).
 double aligned_us(const GemmArgs &a, uint32_t es)
 {
     const CallSize c = call_size(a, es);
     const double f = a.splitK > 1 ? a.splitK : 1.0, wgs = a.sched.coreLoops * f, rounds = ceil(wgs / 256.0), steps = c.kib * 16.0 / f;
-    if (a.sched.m0 == 256) return 10.0 + 0.78 * rounds * steps;
     return 6.6 + rounds * (steps * (0.325 + (a.transB ? 0.060 : 0.0) - (es == 1 ? 0.019 : 0.0)) - 2.0) + (wgs > 512.0 ? 0.104 * (wgs / 256.0 - 2.0) * steps : 0.0) +
            (f > 1.0 ? 10.0 : 0.0) + (a.sched.op == OP_REDUCE_SCATTER ? 1.88 * a.nPeers : 0.0) + 0.134 * c.moved + 0.505 * c.mb;
 }

@@ -128,7 +128,8 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     constexpr int A_DMA = BM / 16 / NW;  // 1 KiB copies per wave per stage
     constexpr int B_DMA = 16 / NW;
     constexpr int STEP_DMA = A_DMA + B_DMA;
-    constexpr int POOL = FX && WM == 2 ? FlexPool<MB, NS>::BYTES : FX ? 160 * 1024 : DmaPool<WM, NS, AQ, TB>::BYTES;
+    static_assert(!FX || WM == 2 || DmaPool<WM, NS, AQ, TB>::BYTES <= FLEX_POOL8, "the rings of eight waves fit");
+    constexpr int POOL = FX && WM == 2 ? FlexPool<MB, NS>::BYTES : FX ? FLEX_POOL8 : DmaPool<WM, NS, AQ, TB>::BYTES;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;

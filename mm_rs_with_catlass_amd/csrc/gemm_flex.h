@@ -136,7 +136,8 @@ enum : uint32_t { FX_SKIP = 0u, FX_KEPT = 1u << 30, FX_OUT = 2u << 30, FX_SUM = 
 
 constexpr int FLEX_STAGING = 4 * 16384;                 // one 16 KiB area per wave
 constexpr int FLEX_POOL = FLEX_STAGING + 128 * 8 + 16 * 8 * 8 + 16 * 4;   // + the row table + the sums of up to 16 tasks, per half wave
-constexpr int FLEX_POOL8 = 2 * FLEX_STAGING + 256 * 8 + 16 * 16 * 8 + 16 * 4;   // of eight waves and 256 rows
+constexpr int FLEX_POOL8 = 160 * 1024;   // of eight waves and 256 rows (mixed launches): the rings, all of the LDS
+static_assert(2 * FLEX_STAGING + 256 * 8 + 16 * 16 * 8 + 16 * 4 <= FLEX_POOL8, "the epilogue of eight waves fits");
 
 // Sums over lanes, always in the same order: cross-lane adds in the vector unit (a shuffle is a trip through the LDS unit).
 template <int CTRL, int ROWS, typename T>

@@ -22,7 +22,8 @@ namespace catcoc {
 template <uint32_t DT, bool TB>
 __global__ void __launch_bounds__(512, 1) gemm_mixed_kernel(const GemmArgs args)
 {
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[160 * 1024];
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[FLEX_POOL8];
+    static_assert(MidGeom<2>::POOL <= FLEX_POOL8, "the small tiles fit");
     const FlexParams &f = args.fx;
     if (blockIdx.x < f.largeTiles) {
         dma_tile<DT, 4, TB, false, false, false, 2, 3, false, false, false, 1>(args, smem, blockIdx.x, 0, 1u, 0);

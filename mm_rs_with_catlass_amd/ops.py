@@ -46,6 +46,9 @@ def _stream():
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())   # of torch.cuda.current_stream(), without the object around it
 
 
+_DECODE = 4   # the W8A8 operator with explicit kept rows, beside the four CocCommTypes (host_call.cpp)
+
+
 def _call(*args):
     """The operator call in csrc/host_call.cpp, which takes this name's place: the output, or None where the call is one for the code below it."""
     global _call
@@ -306,7 +309,7 @@ def quant_matmul_splitk(x1, x2, scale_x1, scale_x2, bias=None, peers=(), rank_si
                         workspace=None, checksum=None, acc_dump=None, c_accum=None, peer_row_offset=0, block_num=0, swizzle=None, out=None, n0=0, trans_b=False,
                         reduce_int32=False):
     """One launch of prepare_quant_matmul_splitk(); returns d_out [kept_rows, n]."""
-    done = _call(4, x1, x2, scale_x1, scale_x2, bias, peers, 0, rank_size, None, False, trans_b, peer_row_offset, _l.FLAG_REDUCE_INT32 if reduce_int32 else 0, None,
+    done = _call(_DECODE, x1, x2, scale_x1, scale_x2, bias, peers, 0, rank_size, None, False, trans_b, peer_row_offset, _l.FLAG_REDUCE_INT32 if reduce_int32 else 0, None,
                  checksum, acc_dump, c_accum, workspace, out, out_dtype, block_num, 0, swizzle, split_k, kept_row_begin, kept_rows, n0)
     if done is not None:
         return done
