@@ -42,10 +42,10 @@ struct FlexParams {
     FastDiv dRank;                 // rows of one rank
     uint32_t hole0, holeRows;      // mixed launches (gemm_mixed.h): rows [hole0, +holeRows) run on the small tiles, `rows` counts the others
     uint32_t largeTiles;           // workgroups that run a 256x256 tile
-    uint32_t keptInHole;           // every kept row is one of the hole's
     uint32_t dealRows, dealRest;   // 128-column tiles with a reduce-scatter's kept rows dealt out evenly (deal_begin; 0 rows: tiles of consecutive rows):
     uint32_t dealKept, dealKeptRest;   // rows, and kept rows, of a row tile, and how many of the first row tiles have one more
     uint32_t sumParts;             // small tiles, sums of floats: places per task for what its tiles add
+    uint32_t keptInHole;           // mixed launches: every kept row is one of the hole's
 };
 
 // First of the rows that tile t is dealt: `each` to every tile, one more to the first `rest`.
