@@ -318,7 +318,12 @@ CATCOC_API uint64_t catcoc_get_workspace_size(int commType, int dataType, const 
  *  - A count of one with some bytes: a reduce-scatter launch whose kept rows meet their peers in a second launch when it is
  *    given them.
  * Float partials are added in slice order, so results are reproducible for any count.  A launch slices only when
- * `workspace` is given.  Counterpart in the reference: SplitkMatmul's k split
+ * `workspace` is given.  The bytes are an upper bound and the count is what the aligned or flexible kernels would take: a launch that leaves
+ * tiles, slices and order to the library may run small or mixed tiles instead (catcoc_last_launch() tells), whole or in
+ * slices of their own inside these bytes, and with checksums uses the counter block for sums that several tiles add up.  Small tiles add
+ * floats in another order than a caller's own count does; of ragged float launches with B as [k,n] and four slices or more the
+ * library runs the count reported, bit for bit what a caller who names it gets.  Equal rows of a float call have equal local sums wherever they lie, except
+ * in mixed launches, whose two kinds of tiles add in different orders.  Counterpart in the reference: SplitkMatmul's k split
  * (3rdparty/catlass/include/catlass/gemm/kernel/splitk_matmul.hpp:68-148), which its communication kernels do not
  * use. */
 CATCOC_API uint64_t catcoc_get_kslice_workspace_size(int commType, int dataType, const CocTilingParams *tiling,
@@ -329,11 +334,13 @@ CATCOC_API uint64_t catcoc_get_kslice_workspace_size(int commType, int dataType,
  * tile and receives the sum of the accumulators of the tile's rows that are not kept).  The path takes int8 A [m,k]
  * and B [k,n] (or, with transB, [n,k]: a weight matrix stored output-major), peers [keptRows, n] as fp32 added after
  * the dequantisation or, with CATCOC_FLAG_REDUCE_INT32, int32 added before it.  k in whole 64-byte steps and n in whole
- * 128-column tiles run the streaming kernels, or flexible tiles (64 x 256, k slices in the same workspace) where those are
- * faster; any other k and n that are multiples of four run flexible tiles over the whole k, without a workspace, and the rest a
- * one-thread-per-element kernel (correct, slow).  At most 32 rows against B as [n,k] (k in whole 128-byte chunks, desc->splitK 0 or 1, no
- * `checksum`) need no k split at all: one workgroup per 32 columns walks the whole k range, and such a launch neither needs
- * nor touches the workspace, whatever this query (which does not know the layout) reports.  CATCOC_OUTBOUND_STORE does not apply (explicit kept rows have no rank structure to lay
+ * 128-column tiles run the streaming kernels, flexible tiles (64 x 256, k slices in the same workspace) or small ones (whole, or in k slices
+ * in the same workspace) by what is faster; any other k and n that are multiples of four run small or flexible tiles over the whole
+ * k, and the rest a one-thread-per-element kernel (correct, slow).  Small tiles need the counter block of a workspace where checksums are
+ * asked for (64 KiB, also where 0 bytes are reported), else flexible tiles run.  At most 32 rows against B as [n,k] (k in whole 128-byte
+ * chunks, desc->splitK 0 or 1, no `checksum`) need no k split at all: one workgroup per 32 columns walks the whole k range,
+ * on 32 x 32 tiles or in deeper rings where k is long, and such a launch neither needs nor touches the workspace, whatever this query
+ * (which does not know the layout) reports.  The split factor reported is that of the streaming kernels.  CATCOC_OUTBOUND_STORE does not apply (explicit kept rows have no rank structure to lay
  * tiles out by).  It stands in for SplitkMatmul (3rdparty/catlass/include/catlass/gemm/kernel/splitk_matmul.hpp:68-330)
  * in front of the dequant / reduce epilogue. */
 CATCOC_API uint64_t catcoc_get_splitk_workspace_size(const CocTilingParams *tiling, const CatcocSymmetricDesc *desc,

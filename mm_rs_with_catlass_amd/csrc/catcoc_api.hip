@@ -294,9 +294,8 @@ bool flex_ptrs_ok(const GemmArgs &a)
 // and 0.16.  The choice takes the tiles with the least, where that is at most the share below of the others' estimate: beyond it calls
 // start to lose (aligned tiles at 0.9: up to 0.15, flexible ones at 1.0: up to 0.3), up to it three of 413 lost more than 0.04.  Calls
 // that had aligned tiles take 0.82 of their time, those that had flexible ones 0.78; the best choice for each would be 0.79 and 0.76.
-// Some of them, other kernels -> 32x32 .. 64x64, 64x128 or 128x128 tiles: bf16 16x1024x8192 of eight ranks 12.9 -> 7.4, W8A8
-// 203x1792x4096 19.7 -> 13.8, fp16 3167x9856x640 182 -> 77, bf16 649x9984x4096 185 -> 83, all-gather 278x4736x4864 of two 87 -> 46, W8A8
-// 760x7264x3072 68 -> 45; the other way round fp16 1116x4000x4160 78 / 92, 8144x5120x1696 188 / 203.  -> mixed: see gemm_mixed.h.
+// Figures of calls stand with the kernels that run them (gemm_few.h, gemm_mid.h, gemm_mixed.h); the other way round, other kernels / small tiles: fp16
+// 1116x4000x4160 78 / 92 us, 8144x5120x1696 on small tiles alone 188 / 203.
 constexpr double kAlignedShare = 0.85, kOtherShare = 0.87;
 struct SmallTile {
     int rows, cols;   // 0: the launch is not one for them; 256x256: the large ones of a mixed launch
@@ -761,7 +760,7 @@ int make_plan(int commType, int dataType, const CocTilingParams *t, const Catcoc
         a.flags = flags;
         // (Floats on ragged rows or columns, B as [k,n], four slices or more: these run the count that the query reports, so that a caller who names it
         // has the bits of one who leaves it open.  All others may run small tiles, which add in another order.  What that holds back, flexible /
-        // small tiles, us, bf16 all-reduce of eight ranks: 257x4096x512 14.3 / 9.9, 300x2048x1032 15.8 / 10.0, 131x8192x1288 17.8 / 19.6.  Whole numbers
+        // small tiles, us, operands in the caches, bf16 all-reduce of eight ranks: 257x4096x512 14.3 / 9.9, 300x2048x1032 15.8 / 10.0, 131x8192x1288 17.8 / 19.6.  Whole numbers
         // are the same in any order: W8A8 290x2496x736 12.7 -> 7.7, two ranks 500x3776x640 15.1 -> 9.2, 30 calls take 0.58 to 0.97 of their time)
         if (plan.preferFlex && plan.edge && !transB && es != 1 && a.fx.slices >= 4) plan.maySmall = false;
     }
@@ -871,9 +870,9 @@ int make_splitk_plan(const CocTilingParams *t, const CatcocSymmetricDesc *d, uin
     const uint32_t P = d->rankSize;
     if (P == 0 || P > CATCOC_MAX_RANKS) return fail(E_RANK, "rankSize %u out of range 1..%d", P, CATCOC_MAX_RANKS);
     if (transA) return fail(E_SHAPE, "the explicit-kept-rows (split-K) path takes A as [m,k] (B as [k,n] or, with transB, as [n,k])");
-    // shapes the two fast routes cannot take (k not in whole 64-byte steps, n not in whole 128-column tiles) run flexible tiles
-    // where k and n are multiples of four, else the one-thread-per-element kernel on the 128x128 grid, a correctness path: whole
-    // tiles and no workspace either way
+    // shapes the two fast routes cannot take (k not in whole 64-byte steps, n not in whole 128-column tiles) run small or
+    // flexible tiles where k and n are multiples of four, else the one-thread-per-element kernel on the 128x128 grid, a correctness path:
+    // whole tiles and nothing behind the counter block either way
     sp.general = t->k % 64 != 0 || t->n % 128 != 0;
     sp.wholeK = false;
     sp.preferFlex = false;
@@ -928,7 +927,7 @@ int make_splitk_plan(const CocTilingParams *t, const CatcocSymmetricDesc *d, uin
         a.sched = make_sched(OP_ALLREDUCE, t->m, t->n, 1, 128, 256, cores, 1, stages, off, dir);
         a.flags |= GF_ROW_MASK;
         sp.rowBlocks = 4;
-        // (whole tiles: the query promises that such a launch touches no workspace)
+        // (whole tiles: the query asks for no workspace; of one that is there small tiles use the counter block, for sums that meet)
         sp.flexBlocks = plan_flex(a, 1, a.checksum != nullptr, 0, 1);
         sp.f = 1;
         sp.workspaceBytes = 0;
@@ -1110,8 +1109,9 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
         }
         if (sp.maySmall) {
             const SmallTile t = small_tile(small, 1, sp.wholeK ? 1e30 : kOtherShare * (blocks ? flex_us(g, 1, blocks) : streaming_us(g)), counter_room(*d, sp.workspaceBytes));
-            // (a call that takes the kept rows' int32 block as well and would run in k slices runs in k slices, as the query says; whole small
-            // tiles would be faster: 203x1792x4096 with all rows kept 18.5 / 10.8 us, 512x1024x1024 of two ranks 12.8 / 6.3)
+            // (a call that takes the kept rows' int32 block as well and would run in k slices runs in k slices, of one kind or the other: what its
+            // workspace query reports is held to be what runs there.  Whole small tiles would be faster: operands in the caches, 203x1792x4096 with
+            // all rows kept 18.5 / 10.8 us, 512x1024x1024 of two ranks 12.8 / 6.3)
             const bool sliced = blocks ? g.fx.slices > 1 : sp.f > 1;
             if (t.rows && !(a.cAccum != nullptr && sliced && small.fx.slices <= 1)) {
                 launched(launch_small(DT_I8, small, t, stream));

@@ -8,20 +8,21 @@
 // after which a thread holds four consecutive columns of a row and finishes them.  The peers' values of the tile's kept rows are
 // requested around the first copies, into registers, so that their stream and the operands' are in flight together on every CU.
 //
-// Bound by launch and latency (of 16x1024x8192's 7.4 us an empty launch is 2.7 and the chain arguments - copies - partial tiles -
+// Bound by launch and latency (of 16x1024x8192's 7.5 us an empty launch is 2.7 and the chain arguments - copies - partial tiles -
 // output about 2.5), past that by what reaches the CUs: 256 of them pull 60-85 GB/s each through their copies.  That is why a tile is
 // small rather than sliced: 64x256 tiles in k slices used 64 to 128 CUs, and the second launch that added the slices and the peers cost
-// 3.5 to 6 us.  GPU time per call, k slices and second launch -> this: bf16 16x1024x8192, eight ranks, 12.9 -> 7.4 us, fp16
-// 512x1024x1024, two ranks, 14.2 -> 8.4, W8A8 203x1792x4096, eight ranks, all rows kept, 19.7 -> 13.8 (33 MB, 23 of them the
-// peers'), off the 64-byte and 128-column grid 2x13472x2432 57 -> 23, 46x15872x3360 144 -> 21; explicit kept rows with the others'
-// sums (MetSum) 2x1408x640 9.6 -> 5.9, 128x2416x1280 24 -> 8.7, 283x14256x1024 77 -> 29, 462x2336x1536 24 -> 12.6.  Which launches:
-// small_tile().
+// 3.5 to 6 us.  Time per call, calls behind each other and their operands out of HBM (more sets of them than the caches hold),
+// what ran these calls before (mostly 64x256 tiles in k slices and a second launch) -> this: bf16 16x1024x8192, eight ranks, 13.6 -> 7.5 us,
+// fp16 512x1024x1024, two ranks, 14.9 -> 7.3, W8A8 203x1792x4096, eight ranks, all rows kept, 21.1 -> 12.2 (33 MB, 23 of them the
+// peers'), off the 64-byte and 128-column grid 2x13472x2432 152 -> 18, 46x15872x3360 144 -> 21; explicit kept rows, an eighth of them, with the
+// others' sums (MetSum) 2x1408x640 11.6 -> 6.0, 128x2416x1280 46 -> 8.4, 283x14256x1024 195 -> 33, 462x2336x1536 44 -> 12.6.  Which
+// launches: small_tile().
 // Where even small tiles are fewer than half the CUs and k is long, a tile has up to eight workgroups, one k slice each (SL).  They meet in the
 // workspace: every slice leaves its partial tile there (4 to 16 KiB, past the caches that other XCDs do not see) and counts itself, and the last
 // to arrive adds all of them in slice order, then the peers, and writes the output.  That costs 2.2 us and the partials' trip through one CU,
-// against 5 for a second launch over 64x256 tiles' slices.  64x256 tiles and second launch -> this: bf16 7x11264x1024 of eight ranks 15.5 ->
-// 10.8 us, fp16 1x13256x1024 all-gather 18.2 -> 11.9, 44x6000x640 reduce-scatter of two 17.0 -> 10.0, W8A8 59x8960x512 14.5 -> 9.6,
-// 9x4864x512 with 3 rows kept, as [k,n], 11.5 -> 9.2, bf16 31x10784x2048 20.1 -> 16.6.
+// against 5 for a second launch over 64x256 tiles' slices.  64x256 tiles and second launch -> this, measured as above: bf16 7x11264x1024 of
+// eight ranks 18.0 -> 10.6 us, fp16 44x6000x640 reduce-scatter of two 16.1 -> 9.4, W8A8 59x8960x512 15.0 -> 8.4, 9x4864x512 with 3
+// rows kept, as [k,n], 14.3 -> 7.9, bf16 31x10784x2048 23.8 -> 16.0.
 // k is divided among the waves because that takes neither barriers nor a shared ring; what it costs is LDS reads (a 64x64 tile reads
 // two fragments per two MFMAs, all the LDS can give), so long loops over many tiles belong to the larger tiles.
 #pragma once
@@ -79,8 +80,9 @@ __device__ __forceinline__ MetSum block_add(const GemmArgs &args, uint32_t row0,
                    slices * ceil_div(umin(128u, rows - br * 128u), (uint32_t)BM) * ceil_div(umin(128u, args.N - bc * 128u), (uint32_t)BN), sum);
 }
 
-// Float reduce-scatters with checksums, tiles that line up with the tasks (and up to three launches) -> these: fp16 2904x2364x640 of eight
-// ranks 44 -> 25 us, bf16 664x3840x512 of four 63 -> 18, fp16 1084x3328x1536 51 -> 27; 70 drawn calls take 0.72 of their time.
+// Float reduce-scatters with checksums as [n,k], tiles that line up with the tasks (and up to three launches) -> these, measured as above: fp16
+// 2904x2364x640 of eight ranks 79 -> 34 us, bf16 664x3840x512 of four 82 -> 19, fp16 1084x3328x1536 74 -> 31; 70 drawn calls take 0.72 of
+// their time.
 // Sums of floats need an order: every tile's part has a place of its own (place of parts), an exchange puts it there and is through when it
 // returns, and the tile that counts last adds the parts in order and leaves zeros behind.
 __device__ __forceinline__ void sum_in_order(const GemmArgs &args, uint32_t task, uint32_t parts, uint32_t place, double sum)
@@ -181,7 +183,7 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
     __shared__ __attribute__((aligned(1024))) unsigned char smem[G::POOL];
 
     // The arguments come from host memory: named here, they arrive in a few wide loads behind one wait instead of one round trip
-    // each where they are used (16x1024x8192, bf16, eight ranks 7.7 -> 7.4 us).
+    // each where they are used (16x1024x8192, bf16, eight ranks, 0.3 us less).
     const void *peer[PF];
 #pragma unroll
     for (int p = 0; p < PF; ++p) peer[p] = args.peers[p];

@@ -15,8 +15,8 @@
 // k, the peers' stream for short k.  Measured against what ran these launches before (a kernel that staged its tiles through
 // registers, or one thread per output element), launches alternating: fp16 all-gather 8 x [1024,6148] x [6148,5120]
 // 243 ms -> 0.522 ms = 988 TFLOP/s (12296-byte rows, 8 bytes of k left over), W8A8 64x8192x8192 with 8 rows kept 22.7 -> 19.9 us.
-// Smaller launches are small tiles' (gemm_few.h, gemm_mid.h): W8A8 reduce-scatter 1000x1376x4096 of eight ranks, stored tiles, 277 us
-// before either, 26 here, 18 there, bf16 all-reduce 16x1024x8192 28.7, 13.0, 6.5.
+// Smaller launches are small tiles' (gemm_few.h, gemm_mid.h): W8A8 reduce-scatter 1000x1376x4096 of eight ranks, stored tiles, took 277 us
+// before either, bf16 all-reduce 16x1024x8192 28.7.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

@@ -8,15 +8,16 @@
 //
 // Bound by the matrix pipes at their power limit where the operands come out of the caches (0.47 us per chunk of a 128x128 tile, bf16 at
 // 1.09 GHz of MFMA issue, as the larger tiles' loops; without MFMAs the copies and reads alone take 0.32, without copies 0.35), by
-// HBM else (0.6), and by a fixed 5.5 us (launch apart) of first copies, partial tiles and output.  GPU time per call, other kernels -> this:
-// all-gather 8 x [512,4096] x [4096,1024] bf16 42.2 -> 39.6 us, fp16 683x7680x4864 153 -> 77, all-gather 278x4736x4864 of two 87 -> 46, W8A8
-// 499x9120x2048 with 63 rows kept 99 -> 51.  Which launches: small_tile().
+// HBM else (0.6), and by a fixed 5.5 us (launch apart) of first copies, partial tiles and output.  Time per call, calls behind each other and
+// their operands out of HBM, other kernels -> this: all-gather 8 x [512,4096] x [4096,1024] bf16 52.8 -> 44.6 us, fp16 all-reduce 683x7680x4864
+// of two ranks 157 -> 77, all-gather 278x4736x4864 of two 95 -> 47, W8A8 reduce-scatter 1000x1376x4096 of eight, stored tiles, 26.3 -> 18.1.
+// Which launches: small_tile().
 //
 // A reduce-scatter's kept rows are dealt out to all row tiles.  One CU draws no more than about 40 bytes a nanosecond out of HBM, so
 // tiles of kept rows only (448 KiB of peers each with eight ranks) take 12 us longer than their neighbours; in shares of 16 rows a tile
-// the peers are all in flight at once and take under 2.  Tiles of consecutive rows -> dealt: W8A8 1000x1376x4096 of eight ranks, stored
-// tiles, 26.9 -> 19.6 us (other kernels 28.1), 2000x1376x4096 48.3 -> 36.2 (37.2), fp16 2784x960x2816 46.4 -> 33.1 (48.0), of two ranks and
-// W8A8 1000x1376x4096 24.6 -> 19.3.
+// the peers are all in flight at once and take under 2.  Tiles of consecutive rows -> dealt, as these kernels were when rows were first dealt:
+// W8A8 1000x1376x4096 of eight ranks, stored tiles, 7 us less, 2000x1376x4096 48.3 -> 36.2 us (other kernels 37.2), fp16 2784x960x2816 46.4 ->
+// 33.1 (48.0), of two ranks and W8A8 1000x1376x4096 24.6 -> 19.3.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

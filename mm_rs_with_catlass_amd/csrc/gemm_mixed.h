@@ -7,10 +7,10 @@
 // kept ones and as many more as fill the CUs that the large tiles leave idle.  The large tiles start first.
 //
 // Bound by the matrix pipes at their power limit: a large tile takes 9 + 1.7 us per 128 bytes of k, a small one 8 + 0.55 (about 1.0
-// PFLOP/s in 16 bits where all CUs have work; a library product of 8192 cubed 1.15).  GPU time per call, 128-row tiles -> this: fp16
-// reduce-scatter 8144x5120x1696 of eight ranks, as [n,k] (7126 rows on 196 large tiles, the kept 1018 on 112 small ones beside them), 197
-// -> 170 us, W8A8 2680x3200x6912 120 -> 84, 1384x6080x7936 134 -> 88, 3824x5632x6400 216 -> 155, bf16 reduce-scatter 4236x4952x3904 of four
-// 280 -> 200, all-gather 8 x [845,3328] x [3328,3936] 217 -> 186.  Which launches: small_tile().
+// PFLOP/s in 16 bits where all CUs have work; a library product of 8192 cubed 1.15).  Time per call, calls behind each other and their
+// operands out of HBM, 128-row tiles -> this, reduce-scatters with stored tiles, as [n,k]: fp16 8144x5120x1696 of eight ranks (7126 rows on
+// 196 large tiles, the kept 1018 on 112 small ones beside them) 184 -> 168 us, W8A8 2680x3200x6912 124 -> 81, 1384x6080x7936 145 -> 85,
+// 3824x5632x6400 217 -> 157, bf16 4236x4952x3904 of four 284 -> 196.  Which launches: small_tile().
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

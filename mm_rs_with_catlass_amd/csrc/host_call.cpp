@@ -1,6 +1,6 @@
 // The ordinary call of an operator from Python, without the Python: operands checked, descriptor filled in, launcher called.
 //
-// A call of a small launch is bound by what it does on the host (16x1024x8192 bf16 all-reduce of eight ranks: 7.4 us on the GPU, 10.8 us per
+// A call of a small launch is bound by what it does on the host (16x1024x8192 bf16 all-reduce of eight ranks: 6 to 7.5 us on the GPU, 10.8 us per
 // call through Python and ctypes, of which the launch itself is 2.9).  call() takes the arguments of one operator call, and either launches
 // it or returns None without having done anything: it accepts only what it has checked to the last condition the Python path
 // checks, and everything else -- subclasses, wrapped tensors, numbers that are no Python integers, and all that is wrong -- goes through
