@@ -443,7 +443,7 @@ CATCOC_API uint32_t catcoc_tail_split_tiles(int commType, int dataType, const Co
 CATCOC_API int catcoc_launch_tile(int commType, const CocTilingParams *tiling, const CatcocSymmetricDesc *desc, uint32_t wg,
                                   uint32_t *task, uint32_t *targetRank, uint32_t *row, uint32_t *col, uint32_t *wsRow);
 /* What the GEMM launch of the calling thread's last accepted call ran (a call of several rounds: the last round), for tests that are
- * about one kernel and for tools.  No counterpart in the reference. */
+ * about one kernel and for tools.  NULL: nothing.  No counterpart in the reference. */
 enum {
     CATCOC_KERNEL_NONE = 0,
     CATCOC_KERNEL_GENERAL = 1,   /* bounds-checked kernels */

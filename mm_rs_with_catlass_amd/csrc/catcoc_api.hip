@@ -1748,7 +1748,10 @@ uint32_t catcoc_tail_split_tiles(int commType, int dataType, const CocTilingPara
     return plan_halves(commType, dataType, tiling, desc, transA, transB, p) ? 8u * split_tail_tiles(p.args, split_kept_tiles(p.args, p.args.K * elem_size(p.dtype) / 64u)) : 0u;
 }
 
-void catcoc_last_launch(CatcocLaunchInfo *info) { *info = g_launch; }
+void catcoc_last_launch(CatcocLaunchInfo *info)
+{
+    if (info != nullptr) *info = g_launch;
+}
 
 uint32_t catcoc_workgroup_task(uint32_t wg, uint32_t tasks, uint32_t flags)
 {

@@ -644,6 +644,13 @@ def test_kept_split_queries_of_launches_on_small_and_mixed_tiles(so):
     assert split(Q, L.INT8, 4096, 1792, 4096, 8, 1, store=False) == [64, 64] == split(Q, L.INT8, 4096, 1792, 4096, 8, 0, m0=128, n0=256)
 
 
+def test_last_launch_without_a_launch(so):
+    so.catcoc_last_launch(None)
+    info = L.CatcocLaunchInfo(kernel=9)
+    so.catcoc_last_launch(C.byref(info))
+    assert info.kernel in range(6)   # (0 unless this thread has launched something)
+
+
 def test_descriptor_takes_what_its_fields_take(so):
     # plain addresses are packed in one go; ctypes objects and numbers outside a field's range as ctypes takes them
     want = bytes(L.make_desc(3, 4, [16, 32, 48], peer_ld=8, outbound=64, outbound_bytes=128, checksum=256, acc_dump=512, flags=5))
