@@ -336,8 +336,8 @@ CATCOC_API uint64_t catcoc_get_kslice_workspace_size(int commType, int dataType,
  * the dequantisation or, with CATCOC_FLAG_REDUCE_INT32, int32 added before it.  k in whole 64-byte steps and n in whole
  * 128-column tiles run the streaming kernels, flexible tiles (64 x 256, k slices in the same workspace) or small ones (whole, or in k slices
  * in the same workspace) by what is faster; any other k and n that are multiples of four run small or flexible tiles over the whole
- * k, and the rest a one-thread-per-element kernel (correct, slow).  Small tiles need the counter block of a workspace where checksums are
- * asked for (64 KiB, also where 0 bytes are reported), else flexible tiles run.  At most 32 rows against B as [n,k] (k in whole 128-byte
+ * k, and the rest a one-thread-per-element kernel (correct, slow).  Where checksums are asked for, the sums of tiles smaller than a 128x128
+ * block meet in the counter block of a workspace (64 KiB, also where 0 bytes are reported); without one larger tiles run.  At most 32 rows against B as [n,k] (k in whole 128-byte
  * chunks, desc->splitK 0 or 1, no `checksum`) need no k split at all: one workgroup per 32 columns walks the whole k range,
  * on 32 x 32 tiles or in deeper rings where k is long, and such a launch neither needs nor touches the workspace, whatever this query
  * (which does not know the layout) reports.  The split factor reported is that of the streaming kernels.  CATCOC_OUTBOUND_STORE does not apply (explicit kept rows have no rank structure to lay
