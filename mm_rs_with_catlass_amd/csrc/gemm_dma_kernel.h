@@ -11,6 +11,7 @@
 
 #include "gemm_flex.h"
 #include "gemm_fused_kernel.h"
+#include "mfma16.h"
 
 namespace catcoc {
 
@@ -62,7 +63,7 @@ __device__ __forceinline__ void dma16_stream(const unsigned char *g, unsigned ch
 //
 // Geometries (every wave computes 64 x 128: MB = 2 row blocks of 32, 4 column blocks of 32; two wave columns):
 //   WM 2 -> 128x256 tile, 4 waves, 3 stages (72 KiB LDS, two workgroups per CU);
-//   WM 4 -> 256x256 tile, 8 waves (128 KiB LDS, one workgroup per CU): half the L2 -> LDS traffic per MAC.
+//   WM 4 -> 256x256 tile, 8 waves (128 KiB LDS, one workgroup per CU): half the L2 -> LDS traffic per MAC; on 16x16 MFMAs (mfma16.h).
 //   W8   -> the 128x256 tile on EIGHT waves (four wave rows of 32 rows, MB = 1; WM stays 2: every tile-level rule of the
 //           128-row geometry applies): for the six-stage ring, whose launches have one workgroup per CU -- with four waves
 //           every wave is alone on its SIMD and pays barrier, LDS latency and copy issue of every k step one after the other.
@@ -249,6 +250,12 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     // chunk slot^((row&7)<<1).  2-byte elements (32 k rows x 512 bytes): copy j covers k rows 2j, 2j+1; lane -> row
     // 2j + lane/32, slot lane&31 holds chunk slot^((row&3)<<2).
     // B given as [n][k]: copy j covers tile columns 16j..16j+15, one 64-byte row of k each, laid out like A.
+    // (256 rows: b16_slot() in the place of these swizzles)
+    auto b_slot = [](uint32_t row) -> uint32_t {
+        if constexpr (WM == 4) return b16_slot<ES>(row);
+        else if constexpr (ES == 1) return (row & 7u) << 1;
+        else return (row & 3u) << 2;
+    };
     const unsigned char *gB[B_DMA];
 #pragma unroll
     for (int jj = 0; jj < B_DMA; ++jj) {
@@ -260,19 +267,19 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
                 gB[jj] = Bg + (size_t)umin(16u * (w + NW * jj) + (lane >> 2), last) * ldbB + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
             } else if constexpr (ES == 1) {
                 const int row = 4 * (w + NW * jj) + (lane >> 4);
-                gB[jj] = Bg + (size_t)row * ldbB + (umin((lane & 15) ^ ((row & 7) << 1), last / 16u) * 16);
+                gB[jj] = Bg + (size_t)row * ldbB + (umin((lane & 15) ^ b_slot(row), last / 16u) * 16);
             } else {
                 const int row = 2 * (w + NW * jj) + (lane >> 5);
-                gB[jj] = Bg + (size_t)row * ldbB + (umin((lane & 31) ^ ((row & 3) << 2), last / 8u) * 16);
+                gB[jj] = Bg + (size_t)row * ldbB + (umin((lane & 31) ^ b_slot(row), last / 8u) * 16);
             }
         } else if constexpr (TB) {
             gB[jj] = Bg + (size_t)(16 * (w + NW * jj) + (lane >> 2)) * ldbB + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
         } else if constexpr (ES == 1) {
             const int row = 4 * (w + NW * jj) + (lane >> 4);
-            gB[jj] = Bg + (size_t)row * ldbB + (((lane & 15) ^ ((row & 7) << 1)) * 16);
+            gB[jj] = Bg + (size_t)row * ldbB + (((lane & 15) ^ b_slot(row)) * 16);
         } else {
             const int row = 2 * (w + NW * jj) + (lane >> 5);
-            gB[jj] = Bg + (size_t)row * ldbB + (((lane & 31) ^ ((row & 3) << 2)) * 16);
+            gB[jj] = Bg + (size_t)row * ldbB + (((lane & 31) ^ b_slot(row)) * 16);
         }
     }
     const size_t bStep = TB ? (size_t)64 : (size_t)(64 / ES) * ldbB;
@@ -285,12 +292,14 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     };
 
     Acc acc[MB][4];
+    if constexpr (WM == 2) {
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
+        for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb)
+            for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[mb][nb][r] = 0;
+                for (int r = 0; r < 16; ++r) acc[mb][nb][r] = 0;
+    }
 
     // fragment addresses
     // 1-byte transpose read: within a 16-lane group, lane i supplies 8 bytes of k row (i>>1), column half (i&1)
@@ -316,14 +325,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     constexpr int B_KK = (ES == 1) ? 32 * 256 : 16 * 512;     // bytes of a stage per 32-byte k slab
     constexpr int B_HALF = (ES == 1) ? 8 * 256 : 4 * 512;     // second transpose read of a fragment
     const uint32_t bt_lds = (wn * 128 + c32) * 64, bt_sw = (c32 >> 2) & 3;   // [n][k] stage: row of column c32, chunk swizzle
-    // 256-row tile with B as [n][k]: B sits in pair buffers like A (rows of 128 bytes, two k steps); bpar = step of the pair
-    uint32_t bpar = 0;
-    const uint32_t bp4_lds = (wn * 128 + c32) * 128, bp4_sw = (c32 >> 1) & 7;
     auto read_b1 = [&](v4i (&bf)[4], const unsigned char *sb, int kk, int nb) {
-        if constexpr (TB && WM == 4) {
-            bf[nb] = *(const v4i *)(sb + bp4_lds + nb * 32 * 128 + (((bpar * 4 + 2 * kk + h) ^ bp4_sw) * 16));
-            return;
-        }
         if constexpr (TB) {
             bf[nb] = *(const v4i *)(sb + bt_lds + nb * 32 * 64 + (((2 * kk + h) ^ bt_sw) * 16));
             return;
@@ -442,6 +444,74 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     };
 #undef CATCOC_MMA
     auto nothing = [] {};
+    // 256 rows: 16x16 MFMAs (mfma16.h), 4 x 8 blocks per wave.  A step's 32 MFMAs lag its fragment reads by half a step as well: the first
+    // sixteen are columns 64 .. 127 of the step before, behind which this step's fragments of A and of columns 0 .. 63 are read, the second
+    // sixteen those columns, behind which the fragments of the others are.
+    typename Acc16Of<DT>::type a16[WM == 4 ? 4 : 1][8];
+    v4i ra[2][4], rbl[4], rbh[4];   // A of a step's parity, B's lower and upper four column blocks
+    const uint32_t l16 = lane & 15, quad = lane >> 4;
+    if constexpr (WM == 4) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) a16[i][j][r] = 0;
+    }
+    auto upper16 = [&](const v4i (&af)[4], auto between) {
+#pragma unroll
+        for (int m = 0; m < 16; ++m) {
+            const int j = m / 4, i = snake16(j, m % 4, 4);
+            a16[i][4 + j] = mfma16<DT>(af[i], rbh[j], a16[i][4 + j]);
+            CATCOC_FENCE();
+            between(m);
+            CATCOC_FENCE();
+        }
+    };
+    auto lower16 = [&](const v4i (&af)[4], auto between) {
+#pragma unroll
+        for (int m = 0; m < 16; ++m) {
+            const int j = m / 4, i = snake16(j, m % 4, 4);
+            a16[i][j] = mfma16<DT>(af[i], rbl[j], a16[i][j]);
+            CATCOC_FENCE();
+            between(m);
+            CATCOC_FENCE();
+        }
+    };
+    // read_a(i), read_b(j): fragments of this step; copyA, copyB: the step's copies.  The two waves that share a SIMD (w and w + 4) issue
+    // them in different halves of the step, so that one of them always has MFMAs to feed the matrix pipe while the other computes addresses.
+    auto step16 = [&](auto PAR, auto read_a, auto read_b, auto copyA, auto copyB) {
+        constexpr int par = decltype(PAR)::value;
+        const bool early = ws < NW / 2;
+        upper16(ra[1 - par], [&](int m) {
+            if (m == 0) rbl[0] = read_b(0);
+            else if (m < 9 && m % 2 == 0) ra[par][m / 2 - 1] = read_a(m / 2 - 1);
+            else if (m == 10 || m == 12 || m == 14) rbl[(m - 8) / 2] = read_b((m - 8) / 2);
+            if (m == 9 && early) copyA();
+            if (m == 13 && early) copyB();
+        });
+        lower16(ra[par], [&](int m) {
+            if (m < 8 && m % 2 == 0) rbh[m / 2] = read_b(4 + m / 2);
+            if (m == 9 && !early) copyA();
+            if (m == 13 && !early) copyB();
+        });
+    };
+    auto barrier16 = [] {   // (the last fragments' reads are long back: sixteen MFMAs were issued since)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        barrier_keep_vmem();
+    };
+    auto first16 = [&](auto read_a, auto read_b) {   // step 0: no MFMAs pending yet
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ra[0][i] = read_a(i);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) rbl[j] = read_b(j);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) rbh[j] = read_b(4 + j);
+        CATCOC_FENCE();
+        lower16(ra[0], [](int) {});
+    };
+    std::integral_constant<int, 0> EVEN{};
+    std::integral_constant<int, 1> ODD{};
     // Flexible mode on 256 rows: what whole pairs of steps leave of k (up to 128 bytes per row) comes first, through registers with
     // bounds checks into the LDS of A's first pair and of B's first pair or two stages.
     auto tail_pair = [&](unsigned char *sa, unsigned char *sb, auto read_a, auto read_b) {
@@ -459,18 +529,14 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             } else {
                 constexpr int CH = 256 * ES / 16;   // pieces of a row of k; the stages of both steps lie behind each other
                 const int r = idx / CH, cb = (idx % CH) * 16, rows = tail / ES, width = ti.colsValid * ES;
-                *(v4i *)(sb + r * (256 * ES) + (((idx % CH) ^ (ES == 1 ? (r & 7u) << 1 : (r & 3u) << 2)) * 16)) =
+                *(v4i *)(sb + r * (256 * ES) + (((idx % CH) ^ b_slot(r)) * 16)) =
                     load16_guarded(b + (kEnd / ES + (r < rows ? r : rows - 1)) * ldbB + (size_t)ti.col * ES + cb, r < rows ? width - cb : 0, width - 4 - cb);
             }
         }
         __syncthreads();
         for (uint32_t t = 0; t < (tail > 64 ? 2u : 1u); ++t) {
-            read_a(fa0, t, 0);
-            read_b(fb0, t, 0);
-            read_a(fa1, t, 1);
-            read_b(fb1, t, 1);
-            mma(fa0, fb0);
-            mma(fa1, fb1);
+            first16([&](int i) { return read_a(t, i); }, [&](int j) { return read_b(t, j); });
+            upper16(ra[0], [](int) {});
         }
         __syncthreads();   // (the prologue's copies land here)
     };
@@ -779,13 +845,10 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
                 gQ[jj] += 128;
             }
         };
-        const uint32_t ap_lds = (wm * 32 * MB + c32) * 128;
-        const uint32_t ap_sw = (c32 >> 1) & 7;
-        auto load_ap = [&](v4i (&af)[MB], uint32_t kt, int kk) {
-            const unsigned char *sa = stAP(kt >> 1) + ap_lds + ((((kt & 1) * 4 + 2 * kk + h) ^ ap_sw) * 16);
-#pragma unroll
-            for (int mb = 0; mb < MB; ++mb) af[mb] = *(const v4i *)(sa + mb * 32 * 128);
-        };
+        // row (column) block i (j): rows 16 i + (lane & 15), piece 4 * (step of the pair) + (lane >> 4)
+        const uint32_t piece16 = l16 * 128 + ((quad ^ (l16 >> 1)) * 16);
+        auto read_ap = [&](uint32_t q, uint32_t par, int i) { return *(const v4i *)(stAP(q) + wm * 64 * 128 + (piece16 ^ (par * 64)) + i * 16 * 128); };
+        auto read_bp = [&](uint32_t q, uint32_t par, int j) { return *(const v4i *)(stBP(q) + wn * 128 * 128 + (piece16 ^ (par * 64)) + j * 16 * 128); };
         auto issue_even_a = [&](uint32_t kt, bool guard) {
             if ((kt & 1) == 0 && (!guard || kt + 2 < nk)) issue_ap((kt + 2) >> 1);
         };
@@ -793,8 +856,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             if ((kt & 1) == 0 && (!guard || kt + 4 < nk)) issue_bp((kt + 4) >> 1);
         };
         if constexpr (FX) {
-            if (args.fx.tail != 0) tail_pair(stAP(0), stBP(0), [&](v4i (&af)[MB], uint32_t t, int kk) { load_ap(af, t, kk); },
-                                             [&](v4i (&bf)[4], uint32_t t, int kk) { bpar = t; load_b(bf, stBP(0), kk); });
+            if (args.fx.tail != 0) tail_pair(stAP(0), stBP(0), [&](uint32_t t, int i) { return read_ap(0, t, i); }, [&](uint32_t t, int j) { return read_bp(0, t, j); });
         }
         // prologue in steady-state order: A pair 0, B pairs 0 and 1
         issue_ap(0);
@@ -803,47 +865,33 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
         // step 0 (peeled: no MFMAs pending yet)
         if (nk > 2) CATCOC_WAIT_VMCNT(APC);
         else CATCOC_WAIT_VMCNT(0);
-        barrier_keep_vmem();
+        barrier16();
         issue_even_a(0, true);
         issue_even_b(0, true);
-        bpar = 0;
-        load_ap(fa0, 0, 0);
-        load_b(fb0, stBP(0), 0);
-        load_ap(fa1, 0, 1);
-        load_b(fb1, stBP(0), 1);
-        CATCOC_FENCE();
-        mma(fa0, fb0);
-        CATCOC_FENCE();
-
-        auto compute = [&](uint32_t kt, bool guard) {
-            // The two waves that share a SIMD (w and w + 4) issue their copies in different halves of the step,
-            // so that one of them always has MFMAs to feed the matrix pipe while the other computes addresses.
-            const bool early = ws < NW / 2;
-            bpar = kt & 1u;
-            sched_step([&](v4i (&af)[MB], int kk) { load_ap(af, kt, kk); }, stBP(kt >> 1),
-                       [&] { if (early) issue_even_a(kt, guard); }, [&] { if (early) issue_even_b(kt, guard); }, nothing,
-                       [&] {
-                           if (!early) {
-                               issue_even_a(kt, guard);
-                               issue_even_b(kt, guard);
-                           }
-                       });
+        first16([&](int i) { return read_ap(0, 0, i); }, [&](int j) { return read_bp(0, 0, j); });
+        auto compute = [&](auto PAR, uint32_t kt, bool guard) {
+            constexpr int par = decltype(PAR)::value;
+            const uint32_t q = kt >> 1;
+            step16(PAR, [&](int i) { return read_ap(q, par, i); }, [&](int j) { return read_bp(q, par, j); }, [&] { if (par == 0) issue_even_a(kt, guard); },
+                   [&] { if (par == 0) issue_even_b(kt, guard); });
         };
         uint32_t kt = 1;
         for (; kt + 6 <= nk; kt += 2) {   // (the even step kt + 1 issues A pair (kt+3)/2 and B pair (kt+5)/2 unguarded)
-            compute(kt, false);
+            compute(ODD, kt, false);
             CATCOC_WAIT_VMCNT(APC);
-            barrier_keep_vmem();
-            compute(kt + 1, false);
+            barrier16();
+            compute(EVEN, kt + 1, false);
         }
-        for (; kt < nk; ++kt) {   // tail: drain fully at every even step
-            if ((kt & 1u) == 0) {
+        for (; kt < nk; kt += 2) {   // tail: drain fully at every even step (steps come in pairs: kt is odd)
+            compute(ODD, kt, true);
+            if (kt + 1 < nk) {
                 CATCOC_WAIT_VMCNT(0);
-                barrier_keep_vmem();
+                barrier16();
+                compute(EVEN, kt + 1, true);
             }
-            compute(kt, true);
         }
-        mma(fa1, fb1);
+        upper16(ra[1], [](int) {});
+        acc16_to_32<DT>(a16, acc);
     } else {
         // ---- 256x256 ---------------------------------------------------------------------------------
         // B: four 64-row stages, copies issued three steps ahead.  A: two "pair" buffers of 256 rows x 128
@@ -879,12 +927,23 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             }
         };
         auto offB4 = [&](uint32_t step) { return 2 * AP + (step & 3) * B_STAGE; };
-        const uint32_t ap_lds = (wm * 32 * MB + c32) * 128;
-        const uint32_t ap_sw = (c32 >> 1) & 7;
-        auto load_ap = [&](v4i (&af)[MB], uint32_t kt, int kk) {
-            const unsigned char *sa = stAP(kt >> 1) + ap_lds + ((((kt & 1) * 4 + 2 * kk + h) ^ ap_sw) * 16);
-#pragma unroll
-            for (int mb = 0; mb < MB; ++mb) af[mb] = *(const v4i *)(sa + mb * 32 * 128);
+        const uint32_t piece16 = l16 * 128 + ((quad ^ (l16 >> 1)) * 16);
+        auto read_ap = [&](uint32_t kt, uint32_t par, int i) { return *(const v4i *)(stAP(kt >> 1) + wm * 64 * 128 + (piece16 ^ (par * 64)) + i * 16 * 128); };
+        // 1-byte transposing read: lane i of 16 supplies 8 bytes of k row 16 * quad + (i >> 1), half i & 1 of column piece j; 2-byte: four elements of
+        // k row 8 * quad + (i >> 2), quarter i & 3 of column pieces 2j, 2j + 1
+        const uint32_t brow16 = ES == 1 ? 16 * quad + (l16 >> 1) : 8 * quad + (l16 >> 2);
+        const uint32_t b16_lds = brow16 * (256 * ES) + (((ES == 1 ? wn * 8u : wn * 16u + ((l16 & 3) >> 1)) ^ b_slot(brow16)) * 16) + (l16 & 1) * 8;
+        auto read_b = [&](const unsigned char *sb, int j) {
+            const unsigned char *p = sb + (b16_lds ^ (uint32_t)(j * (ES == 1 ? 16 : 32)));
+            v2i t0, t1;
+            if constexpr (ES == 1) {
+                t0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((CATCOC_LDS v2i *)p);
+                t1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((CATCOC_LDS v2i *)(p + B_HALF));
+            } else {
+                t0 = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((CATCOC_LDS v4s16 *)p));
+                t1 = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((CATCOC_LDS v4s16 *)(p + B_HALF)));
+            }
+            return v4i{t0.x, t0.y, t1.x, t1.y};
         };
 
         auto issue_step_b = [&](uint32_t kt, bool guard) {
@@ -894,8 +953,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             if ((kt & 1) == 0 && (!guard || kt + 2 < nk)) issue_ap((kt + 2) >> 1);
         };
         if constexpr (FX) {
-            if (args.fx.tail != 0) tail_pair(stAP(0), stB(0), [&](v4i (&af)[MB], uint32_t t, int kk) { load_ap(af, t, kk); },
-                                             [&](v4i (&bf)[4], uint32_t t, int kk) { load_b(bf, stB(t), kk); });
+            if (args.fx.tail != 0) tail_pair(stAP(0), stB(0), [&](uint32_t t, int i) { return read_ap(0, t, i); }, [&](uint32_t t, int j) { return read_b(stB(t), j); });
         }
         // prologue in steady-state order: B0, B1, pair 0, B2
         issue_b(offB4(0));
@@ -905,45 +963,37 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
         // step 0 (peeled: no MFMAs pending yet)
         if (nk > 2) CATCOC_WAIT_VMCNT(B_DMA);
         else CATCOC_WAIT_VMCNT(0);
-        barrier_keep_vmem();
+        barrier16();
         issue_step_b(0, true);
         issue_step_a(0, true);
-        load_ap(fa0, 0, 0);
-        load_b(fb0, stB(0), 0);
-        load_ap(fa1, 0, 1);
-        load_b(fb1, stB(0), 1);
-        CATCOC_FENCE();
-        mma(fa0, fb0);
-        CATCOC_FENCE();
-
-        auto compute = [&](uint32_t kt, bool guard) {
-            // The two waves that share a SIMD (w and w + 4) issue their copies in different halves of the step,
-            // so that one of them always has MFMAs to feed the matrix pipe while the other computes addresses.
-            const bool early = ws < NW / 2;
-            sched_step([&](v4i (&af)[MB], int kk) { load_ap(af, kt, kk); }, stB(kt),
-                       [&] { if (early) issue_step_b(kt, guard); }, [&] { if (early) issue_step_a(kt, guard); }, nothing,
-                       [&] {
-                           if (!early) {
-                               issue_step_b(kt, guard);
-                               issue_step_a(kt, guard);
-                           }
-                       });
+        first16([&](int i) { return read_ap(0, 0, i); }, [&](int j) { return read_b(stB(0), j); });
+        auto compute = [&](auto PAR, uint32_t kt, bool guard) {
+            constexpr int par = decltype(PAR)::value;
+            const unsigned char *sb = stB(kt);
+            step16(PAR, [&](int i) { return read_ap(kt, par, i); }, [&](int j) { return read_b(sb, j); }, [&] { issue_step_b(kt, guard); },
+                   [&] { if (par == 0) issue_step_a(kt, guard); });
         };
         uint32_t kt = 1;
         for (; kt + 5 <= nk; kt += 2) {
             CATCOC_WAIT_VMCNT(WAIT_ODD);
-            barrier_keep_vmem();
-            compute(kt, false);
+            barrier16();
+            compute(ODD, kt, false);
             CATCOC_WAIT_VMCNT(WAIT_EVEN);
-            barrier_keep_vmem();
-            compute(kt + 1, false);
+            barrier16();
+            compute(EVEN, kt + 1, false);
         }
-        for (; kt < nk; ++kt) {   // tail: drain fully at every step
+        for (; kt < nk; kt += 2) {   // tail: drain fully at every step (steps come in pairs: kt is odd)
             CATCOC_WAIT_VMCNT(0);
-            barrier_keep_vmem();
-            compute(kt, true);
+            barrier16();
+            compute(ODD, kt, true);
+            if (kt + 1 < nk) {
+                CATCOC_WAIT_VMCNT(0);
+                barrier16();
+                compute(EVEN, kt + 1, true);
+            }
         }
-        mma(fa1, fb1);
+        upper16(ra[1], [](int) {});
+        acc16_to_32<DT>(a16, acc);
     }
 
 #undef CATCOC_FENCE
