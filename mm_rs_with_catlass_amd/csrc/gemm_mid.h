@@ -6,11 +6,11 @@
 // barrier per chunk.  The two groups' partial tiles meet in LDS after the loop, and a thread then finishes four consecutive columns of
 // eight (four) rows, the peers three at a time in registers.
 //
-// Bound by the matrix pipes at their power limit where the operands come out of the caches (0.47 us per chunk of a 128x128 tile, bf16 at
-// 1.09 GHz of MFMA issue, as the larger tiles' loops; without MFMAs the copies and reads alone take 0.32, without copies 0.35), by
-// HBM else (0.6), and by a fixed 5.5 us (launch apart) of first copies, partial tiles and output.  Time per call, calls behind each other and
-// their operands out of HBM, other kernels -> this: all-gather 8 x [512,4096] x [4096,1024] bf16 52.8 -> 44.6 us, fp16 all-reduce 683x7680x4864
-// of two ranks 157 -> 77, all-gather 278x4736x4864 of two 95 -> 47, W8A8 reduce-scatter 1000x1376x4096 of eight, stored tiles, 26.3 -> 18.1.
+// The MFMAs are 16x16 ones (mfma16.h): where the operands come out of the caches the matrix pipes run at their power limit.  Else HBM bounds (0.6 us
+// per chunk of 128x128), and a fixed 5.5 us (launch apart) of first copies, partial tiles and output.  Time per call, calls behind each other and
+// their operands out of HBM, other kernels -> this on 32x32 MFMAs -> 16x16: all-gather 8 x [512,4096] x [4096,1024] bf16 52.8 -> 44.6 us (operands in the
+// caches in part: 40.2 -> 38.1), fp16 all-reduce 683x7680x4864 of two ranks 157 -> 77, all-gather 278x4736x4864 of two 95 -> 47, W8A8 reduce-scatter
+// 1000x1376x4096 of eight, stored tiles, 26.3 -> 18.1 -> 16.4, 1512x9216x1792 with checksums 40.6 -> 38.3, 2584x11488x2048 123.4 -> 117.6.
 // Which launches: small_tile().
 //
 // A reduce-scatter's kept rows are dealt out to all row tiles.  One CU draws no more than about 40 bytes a nanosecond out of HBM, so
@@ -25,19 +25,21 @@
 #include <type_traits>
 
 #include "gemm_few.h"
+#include "mfma16.h"
 
 namespace catcoc {
 
-// MB: 32-row blocks per wave (2: 128 rows, 1: 64 rows).  Eight waves: two by two positions, two groups that halve every chunk of k.
+// MB: 16-row blocks per wave (tiles of 32 * MB rows).  Eight waves: two by two positions, two groups that halve every chunk of k.
 template <int MB> struct MidGeom
 {
-    static constexpr int BM = 64 * MB, BN = 128, NT = 512;
-    static constexpr int A_STAGE = BM * 128, B_STAGE = BN * 128, STAGE = A_STAGE + B_STAGE;
-    static constexpr int NS = 160 * 1024 / STAGE;   // 5 (128 rows) or 6 stages
-    static constexpr int ACP = BM / 64, BCP = 2, CP = ACP + BCP;   // 1 KiB copies per chunk and wave
-    static constexpr int MEET = 2 * BM * BN * 4;
+    static constexpr int BM = 32 * MB, BN = 128, NT = 512;
+    static constexpr int ACP = (BM + 63) / 64, BCP = 2, CP = ACP + BCP;   // 1 KiB copies per chunk and wave (whole ones: the rows of a stage are up to 32 more than the tile's)
+    static constexpr int A_STAGE = ACP * 64 * 128, B_STAGE = BN * 128, STAGE = A_STAGE + B_STAGE;
+    static constexpr int NS = 160 * 1024 / STAGE;   // 6 (64 rows), 5 (up to 128) or 4 (up to 192) stages
+    static constexpr bool BOTH = 2 * BM * BN * 4 + BM * 16 + 64 <= 160 * 1024;   // both partial tiles fit side by side
+    static constexpr int MEET = (BOTH ? 2 : 1) * BM * BN * 4;
     static constexpr int POOL = NS * STAGE > MEET + BM * 16 + 64 ? NS * STAGE : MEET + BM * 16 + 64;   // the ring, or the partial tiles, the row table, the waves' and the rows' sums
-    static constexpr int UN = BM * BN / 4 / NT;     // groups of four columns per thread: 8 or 4
+    static constexpr int UN = BM * BN / 4 / NT;     // groups of four columns per thread
 };
 
 // Tile number pos of the rowTiles x colTiles over rows [rowBase, rowEnd) and all columns.  GA: A's rows are looked up one by one (all-gather:
@@ -46,11 +48,11 @@ template <uint32_t DT, bool TB, int MB, bool GA>
 __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *smem, uint32_t pos, uint32_t rowTiles, uint32_t colTiles, uint32_t rowBase, uint32_t rowEnd)
 {
     using G = MidGeom<MB>;
-    using Acc = typename AccOf<DT>::type;
+    using Acc = typename Acc16Of<DT>::type;
     constexpr bool I8 = DT == DT_I8;
     constexpr int ES = I8 ? 1 : 2;
     constexpr int ACP = G::ACP, BCP = G::BCP, BM = G::BM, BN = G::BN, UN = G::UN, NS = G::NS, NT = G::NT;
-    constexpr int PF = 3;                            // peers whose values are in flight or in registers at a time
+    constexpr int PF = MB > 4 ? 2 : 3;               // peers whose values are in flight or in registers at a time
     const uint32_t N = args.N, K = args.K, flags = args.flags, keptBegin = args.keptBegin, keptRows = args.keptRows;
     const int64_t peerLd = args.peerLd, peerRowOffset = args.peerRowOffset;
     const void *const a0 = args.a[0], *const b0 = args.b;
@@ -59,7 +61,7 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
     const int tid = threadIdx.x, lane = tid & 63;
     const uint32_t w = __builtin_amdgcn_readfirstlane((uint32_t)tid >> 6);
     const uint32_t wg = w >> 2, wm = (w >> 1) & 1u, wn = w & 1u;   // half of the chunk, position
-    const int c32 = lane & 31, h = lane >> 5;
+    const uint32_t l16 = lane & 15, quad = lane >> 4;
     const SchedParams &sp = args.sched;
     // XCD x takes the x-th eighth of the tiles, in bands of eight tile rows: what is in flight on it is a compact block of the grid
     const uint32_t seq = xcd_eighth(pos, rowTiles * colTiles);
@@ -82,16 +84,16 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
 
     // ---- the stream
     // Stage: A, then B.  A, and B as [n,k]: rows of 128 bytes of k, 16-byte piece c of row r at slot c ^ ((r >> 1) & 7); copy j
-    // covers rows 8j .. 8j+7.  B as [k,n]: 128 / ES rows of k of BN columns, the pieces swizzled so that the 8 (1-byte) or 4
-    // (2-byte elements) rows a half wave's transposing read takes lie in different banks.
+    // covers rows 8j .. 8j+7.  B as [k,n]: 128 / ES rows of k of BN columns, the pieces swizzled so that the 16 (1-byte) or 8
+    // (2-byte elements) rows a half wave's transposing read takes lie in all banks once.
     // k that is no whole number of chunks: in the last one the pieces from the first incomplete one on are the row's last 16 bytes
     // (nothing past a row is read), and the fragment reads put zeros in the place of what is not theirs.
     constexpr int EPP = 16 / ES;                     // elements of a piece
     constexpr int BROW = BN * ES;                    // [k,n]: bytes of a row of the stage
     constexpr int BPR = BROW / 16;                   // pieces of it
     auto bsw = [](uint32_t row) -> uint32_t {        // [k,n]: slot of piece q of row r: q ^ bsw(r)
-        if constexpr (ES == 1) return ((row >> 1) & 3u) << 1;
-        else return (row & 3u) << 2;
+        if constexpr (ES == 1) return (((row >> 1) & 3u) << 1) | ((row >> 4) & 1u);
+        else return b16_slot<2>(row);
     };
     const uint32_t kBytes = K * ES;
     const uint32_t nChunks = (kBytes + 127u) / 128u;
@@ -145,55 +147,49 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
             }
         }
     };
-    Acc acc[MB][2];
+    Acc acc[MB][4];
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
+    for (int i = 0; i < MB; ++i)
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[mb][nb][r] = 0;
-    v4i fa[2][2][MB], fb[2][2][2];
-    // One of this wave's fragments of the chunk at (sa, sb): q = 4 * (32 bytes of the wave's half of k) + {A blocks 0, 1, B blocks 0, 1}
+            for (int r = 0; r < 4; ++r) acc[i][j][r] = 0;
+    v4i fa[2][MB], fb[2][4];
+    // One of this wave's fragments of the chunk at (sa, sb), its half of k: A's blocks, then B's
     const unsigned char *sa = smem, *sb = smem;   // of the stage being read
+    const uint32_t piece16 = l16 * 128 + (((4 * wg + quad) ^ (l16 >> 1)) * 16);   // row l16 of a block of rows of k
+    const uint32_t brow16 = ES == 1 ? 64 * wg + 16 * quad + (l16 >> 1) : 32 * wg + 8 * quad + (l16 >> 2);   // [k,n]: row of k that a lane supplies pieces of
+    const uint32_t b16_lds = brow16 * BROW + (((ES == 1 ? wn * 4 : wn * 8 + ((l16 & 3) >> 1)) ^ bsw(brow16)) * 16) + (l16 & 1) * 8;
     auto read1 = [&](int s, int q) {
-        const int kh = q >> 2, x = q & 3;
-        const uint32_t kk = 2u * wg + kh;
-        if (x < 2) {
-            if (x < MB) fa[s][kh][x] = *(const v4i *)(sa + ((wm * MB + x) * 32 + c32) * 128 + (((2u * kk + h) ^ ((c32 >> 1) & 7)) * 16));
+        if (q < MB) {
+            fa[s][q] = *(const v4i *)(sa + wm * (MB * 16 * 128) + piece16 + q * 2048);
             return;
         }
-        const int nb = x - 2;
+        const int j = q - MB;
         if constexpr (TB) {
-            fb[s][kh][nb] = *(const v4i *)(sb + ((wn * 2 + nb) * 32 + c32) * 128 + (((2u * kk + h) ^ ((c32 >> 1) & 7)) * 16));
+            fb[s][j] = *(const v4i *)(sb + wn * (64 * 128) + piece16 + j * 2048);
         } else {
-            const int i16 = lane & 15, t = (lane >> 4) & 1;
+            const unsigned char *p = sb + (b16_lds ^ (uint32_t)(j * (ES == 1 ? 16 : 32)));
             v2i t0, t1;
             if constexpr (ES == 1) {   // lane i of 16: 8 bytes of k row i >> 1, half i & 1 of a 16-column piece
-                const uint32_t r = 32 * kk + 16 * h + (i16 >> 1);
-                const unsigned char *p = sb + r * BROW + (((wn * 4 + nb * 2 + t) ^ bsw(r)) * 16) + (i16 & 1) * 8;
                 t0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((CATCOC_LDS v2i *)p);
                 t1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((CATCOC_LDS v2i *)(p + 8 * BROW));
             } else {                   // four elements of k row i >> 2, quad i & 3 of a pair of pieces
-                const uint32_t r = 16 * kk + 8 * h + (i16 >> 2);
-                const unsigned char *p = sb + r * BROW + (((wn * 8 + nb * 4 + t * 2 + ((i16 & 3) >> 1)) ^ bsw(r)) * 16) + (i16 & 1) * 8;
                 t0 = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((CATCOC_LDS v4s16 *)p));
                 t1 = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((CATCOC_LDS v4s16 *)(p + 4 * BROW)));
             }
-            fb[s][kh][nb] = v4i{t0.x, t0.y, t1.x, t1.y};
+            fb[s][j] = v4i{t0.x, t0.y, t1.x, t1.y};
         }
     };
     auto mask_last = [&](int s) {   // the last chunk's fragments: zeros past the end of k
+        // (word e of the incomplete piece is byte lastBytes - 16 + 4e of the chunk: its own from byte 16 * lastWhole on)
+        const uint32_t p = 4u * wg + quad, from = p < lastWhole ? 0u : p == lastWhole ? (16u - lastBytes % 16u) / 4u : 4u;
 #pragma unroll
-        for (int kh = 0; kh < 2; ++kh) {
-            // (word e of the incomplete piece is byte lastBytes - 16 + 4e of the chunk: its own from byte 16 * lastWhole on)
-            const uint32_t p = 2u * (2u * wg + kh) + h, from = p < lastWhole ? 0u : p == lastWhole ? (16u - lastBytes % 16u) / 4u : 4u;
+        for (int e = 0; e < 4; ++e) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
+            for (int i = 0; i < MB; ++i) fa[s][i][e] = (uint32_t)e < from ? 0 : fa[s][i][e];
 #pragma unroll
-                for (int mb = 0; mb < MB; ++mb) fa[s][kh][mb][e] = (uint32_t)e < from ? 0 : fa[s][kh][mb][e];
-#pragma unroll
-                for (int nb = 0; nb < 2; ++nb) fb[s][kh][nb][e] = (uint32_t)e < from ? 0 : fb[s][kh][nb][e];
-            }
+            for (int j = 0; j < 4; ++j) fb[s][j][e] = (uint32_t)e < from ? 0 : fb[s][j][e];
         }
     };
     v4f sN = {1.f, 1.f, 1.f, 1.f};
@@ -215,11 +211,11 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
     barrier_keep_vmem();
     sb = sa + G::A_STAGE;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) read1(0, q);
+    for (int q = 0; q < MB + 4; ++q) read1(0, q);
     uint32_t st = 0;   // stage of chunk i
     // Fragment reads and copies behind the MFMAs, where they issue while the matrix pipe is busy: reads in one go in front of them hold
-    // the MFMAs up until the LDS unit has taken all of them, one read behind each of eight MFMAs leaves the last one's latency to the
-    // barrier (4096x4096x1024 bf16 48.2 us, 45, this order 43.7).
+    // the MFMAs up until the LDS unit has taken all of them, one read per 32 cycles of MFMAs leaves the last one's latency to the
+    // barrier (4096x4096x1024 bf16 48.2 us, 45, one per 16 43.7).
     auto step = [&](auto S, auto COPY, uint32_t i) {   // COPY: in the middle of the range, every chunk in flight
         constexpr int s = decltype(S)::value;
         constexpr bool copy = decltype(COPY)::value;
@@ -238,16 +234,13 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int q = 0; q < 4 * MB; ++q) {
-            const int kh = q / (2 * MB), mb = (q % (2 * MB)) / 2, nb = q % 2;
-            acc[mb][nb] = mfma32<DT>(fa[s][kh][mb], fb[s][kh][nb], acc[mb][nb]);
+            const int nb = q / MB, mb = snake16(nb, q % MB, MB);
+            acc[mb][nb] = mfma16<DT>(fa[s][mb], fb[s][nb], acc[mb][nb]);
             __builtin_amdgcn_sched_barrier(0);
             if (copy || i + 1u < nChunks) {
-                if (q < 4) {
-                    read1(1 - s, 2 * q);
-                    read1(1 - s, 2 * q + 1);
-                }
+                if (q < MB + 4) read1(1 - s, q);   // (MB + 4 <= 4 * MB)
             }
-            if (q == (MB == 2 ? 5 : 3) && (copy || i + NS < nChunks)) issue(i + NS, old);
+            if (q == (MB == 2 ? 6 : 3 * MB - 2) && (copy || i + NS < nChunks)) issue(i + NS, old);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -306,17 +299,50 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
     __syncthreads();   // every wave has left the ring
     uint32_t *dst = (uint32_t *)(smem + G::MEET);   // [BM] what row i of the tile does
     float *rowScale = (float *)(dst + BM);         // [BM] W8A8 per-token scale
-    constexpr uint32_t SWZ = BN >= 64 ? 1u : 0u;             // rows with bit 2 set are shifted by 128 bytes: the halves of a wave's write lie in different banks
+    // (the quarters of a wave's write are rows four apart: in columns shifted by 16 they lie in different banks)
+    auto meet_at = [&](int i, int j, int r) -> uint32_t {
+        const uint32_t q4 = ((uint32_t)t2 >> 4) & 3u, row = (wm * MB + i) * 16 + q4 * 4 + r;
+        return (row * BN + (((wn * 4 + j) * 16 + (t2 & 15)) ^ (q4 << 4))) * 4;
+    };
+    if constexpr (G::BOTH) {
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
+        for (int i = 0; i < MB; ++i)
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
+            for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint32_t row = (wm * MB + mb) * 32 + (r >> 2) * 8 + (uint32_t)((t2 >> 5) & 1) * 4 + (r & 3);
-                const auto e = acc[mb][nb][r];
-                *(int *)(smem + ((wg * BM + row) * BN + (((wn * 2 + nb) * 32 + (t2 & 31)) ^ ((uint32_t)((t2 >> 5) & 1) * SWZ << 5))) * 4) = __builtin_bit_cast(int, e);
+                for (int r = 0; r < 4; ++r) {
+                    const auto e = acc[i][j][r];
+                    *(int *)(smem + wg * (BM * BN * 4) + meet_at(i, j, r)) = __builtin_bit_cast(int, e);
+                }
+    } else {
+        // Each group hands over half of the blocks, in their places, and adds what it is handed to its own half.
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+            if ((i < MB / 2 ? 0u : 1u) != wg) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const auto e = acc[i][j][r];
+                        *(int *)(smem + meet_at(i, j, r)) = __builtin_bit_cast(int, e);
+                    }
             }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+            if ((i < MB / 2 ? 0u : 1u) == wg) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        int *const p = (int *)(smem + meet_at(i, j, r));
+                        const auto e = acc[i][j][r];
+                        const int mine = __builtin_bit_cast(int, e), other = *p;
+                        if constexpr (I8) *p = mine + other;
+                        else *p = f2i(__fadd_rn(i2f(mine), i2f(other)));
+                    }
+            }
+    }
     const bool store = (flags & GF_OUTBOUND_STORE) != 0, taskSums = !store && (flags & GF_ROW_MASK) == 0 && args.checksum != nullptr && sp.op == OP_REDUCE_SCATTER;
     if (tid < BM) {
         const uint32_t v = rowOf(tid);
@@ -346,9 +372,9 @@ __device__ __forceinline__ void mid_tile(const GemmArgs &args, unsigned char *sm
 #pragma unroll
     for (int j = 0; j < UN; ++j) {
         const uint32_t row = urow + j * (NT / LPR);
-        const unsigned char *p = smem + (row * BN + (lcol ^ (((row >> 2) & 1u) * SWZ << 5))) * 4;
+        const unsigned char *p = smem + (row * BN + (lcol ^ (((row >> 2) & 3u) << 4))) * 4;
         cur[j] = *(const v4i *)p;
-        {
+        if constexpr (G::BOTH) {
             const v4i t = *(const v4i *)(p + BM * BN * 4);
             if constexpr (I8) {
                 cur[j] += t;
@@ -470,8 +496,8 @@ template <uint32_t DT, bool TB, bool GA>
 inline int launch_mid_tb(const GemmArgs &args, int tileRows, hipStream_t s)
 {
     const dim3 grid(args.fx.rowTiles * args.fx.colTiles), block(512);
-    if (tileRows == 128) hipLaunchKernelGGL((gemm_mid_kernel<DT, TB, 2, GA>), grid, block, 0, s, args);
-    else if (tileRows == 64) hipLaunchKernelGGL((gemm_mid_kernel<DT, TB, 1, GA>), grid, block, 0, s, args);
+    if (tileRows == 64) hipLaunchKernelGGL((gemm_mid_kernel<DT, TB, 2, GA>), grid, block, 0, s, args);
+    else if (tileRows == 128) hipLaunchKernelGGL((gemm_mid_kernel<DT, TB, 4, GA>), grid, block, 0, s, args);
     else return (int)hipErrorInvalidValue;
     return (int)hipGetLastError();
 }

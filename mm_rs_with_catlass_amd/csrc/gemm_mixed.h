@@ -23,12 +23,12 @@ template <uint32_t DT, bool TB>
 __global__ void __launch_bounds__(512, 1) gemm_mixed_kernel(const GemmArgs args)
 {
     __shared__ __attribute__((aligned(1024))) unsigned char smem[FLEX_POOL8];
-    static_assert(MidGeom<2>::POOL <= FLEX_POOL8, "the small tiles fit");
+    static_assert(MidGeom<4>::POOL <= FLEX_POOL8, "the small tiles fit");
     const FlexParams &f = args.fx;
     if (blockIdx.x < f.largeTiles) {
         dma_tile<DT, 4, TB, false, false, false, 2, 3, false, false, false, 1>(args, smem, blockIdx.x, 0, 1u, 0);
     } else {
-        mid_tile<DT, TB, 2, DT != DT_I8>(args, smem, blockIdx.x - f.largeTiles, ceil_div(f.holeRows, 128u), ceil_div(args.N, 128u), f.hole0, f.hole0 + f.holeRows);
+        mid_tile<DT, TB, 4, DT != DT_I8>(args, smem, blockIdx.x - f.largeTiles, ceil_div(f.holeRows, 128u), ceil_div(args.N, 128u), f.hole0, f.hole0 + f.holeRows);
     }
 }
 
