@@ -33,6 +33,10 @@ __device__ __forceinline__ void barrier_keep_vmem()
     asm volatile("" ::: "memory");
 }
 
+// Between a wave's writes to its staging area and its reads of other lanes' values (the LDS unit keeps a wave's accesses in order; the compiler,
+// to which one lane's accesses are all there is, may not: it has moved the last write of a block behind the read of its row).
+__device__ __forceinline__ void lds_turn() { asm volatile("" ::: "memory"); }
+
 // 16 bytes per lane, global -> LDS, lane l lands at lds + 16*l (lds is wave-uniform).
 // Issued as an asm statement on purpose: the kernel orders these copies against LDS reads itself
 // (CATCOC_WAIT_VMCNT + barrier), with several stages in flight across barriers and loop iterations.
@@ -104,7 +108,7 @@ template <int MB, int NS> struct FlexPool
 // AQ = A is copied per pair of k steps, 128 bytes per row (whole cache lines: half as many requests to L2 as two 64-byte
 // halves), as the 256-row geometry does; for the six-stage ring, whose launches have one workgroup per CU and feel every
 // request (with three stages and two workgroups per CU the same change measured slower).
-template <uint32_t DT, int WM, bool TB, bool RM, bool RG, bool TA, int MB, int NS = 3, bool PP = false, bool AQ = false, bool W8 = false, int FX = 0>
+template <uint32_t DT, int WM, bool TB, bool RM, bool RG, bool TA, int MB, int NS = 3, bool PP = false, bool AQ = false, bool W8 = false, int FX = 0, bool M16 = WM == 4>
 __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *smem, uint32_t pos, uint32_t slice /* FX: from pos */, uint32_t kSlices,
                                          uint32_t subRow)
 {
@@ -119,6 +123,9 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     static_assert(!AQ || (WM == 2 && NS == 6 && (MB == 2 || W8) && !TA), "pairs of A steps exist for the six-stage 128-row kernel with A as [m,k]");
     using Acc = typename AccOf<DT>::type;
     constexpr int ES = (DT == DT_I8) ? 1 : 2;   // bytes per operand element; a k step is 64 BYTES of K
+    static_assert(WM == 2 || M16, "256 rows: 16x16 MFMAs");
+    static_assert(WM == 4 || !M16 || (NS == 3 && !TA && !RM && !AQ && !W8 && !FX), "16x16 MFMAs on 128 rows: the plain three-stage ring");
+    constexpr bool X16 = M16 && MB == 2;   // (64-row halves: 32x32)
     constexpr int WR = W8 ? 4 : WM;     // wave rows (two wave columns)
     constexpr int NW = 2 * WR;          // waves
     constexpr int NT = 64 * NW;         // threads
@@ -222,14 +229,24 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     // A given as [k][m], 1-byte elements (64 k rows x 128 bytes): copy j covers k rows 8j..8j+7; lane -> row 8j + lane/8, slot
     // lane&7 holds chunk slot ^ (((row>>1)&3)<<1).  2-byte elements (32 k rows x 256 bytes): copy j covers k rows 4j..4j+3;
     // lane -> row 4j + lane/16, slot lane&15 holds chunk slot ^ ((row&3)<<2).
+    // (16x16 MFMAs: k16_slot() and b16_slot() in the place of these swizzles)
+    auto k_slot = [](uint32_t row) -> uint32_t {   // rows of 64 bytes of k
+        if constexpr (X16) return k16_slot(row);
+        else return (row >> 2) & 3u;
+    };
+    auto b_slot = [](uint32_t row) -> uint32_t {   // rows of columns
+        if constexpr (X16) return b16_slot<ES>(row);
+        else if constexpr (ES == 1) return (row & 7u) << 1;
+        else return (row & 3u) << 2;
+    };
     const unsigned char *gA[A_DMA];
 #pragma unroll
     for (int jj = 0; jj < A_DMA; ++jj) {
         if constexpr (FX) {
             const uint32_t row = ti.row + umin(16u * (w + NW * jj) + (lane >> 2), ti.rowsValid - 1u);
-            gA[jj] = flex_row_ptr(args, flex_row<WM == 4>(args, row), ldaB) + kOff + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
+            gA[jj] = flex_row_ptr(args, flex_row<WM == 4>(args, row), ldaB) + kOff + (((lane & 3) ^ k_slot((lane >> 2) & 15)) * 16);
         } else if constexpr (!TA) {
-            gA[jj] = Ag + (size_t)(16 * (w + NW * jj) + (lane >> 2)) * ldaB + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
+            gA[jj] = Ag + (size_t)(16 * (w + NW * jj) + (lane >> 2)) * ldaB + (((lane & 3) ^ k_slot((lane >> 2) & 15)) * 16);
         } else if constexpr (ES == 1) {
             const int row = 8 * (w + NW * jj) + (lane >> 3);
             gA[jj] = Ag + (size_t)row * ldaB + (((lane & 7) ^ (((row >> 1) & 3) << 1)) * 16);
@@ -250,12 +267,6 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     // chunk slot^((row&7)<<1).  2-byte elements (32 k rows x 512 bytes): copy j covers k rows 2j, 2j+1; lane -> row
     // 2j + lane/32, slot lane&31 holds chunk slot^((row&3)<<2).
     // B given as [n][k]: copy j covers tile columns 16j..16j+15, one 64-byte row of k each, laid out like A.
-    // (256 rows: b16_slot() in the place of these swizzles)
-    auto b_slot = [](uint32_t row) -> uint32_t {
-        if constexpr (WM == 4) return b16_slot<ES>(row);
-        else if constexpr (ES == 1) return (row & 7u) << 1;
-        else return (row & 3u) << 2;
-    };
     const unsigned char *gB[B_DMA];
 #pragma unroll
     for (int jj = 0; jj < B_DMA; ++jj) {
@@ -264,7 +275,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             // whose values land in columns nobody looks at (the last row of B is never read here: it belongs to the checked step)
             const uint32_t last = ti.colsValid - 1u;
             if constexpr (TB) {
-                gB[jj] = Bg + (size_t)umin(16u * (w + NW * jj) + (lane >> 2), last) * ldbB + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
+                gB[jj] = Bg + (size_t)umin(16u * (w + NW * jj) + (lane >> 2), last) * ldbB + (((lane & 3) ^ k_slot((lane >> 2) & 15)) * 16);
             } else if constexpr (ES == 1) {
                 const int row = 4 * (w + NW * jj) + (lane >> 4);
                 gB[jj] = Bg + (size_t)row * ldbB + (umin((lane & 15) ^ b_slot(row), last / 16u) * 16);
@@ -273,7 +284,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
                 gB[jj] = Bg + (size_t)row * ldbB + (umin((lane & 31) ^ b_slot(row), last / 8u) * 16);
             }
         } else if constexpr (TB) {
-            gB[jj] = Bg + (size_t)(16 * (w + NW * jj) + (lane >> 2)) * ldbB + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
+            gB[jj] = Bg + (size_t)(16 * (w + NW * jj) + (lane >> 2)) * ldbB + (((lane & 3) ^ k_slot((lane >> 2) & 15)) * 16);
         } else if constexpr (ES == 1) {
             const int row = 4 * (w + NW * jj) + (lane >> 4);
             gB[jj] = Bg + (size_t)row * ldbB + (((lane & 15) ^ b_slot(row)) * 16);
@@ -292,7 +303,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     };
 
     Acc acc[MB][4];
-    if constexpr (WM == 2) {
+    if constexpr (!X16) {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -444,13 +455,13 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
     };
 #undef CATCOC_MMA
     auto nothing = [] {};
-    // 256 rows: 16x16 MFMAs (mfma16.h), 4 x 8 blocks per wave.  A step's 32 MFMAs lag its fragment reads by half a step as well: the first
+    // 16x16 MFMAs: 4 x 8 blocks per wave.  A step's 32 MFMAs lag its fragment reads by half a step as well: the first
     // sixteen are columns 64 .. 127 of the step before, behind which this step's fragments of A and of columns 0 .. 63 are read, the second
     // sixteen those columns, behind which the fragments of the others are.
-    typename Acc16Of<DT>::type a16[WM == 4 ? 4 : 1][8];
+    typename Acc16Of<DT>::type a16[X16 ? 4 : 1][8];
     v4i ra[2][4], rbl[4], rbh[4];   // A of a step's parity, B's lower and upper four column blocks
     const uint32_t l16 = lane & 15, quad = lane >> 4;
-    if constexpr (WM == 4) {
+    if constexpr (X16) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -478,11 +489,11 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             CATCOC_FENCE();
         }
     };
-    // read_a(i), read_b(j): fragments of this step; copyA, copyB: the step's copies.  The two waves that share a SIMD (w and w + 4) issue
+    // read_a(i), read_b(j): fragments of this step; copyA, copyB: the step's copies.  The two waves of eight that share a SIMD (w and w + 4) issue
     // them in different halves of the step, so that one of them always has MFMAs to feed the matrix pipe while the other computes addresses.
     auto step16 = [&](auto PAR, auto read_a, auto read_b, auto copyA, auto copyB) {
         constexpr int par = decltype(PAR)::value;
-        const bool early = ws < NW / 2;
+        const bool early = WM == 2 || ws < NW / 2;
         upper16(ra[1 - par], [&](int m) {
             if (m == 0) rbl[0] = read_b(0);
             else if (m < 9 && m % 2 == 0) ra[par][m / 2 - 1] = read_a(m / 2 - 1);
@@ -495,6 +506,22 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             if (m == 9 && !early) copyA();
             if (m == 13 && !early) copyB();
         });
+    };
+    // 1-byte transposing read: lane i of 16 supplies 8 bytes of k row 16 * quad + (i >> 1), half i & 1 of column piece j; 2-byte: four elements of
+    // k row 8 * quad + (i >> 2), quarter i & 3 of column pieces 2j, 2j + 1
+    const uint32_t brow16 = ES == 1 ? 16 * quad + (l16 >> 1) : 8 * quad + (l16 >> 2);
+    const uint32_t b16_lds = brow16 * (256 * ES) + (((ES == 1 ? wn * 8u : wn * 16u + ((l16 & 3) >> 1)) ^ b_slot(brow16)) * 16) + (l16 & 1) * 8;
+    auto read_b16 = [&](const unsigned char *sb, int j) {   // column block j of a stage of rows of columns
+        const unsigned char *p = sb + (b16_lds ^ (uint32_t)(j * (ES == 1 ? 16 : 32)));
+        v2i t0, t1;
+        if constexpr (ES == 1) {
+            t0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((CATCOC_LDS v2i *)p);
+            t1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((CATCOC_LDS v2i *)(p + B_HALF));
+        } else {
+            t0 = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((CATCOC_LDS v4s16 *)p));
+            t1 = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((CATCOC_LDS v4s16 *)(p + B_HALF)));
+        }
+        return v4i{t0.x, t0.y, t1.x, t1.y};
     };
     auto barrier16 = [] {   // (the last fragments' reads are long back: sixteen MFMAs were issued since)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -705,6 +732,12 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
                 }
             }
         };
+        const uint32_t row16 = l16 * 64 + ((quad ^ k16_slot(l16)) * 16);   // 16x16: row l16 of a block of rows of k
+        auto read_a16 = [&](const unsigned char *sa, int i) { return *(const v4i *)(sa + wm * 64 * 64 + row16 + i * 16 * 64); };
+        auto read_bk16 = [&](const unsigned char *sb, int j) {
+            if constexpr (TB) return *(const v4i *)(sb + wn * 128 * 64 + row16 + j * 16 * 64);
+            else return read_b16(sb, j);
+        };
 #pragma unroll
         for (int st = 0; st < NS - 1; ++st)
             if (nk > (uint32_t)st) {
@@ -744,18 +777,18 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
 #pragma unroll
                 for (int q = 0; q < PA; ++q) {
                     const uint32_t idx = tid + NT * q, row = idx >> 2, c = idx & 3u;
-                    *(v4i *)(ta + row * 64 + ((c ^ ((row >> 2) & 3u)) * 16)) = pa[q];
+                    *(v4i *)(ta + row * 64 + ((c ^ k_slot(row)) * 16)) = pa[q];
                 }
 #pragma unroll
                 for (int q = 0; q < PB; ++q) {
                     const uint32_t idx = tid + NT * q;
                     if constexpr (TB) {
                         const uint32_t row = idx >> 2, c = idx & 3u;
-                        *(v4i *)(tb + row * 64 + ((c ^ ((row >> 2) & 3u)) * 16)) = pb[q];
+                        *(v4i *)(tb + row * 64 + ((c ^ k_slot(row)) * 16)) = pb[q];
                     } else {
                         constexpr int CH = 256 * ES / 16;
                         const uint32_t row = idx / CH, c = idx % CH;
-                        *(v4i *)(tb + row * (256 * ES) + ((c ^ (ES == 1 ? (row & 7u) << 1 : (row & 3u) << 2)) * 16)) = pb[q];
+                        *(v4i *)(tb + row * (256 * ES) + ((c ^ b_slot(row)) * 16)) = pb[q];
                     }
                 }
                 __syncthreads();
@@ -768,7 +801,55 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
                 mma(fa1, fb1);
             }
         }
-        if (!FX || nk > 0) {
+        if constexpr (X16) {
+            {
+                wait_steps(umin(NS - 2, nk - 1));
+                barrier16();
+                if (nk > NS - 1) {
+                    issue_a(offA(NS - 1));
+                    issue_b(offB(NS - 1));
+                }
+                first16([&](int i) { return read_a16(stA(0), i); }, [&](int j) { return read_bk16(stB(0), j); });
+                // step kt reads stage kt % NS and refills stage (kt - 1) % NS, whose last fragments every wave had at the barrier
+                uint32_t kt = 1, cur = 1, nxt = 0;
+                auto step = [&](auto PAR, bool more) {
+                    const unsigned char *sa = stA(cur), *sb = stB(cur);
+                    step16(PAR, [&](int i) { return read_a16(sa, i); }, [&](int j) { return read_bk16(sb, j); }, [&] { if (more) issue_a(offA(nxt)); },
+                           [&] { if (more) issue_b(offB(nxt)); });
+                    ++kt;
+                    cur = cur == NS - 1 ? 0 : cur + 1;
+                    nxt = nxt == NS - 1 ? 0 : nxt + 1;
+                };
+                while (kt + NS < nk) {   // an odd and an even step in full flight
+                    CATCOC_WAIT_VMCNT((NS - 2) * STEP_DMA);
+                    barrier16();
+                    step(ODD, true);
+                    CATCOC_WAIT_VMCNT((NS - 2) * STEP_DMA);
+                    barrier16();
+                    step(EVEN, true);
+                }
+                while (kt < nk) {
+                    wait_steps(umin(NS - 2, nk - 1 - kt));
+                    barrier16();
+                    step(ODD, kt + (NS - 1) < nk);
+                    if (kt < nk) {
+                        wait_steps(umin(NS - 2, nk - 1 - kt));
+                        barrier16();
+                        step(EVEN, kt + (NS - 1) < nk);
+                    }
+                }
+                v4i last[4];   // (a select: no control flow around the accumulators)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int x0 = ra[0][i][e], x1 = ra[1][i][e];
+                        last[i][e] = (nk & 1u) ? x0 : x1;
+                    }
+                upper16(last, [](int) {});
+            }
+            acc16_to_32<DT>(a16, acc);
+        } else if (!FX || nk > 0) {
         // step 0 (peeled: no MFMAs pending yet)
         wait_steps(umin(NS - 2, nk - 1));
         barrier_keep_vmem();
@@ -891,7 +972,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             }
         }
         upper16(ra[1], [](int) {});
-        acc16_to_32<DT>(a16, acc);
+        if constexpr (!FX) acc16_to_32<DT>(a16, acc);
     } else {
         // ---- 256x256 ---------------------------------------------------------------------------------
         // B: four 64-row stages, copies issued three steps ahead.  A: two "pair" buffers of 256 rows x 128
@@ -929,23 +1010,6 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
         auto offB4 = [&](uint32_t step) { return 2 * AP + (step & 3) * B_STAGE; };
         const uint32_t piece16 = l16 * 128 + ((quad ^ (l16 >> 1)) * 16);
         auto read_ap = [&](uint32_t kt, uint32_t par, int i) { return *(const v4i *)(stAP(kt >> 1) + wm * 64 * 128 + (piece16 ^ (par * 64)) + i * 16 * 128); };
-        // 1-byte transposing read: lane i of 16 supplies 8 bytes of k row 16 * quad + (i >> 1), half i & 1 of column piece j; 2-byte: four elements of
-        // k row 8 * quad + (i >> 2), quarter i & 3 of column pieces 2j, 2j + 1
-        const uint32_t brow16 = ES == 1 ? 16 * quad + (l16 >> 1) : 8 * quad + (l16 >> 2);
-        const uint32_t b16_lds = brow16 * (256 * ES) + (((ES == 1 ? wn * 8u : wn * 16u + ((l16 & 3) >> 1)) ^ b_slot(brow16)) * 16) + (l16 & 1) * 8;
-        auto read_b = [&](const unsigned char *sb, int j) {
-            const unsigned char *p = sb + (b16_lds ^ (uint32_t)(j * (ES == 1 ? 16 : 32)));
-            v2i t0, t1;
-            if constexpr (ES == 1) {
-                t0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((CATCOC_LDS v2i *)p);
-                t1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((CATCOC_LDS v2i *)(p + B_HALF));
-            } else {
-                t0 = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((CATCOC_LDS v4s16 *)p));
-                t1 = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((CATCOC_LDS v4s16 *)(p + B_HALF)));
-            }
-            return v4i{t0.x, t0.y, t1.x, t1.y};
-        };
-
         auto issue_step_b = [&](uint32_t kt, bool guard) {
             if (!guard || kt + 3 < nk) issue_b(offB4(kt + 3));
         };
@@ -953,7 +1017,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             if ((kt & 1) == 0 && (!guard || kt + 2 < nk)) issue_ap((kt + 2) >> 1);
         };
         if constexpr (FX) {
-            if (args.fx.tail != 0) tail_pair(stAP(0), stB(0), [&](uint32_t t, int i) { return read_ap(0, t, i); }, [&](uint32_t t, int j) { return read_b(stB(t), j); });
+            if (args.fx.tail != 0) tail_pair(stAP(0), stB(0), [&](uint32_t t, int i) { return read_ap(0, t, i); }, [&](uint32_t t, int j) { return read_b16(stB(t), j); });
         }
         // prologue in steady-state order: B0, B1, pair 0, B2
         issue_b(offB4(0));
@@ -966,11 +1030,11 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
         barrier16();
         issue_step_b(0, true);
         issue_step_a(0, true);
-        first16([&](int i) { return read_ap(0, 0, i); }, [&](int j) { return read_b(stB(0), j); });
+        first16([&](int i) { return read_ap(0, 0, i); }, [&](int j) { return read_b16(stB(0), j); });
         auto compute = [&](auto PAR, uint32_t kt, bool guard) {
             constexpr int par = decltype(PAR)::value;
             const unsigned char *sb = stB(kt);
-            step16(PAR, [&](int i) { return read_ap(kt, par, i); }, [&](int j) { return read_b(sb, j); }, [&] { issue_step_b(kt, guard); },
+            step16(PAR, [&](int i) { return read_ap(kt, par, i); }, [&](int j) { return read_b16(sb, j); }, [&] { issue_step_b(kt, guard); },
                    [&] { if (par == 0) issue_step_a(kt, guard); });
         };
         uint32_t kt = 1;
@@ -993,14 +1057,15 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             }
         }
         upper16(ra[1], [](int) {});
-        acc16_to_32<DT>(a16, acc);
+        if constexpr (!FX) acc16_to_32<DT>(a16, acc);
     }
 
 #undef CATCOC_FENCE
 
     if constexpr (FX) {
         if constexpr (FX == 2) flex_store_partial<MB>(args, acc, smem, ft, slice);
-        else flex_epilogue<DT, MB, NW>(args, acc, smem, ft);
+        else if constexpr (X16) flex_epilogue<DT, MB, NW, true>(args, a16, smem, ft);
+        else flex_epilogue<DT, MB, NW, false>(args, acc, smem, ft);
         return;
     }
 
@@ -1146,10 +1211,14 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
 
     // ---- epilogue -----------------------------------------------------------------
     // acc[mb][nb][r] is element (row, col) of the tile with
-    //   row = wm*32*MB + mb*32 + (r>>2)*8 + h*4 + (r&3),  col = wn*128 + nb*32 + c32
+    //   row = wm*32*MB + mb*32 + rowOf(r) + ROWS_H*h,  col = wn*128 + nb*32 + c32
+    // (32x32 MFMAs: quads of rows, h the odd ones; acc16_to_32: octets)
+    constexpr uint32_t ROWS_H = X16 ? 8u : 4u;
+    auto rowOf = [](int r) -> uint32_t { return X16 ? (r >> 3) * 16 + (r & 7) : (r >> 2) * 8 + (r & 3); };
+    auto turnOf = [](uint32_t row) -> uint32_t { return ((row / ROWS_H) & 1u) << 7; };   // staging areas: where rows of one h are shifted to
     const uint32_t col0 = wn * 128 + c32;       // + 32*nb
     const uint32_t gcol0 = ti.col + col0;
-    const uint32_t row_base = wm * 32 * MB + h * 4;
+    const uint32_t row_base = wm * 32 * MB + h * ROWS_H;
     bool kept = ti.row >= args.keptBegin && ti.row < args.keptBegin + args.keptRows;
     // RM: bit mb is set when 32-row block mb of this wave is kept (the unsigned compare also rejects blocks above keptBegin:
     // the difference wraps); the tile counts as kept when any of its rows is
@@ -1195,7 +1264,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const uint32_t lrow = row_base + mb * 32 + (r >> 2) * 8 + (r & 3);
+                const uint32_t lrow = row_base + mb * 32 + rowOf(r);
                 if constexpr (DT == DT_I8) {
                     int32_t *o = (int32_t *)args.accDump + (size_t)(ti.row + lrow) * args.N + gcol0;
 #pragma unroll
@@ -1222,7 +1291,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) sMv[mb][r] = args.scaleM[ti.row + row_base + mb * 32 + (r >> 2) * 8 + (r & 3)];
+                for (int r = 0; r < 16; ++r) sMv[mb][r] = args.scaleM[ti.row + row_base + mb * 32 + rowOf(r)];
             __builtin_amdgcn_sched_barrier(0);
         }
     }
@@ -1271,13 +1340,13 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb) {
                     const int32_t *srcb = src + (size_t)(mb * 32) * args.peerLd;
-                    if constexpr (RM) srcb = (keptMb & (1u << mb)) ? srcb : peer + (size_t)(h * 4) * args.peerLd + gcol0;   // (as add_partial)
+                    if constexpr (RM) srcb = (keptMb & (1u << mb)) ? srcb : peer + (size_t)(h * ROWS_H) * args.peerLd + gcol0;   // (as add_partial)
                     int pv[16][4];
 #pragma unroll
                     for (int r = 0; r < 16; ++r)
 #pragma unroll
                         for (int nb = 0; nb < 4; ++nb)
-                            pv[r][nb] = __builtin_nontemporal_load(srcb + (size_t)((r >> 2) * 8 + (r & 3)) * args.peerLd + 32 * nb);
+                            pv[r][nb] = __builtin_nontemporal_load(srcb + (size_t)rowOf(r) * args.peerLd + 32 * nb);
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int r = 0; r < 16; ++r)
@@ -1297,20 +1366,22 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
                 for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
-                        const uint32_t wrow = (r >> 2) * 8 + h * 4 + (r & 3);
+                        const uint32_t wrow = rowOf(r) + h * ROWS_H;
 #pragma unroll
                         for (int nb = 0; nb < 4; ++nb) {
                             const int iv = acc[mb][nb][r];
                             *(int *)(stc + wrow * 512 + (((nb * 32 + c32) * 4) ^ (h << 7))) = iv;
                         }
                     }
+                    lds_turn();
 #pragma unroll
                     for (int j = 0; j < 16; ++j) {
                         const uint32_t wrow = j * 2 + (lane >> 5), chunk = lane & 31;
-                        const v4i v = *(const v4i *)(stc + wrow * 512 + ((chunk * 16) ^ (((wrow >> 2) & 1) << 7)));
+                        const v4i v = *(const v4i *)(stc + wrow * 512 + ((chunk * 16) ^ turnOf(wrow)));
                         if (RM && !(keptMb & (1u << mb))) continue;   // (stores only)
                         *(v4i *)(cw + (int64_t)(mb * 32 + wrow) * args.N + chunk * 4) = v;
                     }
+                    lds_turn();
                 }
             }
             // a round of the pipelined operator whose comm side also writes the dequantised rows: the int32 block is all
@@ -1351,16 +1422,18 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
                 const uint32_t lrow = lane >> 5, chunk = lane & 31;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const uint32_t wrow = (r >> 2) * 8 + h * 4 + (r & 3);
+                    const uint32_t wrow = rowOf(r) + h * ROWS_H;
 #pragma unroll
                     for (int nb = 0; nb < 4; ++nb) *(float *)(st + wrow * 512 + (((nb * 32 + c32) * 4) ^ (h << 7))) = getf(mb, nb, r);
                 }
+                lds_turn();
                 v4f cur[16];
 #pragma unroll
                 for (int j = 0; j < 16; ++j) {
                     const uint32_t wrow = j * 2 + lrow;
-                    cur[j] = *(const v4f *)(st + wrow * 512 + ((chunk * 16) ^ (((wrow >> 2) & 1) << 7)));
+                    cur[j] = *(const v4f *)(st + wrow * 512 + ((chunk * 16) ^ turnOf(wrow)));
                 }
+                lds_turn();
                 // peers and output go through buffer descriptors: a wave-uniform base per unit, one per-lane offset for all
                 // of them, and the row step as a scalar offset, so that a load costs no address arithmetic in vector registers
                 const int64_t rowInKept = (int64_t)(int32_t)out_row0 + (ws >> 1) * 32 * MB + mb * 32;
@@ -1426,13 +1499,13 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb) {
                 const float *srcb = src + (size_t)(mb * 32) * ld;
-                if constexpr (RM) srcb = (keptMb & (1u << mb)) ? srcb : firstKept + (size_t)(h * 4) * ld + gcol0;
+                if constexpr (RM) srcb = (keptMb & (1u << mb)) ? srcb : firstKept + (size_t)(h * ROWS_H) * ld + gcol0;
                 float pv[16][4];
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
 #pragma unroll
                     for (int nb = 0; nb < 4; ++nb)
-                        pv[r][nb] = __builtin_nontemporal_load(srcb + (size_t)((r >> 2) * 8 + (r & 3)) * ld + 32 * nb);
+                        pv[r][nb] = __builtin_nontemporal_load(srcb + (size_t)rowOf(r) * ld + 32 * nb);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
@@ -1459,7 +1532,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const uint32_t wrow = mb * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
+                    const uint32_t wrow = mb * 32 + rowOf(r) + h * ROWS_H;
 #pragma unroll
                     for (int nb = 0; nb < 4; ++nb)
                         *(unsigned short *)(st + wrow * 256 + (((nb * 32 + c32) * 2) ^ (h << 7))) = (unsigned short)cvt(getf(mb, nb, r));
@@ -1467,12 +1540,13 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
         };
         if (args.outDtype == DT_BF16) stage_all([](float f) { return f32_to_bf16_bits(f); });
         else stage_all([](float f) { return f32_to_f16_bits(f); });
+        lds_turn();
         unsigned char *dwave = (unsigned char *)args.d + (((int64_t)(int32_t)out_row0 + wm * 32 * MB) * args.ldd + ti.col + wn * 128) * 2;
 #pragma unroll
         for (int j = 0; j < 8 * MB; ++j) {
             if constexpr (RM) if (!(keptMb & (1u << (j >> 3)))) continue;   // rows 4j .. 4j+3 of the wave: 32-row block j / 8
             const uint32_t wrow = j * 4 + (lane >> 4), chunk = lane & 15;
-            const v4i v = *(const v4i *)(st + wrow * 256 + ((chunk * 16) ^ (((wrow >> 2) & 1) << 7)));
+            const v4i v = *(const v4i *)(st + wrow * 256 + ((chunk * 16) ^ turnOf(wrow)));
             *(v4i *)(dwave + (size_t)wrow * args.ldd * 2 + chunk * 16) = v;
         }
         }
@@ -1492,7 +1566,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
         for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const uint32_t wrow = (r >> 2) * 8 + h * 4 + (r & 3);   // row inside the 32-row block
+                const uint32_t wrow = rowOf(r) + h * ROWS_H;   // row inside the 32-row block
                 float sM = 1.f;
                 if constexpr (DT == DT_I8) sM = sMv[mb][r];
 #pragma unroll
@@ -1507,14 +1581,16 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
                     *(float *)(st + wrow * 512 + (((nb * 32 + c32) * 4) ^ (h << 7))) = v;
                 }
             }
+            lds_turn();
 #pragma unroll
             for (int j = 0; j < 16; ++j) {
                 const uint32_t wrow = j * 2 + (lane >> 5), chunk = lane & 31;
-                const v4f v = *(const v4f *)(st + wrow * 512 + ((chunk * 16) ^ (((wrow >> 2) & 1) << 7)));
+                const v4f v = *(const v4f *)(st + wrow * 512 + ((chunk * 16) ^ turnOf(wrow)));
                 if constexpr (RG)
                     if (wm * 32 * MB + mb * 32 + wrow < shiftM || wn * 128 + chunk * 4 < shiftN) continue;
                 __builtin_nontemporal_store(v, (v4f *)(obw + (size_t)(mb * 32 + wrow) * sp.n0 + chunk * 4));
             }
+            lds_turn();
         }
     } else if (!RM && args.checksum != nullptr) {
         // int64 sum of the int32 accumulators (W8A8) or double sum of the fp32 ones
@@ -1528,7 +1604,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
                 for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
-                        const bool rowOwn = row_base + mb * 32 + (r >> 2) * 8 + (r & 3) >= shiftM;
+                        const bool rowOwn = row_base + mb * 32 + rowOf(r) >= shiftM;
 #pragma unroll
                         for (int nb = 0; nb < 4; ++nb) {
                             const bool own = rowOwn && col0 + 32 * nb >= shiftN;
@@ -1621,7 +1697,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
 }
 
 // One workgroup per tile, or per k slice of a tile.
-template <uint32_t DT, int WM, bool TB = false, bool RM = false, bool RG = false, bool TA = false, int NS = 3, bool PP = false, bool AQ = false, bool W8 = false>
+template <uint32_t DT, int WM, bool TB = false, bool RM = false, bool RG = false, bool TA = false, int NS = 3, bool PP = false, bool AQ = false, bool W8 = false, bool M16 = WM == 4>
 __global__ void __launch_bounds__(128 * WM * (W8 ? 2 : 1), NS == 3 ? 2 : 1) gemm_dma_kernel(const GemmArgs args)
 {
     __shared__ __attribute__((aligned(1024))) unsigned char smem[DmaPool<WM, NS, AQ, TB>::BYTES];
@@ -1639,7 +1715,7 @@ __global__ void __launch_bounds__(128 * WM * (W8 ? 2 : 1), NS == 3 ? 2 : 1) gemm
             pos = blockIdx.x / kSlices;
         }
     }
-    dma_tile<DT, WM, TB, RM, RG, TA, W8 ? 1 : 2, NS, PP, AQ, W8>(args, smem, pos, slice, kSlices, 0);
+    dma_tile<DT, WM, TB, RM, RG, TA, W8 ? 1 : 2, NS, PP, AQ, W8, 0, M16>(args, smem, pos, slice, kSlices, 0);
 }
 
 // Flexible mode: tiles of 64 * MB rows over the rows of all ranks (gemm_flex.h).  SL: k slices (a kernel of their own: either
@@ -1693,7 +1769,7 @@ inline int launch_flex(const GemmArgs &args, int rowBlocks, hipStream_t s)
 //     that have to wait for a slot get the ones the kept halves leave, about one tile time before the end; as halves they
 //     fill those slots for half a tile time (their checksum halves meet through the workspace's counter block).
 // Requires the XCD-block order, whole tiles, A as [m,k], one launch for all tasks.
-template <uint32_t DT, bool TB>
+template <uint32_t DT, bool TB, bool M16>
 __global__ void __launch_bounds__(256, 2) gemm_dma_split_kept_kernel(const GemmArgs args, const uint32_t keptPerXcd, const uint32_t tailPerXcd)
 {
     __shared__ __attribute__((aligned(1024))) unsigned char smem[DmaPool<2>::BYTES];
@@ -1713,7 +1789,7 @@ __global__ void __launch_bounds__(256, 2) gemm_dma_split_kept_kernel(const GemmA
         sub = (t & 1u) * 64u;
     }
     if (half) dma_tile<DT, 2, TB, false, false, false, 1>(args, smem, posJ * 8u + x, 0, 1, sub);
-    else dma_tile<DT, 2, TB, false, false, false, 2>(args, smem, posJ * 8u + x, 0, 1, 0);
+    else dma_tile<DT, 2, TB, false, false, false, 2, 3, false, false, false, 0, M16>(args, smem, posJ * 8u + x, 0, 1, 0);
 }
 
 // A launch of at most one workgroup per CU has the whole LDS of a CU for each workgroup.  When its operands are too large to
@@ -1738,6 +1814,40 @@ inline bool deep_ring_pairs(const GemmArgs &a, uint64_t es)
 
 // Launch of the 128-row geometry: one instantiation per operand layout (A as [m][k] or [k][m], B as [k][n] or [n][k]) and
 // for ragged problems; one workgroup per tile, or per k slice of a tile.
+//
+// 16x16 MFMAs (mfma16.h): W8A8 launches with two workgroups on a CU and 24 steps of k or more.  A single workgroup has one wave per SIMD, which has
+// to issue an MFMA, fragment reads and copies every 16 cycles and falls behind, and a short loop is mostly start and end, where the lane swaps are.
+// 32x32 -> 16x16, us: 4096x1792x4096 pipelined 49.4 -> 47.2, 8192x1792x4096 69.5 -> 68.7 (by box: 71.4 and 67.6 before), 3552x4288x3840 90.9 -> 87.4,
+// pipelined 3328x2560x4864 58.9 -> 56.2, 7376x5056x5376 as [n,k] 245.0 -> 233.3; up to 256 workgroups 5160x2560x1280 30.8 -> 31.6, 17 steps
+// 5550x1088x3584 39.6 -> 43.5.  Not for 16-bit operands: ragged rows, whose epilogue spills more then, 7282x6656x5632 545 -> 546, 3232x7104x4608 214 -> 217.
+inline bool mfma16_pays(const GemmArgs &args, uint32_t workgroups) { return workgroups > 256u && args.K >= 1536u; }
+
+template <uint32_t DT, bool TB>
+inline void launch_split_kept(const GemmArgs &args, uint32_t keptPerXcd, hipStream_t s)
+{
+    const uint32_t tailPerXcd = split_tail_tiles(args, keptPerXcd);
+    const dim3 grid(args.sched.coreLoops + 8u * (keptPerXcd + tailPerXcd)), block(256);
+    if constexpr (DT == DT_I8) {
+        if (mfma16_pays(args, grid.x)) {
+            hipLaunchKernelGGL((gemm_dma_split_kept_kernel<DT, TB, true>), grid, block, 0, s, args, keptPerXcd, tailPerXcd);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((gemm_dma_split_kept_kernel<DT, TB, false>), grid, block, 0, s, args, keptPerXcd, tailPerXcd);
+}
+
+template <uint32_t DT, bool TB, bool RG>
+inline void launch_dma_plain(const GemmArgs &args, const dim3 grid, hipStream_t s)
+{
+    if constexpr (DT == DT_I8) {
+        if (mfma16_pays(args, grid.x)) {
+            hipLaunchKernelGGL((gemm_dma_kernel<DT, 2, TB, false, RG, false, 3, false, false, false, true>), grid, dim3(256), 0, s, args);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((gemm_dma_kernel<DT, 2, TB, false, RG, false>), grid, dim3(256), 0, s, args);
+}
+
 template <uint32_t DT>
 inline int launch_dma_128(const GemmArgs &args, hipStream_t s)
 {
@@ -1745,11 +1855,7 @@ inline int launch_dma_128(const GemmArgs &args, hipStream_t s)
     switch ((args.transA ? 4 : 0) | (args.transB ? 2 : 0) | ((args.flags & GF_RAGGED) ? 1 : 0)) {
         case 0:
             if (const uint32_t keptPerXcd = split_kept_tiles(args, args.K * (DT == DT_I8 ? 1u : 2u) / 64u))
-{
-                const uint32_t tailPerXcd = split_tail_tiles(args, keptPerXcd);
-                hipLaunchKernelGGL((gemm_dma_split_kept_kernel<DT, false>), dim3(args.sched.coreLoops + 8u * (keptPerXcd + tailPerXcd)), block, 0, s, args,
-                                   keptPerXcd, tailPerXcd);
-            }
+                launch_split_kept<DT, false>(args, keptPerXcd, s);
             else if (deep_ring(args, grid.x, DT == DT_I8 ? 1u : 2u)) {
                 if (deep_ring_pairs(args, DT == DT_I8 ? 1u : 2u))
                     hipLaunchKernelGGL((gemm_dma_kernel<DT, 2, false, false, false, false, 6, true, true>), grid, block, 0, s, args);
@@ -1757,20 +1863,16 @@ inline int launch_dma_128(const GemmArgs &args, hipStream_t s)
                     hipLaunchKernelGGL((gemm_dma_kernel<DT, 2, false, false, false, false, 6, true>), grid, block, 0, s, args);
             }
             else
-                hipLaunchKernelGGL((gemm_dma_kernel<DT, 2, false, false, false, false>), grid, block, 0, s, args);
+                launch_dma_plain<DT, false, false>(args, grid, s);
             break;
-        case 1: hipLaunchKernelGGL((gemm_dma_kernel<DT, 2, false, false, true, false>), grid, block, 0, s, args); break;
+        case 1: launch_dma_plain<DT, false, true>(args, grid, s); break;
         case 2:
             if (const uint32_t keptPerXcd = split_kept_tiles(args, args.K * (DT == DT_I8 ? 1u : 2u) / 64u))
-{
-                const uint32_t tailPerXcd = split_tail_tiles(args, keptPerXcd);
-                hipLaunchKernelGGL((gemm_dma_split_kept_kernel<DT, true>), dim3(args.sched.coreLoops + 8u * (keptPerXcd + tailPerXcd)), block, 0, s, args,
-                                   keptPerXcd, tailPerXcd);
-            }
+                launch_split_kept<DT, true>(args, keptPerXcd, s);
             else
-                hipLaunchKernelGGL((gemm_dma_kernel<DT, 2, true, false, false, false>), grid, block, 0, s, args);
+                launch_dma_plain<DT, true, false>(args, grid, s);
             break;
-        case 3: hipLaunchKernelGGL((gemm_dma_kernel<DT, 2, true, false, true, false>), grid, block, 0, s, args); break;
+        case 3: launch_dma_plain<DT, true, true>(args, grid, s); break;
         case 4: hipLaunchKernelGGL((gemm_dma_kernel<DT, 2, false, false, false, true>), grid, block, 0, s, args); break;
         case 5: hipLaunchKernelGGL((gemm_dma_kernel<DT, 2, false, false, true, true>), grid, block, 0, s, args); break;
         case 6: hipLaunchKernelGGL((gemm_dma_kernel<DT, 2, true, false, false, true>), grid, block, 0, s, args); break;

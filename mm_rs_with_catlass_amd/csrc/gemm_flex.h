@@ -165,11 +165,46 @@ __device__ __forceinline__ T wave_sum64(T v)
     return dpp_add64<0x143, 0xc>(half_sum64(v));   // row_bcast:31 into rows 2 and 3
 }
 
-// acc[mb][nb][r] of wave (wm, wn) is element (row, col) of the tile with
-//   row = wm*32*MB + mb*32 + (r>>2)*8 + h*4 + (r&3),  col = wn*128 + nb*32 + c32
-// NW waves, two of them side by side: tiles of 16 * MB * NW rows.
-template <uint32_t DT, int MB, int NW = 4>
-__device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename AccOf<DT>::type (&acc)[MB][4], unsigned char *smem, const FlexTile &t)
+// A wave's rows [32 * mb, +32) of its 128 columns into its staging area: rows of 512 bytes, 16-byte piece c of row r at c * 16 ^ flex_turn(r), which
+// keeps what is written together in different banks.  acc[mb][nb][r] of 32x32 MFMAs is row mb*32 + (r>>2)*8 + (lane>>5)*4 + (r&3), column nb*32 +
+// (lane&31); acc[i][j][r] of 16x16 ones (L16) row i*16 + (lane>>4)*4 + r, column j*16 + (lane&15).  What follows reads other lanes' values: the LDS
+// unit keeps a wave's accesses in order, the compiler is told by the empty asm statements.
+template <bool L16>
+__device__ __forceinline__ uint32_t flex_turn(uint32_t row) { return L16 ? ((row >> 2) & 3u) << 6 : ((row >> 2) & 1u) << 7; }
+
+template <bool L16, typename Acc>
+__device__ __forceinline__ void flex_stage(const Acc &acc, int mb, unsigned char *st, uint32_t lane)
+{
+    asm volatile("" ::: "memory");
+    if constexpr (L16) {
+        const uint32_t l16 = lane & 15, quad = lane >> 4;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const auto e = acc[2 * mb + i][j][r];
+                    *(int *)(st + (i * 16 + quad * 4 + r) * 512 + (((j * 16 + l16) * 4) ^ (quad << 6))) = __builtin_bit_cast(int, e);
+                }
+    } else {
+        const uint32_t c32 = lane & 31, h = lane >> 5;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const uint32_t wrow = (r >> 2) * 8 + h * 4 + (r & 3);
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) {
+                const auto e = acc[mb][nb][r];
+                *(int *)(st + wrow * 512 + (((nb * 32 + c32) * 4) ^ (h << 7))) = __builtin_bit_cast(int, e);
+            }
+        }
+    }
+    asm volatile("" ::: "memory");
+}
+
+// Wave (wm, wn) has rows wm*32*MB and columns wn*128 of the tile.  NW waves, two of them side by side: tiles of 16 * MB * NW rows.
+template <uint32_t DT, int MB, int NW, bool L16, typename Acc>
+__device__ __forceinline__ void flex_epilogue(const GemmArgs &args, const Acc &acc, unsigned char *smem, const FlexTile &t)
 {
     constexpr bool I8 = DT == DT_I8;
     constexpr uint32_t ROWS = 16u * MB * NW, TABLE = NW == 4 ? 128u : ROWS;
@@ -177,7 +212,6 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
     const int tid = threadIdx.x, lane = tid & 63;
     const uint32_t w = __builtin_amdgcn_readfirstlane((uint32_t)tid >> 6);
     const uint32_t wm = w >> 1, wn = w & 1u;
-    const int c32 = lane & 31, h = lane >> 5;
     const bool redI32 = I8 && (args.flags & GF_REDUCE_INT32) != 0;
     const bool store = (args.flags & GF_OUTBOUND_STORE) != 0;
 
@@ -274,15 +308,7 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
 
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const uint32_t wrow = (r >> 2) * 8 + h * 4 + (r & 3);
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb) {
-                const auto e = acc[mb][nb][r];
-                *(int *)(st + wrow * 512 + (((nb * 32 + c32) * 4) ^ (h << 7))) = __builtin_bit_cast(int, e);
-            }
-        }
+        flex_stage<L16>(acc, mb, st, lane);
 #pragma unroll
         for (int half = 0; half < 2; ++half) {   // 16 rows: a lane has eight of them, two apart
             __builtin_amdgcn_sched_barrier(0);   // (one block's registers at a time)
@@ -291,7 +317,7 @@ __device__ __forceinline__ void flex_epilogue(const GemmArgs &args, typename Acc
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const uint32_t wrow = half * 16 + j * 2 + lrow;
-                cur[j] = *(const v4i *)(st + wrow * 512 + ((chunk * 16) ^ (((wrow >> 2) & 1) << 7)));
+                cur[j] = *(const v4i *)(st + wrow * 512 + ((chunk * 16) ^ flex_turn<L16>(wrow)));
                 d[j] = dst[wm * 32 * MB + mb * 32 + wrow];
                 if constexpr (I8) cur[j] += bv;
             }
@@ -497,19 +523,11 @@ __device__ __forceinline__ void flex_store_partial(const GemmArgs &args, Acc (&a
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
         if (wm * 32 * MB + mb * 32 >= kHi || wm * 32 * MB + mb * 32 + 32 <= kLo) continue;   // (wave-uniform)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const uint32_t wrow = (r >> 2) * 8 + h * 4 + (r & 3);
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb) {
-                const auto e = acc[mb][nb][r];
-                *(int *)(st + wrow * 512 + (((nb * 32 + c32) * 4) ^ (h << 7))) = __builtin_bit_cast(int, e);
-            }
-        }
+        flex_stage<false>(acc, mb, st, lane);
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
             const uint32_t wrow = j * 2 + lrow, i = wm * 32 * MB + mb * 32 + wrow;
-            const v4i v = *(const v4i *)(st + wrow * 512 + ((chunk * 16) ^ (((wrow >> 2) & 1) << 7)));
+            const v4i v = *(const v4i *)(st + wrow * 512 + ((chunk * 16) ^ flex_turn<false>(wrow)));
             if (i >= kLo && i < kHi && lcol < t.colsValid) *(v4i *)(part + (size_t)i * args.N) = v;
         }
     }

@@ -42,9 +42,17 @@ __device__ __forceinline__ uint32_t b16_slot(uint32_t row)
     else return ((row & 3u) << 2) | (((row >> 3) & 1u) << 1);
 }
 
-// The same values as a 32x32 MFMA's: block (2 * mb + br, 2 * nb + bc) of 16x16 holds rows 16 * br + 4 * (lane >> 4) + r; of a 32x32 block a lane holds column
-// lane & 31 and rows 8 * (reg >> 2) + 4 * (lane >> 5) + (reg & 3).  Bits 5 and 4 of the lane are a, b; swapping b with bc, then a with b, takes
-// (lane a b, register bc) to (lane b bc, register a).
+// Rows of 64 bytes of k: piece c of row `row` lies at slot c ^ k16_slot(row).  A 16-byte read is served 16 lanes at a time, of rows 0-3 and 12-15
+// the one piece and of rows 4-11 the next, or the other way round.
+__device__ __forceinline__ uint32_t k16_slot(uint32_t row)
+{
+    const uint32_t q = row >> 2;
+    return (((q ^ (q >> 1)) & 1u) << 1) | ((q >> 1) & 1u);
+}
+
+// The same values, 32 columns to a register as with 32x32 MFMAs: block (2 * mb + br, 2 * nb + bc) of 16x16 holds rows 16 * br + 4 * (lane >> 4) + r; of
+// a 32x32 block a lane then holds column lane & 31 and rows 16 * (reg >> 3) + 8 * (lane >> 5) + (reg & 7).  (Bit 4 of the lane, four rows, changes
+// places with bc.  The rows of 32x32 MFMAs' registers would take as many swaps again.)
 template <uint32_t DT, int MB, int NB>
 __device__ __forceinline__ void acc16_to_32(const typename Acc16Of<DT>::type (&x)[2 * MB][2 * NB], typename AccOf<DT>::type (&acc)[MB][NB])
 {
@@ -59,10 +67,8 @@ __device__ __forceinline__ void acc16_to_32(const typename Acc16Of<DT>::type (&x
                     const auto e0 = x[2 * mb + br][2 * nb][r], e1 = x[2 * mb + br][2 * nb + 1][r];
                     const auto s = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, e0), __builtin_bit_cast(uint32_t, e1), false, false);
                     const uint32_t s0 = s[0], s1 = s[1];
-                    const auto t = __builtin_amdgcn_permlane32_swap(s0, s1, false, false);
-                    const uint32_t t0 = t[0], t1 = t[1];
-                    acc[mb][nb][4 * (2 * br) + r] = __builtin_bit_cast(std::remove_const_t<decltype(e0)>, t0);
-                    acc[mb][nb][4 * (2 * br + 1) + r] = __builtin_bit_cast(std::remove_const_t<decltype(e0)>, t1);
+                    acc[mb][nb][8 * br + r] = __builtin_bit_cast(std::remove_const_t<decltype(e0)>, s0);
+                    acc[mb][nb][8 * br + 4 + r] = __builtin_bit_cast(std::remove_const_t<decltype(e0)>, s1);
                 }
 }
 
