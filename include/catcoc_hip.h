@@ -449,7 +449,7 @@ enum {
     CATCOC_KERNEL_GENERAL = 1,   /* bounds-checked kernels */
     CATCOC_KERNEL_ALIGNED = 2,   /* 128x256 and 256x256 tiles of whole or ragged problems */
     CATCOC_KERNEL_FLEXIBLE = 3,  /* 64x256 and 128x256 tiles over any rows */
-    CATCOC_KERNEL_SMALL = 4,     /* 32x32 to 128x128 tiles; 256x256: mixed with 128x128 ones */
+    CATCOC_KERNEL_SMALL = 4,     /* 32x32 to 192x128 tiles; 256x256: mixed with 128x128 ones */
     CATCOC_KERNEL_STREAMING = 5  /* explicit kept rows: 128x128 tiles in k slices, 32 columns over the whole k */
 };
 typedef struct CatcocLaunchInfo {

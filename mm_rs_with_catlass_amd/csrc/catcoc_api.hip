@@ -291,12 +291,20 @@ bool flex_ptrs_ok(const GemmArgs &a)
 // KiB a workgroup pulls in through its CU (more from the second round of workgroups on: the first leaves the caches cold), per MB of
 // operands, per MB of peers and outputs; rows of k off the 16-byte grid and B as [k,n] cost more per KiB, rows of a B tile that are no whole
 // cache line more per MB.  Half of the estimates are within 0.10 of the tiles' times and 0.06 of the others', nine in ten within 0.22
-// and 0.16.  The choice takes the tiles with the least, where that is at most the share below of the others' estimate: beyond it calls
-// start to lose (aligned tiles at 0.9: up to 0.15, flexible ones at 1.0: up to 0.3), up to it three of 413 lost more than 0.04.  Calls
-// that had aligned tiles take 0.82 of their time, those that had flexible ones 0.78; the best choice for each would be 0.79 and 0.76.
-// Figures of calls stand with the kernels that run them (gemm_few.h, gemm_mid.h, gemm_mixed.h); the other way round, other kernels / small tiles: fp16
-// 1116x4000x4160 78 / 92 us, 8144x5120x1696 on small tiles alone 188 / 203.
-constexpr double kAlignedShare = 0.85, kOtherShare = 0.87;
+// and 0.16.  The tiles of 96, 160 and 192 rows stand on the scale of the 128-row one's (their times relative to it, 1600 calls).  The estimates of
+// 128-column tiles are from when these ran 32x32 MFMAs and come out 0.11 high, of flexible tiles in k slices 0.12, of mixed launches 0.02, of aligned
+// tiles 0.05, so the choice, the tiles with the least, compares shares (other_share): 1571 drawn calls of 1e9 operations and more, each timed on every
+// tile, then take 1.015 of the best choice's time for each and 0.69 of the time of the kernels that would run else; 39 of them lose more than 0.04
+// against those.  With five tiles and the shares before that it was 1.065 and 0.72.  Those still hold for calls unlike the fitted ones: k below 512,
+// columns that are no multiple of 32, one rank or more than eight.
+// Figures of calls stand with the kernels that run them (gemm_few.h, gemm_mid.h, gemm_mixed.h).
+constexpr double kMixedShare = 1.1;   // of a mixed launch's estimate, against the other tiles'
+enum OtherKernel { OTHER_NONE, OTHER_ALIGNED, OTHER_FLEXIBLE, OTHER_SLICED, OTHER_STREAMING };
+struct Other {        // what a launch would run else, and for how long by its estimate
+    OtherKernel kernel;
+    double us;
+    bool pipelined;   // its GEMM launch and the comm launch behind it
+};
 struct SmallTile {
     int rows, cols;   // 0: the launch is not one for them; 256x256: the large ones of a mixed launch
 };
@@ -304,10 +312,11 @@ struct SmallTileCost {
     int rows, cols;
     double launch, workgroup, kib, mb, partLine, moved, off16, kn, later;
 };
-constexpr SmallTileCost kSmallTiles[5] = {
+constexpr SmallTileCost kSmallTiles[] = {
     {32, 32, 1.84, 2.42, 0.0118, 0.051, 0.044, 0.234, 0.0049, 0.0053, 0.0},  {32, 64, 2.00, 2.86, 0.0101, 0.079, 0.220, 0.248, 0.0039, 0.0014, 0.0},
     {64, 64, 1.59, 3.86, 0.0120, 0.038, 0.174, 0.238, 0.0033, 0.0010, 0.0},  {64, 128, 3.47, 3.94, 0.0086, 0.187, 0.0, 0.174, 0.0040, 0.0008, 0.0039},
-    {128, 128, 4.98, 4.59, 0.0085, 0.235, 0.0, 0.185, 0.0045, 0.0010, 0.0051}};
+    {96, 128, 3.52, 5.10, 0.0086, 0.213, 0.0, 0.167, 0.0046, 0.0011, 0.0049},  {128, 128, 4.98, 4.59, 0.0085, 0.235, 0.0, 0.185, 0.0045, 0.0010, 0.0051},
+    {160, 128, 5.10, 6.26, 0.0093, 0.245, 0.0, 0.190, 0.0042, 0.0011, 0.0053}, {192, 128, 6.15, 6.57, 0.0092, 0.264, 0.0, 0.192, 0.0038, 0.0010, 0.0051}};
 
 struct CallSize {
     double rows, kib, mb, moved;   // rows of the problem, KiB of a row of k, MB of operands, MB of peers and outputs
@@ -339,6 +348,8 @@ double flex_us(const GemmArgs &a, uint32_t es, int blocks)
     return 2.5 + rounds * (steps * (0.239 + (a.transB ? 0.126 : 0.0) + (blocks == 2 ? 0.230 : 0.0)) + 3.2) - (wgs > 256.0 ? 0.0855 * wgs / 256.0 * steps : 0.0) +
            (a.sched.op == OP_REDUCE_SCATTER ? 1.11 * a.nPeers : 0.0) + 0.156 * c.moved + 0.150 * c.mb;
 }
+
+Other other_flexible(const GemmArgs &a, uint32_t es, int blocks) { return {a.fx.slices > 1 ? OTHER_SLICED : OTHER_FLEXIBLE, flex_us(a, es, blocks), false}; }
 
 // Rows of a mixed launch that run on 256x256 tiles: all but a reduce-scatter's kept ones and what fills the CUs that whole rounds of
 // large tiles leave idle.  A CU takes one workgroup at a time, the large ones first; `us` is when the last is done.
@@ -413,9 +424,29 @@ double streaming_us(const GemmArgs &a)
 // Sliced small tiles: of a row tile that somebody keeps or stores, every slice leaves its partial tile in the workspace.
 uint64_t few_partials(const SmallTileCost &t, uint32_t keptTiles, uint32_t n, uint32_t slices) { return (uint64_t)keptTiles * ceil_div(n, (uint32_t)t.cols) * slices * t.rows * t.cols * 4u; }
 
-// The small tile a launch (operands, schedule, kept rows, flags and pointers filled in) runs, where the others would take `other` us;
+// A call like those the estimates were compared on (explicit kept rows: any number of ranks).
+bool fitted_call(const GemmArgs &a) { return a.N % 32 == 0 && a.K >= 512 && ((a.flags & GF_ROW_MASK) != 0 || (a.sched.P >= 2 && a.sched.P <= 8)); }
+
+// The share of the other kernels' estimate up to which small tiles (wide: of 128 columns, or mixed) run.
+double other_share(const GemmArgs &a, uint32_t es, const Other &o, bool sums, bool wide)
+{
+    const bool rowMask = (a.flags & GF_ROW_MASK) != 0, rs = a.sched.op == OP_REDUCE_SCATTER;
+    if (fitted_call(a)) {
+        // (pipelined calls at 0.8 miss 0.01, but none of those below 640 of k does; two ranks' kept rows are half of all, and aligned tiles then stream
+        // peers under each other's loops; the 62 calls with 16-bit operands on whole flexible tiles as [k,n] miss 0.015)
+        if (o.pipelined) return a.K < 640 ? 0.8 : 0.95;
+        if (o.kernel == OTHER_STREAMING) return 0.87;
+        return o.kernel == OTHER_SLICED ? 0.9 : o.kernel == OTHER_FLEXIBLE && es == 2 && !a.transB ? 0.95 : rs && a.sched.P == 2 ? 1.0 : 1.1;
+    }
+    double share = o.kernel == OTHER_ALIGNED ? 0.85 : 0.87;
+    if (rs && !sums && wide) share *= 1.15;   // (kept rows are dealt out)
+    if (!rs && !rowMask) share *= 1.05;
+    return o.pipelined ? 0.9 * share : share;
+}
+
+// The small tile a launch (operands, schedule, kept rows, flags and pointers filled in) runs, given what would run else;
 // fills args.fx for it.  room: the bytes behind the workspace's counter block (a.skCount, if there is one) that the launch may use.
-SmallTile small_tile(GemmArgs &a, uint32_t es, double other, uint64_t room = 0)
+SmallTile small_tile(GemmArgs &a, uint32_t es, const Other &other, uint64_t room = 0)
 {
     const SmallTile no = {0, 0};
     const SchedParams &s = a.sched;
@@ -444,7 +475,14 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other, uint64_t room = 0)
         const uint32_t least = t.cols != 128 || dealt < 2 ? t.rows : (uint32_t)rows / dealt - a.keptRows / dealt - 1u;   // rows of others that a tile has
         return (int32_t)least < 1 ? 0u : ((h + least - 2u) / least + 1u) * (256u / t.cols);
     };
+    const bool fitted = fitted_call(a);
     for (const SmallTileCost &t : kSmallTiles) {
+        if (t.cols == 128 && t.rows != 64 && t.rows != 128) {
+            // (rows of A and of the peers in 31-bit offsets from a tile's first; the blocks of 128 rows that explicit kept rows' sums are of end where
+            // tiles do.  96 rows of an all-reduce or all-gather as [k,n] are left out: with them 1.0144 of the best choices' time, without 1.0149)
+            if (!fitted || ldaB * t.rows > 0x7fffffffull || (a.nPeers && (uint64_t)a.peerLd * 4u * t.rows > 0x7fffffffull) || (sums && rowMask)) continue;
+            if (t.rows == 96 && s.op != OP_REDUCE_SCATTER && !rowMask && !a.transB) continue;
+        }
         if (sums && es != 1 && (sum_parts(t) == 0 || s.coreLoops * sum_parts(t) > kCounterBlockBytes / 16u)) continue;
         if (sums && rowMask && (t.cols != 128 || (t.rows < 128 && rows > (uint64_t)t.rows)) && (a.skCount == nullptr || (rows + 127) / 128 * ceil_div(a.N, 128u) > kCounterBlockBytes / 16u))
             continue;
@@ -478,14 +516,10 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, double other, uint64_t room = 0)
     if (!sums && rows >= 512 && !(s.op == OP_REDUCE_SCATTER && s.P == 2) && kBytes >= 1024 && rows * a.N >= 128ull * 256ull * 256ull) {
         mixed = mixed_rows(a, es, (uint32_t)rows);
         mixed.us = mixed.us * (kBytes % 16 ? 0.81 : 0.68) + 0.113 * c.moved + 0.35 * c.mb;
-        if (mixed.us > least) mixed.large = 0;
+        if ((fitted ? kMixedShare * mixed.us : mixed.us) > least) mixed.large = 0;
     }
-    // (with the kept rows dealt out the shares' margin is not needed: 199 reduce-scatters then take 1.009 of the best choice's time for each, 1.018
-    // with it; two of them lost 0.12 and 0.20, one of the two with the margin as well)
-    if (s.op == OP_REDUCE_SCATTER && !rowMask && !sums && (mixed.large || best->cols == 128)) other *= 1.15;
-    // (all-reduce and all-gather: 52 of 64 rows and more take 1.013 of the best choice's time for each, 1.025 without this; the same one loses)
-    if (s.op != OP_REDUCE_SCATTER && !rowMask) other *= 1.05;
-    if ((mixed.large ? mixed.us : least) > other || tiles > (1u << 24) || !flex_ptrs_ok(a)) return no;
+    if (other.kernel != OTHER_NONE && (mixed.large ? mixed.us : least) > other_share(a, es, other, sums, mixed.large || best->cols == 128) * other.us) return no;
+    if (tiles > (1u << 24) || !flex_ptrs_ok(a)) return no;
     a.fx.dRank = make_fast_div(s.mRank);
     a.splitK = 0;
     if (mixed.large) {
@@ -795,7 +829,7 @@ SmallTile planned_small(const Plan &p, bool dma, bool flex, GemmArgs &g)
     if ((dma || p.preferFlex) && (g.flags & GF_OUTBOUND_STORE) == 0 && g.checksum == nullptr && g.sched.op == OP_REDUCE_SCATTER && splittable_kept_tiles(g) != 0) return {0, 0};
     g.skCount = p.counters;
     const uint32_t es = elem_size(p.dtype);
-    return small_tile(g, es, dma ? kAlignedShare * aligned_us(p.args, es) : flex ? kOtherShare * flex_us(p.args, es, p.flexBlocks) : 1e30, p.room);
+    return small_tile(g, es, dma ? Other{OTHER_ALIGNED, aligned_us(p.args, es), false} : flex ? other_flexible(p.args, es, p.flexBlocks) : Other{OTHER_NONE, 0.0, false}, p.room);
 }
 
 // CATCOC_FLAG_KEPT_WHOLE and CATCOC_FLAG_KEPT_SPLIT change no bit of a result: sums of floats in another order would.  So they do not enter the
@@ -1038,7 +1072,7 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
         if (sp.maySmall) {   // (the rest of these shapes runs whole 64x256 tiles or one thread per element, many times slower)
             GemmArgs g = a;
             g.skCount = counter_block(*d);
-            const SmallTile t = small_tile(g, 1, 1e30);
+            const SmallTile t = small_tile(g, 1, {OTHER_NONE, 0.0, false});
             if (t.rows) { launched(launch_small(DT_I8, g, t, stream)); return; }
         }
         const bool flex = sp.flexBlocks != 0 && flex_ptrs_ok(a);
@@ -1108,7 +1142,8 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
             if ((c.slices > 1 && g.fx.slices < 2 && (sp.large || sp.f > 1)) || !decode_flex_pays(g, sp.large) || !flex_ptrs_ok(g)) blocks = 0;
         }
         if (sp.maySmall) {
-            const SmallTile t = small_tile(small, 1, sp.wholeK ? 1e30 : kOtherShare * (blocks ? flex_us(g, 1, blocks) : streaming_us(g)), counter_room(*d, sp.workspaceBytes));
+            const SmallTile t = small_tile(small, 1, sp.wholeK ? Other{OTHER_NONE, 0.0, false} : blocks ? other_flexible(g, 1, blocks) : Other{OTHER_STREAMING, streaming_us(g), false},
+                                           counter_room(*d, sp.workspaceBytes));
             // (a call that takes the kept rows' int32 block as well and would run in k slices runs in k slices, of one kind or the other: what its
             // workspace query reports is held to be what runs there.  Whole small tiles would be faster: operands in the caches, 203x1792x4096 with
             // all rows kept 18.5 / 10.8 us, 512x1024x1024 of two ranks 12.8 / 6.3)
@@ -1307,8 +1342,7 @@ void launch_pipelined(bool quant, int dataType, void *computeStream, void *commS
                  (sp.coreLoops >= 384u || sp.coreLoops <= 128u || P == 2 || (P <= 4 && tiling->k <= 2048u));
     if (fused) g.nPeers = P - 1;
     // Small or mixed tiles do the same in one launch, for problems of any alignment.  The fused operator's choice, with the comm launch on the
-    // other side where it is not fused, and 0.9 of that (102 calls: none loses; at 1.0 eight lose 0.02 to 0.14, at 0.8 eight more miss 0.06 to
-    // 0.6).  GEMM and comm launch -> one, us, one row-block round of eight ranks: 1024x3904x768 40.4 ->
+    // other side where it is not fused.  GEMM and comm launch -> one, us, one row-block round of eight ranks: 1024x3904x768 40.4 ->
     // 16.3, 2048x10672x1024 68.8 -> 38.7, 3072x2304x6176 91.5 -> 70.9, 4096x8960x7072 325 -> 280, of four 512x3604x640 45.0 -> 11.8, of two
     // 1792x6784x1024 49.7 -> 24.7; the other way round 4096x1792x4096 48.9 / 59.7, 3072x576x1792 24.1 / 26.6.
     SmallTile small = {0, 0};
@@ -1316,7 +1350,7 @@ void launch_pipelined(bool quant, int dataType, void *computeStream, void *commS
     if (quant && P > 1 && oneRound && (given->flags & (CATCOC_FLAG_LINEAR_ORDER | CATCOC_FLAG_KEPT_WHOLE | CATCOC_FLAG_KEPT_SPLIT)) == 0) {
         const double comm = fused ? 0.0 : 4.5 + 0.8 * (P - 1) + 0.1e-6 * 4.0 * (P - 1) * g.keptRows * g.N;
         gs.nPeers = P - 1;
-        small = small_tile(gs, 1, flexBlocks ? 0.9 * kOtherShare * (flex_us(g, 1, flexBlocks) + comm) : dma ? 0.9 * kAlignedShare * (aligned_us(g, 1) + comm) : 1e30);
+        small = small_tile(gs, 1, flexBlocks ? Other{OTHER_FLEXIBLE, flex_us(g, 1, flexBlocks) + comm, true} : dma ? Other{OTHER_ALIGNED, aligned_us(g, 1) + comm, true} : Other{OTHER_NONE, 0.0, false});
     }
     if (small.rows) fused = true;
     // (a single round may run in the order of the fused operators: 4096x8192x8192 of two ranks, as [n,k], two launches 405 -> 337)

@@ -1,10 +1,15 @@
-// Tiles of 128 or 64 rows by 128 columns over the whole k range, one workgroup of eight waves per CU: the calls between few small tiles
+// Tiles of 64 to 192 rows by 128 columns over the whole k range, one workgroup of eight waves per CU: the calls between few small tiles
 // (gemm_few.h) and the two rounds of 128x256 tiles the aligned kernels want, and those whose rows, columns or k line up with nothing.
 //
-// The eight waves are two by two positions of 64x64 (or 32x64) times two groups that take the two halves of every chunk of 128 bytes
-// of k, so that each SIMD has two waves; the operands of a chunk sit in one of five (six) LDS stages, copied four (five) chunks ahead, one
-// barrier per chunk.  The two groups' partial tiles meet in LDS after the loop, and a thread then finishes four consecutive columns of
-// eight (four) rows, the peers three at a time in registers.
+// The eight waves are two by two positions of 16 * MB rows by 64 columns times two groups that take the two halves of every chunk of 128 bytes
+// of k, so that each SIMD has two waves; the operands of a chunk sit in one of four to six LDS stages, copied as many chunks ahead less one, one
+// barrier per chunk.  The two groups' partial tiles meet in LDS after the loop (side by side, or, from 160 rows on, each group handing over half of
+// its own), and a thread then finishes four consecutive columns of two rows per 32 of the tile, the peers two or three at a time in registers.
+//
+// Five numbers of rows, so that most calls find one that takes all CUs once: with one workgroup per CU a second round costs as much as the first.
+// 64 and 128 rows (or other kernels) -> one in between, us, calls behind each other: fp16 reduce-scatter 1312x7424x3840 of eight ranks 133 -> 80.5 (192
+// rows, 210 tiles; 128x256 tiles before), W8A8 with checksums 2584x11488x2048 123 -> 77.6 (192), bf16 all-gather 8 x [489,13232] x [13232,1280] 291 -> 206
+// (160), W8A8 two ranks 754x5808x7808 52.9 -> 42.9 (192), 1512x7232x1536 of four 36.8 -> 31.4 (96), fp16 420x1664x2688 of four 21.3 -> 16.6 (96).
 //
 // The MFMAs are 16x16 ones (mfma16.h): where the operands come out of the caches the matrix pipes run at their power limit.  Else HBM bounds (0.6 us
 // per chunk of 128x128), and a fixed 5.5 us (launch apart) of first copies, partial tiles and output.  Time per call, calls behind each other and
@@ -497,7 +502,10 @@ inline int launch_mid_tb(const GemmArgs &args, int tileRows, hipStream_t s)
 {
     const dim3 grid(args.fx.rowTiles * args.fx.colTiles), block(512);
     if (tileRows == 64) hipLaunchKernelGGL((gemm_mid_kernel<DT, TB, 2, GA>), grid, block, 0, s, args);
+    else if (tileRows == 96) hipLaunchKernelGGL((gemm_mid_kernel<DT, TB, 3, GA>), grid, block, 0, s, args);
     else if (tileRows == 128) hipLaunchKernelGGL((gemm_mid_kernel<DT, TB, 4, GA>), grid, block, 0, s, args);
+    else if (tileRows == 160) hipLaunchKernelGGL((gemm_mid_kernel<DT, TB, 5, GA>), grid, block, 0, s, args);
+    else if (tileRows == 192) hipLaunchKernelGGL((gemm_mid_kernel<DT, TB, 6, GA>), grid, block, 0, s, args);
     else return (int)hipErrorInvalidValue;
     return (int)hipGetLastError();
 }

@@ -757,3 +757,31 @@ def test_equal_rows_have_equal_sums_wherever_they_lie(case):
     assert ran() == tiles
     torch.cuda.synchronize()
     assert torch.equal(dump, dump[:1].expand(M, N))
+
+
+# 128-column tiles of 96, 160 and 192 rows: both layouts of the weights, rows, columns and k past a tile, a chunk and a 16-byte piece, dealt and consecutive rows
+@pytest.mark.parametrize("case", [(66, 5088, 616, 8, 7, False, False, "96x128 dealt"), (171, 1824, 808, 8, 0, True, True, "96x128 dealt"),
+                                  (306, 3392, 528, 4, 3, False, False, "160x128 dealt"), (158, 3328, 556, 8, 5, True, True, "160x128 dealt"),
+                                  (171, 3744, 568, 8, 5, False, True, "192x128 dealt"), (266, 4768, 544, 4, 3, True, False, "192x128 dealt")])
+def test_quant_rows_between(case):
+    test_quant_mixed_tiles(case)
+
+
+@pytest.mark.parametrize("case", [("allreduce", 630, 3680, 552, 2, 0, True, "96x128"), ("allgather", 637, 1568, 646, 2, 0, True, "96x128"),
+                                  ("reduce_scatter", 640, 4480, 894, 8, 4, False, "96x128 dealt"), ("allreduce", 586, 7680, 606, 2, 0, True, "160x128"),
+                                  ("allgather", 366, 6304, 564, 2, 1, True, "160x128"), ("reduce_scatter", 880, 5056, 668, 8, 2, False, "160x128 dealt"),
+                                  ("allgather", 95, 7424, 512, 8, 4, True, "192x128"), ("reduce_scatter", 1240, 4416, 524, 8, 2, True, "192x128 dealt")])
+def test_float_rows_between(case):
+    test_float_larger_tiles(case)
+
+
+@pytest.mark.parametrize("case", [(171, 1952, 556, 8, 2, False, True, "96x128 dealt"), (159, 3392, 524, 8, 4, False, False, "160x128 dealt"),
+                                  (117, 5440, 536, 8, 4, True, True, "192x128 dealt")])
+def test_quant_task_sums_rows_between(case):
+    test_quant_task_sums(case)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", [(334, 1696, 794, 4, 3, False, "96x128 dealt"), (132, 4288, 624, 8, 4, False, "160x128 dealt"), (141, 4768, 514, 8, 1, True, "192x128 dealt")])
+def test_float_task_sums_rows_between(case, dtype):
+    test_float_task_sums(case, dtype)
