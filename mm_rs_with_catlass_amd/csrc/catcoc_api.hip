@@ -292,7 +292,7 @@ bool flex_ptrs_ok(const GemmArgs &a)
 // operands, per MB of peers and outputs; rows of k off the 16-byte grid and B as [k,n] cost more per KiB, rows of a B tile that are no whole
 // cache line more per MB.  Half of the estimates are within 0.10 of the tiles' times and 0.06 of the others', nine in ten within 0.22
 // and 0.16.  The tiles of 96, 160 and 192 rows stand on the scale of the 128-row one's (their times relative to it, 1600 calls).  The estimates of
-// 128-column tiles are from when these ran 32x32 MFMAs and come out 0.11 high, of flexible tiles in k slices 0.12, of mixed launches 0.02, of aligned
+// 128-column tiles are from when these ran 32x32 MFMAs and come out 0.11 high, of flexible tiles in k slices 0.12, of aligned
 // tiles 0.05, so the choice, the tiles with the least, compares shares (other_share): 1571 drawn calls of 1e9 operations and more, each timed on every
 // tile, then take 1.015 of the best choice's time for each and 0.69 of the time of the kernels that would run else; 39 of them lose more than 0.04
 // against those.  With five tiles and the shares before that it was 1.065 and 0.72.  Those still hold for calls unlike the fitted ones: k below 512,
@@ -345,14 +345,16 @@ double flex_us(const GemmArgs &a, uint32_t es, int blocks)
     if (f > 1.0)
         return 9.1 + rounds * steps * (a.transB ? 0.434 : 0.345) + 4e-6 * 0.095 * f * (a.fx.keptOnly ? (double)a.keptRows : c.rows) * a.N + 0.263 * c.moved + 0.112 * c.mb;
     if (a.fx.late) return 8.1 + rounds * steps * (a.transB ? 0.59 : 0.44) + 0.45 * c.moved;
-    return 2.5 + rounds * (steps * (0.239 + (a.transB ? 0.126 : 0.0) + (blocks == 2 ? 0.230 : 0.0)) + 3.2) - (wgs > 256.0 ? 0.0855 * wgs / 256.0 * steps : 0.0) +
-           (a.sched.op == OP_REDUCE_SCATTER ? 1.11 * a.nPeers : 0.0) + 0.156 * c.moved + 0.150 * c.mb;
+    const double us = 2.5 + rounds * (steps * (0.239 + (a.transB ? 0.126 : 0.0) + (blocks == 2 ? 0.230 : 0.0)) + 3.2) - (wgs > 256.0 ? 0.0855 * wgs / 256.0 * steps : 0.0) +
+                      (a.sched.op == OP_REDUCE_SCATTER ? 1.11 * a.nPeers : 0.0) + 0.156 * c.moved + 0.150 * c.mb;
+    // (rows of k off the 16-byte grid, many tiles: their copies are bound by the caches)
+    const double off16 = blocks == 2 && (uint64_t)a.K * es % 16 != 0 ? wgs / 512.0 * c.kib * 8.0 * (a.transB ? 3.0 : 2.05) + 0.12 * c.moved : 0.0;
+    return us > off16 ? us : off16;
 }
 
 Other other_flexible(const GemmArgs &a, uint32_t es, int blocks) { return {a.fx.slices > 1 ? OTHER_SLICED : OTHER_FLEXIBLE, flex_us(a, es, blocks), false}; }
 
-// Rows of a mixed launch that run on 256x256 tiles: all but a reduce-scatter's kept ones and what fills the CUs that whole rounds of
-// large tiles leave idle.  A CU takes one workgroup at a time, the large ones first; `us` is when the last is done.
+// Rows of a mixed launch that run on 256x256 tiles, of all but a reduce-scatter's kept ones; `us`: the launch's estimate.
 struct MixedRows {
     uint32_t large;
     double us;
@@ -361,27 +363,45 @@ struct MixedRows {
 // A reduce-scatter's kept rows, with their peers, all run on the small tiles; with one rank every row is kept and there are no peers.
 bool kept_apart(const GemmArgs &a) { return a.sched.op == OP_REDUCE_SCATTER && a.sched.P > 1; }
 
+// When the last of the workgroups that `cus` CUs get of a launch is done: large ones first, then small ones, each on the first CU that is free.
+double part_us(uint64_t large, uint64_t small, double largeUs, double smallUs, uint32_t cus)
+{
+    const uint64_t l = (large * cus + 255u) / 256u, s = (small * cus + 255u) / 256u, part = l % cus, idle = cus - part;
+    const double start = (double)(l / cus) * largeUs, end = start + largeUs;   // of the last round of large ones
+    if (part == 0) return start + (double)((s + cus - 1u) / cus) * smallUs;
+    const uint64_t first = (uint64_t)(largeUs / smallUs) + 1u;   // small ones that a CU without one of those starts by the time they end
+    if (s <= idle * first) return fmax(end, start + (double)((s + idle - 1u) / idle) * smallUs);
+    const uint64_t left = s - idle * first, more = left / cus, rest = left % cus;
+    return fmax(end + (double)(more + (rest ? 1u : 0u)) * smallUs, start + (double)(first + more + (rest > part ? 1u : 0u)) * smallUs);
+}
+
+// Two bounds: the CUs' schedule (workgroups go to the XCDs and, mostly, to their four shader engines in turn: the mean of
+// what 32 and 8 CUs take, with small tiles a little longer for the 32, so that a row count that just fits does not look as good as one that fits easily), and the power limit, at which
+// large tiles on half of the CUs take less time each than on all.  Fitted to 11200 launches of 1860 calls with one to all of their rows on large
+// tiles: half of them within 0.04, nine in ten within 0.11; the count with the least estimate takes 1.011 of the best one's time.  With large tiles at
+// 9 us + 1.7 per chunk whatever the others do, as before 16x16 MFMAs, it was 1.03 of it, and calls on them 1.055 of their best choice's time (1.025
+// now): pipelined W8A8 3584x15600x5120 as [n,k] of four ranks 378 -> 297 us, all-gather 4 x [591,8296] x [8296,6400] 277 -> 219,
+// W8A8 with stored tiles 6720x6144x2048 104 -> 83.8.
 MixedRows mixed_rows(const GemmArgs &a, uint32_t es, uint32_t rows)
 {
-    const double chunks = call_size(a, es).kib * 8.0;
+    const CallSize c = call_size(a, es);
+    const double chunks = c.kib * 8.0;
+    const bool off16 = (uint64_t)a.K * es % 16 != 0;
     const uint32_t kept = kept_apart(a) ? a.keptRows : 0u;
-    const double large = 9.0 + 1.70 * chunks + (kept ? 0.0 : 4.4 * a.nPeers), small = 8.0 + 0.55 * chunks + 1.1 * a.nPeers;
-    const uint32_t largeCols = ceil_div(a.N, 256u), smallCols = ceil_div(a.N, 128u);
+    const double large = 5.1 + chunks * (off16 ? 1.28 : 1.11) + (kept ? 0.0 : 2.4 * a.nPeers), small = 5.2 + chunks * (off16 ? 0.515 : 0.37) + 0.175 * a.nPeers;
+    const uint32_t largeCols = ceil_div(a.N, 256u), smallCols = ceil_div(a.N, 128u), most = ceil_div(rows - kept, 256u);
+    // (as few rows on large tiles as leave two rounds of them to the small ones; of a wide range every second, third .. count)
+    const uint32_t range = umin(most - 1u, ceil_div(512u, largeCols)), step = range / 32u + 1u;
     MixedRows best = {0, 0.0};
-    for (uint32_t t = 1; t <= ceil_div(rows - kept, 256u); ++t) {
+    for (uint32_t t = most - range / step * step; t <= most; t += step) {
         const uint32_t r = umin(256u * t, rows - kept);
-        const double nLarge = (double)t * largeCols, nSmall = (double)ceil_div(rows - r, 128u) * smallCols;
-        const double full = floor(nLarge / 256.0), part = nLarge - 256.0 * full;
-        double us = full * large;
-        if (part == 0.0) {
-            us += ceil(nSmall / 256.0) * small;
-        } else {
-            const double idle = (256.0 - part) * floor(large / small), beside = ceil(nSmall / (256.0 - part)) * small;
-            if (nSmall <= idle) us += beside > large ? beside : large;
-            else us += large + ceil((nSmall - idle) / 256.0) * small;
-        }
-        if (best.large == 0 || us < best.us) best = {r, us};
+        const uint64_t l = (uint64_t)t * largeCols, s = (uint64_t)ceil_div(rows - r, 128u) * smallCols;
+        const double cus = 0.5 * (part_us(l, s, large, 1.1 * small, 32u) + part_us(l, s, large, small, 8u));
+        const double power = 1.48 * chunks * ((double)l + 0.306 * s) / 256.0, c2 = cus * cus, p2 = power * power;
+        const double us = sqrt(sqrt(c2 * c2 + p2 * p2));
+        if (best.large == 0 || us <= best.us) best = {r, us};
     }
+    best.us += 4.0 + 0.124 * c.moved + 0.05 * c.mb;
     return best;
 }
 
@@ -428,10 +448,15 @@ uint64_t few_partials(const SmallTileCost &t, uint32_t keptTiles, uint32_t n, ui
 bool fitted_call(const GemmArgs &a) { return a.N % 32 == 0 && a.K >= 512 && ((a.flags & GF_ROW_MASK) != 0 || (a.sched.P >= 2 && a.sched.P <= 8)); }
 
 // The share of the other kernels' estimate up to which small tiles (wide: of 128 columns, or mixed) run.
-double other_share(const GemmArgs &a, uint32_t es, const Other &o, bool sums, bool wide)
+double other_share(const GemmArgs &a, uint32_t es, const Other &o, bool sums, bool wide, bool large)
 {
     const bool rowMask = (a.flags & GF_ROW_MASK) != 0, rs = a.sched.op == OP_REDUCE_SCATTER;
     if (fitted_call(a)) {
+        // (aligned tiles that are all whole come out 0.07 to 0.2 shorter than their estimate in reduce-scatters, most with checksums, which store
+        // nothing; 770 calls of whole tiles: W8A8 8192x2048x3072 as [n,k] 69.6 aligned, 90.5 mixed; with checksums 2048x4096x6144 67.5, 76.6 on 128x128)
+        const bool whole = o.kernel == OTHER_ALIGNED && rs && a.sched.P > 2 && a.sched.mRank % a.sched.m0 == 0 && a.N % a.sched.n0 == 0;
+        if (large) return whole ? (o.pipelined ? 0.9 : 0.96) : rs ? 1.0 : 1.05;
+        if (whole && sums) return 0.95;
         // (pipelined calls at 0.8 miss 0.01, but none of those below 640 of k does; two ranks' kept rows are half of all, and aligned tiles then stream
         // peers under each other's loops; the 62 calls with 16-bit operands on whole flexible tiles as [k,n] miss 0.015)
         if (o.pipelined) return a.K < 640 ? 0.8 : 0.95;
@@ -510,15 +535,13 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, const Other &other, uint64_t room
         }
     }
     if (best == nullptr) return no;
-    // (from half a round of large tiles' work on; k in at least a few pairs of steps; two ranks keep so many rows that small tiles are
-    // most of the launch: W8A8 3906x5600x3200 113 / 131, fp16 4790x6016x6272 369 / 394)
+    // (from three eighths of a round of large tiles on; k in at least a few pairs of steps)
     MixedRows mixed = {0, 0.0};
-    if (!sums && rows >= 512 && !(s.op == OP_REDUCE_SCATTER && s.P == 2) && kBytes >= 1024 && rows * a.N >= 128ull * 256ull * 256ull) {
+    if (!sums && rows >= 512 && kBytes >= 1024 && rows * a.N >= 96ull * 256ull * 256ull) {
         mixed = mixed_rows(a, es, (uint32_t)rows);
-        mixed.us = mixed.us * (kBytes % 16 ? 0.81 : 0.68) + 0.113 * c.moved + 0.35 * c.mb;
         if ((fitted ? kMixedShare * mixed.us : mixed.us) > least) mixed.large = 0;
     }
-    if (other.kernel != OTHER_NONE && (mixed.large ? mixed.us : least) > other_share(a, es, other, sums, mixed.large || best->cols == 128) * other.us) return no;
+    if (other.kernel != OTHER_NONE && (mixed.large ? mixed.us : least) > other_share(a, es, other, sums, mixed.large || best->cols == 128, mixed.large != 0) * other.us) return no;
     if (tiles > (1u << 24) || !flex_ptrs_ok(a)) return no;
     a.fx.dRank = make_fast_div(s.mRank);
     a.splitK = 0;
