@@ -1,14 +1,19 @@
 // Few small tiles, each over the whole k range or in k slices, in ONE launch: the calls whose 64x256 tiles would leave most CUs idle (a decode batch
 // of a float model, a short prompt, a mixed batch of W8A8 rows).
 //
-// A tile is 32 or 64 rows by 32 or 64 columns, a workgroup of four waves per tile, and the waves divide k between them instead of
-// the tile: the k range is cut into chunks of 128 bytes, dealt round-robin, and every wave streams its chunks of A and B into a ring
-// of its own in LDS with direct-to-LDS copies, reads a chunk's fragments while the MFMAs of the chunk before run, and waits for
-// nobody: a ring is ordered by its wave's vector-memory counter alone, no barrier in the loop.  The four partial tiles meet in LDS,
-// after which a thread holds four consecutive columns of a row and finishes them.  The peers' values of the tile's kept rows are
-// requested around the first copies, into registers, so that their stream and the operands' are in flight together on every CU.
+// A tile is 32 or 64 rows by 32 or 64 columns, a workgroup of eight waves per tile.  Four of them stream the operands and divide k between them instead
+// of the tile: the k range is cut into chunks of 128 bytes, dealt round-robin, and every wave streams its chunks of A and B into a ring
+// of its own in LDS with direct-to-LDS copies, reads a chunk's fragments (64x64: half a chunk's) while the MFMAs of the one before run, and waits for
+// nobody: a ring is ordered by its wave's vector-memory counter alone, no barrier in the loop.  The other four finish the tile: they fetch scales
+// and the peers' values of the tile's kept rows into registers while the loop runs, work out where rows go, and once the partial tiles are in LDS
+// each of their threads holds four consecutive columns of a row, adds the peers and writes.  With one set of waves for both, a ring's copies
+// waited for the peers in front of them, as a wave's counter retires in order, and their registers for the loop.  Where k is longer than the rings
+// the finishing waves ask for the peers once the first copies are on their way (one barrier): a CU's requests are answered in order, so peers in front
+// of those hold the loop up (43x6912x672 14.4 -> 15.3 us) and behind them they do not (14.5); shorter loops take both at once (92x768x5248 6.8 -> 5.9).
+// One set of four waves -> this, same results: 270 drawn calls take 0.95 of their time, 203x1792x4096 12.55 -> 11.3 us, 16x1024x8192 6.49 -> 6.07,
+// W8A8 reduce-scatter 192x520x2912 of eight ranks 8.6 -> 6.4, two ranks' 284x576x1408 with explicit kept rows 7.1 -> 5.4.
 //
-// Bound by launch and latency (of 16x1024x8192's 7.5 us an empty launch is 2.7 and the chain arguments - copies - partial tiles -
+// Bound by launch and latency (of 16x1024x8192's 7.1 us out of HBM an empty launch is 2.7 and the chain arguments - copies - partial tiles -
 // output about 2.5), past that by what reaches the CUs: 256 of them pull 60-85 GB/s each through their copies.  That is why a tile is
 // small rather than sliced: 64x256 tiles in k slices used 64 to 128 CUs, and the second launch that added the slices and the peers cost
 // 3.5 to 6 us.  Time per call, calls behind each other and their operands out of HBM (more sets of them than the caches hold),
@@ -172,14 +177,14 @@ template <int MB, int NB> struct FewGeom
 
 // GA: all-gather; the rows of A lie in the ranks' shards, one behind the other.  SL: k slices, args.fx.slices workgroups per tile.
 template <uint32_t DT, bool TB, int MB, int NB, bool GA, bool SL>
-__global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
+__global__ void __launch_bounds__(512, 1) gemm_few_kernel(const GemmArgs args)
 {
     using G = FewGeom<MB, NB>;
     using Acc = typename AccOf<DT>::type;
     constexpr bool I8 = DT == DT_I8;
     constexpr int ES = I8 ? 1 : 2;
     constexpr int ACP = G::ACP, BM = G::BM, BN = G::BN, UN = G::UN, NS = G::NS, BCP = BN / 8;
-    constexpr int PF = 8;                            // peers held in registers from the start
+    constexpr int PF = UN >= 4 ? 7 : 8;              // peers held in registers from the start
     __shared__ __attribute__((aligned(1024))) unsigned char smem[G::POOL];
 
     // The arguments come from host memory: named here, they arrive in a few wide loads behind one wait instead of one round trip
@@ -194,9 +199,10 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
         asm volatile("" : : "s"(peer[0]), "s"(peer[1]), "s"(peer[2]), "s"(peer[3]), "s"(peer[4]), "s"(peer[5]), "s"(peer[6]), "s"(peer[7]), "s"(a0), "s"(b0),
                  "s"(args.d), "s"(args.scaleM), "s"(args.scaleN), "s"(args.bias), "s"(args.lda), "s"(args.ldb), "s"(args.ldd), "s"(peerLd), "s"(peerRowOffset),
                  "s"(N), "s"(K), "s"(args.nPeers), "s"(keptBegin), "s"(keptRows), "s"(flags), "s"(args.outDtype), "s"(rows), "s"(rowTiles), "s"(colTiles));
-    else asm volatile("" : : "s"(peer[0]), "s"(peer[1]), "s"(peer[2]), "s"(peer[3]), "s"(peer[4]), "s"(peer[5]), "s"(peer[6]), "s"(peer[7]));
-    const int tid = threadIdx.x, lane = tid & 63;
-    const uint32_t w = __builtin_amdgcn_readfirstlane((uint32_t)tid >> 6);
+    else asm volatile("" : : "s"(peer[0]), "s"(peer[1]), "s"(peer[2]), "s"(peer[3]), "s"(peer[4]), "s"(peer[5]), "s"(peer[6]));
+    const uint32_t wave = __builtin_amdgcn_readfirstlane((uint32_t)threadIdx.x >> 6), w = wave & 3u;
+    const bool streams = wave < 4u;   // waves 0 to 3 stream the operands, 4 to 7 finish
+    const int tid = threadIdx.x & 255, lane = tid & 63;
     const int c32 = lane & 31, h = lane >> 5;
     const SchedParams &sp = args.sched;
     // XCD x takes the x-th eighth of the tiles, row tiles of a column strip behind each other: they share its columns of B
@@ -288,28 +294,31 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
         for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[mb][nb][r] = 0;
-    v4i fa[2][4][MB], fb[2][4][NB];
+    // Fragments in registers: of two chunks, or of two halves of a chunk (64x64: two chunks do not fit beside the accumulators).
+    constexpr int HALVES = UN >= 4 ? 2 : 1, KK = 4 / HALVES;
+    v4i fa[2][KK][MB], fb[2][KK][NB];
     uint32_t atRead = at;
-    auto read = [&](int s, uint32_t st) {   // the fragments of the chunk in stage st
+    auto read = [&](int s, uint32_t st, int half) {   // the fragments of the chunk, or half, in stage st
         const unsigned char *sa = ring + st * G::STAGE, *sb = sa + G::A_STAGE;
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
+        for (int kk = 0; kk < KK; ++kk) {
+            const int k4 = half * KK + kk;
 #pragma unroll
-            for (int mb = 0; mb < MB; ++mb) fa[s][kk][mb] = *(const v4i *)(sa + (mb * 32 + c32) * 128 + (((2 * kk + h) ^ ((c32 >> 1) & 7)) * 16));
+            for (int mb = 0; mb < MB; ++mb) fa[s][kk][mb] = *(const v4i *)(sa + (mb * 32 + c32) * 128 + (((2 * k4 + h) ^ ((c32 >> 1) & 7)) * 16));
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
                 if constexpr (TB) {
-                    fb[s][kk][nb] = *(const v4i *)(sb + (nb * 32 + c32) * 128 + (((2 * kk + h) ^ ((c32 >> 1) & 7)) * 16));
+                    fb[s][kk][nb] = *(const v4i *)(sb + (nb * 32 + c32) * 128 + (((2 * k4 + h) ^ ((c32 >> 1) & 7)) * 16));
                 } else {
                     const int i16 = lane & 15, t = (lane >> 4) & 1;
                     v2i t0, t1;
                     if constexpr (ES == 1) {   // lane i of 16: 8 bytes of k row i >> 1, half i & 1 of a 16-column piece
-                        const uint32_t r = 32 * kk + 16 * h + (i16 >> 1);
+                        const uint32_t r = 32 * k4 + 16 * h + (i16 >> 1);
                         const unsigned char *p = sb + r * BROW + (((nb * 2 + t) ^ bsw(r)) * 16) + (i16 & 1) * 8;
                         t0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((CATCOC_LDS v2i *)p);
                         t1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((CATCOC_LDS v2i *)(p + 8 * BROW));
                     } else {                   // four elements of k row i >> 2, quad i & 3 of a pair of pieces
-                        const uint32_t r = 16 * kk + 8 * h + (i16 >> 2);
+                        const uint32_t r = 16 * k4 + 8 * h + (i16 >> 2);
                         const unsigned char *p = sb + r * BROW + (((nb * 4 + t * 2 + ((i16 & 3) >> 1)) ^ bsw(r)) * 16) + (i16 & 1) * 8;
                         t0 = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((CATCOC_LDS v4s16 *)p));
                         t1 = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((CATCOC_LDS v4s16 *)(p + 4 * BROW)));
@@ -319,12 +328,12 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
             }
         }
         const uint32_t c = cw + 4u * atRead;
-        atRead = atRead + 1u == mine ? 0u : atRead + 1u;
+        if (half == HALVES - 1) atRead = atRead + 1u == mine ? 0u : atRead + 1u;
         if (c + 1u == nChunks && lastBytes != 128u) {
 #pragma unroll
-            for (int kk = 0; kk < 4; ++kk) {
+            for (int kk = 0; kk < KK; ++kk) {
                 // (word e of the incomplete piece is byte lastBytes - 16 + 4e of the chunk: its own from byte 16 * lastWhole on)
-                const uint32_t p = 2 * kk + h, from = p < lastWhole ? 0u : p == lastWhole ? (16u - lastBytes % 16u) / 4u : 4u;
+                const uint32_t p = 2 * (half * KK + kk) + h, from = p < lastWhole ? 0u : p == lastWhole ? (16u - lastBytes % 16u) / 4u : 4u;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
 #pragma unroll
@@ -368,8 +377,7 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
             }
         }
     };
-    auto fetch_all = [&]() {
-        if constexpr (!SL) fetch_peers();   // (else the last slice's)
+    auto fetch_scales = [&]() {
         if constexpr (I8) {
             if (colOk) {
                 sN = *(const v4f *)(args.scaleN + gcol);
@@ -380,14 +388,25 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
         }
     };
 
-    // In front of the first copies where a thread has many (a stream of its own), else right behind them.
-    if constexpr (UN >= 4) fetch_all();
     uint32_t issued = 0;
-    for (; issued < umin(mine, (uint32_t)NS); ++issued) issue(issued);
-    if constexpr (UN < 4) fetch_all();
     uint32_t st = 0;   // stage of chunk i
-    auto step = [&](auto S, uint32_t i) {
+    auto products = [&](int s) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = mfma32<DT>(fa[s][kk][mb], fb[s][kk][nb], acc[mb][nb]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto step = [&](auto S, uint32_t i) {   // S: where the fragments of chunk i, or of its last half, are
         constexpr int s = decltype(S)::value;
+        if constexpr (HALVES == 2) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the first half's are in registers
+            read(1, st, 1);
+            products(0);
+        }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // chunk i's fragments are in registers: its stage is free
         if (issued < mine) {
             issue(st);
@@ -397,64 +416,74 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
         if (i + 1u < mine) {
             wait_copies_but<G::CP, NS - 1>(issued - (i + 2u));
             asm volatile("" ::: "memory");
-            read(1 - s, st);
+            read(1 - s, st, 0);
         }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-            for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = mfma32<DT>(fa[s][kk][mb], fb[s][kk][nb], acc[mb][nb]);
-        __builtin_amdgcn_sched_barrier(0);
+        products(s);
     };
-    if (mine) {
+    const bool inTurn = !SL && nPeers && chunks > 4u * NS;   // the peers' requests go behind the first copies (see the top)
+    if (streams) {
+        for (; issued < umin(mine, (uint32_t)NS); ++issued) issue(issued);
+        if (inTurn) barrier_keep_vmem();
+    }
+    if (streams && mine) {
         wait_copies_but<G::CP, NS - 1>(issued - 1u);
         asm volatile("" ::: "memory");
-        read(0, 0);
+        read(0, 0, 0);
         uint32_t i = 0;
-        for (; i + 1u < mine; i += 2u) {
-            step(std::integral_constant<int, 0>{}, i);
-            step(std::integral_constant<int, 1>{}, i + 1u);
+        if constexpr (HALVES == 2) {
+            for (; i < mine; ++i) step(std::integral_constant<int, 1>{}, i);
+        } else {
+            for (; i + 1u < mine; i += 2u) {
+                step(std::integral_constant<int, 0>{}, i);
+                step(std::integral_constant<int, 1>{}, i + 1u);
+            }
+            if (i < mine) step(std::integral_constant<int, 0>{}, i);
         }
-        if (i < mine) step(std::integral_constant<int, 0>{}, i);
     }
 
-    // ---- the four partial tiles meet
-    __syncthreads();   // every wave has left its ring
+    // ---- the four partial tiles meet (the same two barriers on both ways)
     uint32_t *dst = (uint32_t *)(smem + G::MEET);   // [BM] what row i of the tile does
     constexpr uint32_t SWZ = BN >= 64 ? 1u : 0u;             // rows with bit 2 set are shifted by 128 bytes: the halves of a wave's write lie in different banks
+    if (streams) {
+        __syncthreads();   // every wave has left its ring
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
+        for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
+            for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint32_t row = mb * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
-                const auto e = acc[mb][nb][r];
-                *(int *)(smem + ((w * BM + row) * BN + ((nb * 32 + c32) ^ ((uint32_t)h * SWZ << 5))) * 4) = __builtin_bit_cast(int, e);
-            }
-    const bool store = (flags & GF_OUTBOUND_STORE) != 0, taskSums = !store && (flags & GF_ROW_MASK) == 0 && args.checksum != nullptr && sp.op == OP_REDUCE_SCATTER;
-    if (tid < BM) {
-        const uint32_t v = row0 + tid;
-        uint32_t e = FX_SKIP;
-        if ((uint32_t)tid < rowsValid) {
-            if (v - keptBegin < keptRows) {
-                e = FX_KEPT;
-            } else if (store) {
-                uint32_t ri, task, ws;
-                const uint32_t r = fast_div(v, args.fx.dRank, ri);
-                flex_task_of(sp, r, ri, col0 / sp.n0, task, ws);
-                e = FX_OUT | ws;
-            } else if (taskSums) {
-                uint32_t ri, task, ws;
-                const uint32_t r = fast_div(v, args.fx.dRank, ri);
-                flex_task_of(sp, r, ri, col0 / sp.n0, task, ws);
-                e = FX_SUM | task;
-            }
-        }
-        dst[tid] = e;
+                for (int r = 0; r < 16; ++r) {
+                    const uint32_t row = mb * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
+                    const auto e = acc[mb][nb][r];
+                    *(int *)(smem + ((w * BM + row) * BN + ((nb * 32 + c32) ^ ((uint32_t)h * SWZ << 5))) * 4) = __builtin_bit_cast(int, e);
+                }
+        __syncthreads();
+        return;
     }
+    fetch_scales();
+    const bool store = (flags & GF_OUTBOUND_STORE) != 0, taskSums = !store && (flags & GF_ROW_MASK) == 0 && args.checksum != nullptr && sp.op == OP_REDUCE_SCATTER;
+    uint32_t e = FX_SKIP;   // what row tid of the tile does
+    if ((uint32_t)tid < rowsValid) {
+        const uint32_t v = row0 + tid;
+        if (v - keptBegin < keptRows) {
+            e = FX_KEPT;
+        } else if (store) {
+            uint32_t ri, task, ws;
+            const uint32_t r = fast_div(v, args.fx.dRank, ri);
+            flex_task_of(sp, r, ri, col0 / sp.n0, task, ws);
+            e = FX_OUT | ws;
+        } else if (taskSums) {
+            uint32_t ri, task, ws;
+            const uint32_t r = fast_div(v, args.fx.dRank, ri);
+            flex_task_of(sp, r, ri, col0 / sp.n0, task, ws);
+            e = FX_SUM | task;
+        }
+    }
+    if constexpr (!SL) {   // (else the last slice's)
+        if (inTurn) barrier_keep_vmem();
+        fetch_peers();
+    }
+    __syncthreads();
+    if (tid < BM) dst[tid] = e;
     __syncthreads();
 
     v4i cur[UN];
@@ -629,7 +658,7 @@ __global__ void __launch_bounds__(256, 1) gemm_few_kernel(const GemmArgs args)
 template <uint32_t DT, bool TB, bool GA, bool SL>
 inline int launch_few_sl(const GemmArgs &args, int tileRows, int tileCols, hipStream_t s)
 {
-    const dim3 grid(args.fx.rowTiles * args.fx.colTiles * args.fx.slices), block(256);
+    const dim3 grid(args.fx.rowTiles * args.fx.colTiles * args.fx.slices), block(512);
     if (tileRows == 32 && tileCols == 32) hipLaunchKernelGGL((gemm_few_kernel<DT, TB, 1, 1, GA, SL>), grid, block, 0, s, args);
     else if (tileRows == 32 && tileCols == 64) hipLaunchKernelGGL((gemm_few_kernel<DT, TB, 1, 2, GA, SL>), grid, block, 0, s, args);
     else if (tileRows == 64 && tileCols == 64) hipLaunchKernelGGL((gemm_few_kernel<DT, TB, 2, 2, GA, SL>), grid, block, 0, s, args);
