@@ -95,6 +95,17 @@ def test_quant_kept_rows(case):
     torch.cuda.synchronize()
     assert np.array_equal(host16(out), want) and np.array_equal(dump.cpu().numpy(), acc) and not ws[:65536].any()
 
+# The peers are asked for at once where a wave's chunks of 128 bytes of k fill its ring at most (20 chunks of 32x32 tiles, 12 of 32x64, 8 of 64x64),
+# behind the first copies else; seven (64x64) or eight of them are held in registers.
+@pytest.mark.parametrize("case", [(33, 1344, 2560, 8, 0, 33, True, False, "32x32"), (33, 1344, 2564, 9, 5, 20, True, False, "32x32"), (33, 1344, 2560, 10, 0, 33, False, True, "32x32"),
+                                  (250, 1376, 1536, 8, 0, 250, True, False, "32x64"), (250, 1376, 1540, 9, 40, 100, True, True, "32x64"),
+                                  (250, 1376, 1536, 10, 0, 250, False, False, "32x64"),
+                                  (330, 1696, 1024, 8, 0, 330, True, False, "64x64"), (330, 1696, 1028, 9, 60, 70, True, False, "64x64"),
+                                  (330, 1696, 1020, 9, 0, 330, False, True, "64x64")])
+def test_quant_peers_at_once_or_in_turn(case):
+    test_quant_kept_rows(case)
+
+
 
 # (rows per rank, N, K, P, rank, weights as [n,k], int32 peers): kept rows inside a tile and across two, other ranks' rows beside them
 @pytest.mark.parametrize("case", [(5, 260, 132, 8, 3, True, False, "32x32", "32x32"), (20, 512, 416, 4, 0, False, True, "32x32", "32x32"),
