@@ -541,6 +541,13 @@ __global__ void __launch_bounds__(256) flex_finish_kernel(const GemmArgs args, c
 {
     constexpr bool I8 = DT == DT_I8;
     using Sum = typename std::conditional<I8, unsigned long long, double>::type;
+    // (named here, the arguments arrive in a few wide loads: they come from host memory)
+    const void *peer[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) peer[q] = args.peers[q];
+    asm volatile("" : : "s"(peer[0]), "s"(peer[1]), "s"(peer[2]), "s"(peer[3]), "s"(peer[4]), "s"(peer[5]), "s"(peer[6]), "s"(peer[7]), "s"(args.skPart), "s"(args.d),
+                 "s"(args.scaleM), "s"(args.scaleN), "s"(args.bias), "s"(args.checksum), "s"(args.accDump), "s"(args.cAccum), "s"(args.ldd), "s"(args.peerLd), "s"(args.peerRowOffset),
+                 "s"(args.N), "s"(args.flags), "s"(args.nPeers), "s"(args.keptBegin), "s"(args.keptRows), "s"(args.outDtype), "s"(args.fx.slices), "s"(args.fx.sliceSums));
     const int lane = threadIdx.x & 63;
     const uint32_t w = __builtin_amdgcn_readfirstlane((uint32_t)threadIdx.x >> 6);
     const bool redI32 = I8 && (args.flags & GF_REDUCE_INT32) != 0;
@@ -602,25 +609,32 @@ __global__ void __launch_bounds__(256) flex_finish_kernel(const GemmArgs args, c
         if (colOk) {
 #pragma unroll
             for (int q = 0; q < 8; ++q)
-                if ((uint32_t)q < nP) pv[q] = load((const int *)args.peers[q] + peerAt, NT);
+                if ((uint32_t)q < nP) pv[q] = load((const int *)peer[q] + peerAt, NT);
             const int32_t *part = args.skPart + (size_t)(v - first) * args.N + blockIdx.x * 256u;
             const size_t pitch = (size_t)stored * args.N;
-            for (uint32_t s0 = 0; s0 < slices; s0 += 8u) {
+            auto add_part = [&](const v4i &t) {
+                if constexpr (I8) {
+                    cur += t;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) cur[e] = f2i(__fadd_rn(i2f(cur[e]), i2f(t[e])));
+                }
+            };
+            uint32_t s0 = 0;   // (whole eights without a branch per slice: with the arguments named above, bf16 all-reduce 2x12800x576 in 34 slices 14.0 -> 13.0 us)
+            for (; s0 + 8u <= slices; s0 += 8u) {
                 v4i t[8];
 #pragma unroll
-                for (int q = 0; q < 8; ++q)
-                    if (s0 + q < slices) t[q] = load(part + (s0 + q) * pitch, KEEP);
+                for (int q = 0; q < 8; ++q) t[q] = load(part + (s0 + q) * pitch, KEEP);
 #pragma unroll
-                for (int q = 0; q < 8; ++q)
-                    if (s0 + q < slices) {
-                        if constexpr (I8) {
-                            cur += t[q];
-                        } else {
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) cur[e] = f2i(__fadd_rn(i2f(cur[e]), i2f(t[q][e])));
-                        }
-                    }
+                for (int q = 0; q < 8; ++q) add_part(t[q]);
             }
+            v4i t[7];
+#pragma unroll
+            for (int q = 0; q < 7; ++q)
+                if (s0 + q < slices) t[q] = load(part + (s0 + q) * pitch, KEEP);
+#pragma unroll
+            for (int q = 0; q < 7; ++q)
+                if (s0 + q < slices) add_part(t[q]);
             if (I8 && !late) cur += bv;   // (late: the first launch has added the bias and written the dump)
             if (args.accDump && !late) *(v4i *)((int32_t *)args.accDump + (size_t)v * args.N + gcol) = cur;
         }
