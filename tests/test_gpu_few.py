@@ -305,6 +305,16 @@ def test_float_mixed_tiles(case):
     test_float_larger_tiles(case)
 
 
+# Two ranks' reduce-scatters (half of all rows kept, on small tiles) and k off the 16-byte grid, where flexible tiles ran before
+@pytest.mark.parametrize("case", [(1513, 3584, 6280, 2, 1, False, False, "256x256 dealt"), (3978, 2048, 5604, 2, 0, True, True, "256x256 dealt")])
+def test_quant_mixed_tiles_of_two_ranks(case):
+    test_quant_mixed_tiles(case)
+
+
+def test_float_mixed_tiles_off_the_16_byte_grid():
+    test_float_larger_tiles(("allgather", 1024, 5120, 6148, 8, 3, False, "256x256"))
+
+
 # Kept rows dealt out to the 128- and 64-row tiles: 16 or fewer to a tile (one group of a thread's rows; of 16 ranks more peers than fit at
 # once), up to 32, up to 64 and as many as two ranks leave, tiles of unequal shares, first, last and a middle rank, columns past a tile; one rank, where none is dealt
 @pytest.mark.parametrize("case", [(125, 4096, 1376, 8, 5, True, False, "128x128 dealt"), (65, 4096, 1040, 16, 15, False, True, "128x128 dealt"),
