@@ -1815,12 +1815,13 @@ inline bool deep_ring_pairs(const GemmArgs &a, uint64_t es)
 // Launch of the 128-row geometry: one instantiation per operand layout (A as [m][k] or [k][m], B as [k][n] or [n][k]) and
 // for ragged problems; one workgroup per tile, or per k slice of a tile.
 //
-// 16x16 MFMAs (mfma16.h): W8A8 launches with two workgroups on a CU and 24 steps of k or more.  A single workgroup has one wave per SIMD, which has
+// 16x16 MFMAs (mfma16.h): W8A8 launches with two workgroups on a CU and 24 steps of k or more in each.  A single workgroup has one wave per SIMD, which has
 // to issue an MFMA, fragment reads and copies every 16 cycles and falls behind, and a short loop is mostly start and end, where the lane swaps are.
 // 32x32 -> 16x16, us: 4096x1792x4096 pipelined 49.4 -> 47.2, 8192x1792x4096 69.5 -> 68.7 (by box: 71.4 and 67.6 before), 3552x4288x3840 90.9 -> 87.4,
 // pipelined 3328x2560x4864 58.9 -> 56.2, 7376x5056x5376 as [n,k] 245.0 -> 233.3; up to 256 workgroups 5160x2560x1280 30.8 -> 31.6, 17 steps
-// 5550x1088x3584 39.6 -> 43.5.  Not for 16-bit operands: ragged rows, whose epilogue spills more then, 7282x6656x5632 545 -> 546, 3232x7104x4608 214 -> 217.
-inline bool mfma16_pays(const GemmArgs &args, uint32_t workgroups) { return workgroups > 256u && args.K >= 1536u; }
+// 5550x1088x3584 39.6 -> 43.5.  (Of k slices it is a slice's steps that count: eight slices of 6 steps, 1536x3072x768, 46.0 -> 45.0 back on 32x32, of 12 steps
+// 50.2 -> 49.3; two of 12, 4096x1536x1536, 34.2 both.)  Not for 16-bit operands: ragged rows, whose epilogue spills more then, 7282x6656x5632 545 -> 546, 3232x7104x4608 214 -> 217.
+inline bool mfma16_pays(const GemmArgs &args, uint32_t workgroups) { return workgroups > 256u && args.K / (args.splitK > 1 ? args.splitK : 1u) >= 1536u; }
 
 template <uint32_t DT, bool TB>
 inline void launch_split_kept(const GemmArgs &args, uint32_t keptPerXcd, hipStream_t s)

@@ -291,6 +291,71 @@ def test_quant_rs_kept_tiles_whole_or_split_give_the_same_bits(tb):
         assert int(res[0][1].ne(0).sum()) >= ntasks * 7 // 8 - 2
 
 
+# (rows per rank, N, K, P, rank, weights as [n,k], stored tiles instead of checksums, int32 peers, kept tiles as halves, k slices): 128x256 tiles on
+# more than 256 workgroups with 24 and 25 steps of k each; whole and ragged rows and columns, kept tiles as halves beside whole tiles
+@pytest.mark.parametrize("case", [(512, 2304, 1536, 8, 3, False, False, False, False, 1), (512, 2304, 1600, 8, 7, True, True, False, False, 1),
+                                  (512, 2304, 1600, 8, 0, True, False, True, False, 1), (1024, 2304, 1600, 4, 1, False, True, True, False, 1),
+                                  (600, 2128, 1536, 8, 5, False, False, False, False, 1), (600, 2128, 1600, 8, 2, False, True, True, False, 1),
+                                  (600, 2120, 1536, 8, 7, True, True, False, False, 1), (600, 2120, 1600, 8, 0, True, False, True, False, 1),
+                                  (512, 2560, 1600, 8, 4, False, False, True, True, 1), (512, 2560, 1536, 8, 3, False, True, False, True, 1),
+                                  (512, 2560, 1536, 8, 3, True, False, True, True, 1), (512, 2560, 1600, 8, 6, True, True, False, True, 1),
+                                  (384, 768, 12352, 4, 2, False, False, False, False, 8), (384, 768, 12288, 4, 1, True, True, True, False, 8),
+                                  (384, 768, 3072, 4, 1, False, False, False, False, 8)])
+def test_quant_rs_two_workgroups_per_cu(case):
+    _need_gpu()
+    import ctypes as C
+    rows, N, K, P, rank, tb, stored, ri, halves, f = case
+    M, comm = rows * P, L.QUANT_MATMUL_REDUCE_SCATTER
+    g = torch.Generator(device=DEV).manual_seed(K + rank)
+    x1, x2 = (torch.randint(-127, 128, shape, dtype=torch.int8, device=DEV, generator=g) for shape in ((M, K), (K, N)))
+    s1, s2 = (torch.empty(c, device=DEV).uniform_(0.001, 0.02, generator=g) for c in (M, N))
+    b = torch.randint(-1000, 1000, (N,), dtype=torch.int32, device=DEV, generator=g)
+    peers = [torch.randint(-2 ** 20, 2 ** 20, (rows, N), dtype=torch.int32, device=DEV, generator=g) if ri else torch.randn((rows, N), device=DEV, generator=g)
+             for _ in range(P - 1)]
+    t, d = ops.default_tiling(M, K, N, P, m0=128, n0=256, k0=0, commInterval=4), L.make_desc(rank, P, [16] * (P - 1))
+    so = L.load()
+    tasks = so.catcoc_get_task_count(comm, C.byref(t), C.byref(d))
+    kw = {"kept_split": halves}
+    if stored:
+        size = so.catcoc_get_workspace_size(comm, L.INT8, C.byref(t), C.byref(d)) // 4
+        kw["outbound"] = torch.full((size,), 3, dtype=torch.int32 if ri else torch.float32, device=DEV)
+        d.flags |= L.OUTBOUND_STORE
+    else:
+        kw["checksum"] = torch.full((tasks,), -1, dtype=torch.int64, device=DEV)
+        d.checksum = 4096
+    if f > 1:
+        kw.update(split_k=f, workspace=torch.zeros(ops.kslice_plan(comm, torch.int8, M, K, N, rank, P, tiling=t, split_k=f)[0], dtype=torch.uint8, device=DEV))
+    if halves:
+        d.flags |= L.FLAG_KEPT_SPLIT
+        d.outbound, d.outboundBytes = 4096, 1 << 40
+        assert so.catcoc_kept_split_tiles(comm, L.INT8, C.byref(t), C.byref(d), 0, int(tb)) > 0
+    dump, sums = torch.full((M, N), -7, dtype=torch.int32, device=DEV), torch.full((rows, N), -7, dtype=torch.int32, device=DEV)
+    out = ops.quant_matmul_reduce_scatter(x1, x2.T.contiguous() if tb else x2, s1, s2, b, peers, rank, P, tiling=t, trans_b=tb, reduce_int32=ri,
+                                          acc_dump=dump, c_accum=sums, **kw)
+    i = L.last_launch()
+    assert (i.kernel, i.tileRows, i.tileCols, i.kSlices) == (L.KERNEL_ALIGNED, 128, 256, f) and tasks * f > 256
+    acc = (x1.double() @ x2.double()).to(torch.int32) + b   # (exact)
+    kept = acc[rank * rows:(rank + 1) * rows]
+    if ri:
+        kept = kept + sum(peers)
+    assert torch.equal(dump, acc) and torch.equal(sums, kept)
+    deq = lambda a, sm: (a.float() * s2) * sm[:, None]
+    want = deq(kept, s1[rank * rows:(rank + 1) * rows])
+    for p in ([] if ri else peers):
+        want = want + p
+    assert torch.equal(out, want.bfloat16())
+    full, blocks = (acc if ri else deq(acc, s1)), (kw["outbound"].reshape(-1, 256) if stored else kw["checksum"].tolist())
+    tr, row, col, ws = (C.c_uint32() for _ in range(4))
+    for task in range(tasks):
+        so.catcoc_task_tile(comm, C.byref(t), C.byref(d), task, C.byref(tr), C.byref(row), C.byref(col), C.byref(ws))
+        if tr.value != rank:
+            r0, c0, r1, c1 = row.value, col.value, min(row.value + 128, (tr.value + 1) * rows), min(col.value + 256, N)
+            if stored:
+                assert torch.equal(blocks[ws.value:ws.value + r1 - r0, :c1 - c0], full[r0:r1, c0:c1]), task
+            else:
+                assert blocks[task] == int(acc[r0:r1, c0:c1].sum()), task
+
+
 @pytest.mark.parametrize("kind", ["int8", "fp16"])
 def test_rs_tiles_that_wait_for_kept_halves_run_as_halves(kind):
     """512 tiles with split kept tiles are 576 workgroups on 512 slots; with a workspace (the checksum halves of a task meet
