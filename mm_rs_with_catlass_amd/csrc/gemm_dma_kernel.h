@@ -374,8 +374,8 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
 #define CATCOC_MMA(FA, FB, MBI, NBI)                                              \
     acc[MBI][NBI] = mfma32<DT>(FA[MBI], FB[NBI], acc[MBI][NBI]);                  \
     CATCOC_FENCE();
-    // read_a(af, kk): A fragments of this step; sb: B stage of this step; slot1/2/3/4: the step's other work
-    auto sched_step = [&](auto read_a, const unsigned char *sb, auto slot1, auto slot2, auto slot3, auto slot4) {
+    // read_a(af, kk): A fragments of this step; sb: B stage of this step; copyA, copyB: the step's copies
+    auto sched_step = [&](auto read_a, const unsigned char *sb, auto copyA, auto copyB) {
         if constexpr (MB == 1) {   // eight MFMAs per step: the same lag of half a step, two reads per gap
             CATCOC_MMA(fa1, fb1, 0, 0)
             read_a(fa0, 0);
@@ -387,11 +387,10 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             CATCOC_FENCE();
             CATCOC_MMA(fa1, fb1, 0, 2)
             read_b1(fb0, sb, 0, 3);
-            slot1();
+            copyA();
             CATCOC_FENCE();
             CATCOC_MMA(fa1, fb1, 0, 3)
-            slot2();
-            slot3();
+            copyB();
             CATCOC_FENCE();
             CATCOC_MMA(fa0, fb0, 0, 0)
             read_a(fa1, 1);
@@ -403,7 +402,6 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             CATCOC_FENCE();
             CATCOC_MMA(fa0, fb0, 0, 2)
             read_b1(fb1, sb, 1, 3);
-            slot4();
             CATCOC_FENCE();
             CATCOC_MMA(fa0, fb0, 0, 3)
         } else {
@@ -423,13 +421,12 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
         read_b1(fb0, sb, 0, 3);
         CATCOC_FENCE();
         CATCOC_MMA(fa1, fb1, 1, 2)
-        slot1();
+        copyA();
         CATCOC_FENCE();
         CATCOC_MMA(fa1, fb1, 0, 3)
-        slot2();
+        copyB();
         CATCOC_FENCE();
         CATCOC_MMA(fa1, fb1, 1, 3)
-        slot3();
         CATCOC_FENCE();
         CATCOC_MMA(fa0, fb0, 0, 0)
         read_a(fa1, 1);
@@ -447,14 +444,12 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
         read_b1(fb1, sb, 1, 3);
         CATCOC_FENCE();
         CATCOC_MMA(fa0, fb0, 1, 2)
-        slot4();
         CATCOC_FENCE();
         CATCOC_MMA(fa0, fb0, 0, 3)
         CATCOC_MMA(fa0, fb0, 1, 3)
         }
     };
 #undef CATCOC_MMA
-    auto nothing = [] {};
     // 16x16 MFMAs: 4 x 8 blocks per wave.  A step's 32 MFMAs lag its fragment reads by half a step as well: the first
     // sixteen are columns 64 .. 127 of the step before, behind which this step's fragments of A and of columns 0 .. 63 are read, the second
     // sixteen those columns, behind which the fragments of the others are.
@@ -523,7 +518,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
         }
         return v4i{t0.x, t0.y, t1.x, t1.y};
     };
-    auto barrier16 = [] {   // (the last fragments' reads are long back: sixteen MFMAs were issued since)
+    auto barrier16 = [] {   // (the last fragments' reads are back: nine MFMAs were issued since, sixteen after the first step)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         barrier_keep_vmem();
     };
@@ -650,7 +645,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
             const uint32_t k = kt;
             const bool moreB = k + (uint32_t)(NS - 1) < nk, moreP = (k & 1u) == 0 && k + (uint32_t)(NS + 2) <= nk;
             sched_step([&](v4i (&af)[MB], int kk) { load_ap(af, k, kk); }, stB(cur), [&] { if (moreB) issue_b(offB(nxt)); },
-                       [&] { if (moreP) issue_ap((k + (uint32_t)NS) >> 1); }, nothing, nothing);
+                       [&] { if (moreP) issue_ap((k + (uint32_t)NS) >> 1); });
             ++kt;
             cur = cur == NS - 1 ? 0 : cur + 1;
             nxt = nxt == NS - 1 ? 0 : nxt + 1;
@@ -869,7 +864,7 @@ __device__ __forceinline__ void dma_tile(const GemmArgs &args, unsigned char *sm
         auto step = [&](bool more) {
             const unsigned char *sa = stA(cur);
             sched_step([&](v4i (&af)[MB], int kk) { load_a(af, sa, kk); }, stB(cur),
-                       [&] { if (more) issue_a(offA(nxt)); }, [&] { if (more) issue_b(offB(nxt)); }, nothing, nothing);
+                       [&] { if (more) issue_a(offA(nxt)); }, [&] { if (more) issue_b(offB(nxt)); });
             ++kt;
             cur = cur == NS - 1 ? 0 : cur + 1;
             nxt = nxt == NS - 1 ? 0 : nxt + 1;
