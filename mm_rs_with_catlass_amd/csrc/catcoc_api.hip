@@ -292,18 +292,19 @@ bool flex_ptrs_ok(const GemmArgs &a)
 // operands, per MB of peers and outputs; rows of k off the 16-byte grid and B as [k,n] cost more per KiB, rows of a B tile that are no whole
 // cache line more per MB.  Half of the estimates are within 0.10 of the tiles' times and 0.06 of the others', nine in ten within 0.22
 // and 0.16.  The tiles of 96, 160 and 192 rows stand on the scale of the 128-row one's (their times relative to it, 1600 calls).  The estimates of
-// 128-column tiles are from when these ran 32x32 MFMAs and come out 0.11 high, of flexible tiles in k slices 0.12, of aligned
-// tiles 0.05, so the choice, the tiles with the least, compares shares (other_share): 1571 drawn calls of 1e9 operations and more, each timed on every
-// tile, then take 1.015 of the best choice's time for each and 0.69 of the time of the kernels that would run else; 39 of them lose more than 0.04
-// against those.  With five tiles and the shares before that it was 1.065 and 0.72.  Those still hold for calls unlike the fitted ones: k below 512,
-// columns that are no multiple of 32, one rank or more than eight.
+// 128-column tiles are from when these ran 32x32 MFMAs and come out up to 0.2 high, of flexible tiles in k slices 0.12, so the choice, the tiles with the least, compares
+// shares (other_share), set on 5100 drawn calls, each timed on every tile in reach.  2000 others take 1.015 of the best of these and 0.921 of the time they took before
+// the 16x16 MFMAs and the tiles of 96, 160 and 192 rows, 24 of them more than 1.04; with the shares and the estimate of mixed launches that those came with 0.929, 42 of them.
+// For calls unlike those (k below 512, columns that are no multiple of 32, one rank or more than eight) the shares are older and the tiles of 96, 160 and 192 rows
+// left out: 283 drawn ones take 1.032 of the best choice's time, and none lost more than 0.04 by the re-fitted estimates of mixed launches.
 // Figures of calls stand with the kernels that run them (gemm_few.h, gemm_mid.h, gemm_mixed.h).
-constexpr double kMixedShare = 1.1;   // of a mixed launch's estimate, against the other tiles'
+constexpr double kMixedShare = 1.15;   // of a mixed launch's estimate, against the other small tiles', which come out that much high
 enum OtherKernel { OTHER_NONE, OTHER_ALIGNED, OTHER_FLEXIBLE, OTHER_SLICED, OTHER_STREAMING };
 struct Other {        // what a launch would run else, and for how long by its estimate
     OtherKernel kernel;
     double us;
-    bool pipelined;   // its GEMM launch and the comm launch behind it
+    bool pipelined;   // a call of the pipelined operator
+    bool comm;        // its GEMM launch is followed by a comm launch
 };
 struct SmallTile {
     int rows, cols;   // 0: the launch is not one for them; 256x256: the large ones of a mixed launch
@@ -328,13 +329,20 @@ CallSize call_size(const GemmArgs &a, uint32_t es)
     return {rows, kB / 1024.0, 1e-6 * kB * (a.N + rows), 1e-6 * a.N * (4.0 * a.nPeers * a.keptRows + (a.sched.op == OP_REDUCE_SCATTER ? 4.0 : 2.0) * rows)};
 }
 
-// 128-row tiles of the aligned kernels (launches of 256-row ones run nothing else).
-double aligned_us(const GemmArgs &a, uint32_t es)
+// 128-row tiles of the aligned kernels (launches of 256-row ones run nothing else).  Kept tiles that are spread over all XCDs alike are the first that each of
+// them starts.  Where they run as halves and all workgroups find a slot at once the launch takes 0.8 of what others of its size take: of four and eight ranks 150
+// calls 0.75 to 0.85, W8A8 4096x1280x3072 pipelined 35.5 us (3072x1600x4096, as many tiles but not spread alike: 51.5).  With more workgroups eight ranks' take 0.8 to 0.95 (pipelined
+// 2048x1088x8192 as [n,k] 41.0; not 16 bits as [n,k] in one round, 4096x1792x4096 87, 83.5 mixed), four ranks' 0.95 to 1.1.
+double aligned_us(const GemmArgs &a, uint32_t es, bool pipelined)
 {
     const CallSize c = call_size(a, es);
     const double f = a.splitK > 1 ? a.splitK : 1.0, wgs = a.sched.coreLoops * f, rounds = ceil(wgs / 256.0), steps = c.kib * 16.0 / f;
-    return 6.6 + rounds * (steps * (0.325 + (a.transB ? 0.060 : 0.0) - (es == 1 ? 0.019 : 0.0)) - 2.0) + (wgs > 512.0 ? 0.104 * (wgs / 256.0 - 2.0) * steps : 0.0) +
-           (f > 1.0 ? 10.0 : 0.0) + (a.sched.op == OP_REDUCE_SCATTER ? 1.88 * a.nPeers : 0.0) + 0.134 * c.moved + 0.505 * c.mb;
+    const double us = 6.6 + rounds * (steps * (0.325 + (a.transB ? 0.060 : 0.0) - (es == 1 ? 0.019 : 0.0)) - 2.0) + (wgs > 512.0 ? 0.104 * (wgs / 256.0 - 2.0) * steps : 0.0) +
+                      (f > 1.0 ? 10.0 : 0.0) + (a.sched.op == OP_REDUCE_SCATTER ? 1.88 * a.nPeers : 0.0) + 0.134 * c.moved + 0.505 * c.mb;
+    const uint32_t kept = a.sched.P > 2 ? 8u * splittable_kept_tiles(a) : 0u;
+    if (kept == 0) return us;
+    if (a.sched.coreLoops + kept <= 512u) return 0.8 * us;
+    return a.sched.P >= 8 && (pipelined || !a.transB || a.sched.coreLoops > 512u) ? 0.87 * us : us;
 }
 
 // Flexible tiles as plan_flex left them in args.fx (blocks = rows / 64): whole, with a second launch for the peers, in k slices.
@@ -352,7 +360,7 @@ double flex_us(const GemmArgs &a, uint32_t es, int blocks)
     return us > off16 ? us : off16;
 }
 
-Other other_flexible(const GemmArgs &a, uint32_t es, int blocks) { return {a.fx.slices > 1 ? OTHER_SLICED : OTHER_FLEXIBLE, flex_us(a, es, blocks), false}; }
+Other other_flexible(const GemmArgs &a, uint32_t es, int blocks) { return {a.fx.slices > 1 ? OTHER_SLICED : OTHER_FLEXIBLE, flex_us(a, es, blocks), false, false}; }
 
 // Rows of a mixed launch that run on 256x256 tiles, of all but a reduce-scatter's kept ones; `us`: the launch's estimate.
 struct MixedRows {
@@ -366,7 +374,8 @@ bool kept_apart(const GemmArgs &a) { return a.sched.op == OP_REDUCE_SCATTER && a
 // When the last of the workgroups that `cus` CUs get of a launch is done: large ones first, then small ones, each on the first CU that is free.
 double part_us(uint64_t large, uint64_t small, double largeUs, double smallUs, uint32_t cus)
 {
-    const uint64_t l = (large * cus + 255u) / 256u, s = (small * cus + 255u) / 256u, part = l % cus, idle = cus - part;
+    const uint32_t parts = 256u / cus;
+    const uint64_t l = (large + parts - 1u) / parts, s = (large + small + parts - 1u) / parts - l, part = l % cus, idle = cus - part;
     const double start = (double)(l / cus) * largeUs, end = start + largeUs;   // of the last round of large ones
     if (part == 0) return start + (double)((s + cus - 1u) / cus) * smallUs;
     const uint64_t first = (uint64_t)(largeUs / smallUs) + 1u;   // small ones that a CU without one of those starts by the time they end
@@ -375,20 +384,19 @@ double part_us(uint64_t large, uint64_t small, double largeUs, double smallUs, u
     return fmax(end + (double)(more + (rest ? 1u : 0u)) * smallUs, start + (double)(first + more + (rest > part ? 1u : 0u)) * smallUs);
 }
 
-// Two bounds: the CUs' schedule (workgroups go to the XCDs and, mostly, to their four shader engines in turn: the mean of
-// what 32 and 8 CUs take, with small tiles a little longer for the 32, so that a row count that just fits does not look as good as one that fits easily), and the power limit, at which
-// large tiles on half of the CUs take less time each than on all.  Fitted to 11200 launches of 1860 calls with one to all of their rows on large
-// tiles: half of them within 0.04, nine in ten within 0.11; the count with the least estimate takes 1.011 of the best one's time.  With large tiles at
-// 9 us + 1.7 per chunk whatever the others do, as before 16x16 MFMAs, it was 1.03 of it, and calls on them 1.055 of their best choice's time (1.025
-// now): pipelined W8A8 3584x15600x5120 as [n,k] of four ranks 378 -> 297 us, all-gather 4 x [591,8296] x [8296,6400] 277 -> 219,
-// W8A8 with stored tiles 6720x6144x2048 104 -> 83.8.
+// Two bounds: the CUs' schedule (workgroups go to the XCDs and, mostly, to their four shader engines in turn: the mean of what 32 and
+// 8 CUs take) and the power limit, at which large tiles on half of the CUs take less time each than on all.  A small tile's peers come through one CU: the
+// fewer small tiles the kept rows are dealt to, the longer each takes.  Fitted to 5953 launches of 899 calls with one to seven counts of rows on large
+// tiles each: half of them within 0.04, nine in ten within 0.10; the count with the least estimate takes 1.009 of the best one's time.  Without the peers and with large
+// and small tiles rounded up each for itself, so that 253 of them did not fit 256 CUs, it was 1.019 of it, 1.34 at worst: fp16 1800x1344x5888 of eight ranks with stored
+// tiles 48.1 -> 38.7 us (161 large and 92 small), W8A8 2440x1728x4224 43.4 -> 36.6, pipelined 4096x1280x3072 as [n,k] 45.3 -> 40.1.
 MixedRows mixed_rows(const GemmArgs &a, uint32_t es, uint32_t rows)
 {
     const CallSize c = call_size(a, es);
     const double chunks = c.kib * 8.0;
     const bool off16 = (uint64_t)a.K * es % 16 != 0;
     const uint32_t kept = kept_apart(a) ? a.keptRows : 0u;
-    const double large = 5.1 + chunks * (off16 ? 1.28 : 1.11) + (kept ? 0.0 : 2.4 * a.nPeers), small = 5.2 + chunks * (off16 ? 0.515 : 0.37) + 0.175 * a.nPeers;
+    const double large = 5.6 + chunks * (off16 ? 1.33 : 1.085) + (kept ? 0.0 : 3.0 * a.nPeers), small = 5.35 + chunks * (off16 ? 0.518 : 0.363) + 0.17 * a.nPeers;
     const uint32_t largeCols = ceil_div(a.N, 256u), smallCols = ceil_div(a.N, 128u), most = ceil_div(rows - kept, 256u);
     // (as few rows on large tiles as leave two rounds of them to the small ones; of a wide range every second, third .. count)
     const uint32_t range = umin(most - 1u, ceil_div(512u, largeCols)), step = range / 32u + 1u;
@@ -396,12 +404,13 @@ MixedRows mixed_rows(const GemmArgs &a, uint32_t es, uint32_t rows)
     for (uint32_t t = most - range / step * step; t <= most; t += step) {
         const uint32_t r = umin(256u * t, rows - kept);
         const uint64_t l = (uint64_t)t * largeCols, s = (uint64_t)ceil_div(rows - r, 128u) * smallCols;
-        const double cus = 0.5 * (part_us(l, s, large, 1.1 * small, 32u) + part_us(l, s, large, small, 8u));
-        const double power = 1.48 * chunks * ((double)l + 0.306 * s) / 256.0, c2 = cus * cus, p2 = power * power;
+        const double dealt = small + (kept ? 0.9 * a.nPeers * kept / (double)(rows - r) : 0.0);
+        const double cus = 0.5 * (part_us(l, s, large, dealt, 32u) + part_us(l, s, large, dealt, 8u));
+        const double power = 1.36 * chunks * ((double)l + 0.327 * s) / 256.0, c2 = cus * cus, p2 = power * power;
         const double us = sqrt(sqrt(c2 * c2 + p2 * p2));
         if (best.large == 0 || us <= best.us) best = {r, us};
     }
-    best.us += 4.0 + 0.124 * c.moved + 0.05 * c.mb;
+    best.us += 4.4 + 0.108 * c.moved + 0.047 * c.mb;
     return best;
 }
 
@@ -447,22 +456,29 @@ uint64_t few_partials(const SmallTileCost &t, uint32_t keptTiles, uint32_t n, ui
 // A call like those the estimates were compared on (explicit kept rows: any number of ranks).
 bool fitted_call(const GemmArgs &a) { return a.N % 32 == 0 && a.K >= 512 && ((a.flags & GF_ROW_MASK) != 0 || (a.sched.P >= 2 && a.sched.P <= 8)); }
 
-// The share of the other kernels' estimate up to which small tiles (wide: of 128 columns, or mixed) run.
+// The share of the other kernels' estimate up to which small tiles (wide: of 128 columns; large: mixed ones) run.
 double other_share(const GemmArgs &a, uint32_t es, const Other &o, bool sums, bool wide, bool large)
 {
     const bool rowMask = (a.flags & GF_ROW_MASK) != 0, rs = a.sched.op == OP_REDUCE_SCATTER;
     if (fitted_call(a)) {
-        // (aligned tiles that are all whole come out 0.07 to 0.2 shorter than their estimate in reduce-scatters, most with checksums, which store
-        // nothing; 770 calls of whole tiles: W8A8 8192x2048x3072 as [n,k] 69.6 aligned, 90.5 mixed; with checksums 2048x4096x6144 67.5, 76.6 on 128x128)
-        const bool whole = o.kernel == OTHER_ALIGNED && rs && a.sched.P > 2 && a.sched.mRank % a.sched.m0 == 0 && a.N % a.sched.n0 == 0;
-        if (large) return whole ? (o.pipelined ? 0.9 : 0.96) : rs ? 1.0 : 1.05;
-        if (whole && sums) return 0.95;
+        // (mixed launches, 1200 calls by what would run else: two ranks keep half of all rows, and the other tiles stream the peers under each other's loops; W8A8 launches
+        // of more than 512 aligned tiles, those with a comm launch, flexible ones of k on the 16-byte grid and ragged all-gathers come out shorter than their estimate: pipelined
+        // 4096x2880x5120 as [n,k] 79.8 us aligned, 96.8 mixed; two ranks' 4128x1056x3072 37.0 flexible, 43.4)
+        if (large) {
+            if (!rs) return o.kernel == OTHER_FLEXIBLE && a.sched.op == OP_ALLGATHER ? 0.92 : 1.02;
+            if (o.kernel == OTHER_FLEXIBLE) return o.pipelined || (uint64_t)a.K * es % 16 != 0 ? 1.0 : 0.9;
+            return a.sched.P == 2 || (es == 1 && a.sched.coreLoops > 512u) ? 0.9 : o.comm ? 0.88 : 0.98;
+        }
+        // (aligned tiles that are all whole, with checksums: they store nothing; 2048x4096x6144 67.5, 76.6 on 128x128)
+        if (o.kernel == OTHER_ALIGNED && rs && sums && a.sched.P > 2 && a.sched.mRank % a.sched.m0 == 0 && a.N % a.sched.n0 == 0) return 0.95;
         // (pipelined calls, a GEMM and a comm launch or one with peers under its loops, come out longer than their estimate, 37 small ones 1.025 -> 1.008 of their
         // best choice's time with 1.1 for 0.95, W8A8 1024x2272x5888 37.7 -> 31.7 us; but none below 640 of k does; two ranks' kept rows are half of all, and aligned tiles then stream
-        // peers under each other's loops; the 62 calls with 16-bit operands on whole flexible tiles as [k,n] miss 0.015)
+        // peers under each other's loops; the 62 calls with 16-bit operands on whole flexible tiles as [k,n] miss 0.015, and with checksums 4520x784x1440 is 28.0 on flexible and
+        // 31.3 on 128x128 tiles; decode calls that could run in k slices, as [k,n], eight ranks 388x7936x512 16.1 there and 18.0 on 32x32 tiles)
         if (o.pipelined) return a.K < 640 ? 0.8 : 1.1;
         if (o.kernel == OTHER_STREAMING) return 0.87;
-        return o.kernel == OTHER_SLICED ? 0.9 : o.kernel == OTHER_FLEXIBLE && es == 2 && !a.transB ? 0.95 : rs && a.sched.P == 2 ? 1.0 : 1.1;
+        if (o.kernel == OTHER_SLICED) return rowMask ? 0.875 : 0.9;
+        return o.kernel == OTHER_FLEXIBLE && (sums || (es == 2 && !a.transB)) ? 0.95 : rs && a.sched.P == 2 ? 1.0 : 1.1;
     }
     double share = o.kernel == OTHER_ALIGNED ? 0.85 : 0.87;
     if (rs && !sums && wide) share *= 1.15;   // (kept rows are dealt out)
@@ -540,7 +556,7 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, const Other &other, uint64_t room
     MixedRows mixed = {0, 0.0};
     if (!sums && rows >= 512 && kBytes >= 1024 && rows * a.N >= 96ull * 256ull * 256ull) {
         mixed = mixed_rows(a, es, (uint32_t)rows);
-        if ((fitted ? kMixedShare * mixed.us : mixed.us) > least) mixed.large = 0;
+        if (kMixedShare * mixed.us > least) mixed.large = 0;
     }
     if (other.kernel != OTHER_NONE && (mixed.large ? mixed.us : least) > other_share(a, es, other, sums, mixed.large || best->cols == 128, mixed.large != 0) * other.us) return no;
     if (tiles > (1u << 24) || !flex_ptrs_ok(a)) return no;
@@ -853,7 +869,7 @@ SmallTile planned_small(const Plan &p, bool dma, bool flex, GemmArgs &g)
     if ((dma || p.preferFlex) && (g.flags & GF_OUTBOUND_STORE) == 0 && g.checksum == nullptr && g.sched.op == OP_REDUCE_SCATTER && splittable_kept_tiles(g) != 0) return {0, 0};
     g.skCount = p.counters;
     const uint32_t es = elem_size(p.dtype);
-    return small_tile(g, es, dma ? Other{OTHER_ALIGNED, aligned_us(p.args, es), false} : flex ? other_flexible(p.args, es, p.flexBlocks) : Other{OTHER_NONE, 0.0, false}, p.room);
+    return small_tile(g, es, dma ? Other{OTHER_ALIGNED, aligned_us(p.args, es, false), false, false} : flex ? other_flexible(p.args, es, p.flexBlocks) : Other{OTHER_NONE, 0.0, false, false}, p.room);
 }
 
 // CATCOC_FLAG_KEPT_WHOLE and CATCOC_FLAG_KEPT_SPLIT change no bit of a result: sums of floats in another order would.  So they do not enter the
@@ -1096,7 +1112,7 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
         if (sp.maySmall) {   // (the rest of these shapes runs whole 64x256 tiles or one thread per element, many times slower)
             GemmArgs g = a;
             g.skCount = counter_block(*d);
-            const SmallTile t = small_tile(g, 1, {OTHER_NONE, 0.0, false});
+            const SmallTile t = small_tile(g, 1, {OTHER_NONE, 0.0, false, false});
             if (t.rows) { launched(launch_small(DT_I8, g, t, stream)); return; }
         }
         const bool flex = sp.flexBlocks != 0 && flex_ptrs_ok(a);
@@ -1166,7 +1182,7 @@ void launch_quant_splitk(void *stream, uint8_t *x1, uint8_t *x2, uint8_t *scale_
             if ((c.slices > 1 && g.fx.slices < 2 && (sp.large || sp.f > 1)) || !decode_flex_pays(g, sp.large) || !flex_ptrs_ok(g)) blocks = 0;
         }
         if (sp.maySmall) {
-            const SmallTile t = small_tile(small, 1, sp.wholeK ? Other{OTHER_NONE, 0.0, false} : blocks ? other_flexible(g, 1, blocks) : Other{OTHER_STREAMING, streaming_us(g), false},
+            const SmallTile t = small_tile(small, 1, sp.wholeK ? Other{OTHER_NONE, 0.0, false, false} : blocks ? other_flexible(g, 1, blocks) : Other{OTHER_STREAMING, streaming_us(g), false, false},
                                            counter_room(*d, sp.workspaceBytes));
             // (a call that takes the kept rows' int32 block as well and would run in k slices runs in k slices, of one kind or the other: what its
             // workspace query reports is held to be what runs there.  Whole small tiles would be faster: operands in the caches, 203x1792x4096 with
@@ -1365,6 +1381,8 @@ void launch_pipelined(bool quant, int dataType, void *computeStream, void *commS
     bool fused = quant && dma && flexBlocks == 0 && P > 1 && oneRound &&
                  (sp.coreLoops >= 384u || sp.coreLoops <= 128u || P == 2 || (P <= 4 && tiling->k <= 2048u));
     if (fused) g.nPeers = P - 1;
+    // (a single round may run in the order of the fused operators: 4096x8192x8192 of two ranks, as [n,k], two launches 405 -> 337)
+    if (oneRound && (given->flags & CATCOC_FLAG_LINEAR_ORDER) == 0) g.flags &= ~(uint32_t)GF_LINEAR_ORDER;
     // Small or mixed tiles do the same in one launch, for problems of any alignment.  The fused operator's choice, with the comm launch on the
     // other side where it is not fused.  GEMM and comm launch -> one, us, one row-block round of eight ranks: 1024x3904x768 40.4 ->
     // 16.3, 2048x10672x1024 68.8 -> 38.7, 3072x2304x6176 91.5 -> 70.9, 4096x8960x7072 325 -> 280, of four 512x3604x640 45.0 -> 11.8, of two
@@ -1374,11 +1392,9 @@ void launch_pipelined(bool quant, int dataType, void *computeStream, void *commS
     if (quant && P > 1 && oneRound && (given->flags & (CATCOC_FLAG_LINEAR_ORDER | CATCOC_FLAG_KEPT_WHOLE | CATCOC_FLAG_KEPT_SPLIT)) == 0) {
         const double comm = fused ? 0.0 : 4.5 + 0.8 * (P - 1) + 0.1e-6 * 4.0 * (P - 1) * g.keptRows * g.N;
         gs.nPeers = P - 1;
-        small = small_tile(gs, 1, flexBlocks ? Other{OTHER_FLEXIBLE, flex_us(g, 1, flexBlocks) + comm, true} : dma ? Other{OTHER_ALIGNED, aligned_us(g, 1) + comm, true} : Other{OTHER_NONE, 0.0, false});
+        small = small_tile(gs, 1, flexBlocks ? Other{OTHER_FLEXIBLE, flex_us(g, 1, flexBlocks) + comm, true, true} : dma ? Other{OTHER_ALIGNED, aligned_us(g, 1, true) + comm, true, !fused} : Other{OTHER_NONE, 0.0, false, false});
     }
     if (small.rows) fused = true;
-    // (a single round may run in the order of the fused operators: 4096x8192x8192 of two ranks, as [n,k], two launches 405 -> 337)
-    if (oneRound && (given->flags & CATCOC_FLAG_LINEAR_ORDER) == 0) g.flags &= ~(uint32_t)GF_LINEAR_ORDER;
     const bool commWritesOutput = quant && !fused && deterministic != 0 && P > 1 && (uintptr_t)scale_x2 % 16 == 0 && (uintptr_t)d_out % 8 == 0;
     if ((dma || flexBlocks) && commWritesOutput) g.flags |= GF_KEPT_INT32_ONLY;   // (the comm rounds write every kept row's output)
 

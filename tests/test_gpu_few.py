@@ -806,3 +806,18 @@ def test_quant_task_sums_rows_between(case):
 @pytest.mark.parametrize("case", [(334, 1696, 794, 4, 3, False, "96x128 dealt"), (132, 4288, 624, 8, 4, False, "160x128 dealt"), (141, 4768, 514, 8, 1, True, "192x128 dealt")])
 def test_float_task_sums_rows_between(case, dtype):
     test_float_task_sums(case, dtype)
+
+
+# Calls beside which other kernels are slower, or that were slower on others: large and small tiles that fill the CUs exactly once; checksums on
+# flexible tiles; k slices of a decode call as [k,n]
+def test_mixed_tiles_that_fill_the_cus_once():
+    test_float_larger_tiles(("reduce_scatter", 1800, 5888, 1344, 8, 3, False, "256x256 dealt"))
+    assert L.last_launch().largeTiles == 161   # (and 92 of 128x128)
+
+
+def test_checksums_on_flexible_tiles_beside_small_ones():
+    test_quant_task_sums((565, 1440, 784, 8, 3, False, False, "flexible 128x256"))
+
+
+def test_k_slices_beside_small_tiles():
+    test_quant_kept_rows((388, 512, 7936, 8, 0, 388, False, False, "flexible 64x256/9"))

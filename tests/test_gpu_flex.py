@@ -298,6 +298,12 @@ def test_pipelined_quant_one_round_on_aligned_tiles(case, deterministic):
     test_pipelined_quant_one_round(case, deterministic, L.KERNEL_ALIGNED if rows * P * N >= 48 * 128 * 256 else L.KERNEL_SMALL)
 
 
+# kept tiles as halves in one round of workgroups, faster than mixed tiles
+@pytest.mark.parametrize("case", [(512, 3072, 1280, 8, 2, False), (512, 3072, 1280, 8, 5, True)])
+def test_pipelined_quant_one_round_with_halves(case):
+    test_pipelined_quant_one_round(case, True, L.KERNEL_ALIGNED)
+
+
 # one-round pipelined calls that one launch of small tiles takes: 128 and 64 rows by 128 columns, 32 and 64 rows by 64, ranks of ragged rows
 @pytest.mark.parametrize("case", [(512, 2048, 1664, 4, 1, True), (128, 1408, 1504, 8, 6, True), (61, 1540, 1236, 8, 2, True), (96, 1040, 1280, 8, 0, False), (384, 1024, 1028, 2, 1, True)])
 def test_pipelined_quant_one_round_on_small_tiles(case):
