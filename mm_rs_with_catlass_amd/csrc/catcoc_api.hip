@@ -521,7 +521,8 @@ SmallTile small_tile(GemmArgs &a, uint32_t es, const Other &other, uint64_t room
     for (const SmallTileCost &t : kSmallTiles) {
         if (t.cols == 128 && t.rows != 64 && t.rows != 128) {
             // (rows of A and of the peers in 31-bit offsets from a tile's first; the blocks of 128 rows that explicit kept rows' sums are of end where
-            // tiles do.  96 rows of an all-reduce or all-gather as [k,n] are left out: with them 1.0144 of the best choices' time, without 1.0149)
+            // tiles do.  96 rows of an all-reduce or all-gather as [k,n] are not taken, though 58 drawn calls would take 0.94 of their time: 278x4736x4864 of two ranks and
+            // 610x4608x5000 of eight are held to the tiles, and so to the bits, that they had)
             if (!fitted || ldaB * t.rows > 0x7fffffffull || (a.nPeers && (uint64_t)a.peerLd * 4u * t.rows > 0x7fffffffull) || (sums && rowMask)) continue;
             if (t.rows == 96 && s.op != OP_REDUCE_SCATTER && !rowMask && !a.transB) continue;
         }

@@ -502,11 +502,18 @@ inline int launch_mid_tb(const GemmArgs &args, int tileRows, hipStream_t s)
 {
     const dim3 grid(args.fx.rowTiles * args.fx.colTiles), block(512);
     if (tileRows == 64) hipLaunchKernelGGL((gemm_mid_kernel<DT, TB, 2, GA>), grid, block, 0, s, args);
-    else if (tileRows == 96) hipLaunchKernelGGL((gemm_mid_kernel<DT, TB, 3, GA>), grid, block, 0, s, args);
     else if (tileRows == 128) hipLaunchKernelGGL((gemm_mid_kernel<DT, TB, 4, GA>), grid, block, 0, s, args);
     else if (tileRows == 160) hipLaunchKernelGGL((gemm_mid_kernel<DT, TB, 5, GA>), grid, block, 0, s, args);
     else if (tileRows == 192) hipLaunchKernelGGL((gemm_mid_kernel<DT, TB, 6, GA>), grid, block, 0, s, args);
-    else return (int)hipErrorInvalidValue;
+    else {
+        if constexpr (TB || !GA) {   // (all-gathers as [k,n] do not run 96 rows: small_tile())
+            if (tileRows == 96) {
+                hipLaunchKernelGGL((gemm_mid_kernel<DT, TB, 3, GA>), grid, block, 0, s, args);
+                return (int)hipGetLastError();
+            }
+        }
+        return (int)hipErrorInvalidValue;
+    }
     return (int)hipGetLastError();
 }
 

@@ -808,6 +808,14 @@ def test_float_task_sums_rows_between(case, dtype):
     test_float_task_sums(case, dtype)
 
 
+# Explicit kept rows on tiles of 96, 160 and 192 rows: kept rows that end inside a tile, all rows, nine ranks
+@pytest.mark.parametrize("case", [(335, 5472, 544, 8, 62, 270, False, False, "96x128"), (323, 5536, 540, 8, 0, 323, True, True, "96x128"),
+                                  (773, 5024, 516, 9, 169, 602, False, False, "160x128"), (657, 5824, 512, 2, 115, 295, True, True, "160x128"),
+                                  (862, 5664, 520, 4, 309, 433, False, True, "192x128"), (837, 5568, 528, 8, 178, 438, True, False, "192x128")])
+def test_quant_kept_rows_on_rows_between(case):
+    test_quant_kept_rows(case)
+
+
 # Calls beside which other kernels are slower, or that were slower on others: large and small tiles that fill the CUs exactly once; checksums on
 # flexible tiles; k slices of a decode call as [k,n]
 def test_mixed_tiles_that_fill_the_cus_once():
