@@ -25,7 +25,7 @@ PEAK_INT8_TOPS = 5000.0   # MI355X dense int8 MFMA, published
 PEAK_HBM_GBS = 8000.0     # MI355X HBM3E, published
 # Which build of the dominant kernel profiles/traffic.json was recorded for; change both together whenever the kernel
 # or the launch routing of config 4 changes (the counter runs have to be repeated then).
-KERNEL_ID = "gemm_dma_kernel<int8,128x256,3 stages>+int32-reduce epilogue"
+KERNEL_ID = "gemm_dma_kernel<int8,128x256,3 stages,16x16 MFMAs>+int32-reduce epilogue"
 
 
 def cpu_baseline(M, N, K, P, rank, repeats):

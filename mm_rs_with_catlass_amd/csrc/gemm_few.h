@@ -10,7 +10,7 @@
 // waited for the peers in front of them, as a wave's counter retires in order, and their registers for the loop.  Where k is longer than the rings
 // the finishing waves ask for the peers once the first copies are on their way (one barrier): a CU's requests are answered in order, so peers in front
 // of those hold the loop up (43x6912x672 14.4 -> 15.3 us) and behind them they do not (14.5); shorter loops take both at once (92x768x5248 6.8 -> 5.9).
-// One set of four waves -> this, same results: 270 drawn calls take 0.95 of their time, 203x1792x4096 12.55 -> 11.3 us, 16x1024x8192 6.49 -> 6.07,
+// One set of four waves -> this, same results: 272 drawn calls take 0.95 of their time, 203x1792x4096 12.55 -> 11.3 us, 16x1024x8192 6.49 -> 6.07,
 // W8A8 reduce-scatter 192x520x2912 of eight ranks 8.6 -> 6.4, two ranks' 284x576x1408 with explicit kept rows 7.1 -> 5.4.
 //
 // Bound by launch and latency (of 16x1024x8192's 7.1 us out of HBM an empty launch is 2.7 and the chain arguments - copies - partial tiles -
@@ -441,7 +441,8 @@ __global__ void __launch_bounds__(512, 1) gemm_few_kernel(const GemmArgs args)
         }
     }
 
-    // ---- the four partial tiles meet (the same two barriers on both ways)
+    // ---- the four partial tiles meet (two barriers on both ways; the streaming waves then end, and the barriers behind these, of sums and slices, wait for the
+    // waves that are left: s_barrier counts ended ones out)
     uint32_t *dst = (uint32_t *)(smem + G::MEET);   // [BM] what row i of the tile does
     constexpr uint32_t SWZ = BN >= 64 ? 1u : 0u;             // rows with bit 2 set are shifted by 128 bytes: the halves of a wave's write lie in different banks
     if (streams) {

@@ -1,9 +1,9 @@
 // Main loops on 16x16 MFMAs: the instruction, where its operands lie in LDS, and the way back to the layout of 32x32 ones, which the epilogues know.
 //
 // At the board's power limit, where the long loops run, products per second are products per joule.  A 16x16 MFMA takes as many cycles per
-// product as a 32x32 one and less energy: fragment reads and MFMAs alone, 64x128 per wave, eight waves per CU, sustain 1553 TFLOP/s on 32x32
-// and 1766 on 16x16 ones (fp16, normal operands), 3200 and 3730 TOPS (uniform int8).  In the order of snake16() a fragment of B meets four of A
-// and the next one starts with the last of these, so one operand changes at a time: 1734 without the turn.
+// product as a 32x32 one and less energy: fragment reads and MFMAs alone, 64x128 per wave, eight waves per CU, sustain 1505 TFLOP/s on 32x32
+// and 1676 on 16x16 ones (fp16, normal operands), 3083 and 3503 TOPS (uniform int8; profiles/probe_mfma_16x16_and_32x32.md).  In the order of snake16() a fragment
+// of B meets four of A and the next one starts with the last of these, so one operand changes at a time: 1661 and 3473 without the turn.
 // Whole launches on 256x256 tiles, 32x32 -> 16x16, calls behind each other: fp16 8192x27392x4096 as [n,k] 1533 -> 1409 us (1199 -> 1304 TFLOP/s),
 // fp16 all-gather 4 x [610,13632] x [13632,2560] 355 -> 339, 8144x5120x1696 167.5 -> 159.9.
 #pragma once
