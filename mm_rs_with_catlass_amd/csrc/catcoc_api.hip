@@ -293,8 +293,8 @@ bool flex_ptrs_ok(const GemmArgs &a)
 // cache line more per MB.  Half of the estimates are within 0.10 of the tiles' times and 0.06 of the others', nine in ten within 0.22
 // and 0.16.  The tiles of 96, 160 and 192 rows stand on the scale of the 128-row one's (their times relative to it, 1600 calls).  The estimates of
 // 128-column tiles are from when these ran 32x32 MFMAs and come out up to 0.2 high, of flexible tiles in k slices 0.12, so the choice, the tiles with the least, compares
-// shares (other_share), set on 5100 drawn calls, each timed on every tile in reach.  2000 others take 1.015 of the best of these and 0.921 of the time they took before
-// the 16x16 MFMAs and the tiles of 96, 160 and 192 rows, 24 of them more than 1.04; with the shares and the estimate of mixed launches that those came with 0.929, 42 of them.
+// shares (other_share), set on 7100 drawn calls, each timed on every tile in reach.  2100 others take 0.913 of the time they took before
+// the 16x16 MFMAs and the tiles of 96, 160 and 192 rows, 25 of them more than 1.04; with the shares and the estimate of mixed launches that those came with 0.923, 61 of them.
 // For calls unlike those (k below 512, columns that are no multiple of 32, one rank or more than eight) the shares are older and the tiles of 96, 160 and 192 rows
 // left out: 283 drawn ones take 1.032 of the best choice's time, and none lost more than 0.04 by the re-fitted estimates of mixed launches.
 // Figures of calls stand with the kernels that run them (gemm_few.h, gemm_mid.h, gemm_mixed.h).
@@ -329,20 +329,26 @@ CallSize call_size(const GemmArgs &a, uint32_t es)
     return {rows, kB / 1024.0, 1e-6 * kB * (a.N + rows), 1e-6 * a.N * (4.0 * a.nPeers * a.keptRows + (a.sched.op == OP_REDUCE_SCATTER ? 4.0 : 2.0) * rows)};
 }
 
-// 128-row tiles of the aligned kernels (launches of 256-row ones run nothing else).  Kept tiles that are spread over all XCDs alike are the first that each of
-// them starts.  Where they run as halves and all workgroups find a slot at once the launch takes 0.8 of what others of its size take: of four and eight ranks 150
-// calls 0.75 to 0.85, W8A8 4096x1280x3072 pipelined 35.5 us (3072x1600x4096, as many tiles but not spread alike: 51.5).  With more workgroups eight ranks' take 0.8 to 0.95 (pipelined
-// 2048x1088x8192 as [n,k] 41.0; not 16 bits as [n,k] in one round, 4096x1792x4096 87, 83.5 mixed), four ranks' 0.95 to 1.1.
+// Kept tiles that are spread over all XCDs alike are the first that each of them starts.  Where they run as halves and all workgroups find a slot at once the
+// launch takes 0.8 of what others of its size take: of four and eight ranks 150 calls 0.75 to 0.85, W8A8 4096x1280x3072 pipelined 35.5 us (3072x1600x4096, as
+// many tiles but not spread alike: 51.5).  With more workgroups eight ranks' take 0.8 to 0.95 (pipelined 2048x1088x8192 as [n,k] 41.0; not 16 bits as [n,k] in
+// one round, 4096x1792x4096 87, 83.5 mixed), four ranks' 0.95 to 1.1.
+double kept_alike(const GemmArgs &a, bool pipelined)
+{
+    const uint32_t kept = a.sched.P > 2 ? 8u * splittable_kept_tiles(a) : 0u;
+    if (kept == 0) return 1.0;
+    if (a.sched.coreLoops + kept <= 512u) return 0.8;
+    return a.sched.P >= 8 && (pipelined || !a.transB || a.sched.coreLoops > 512u) ? 0.87 : 1.0;
+}
+
+// 128-row tiles of the aligned kernels (launches of 256-row ones run nothing else).
 double aligned_us(const GemmArgs &a, uint32_t es, bool pipelined)
 {
     const CallSize c = call_size(a, es);
     const double f = a.splitK > 1 ? a.splitK : 1.0, wgs = a.sched.coreLoops * f, rounds = ceil(wgs / 256.0), steps = c.kib * 16.0 / f;
     const double us = 6.6 + rounds * (steps * (0.325 + (a.transB ? 0.060 : 0.0) - (es == 1 ? 0.019 : 0.0)) - 2.0) + (wgs > 512.0 ? 0.104 * (wgs / 256.0 - 2.0) * steps : 0.0) +
                       (f > 1.0 ? 10.0 : 0.0) + (a.sched.op == OP_REDUCE_SCATTER ? 1.88 * a.nPeers : 0.0) + 0.134 * c.moved + 0.505 * c.mb;
-    const uint32_t kept = a.sched.P > 2 ? 8u * splittable_kept_tiles(a) : 0u;
-    if (kept == 0) return us;
-    if (a.sched.coreLoops + kept <= 512u) return 0.8 * us;
-    return a.sched.P >= 8 && (pipelined || !a.transB || a.sched.coreLoops > 512u) ? 0.87 * us : us;
+    return us * kept_alike(a, pipelined);
 }
 
 // Flexible tiles as plan_flex left them in args.fx (blocks = rows / 64): whole, with a second launch for the peers, in k slices.
@@ -461,24 +467,25 @@ double other_share(const GemmArgs &a, uint32_t es, const Other &o, bool sums, bo
 {
     const bool rowMask = (a.flags & GF_ROW_MASK) != 0, rs = a.sched.op == OP_REDUCE_SCATTER;
     if (fitted_call(a)) {
-        // (mixed launches, 1200 calls by what would run else: two ranks keep half of all rows, and the other tiles stream the peers under each other's loops; W8A8 launches
-        // of more than 512 aligned tiles, those with a comm launch, flexible ones of k on the 16-byte grid and ragged all-gathers come out shorter than their estimate: pipelined
-        // 4096x2880x5120 as [n,k] 79.8 us aligned, 96.8 mixed; two ranks' 4128x1056x3072 37.0 flexible, 43.4)
+        // (mixed launches, 1400 calls by what would run else: two ranks keep half of all rows, and the other tiles stream the peers under each other's loops; more
+        // than 512 aligned tiles, those with a comm launch, flexible ones of k on the 16-byte grid and ragged all-gathers come out shorter than their
+        // estimate: pipelined 4096x2880x5120 as [n,k] 79.8 us aligned, 96.8 mixed; two ranks' 4128x1056x3072 37.0 flexible, 43.4)
         if (large) {
-            if (!rs) return o.kernel == OTHER_FLEXIBLE && a.sched.op == OP_ALLGATHER ? 0.92 : 1.02;
+            if (!rs) return o.kernel == OTHER_FLEXIBLE && a.sched.op == OP_ALLGATHER ? 0.92 : 1.05;
             if (o.kernel == OTHER_FLEXIBLE) return o.pipelined || (uint64_t)a.K * es % 16 != 0 ? 1.0 : 0.9;
-            return a.sched.P == 2 || (es == 1 && a.sched.coreLoops > 512u) ? 0.9 : o.comm ? 0.88 : 0.98;
+            return a.sched.P == 2 ? 0.92 : a.sched.coreLoops > 512u ? 0.95 : o.comm ? 0.88 : 0.98;
         }
-        // (aligned tiles that are all whole, with checksums: they store nothing; 2048x4096x6144 67.5, 76.6 on 128x128)
-        if (o.kernel == OTHER_ALIGNED && rs && sums && a.sched.P > 2 && a.sched.mRank % a.sched.m0 == 0 && a.N % a.sched.n0 == 0) return 0.95;
+        // (aligned tiles that are all whole, with checksums: they store nothing; 2048x4096x6144 67.5, 76.6 on 128x128; of 450 calls 10 lose more than 0.04, with 1.1 17)
+        if (o.kernel == OTHER_ALIGNED && rs && sums && a.sched.P > 2 && a.sched.mRank % a.sched.m0 == 0 && a.N % a.sched.n0 == 0 && kept_alike(a, false) == 1.0) return 1.0;
         // (pipelined calls, a GEMM and a comm launch or one with peers under its loops, come out longer than their estimate, 37 small ones 1.025 -> 1.008 of their
         // best choice's time with 1.1 for 0.95, W8A8 1024x2272x5888 37.7 -> 31.7 us; but none below 640 of k does; two ranks' kept rows are half of all, and aligned tiles then stream
-        // peers under each other's loops; the 62 calls with 16-bit operands on whole flexible tiles as [k,n] miss 0.015, and with checksums 4520x784x1440 is 28.0 on flexible and
-        // 31.3 on 128x128 tiles; decode calls that could run in k slices, as [k,n], eight ranks 388x7936x512 16.1 there and 18.0 on 32x32 tiles)
+        // peers under each other's loops; the 62 calls with 16-bit operands on whole flexible tiles as [k,n] miss 0.015; with checksums, k on the 16-byte grid, 4520x784x1440 is
+        // 28.0 on flexible and 31.3 on 128x128 tiles, off it 2176x6820x4544 133 on flexible and 101 on 160x128; decode calls that could run in k slices, as [k,n], eight ranks 388x7936x512 16.1 there
+        // and 18.0 on 32x32 tiles)
         if (o.pipelined) return a.K < 640 ? 0.8 : 1.1;
         if (o.kernel == OTHER_STREAMING) return 0.87;
         if (o.kernel == OTHER_SLICED) return rowMask ? 0.875 : 0.9;
-        return o.kernel == OTHER_FLEXIBLE && (sums || (es == 2 && !a.transB)) ? 0.95 : rs && a.sched.P == 2 ? 1.0 : 1.1;
+        return o.kernel == OTHER_FLEXIBLE && ((sums && (uint64_t)a.K * es % 16 == 0) || (es == 2 && !a.transB)) ? 0.95 : rs && a.sched.P == 2 ? 1.0 : 1.1;
     }
     double share = o.kernel == OTHER_ALIGNED ? 0.85 : 0.87;
     if (rs && !sums && wide) share *= 1.15;   // (kept rows are dealt out)
